@@ -1,0 +1,78 @@
+"""The paged attention's tiled form (many rows per sequence) and its grouped 16-row form against a dense float64
+attention: one and two row tiles per wave, tiles cut by sequences and by prefixes, window and kept-prefix edges, score
+modifiers."""
+import math
+
+import pytest
+import torch
+
+from butterfly_amd import ops
+
+F64 = torch.float64
+BS = 32
+
+
+def dense(q, k, v, pos, scale, window, keep, sink, slopes, chunk, qt):
+    """q [n, H, D] at positions pos over k [L, G, D], v [L, G, Dv] of one sequence."""
+    H, G = q.shape[1], k.shape[1]
+    i, j = pos[:, None], torch.arange(k.shape[0])[None]
+    low = i - i % chunk if chunk else i - window + 1
+    see = (j <= i) & ((j >= low) | (j < keep))
+    out = torch.empty(q.shape[0], H, v.shape[2], dtype=F64)
+    for h in range(H):
+        g = h // (H // G)
+        s = q[:, h] @ k[:, g].T * scale
+        if qt:
+            s = s * (1 + qt[0] * torch.log(torch.floor((i + 1) / qt[1]) + 1))
+        if slopes is not None:
+            s = s - slopes[h] * (i - j)
+        s = s.masked_fill(~see, -math.inf)
+        if sink is not None:
+            s = torch.cat([s, sink[h].expand(len(s), 1)], 1)
+        out[:, h] = torch.softmax(s, -1)[:, :k.shape[0]] @ v[:, g]
+    return out
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("H,G,D,Dv,window,keep,mods,seqs", [
+    (16, 4, 128, 128, 1 << 30, 0, "", [(0, 700), (0, 1501)]),         # two row tiles per wave; a ragged last tile
+    (16, 4, 128, 128, 300, 5, "sink", [(0, 2400), (0, 33)]),          # window edges and a kept prefix, pages skipped
+    (16, 4, 128, 128, 64, 40, "sink", [(37, 1100), (1000, 1100)]),    # chunks over a cached prefix, a kept prefix of two pages
+    (8, 2, 128, 128, 300, 0, "slope temp", [(0, 300), (77, 411)]),    # one row tile per wave; distance bias, temperature
+    (16, 16, 64, 64, 100, 0, "chunk", [(0, 640)]),                    # no grouping, chunks instead of a window
+    (32, 2, 128, 128, 512, 0, "slope", [(0, 1030), (5, 1000)]),       # sixteen query heads per key head, two tiles per wave
+    (16, 4, 128, 128, 40, 3, "sink", [(700, 1), (31, 1), (32, 1), (0, 1)]),   # decoded rows: the 16-row form
+])
+def test_paged_tiles_match_dense_attention(H, G, D, Dv, window, keep, mods, seqs):
+    g = torch.Generator().manual_seed(H + D + window % 1000)
+    bf = lambda *s: torch.randn(*s, generator=g).to(torch.bfloat16)                  # noqa: E731
+    dev, scale = "cuda", 2.0 / math.sqrt(D)
+    sink = torch.randn(H, generator=g) if "sink" in mods else None
+    slopes = 0.5 ** torch.linspace(2, 9, H) if "slope" in mods else None
+    qt = (0.3, 50) if "temp" in mods else None
+    chunk = 90 if "chunk" in mods else 0
+    need = [(s + n + BS - 1) // BS for s, n in seqs]
+    order = torch.randperm(sum(need), generator=g)
+    kc = torch.zeros(sum(need), G, BS, D, dtype=torch.bfloat16)
+    vc = torch.zeros(sum(need), G, Dv, BS, dtype=torch.bfloat16)
+    tables = torch.zeros(len(seqs), max(need) + 2, dtype=torch.int32)
+    qs, want, at = [], [], 0
+    for s, (start, n) in enumerate(seqs):
+        pages = order[at:at + need[s]]
+        at += need[s]
+        tables[s, :need[s]] = pages.int()
+        q, k, v = bf(n, H, D), bf(need[s] * BS, G, D), bf(need[s] * BS, G, Dv)      # (pages hold values past the last row)
+        kc[pages] = k.view(-1, BS, G, D).transpose(1, 2)
+        vc[pages] = v.view(-1, BS, G, Dv).permute(0, 2, 3, 1)
+        qs.append(q)
+        L = start + n
+        want.append(dense(q.to(F64), k[:L].to(F64), v[:L].to(F64), torch.arange(start, L), scale, window, keep, sink,
+                          slopes, chunk, qt))
+    cu = torch.tensor([sum(n for _, n in seqs[:i]) for i in range(len(seqs) + 1)], dtype=torch.int32, device=dev)
+    pos = torch.cat([torch.arange(s, s + n) for s, n in seqs]).int().to(dev)
+    got = ops.attn_window_paged(torch.cat(qs).to(dev), kc.to(dev), vc.to(dev), tables.to(dev), cu, pos, scale, window, keep,
+                                None if sink is None else sink.to(dev), chunk=chunk, q_temp=qt,
+                                dist_bias=None if slopes is None else (slopes.to(dev), None))
+    # weights rounded to bf16 (2^-9 each, together at most 2^-9 of the largest value), the output rounded once more
+    err = (got.cpu().to(F64) - torch.cat(want)).abs().max()
+    assert err < 2.0 ** -8 * vc.float().abs().max() + 1e-3
