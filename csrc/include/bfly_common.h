@@ -113,6 +113,18 @@ __device__ __forceinline__ float gelu_tanh(float x) {
   return 0.5f * x * (1.f + tanhf(k0 * (x + k1 * x * x * x)));
 }
 
+// Grouped expert GEMMs of the score-routed experts (gemm_big4_kernel GROUPED 2 / 3): moe_sort's groups and what the
+// epilogues need
+struct ExpertArgs {
+  const int* perm = nullptr;        // row -> (token, choice) pair
+  const int* offsets = nullptr;     // [E + 1] group bounds
+  const int* tiles = nullptr;       // [..][2] (expert, first row)
+  const float* topk_w = nullptr;    // up: the pair's score scales the row (nullptr: 1)
+  int choices = 1, plain = 0;       // choices per token; plain: squared ReLU without a gate
+  float limit = 0.f, alpha = 0.f, up_offset = 0.f;
+  float* y = nullptr;               // down: f32 rows in pair order
+};
+
 }  // namespace bfly
 
 #define BFLY_HIP_CHECK(expr)                                                  \

@@ -126,8 +126,13 @@ void launch_moe_topk_scores(const float* logits, const float* bias, int top_k, i
 void launch_moe_sort(const int* ids, int TK, int E, int* perm, int* offsets, int* tiles, int* ntiles, int tile_rows,
                      hipStream_t s);
 int moe_sort_max_tiles(int TK, int E);
-// rows per tile of the grouped expert GEMMs for this problem (64, or 128 for large bf16 groups)
-int moe_tile_rows(int TK, int E, bool f32);
+// rows per tile of the grouped expert GEMMs for this problem (64, 128 for large bf16 groups, 256 where `big` allows the
+// LDS-DMA tile: moe_big_ok)
+int moe_tile_rows(int TK, int E, bool f32, bool big, int Hd);
+// whether the operands fit the 256 x 256 LDS-DMA tile: bf16, 16-byte aligned rows, byte offsets below 2^31, K steps and
+// column tiles without a remainder. plain: experts without a gate
+bool moe_big_ok(const void* x, long ldx, const void* gate_up_w, const void* down_w, const void* hmid, const void* y, int T,
+                int TK, int Hd, int F, bool plain, bool f32);
 // hmid[r, f] = g' sigmoid(alpha g') (u' + up_offset), (g', u') the clamped gate / up products of
 // expert e(r) on (w x) for grouped row r (topk_w == nullptr: on x itself). plain_act != ACT_NONE: experts
 // without a gate, gate_up_w [E, F, Hd] and hmid = act(up product) (ACT_RELU2)

@@ -943,17 +943,23 @@ __device__ __forceinline__ void b4_dma(__amdgpu_buffer_rsrc_t r, char* lds, int 
   __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_ptr_t)lds, 16, voff, soff, 0, 0);
 }
 
-// GROUPED (MoE expert GEMM at prefill scale): as gemm_big8_kernel<true> — M tiles are the
+// GROUPED 1 (MoE expert GEMM at prefill scale): as gemm_big8_kernel<true> — M tiles are the
 // entries of the device tile list {expert, first row slot, end slot}, W is offset by the expert,
 // A rows are gathered through grows[slot] by per-lane LDS-DMA offsets from X (rows past the
 // tile's end re-read its last row; their outputs are not stored).
-template <bool GROUPED = false>
+// GROUPED 2 / 3 (ExpertArgs, the score-routed experts of the heterogeneous stacks): the up / gate-and-up
+// projection and the down projection over the row groups of moe_sort. A gate's 64 rows and the up rows of the same
+// 64 columns are the two halves of a wave's 128 columns (the weight DMA picks the rows: the stored panels stay
+// [gate | up]), so the clamped GLU runs on a lane's own accumulators; an expert that runs on (score x row) scales
+// the accumulators by the score instead of rounding scaled rows. The down projection leaves f32 rows at their
+// (token, choice) pair. Measured beside the smaller tiles: moe_tile_rows.
+template <int GROUPED = 0>
 __global__ void __launch_bounds__(kB4Threads) __attribute__((amdgpu_waves_per_eu(1, 1)))
 gemm_big4_kernel(const bf16* __restrict__ X, long ldx, const bf16* __restrict__ W, long ldw,
                  int M, int N, int K, int epi, const bf16* __restrict__ bias,
                  bf16* __restrict__ out, long ldo, float* __restrict__ part,
                  const int* __restrict__ grows = nullptr, const int4* __restrict__ gtiles = nullptr,
-                 const int* __restrict__ gcount = nullptr, long w_estride = 0) {
+                 const int* __restrict__ gcount = nullptr, long w_estride = 0, ExpertArgs ex = ExpertArgs()) {
   constexpr int BM = 256, BN = 256;
   extern __shared__ __attribute__((aligned(16))) char smem[];
   // wave index in an SGPR: the DMA's LDS destinations (M0) and the fragment row bases are then
@@ -967,7 +973,15 @@ gemm_big4_kernel(const bf16* __restrict__ X, long ldx, const bf16* __restrict__ 
   const int gsize = min(mtiles - first_m, kBigGroupM);
   int m0 = (first_m + (t % per_group) % gsize) * BM;
   const int n0 = ((t % per_group) / gsize) * BN;
-  if constexpr (GROUPED) {
+  if constexpr (GROUPED >= 2) {
+    const int ti = m0 / BM;
+    if (ti >= *gcount) return;
+    const int e = ex.tiles[2 * ti];
+    W += (long)e * w_estride;
+    m0 = ex.tiles[2 * ti + 1];
+    M = ex.offsets[e + 1];         // rows [m0, M) of the expert's group
+  }
+  if constexpr (GROUPED == 1) {
     const int ti = m0 / BM;
     if (ti >= *gcount) return;
     const int4 info = gtiles[ti];
@@ -984,27 +998,30 @@ gemm_big4_kernel(const bf16* __restrict__ X, long ldx, const bf16* __restrict__ 
   // linear); lane L supplies row 8 (8 w + s) + (L >> 3) at the chunk lds_frag expects in
   // position L & 7: chunk = (L & 7) ^ ((row >> 1) & 7) = (L & 7) ^ ((L >> 4) + 4 (s & 1)) & 7
   const auto rsa = b8_rsrc(X + (long)m0 * ldx, M - m0, ldx);   // A rows past M read zeros
-  const auto rsb = b8_rsrc(W + (long)n0 * ldw, N - n0, ldw);
+  const bool glu = GROUPED == 2 && !ex.plain;
+  const auto rsb = glu ? b8_rsrc(W, N, ldw) : b8_rsrc(W + (long)n0 * ldw, N - n0, ldw);
   const int drow = 64 * wid + (lane >> 3);
+  // weight row of LDS row drow: with a gate, waves 0 / 2 stage gate rows and 1 / 3 the up rows of the same columns
+  const int brow = glu ? (wid & 1) * (N >> 1) + (n0 >> 1) + (wid >> 1) * 64 + (lane >> 3) : drow;
   int va[2], vb[2];
 #pragma unroll
   for (int e = 0; e < 2; ++e) {
     const int ch = (lane & 7) ^ (((lane >> 4) + 4 * e) & 7);
     va[e] = (int)((drow * ldx + ch * 8) * 2);
-    vb[e] = (int)((drow * ldw + ch * 8) * 2);
+    vb[e] = (int)((brow * ldw + ch * 8) * 2);
   }
   int ga[8] = {};   // GROUPED: byte offsets from X of this lane's gathered rows (at its chunk)
   const auto rsx = b8_rsrc(X, 1L << 30, 1);
-  if constexpr (GROUPED) {
+  if constexpr (GROUPED == 1 || GROUPED == 2) {
 #pragma unroll
     for (int q = 0; q < 8; ++q) {
       const int slot = min(m0 + drow + 8 * q, M - 1);
-      const long src = grows != nullptr ? grows[slot] : slot;
+      const long src = GROUPED == 2 ? ex.perm[slot] / ex.choices : grows != nullptr ? grows[slot] : slot;
       ga[q] = (int)((src * ldx + (((lane & 7) ^ (((lane >> 4) + 4 * (q & 1)) & 7)) * 8)) * 2);
     }
   }
   auto dma_a = [&](int k, int slot, int s) {
-    if constexpr (GROUPED)
+    if constexpr (GROUPED == 1 || GROUPED == 2)
       b4_dma(rsx, smem + slot * kB4Slot + (8 * wid + s) * 1024, ga[s], (kt0 + k) * 128);
     else
       b4_dma(rsa, smem + slot * kB4Slot + (8 * wid + s) * 1024, va[s & 1], (kt0 + k) * 128 + (int)(8 * s * ldx * 2));
@@ -1093,6 +1110,48 @@ gemm_big4_kernel(const bf16* __restrict__ X, long ldx, const bf16* __restrict__ 
   }
   ks1(nk - 1, sa, (nk - 1) & 1, sa == 2 ? 0 : sa + 1);
   vm_wait<0>();                       // no LDS-DMA may outlive the workgroup
+  if constexpr (GROUPED >= 2) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int r = m0 + wr * 128 + 16 * i + fr;
+      if (r >= M) continue;
+      const int p = ex.perm[r];
+      if constexpr (GROUPED == 3) {
+        float* yr = ex.y + (long)p * ldo + n0 + wc * 128 + 4 * fq;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) *reinterpret_cast<f32x4*>(yr + 16 * j) = acc[i][j];
+      } else {
+        const float sc = ex.topk_w ? ex.topk_w[p] : 1.f;
+        if (ex.plain) {      // squared ReLU
+          bf16* hr = out + (long)r * ldo + n0 + wc * 128 + 4 * fq;
+#pragma unroll
+          for (int j = 0; j < 8; ++j) {
+            bf16x4 w;
+#pragma unroll
+            for (int x = 0; x < 4; ++x) {
+              const float v = fmaxf(acc[i][j][x] * sc, 0.f);
+              w[x] = (bf16)(v * v);
+            }
+            *reinterpret_cast<bf16x4*>(hr + 16 * j) = w;
+          }
+        } else {
+          bf16* hr = out + (long)r * ldo + (n0 >> 1) + wc * 64 + 4 * fq;
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            bf16x4 w;
+#pragma unroll
+            for (int x = 0; x < 4; ++x) {
+              const float g = fminf(acc[i][j][x] * sc, ex.limit);
+              const float u = fminf(fmaxf(acc[i][j + 4][x] * sc, -ex.limit), ex.limit);
+              w[x] = (bf16)(glu_gate(g, ex.alpha, __expf(-ex.alpha * g)) * (u + ex.up_offset));
+            }
+            *reinterpret_cast<bf16x4*>(hr + 16 * j) = w;
+          }
+        }
+      }
+    }
+    return;
+  }
   tile_epilogue<8, 8>(acc, m0 + wr * 128, n0 + wc * 128, lane, M, N, epi, bias, out, ldo,
                       part ? part + (long)blockIdx.y * M * N + (long)m0 * N : nullptr, m0,
                       RowScale{nullptr, 0, 0.f, 0.f});
@@ -1955,6 +2014,26 @@ int launch_gemm_grouped(const bf16* X, long ldx, const bf16* W, long ldw, long w
     return launch_grouped_bm<64>(X, ldx, W, ldw, w_estride, N, K, epi, rows, tiles, count, max_tiles,
                                  slots, sk, part, out, ldo, stream);
   return -3;
+}
+
+// 256-row groups of the score-routed experts on gemm_big4_kernel (bfly_mixers.h)
+void launch_moe_big(bool down, const bf16* X, long ldx, const bf16* W, int N, int K, int max_tiles, const int* ntiles,
+                    bf16* out, long ldo, const ExpertArgs& ex, hipStream_t stream) {
+  static bool attr = false;
+  if (!attr) {
+    hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_big4_kernel<2>), hipFuncAttributeMaxDynamicSharedMemorySize,
+                        kB4LdsBytes);
+    hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_big4_kernel<3>), hipFuncAttributeMaxDynamicSharedMemorySize,
+                        kB4LdsBytes);
+    attr = true;
+  }
+  const dim3 grid(max_tiles * (N / 256), 1);
+  if (down)
+    gemm_big4_kernel<3><<<grid, kB4Threads, kB4LdsBytes, stream>>>(X, ldx, W, K, max_tiles * 256, N, K, EPI_NONE, nullptr, out,
+                                                                   ldo, nullptr, nullptr, nullptr, ntiles, (long)N * K, ex);
+  else
+    gemm_big4_kernel<2><<<grid, kB4Threads, kB4LdsBytes, stream>>>(X, ldx, W, K, max_tiles * 256, N, K, EPI_NONE, nullptr, out,
+                                                                   ldo, nullptr, nullptr, nullptr, ntiles, (long)N * K, ex);
 }
 
 int gemm_check(int M, int N, int K, int epi) {

@@ -760,8 +760,28 @@ void launch_moe_topk_scores(const float* logits, const float* bias, int top_k, i
 
 int moe_sort_max_tiles(int TKp, int E) { return (TKp + 63) / 64 + E; }
 
-// 128-row tiles when the experts average at least 256 grouped rows (bf16 only), else 64
-int moe_tile_rows(int TKp, int E, bool f32) { return (!f32 && TKp >= 256 * E) ? 128 : 64; }
+void launch_moe_big(bool down, const bf16* X, long ldx, const bf16* W, int N, int K, int max_tiles, const int* ntiles,
+                    bf16* out, long ldo, const ExpertArgs& ex, hipStream_t stream);      // gemm.hip
+
+bool moe_big_ok(const void* x, long ldx, const void* gate_up_w, const void* down_w, const void* hmid, const void* y, int T,
+                int TKp, int Hd, int F, bool plain, bool f32) {
+  const auto al = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
+  const long lim = 0x7fffffffL;
+  return !f32 && Hd % 256 == 0 && F % (plain ? 256 : 128) == 0 && F >= 128 && ldx % 8 == 0 && al(x) && al(gate_up_w) &&
+         al(down_w) && al(hmid) && al(y) && (long)T * ldx * 2 < lim && (plain ? 1L : 2L) * F * Hd * 2 < lim &&
+         (long)TKp * F * 2 < lim;
+}
+
+// 256-row tiles on the LDS-DMA kernel from an average of 256 grouped rows per expert, and from 128 where the width gives
+// a group at least 8 column tiles; below that the 64-row tiles have more workgroups. Whole op, 8 experts, us before
+// (64 / 128-row tiles) -> now: width 2048, GLU of 2048, 16384 rows 1343 -> 483 (0.93 PFLOP/s in the two GEMMs), 2048
+// rows 273 -> 114, 1024 rows 119 -> 104; width 4096, 4096: 16384 rows 4774 -> 1481; width 1024, plain 1536: 16384 rows
+// 358 -> 174, 2048 rows 102 -> 77, but 1024 rows 58 -> 69. Shapes outside moe_big_ok: 128-row tiles from 256 rows
+// (bf16 only), else 64.
+int moe_tile_rows(int TKp, int E, bool f32, bool big, int Hd) {
+  if (big && TKp >= (Hd >= 2048 ? 128 : 256) * E) return 256;
+  return (!f32 && TKp >= 256 * E) ? 128 : 64;
+}
 
 void launch_moe_sort(const int* ids, int TKp, int E, int* perm, int* offsets, int* tiles, int* ntiles, int tile_rows,
                      hipStream_t s) {
@@ -772,6 +792,14 @@ void launch_moe_glu_up(const void* x, long ldx, const float* topk_w, int K, cons
                        const int* tiles, const int* ntiles, int max_tiles, const void* gate_up_w, float limit,
                        float alpha, float up_offset, void* hmid, int Hd, int F, bool f32, int tile_rows, hipStream_t s,
                        int plain_act) {
+  if (tile_rows == 256) {
+    ExpertArgs ex;
+    ex.perm = perm; ex.offsets = offsets; ex.tiles = tiles; ex.topk_w = topk_w; ex.choices = K;
+    ex.plain = plain_act != ACT_NONE; ex.limit = limit; ex.alpha = alpha; ex.up_offset = up_offset;
+    launch_moe_big(false, (const bf16*)x, ldx, (const bf16*)gate_up_w, (ex.plain ? 1 : 2) * F, Hd, max_tiles, ntiles,
+                   (bf16*)hmid, F, ex, s);
+    return;
+  }
   if (tile_rows == 128) {
     dim3 g2((F + 127) / 128, max_tiles);
     moe_glu_up_mfma_kernel<4><<<g2, 256, 0, s>>>((const bf16*)x, ldx, topk_w, K, perm, offsets, tiles, ntiles,
@@ -792,6 +820,12 @@ void launch_moe_glu_up(const void* x, long ldx, const float* topk_w, int K, cons
 
 void launch_moe_down(const void* hmid, const int* perm, const int* offsets, const int* tiles, const int* ntiles,
                      int max_tiles, const void* down_w, float* y, int Hd, int F, bool f32, int tile_rows, hipStream_t s) {
+  if (tile_rows == 256) {
+    ExpertArgs ex;
+    ex.perm = perm; ex.offsets = offsets; ex.tiles = tiles; ex.y = y;
+    launch_moe_big(true, (const bf16*)hmid, F, (const bf16*)down_w, Hd, F, max_tiles, ntiles, nullptr, Hd, ex, s);
+    return;
+  }
   if (tile_rows == 128) {
     dim3 g2((Hd + 127) / 128, max_tiles);
     moe_down_mfma_kernel<4><<<g2, 256, 0, s>>>((const bf16*)hmid, perm, offsets, tiles, ntiles, (const bf16*)down_w, y,

@@ -1,0 +1,60 @@
+"""Score-routed experts over large row groups (the 256-row LDS-DMA tiles and the smaller ones beside them) against float64."""
+import math
+
+import pytest
+import torch
+
+from butterfly_amd import ops
+
+F64 = torch.float64
+
+
+def reference(x, ids, w, gu, dn, limit, alpha, offset, scaled, plain):
+    T, K = ids.shape
+    F = dn.shape[2]
+    y = torch.zeros(T, x.shape[1], dtype=F64)
+    for e in range(gu.shape[0]):
+        t, j = (ids == e).nonzero(as_tuple=True)
+        if not t.numel():
+            continue
+        s = w[t, j][:, None]
+        h = (x[t] * s if scaled else x[t]) @ gu[e].T
+        if plain:
+            a = torch.relu(h) ** 2
+        else:
+            g = torch.clamp(h[:, :F], max=limit)
+            a = g * torch.sigmoid(alpha * g) * (torch.clamp(h[:, F:], -limit, limit) + offset)
+        o = a @ dn[e].T
+        y.index_add_(0, t, o if scaled else s * o)
+    return y
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("counts,Hd,F,plain,scaled,limit", [
+    ([256, 257, 255, 1], 256, 128, False, True, 7.0),        # tile edges; the smallest panel; one row in a tile
+    ([700, 0, 600], 512, 384, False, False, math.inf),       # an expert without rows; weighted outputs
+    ([513, 256, 40, 300], 768, 256, True, False, math.inf),  # plain experts
+    ([600, 500], 256, 192, False, True, 7.0),                # F not a multiple of 128: the 128-row tiles
+    ([300, 290], 320, 128, True, True, math.inf),            # Hd not a multiple of 256; scores on plain experts
+    ([60, 50, 70], 256, 256, False, True, 7.0),              # small groups: the 64-row tiles
+])
+@pytest.mark.parametrize("stride", [0, 8])
+def test_experts_over_row_groups(counts, Hd, F, plain, scaled, limit, stride):
+    g = torch.Generator().manual_seed(sum(counts) + F)
+    E, TK = len(counts), sum(counts)
+    K = 2 if TK % 2 == 0 else 1
+    flat = torch.cat([torch.full((c,), e) for e, c in enumerate(counts)])[torch.randperm(TK, generator=g)]
+    ids = flat.view(-1, K)
+    T = ids.shape[0]
+    bf = lambda *s, k=1.0: (k * torch.randn(*s, generator=g)).to(torch.bfloat16)            # noqa: E731
+    x = bf(T, Hd + stride)[:, :Hd]
+    w = torch.rand(T, K, generator=g) + 0.2
+    gu, dn = bf(E, F if plain else 2 * F, Hd, k=2 * Hd ** -0.5), bf(E, Hd, F, k=F ** -0.5)
+    d = lambda t: t.to("cuda")                                                           # noqa: E731
+    xd = torch.empty(T, Hd + stride, dtype=torch.bfloat16, device="cuda")[:, :Hd].copy_(x)
+    got = ops.moe_glu_ffn(xd, d(ids.int()), d(w), d(gu), d(dn), limit, 1.702, 1.0, scaled, "relu2" if plain else None)
+    want = reference(x.to(F64), ids, w.to(F64), gu.to(F64), dn.to(F64), limit, 1.702, 1.0, scaled, plain)
+    # bf16 hidden rows and output (2^-9 each); the smaller tiles also round the scaled input rows, whose error the
+    # squared activation can double
+    err = (got.cpu().to(F64) - want).norm() / want.norm()
+    assert err < 2.0 ** -7
