@@ -2,7 +2,8 @@
 // follows a linear attention; generic in every size and in the activation type (bf16 or f32; gates, decays, states
 // and the recurrence are f32 in both):
 //   forget_chunk_kernel, forget_step_kernel   f = l + (1 - l) sigmoid(z + b), S <- diag(f) S + (1 - f) v^T, o = S^T q,
-//                                             in chunks on the f32 matrix cores or row by row
+//                                             in chunks on the f32 matrix cores or row by row; the chunk form also runs
+//                                             gated linear attention, whose key is an input (GLA)
 //   head_norm_gate_kernel                     RMS norm per head, times an optional weight, a gate and a factor
 // Rows of a step are packed: sequence s owns rows row_cu[s] .. row_cu[s+1]; a sequence whose first row is at
 // position 0 starts from a zero state whatever its slot holds.
@@ -23,6 +24,14 @@ __device__ __forceinline__ void sigmoid2(float x, float& s, float& c) {
   const float r = FAST ? __builtin_amdgcn_rcpf(1.f + e) : 1.f / (1.f + e);
   s = x < 0.f ? e * r : r;
   c = x < 0.f ? r : e * r;
+}
+
+// sigmoid(z)^(1 / tau): exp of the log sigmoid, stable on both sides
+template <bool FAST>
+__device__ __forceinline__ float gla_decay(float z, float inv_tau) {
+  const float e = FAST ? __expf(-fabsf(z)) : expf(-fabsf(z));
+  const float ls = fminf(z, 0.f) - (FAST ? __logf(1.f + e) : log1pf(e));
+  return FAST ? __expf(ls * inv_tau) : expf(ls * inv_tau);
 }
 
 // One element at a byte offset below 2^31 from a uniform base. (Rows of one chunk; callers clamp row and channel to the
@@ -55,9 +64,11 @@ __device__ __forceinline__ float half_sum(float v) {
 // products); the two 8 x 8 blocks on the diagonal are formed on the vector units while the matrix cores are busy: 32
 // lanes per row t share its channels, and q_t times the decays so far is carried down j. Rows past the sequence have f = 1,
 // k = q = 0. D <= 16 NT, NT even.
-template <typename T, int NT>
-__global__ __launch_bounds__(512, NT <= 8 ? 4 : 2) void forget_chunk_kernel(const T* __restrict__ q, long q_ld, const T* __restrict__ z,
-                                                           long z_ld, const T* __restrict__ v, long v_ld,
+// GLA: f = sigmoid(z)^(1 / tau) and k is an input, loaded by the lanes that hold k's channels.
+template <typename T, int NT, bool GLA>
+__global__ __launch_bounds__(512, NT <= 8 ? 4 : 2) void forget_chunk_kernel(const T* __restrict__ q, long q_ld,
+                                                           const T* __restrict__ key, long k_ld, float inv_tau, float q_scale,
+                                                           const T* __restrict__ z, long z_ld, const T* __restrict__ v, long v_ld,
                                                            const float* __restrict__ f_bias,
                                                            const float* __restrict__ lower, float* __restrict__ state,
                                                            const int* __restrict__ state_slots,
@@ -118,8 +129,8 @@ __global__ __launch_bounds__(512, NT <= 8 ? 4 : 2) void forget_chunk_kernel(cons
 #pragma unroll
   for (int u = 0; u < NI; ++u) {
     const int idx = role + 256 * u, d = min(idx < DP ? idx : idx - DP, D - 1);
-    rb[u] = f_bias[(long)h * D + d];
-    rl[u] = lower[(long)h * D + d];
+    rb[u] = GLA ? 0.f : f_bias[(long)h * D + d];
+    rl[u] = GLA ? 0.f : lower[(long)h * D + d];
   }
   // the next chunk's inputs as they are stored (rows past the sequence: its last row again)
   typedef T t4 __attribute__((ext_vector_type(4)));
@@ -128,7 +139,9 @@ __global__ __launch_bounds__(512, NT <= 8 ? 4 : 2) void forget_chunk_kernel(cons
   auto fetch = [&](int t0) {
     const __amdgpu_buffer_rsrc_t qb = rows_rsrc(q + (long)t0 * q_ld + (long)h * D);
     const __amdgpu_buffer_rsrc_t zb = rows_rsrc(z + (long)t0 * z_ld + (long)h * D);
-    const int qs = (int)q_ld * (int)sizeof(T), zs = (int)z_ld * (int)sizeof(T), last = r1 - 1 - t0;
+    const __amdgpu_buffer_rsrc_t kb = rows_rsrc(GLA ? key + (long)t0 * k_ld + (long)h * D : q);
+    const int qs = (int)q_ld * (int)sizeof(T), zs = (int)z_ld * (int)sizeof(T), ks = (int)k_ld * (int)sizeof(T);
+    const int last = r1 - 1 - t0;
 #pragma unroll
     for (int u = 0; u < NI; ++u) {
       const int idx = role + 256 * u;
@@ -136,6 +149,9 @@ __global__ __launch_bounds__(512, NT <= 8 ? 4 : 2) void forget_chunk_kernel(cons
       if (idx < DP) {
 #pragma unroll
         for (int i = 0; i < HC; ++i) rq[u][i] = row_load<T>(qb, __umul24(min(ra + i, last), qs) + d);
+      } else if (GLA && (WHOLE || idx < 2 * DP)) {
+#pragma unroll
+        for (int i = 0; i < HC; ++i) rq[u][i] = row_load<T>(kb, __umul24(min(ra + i, last), ks) + d);
       }
       if (WHOLE || idx < 2 * DP) {
 #pragma unroll
@@ -165,9 +181,16 @@ __global__ __launch_bounds__(512, NT <= 8 ? 4 : 2) void forget_chunk_kernel(cons
         float F = 1.f, w[HC];
 #pragma unroll
         for (int i = 0; i < HC; ++i) {
-          float sg, cg;
-          sigmoid2<FAST>((float)rz[u][i] + rb[u], sg, cg);
-          float f = fmaf(one, sg, rl[u]), qv = act_in<FAST>((float)rq[u][i], act) * qm;
+          float f, qv;
+          if constexpr (GLA) {
+            f = gla_decay<FAST>((float)rz[u][i], inv_tau);
+            qv = (float)rq[u][i] * q_scale * qm;
+          } else {
+            float sg, cg;
+            sigmoid2<FAST>((float)rz[u][i] + rb[u], sg, cg);
+            f = fmaf(one, sg, rl[u]);
+            qv = act_in<FAST>((float)rq[u][i], act) * qm;
+          }
           if (decltype(tail)::value) {
             const float in = ra + i < n ? 1.f : 0.f;
             f = fmaf(in, f, 1.f - in);
@@ -190,9 +213,16 @@ __global__ __launch_bounds__(512, NT <= 8 ? 4 : 2) void forget_chunk_kernel(cons
         float B = 1.f, w[HC];
 #pragma unroll
         for (int i = HC - 1; i >= 0; --i) {
-          float sg, cg;
-          sigmoid2<FAST>((float)rz[u][i] + rb[u], sg, cg);
-          float f = fmaf(one, sg, rl[u]), k = one * cg;
+          float f, k;
+          if constexpr (GLA) {
+            f = gla_decay<FAST>((float)rz[u][i], inv_tau);
+            k = (float)rq[u][i];
+          } else {
+            float sg, cg;
+            sigmoid2<FAST>((float)rz[u][i] + rb[u], sg, cg);
+            f = fmaf(one, sg, rl[u]);
+            k = one * cg;
+          }
           if (decltype(tail)::value) {
             const float in = ra + i < n ? 1.f : 0.f;
             f = fmaf(in, f, 1.f - in);
@@ -446,21 +476,21 @@ __global__ __launch_bounds__(256) void head_norm_gate_kernel(const float* __rest
   }
 }
 
-template <typename T, int NT>
-void forget_chunk_launch(const T* q, long q_ld, const T* z, long z_ld, const T* v, long v_ld, const float* f_bias,
+template <typename T, int NT, bool GLA>
+void forget_chunk_launch(const T* q, long q_ld, const T* key, long k_ld, float inv_tau, float q_scale, const T* z, long z_ld, const T* v, long v_ld, const float* f_bias,
                          const float* lower, float* state, const int* state_slots, const int* row_cu, int nseq,
                          const int* positions, int act, int vec, float* o, int H, int D, int Dv, hipStream_t s) {
   constexpr int DP = 16 * NT, KP = (DP + 127) / 128 * 128 + 4;
   constexpr size_t lds = (size_t)(97 * KP + 2 * 16 * 68 + 16 * 20 + 64 * (NT < 8 ? NT : 8) + DP) * sizeof(float);
   static bool once = false;
   if (!once) {
-    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&forget_chunk_kernel<T, NT>),
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&forget_chunk_kernel<T, NT, GLA>),
                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     once = true;
   }
   dim3 grid(nseq, H, (Dv + 63) / 64);
-  forget_chunk_kernel<T, NT><<<grid, 512, lds, s>>>(q, q_ld, z, z_ld, v, v_ld, f_bias, lower, state, state_slots, row_cu,
-                                                    positions, act, vec, o, H, D, Dv);
+  forget_chunk_kernel<T, NT, GLA><<<grid, 512, lds, s>>>(q, q_ld, key, k_ld, inv_tau, q_scale, z, z_ld, v, v_ld, f_bias, lower,
+                                                         state, state_slots, row_cu, positions, act, vec, o, H, D, Dv);
 }
 
 template <typename T>
@@ -478,7 +508,7 @@ void forget_scan_t(const T* q, long q_ld, const T* z, long z_ld, const T* v, lon
     return;
   }
 #define BFLY_FCH(NT)                                                                                                  \
-  forget_chunk_launch<T, NT>(q, q_ld, z, z_ld, v, v_ld, f_bias, lower, state, state_slots, row_cu, nseq, positions, act, \
+  forget_chunk_launch<T, NT, false>(q, q_ld, nullptr, 0, 1.f, 1.f, z, z_ld, v, v_ld, f_bias, lower, state, state_slots, row_cu, nseq, positions, act, \
                              vec, o, H, D, Dv, s)
   if (D <= 32) BFLY_FCH(2);
   else if (D <= 64) BFLY_FCH(4);
@@ -487,6 +517,23 @@ void forget_scan_t(const T* q, long q_ld, const T* z, long z_ld, const T* v, lon
   else if (D <= 192) BFLY_FCH(12);
   else BFLY_FCH(16);
 #undef BFLY_FCH
+}
+
+template <typename T>
+void gla_chunks_t(const T* q, long q_ld, const T* k, long k_ld, const T* v, long v_ld, const T* z, long z_ld, float* state,
+                  const int* state_slots, const int* row_cu, int nseq, const int* positions, float tau, float q_scale, float* o,
+                  int H, int D, int Dv, hipStream_t s) {
+  const int vec = (Dv % 4 == 0 && rows_aligned(v, v_ld, sizeof(T))) ? 2 : 0;
+#define BFLY_GCH(NT)                                                                                                   \
+  forget_chunk_launch<T, NT, true>(q, q_ld, k, k_ld, 1.f / tau, q_scale, z, z_ld, v, v_ld, nullptr, nullptr, state,    \
+                                   state_slots, row_cu, nseq, positions, 0, vec, o, H, D, Dv, s)
+  if (D <= 32) BFLY_GCH(2);
+  else if (D <= 64) BFLY_GCH(4);
+  else if (D <= 96) BFLY_GCH(6);
+  else if (D <= 128) BFLY_GCH(8);
+  else if (D <= 192) BFLY_GCH(12);
+  else BFLY_GCH(16);
+#undef BFLY_GCH
 }
 
 template <typename T, int V>
@@ -516,6 +563,17 @@ void launch_forget_scan(const void* q, long q_ld, const void* z, long z_ld, cons
   else
     forget_scan_t<bf16>((const bf16*)q, q_ld, (const bf16*)z, z_ld, (const bf16*)v, v_ld, f_bias, lower, state, state_slots,
                         row_cu, nseq, positions, act, o, H, D, Dv, one_row, s);
+}
+
+void launch_gla_chunks(const void* q, long q_ld, const void* k, long k_ld, const void* v, long v_ld, const void* z, long z_ld,
+                       float* state, const int* state_slots, const int* row_cu, int nseq, const int* positions, float tau,
+                       float q_scale, float* o, int H, int D, int Dv, bool f32, hipStream_t s) {
+  if (f32)
+    gla_chunks_t<float>((const float*)q, q_ld, (const float*)k, k_ld, (const float*)v, v_ld, (const float*)z, z_ld, state,
+                        state_slots, row_cu, nseq, positions, tau, q_scale, o, H, D, Dv, s);
+  else
+    gla_chunks_t<bf16>((const bf16*)q, q_ld, (const bf16*)k, k_ld, (const bf16*)v, v_ld, (const bf16*)z, z_ld, state,
+                       state_slots, row_cu, nseq, positions, tau, q_scale, o, H, D, Dv, s);
 }
 
 void launch_head_norm_gate(const float* o, const float* w, float eps, const void* gate, long g_ld, int act, float mul,

@@ -286,11 +286,22 @@ static int gla_scan_t(const T* q, long q_ld, const T* k, long k_ld, const T* v, 
   return 0;
 }
 
+void launch_gla_chunks(const void* q, long q_ld, const void* k, long k_ld, const void* v, long v_ld, const void* z, long z_ld,
+                       float* state, const int* state_slots, const int* row_cu, int nseq, const int* positions, float tau,
+                       float q_scale, float* o, int H, int D, int Dv, bool f32, hipStream_t s);      // forget.hip
+
 int launch_gla_scan(const void* q, long q_ld, const void* k, long k_ld, const void* v, long v_ld, const void* z,
                     long z_ld, float* state, const int* state_slots, const int* row_cu, int nseq,
                     const int* positions, float tau, float q_scale, float* o, int T, int H, int D, int Dv, bool f32,
                     hipStream_t s) {
   if (T <= 0 || nseq <= 0) return 0;
+  // any prompt rows (some sequence has more than one): chunks on the f32 matrix cores; the token loop keeps the steps of
+  // single rows, where a chunk would be 15 / 16 padding
+  if (T > nseq && D <= 256 && std::max({q_ld, k_ld, z_ld}) < (1L << 21)) {
+    launch_gla_chunks(q, q_ld, k, k_ld, v, v_ld, z, z_ld, state, state_slots, row_cu, nseq, positions, tau, q_scale, o, H, D,
+                      Dv, f32, s);
+    return 0;
+  }
   if (f32)
     return gla_scan_t<float>((const float*)q, q_ld, (const float*)k, k_ld, (const float*)v, v_ld, (const float*)z, z_ld,
                              state, state_slots, row_cu, nseq, positions, tau, q_scale, o, H, D, Dv, s);

@@ -1,0 +1,41 @@
+"""Gated linear attention over prompt rows (chunks of 16 on the f32 matrix cores) against a float64 token loop."""
+import pytest
+import torch
+
+from butterfly_amd import ops
+
+F64 = torch.float64
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dt,tol", [(torch.float32, 3e-6), (torch.bfloat16, 3e-5)])
+@pytest.mark.parametrize("H,D,Dv,seqs", [
+    (2, 128, 128, [(0, 17), (5, 16), (0, 1), (3, 2)]),       # chunk edges; fresh and continued sequences; one row beside prompts
+    (3, 24, 40, [(0, 33)]), (1, 96, 64, [(7, 15), (0, 48)]),   # sizes between the channel tiles
+    (1, 200, 70, [(0, 31)]), (2, 256, 128, [(1, 100)]), (2, 64, 256, [(0, 300), (0, 3)]),
+])
+def test_prompt_chunks_match_the_token_loop(dt, tol, H, D, Dv, seqs):
+    g = torch.Generator().manual_seed(D + Dv)
+    T, nslots, tau = sum(n for _, n in seqs), len(seqs) + 1, 16.0
+    rnd = lambda *s: torch.randn(*s, generator=g).to(torch.bfloat16).to(dt)            # noqa: E731
+    q, k, v, z = rnd(T, H, D), rnd(T, H, D), rnd(T, H, Dv), 2 + 2 * rnd(T, H * D)
+    z[:, ::7] -= 40.0                                       # channels that forget at once, and others that never do
+    z[:, 3::11] += 60.0
+    st = torch.randn(nslots, H, D, Dv, generator=g)
+    slots = torch.randperm(nslots, generator=g)[:len(seqs)].int()
+    cu = torch.tensor([sum(n for _, n in seqs[:i]) for i in range(len(seqs) + 1)], dtype=torch.int32)
+    pos = torch.cat([torch.arange(s, s + n) for s, n in seqs]).int()
+    a = torch.sigmoid(z.to(F64)).view(T, H, D) ** (1 / tau)
+    want, state = torch.empty(T, H, Dv, dtype=F64), st.to(F64).clone()
+    for s, (start, n) in enumerate(seqs):
+        m = state[slots[s]] if start else torch.zeros(H, D, Dv, dtype=F64)
+        for t in range(int(cu[s]), int(cu[s]) + n):
+            m = a[t][:, :, None] * m + k[t].to(F64)[:, :, None] * v[t].to(F64)[:, None]
+            want[t] = ((q[t].to(F64) * D ** -0.5)[:, None] @ m)[:, 0]
+        state[slots[s]] = m
+    d = lambda t: t.to("cuda")                             # noqa: E731
+    sd = d(st)
+    o = ops.gla_scan(d(q), d(k), d(v), d(z), sd, d(slots), d(cu), d(pos), tau, D ** -0.5)
+    # f32 sums of up to 256 channels and products of 16 decays (f32 eps 6e-8 each); hardware exp / log for bf16 inputs
+    for got, ref in ((o, want), (sd, state)):
+        assert (got.cpu().to(F64) - ref).abs().max() < tol * ref.abs().max()
