@@ -703,7 +703,8 @@ void attn_decode(const Tensor& q, const Tensor& k_cache, const Tensor& v_cache,
 // Chunked prefill over the paged cache (attention_paged.hip): q [T, Hq, D] rows grouped per
 // sequence by cu_q, positions [T] their absolute positions, tables [nseq, max_blocks].
 void attn_prefill_paged(const Tensor& q, const Tensor& k_cache, const Tensor& v_cache, const Tensor& tables,
-                        const Tensor& cu_q, const Tensor& positions, int64_t max_q, double scale, Tensor& out) {
+                        const Tensor& cu_q, const Tensor& positions, int64_t max_q, double scale, Tensor& out,
+                        const c10::optional<Tensor>& part) {
   CHECK_GPU(q); CHECK_BF16(q); CHECK_KV(k_cache, v_cache); CHECK_BF16(out);
   TORCH_CHECK(q.dim() == 3 && q.stride(2) == 1 && q.stride(1) == q.size(2), "attn_prefill_paged: q [T, Hq, D]");
   TORCH_CHECK(out.dim() == 3 && out.sizes() == q.sizes() && out.stride(2) == 1 && out.stride(1) == out.size(2),
@@ -717,12 +718,19 @@ void attn_prefill_paged(const Tensor& q, const Tensor& k_cache, const Tensor& v_
   TORCH_CHECK(tables.dim() == 2 && tables.size(0) >= nseq && tables.stride(1) == 1, "attn_prefill_paged: tables");
   TORCH_CHECK(positions.numel() >= q.size(0) && cu_q.is_contiguous() && positions.is_contiguous(),
               "attn_prefill_paged: positions / cu_q");
+  float* partp = nullptr;
+  long part_n = 0;
+  if (part.has_value()) {
+    TORCH_CHECK(part->is_cuda() && part->scalar_type() == at::kFloat && part->is_contiguous(), "attn_prefill_paged: part f32");
+    partp = part->data_ptr<float>();
+    part_n = part->numel();
+  }
   c10::DeviceGuard g(q.device());
   const int rc = bfly::launch_attn_prefill_paged(bf(q), q.stride(0), k_cache.data_ptr(), v_cache.data_ptr(),
                                                  tables.data_ptr<int>(), tables.stride(0), cu_q.data_ptr<int>(),
                                                  positions.data_ptr<int>(), nseq, (int)max_q, Hq, Hkv, D, BS,
                                                  (float)scale, bf(out), out.stride(0), cur_stream(),
-                                                 k_cache.scalar_type() == at::kFloat8_e4m3fn);
+                                                 k_cache.scalar_type() == at::kFloat8_e4m3fn, (int)q.size(0), partp, part_n);
   TORCH_CHECK(rc == 0, "attn_prefill_paged: unsupported configuration (rc=", rc, ")");
 }
 
@@ -1240,7 +1248,7 @@ TORCH_LIBRARY(bfly, m) {
   m.def("ep_ipc_stats(int ptr) -> int[]", &ep_ipc_stats);
   m.def("ep_ipc_error(int ptr) -> int", [](int64_t p) -> int64_t { return bfly::ep_ipc_error(reinterpret_cast<const void*>(p)); });
   m.def("attn_prefill_paged(Tensor q, Tensor k_cache, Tensor v_cache, Tensor tables, Tensor cu_q, "
-        "Tensor positions, int max_q, float scale, Tensor(a!) out) -> ()");
+        "Tensor positions, int max_q, float scale, Tensor(a!) out, Tensor(b!)? part=None) -> ()");
   m.def("attn_prefill(Tensor q, Tensor k, Tensor v, Tensor cu_seqlens, int max_seqlen, float scale, "
         "bool causal, Tensor(a!) out, Tensor? cu_seqlens_k=None, Tensor(b!)? lse=None) -> ()");
   m.def("attn_lse_merge(Tensor(a!) acc_o, Tensor(b!) acc_lse, Tensor o, Tensor lse) -> ()");

@@ -25,6 +25,7 @@
 #include "bfly_common.h"
 #include "bfly_kernels.h"
 #include "bfly_kv.h"
+#include "bfly_mixers.h"
 
 namespace bfly {
 
@@ -458,15 +459,38 @@ attn_prefill_paged_lds_kernel(const bf16* __restrict__ q, long q_stride, const C
 
 }  // namespace
 
+// attn_ext.hip
+bool launch_attn_window_mfma_ext(const void* q, long q_ld, const void* k_cache, const void* v_cache, const int* tables,
+                                 int max_blocks, const int* row_cu, int nseq, const int* positions, float scale,
+                                 int window, int keep_first, const float* sink, const float* out_scale, void* out, int T,
+                                 int H, int G, int D, int Dv, int block_size, float* part, long part_floats,
+                                 hipStream_t s, const AttnMod& md);
+
 int launch_attn_prefill_paged(const bf16* q, long q_stride, const void* k_cache, const void* v_cache,
                               const int* tables, int bt_stride, const int* cu_q, const int* positions,
                               int nseq, int max_q, int Hq, int Hkv, int D, int block_size, float scale,
-                              bf16* out, long o_stride, hipStream_t stream, int kv_fp8) {
+                              bf16* out, long o_stride, hipStream_t stream, int kv_fp8, int rows,
+                              float* part, long part_floats) {
   if (D != 128 || block_size != 32 || Hkv <= 0 || Hq % Hkv != 0) return -1;
   const int G = Hq / Hkv;
   if (G > 8) return -2;
   if (nseq <= 0 || max_q <= 0) return 0;
   const float scale_log2 = scale * 1.4426950408889634f;
+  // bf16 pages, at least 128 (row, head) pairs of a key / value head per chunk: the tiled kernel of the windowed attention
+  // (two row tiles per wave, pages staged once per 128 pairs and split over workgroups where chunks are few). 32 heads on
+  // 8, us of the kernels below -> tiled: 900 rows over 3000 keys 318 -> 138, 2000 over 6000 1290 -> 374, 64 over 8000
+  // 331 -> 59, three chunks of 128 over 1000 56 -> 41, four of 1000 over 2000 404 -> 296 (0.55 PFLOP/s). Shorter chunks and
+  // FP8 pages keep the kernels below.
+  if (!kv_fp8 && (long)rows * G >= 128L * nseq && (long)rows * Hq >= 512 && q_stride % 8 == 0 &&
+      reinterpret_cast<uintptr_t>(q) % 16 == 0) {
+    AttnMod md;
+    md.dv_out = D;
+    md.out_ld = o_stride;
+    md.out_vec = o_stride % 4 == 0 && reinterpret_cast<uintptr_t>(out) % 8 == 0;
+    if (launch_attn_window_mfma_ext(q, q_stride, k_cache, v_cache, tables, bt_stride, cu_q, nseq, positions, scale, 1 << 30, 0,
+                                    nullptr, nullptr, out, rows, Hq, Hkv, D, D, block_size, part, part_floats, stream, md))
+      return 0;
+  }
   // BFLY_ATTN_PAGED_LDS=0: the register kernel (every wave fetches its own pages; A/B runs)
   static const bool lds = [] {
     const char* e = getenv("BFLY_ATTN_PAGED_LDS");

@@ -76,3 +76,41 @@ def test_paged_tiles_match_dense_attention(H, G, D, Dv, window, keep, mods, seqs
     # weights rounded to bf16 (2^-9 each, together at most 2^-9 of the largest value), the output rounded once more
     err = (got.cpu().to(F64) - torch.cat(want)).abs().max()
     assert err < 2.0 ** -8 * vc.float().abs().max() + 1e-3
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("Hq,Hkv,seqs", [
+    (32, 8, [(2000, 64)]),               # few rows: one row tile per wave, pages split over workgroups
+    (32, 8, [(3001, 700)]),              # two row tiles per wave, split
+    (64, 8, [(100, 40), (0, 33)]),       # too few keys to split; a chunk without a prefix
+    (8, 8, [(31, 130), (1500, 257)]),    # no grouping
+    (32, 4, [(640, 15)]),                # fewer than 128 pairs: the 16-row kernels
+])
+def test_chunks_over_a_cached_prefix(Hq, Hkv, seqs):
+    g = torch.Generator().manual_seed(Hq + len(seqs))
+    bf = lambda *s: torch.randn(*s, generator=g).to(torch.bfloat16)                  # noqa: E731
+    dev, D, scale = "cuda", 128, 1.5 / math.sqrt(128)
+    need = [(s + n + BS - 1) // BS for s, n in seqs]
+    order = torch.randperm(sum(need), generator=g)
+    kc, vc = bf(sum(need), Hkv, BS, D), bf(sum(need), Hkv, D, BS)
+    tables = torch.zeros(len(seqs), max(need) + 3, dtype=torch.int32)
+    qs, want, at = [], [], 0
+    for s, (start, n) in enumerate(seqs):
+        pages = order[at:at + need[s]]
+        at += need[s]
+        tables[s, :need[s]] = pages.int()
+        k = kc[pages].transpose(1, 2).reshape(-1, Hkv, D)[:start + n]
+        v = vc[pages].permute(0, 3, 1, 2).reshape(-1, Hkv, D)[:start + n]
+        qs.append(bf(n, Hq, D))
+        want.append(dense(qs[-1].to(F64), k.to(F64), v.to(F64), torch.arange(start, start + n), scale, 1 << 30, 0, None, None, 0,
+                          None))
+    cu = torch.tensor([sum(n for _, n in seqs[:i]) for i in range(len(seqs) + 1)], dtype=torch.int32, device=dev)
+    pos = torch.cat([torch.arange(s, s + n) for s, n in seqs]).int().to(dev)
+    wide = torch.zeros(len(pos), Hq + 2, D, dtype=torch.bfloat16, device=dev)        # strided query and output rows
+    wide[:, :Hq] = torch.cat(qs).to(dev)
+    out = torch.zeros_like(wide)
+    ops.attn_prefill_paged(wide[:, :Hq], kc.to(dev), vc.to(dev), tables.to(dev), cu, pos, max(n for _, n in seqs), scale,
+                           out=out[:, :Hq])
+    err = (out[:, :Hq].cpu().to(F64) - torch.cat(want)).abs().max()
+    assert err < 2.0 ** -8 * vc.float().abs().max() + 1e-3
+    assert not out[:, Hq:].any()
