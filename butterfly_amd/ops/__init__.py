@@ -936,9 +936,9 @@ def moe_route_scores(x, wr, top_k: int, scoring: str = "softmax", renorm: bool =
     if not _gpu(x):
         return ref.moe_route_scores(x, wr, top_k, scoring, renorm, bias, select_bias, groups, renorm_eps, scale)
     T = x.shape[0]
-    # logits: a GEMM with f32 accumulation and f32 output (steps of a few rows: one wave per
-    # (token, expert) instead of a one-workgroup GEMM), then one wave per token picks
-    if T * wr.shape[0] <= 4096:
+    # logits: up to 64 experts one wave per token (steps of a few rows: per token and expert), beyond that a
+    # GEMM with f32 accumulation and f32 output; then one wave per token picks
+    if T * wr.shape[0] <= 4096 or wr.shape[0] <= 64:
         logits = _empty(T, wr.shape[0], dtype=torch.float32, device=x.device)
         torch.ops.bfly.router_logits(x, wr, logits)
     else:

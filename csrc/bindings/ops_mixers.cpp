@@ -285,6 +285,13 @@ void attn_window_paged(const Tensor& q, const Tensor& k_cache, const Tensor& v_c
                                                   (int)T, (int)H, (int)G, (int)D, (int)Dv, (int)bs, fold_heads, partp,
                                                   (long)part_n, cur_stream(), md))
     return;
+  if (is_f32(q) && bfly::launch_attn_window_f32(q.data_ptr<float>(), q.stride(0), k_cache.data_ptr<float>(),
+                                                v_cache.data_ptr<float>(), tables.data_ptr<int>(), (int)tables.size(1),
+                                                row_cu.data_ptr<int>(), (int)tables.size(0), positions.data_ptr<int>(),
+                                                (float)scale, (int)window, (int)keep_first, sinkp, gatep,
+                                                out.data_ptr<float>(), (int)T, (int)H, (int)G, (int)D, (int)Dv, (int)bs,
+                                                cur_stream(), md))
+    return;
   bfly::launch_attn_window_paged(q.data_ptr(), q.stride(0), k_cache.data_ptr(), v_cache.data_ptr(),
                                  tables.data_ptr<int>(), (int)tables.size(1), row_seq_t.data_ptr<int>(),
                                  (int)tables.size(0), positions.data_ptr<int>(), (float)scale, (int)window,

@@ -101,6 +101,12 @@ bool launch_attn_window_mfma(const void* q, long q_ld, const void* k_cache, cons
                              int D, int Dv, int block_size, bool fold, float* part, long part_floats, hipStream_t s,
                              const AttnMod& md = AttnMod());
 
+// The true-f32 matrix-core form of launch_attn_window_paged for prompts: false if the shape has no such form.
+bool launch_attn_window_f32(const float* q, long q_ld, const float* k_cache, const float* v_cache, const int* tables,
+                            int max_blocks, const int* row_cu, int nseq, const int* positions, float scale, int window,
+                            int keep_first, const float* sink, const float* out_scale, float* out, int T, int H, int G,
+                            int D, int Dv, int block_size, hipStream_t s, const AttnMod& md);
+
 // Gated linear attention scan over packed rows (see ops.gla_scan). Returns < 0 if D > 256.
 int launch_gla_scan(const void* q, long q_ld, const void* k, long k_ld, const void* v, long v_ld, const void* z,
                     long z_ld, float* state, const int* state_slots, const int* row_cu, int nseq,

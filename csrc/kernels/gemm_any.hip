@@ -1,9 +1,9 @@
 // Shape-generic GEMM family: any (M, N, K), bf16 or f32 operands, f32 accumulation in K order
 // (the sum of an output element never depends on M or on the other rows of the batch).
-// 64 x 64 output tile and 256 threads in both forms, operands staged through LDS with bounds
-// checks, so no shape or alignment restriction. f32 operands: 16-deep K step, a 4 x 4 register
-// block per thread on the VALU. bf16 operands: 64-deep K step staged as bf16, a 32 x 32 quadrant
-// per wave as 2 x 2 MFMA 16x16x32 tiles (tile_mac_mfma below).
+// 64 x 64 or 128 x 128 output tile and 256 threads in both forms, operands staged through LDS with bounds
+// checks, so no shape or alignment restriction. f32 operands: 32-deep K step on the f32 matrix cores
+// (tile_mac_f32). bf16 operands: 64-deep K step staged as bf16, a quadrant per wave as MFMA 16x16x32
+// tiles (tile_mac_mfma below).
 // The same tile core serves the plain projection (bias / squared-ReLU epilogues) and the two
 // grouped expert GEMMs of a score-routed MoE with clamped GLU experts: rows are grouped by
 // expert (moe_sort_kernel), the up kernel gathers token rows scaled by their routing score and
@@ -18,10 +18,9 @@ namespace bfly {
 
 namespace {
 
-constexpr int TM = 64, TN = 64, TK = 16, LDP = TM + 4;
+constexpr int TM = 64, TN = 64;
 
 template <typename T> __device__ __forceinline__ float ldf(const T* p) { return (float)*p; }
-template <typename T> __device__ __forceinline__ T cvt(float v) { return (T)v; }
 
 // epilogue activations: squared ReLU; xIELU with coefficients (a0, a1): v > 0: a0 v^2 + v / 2,
 // else a1 (exp(v) - 1 - v) + v / 2
@@ -31,65 +30,142 @@ __device__ __forceinline__ float apply_act(float v, int act, float a0, float a1)
   return v;
 }
 
-// acc[i][j] += sum_k A(row0 + ty*4 + i, k) * B(col0 + tx*4 + j, k); la(r, k) / lb(c, k) return
-// the operand element as float (0 outside the problem).
-template <typename LA, typename LB>
-__device__ __forceinline__ void tile_mac(float (&acc)[4][4], LA la, LB lb, int K, float (*As)[LDP], float (*Bs)[LDP]) {
-  const int tid = threadIdx.x;
-  const int lr = tid >> 2, lk = (tid & 3) * 4;      // staging: row lr, k lk..lk+3
-  const int ty = tid >> 4, tx = tid & 15;
-  for (int k0 = 0; k0 < K; k0 += TK) {
+// ---------------------------------------------------------------------------------------
+// f32 tile core on the f32 matrix cores (v_mfma_f32_16x16x4: f32 operands, f32 accumulation, twice the rate of scalar
+// f32 FMAs). A workgroup's (32 WT) x (32 WT) tile is 2 x 2 wave quadrants of WT x WT MFMA tiles; K goes through LDS
+// in steps of 32, double buffered (the next step's segments travel while this one multiplies, one LDS-only barrier per
+// step). A lane reads four consecutive k of a row at once: the four MFMAs of a 16-deep slice take k = e, 4 + e, 8 + e,
+// 12 + e from both operands. K is accumulated in the same order for every element, so a row's result does not
+// depend on the rest of the batch. PN weight panels share the staged X rows (an expert's gate and up rows).
+// Bound by the barrier-to-barrier chain of small problems and by the matrix cores of large ones: 1838 x 1024 x 1024
+// 182 us as scalar FMAs on 64 x 64 x 16 tiles -> see launch_gemm_any.
+// ---------------------------------------------------------------------------------------
+constexpr int FK = 32, FLD = FK + 4;      // LDS row pitch 144 B
+
+struct RowF {
+  const float* p;   // nullptr: a row of zeros
+  float s;          // the row is multiplied by s
+};
+
+__device__ __forceinline__ f32x4 load_row4(const RowF r, int k, int K) {
+  f32x4 v = {0.f, 0.f, 0.f, 0.f};
+  if (r.p == nullptr || k >= K) return v;
+  if (k + 4 <= K && (reinterpret_cast<uintptr_t>(r.p + k) & 15) == 0) {
+    v = *reinterpret_cast<const f32x4*>(r.p + k);
+  } else {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      As[lk + i][lr] = la(lr, k0 + lk + i);
-      Bs[lk + i][lr] = lb(lr, k0 + lk + i);
+    for (int j = 0; j < 4; ++j) v[j] = k + j < K ? r.p[k + j] : 0.f;
+  }
+  if (r.s != 1.f) v *= r.s;
+  return v;
+}
+
+__device__ __forceinline__ f32x4 mfma_f32(float a, float b, f32x4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+
+// Workgroup barrier that orders LDS traffic only. __syncthreads() also drains every global load
+// in flight, which here are the next K step's prefetched segments: with it each K step would wait
+// out a full memory latency.
+__device__ __forceinline__ void lds_barrier() {
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+}
+
+template <int WT, int PN>
+using FTile = float[2][(1 + PN) * 32 * WT][FLD];
+
+// acc[p][tn][tm][i] += sum_k X(m, k) W_p(n, k); wave quadrant m = 16 WT * (wave >> 1) + 16 tm + (lane & 15),
+// n = 16 WT * (wave & 1) + 16 tn + 4 * (lane >> 4) + i; rowX(r) / rowW(p, c): the tile's rows
+template <int WT, int PN, typename FX, typename FW>
+__device__ __forceinline__ void tile_mac_f32(f32x4 (&acc)[PN][WT][WT], FX rowX, FW rowW, int K, FTile<WT, PN>& S) {
+  constexpr int BT = 32 * WT;
+  const int tid = threadIdx.x, lr = tid >> 3, lk = (tid & 7) * 4;      // staging: rows lr + 32 j, k lk .. lk + 3
+  RowF rx[WT], rw[PN][WT];
+#pragma unroll
+  for (int j = 0; j < WT; ++j) {
+    rx[j] = rowX(lr + 32 * j);
+#pragma unroll
+    for (int p = 0; p < PN; ++p) rw[p][j] = rowW(p, lr + 32 * j);
+  }
+  const int wave = tid >> 6, lane = tid & 63;
+  const int wm = (wave >> 1) * 16 * WT, wn = (wave & 1) * 16 * WT, r = lane & 15, g = lane >> 4;
+  f32x4 xv[WT], wv[PN][WT];
+  auto fetch = [&](int k0) {
+#pragma unroll
+    for (int j = 0; j < WT; ++j) {
+      xv[j] = load_row4(rx[j], k0 + lk, K);
+#pragma unroll
+      for (int p = 0; p < PN; ++p) wv[p][j] = load_row4(rw[p][j], k0 + lk, K);
     }
-    __syncthreads();
+  };
+  fetch(0);
+  int buf = 0;
+  for (int k0 = 0; k0 < K; k0 += FK, buf ^= 1) {
 #pragma unroll
-    for (int kk = 0; kk < TK; ++kk) {
-      float a[4], b[4];
+    for (int j = 0; j < WT; ++j) {
+      *reinterpret_cast<f32x4*>(&S[buf][lr + 32 * j][lk]) = xv[j];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) a[i] = As[kk][ty * 4 + i];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) b[j] = Bs[kk][tx * 4 + j];
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = fmaf(a[i], b[j], acc[i][j]);
+      for (int p = 0; p < PN; ++p) *reinterpret_cast<f32x4*>(&S[buf][(1 + p) * BT + lr + 32 * j][lk]) = wv[p][j];
     }
-    __syncthreads();
+    lds_barrier();      // (the other buffer's readers passed it one step ago)
+    if (k0 + FK < K) fetch(k0 + FK);
+#pragma unroll
+    for (int ks = 0; ks < FK; ks += 16) {
+      f32x4 xf[WT], wf[PN][WT];
+#pragma unroll
+      for (int t = 0; t < WT; ++t) {
+        xf[t] = *reinterpret_cast<const f32x4*>(&S[buf][wm + 16 * t + r][ks + 4 * g]);
+#pragma unroll
+        for (int p = 0; p < PN; ++p)
+          wf[p][t] = *reinterpret_cast<const f32x4*>(&S[buf][(1 + p) * BT + wn + 16 * t + r][ks + 4 * g]);
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int p = 0; p < PN; ++p)
+#pragma unroll
+          for (int tn = 0; tn < WT; ++tn)
+#pragma unroll
+            for (int tm = 0; tm < WT; ++tm) acc[p][tn][tm] = mfma_f32(wf[p][tn][e], xf[tm][e], acc[p][tn][tm]);
+    }
   }
 }
 
-template <typename T, typename TO>
-__global__ __launch_bounds__(256) void gemm_any_kernel(const T* __restrict__ x, long ldx, const T* __restrict__ w,
-                                                       long ldw, const T* __restrict__ bias, TO* __restrict__ out,
+// f(m, n, value) over this lane's results of a tile
+template <int WT, typename F>
+__device__ __forceinline__ void tile_each(const f32x4 (&acc)[WT][WT], F f) {
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int wm = (wave >> 1) * 16 * WT, wn = (wave & 1) * 16 * WT;
+#pragma unroll
+  for (int tn = 0; tn < WT; ++tn)
+#pragma unroll
+    for (int tm = 0; tm < WT; ++tm)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) f(wm + 16 * tm + (lane & 15), wn + 16 * tn + 4 * (lane >> 4) + i, acc[tn][tm][i]);
+}
+
+template <int WT>
+__global__ __launch_bounds__(256) void gemm_any_kernel(const float* __restrict__ x, long ldx, const float* __restrict__ w,
+                                                       long ldw, const float* __restrict__ bias, float* __restrict__ out,
                                                        long ldo, int M, int N, int K, int act, float a0, float a1,
                                                        long bx, long bw, long bo) {
-  __shared__ float As[TK][LDP], Bs[TK][LDP];
-  const int row0 = blockIdx.y * TM, col0 = blockIdx.x * TN;
+  constexpr int BT = 32 * WT;
+  __shared__ __attribute__((aligned(16))) FTile<WT, 1> S;
+  const int row0 = blockIdx.y * BT, col0 = blockIdx.x * BT;
   x += blockIdx.z * bx;            // batched form: one problem per blockIdx.z (e.g. per head)
   w += blockIdx.z * bw;
   out += blockIdx.z * bo;
-  float acc[4][4] = {};
-  tile_mac(
-      acc,
-      [&](int r, int k) { return (row0 + r < M && k < K) ? ldf(x + (long)(row0 + r) * ldx + k) : 0.f; },
-      [&](int c, int k) { return (col0 + c < N && k < K) ? ldf(w + (long)(col0 + c) * ldw + k) : 0.f; }, K, As, Bs);
-  const int ty = threadIdx.x >> 4, tx = threadIdx.x & 15;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int r = row0 + ty * 4 + i;
-    if (r >= M) continue;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int c = col0 + tx * 4 + j;
-      if (c >= N) continue;
-      float v = acc[i][j];
-      if (bias) v += ldf(bias + c);
-      out[(long)r * ldo + c] = cvt<TO>(apply_act(v, act, a0, a1));
-    }
-  }
+  f32x4 acc[1][WT][WT] = {};
+  tile_mac_f32<WT, 1>(
+      acc, [&](int r) { return RowF{row0 + r < M ? x + (long)(row0 + r) * ldx : nullptr, 1.f}; },
+      [&](int, int c) { return RowF{col0 + c < N ? w + (long)(col0 + c) * ldw : nullptr, 1.f}; }, K, S);
+  tile_each<WT>(acc[0], [&](int m, int n, float v) {
+    const int r = row0 + m, c = col0 + n;
+    if (r >= M || c >= N) return;
+    if (bias) v += bias[c];
+    out[(long)r * ldo + c] = apply_act(v, act, a0, a1);
+  });
 }
 
 template <typename T>
@@ -136,91 +212,72 @@ __global__ __launch_bounds__(1024) void moe_sort_kernel(const int* __restrict__ 
   }
 }
 
-template <typename T>
-__global__ __launch_bounds__(256) void moe_glu_up_kernel(const T* __restrict__ x, long ldx,
+// `tiles` lists (expert, first row) of every 64-row tile of the grouped rows; gate and up share one K loop
+__global__ __launch_bounds__(256) void moe_glu_up_kernel(const float* __restrict__ x, long ldx,
                                                          const float* __restrict__ topk_w, int Kc,
                                                          const int* __restrict__ perm, const int* __restrict__ offsets_e,
                                                          const int* __restrict__ tiles, const int* __restrict__ ntiles,
-                                                         const T* __restrict__ gu_w, float limit, float alpha,
-                                                         float up_offset, T* __restrict__ hmid, int Hd, int F,
+                                                         const float* __restrict__ gu_w, float limit, float alpha,
+                                                         float up_offset, float* __restrict__ hmid, int Hd, int F,
                                                          int plain) {
   if ((int)blockIdx.y >= ntiles[0]) return;
-  __shared__ float As[TK][LDP], Bs[TK][LDP];
-  __shared__ int tok[TM];
-  __shared__ float wt[TM];
+  __shared__ __attribute__((aligned(16))) FTile<2, 2> S;
   const int e = tiles[2 * blockIdx.y], r0 = tiles[2 * blockIdx.y + 1];
   const int rend = offsets_e[e + 1];
-  const int col0 = blockIdx.x * TN;
-  if (threadIdx.x < TM) {
-    const int r = r0 + threadIdx.x;
-    int p = r < rend ? perm[r] : -1;
-    tok[threadIdx.x] = p < 0 ? -1 : p / Kc;
-    wt[threadIdx.x] = p < 0 ? 0.f : (topk_w ? topk_w[p] : 1.f);      // no scores: the row as it is
-  }
-  __syncthreads();
+  const int col0 = blockIdx.x * 64;
   // plain experts (no gate): F rows per expert, hmid = act(W x)
-  const T* wg = gu_w + (long)e * (plain ? 1 : 2) * F * Hd;
-  const T* wu = wg + (long)F * Hd;
-  // the expert's input is the token row times its routing score, rounded to the activation type
-  auto la = [&](int r, int k) {
-    const int t = tok[r];
-    return (t >= 0 && k < Hd) ? (float)cvt<T>(ldf(x + (long)t * ldx + k) * wt[r]) : 0.f;
+  const float* wg = gu_w + (long)e * (plain ? 1 : 2) * F * Hd;
+  // the expert's input is the token row times its routing score
+  auto rowX = [&](int r) {
+    const int p = r0 + r < rend ? perm[r0 + r] : -1;
+    return p < 0 ? RowF{nullptr, 1.f} : RowF{x + (long)(p / Kc) * ldx, topk_w ? topk_w[p] : 1.f};
   };
-  float g[4][4] = {}, u[4][4] = {};
-  tile_mac(g, la, [&](int c, int k) { return (col0 + c < F && k < Hd) ? ldf(wg + (long)(col0 + c) * Hd + k) : 0.f; },
-           Hd, As, Bs);
-  if (!plain)
-    tile_mac(u, la, [&](int c, int k) { return (col0 + c < F && k < Hd) ? ldf(wu + (long)(col0 + c) * Hd + k) : 0.f; },
-             Hd, As, Bs);
-  const int ty = threadIdx.x >> 4, tx = threadIdx.x & 15;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int r = r0 + ty * 4 + i;
-    if (r >= rend) continue;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int c = col0 + tx * 4 + j;
-      if (c >= F) continue;
-      if (plain) {
-        hmid[(long)r * F + c] = cvt<T>(apply_act(g[i][j], plain, 0.f, 0.f));
-        continue;
-      }
-      const float gg = fminf(g[i][j], limit);
-      const float uu = fminf(fmaxf(u[i][j], -limit), limit);
-      const float y = glu_gate(gg, alpha, expf(-alpha * gg)) * (uu + up_offset);
-      hmid[(long)r * F + c] = cvt<T>(y);
-    }
+  auto rowW = [&](int p, int c) { return RowF{col0 + c < F ? wg + ((long)p * F + col0 + c) * Hd : nullptr, 1.f}; };
+  if (plain) {
+    f32x4 acc[1][2][2] = {};
+    tile_mac_f32<2, 1>(acc, rowX, rowW, Hd, reinterpret_cast<FTile<2, 1>&>(S));
+    tile_each<2>(acc[0], [&](int m, int n, float v) {
+      const int r = r0 + m, c = col0 + n;
+      if (r < rend && c < F) hmid[(long)r * F + c] = apply_act(v, plain, 0.f, 0.f);
+    });
+    return;
   }
+  f32x4 acc[2][2][2] = {};
+  tile_mac_f32<2, 2>(acc, rowX, rowW, Hd, S);
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+#pragma unroll
+  for (int tn = 0; tn < 2; ++tn)
+#pragma unroll
+    for (int tm = 0; tm < 2; ++tm)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int r = r0 + (wave >> 1) * 32 + 16 * tm + (lane & 15), c = col0 + (wave & 1) * 32 + 16 * tn + 4 * (lane >> 4) + i;
+        if (r >= rend || c >= F) continue;
+        const float gg = fminf(acc[0][tn][tm][i], limit);
+        const float uu = fminf(fmaxf(acc[1][tn][tm][i], -limit), limit);
+        hmid[(long)r * F + c] = glu_gate(gg, alpha, expf(-alpha * gg)) * (uu + up_offset);
+      }
 }
 
-template <typename T>
-__global__ __launch_bounds__(256) void moe_down_kernel(const T* __restrict__ hmid, const int* __restrict__ perm,
+__global__ __launch_bounds__(256) void moe_down_kernel(const float* __restrict__ hmid, const int* __restrict__ perm,
                                                        const int* __restrict__ offsets_e,
                                                        const int* __restrict__ tiles, const int* __restrict__ ntiles,
-                                                       const T* __restrict__ down_w, float* __restrict__ y, int Hd,
+                                                       const float* __restrict__ down_w, float* __restrict__ y, int Hd,
                                                        int F) {
   if ((int)blockIdx.y >= ntiles[0]) return;
-  __shared__ float As[TK][LDP], Bs[TK][LDP];
+  __shared__ __attribute__((aligned(16))) FTile<2, 1> S;
   const int e = tiles[2 * blockIdx.y], r0 = tiles[2 * blockIdx.y + 1];
   const int rend = offsets_e[e + 1];
-  const int col0 = blockIdx.x * TN;
-  const T* wd = down_w + (long)e * Hd * F;
-  float acc[4][4] = {};
-  tile_mac(
-      acc, [&](int r, int k) { return (r0 + r < rend && k < F) ? ldf(hmid + (long)(r0 + r) * F + k) : 0.f; },
-      [&](int c, int k) { return (col0 + c < Hd && k < F) ? ldf(wd + (long)(col0 + c) * F + k) : 0.f; }, F, As, Bs);
-  const int ty = threadIdx.x >> 4, tx = threadIdx.x & 15;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int r = r0 + ty * 4 + i;
-    if (r >= rend) continue;
-    const long p = perm[r];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int c = col0 + tx * 4 + j;
-      if (c < Hd) y[p * Hd + c] = acc[i][j];
-    }
-  }
+  const int col0 = blockIdx.x * 64;
+  const float* wd = down_w + (long)e * Hd * F;
+  f32x4 acc[1][2][2] = {};
+  tile_mac_f32<2, 1>(
+      acc, [&](int r) { return RowF{r0 + r < rend ? hmid + (long)(r0 + r) * F : nullptr, 1.f}; },
+      [&](int, int c) { return RowF{col0 + c < Hd ? wd + (long)(col0 + c) * F : nullptr, 1.f}; }, F, S);
+  tile_each<2>(acc[0], [&](int m, int n, float v) {
+    const int r = r0 + m, c = col0 + n;
+    if (r < rend && c < Hd) y[(long)perm[r] * Hd + c] = v;
+  });
 }
 
 // ids (nullable, with wts): choices from E on are identity experts, whose output is the row of x itself
@@ -311,6 +368,36 @@ __global__ __launch_bounds__(256) void router_logits_kernel(const T* __restrict_
   }
   a = wave_sum(a);
   if (lane == 0) logits[(long)t * E + e] = a;
+}
+
+// Router logits of a large step: one wave per token holds the row once for eight experts at a time (the router's rows come
+// from the caches); Hd and ldx multiples of 8, aligned rows. A GEMM tile would be 1 / 8 columns wide: 8192 tokens,
+// 8 experts of width 2048 in bf16 30 us, 1838 tokens of width 1024 in f32 105 us as such; see launch_router_logits.
+template <typename T>
+__global__ __launch_bounds__(256) void router_rows_kernel(const T* __restrict__ x, long ldx, const T* __restrict__ wr,
+                                                          float* __restrict__ logits, int T_, int E, int Hd) {
+  typedef T tv __attribute__((ext_vector_type(8)));
+  const int t = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+  if (t >= T_) return;
+  const T* xr = x + (long)t * ldx;
+  for (int e0 = 0; e0 < E; e0 += 8) {
+    float a[8] = {};
+    for (int k = 8 * lane; k < Hd; k += 512) {
+      const tv xv = *reinterpret_cast<const tv*>(xr + k);
+      tv wv[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) wv[e] = *reinterpret_cast<const tv*>(wr + (long)min(e0 + e, E - 1) * Hd + k);
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) a[e] = fmaf((float)xv[j], (float)wv[e][j], a[e]);
+    }
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const float v = wave_sum(a[e]);
+      if (lane == 0 && e0 + e < E) logits[(long)t * E + e0 + e] = v;
+    }
+  }
 }
 
 // Router choice of one token per wave from its f32 logits [E]: softmax or sigmoid scores, K rounds
@@ -439,14 +526,6 @@ __device__ __forceinline__ bf16x8 load_row8(const RowRef r, int k, int K) {
 // WT = 4: 128 x 128 for large row counts). Wave quadrant: m = 16 WT * (wave >> 1) + 16 tm +
 // (lane & 15), n = 16 WT * (wave & 1) + 16 tn + 4 * (lane >> 4) + i; rowX(r) / rowW(c) give the
 // r-th X row / c-th W row of the tile.
-// Workgroup barrier that orders LDS traffic only. __syncthreads() also drains every global load
-// in flight, which here are the next K step's prefetched segments: with it each K step would wait
-// out a full memory latency.
-__device__ __forceinline__ void lds_barrier() {
-  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-  __builtin_amdgcn_s_barrier();
-}
-
 template <int WT, typename FX, typename FW>
 __device__ __forceinline__ void tile_mac_mfma(f32x4 (&acc)[WT][WT], FX rowX, FW rowW, int K, bf16 (*Xs)[MLD],
                                               bf16 (*Ws)[MLD]) {
@@ -571,19 +650,6 @@ __device__ __forceinline__ void tile_mac_mfma2(f32x4 (&acc)[WT][WT], f32x4 (&acc
     }
     lds_barrier();
   }
-}
-
-// f(m, n, value) over this lane's results of the tile
-template <int WT, typename F>
-__device__ __forceinline__ void tile_each(const f32x4 (&acc)[WT][WT], F f) {
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int wm = (wave >> 1) * 16 * WT, wn = (wave & 1) * 16 * WT;
-#pragma unroll
-  for (int tn = 0; tn < WT; ++tn)
-#pragma unroll
-    for (int tm = 0; tm < WT; ++tm)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) f(wm + 16 * tm + (lane & 15), wn + 16 * tn + 4 * (lane >> 4) + i, acc[tn][tm][i]);
 }
 
 #define BFLY_ZERO_ACC(a)                                    \
@@ -720,9 +786,12 @@ void launch_gemm_any(const void* x, long ldx, const void* w, long ldw, const voi
                                                        (bf16*)out, ldo, M, N, K, act, a0, a1, bx, bw, bo);
     return;
   }
-  if (f32)
-    gemm_any_kernel<float, float><<<grid, 256, 0, s>>>((const float*)x, ldx, (const float*)w, ldw, (const float*)bias,
-                                                       (float*)out, ldo, M, N, K, act, a0, a1, bx, bw, bo);
+  if (f32 && (long)((M + 127) / 128) * ((N + 127) / 128) * batch >= 256)
+    gemm_any_kernel<4><<<dim3((N + 127) / 128, (M + 127) / 128, batch), 256, 0, s>>>(
+        (const float*)x, ldx, (const float*)w, ldw, (const float*)bias, (float*)out, ldo, M, N, K, act, a0, a1, bx, bw, bo);
+  else if (f32)
+    gemm_any_kernel<2><<<grid, 256, 0, s>>>((const float*)x, ldx, (const float*)w, ldw, (const float*)bias, (float*)out, ldo, M,
+                                            N, K, act, a0, a1, bx, bw, bo);
   else if (out_f32)
     gemm_any_mfma_kernel<float, 2><<<grid, 256, 0, s>>>((const bf16*)x, ldx, (const bf16*)w, ldw, (const bf16*)bias,
                                                      (float*)out, ldo, M, N, K, act, a0, a1, bx, bw, bo);
@@ -744,6 +813,12 @@ void launch_router_logits(const void* x, long ldx, const void* wr, float* logits
   const size_t al = f32 ? 32 : 16;
   const bool vec = Hd % 8 == 0 && ldx % 8 == 0 && reinterpret_cast<uintptr_t>(x) % al == 0 &&
                    reinterpret_cast<uintptr_t>(wr) % al == 0;
+  if (vec && (long)T * E > 4096) {
+    const int g4 = (T + 3) / 4;
+    if (f32) router_rows_kernel<float><<<g4, 256, 0, s>>>((const float*)x, ldx, (const float*)wr, logits, T, E, Hd);
+    else router_rows_kernel<bf16><<<g4, 256, 0, s>>>((const bf16*)x, ldx, (const bf16*)wr, logits, T, E, Hd);
+    return;
+  }
 #define BFLY_RL(TT, V) router_logits_kernel<TT, V><<<grid, 256, 0, s>>>((const TT*)x, ldx, (const TT*)wr, logits, E, Hd)
   if (f32) { if (vec) BFLY_RL(float, 8); else BFLY_RL(float, 1); }
   else { if (vec) BFLY_RL(bf16, 8); else BFLY_RL(bf16, 1); }
@@ -809,7 +884,7 @@ void launch_moe_glu_up(const void* x, long ldx, const float* topk_w, int K, cons
   }
   dim3 grid((F + TN - 1) / TN, max_tiles);
   if (f32)
-    moe_glu_up_kernel<float><<<grid, 256, 0, s>>>((const float*)x, ldx, topk_w, K, perm, offsets, tiles, ntiles,
+    moe_glu_up_kernel<<<grid, 256, 0, s>>>((const float*)x, ldx, topk_w, K, perm, offsets, tiles, ntiles,
                                                   (const float*)gate_up_w, limit, alpha, up_offset, (float*)hmid, Hd, F,
                                                   plain_act);
   else
@@ -834,7 +909,7 @@ void launch_moe_down(const void* hmid, const int* perm, const int* offsets, cons
   }
   dim3 grid((Hd + TN - 1) / TN, max_tiles);
   if (f32)
-    moe_down_kernel<float><<<grid, 256, 0, s>>>((const float*)hmid, perm, offsets, tiles, ntiles,
+    moe_down_kernel<<<grid, 256, 0, s>>>((const float*)hmid, perm, offsets, tiles, ntiles,
                                                 (const float*)down_w, y, Hd, F);
   else
     moe_down_mfma_kernel<2><<<grid, 256, 0, s>>>((const bf16*)hmid, perm, offsets, tiles, ntiles, (const bf16*)down_w, y,

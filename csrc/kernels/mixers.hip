@@ -195,7 +195,211 @@ __global__ __launch_bounds__(64) void gla_out_kernel(const float* __restrict__ o
   }
 }
 
+// The same attention for prompts in true f32 (32-token pages, D = 16 DT, Dv = 16 DVT) on the f32 matrix cores: a workgroup
+// owns 64 (token, query head of key / value head blockIdx.y) rows, 16 per wave, and stages each visible page
+// once for all of them (double buffered in LDS, one barrier per page). S^T = K Q^T and O^T += V^T P as
+// 16x16x4 tiles: the scores come out with a row per lane and four keys per lane group, which is the order in which the
+// second product takes them, so nothing is rearranged or rounded between the two. Modifiers, window, kept prefix and
+// sink as in attn_window_paged_kernel, with its precise functions. The one-wave-per-row form reads every key row once
+// per query head, a row per lane: 5 prompts of 370 tokens, 8 heads on 2 of 128, 846 us; this form: see the launch rule.
+template <int DT, int DVT>
+__global__ __launch_bounds__(256) void attn_window_f32_kernel(const float* __restrict__ q, long q_ld,
+                                                              const float* __restrict__ k_cache,
+                                                              const float* __restrict__ v_cache,
+                                                              const int* __restrict__ tables, int max_blocks,
+                                                              const int* __restrict__ row_cu, int nseq,
+                                                              const int* __restrict__ positions, float scale, int window,
+                                                              int keep_first, const float* __restrict__ sink,
+                                                              const float* __restrict__ out_scale,
+                                                              float* __restrict__ out, int T, int H, int G, AttnMod md) {
+  constexpr int D = 16 * DT, Dv = 16 * DVT, BS = 32, KP = D + 4, VP = BS + 4;
+  constexpr int NKS = BS * D / 4 / 256, NVS = Dv * BS / 4 / 256;      // 16-byte segments per thread
+  static_assert(BS * D % 1024 == 0 && Dv * BS % 1024 == 0, "whole segments");
+  extern __shared__ __attribute__((aligned(16))) float f32_smem[];
+  float* Ks = f32_smem;                  // [2][BS][KP]
+  float* Vs = Ks + 2 * BS * KP;          // [2][Dv][VP]
+  __shared__ int s_range[4][2];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, qr = lane & 15, gg = lane >> 4;
+  int tile = (int)(gridDim.x - 1 - blockIdx.x);
+  const int g = blockIdx.y, R = H / G;
+  int s = 0, row0 = 0, rend = 0;
+  for (; s < nseq; ++s) {
+    const int a = row_cu[s] * R, b = row_cu[s + 1] * R;
+    const int nt = (b - a + 63) >> 6;
+    if (tile < nt) { row0 = a + 64 * tile; rend = b; break; }
+    tile -= nt;
+  }
+  if (s >= nseq) {                       // (the whole workgroup; at least one has no tile: it clears rows of no sequence)
+    const int dvo = md.ext() ? md.dv_out : Dv, first = row_cu[0], last = row_cu[nseq];
+    const long pad = tile == 0 ? (long)(first + T - last) * R * dvo : 0;
+    for (long i = tid; i < pad; i += 256) {
+      const int d = (int)(i % dvo), hd = g * R + (int)(i / dvo % R);
+      const long r = i / dvo / R, t = r < first ? r : last + (r - first);
+      if (md.ext()) attn_store_ext<false, float>(0.f, t, hd, d, dvo, out, md);
+      else out[(t * H + hd) * Dv + d] = 0.f;
+    }
+    return;
+  }
+  const int fr = row0 + 16 * wave + qr;
+  const bool rv = fr < rend;
+  const long frow = rv ? fr : row0, row = frow / R;
+  const int h = g * R + (int)(frow % R);
+  const int p = rv ? positions[row] : -1;
+  const int plo = rv ? attn_row_lo(p, window, md.chunk) : 0;
+  const float rscale = attn_row_scale(max(p, 0), scale, md);
+  const float da = md.dist_a ? md.dist_a[h] : 0.f, db = md.dist_b ? md.dist_b[h] : 0.f;
+  int pmin = rv ? p : 0x7fffffff, pmax = p;
+#pragma unroll
+  for (int x = 1; x < 16; x <<= 1) {
+    pmin = min(pmin, __shfl_xor(pmin, x, 64));
+    pmax = max(pmax, __shfl_xor(pmax, x, 64));
+  }
+  if (lane == 0) { s_range[wave][0] = pmin; s_range[wave][1] = pmax; }
+  f32x4 qf[DT];
+#pragma unroll
+  for (int c = 0; c < DT; ++c) {
+    const float* qp = q + row * q_ld + (long)h * D + 16 * c + 4 * gg;
+    qf[c] = f32x4{qp[0], qp[1], qp[2], qp[3]};
+  }
+  __syncthreads();
+  int tmin = s_range[0][0], tmax = s_range[0][1];
+#pragma unroll
+  for (int w = 1; w < 4; ++w) { tmin = min(tmin, s_range[w][0]); tmax = max(tmax, s_range[w][1]); }
+  const int wlo = pmax < 0 ? 0 : attn_row_lo(pmin, window, md.chunk);
+  const int* tab = tables + (long)s * max_blocks;
+  const int kp = (min(keep_first, tmax + 1) + BS - 1) / BS;          // pages of the kept prefix
+  const int wp0 = max(attn_row_lo(max(tmin, 0), window, md.chunk) / BS, kp);
+  const int npages = kp + max(0, tmax / BS - wp0 + 1);
+  auto page_of = [&](int i) { return i < kp ? i : wp0 + (i - kp); };
+  const bool seeded = sink != nullptr;
+  float m = seeded ? sink[h] : -1e30f, l = seeded && gg == 0 ? 1.f : 0.f;      // (per-lane partial sums)
+  f32x4 o[DVT];
+#pragma unroll
+  for (int t = 0; t < DVT; ++t) o[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+  f32x4 kreg[NKS], vreg[NVS];
+  auto gload = [&](int i0) {
+    const long blk = (long)tab[page_of(i0)] * G + g;
+    const float *Kp = k_cache + blk * BS * D, *Vp = v_cache + blk * Dv * BS;
+#pragma unroll
+    for (int i = 0; i < NKS; ++i) kreg[i] = *reinterpret_cast<const f32x4*>(Kp + 4 * (tid + 256 * i));
+#pragma unroll
+    for (int i = 0; i < NVS; ++i) vreg[i] = *reinterpret_cast<const f32x4*>(Vp + 4 * (tid + 256 * i));
+  };
+  if (npages > 0) gload(0);
+  for (int pi = 0; pi < npages; ++pi) {
+    float* Kb = Ks + (long)(pi & 1) * BS * KP;
+    float* Vb = Vs + (long)(pi & 1) * Dv * VP;
+#pragma unroll
+    for (int i = 0; i < NKS; ++i) {
+      const int idx = tid + 256 * i;
+      *reinterpret_cast<f32x4*>(Kb + idx / (D / 4) * KP + 4 * (idx % (D / 4))) = kreg[i];
+    }
+#pragma unroll
+    for (int i = 0; i < NVS; ++i) {
+      const int idx = tid + 256 * i;
+      *reinterpret_cast<f32x4*>(Vb + idx / 8 * VP + 4 * (idx & 7)) = vreg[i];
+    }
+    __syncthreads();      // the page is in LDS; every wave has left the buffer written next
+    if (pi + 1 < npages) gload(pi + 1);
+    const int j0 = page_of(pi) * BS;
+    if (j0 > pmax || (j0 + BS <= wlo && j0 >= keep_first)) continue;      // no row of this wave sees the page
+    f32x4 st[2];
+#pragma unroll
+    for (int kh = 0; kh < 2; ++kh) {
+      st[kh] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int c = 0; c < DT; ++c) {
+        const f32x4 kf = *reinterpret_cast<const f32x4*>(Kb + (16 * kh + qr) * KP + 16 * c + 4 * gg);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) st[kh] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[e], qf[c][e], st[kh], 0, 0, 0);
+      }
+    }
+    const unsigned span = (unsigned)(p - plo + 1);      // visible: p - j in [0, span) or j < kept
+    const int kept = min(keep_first, p + 1);
+    float sc[8], mx = -INFINITY;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const int j = j0 + 16 * (e >> 2) + 4 * gg + (e & 3);
+      const int ok = (int)((unsigned)(p - j) < span) | (int)(j < kept);
+      const float x = attn_score<false>(st[e >> 2][e & 3], rscale, p - j, da, db, md);
+      sc[e] = ok ? x : -INFINITY;
+      mx = fmaxf(mx, sc[e]);
+    }
+    const float mn = fmaxf(m, quad_max(mx));
+    const float corr = expf(m - mn);
+    m = mn;
+    l *= corr;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      sc[e] = expf(sc[e] - mn);      // exp(-inf) = 0 for masked keys
+      l += sc[e];
+    }
+#pragma unroll
+    for (int t = 0; t < DVT; ++t) {
+      o[t] *= corr;
+#pragma unroll
+      for (int kh = 0; kh < 2; ++kh) {
+        const f32x4 vf = *reinterpret_cast<const f32x4*>(Vb + (16 * t + qr) * VP + 16 * kh + 4 * gg);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) o[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[i], sc[4 * kh + i], o[t], 0, 0, 0);
+      }
+    }
+  }
+  l = quad_sum(l);
+  if (!rv) return;
+  const float inv = (out_scale ? out_scale[row * H + h] : 1.f) / l;
+#pragma unroll
+  for (int t = 0; t < DVT; ++t)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int d = 16 * t + 4 * gg + i;
+      if (!md.ext()) out[(row * H + h) * Dv + d] = o[t][i] * inv;
+      else if (d < md.dv_out) attn_store_ext<false, float>(o[t][i] * inv, row, h, d, md.dv_out, out, md);
+    }
+}
+
+template <int DT, int DVT>
+bool attn_window_f32_launch(const float* q, long q_ld, const float* kc, const float* vc, const int* tables, int max_blocks,
+                            const int* row_cu, int nseq, const int* positions, float scale, int window, int keep_first,
+                            const float* sink, const float* out_scale, float* out, int T, int H, int G, hipStream_t s,
+                            const AttnMod& md) {
+  constexpr size_t lds = 2 * (32 * (16 * DT + 4) + 16 * DVT * 36) * sizeof(float);
+  static bool once = false;
+  if (!once) {
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_window_f32_kernel<DT, DVT>),
+                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    once = true;
+  }
+  const dim3 grid((unsigned)(((long)T * (H / G) + 63) / 64 + nseq), G);
+  attn_window_f32_kernel<DT, DVT><<<grid, 256, lds, s>>>(q, q_ld, kc, vc, tables, max_blocks, row_cu, nseq, positions, scale,
+                                                         window, keep_first, sink, out_scale, out, T, H, G, md);
+  return true;
+}
+
 }  // namespace
+
+bool launch_attn_window_f32(const float* q, long q_ld, const float* kc, const float* vc, const int* tables, int max_blocks,
+                            const int* row_cu, int nseq, const int* positions, float scale, int window, int keep_first,
+                            const float* sink, const float* out_scale, float* out, int T, int H, int G, int D, int Dv,
+                            int block_size, hipStream_t s, const AttnMod& md) {
+  // prompts: from 32 (row, head) pairs per sequence and key / value head on, at head sizes of whole segments; decoded rows
+  // and other shapes keep the one-wave-per-row form
+  if ((reinterpret_cast<uintptr_t>(kc) | reinterpret_cast<uintptr_t>(vc)) & 15) return false;
+  if (block_size != 32 || md.maps != 1 || md.pool > 0 || md.sigmoid || T <= 0 || (long)T * (H / G) < 32L * nseq) return false;
+#define BFLY_AF(DT, DVT)                                                                                                \
+  return attn_window_f32_launch<DT, DVT>(q, q_ld, kc, vc, tables, max_blocks, row_cu, nseq, positions, scale, window,   \
+                                         keep_first, sink, out_scale, out, T, H, G, s, md)
+  if (D == 32 && Dv == 32) BFLY_AF(2, 2);
+  if (D == 64 && Dv == 64) BFLY_AF(4, 4);
+  if (D == 96 && Dv == 96) BFLY_AF(6, 6);
+  if (D == 128 && Dv == 128) BFLY_AF(8, 8);
+  if (D == 128 && Dv == 256) BFLY_AF(8, 16);
+  if (D == 192 && Dv == 192) BFLY_AF(12, 12);
+  if (D == 256 && Dv == 192) BFLY_AF(16, 12);
+  if (D == 256 && Dv == 256) BFLY_AF(16, 16);
+#undef BFLY_AF
+  return false;
+}
 
 void launch_rope_partial_kv(void* q, long q_ld, void* k, long k_ld, const void* v, long v_ld, const int* positions,
                             const float* inv_freq, int nrot, const int* slots, void* k_cache, void* v_cache,

@@ -34,6 +34,7 @@ def dense(q, k, v, pos, scale, window, keep, sink, slopes, chunk, qt):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("H,G,D,Dv,window,keep,mods,seqs", [
     (16, 4, 128, 128, 1 << 30, 0, "", [(0, 700), (0, 1501)]),         # two row tiles per wave; a ragged last tile
     (16, 4, 128, 128, 300, 5, "sink", [(0, 2400), (0, 33)]),          # window edges and a kept prefix, pages skipped
@@ -43,7 +44,7 @@ def dense(q, k, v, pos, scale, window, keep, sink, slopes, chunk, qt):
     (32, 2, 128, 128, 512, 0, "slope", [(0, 1030), (5, 1000)]),       # sixteen query heads per key head, two tiles per wave
     (16, 4, 128, 128, 40, 3, "sink", [(700, 1), (31, 1), (32, 1), (0, 1)]),   # decoded rows: the 16-row form
 ])
-def test_paged_tiles_match_dense_attention(H, G, D, Dv, window, keep, mods, seqs):
+def test_paged_tiles_match_dense_attention(dt, H, G, D, Dv, window, keep, mods, seqs):
     g = torch.Generator().manual_seed(H + D + window % 1000)
     bf = lambda *s: torch.randn(*s, generator=g).to(torch.bfloat16)                  # noqa: E731
     dev, scale = "cuda", 2.0 / math.sqrt(D)
@@ -70,12 +71,13 @@ def test_paged_tiles_match_dense_attention(H, G, D, Dv, window, keep, mods, seqs
                           slopes, chunk, qt))
     cu = torch.tensor([sum(n for _, n in seqs[:i]) for i in range(len(seqs) + 1)], dtype=torch.int32, device=dev)
     pos = torch.cat([torch.arange(s, s + n) for s, n in seqs]).int().to(dev)
-    got = ops.attn_window_paged(torch.cat(qs).to(dev), kc.to(dev), vc.to(dev), tables.to(dev), cu, pos, scale, window, keep,
+    got = ops.attn_window_paged(torch.cat(qs).to(dev, dt), kc.to(dev, dt), vc.to(dev, dt), tables.to(dev), cu, pos, scale, window, keep,
                                 None if sink is None else sink.to(dev), chunk=chunk, q_temp=qt,
                                 dist_bias=None if slopes is None else (slopes.to(dev), None))
-    # weights rounded to bf16 (2^-9 each, together at most 2^-9 of the largest value), the output rounded once more
+    # bf16: weights rounded to bf16 (2^-9 each, together at most 2^-9 of the largest value), the output rounded once more;
+    # f32: scores of up to 20 with a few eps (6e-8) of their size, which is the relative error of a weight
     err = (got.cpu().to(F64) - torch.cat(want)).abs().max()
-    assert err < 2.0 ** -8 * vc.float().abs().max() + 1e-3
+    assert err < (2.0 ** -8 if dt == torch.bfloat16 else 1e-5) * vc.float().abs().max() + (1e-3 if dt == torch.bfloat16 else 0)
 
 
 @pytest.mark.gpu

@@ -1,0 +1,55 @@
+"""True-f32 products on the f32 matrix cores: plain GEMM, router logits and grouped experts against float64."""
+import pytest
+import torch
+
+from butterfly_amd import ops
+
+F64 = torch.float64
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(1, 1, 1), (63, 65, 31), (64, 64, 32), (65, 130, 33), (3, 300, 257), (129, 127, 100),
+                                   (2100, 2050, 70)])      # the last one: the 128 x 128 tile
+@pytest.mark.parametrize("pad", [0, 3])
+def test_gemm_matches_float64(M, N, K, pad):
+    g = torch.Generator().manual_seed(M * N + K)
+    x, w, b = (torch.randn(*s, generator=g) for s in ((M, K + pad), (N, K + pad), (N,)))
+    xd, wd = x.cuda()[:, :K], w.cuda()[:, :K].contiguous()
+    got = ops.linear_act(xd, wd, bias=b.cuda(), act="relu2").cpu().to(F64)
+    acc = x[:, :K].to(F64) @ w[:, :K].to(F64).T + b.to(F64)
+    want = torch.relu(acc) ** 2
+    # K products of N(0, 1) values summed in f32: K eps / 2 of sqrt(K) at most, doubled by the square
+    tol = 2 * K * 6e-8 * max(1.0, K ** 0.5) * (acc.abs().max() + 1)
+    assert (got - want).abs().max() < tol
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("T,E,W", [(600, 8, 256), (1025, 5, 512), (700, 64, 264), (41, 100, 64), (515, 9, 130)])
+def test_router_choice(dt, T, E, W):
+    g = torch.Generator().manual_seed(T + E)
+    x, wr = torch.randn(T, W, generator=g).to(dt), (torch.randn(E, W, generator=g) * W ** -0.5).to(dt)
+    ids, w = ops.moe_route_scores(x.cuda(), wr.cuda(), 2, scoring="sigmoid", renorm=False)
+    s = torch.sigmoid(x.to(F64) @ wr.to(F64).T)
+    got = s.gather(1, ids.cpu().long())
+    top = s.topk(2, -1).values
+    assert (got - top).abs().max() < 1e-5 and (w.cpu().to(F64) - got).abs().max() < 1e-5      # (ties within rounding may swap)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T,E,Hd,F,plain", [(70, 3, 64, 96, False), (130, 4, 100, 65, False), (200, 2, 96, 64, True)])
+def test_experts(T, E, Hd, F, plain):
+    g = torch.Generator().manual_seed(T)
+    x, ids = torch.randn(T, Hd, generator=g), torch.rand(T, E, generator=g).topk(2, -1).indices
+    w = torch.rand(T, 2, generator=g)
+    gu, dn = torch.randn(E, F if plain else 2 * F, Hd, generator=g) * Hd ** -0.5, torch.randn(E, Hd, F, generator=g) * F ** -0.5
+    got = ops.moe_glu_ffn(x.cuda(), ids.int().cuda(), w.cuda(), gu.cuda(), dn.cuda(), 7.0, 1.702, 1.0, True,
+                          "relu2" if plain else None).cpu().to(F64)
+    want = torch.zeros(T, Hd, dtype=F64)
+    for e in range(E):
+        t, j = (ids == e).nonzero(as_tuple=True)
+        h = (x[t].to(F64) * w[t, j].to(F64)[:, None]) @ gu[e].to(F64).T
+        c = torch.clamp(h[:, :F], max=7.0)
+        a = torch.relu(h) ** 2 if plain else c * torch.sigmoid(1.702 * c) * (torch.clamp(h[:, F:], -7.0, 7.0) + 1)
+        want.index_add_(0, t, a @ dn[e].to(F64).T)
+    assert (got - want).abs().max() < 1e-5 * (1 + want.abs().max())
