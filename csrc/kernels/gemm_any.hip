@@ -18,8 +18,6 @@ namespace bfly {
 
 namespace {
 
-constexpr int TM = 64, TN = 64;
-
 template <typename T> __device__ __forceinline__ float ldf(const T* p) { return (float)*p; }
 
 // epilogue activations: squared ReLU; xIELU with coefficients (a0, a1): v > 0: a0 v^2 + v / 2,
@@ -38,7 +36,7 @@ __device__ __forceinline__ float apply_act(float v, int act, float a0, float a1)
 // 12 + e from both operands. K is accumulated in the same order for every element, so a row's result does not
 // depend on the rest of the batch. PN weight panels share the staged X rows (an expert's gate and up rows).
 // Bound by the barrier-to-barrier chain of small problems and by the matrix cores of large ones: 1838 x 1024 x 1024
-// 182 us as scalar FMAs on 64 x 64 x 16 tiles -> see launch_gemm_any.
+// 182 us as scalar FMAs on 64 x 64 x 16 tiles -> 69 us; 1838 x 4224 x 1024 466 -> 160 us (0.1 PFLOP/s).
 // ---------------------------------------------------------------------------------------
 constexpr int FK = 32, FLD = FK + 4;      // LDS row pitch 144 B
 
@@ -47,16 +45,15 @@ struct RowF {
   float s;          // the row is multiplied by s
 };
 
-__device__ __forceinline__ f32x4 load_row4(const RowF r, int k, int K) {
+__device__ __forceinline__ f32x4 load_row4(const float* p, int k, int K) {
   f32x4 v = {0.f, 0.f, 0.f, 0.f};
-  if (r.p == nullptr || k >= K) return v;
-  if (k + 4 <= K && (reinterpret_cast<uintptr_t>(r.p + k) & 15) == 0) {
-    v = *reinterpret_cast<const f32x4*>(r.p + k);
+  if (p == nullptr || k >= K) return v;
+  if (k + 4 <= K && (reinterpret_cast<uintptr_t>(p + k) & 15) == 0) {
+    v = *reinterpret_cast<const f32x4*>(p + k);
   } else {
 #pragma unroll
-    for (int j = 0; j < 4; ++j) v[j] = k + j < K ? r.p[k + j] : 0.f;
+    for (int j = 0; j < 4; ++j) v[j] = k + j < K ? p[k + j] : 0.f;
   }
-  if (r.s != 1.f) v *= r.s;
   return v;
 }
 
@@ -65,7 +62,7 @@ __device__ __forceinline__ f32x4 mfma_f32(float a, float b, f32x4 c) {
 }
 
 // Workgroup barrier that orders LDS traffic only. __syncthreads() also drains every global load
-// in flight, which here are the next K step's prefetched segments: with it each K step would wait
+// in flight, which here are the next K steps' prefetched segments: with it each K step would wait
 // out a full memory latency.
 __device__ __forceinline__ void lds_barrier() {
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
@@ -76,58 +73,79 @@ template <int WT, int PN>
 using FTile = float[2][(1 + PN) * 32 * WT][FLD];
 
 // acc[p][tn][tm][i] += sum_k X(m, k) W_p(n, k); wave quadrant m = 16 WT * (wave >> 1) + 16 tm + (lane & 15),
-// n = 16 WT * (wave & 1) + 16 tn + 4 * (lane >> 4) + i; rowX(r) / rowW(p, c): the tile's rows
-template <int WT, int PN, typename FX, typename FW>
+// n = 16 WT * (wave & 1) + 16 tn + 4 * (lane >> 4) + i; rowX(r) / rowW(p, c): the tile's rows (the first of each
+// exists). VEC (16-byte aligned rows, whole K steps): loads without branches, rows outside the problem read the
+// tile's first row (their results are never stored); a branch around a load makes the compiler wait for it. SC: X
+// rows are scaled on their way into LDS. Two K steps travel while one multiplies.
+template <int WT, int PN, bool VEC, bool SC, typename FX, typename FW>
 __device__ __forceinline__ void tile_mac_f32(f32x4 (&acc)[PN][WT][WT], FX rowX, FW rowW, int K, FTile<WT, PN>& S) {
-  constexpr int BT = 32 * WT;
+  constexpr int BT = 32 * WT, PF = WT == 2 ? 2 : 1;
   const int tid = threadIdx.x, lr = tid >> 3, lk = (tid & 7) * 4;      // staging: rows lr + 32 j, k lk .. lk + 3
-  RowF rx[WT], rw[PN][WT];
+  const float *px[WT], *pw[PN][WT];
+  float sx[WT];
 #pragma unroll
   for (int j = 0; j < WT; ++j) {
-    rx[j] = rowX(lr + 32 * j);
+    const RowF r = rowX(lr + 32 * j);
+    px[j] = VEC && !r.p ? rowX(0).p : r.p;
+    sx[j] = r.s;
 #pragma unroll
-    for (int p = 0; p < PN; ++p) rw[p][j] = rowW(p, lr + 32 * j);
+    for (int p = 0; p < PN; ++p) {
+      const float* w = rowW(p, lr + 32 * j).p;
+      pw[p][j] = VEC && !w ? rowW(p, 0).p : w;
+    }
   }
   const int wave = tid >> 6, lane = tid & 63;
   const int wm = (wave >> 1) * 16 * WT, wn = (wave & 1) * 16 * WT, r = lane & 15, g = lane >> 4;
-  f32x4 xv[WT], wv[PN][WT];
-  auto fetch = [&](int k0) {
+  f32x4 xv[PF][WT], wv[PF][PN][WT];
+  auto load = [&](const float* p, int k) {
+    if constexpr (VEC) return *reinterpret_cast<const f32x4*>(p + k);
+    else return load_row4(p, k, K);
+  };
+  auto fetch = [&](int k0, f32x4 (&x)[WT], f32x4 (&w)[PN][WT]) {
 #pragma unroll
     for (int j = 0; j < WT; ++j) {
-      xv[j] = load_row4(rx[j], k0 + lk, K);
+      x[j] = load(px[j], k0 + lk);
 #pragma unroll
-      for (int p = 0; p < PN; ++p) wv[p][j] = load_row4(rw[p][j], k0 + lk, K);
+      for (int p = 0; p < PN; ++p) w[p][j] = load(pw[p][j], k0 + lk);
     }
   };
-  fetch(0);
+#pragma unroll
+  for (int u = 0; u < PF; ++u)
+    if (u * FK < K) fetch(u * FK, xv[u], wv[u]);
   int buf = 0;
-  for (int k0 = 0; k0 < K; k0 += FK, buf ^= 1) {
+  for (int k0 = 0; k0 < K; k0 += PF * FK) {
 #pragma unroll
-    for (int j = 0; j < WT; ++j) {
-      *reinterpret_cast<f32x4*>(&S[buf][lr + 32 * j][lk]) = xv[j];
+    for (int u = 0; u < PF; ++u) {
+      const int k = k0 + u * FK;
+      if (k >= K) break;
 #pragma unroll
-      for (int p = 0; p < PN; ++p) *reinterpret_cast<f32x4*>(&S[buf][(1 + p) * BT + lr + 32 * j][lk]) = wv[p][j];
-    }
-    lds_barrier();      // (the other buffer's readers passed it one step ago)
-    if (k0 + FK < K) fetch(k0 + FK);
+      for (int j = 0; j < WT; ++j) {
+        *reinterpret_cast<f32x4*>(&S[buf][lr + 32 * j][lk]) = SC ? xv[u][j] * sx[j] : xv[u][j];
 #pragma unroll
-    for (int ks = 0; ks < FK; ks += 16) {
-      f32x4 xf[WT], wf[PN][WT];
-#pragma unroll
-      for (int t = 0; t < WT; ++t) {
-        xf[t] = *reinterpret_cast<const f32x4*>(&S[buf][wm + 16 * t + r][ks + 4 * g]);
-#pragma unroll
-        for (int p = 0; p < PN; ++p)
-          wf[p][t] = *reinterpret_cast<const f32x4*>(&S[buf][(1 + p) * BT + wn + 16 * t + r][ks + 4 * g]);
+        for (int p = 0; p < PN; ++p) *reinterpret_cast<f32x4*>(&S[buf][(1 + p) * BT + lr + 32 * j][lk]) = wv[u][p][j];
       }
+      lds_barrier();      // (the other buffer's readers passed it one step ago)
+      if (k + PF * FK < K) fetch(k + PF * FK, xv[u], wv[u]);
 #pragma unroll
-      for (int e = 0; e < 4; ++e)
+      for (int ks = 0; ks < FK; ks += 16) {
+        f32x4 xf[WT], wf[PN][WT];
 #pragma unroll
-        for (int p = 0; p < PN; ++p)
+        for (int t = 0; t < WT; ++t) {
+          xf[t] = *reinterpret_cast<const f32x4*>(&S[buf][wm + 16 * t + r][ks + 4 * g]);
 #pragma unroll
-          for (int tn = 0; tn < WT; ++tn)
+          for (int p = 0; p < PN; ++p)
+            wf[p][t] = *reinterpret_cast<const f32x4*>(&S[buf][(1 + p) * BT + wn + 16 * t + r][ks + 4 * g]);
+        }
 #pragma unroll
-            for (int tm = 0; tm < WT; ++tm) acc[p][tn][tm] = mfma_f32(wf[p][tn][e], xf[tm][e], acc[p][tn][tm]);
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+          for (int p = 0; p < PN; ++p)
+#pragma unroll
+            for (int tn = 0; tn < WT; ++tn)
+#pragma unroll
+              for (int tm = 0; tm < WT; ++tm) acc[p][tn][tm] = mfma_f32(wf[p][tn][e], xf[tm][e], acc[p][tn][tm]);
+      }
+      buf ^= 1;
     }
   }
 }
@@ -145,7 +163,7 @@ __device__ __forceinline__ void tile_each(const f32x4 (&acc)[WT][WT], F f) {
       for (int i = 0; i < 4; ++i) f(wm + 16 * tm + (lane & 15), wn + 16 * tn + 4 * (lane >> 4) + i, acc[tn][tm][i]);
 }
 
-template <int WT>
+template <int WT, bool VEC>
 __global__ __launch_bounds__(256) void gemm_any_kernel(const float* __restrict__ x, long ldx, const float* __restrict__ w,
                                                        long ldw, const float* __restrict__ bias, float* __restrict__ out,
                                                        long ldo, int M, int N, int K, int act, float a0, float a1,
@@ -157,7 +175,7 @@ __global__ __launch_bounds__(256) void gemm_any_kernel(const float* __restrict__
   w += blockIdx.z * bw;
   out += blockIdx.z * bo;
   f32x4 acc[1][WT][WT] = {};
-  tile_mac_f32<WT, 1>(
+  tile_mac_f32<WT, 1, VEC, false>(
       acc, [&](int r) { return RowF{row0 + r < M ? x + (long)(row0 + r) * ldx : nullptr, 1.f}; },
       [&](int, int c) { return RowF{col0 + c < N ? w + (long)(col0 + c) * ldw : nullptr, 1.f}; }, K, S);
   tile_each<WT>(acc[0], [&](int m, int n, float v) {
@@ -213,6 +231,7 @@ __global__ __launch_bounds__(1024) void moe_sort_kernel(const int* __restrict__ 
 }
 
 // `tiles` lists (expert, first row) of every 64-row tile of the grouped rows; gate and up share one K loop
+template <bool VEC>
 __global__ __launch_bounds__(256) void moe_glu_up_kernel(const float* __restrict__ x, long ldx,
                                                          const float* __restrict__ topk_w, int Kc,
                                                          const int* __restrict__ perm, const int* __restrict__ offsets_e,
@@ -235,7 +254,7 @@ __global__ __launch_bounds__(256) void moe_glu_up_kernel(const float* __restrict
   auto rowW = [&](int p, int c) { return RowF{col0 + c < F ? wg + ((long)p * F + col0 + c) * Hd : nullptr, 1.f}; };
   if (plain) {
     f32x4 acc[1][2][2] = {};
-    tile_mac_f32<2, 1>(acc, rowX, rowW, Hd, reinterpret_cast<FTile<2, 1>&>(S));
+    tile_mac_f32<2, 1, VEC, true>(acc, rowX, rowW, Hd, reinterpret_cast<FTile<2, 1>&>(S));
     tile_each<2>(acc[0], [&](int m, int n, float v) {
       const int r = r0 + m, c = col0 + n;
       if (r < rend && c < F) hmid[(long)r * F + c] = apply_act(v, plain, 0.f, 0.f);
@@ -243,7 +262,7 @@ __global__ __launch_bounds__(256) void moe_glu_up_kernel(const float* __restrict
     return;
   }
   f32x4 acc[2][2][2] = {};
-  tile_mac_f32<2, 2>(acc, rowX, rowW, Hd, S);
+  tile_mac_f32<2, 2, VEC, true>(acc, rowX, rowW, Hd, S);
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
 #pragma unroll
   for (int tn = 0; tn < 2; ++tn)
@@ -259,6 +278,7 @@ __global__ __launch_bounds__(256) void moe_glu_up_kernel(const float* __restrict
       }
 }
 
+template <bool VEC>
 __global__ __launch_bounds__(256) void moe_down_kernel(const float* __restrict__ hmid, const int* __restrict__ perm,
                                                        const int* __restrict__ offsets_e,
                                                        const int* __restrict__ tiles, const int* __restrict__ ntiles,
@@ -271,7 +291,7 @@ __global__ __launch_bounds__(256) void moe_down_kernel(const float* __restrict__
   const int col0 = blockIdx.x * 64;
   const float* wd = down_w + (long)e * Hd * F;
   f32x4 acc[1][2][2] = {};
-  tile_mac_f32<2, 1>(
+  tile_mac_f32<2, 1, VEC, false>(
       acc, [&](int r) { return RowF{r0 + r < rend ? hmid + (long)(r0 + r) * F : nullptr, 1.f}; },
       [&](int, int c) { return RowF{col0 + c < Hd ? wd + (long)(col0 + c) * F : nullptr, 1.f}; }, F, S);
   tile_each<2>(acc[0], [&](int m, int n, float v) {
@@ -372,7 +392,7 @@ __global__ __launch_bounds__(256) void router_logits_kernel(const T* __restrict_
 
 // Router logits of a large step: one wave per token holds the row once for eight experts at a time (the router's rows come
 // from the caches); Hd and ldx multiples of 8, aligned rows. A GEMM tile would be 1 / 8 columns wide: 8192 tokens,
-// 8 experts of width 2048 in bf16 30 us, 1838 tokens of width 1024 in f32 105 us as such; see launch_router_logits.
+// 8 experts of width 2048 in bf16 took 30 us as such, 1838 tokens of width 1024 in f32 105 us; now 16 and 7 us.
 template <typename T>
 __global__ __launch_bounds__(256) void router_rows_kernel(const T* __restrict__ x, long ldx, const T* __restrict__ wr,
                                                           float* __restrict__ logits, int T_, int E, int Hd) {
@@ -502,178 +522,127 @@ struct RowRef {
   float s;         // the row is multiplied by s and rounded to bf16 (1: as stored)
 };
 
-__device__ __forceinline__ bf16x8 load_row8(const RowRef r, int k, int K) {
+__device__ __forceinline__ bf16x8 load_row8(const bf16* p, int k, int K) {
   bf16x8 v;
-  if (r.p == nullptr || k >= K) {
+  if (p == nullptr || k >= K) {
 #pragma unroll
     for (int j = 0; j < 8; ++j) v[j] = (bf16)0.f;
     return v;
   }
-  if (k + 8 <= K && (reinterpret_cast<uintptr_t>(r.p + k) & 15) == 0) {
-    v = *reinterpret_cast<const bf16x8*>(r.p + k);
+  if (k + 8 <= K && (reinterpret_cast<uintptr_t>(p + k) & 15) == 0) {
+    v = *reinterpret_cast<const bf16x8*>(p + k);
   } else {
 #pragma unroll
-    for (int j = 0; j < 8; ++j) v[j] = (k + j < K) ? r.p[k + j] : (bf16)0.f;
-  }
-  if (r.s != 1.f) {
-#pragma unroll
-    for (int j = 0; j < 8; ++j) v[j] = (bf16)((float)v[j] * r.s);
+    for (int j = 0; j < 8; ++j) v[j] = (k + j < K) ? p[k + j] : (bf16)0.f;
   }
   return v;
 }
 
-// acc[tn][tm][i] += sum_k X(m, k) W(n, k) over a (32 WT) x (32 WT) workgroup tile (WT = 2: 64 x 64,
-// WT = 4: 128 x 128 for large row counts). Wave quadrant: m = 16 WT * (wave >> 1) + 16 tm +
-// (lane & 15), n = 16 WT * (wave & 1) + 16 tn + 4 * (lane >> 4) + i; rowX(r) / rowW(c) give the
-// r-th X row / c-th W row of the tile.
-template <int WT, typename FX, typename FW>
-__device__ __forceinline__ void tile_mac_mfma(f32x4 (&acc)[WT][WT], FX rowX, FW rowW, int K, bf16 (*Xs)[MLD],
-                                              bf16 (*Ws)[MLD]) {
-  constexpr int NS = WT / 2;                           // staged rows per thread and operand
+template <int WT, int PN>
+using BTile = bf16[2][(1 + PN) * 32 * WT][MLD];
+
+// acc[p][tn][tm][i] += sum_k X(m, k) W_p(n, k) over a (32 WT) x (32 WT) workgroup tile (WT = 2: 64 x 64, WT = 4: 128 x 128
+// for large row counts) and PN weight panels that share the staged X rows (an expert's gate and up rows). Wave
+// quadrant: m = 16 WT * (wave >> 1) + 16 tm + (lane & 15), n = 16 WT * (wave & 1) + 16 tn + 4 * (lane >> 4) + i;
+// rowX(r) / rowW(p, c) give the r-th X row / c-th row of panel p. VEC, SC and the two K steps in flight as in
+// tile_mac_f32 (a scaled row is rounded to bf16). Small groups are bound by the latency of their weight stream:
+// with branches around the loads and one step in flight, 16 tokens through 8 experts of 2048 (width 2048, 134 MB of gate
+// and up rows) took 63 us in the gate / up product and 33 in the down product, now 41 and 24.
+template <int WT, int PN, bool VEC, bool SC, typename FX, typename FW>
+__device__ __forceinline__ void tile_mac_mfma(f32x4 (&acc)[PN][WT][WT], FX rowX, FW rowW, int K, BTile<WT, PN>& S) {
+  constexpr int NS = WT / 2, BT = 32 * WT, PF = WT == 2 ? 2 : 1;      // staged rows per thread and operand; steps in flight
   const int tid = threadIdx.x;
   const int lr = tid >> 2, lk = (tid & 3) * 16;        // staging: rows lr + 64 j, k lk .. lk + 15
-  RowRef rx[NS], rw[NS];
+  const bf16 *px[NS], *pw[PN][NS];
+  float sx[NS];
 #pragma unroll
   for (int j = 0; j < NS; ++j) {
-    rx[j] = rowX(lr + 64 * j);
-    rw[j] = rowW(lr + 64 * j);
+    const RowRef r = rowX(lr + 64 * j);
+    px[j] = VEC && !r.p ? rowX(0).p : r.p;
+    sx[j] = r.s;
+#pragma unroll
+    for (int p = 0; p < PN; ++p) {
+      const bf16* w = rowW(p, lr + 64 * j).p;
+      pw[p][j] = VEC && !w ? rowW(p, 0).p : w;
+    }
   }
   const int wave = tid >> 6, lane = tid & 63;
   const int wm = (wave >> 1) * 16 * WT, wn = (wave & 1) * 16 * WT, r = lane & 15, g = lane >> 4;
-  bf16x8 xv[NS][2], wv[NS][2];
-#pragma unroll
-  for (int j = 0; j < NS; ++j)
-#pragma unroll
-    for (int e = 0; e < 2; ++e) {
-      xv[j][e] = load_row8(rx[j], lk + 8 * e, K);
-      wv[j][e] = load_row8(rw[j], lk + 8 * e, K);
-    }
-  for (int k0 = 0; k0 < K; k0 += MK) {
+  bf16x8 xv[PF][NS][2], wv[PF][PN][NS][2];
+  auto load = [&](const bf16* p, int k) {
+    if constexpr (VEC) return *reinterpret_cast<const bf16x8*>(p + k);
+    else return load_row8(p, k, K);
+  };
+  auto fetch = [&](int k0, bf16x8 (&x)[NS][2], bf16x8 (&w)[PN][NS][2]) {
 #pragma unroll
     for (int j = 0; j < NS; ++j)
 #pragma unroll
       for (int e = 0; e < 2; ++e) {
-        *reinterpret_cast<bf16x8*>(&Xs[lr + 64 * j][lk + 8 * e]) = xv[j][e];
-        *reinterpret_cast<bf16x8*>(&Ws[lr + 64 * j][lk + 8 * e]) = wv[j][e];
+        x[j][e] = load(px[j], k0 + lk + 8 * e);
+#pragma unroll
+        for (int p = 0; p < PN; ++p) w[p][j][e] = load(pw[p][j], k0 + lk + 8 * e);
       }
-    lds_barrier();
-    if (k0 + MK < K) {          // the next K step's segments travel while this one multiplies
+  };
+#pragma unroll
+  for (int u = 0; u < PF; ++u)
+    if (u * MK < K) fetch(u * MK, xv[u], wv[u]);
+  int buf = 0;
+  for (int k0 = 0; k0 < K; k0 += PF * MK) {
+#pragma unroll
+    for (int u = 0; u < PF; ++u) {
+      const int k = k0 + u * MK;
+      if (k >= K) break;
 #pragma unroll
       for (int j = 0; j < NS; ++j)
 #pragma unroll
         for (int e = 0; e < 2; ++e) {
-          xv[j][e] = load_row8(rx[j], k0 + MK + lk + 8 * e, K);
-          wv[j][e] = load_row8(rw[j], k0 + MK + lk + 8 * e, K);
+          bf16x8 v = xv[u][j][e];
+          if constexpr (SC)
+            if (sx[j] != 1.f)
+#pragma unroll
+              for (int i = 0; i < 8; ++i) v[i] = (bf16)((float)v[i] * sx[j]);
+          *reinterpret_cast<bf16x8*>(&S[buf][lr + 64 * j][lk + 8 * e]) = v;
+#pragma unroll
+          for (int p = 0; p < PN; ++p) *reinterpret_cast<bf16x8*>(&S[buf][(1 + p) * BT + lr + 64 * j][lk + 8 * e]) = wv[u][p][j][e];
         }
-    }
+      lds_barrier();      // (the other buffer's readers passed it one step ago)
+      if (k + PF * MK < K) fetch(k + PF * MK, xv[u], wv[u]);
 #pragma unroll
-    for (int ks = 0; ks < MK; ks += 32) {
-      bf16x8 xf[WT], wf[WT];
+      for (int ks = 0; ks < MK; ks += 32) {
+        bf16x8 xf[WT];
 #pragma unroll
-      for (int t = 0; t < WT; ++t) {
-        xf[t] = *reinterpret_cast<const bf16x8*>(&Xs[wm + 16 * t + r][ks + 8 * g]);
-        wf[t] = *reinterpret_cast<const bf16x8*>(&Ws[wn + 16 * t + r][ks + 8 * g]);
+        for (int t = 0; t < WT; ++t) xf[t] = *reinterpret_cast<const bf16x8*>(&S[buf][wm + 16 * t + r][ks + 8 * g]);
+#pragma unroll
+        for (int p = 0; p < PN; ++p)
+#pragma unroll
+          for (int tn = 0; tn < WT; ++tn) {
+            const bf16x8 wf = *reinterpret_cast<const bf16x8*>(&S[buf][(1 + p) * BT + wn + 16 * tn + r][ks + 8 * g]);
+#pragma unroll
+            for (int tm = 0; tm < WT; ++tm) acc[p][tn][tm] = mfma16(wf, xf[tm], acc[p][tn][tm]);
+          }
       }
-#pragma unroll
-      for (int tn = 0; tn < WT; ++tn)
-#pragma unroll
-        for (int tm = 0; tm < WT; ++tm) acc[tn][tm] = mfma16(wf[tn], xf[tm], acc[tn][tm]);
+      buf ^= 1;
     }
-    lds_barrier();
   }
 }
 
-// tile_mac_mfma for two weight panels that share the X tile (an expert's gate and up rows): one K
-// loop, X staged once, both panels' segments in flight together.
-template <int WT, typename FX, typename FW, typename FV>
-__device__ __forceinline__ void tile_mac_mfma2(f32x4 (&acc)[WT][WT], f32x4 (&acc2)[WT][WT], FX rowX, FW rowW, FV rowV,
-                                               int K, bf16 (*Xs)[MLD], bf16 (*Ws)[MLD], bf16 (*Vs)[MLD]) {
-  constexpr int NS = WT / 2;
-  const int tid = threadIdx.x;
-  const int lr = tid >> 2, lk = (tid & 3) * 16;
-  RowRef rx[NS], rw[NS], rv[NS];
-#pragma unroll
-  for (int j = 0; j < NS; ++j) {
-    rx[j] = rowX(lr + 64 * j);
-    rw[j] = rowW(lr + 64 * j);
-    rv[j] = rowV(lr + 64 * j);
-  }
-  const int wave = tid >> 6, lane = tid & 63;
-  const int wm = (wave >> 1) * 16 * WT, wn = (wave & 1) * 16 * WT, r = lane & 15, g = lane >> 4;
-  bf16x8 xv[NS][2], wv[NS][2], vv[NS][2];
-#pragma unroll
-  for (int j = 0; j < NS; ++j)
-#pragma unroll
-    for (int e = 0; e < 2; ++e) {
-      xv[j][e] = load_row8(rx[j], lk + 8 * e, K);
-      wv[j][e] = load_row8(rw[j], lk + 8 * e, K);
-      vv[j][e] = load_row8(rv[j], lk + 8 * e, K);
-    }
-  for (int k0 = 0; k0 < K; k0 += MK) {
-#pragma unroll
-    for (int j = 0; j < NS; ++j)
-#pragma unroll
-      for (int e = 0; e < 2; ++e) {
-        *reinterpret_cast<bf16x8*>(&Xs[lr + 64 * j][lk + 8 * e]) = xv[j][e];
-        *reinterpret_cast<bf16x8*>(&Ws[lr + 64 * j][lk + 8 * e]) = wv[j][e];
-        *reinterpret_cast<bf16x8*>(&Vs[lr + 64 * j][lk + 8 * e]) = vv[j][e];
-      }
-    lds_barrier();
-    if (k0 + MK < K) {
-#pragma unroll
-      for (int j = 0; j < NS; ++j)
-#pragma unroll
-        for (int e = 0; e < 2; ++e) {
-          xv[j][e] = load_row8(rx[j], k0 + MK + lk + 8 * e, K);
-          wv[j][e] = load_row8(rw[j], k0 + MK + lk + 8 * e, K);
-          vv[j][e] = load_row8(rv[j], k0 + MK + lk + 8 * e, K);
-        }
-    }
-#pragma unroll
-    for (int ks = 0; ks < MK; ks += 32) {
-      bf16x8 xf[WT], wf[WT];
-#pragma unroll
-      for (int t = 0; t < WT; ++t) {
-        xf[t] = *reinterpret_cast<const bf16x8*>(&Xs[wm + 16 * t + r][ks + 8 * g]);
-        wf[t] = *reinterpret_cast<const bf16x8*>(&Ws[wn + 16 * t + r][ks + 8 * g]);
-      }
-#pragma unroll
-      for (int tn = 0; tn < WT; ++tn)
-#pragma unroll
-        for (int tm = 0; tm < WT; ++tm) acc[tn][tm] = mfma16(wf[tn], xf[tm], acc[tn][tm]);
-#pragma unroll
-      for (int t = 0; t < WT; ++t) wf[t] = *reinterpret_cast<const bf16x8*>(&Vs[wn + 16 * t + r][ks + 8 * g]);
-#pragma unroll
-      for (int tn = 0; tn < WT; ++tn)
-#pragma unroll
-        for (int tm = 0; tm < WT; ++tm) acc2[tn][tm] = mfma16(wf[tn], xf[tm], acc2[tn][tm]);
-    }
-    lds_barrier();
-  }
-}
-
-#define BFLY_ZERO_ACC(a)                                    \
-  f32x4 a[WT][WT];                                          \
-  _Pragma("unroll") for (int _i = 0; _i < WT; ++_i)         \
-      _Pragma("unroll") for (int _j = 0; _j < WT; ++_j) a[_i][_j] = f32x4{0.f, 0.f, 0.f, 0.f}
-
-template <typename TO, int WT>
+template <typename TO, int WT, bool VEC>
 __global__ __launch_bounds__(256) void gemm_any_mfma_kernel(const bf16* __restrict__ x, long ldx,
                                                             const bf16* __restrict__ w, long ldw,
                                                             const bf16* __restrict__ bias, TO* __restrict__ out,
                                                             long ldo, int M, int N, int K, int act, float a0, float a1,
                                                             long bx, long bw, long bo) {
   constexpr int BT = 32 * WT;
-  __shared__ __attribute__((aligned(16))) bf16 Xs[BT][MLD], Ws[BT][MLD];
+  __shared__ __attribute__((aligned(16))) BTile<WT, 1> S;
   const int row0 = blockIdx.y * BT, col0 = blockIdx.x * BT;
   x += blockIdx.z * bx;
   w += blockIdx.z * bw;
   out += blockIdx.z * bo;
-  BFLY_ZERO_ACC(acc);
-  tile_mac_mfma<WT>(
+  f32x4 acc[1][WT][WT] = {};
+  tile_mac_mfma<WT, 1, VEC, false>(
       acc, [&](int r) { return RowRef{row0 + r < M ? x + (long)(row0 + r) * ldx : nullptr, 1.f}; },
-      [&](int c) { return RowRef{col0 + c < N ? w + (long)(col0 + c) * ldw : nullptr, 1.f}; }, K, Xs, Ws);
-  tile_each<WT>(acc, [&](int m, int n, float v) {
+      [&](int, int c) { return RowRef{col0 + c < N ? w + (long)(col0 + c) * ldw : nullptr, 1.f}; }, K, S);
+  tile_each<WT>(acc[0], [&](int m, int n, float v) {
     const int r = row0 + m, c = col0 + n;
     if (r >= M || c >= N) return;
     if (bias) v += (float)bias[c];
@@ -682,7 +651,7 @@ __global__ __launch_bounds__(256) void gemm_any_mfma_kernel(const bf16* __restri
 }
 
 // `tiles` lists (expert, first row) of every (32 WT)-row tile of the grouped rows
-template <int WT>
+template <int WT, bool VEC>
 __global__ __launch_bounds__(256) void moe_glu_up_mfma_kernel(const bf16* __restrict__ x, long ldx,
                                                               const float* __restrict__ topk_w, int Kc,
                                                               const int* __restrict__ perm,
@@ -697,35 +666,36 @@ __global__ __launch_bounds__(256) void moe_glu_up_mfma_kernel(const bf16* __rest
   // small groups (decode): gate and up share one K loop, so both panels' weight segments are in
   // flight together; large groups (128-row tiles): two passes, which keep registers and LDS for
   // a second resident workgroup
-  __shared__ __attribute__((aligned(16))) bf16 Xs[BT][MLD], Ws[BT][MLD], Vs[WT == 2 ? BT : 1][MLD];
+  constexpr int PN = WT == 2 ? 2 : 1;
+  __shared__ __attribute__((aligned(16))) BTile<WT, PN> S;
   const int e = tiles[2 * blockIdx.y], r0 = tiles[2 * blockIdx.y + 1];
   const int rend = offsets_e[e + 1];
   const int col0 = blockIdx.x * BT;
   // plain experts (no gate): F rows per expert, hmid = act(W x)
   const bf16* wg = gu_w + (long)e * (plain ? 1 : 2) * F * Hd;
-  const bf16* wu = wg + (long)F * Hd;
   // the expert's input row: the token row times its routing score, rounded to bf16
   auto rowX = [&](int r) {
     const int p = r0 + r < rend ? perm[r0 + r] : -1;
     return p < 0 ? RowRef{nullptr, 1.f} : RowRef{x + (long)(p / Kc) * ldx, topk_w ? topk_w[p] : 1.f};
   };
-  BFLY_ZERO_ACC(g);
-  BFLY_ZERO_ACC(u);
-  auto rowG = [&](int c) { return RowRef{col0 + c < F ? wg + (long)(col0 + c) * Hd : nullptr, 1.f}; };
-  auto rowU = [&](int c) { return RowRef{col0 + c < F ? wu + (long)(col0 + c) * Hd : nullptr, 1.f}; };
+  auto rowW = [&](int p, int c) { return RowRef{col0 + c < F ? wg + ((long)p * F + col0 + c) * Hd : nullptr, 1.f}; };
   if (plain) {
-    tile_mac_mfma<WT>(g, rowX, rowG, Hd, Xs, Ws);
-    tile_each<WT>(g, [&](int m, int n, float v) {
+    f32x4 acc[1][WT][WT] = {};
+    tile_mac_mfma<WT, 1, VEC, true>(acc, rowX, rowW, Hd, reinterpret_cast<BTile<WT, 1>&>(S));
+    tile_each<WT>(acc[0], [&](int m, int n, float v) {
       const int r = r0 + m, c = col0 + n;
       if (r < rend && c < F) hmid[(long)r * F + c] = (bf16)apply_act(v, plain, 0.f, 0.f);
     });
     return;
   }
-  if constexpr (WT == 2) {
-    tile_mac_mfma2<WT>(g, u, rowX, rowG, rowU, Hd, Xs, Ws, Vs);
+  f32x4 acc[2][WT][WT] = {};
+  if constexpr (PN == 2) {
+    tile_mac_mfma<WT, 2, VEC, true>(acc, rowX, rowW, Hd, S);
   } else {
-    tile_mac_mfma<WT>(g, rowX, rowG, Hd, Xs, Ws);
-    tile_mac_mfma<WT>(u, rowX, rowU, Hd, Xs, Ws);
+    tile_mac_mfma<WT, 1, VEC, true>(reinterpret_cast<f32x4(&)[1][WT][WT]>(acc[0]), rowX, rowW, Hd, S);
+    __syncthreads();      // (the second pass starts over in the first buffer)
+    tile_mac_mfma<WT, 1, VEC, true>(reinterpret_cast<f32x4(&)[1][WT][WT]>(acc[1]), rowX,
+                                    [&](int, int c) { return rowW(1, c); }, Hd, S);
   }
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int wm = (wave >> 1) * 16 * WT, wn = (wave & 1) * 16 * WT;
@@ -737,13 +707,13 @@ __global__ __launch_bounds__(256) void moe_glu_up_mfma_kernel(const bf16* __rest
       for (int i = 0; i < 4; ++i) {
         const int r = r0 + wm + 16 * tm + (lane & 15), c = col0 + wn + 16 * tn + 4 * (lane >> 4) + i;
         if (r >= rend || c >= F) continue;
-        const float gg = fminf(g[tn][tm][i], limit);
-        const float uu = fminf(fmaxf(u[tn][tm][i], -limit), limit);
+        const float gg = fminf(acc[0][tn][tm][i], limit);
+        const float uu = fminf(fmaxf(acc[1][tn][tm][i], -limit), limit);
         hmid[(long)r * F + c] = (bf16)(glu_gate(gg, alpha, expf(-alpha * gg)) * (uu + up_offset));
       }
 }
 
-template <int WT>
+template <int WT, bool VEC>
 __global__ __launch_bounds__(256) void moe_down_mfma_kernel(const bf16* __restrict__ hmid, const int* __restrict__ perm,
                                                             const int* __restrict__ offsets_e,
                                                             const int* __restrict__ tiles,
@@ -752,20 +722,23 @@ __global__ __launch_bounds__(256) void moe_down_mfma_kernel(const bf16* __restri
                                                             int Hd, int F) {
   if ((int)blockIdx.y >= ntiles[0]) return;
   constexpr int BT = 32 * WT;
-  __shared__ __attribute__((aligned(16))) bf16 Xs[BT][MLD], Ws[BT][MLD];
+  __shared__ __attribute__((aligned(16))) BTile<WT, 1> S;
   const int e = tiles[2 * blockIdx.y], r0 = tiles[2 * blockIdx.y + 1];
   const int rend = offsets_e[e + 1];
   const int col0 = blockIdx.x * BT;
   const bf16* wd = down_w + (long)e * Hd * F;
-  BFLY_ZERO_ACC(acc);
-  tile_mac_mfma<WT>(
+  f32x4 acc[1][WT][WT] = {};
+  tile_mac_mfma<WT, 1, VEC, false>(
       acc, [&](int r) { return RowRef{r0 + r < rend ? hmid + (long)(r0 + r) * F : nullptr, 1.f}; },
-      [&](int c) { return RowRef{col0 + c < Hd ? wd + (long)(col0 + c) * F : nullptr, 1.f}; }, F, Xs, Ws);
-  tile_each<WT>(acc, [&](int m, int n, float v) {
+      [&](int, int c) { return RowRef{col0 + c < Hd ? wd + (long)(col0 + c) * F : nullptr, 1.f}; }, F, S);
+  tile_each<WT>(acc[0], [&](int m, int n, float v) {
     const int r = r0 + m, c = col0 + n;
     if (r < rend && c < Hd) y[(long)perm[r] * Hd + c] = v;
   });
 }
+
+// rows of `ld` elements of es bytes that allow 16-byte accesses everywhere
+inline bool rows16(const void* p, long ld, int es) { return ld * es % 16 == 0 && reinterpret_cast<uintptr_t>(p) % 16 == 0; }
 
 inline int ew_blocks(long n) { return (int)std::min<long>(4096, std::max<long>(1, (n + 255) / 256)); }
 
@@ -775,29 +748,26 @@ void launch_gemm_any(const void* x, long ldx, const void* w, long ldw, const voi
                      int M, int N, int K, int act, float a0, float a1, bool f32, bool out_f32, hipStream_t s,
                      int batch, long bx, long bw, long bo) {
   if (M <= 0 || N <= 0 || batch <= 0) return;
-  dim3 grid((N + TN - 1) / TN, (M + TM - 1) / TM, batch);
-  if (!f32 && M >= 512 && N >= 128) {        // large row counts: the 128 x 128 workgroup tile
-    dim3 g2((N + 127) / 128, (M + 127) / 128, batch);
-    if (out_f32)
-      gemm_any_mfma_kernel<float, 4><<<g2, 256, 0, s>>>((const bf16*)x, ldx, (const bf16*)w, ldw, (const bf16*)bias,
-                                                        (float*)out, ldo, M, N, K, act, a0, a1, bx, bw, bo);
-    else
-      gemm_any_mfma_kernel<bf16, 4><<<g2, 256, 0, s>>>((const bf16*)x, ldx, (const bf16*)w, ldw, (const bf16*)bias,
-                                                       (bf16*)out, ldo, M, N, K, act, a0, a1, bx, bw, bo);
-    return;
+  const int es = f32 ? 4 : 2;
+  const bool vec = K % (f32 ? FK : MK) == 0 && rows16(x, ldx, es) && rows16(w, ldw, es) && bx * es % 16 == 0 && bw * es % 16 == 0;
+#define BFLY_GA(KERNEL, TI, TO, ...)                                                                                     \
+  {                                                                                                                      \
+    if (vec) KERNEL<__VA_ARGS__, true><<<grid, 256, 0, s>>>((const TI*)x, ldx, (const TI*)w, ldw, (const TI*)bias, (TO*)out, ldo, \
+                                                            M, N, K, act, a0, a1, bx, bw, bo);                           \
+    else KERNEL<__VA_ARGS__, false><<<grid, 256, 0, s>>>((const TI*)x, ldx, (const TI*)w, ldw, (const TI*)bias, (TO*)out, ldo,   \
+                                                         M, N, K, act, a0, a1, bx, bw, bo);                              \
   }
-  if (f32 && (long)((M + 127) / 128) * ((N + 127) / 128) * batch >= 256)
-    gemm_any_kernel<4><<<dim3((N + 127) / 128, (M + 127) / 128, batch), 256, 0, s>>>(
-        (const float*)x, ldx, (const float*)w, ldw, (const float*)bias, (float*)out, ldo, M, N, K, act, a0, a1, bx, bw, bo);
-  else if (f32)
-    gemm_any_kernel<2><<<grid, 256, 0, s>>>((const float*)x, ldx, (const float*)w, ldw, (const float*)bias, (float*)out, ldo, M,
-                                            N, K, act, a0, a1, bx, bw, bo);
-  else if (out_f32)
-    gemm_any_mfma_kernel<float, 2><<<grid, 256, 0, s>>>((const bf16*)x, ldx, (const bf16*)w, ldw, (const bf16*)bias,
-                                                     (float*)out, ldo, M, N, K, act, a0, a1, bx, bw, bo);
-  else
-    gemm_any_mfma_kernel<bf16, 2><<<grid, 256, 0, s>>>((const bf16*)x, ldx, (const bf16*)w, ldw, (const bf16*)bias,
-                                                    (bf16*)out, ldo, M, N, K, act, a0, a1, bx, bw, bo);
+  // large row counts, and f32 problems that fill the chip with them: the 128 x 128 workgroup tile
+  const bool large = f32 ? (long)((M + 127) / 128) * ((N + 127) / 128) * batch >= 256 : M >= 512 && N >= 128;
+  const int bt = large ? 128 : 64;
+  const dim3 grid((N + bt - 1) / bt, (M + bt - 1) / bt, batch);
+  if (f32 && large) BFLY_GA(gemm_any_kernel, float, float, 4)
+  else if (f32) BFLY_GA(gemm_any_kernel, float, float, 2)
+  else if (out_f32 && large) BFLY_GA(gemm_any_mfma_kernel, bf16, float, float, 4)
+  else if (out_f32) BFLY_GA(gemm_any_mfma_kernel, bf16, float, float, 2)
+  else if (large) BFLY_GA(gemm_any_mfma_kernel, bf16, bf16, bf16, 4)
+  else BFLY_GA(gemm_any_mfma_kernel, bf16, bf16, bf16, 2)
+#undef BFLY_GA
 }
 
 void launch_act(void* x, long n, int act, float a0, float a1, bool f32, hipStream_t s) {
@@ -847,15 +817,15 @@ bool moe_big_ok(const void* x, long ldx, const void* gate_up_w, const void* down
          (long)TKp * F * 2 < lim;
 }
 
-// 256-row tiles on the LDS-DMA kernel from an average of 256 grouped rows per expert, and from 128 where the width gives
-// a group at least 8 column tiles; below that the 64-row tiles have more workgroups. Whole op, 8 experts, us before
-// (64 / 128-row tiles) -> now: width 2048, GLU of 2048, 16384 rows 1343 -> 483 (0.93 PFLOP/s in the two GEMMs), 2048
-// rows 273 -> 114, 1024 rows 119 -> 104; width 4096, 4096: 16384 rows 4774 -> 1481; width 1024, plain 1536: 16384 rows
-// 358 -> 174, 2048 rows 102 -> 77, but 1024 rows 58 -> 69. Shapes outside moe_big_ok: 128-row tiles from 256 rows
-// (bf16 only), else 64.
+// 256-row tiles on the LDS-DMA kernel from an average of 128 (width 4096 on), 160 (2048 on) or 384 grouped rows per
+// expert: below that the 64-row tiles have more workgroups. Whole op, 8 experts, two choices, us of 64 / 128-row tiles ->
+// 256-row tiles: width 2048, GLU of 2048, 8192 tokens 1343 -> 458 (0.95 PFLOP/s in the two GEMMs), 1024 tokens 144 -> 112,
+// 768 tokens 117 -> 107, but 512 tokens 98 -> 102; width 4096, 4096: 8192 tokens 4774 -> 1397, 512 tokens 352 -> 295;
+// width 1024, plain 1536: 2048 tokens 103 -> 82, but 1024 tokens 66 -> 77. Shapes outside moe_big_ok: 128-row tiles
+// from 512 rows (bf16 only), else 64.
 int moe_tile_rows(int TKp, int E, bool f32, bool big, int Hd) {
-  if (big && TKp >= (Hd >= 2048 ? 128 : 256) * E) return 256;
-  return (!f32 && TKp >= 256 * E) ? 128 : 64;
+  if (big && TKp >= (Hd >= 4096 ? 128 : Hd >= 2048 ? 160 : 384) * E) return 256;
+  return (!f32 && TKp >= 512 * E) ? 128 : 64;
 }
 
 void launch_moe_sort(const int* ids, int TKp, int E, int* perm, int* offsets, int* tiles, int* ntiles, int tile_rows,
@@ -875,22 +845,19 @@ void launch_moe_glu_up(const void* x, long ldx, const float* topk_w, int K, cons
                    (bf16*)hmid, F, ex, s);
     return;
   }
-  if (tile_rows == 128) {
-    dim3 g2((F + 127) / 128, max_tiles);
-    moe_glu_up_mfma_kernel<4><<<g2, 256, 0, s>>>((const bf16*)x, ldx, topk_w, K, perm, offsets, tiles, ntiles,
-                                                 (const bf16*)gate_up_w, limit, alpha, up_offset, (bf16*)hmid, Hd, F,
-                                                 plain_act);
-    return;
+  const int es = f32 ? 4 : 2;
+  const bool vec = Hd % (f32 ? FK : MK) == 0 && rows16(x, ldx, es) && rows16(gate_up_w, Hd, es);
+  const dim3 grid((F + tile_rows - 1) / tile_rows, max_tiles);
+#define BFLY_MU(KERNEL, TI)                                                                                               \
+  KERNEL<<<grid, 256, 0, s>>>((const TI*)x, ldx, topk_w, K, perm, offsets, tiles, ntiles, (const TI*)gate_up_w, limit, alpha, \
+                              up_offset, (TI*)hmid, Hd, F, plain_act)
+  if (f32) { if (vec) BFLY_MU(moe_glu_up_kernel<true>, float); else BFLY_MU(moe_glu_up_kernel<false>, float); }
+  else if (tile_rows == 128) {
+    if (vec) BFLY_MU((moe_glu_up_mfma_kernel<4, true>), bf16); else BFLY_MU((moe_glu_up_mfma_kernel<4, false>), bf16);
+  } else {
+    if (vec) BFLY_MU((moe_glu_up_mfma_kernel<2, true>), bf16); else BFLY_MU((moe_glu_up_mfma_kernel<2, false>), bf16);
   }
-  dim3 grid((F + TN - 1) / TN, max_tiles);
-  if (f32)
-    moe_glu_up_kernel<<<grid, 256, 0, s>>>((const float*)x, ldx, topk_w, K, perm, offsets, tiles, ntiles,
-                                                  (const float*)gate_up_w, limit, alpha, up_offset, (float*)hmid, Hd, F,
-                                                  plain_act);
-  else
-    moe_glu_up_mfma_kernel<2><<<grid, 256, 0, s>>>((const bf16*)x, ldx, topk_w, K, perm, offsets, tiles, ntiles,
-                                                (const bf16*)gate_up_w, limit, alpha, up_offset, (bf16*)hmid, Hd, F,
-                                                plain_act);
+#undef BFLY_MU
 }
 
 void launch_moe_down(const void* hmid, const int* perm, const int* offsets, const int* tiles, const int* ntiles,
@@ -901,19 +868,18 @@ void launch_moe_down(const void* hmid, const int* perm, const int* offsets, cons
     launch_moe_big(true, (const bf16*)hmid, F, (const bf16*)down_w, Hd, F, max_tiles, ntiles, nullptr, Hd, ex, s);
     return;
   }
-  if (tile_rows == 128) {
-    dim3 g2((Hd + 127) / 128, max_tiles);
-    moe_down_mfma_kernel<4><<<g2, 256, 0, s>>>((const bf16*)hmid, perm, offsets, tiles, ntiles, (const bf16*)down_w, y,
-                                               Hd, F);
-    return;
+  const int es = f32 ? 4 : 2;
+  const bool vec = F % (f32 ? FK : MK) == 0 && rows16(hmid, F, es) && rows16(down_w, F, es);
+  const dim3 grid((Hd + tile_rows - 1) / tile_rows, max_tiles);
+#define BFLY_MD(KERNEL, TI) \
+  KERNEL<<<grid, 256, 0, s>>>((const TI*)hmid, perm, offsets, tiles, ntiles, (const TI*)down_w, y, Hd, F)
+  if (f32) { if (vec) BFLY_MD(moe_down_kernel<true>, float); else BFLY_MD(moe_down_kernel<false>, float); }
+  else if (tile_rows == 128) {
+    if (vec) BFLY_MD((moe_down_mfma_kernel<4, true>), bf16); else BFLY_MD((moe_down_mfma_kernel<4, false>), bf16);
+  } else {
+    if (vec) BFLY_MD((moe_down_mfma_kernel<2, true>), bf16); else BFLY_MD((moe_down_mfma_kernel<2, false>), bf16);
   }
-  dim3 grid((Hd + TN - 1) / TN, max_tiles);
-  if (f32)
-    moe_down_kernel<<<grid, 256, 0, s>>>((const float*)hmid, perm, offsets, tiles, ntiles,
-                                                (const float*)down_w, y, Hd, F);
-  else
-    moe_down_mfma_kernel<2><<<grid, 256, 0, s>>>((const bf16*)hmid, perm, offsets, tiles, ntiles, (const bf16*)down_w, y,
-                                              Hd, F);
+#undef BFLY_MD
 }
 
 void launch_moe_sum(const float* y, const float* wts, int K, void* out, int T, int Hd, bool f32, hipStream_t s,

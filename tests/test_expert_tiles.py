@@ -31,9 +31,10 @@ def reference(x, ids, w, gu, dn, limit, alpha, offset, scaled, plain):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("counts,Hd,F,plain,scaled,limit", [
-    ([256, 257, 255, 1], 256, 128, False, True, 7.0),        # tile edges; the smallest panel; one row in a tile
+    ([512, 769, 255, 1], 256, 128, False, True, 7.0),        # tile edges; the smallest panel; one row in a tile
     ([700, 0, 600], 512, 384, False, False, math.inf),       # an expert without rows; weighted outputs
-    ([513, 256, 40, 300], 768, 256, True, False, math.inf),  # plain experts
+    ([200, 220], 2048, 128, False, True, 7.0),               # a wide model's smaller groups
+    ([513, 756, 40, 300], 768, 256, True, False, math.inf),  # plain experts
     ([600, 500], 256, 192, False, True, 7.0),                # F not a multiple of 128: the 128-row tiles
     ([300, 290], 320, 128, True, True, math.inf),            # Hd not a multiple of 256; scores on plain experts
     ([60, 50, 70], 256, 256, False, True, 7.0),              # small groups: the 64-row tiles
