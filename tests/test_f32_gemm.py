@@ -53,3 +53,18 @@ def test_experts(T, E, Hd, F, plain):
         a = torch.relu(h) ** 2 if plain else c * torch.sigmoid(1.702 * c) * (torch.clamp(h[:, F:], -7.0, 7.0) + 1)
         want.index_add_(0, t, a @ dn[e].to(F64).T)
     assert (got - want).abs().max() < 1e-5 * (1 + want.abs().max())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(257, 1152, 64 * 4), (300, 1408, 128), (1000, 1152, 1024), (512, 8320, 256), (513, 1024 + 128, 64 * 9)])
+@pytest.mark.parametrize("bias", [False, True])
+def test_prefill_tile_with_half_a_column_tile(M, N, K, bias):
+    g = torch.Generator().manual_seed(M + N)
+    x, w = torch.randn(M, K, generator=g).bfloat16(), torch.randn(N, K, generator=g).bfloat16()
+    b = torch.randn(N, generator=g).bfloat16() if bias else None
+    out = torch.full((M, N + 8), 7.0, dtype=torch.bfloat16, device="cuda")
+    ops.linear(x.cuda(), w.cuda(), bias=None if b is None else b.cuda(), out=out[:, :N])
+    want = x.to(F64) @ w.to(F64).T + (0 if b is None else b.to(F64))
+    # one rounding to bf16 (2^-9) of f32 sums
+    assert ((out[:, :N].cpu().to(F64) - want).abs() < 2.0 ** -8 * want.abs() + 1e-3 * K ** 0.5).all()
+    assert (out[:, N:] == 7.0).all()
