@@ -24,7 +24,7 @@ _LIB_PATH = Path(__file__).resolve().parent.parent / "_C.so"
 _loaded = False
 _load_error: str | None = None
 
-EPILOGUES = {"none": 0, "bias": 1, "silu": 2, "glu": 4}
+EPILOGUES = {"none": 0, "bias": 1, "silu": 2, "glu": 4, "relu2": 5}
 DECODE_PART_TOKENS = 0   # 0 = pick the context split per call (attn_decode_part_tokens)
 
 
@@ -477,7 +477,7 @@ def pack_w256(w: torch.Tensor) -> torch.Tensor:
 
 def linear(x, w, bias=None, epilogue: str = "none", out=None, defer: bool = False, packed=None):
     """y = x @ w.T (+ bias) with optional fused SwiGLU epilogue ('silu': w rows gate/up
-    interleaved in 16-row groups, output width w.shape[0] // 2) or fused clamped GLU with biases
+    interleaved in 16-row groups, output width w.shape[0] // 2), squared ReLU ('relu2') or fused clamped GLU with biases
     ('glu': the same row layout, `bias` = glu_bias_block(interleaved biases, limit, alpha,
     up_offset): g sigmoid(alpha g) (u + up_offset), g = min(gate, limit), u = clamp(up,
     +-limit)). `defer=True` (no bias /
@@ -773,12 +773,14 @@ def linear_act(x, w, bias=None, act: str = "none", out_dtype=None, act_params=No
     """y = act(x w^T + bias) for any shape, bf16 or f32 (`out_dtype` f32: keep the f32
     accumulator). act: "none" | "relu2" | "xielu" (act_params = its two coefficients (a_pos,
     a_neg): z > 0: a_pos z^2 + z / 2, else a_neg (exp(z) - 1 - z) + z / 2). bf16 shapes the MFMA
-    GEMMs tile go to them (the activation as a pass over the result); every other shape, and f32,
-    runs the generic tile kernel."""
+    GEMMs tile go to them (relu2 without a bias in their epilogue, other activations as a pass over the
+    result); every other shape, and f32, runs the generic tile kernel."""
     if not _gpu(x):
         return ref.linear_act(x, w, bias, act, out_dtype, act_params)
     a0, a1 = (float(act_params[0]), float(act_params[1])) if act == "xielu" else (0.0, 0.0)
     if _mfma_gemm_ok(x, w, out_dtype, bias):
+        if act == "relu2" and bias is None:      # in the GEMM's epilogue, on the f32 sums
+            return linear(x, w, epilogue="relu2")
         y = linear(x, w, bias=bias)
         if act != "none":
             torch.ops.bfly.act_(y, ACTS[act], a0, a1)

@@ -339,6 +339,8 @@ def linear(x, w, bias=None, epilogue="none", out=None):
     if epilogue == "silu":
         g, u = split_gate_up(y, SILU_INTERLEAVE)
         y = F.silu(g) * u
+    if epilogue == "relu2":
+        y = torch.relu(y) ** 2
     y = y.to(x.dtype)
     if out is None:
         return y

@@ -17,7 +17,7 @@ typedef __bf16 bf16;
 //   `bias` then points at the epilogue's block: N bias values (bf16, interleaved like the rows)
 //   followed by the three f32 values {limit, alpha, offset} (N is even, so they are 4-byte
 //   aligned): the parameters travel with the bias, the kernels' signatures stay as they are.
-enum GemmEpilogue { EPI_NONE = 0, EPI_BIAS = 1, EPI_SILU = 2, EPI_SILU_GATE = 3, EPI_GLU = 4 };
+enum GemmEpilogue { EPI_NONE = 0, EPI_BIAS = 1, EPI_SILU = 2, EPI_SILU_GATE = 3, EPI_GLU = 4, EPI_RELU2 = 5 };
 constexpr int kGluBlockTail = 6;      // bf16 slots of the three f32 parameters after the N bias values
 // epilogues that pair gate / up 16-row groups and write N / 2 columns
 inline bool epi_halves(int epi) { return epi == EPI_SILU || epi == EPI_GLU; }

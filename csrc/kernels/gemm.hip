@@ -5,6 +5,7 @@
 // Epilogues (fused, so the activation never makes an extra HBM round trip):
 //   EPI_NONE  : Y = acc
 //   EPI_BIAS  : Y = acc + bias[n]
+//   EPI_RELU2 : Y = max(acc, 0)^2
 //   EPI_SILU  : W's rows are gate/up interleaved in 16-row groups (g0 u0 g1 u1 ...);
 //               Y[M, N/2] = silu(gate) * up  (the SwiGLU FFN's first half in one kernel)
 //   EPI_GLU   : the same row layout; Y[M, N/2] = g sigmoid(alpha g) (u + offset) with g = min(gate
@@ -123,6 +124,7 @@ __global__ void gemm_splitk_reduce_kernel(const float* __restrict__ part, int SK
       float acc = 0.f;
       for (int s = 0; s < SK; ++s) acc += part[s * slab + i];
       if (epi == EPI_BIAS) acc += bf2f(bias[f]);
+      if (epi == EPI_RELU2) acc = fmaxf(acc, 0.f) * fmaxf(acc, 0.f);
       store_out(out, ldo, m, f, acc);
     }
   }
@@ -249,7 +251,7 @@ gemm_skinny_kernel(const bf16* __restrict__ X, long ldx, const bf16* __restrict_
       else
         store_out(out, ldo, m, f, silu(v) * u);
     } else {
-      store_out(out, ldo, m, n, epi == EPI_BIAS ? v + bf2f(bias[n]) : v);
+      store_out(out, ldo, m, n, epi == EPI_BIAS ? v + bf2f(bias[n]) : epi == EPI_RELU2 ? fmaxf(v, 0.f) * fmaxf(v, 0.f) : v);
     }
   }
 }
@@ -387,6 +389,10 @@ __device__ __forceinline__ void tile_epilogue(const f32x4 (&acc)[TI][TJ], int mw
         if (epi == EPI_BIAS) {
 #pragma unroll
           for (int r = 0; r < 4; ++r) v[r] += bf2f(bias[n + r]);
+        }
+        if (epi == EPI_RELU2) {
+#pragma unroll
+          for (int r = 0; r < 4; ++r) v[r] = fmaxf(v[r], 0.f) * fmaxf(v[r], 0.f);
         }
         store_out4(out, ldo, m, n, v, vec);
       }

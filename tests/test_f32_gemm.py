@@ -68,3 +68,44 @@ def test_prefill_tile_with_half_a_column_tile(M, N, K, bias):
     # one rounding to bf16 (2^-9) of f32 sums
     assert ((out[:, :N].cpu().to(F64) - want).abs() < 2.0 ** -8 * want.abs() + 1e-3 * K ** 0.5).all()
     assert (out[:, N:] == 7.0).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(1, 128, 128), (40, 256, 512), (300, 512, 2048), (2100, 1152, 256)])      # skinny, tile + split K, prefill
+def test_squared_relu_epilogue(M, N, K):
+    g = torch.Generator().manual_seed(M + N)
+    x, w = torch.randn(M, K, generator=g).bfloat16(), torch.randn(N, K, generator=g).bfloat16()
+    got = ops.linear_act(x.cuda(), w.cuda(), act="relu2").cpu().to(F64)
+    want = torch.relu(x.to(F64) @ w.to(F64).T) ** 2
+    assert ((got - want).abs() < 2.0 ** -8 * want + 1e-2).all()      # one rounding to bf16 of the squared f32 sum
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("T,S,W", [(3, 1, 4), (5, 2, 1024), (2, 3, 1028), (4, 4, 4096), (2, 2, 8192), (3, 2, 2050), (2, 5, 64)])
+def test_stream_passes(dt, T, S, W):
+    g = torch.Generator().manual_seed(S * W)
+    r = lambda *s: torch.randn(*s, generator=g)                                     # noqa: E731
+    xs, y, mix, wo, wi, nw = r(T, S, W), r(T, W).to(dt), r(S, S), r(S), r(S), r(W)
+    unit = lambda u: u / torch.sqrt((u * u).mean(-1, keepdim=True) + 1e-6) * (nw.to(F64) + 1)          # noqa: E731
+    new = torch.einsum("tsw,sr->trw", xs.to(F64), mix.to(F64)) + wo.to(F64)[None, :, None] * y.to(F64)[:, None]
+    tol = 2e-5 if dt == torch.float32 else 2.0 ** -7
+    c = lambda t: t.cuda()                                                         # noqa: E731
+
+    def same(got, want, tol=tol):
+        assert (got.cpu().to(F64) - want).abs().max() < tol * (1 + want.abs().max())
+
+    a = c(xs).clone()
+    h = ops.hc_post_pre_(a, c(y), c(mix), c(wo), c(wi), c(nw), 1e-6, 1.0, dt)
+    same(a, new, 2e-6)
+    same(h, unit(torch.einsum("s,tsw->tw", wi.to(F64), new)))
+    b = c(xs).clone()
+    ops.hc_post_(b, c(y), c(mix), c(wo))
+    assert torch.equal(a, b)
+    same(ops.hc_pre(c(xs), c(wi), c(nw), 1e-6, 1.0, dt), unit(torch.einsum("s,tsw->tw", wi.to(F64), xs.to(F64))))
+    rows = torch.tensor([T - 1, 0])
+    same(ops.hc_final(c(xs), c(nw), 1e-6, 1.0, c(rows), dt), unit(xs.to(F64).sum(1))[rows])
+    table, ids = r(9, W).to(dt), torch.tensor([8, 0, 3], dtype=torch.int32)
+    e = ops.embed_norm_streams(c(ids), c(table), c(nw), 1e-6, 1.0, S)
+    for s in range(S):
+        same(e[:, s], unit(table.to(F64)[ids.long()]), 2e-6)
