@@ -1,6 +1,6 @@
 // Attention kernels (K3 flash prefill, K4 paged decode, split-K combine) for GQA, head_dim 128.
 //
-// Decode (attn_decode_kernel): one workgroup per (context split, kv head, sequence), 4 waves
+// Decode (attn_decode_kernel): one workgroup per (context split, kv head, sequence), 4 or 8 waves
 // that walk the split's KV pages round-robin. The whole query group of a kv head (Hq/Hkv <= 16
 // rows, padded to 16) rides in ONE mfma_f32_16x16x32_bf16 B operand, so every K/V byte
 // streamed from HBM feeds all query heads that share it. K/V go straight to VGPRs (decode
@@ -21,6 +21,7 @@
 // read by ds_read_b128 as the 32x32x16 A operand of S^T = K . Q^T, V by ds_read_b64_tr_b16 as
 // the A operand of O^T = V^T . P^T; the S^T accumulator is converted in registers into the
 // P^T B operand (§3 "An accumulator tile as the next MFMA's operand").
+#include <algorithm>
 #include <type_traits>
 
 #include "bfly_common.h"
@@ -39,8 +40,8 @@ constexpr float kNegInf = -INFINITY;
 // ---------------------------------------------------------------------------------------
 // Decode
 // ---------------------------------------------------------------------------------------
-template <int D, int BS, typename CT>
-__global__ void __launch_bounds__(kAttnThreads)
+template <int D, int BS, typename CT, int NW>
+__global__ void __launch_bounds__(64 * NW)
 attn_decode_kernel(const bf16* __restrict__ q, long q_stride, const CT* __restrict__ k_cache,
                    const CT* __restrict__ v_cache, const int* __restrict__ block_tables,
                    int bt_stride, const int* __restrict__ ctx_lens, int Hq, int Hkv,
@@ -56,8 +57,10 @@ attn_decode_kernel(const bf16* __restrict__ q, long q_stride, const CT* __restri
   const int tok1 = min(ctx, tok0 + part_tokens);
   const long part_base = ((long)(b * Hkv + h) * nsplit + s);
 
-  __shared__ float s_o[4][8][4][64];
-  __shared__ float s_m[4][16], s_l[4][16];
+  extern __shared__ __attribute__((aligned(16))) float dec_smem[];
+  float* s_o = dec_smem;                       // [NW][8 dt][4 i][4 g][G rows]
+  float(*s_m)[16] = reinterpret_cast<float(*)[16]>(dec_smem + NW * 128 * G);      // [NW][16]
+  float(*s_l)[16] = s_m + NW;
 
   if (tok0 >= tok1) {  // empty split: mark it so the combine skips it
     if (nsplit > 1 && threadIdx.x < 16) {
@@ -128,102 +131,101 @@ attn_decode_kernel(const bf16* __restrict__ q, long q_stride, const CT* __restri
 #pragma unroll
       for (int ds = 0; ds < 4; ++ds) st[kt] = mfma16(KV<CT>::widen(kf[kt][ds]), qf[ds], st[kt]);
     }
-    // st[kt][i] = S[key = p*BS + 8g + 4kt + i][query r]
+    // st[kt][i] = S[key = p*BS + 8g + 4kt + i][query r]; only the context's last page has keys past its end
     float x[8];
     float tmax = kNegInf;
+    if ((p + 1) * BS <= tok1) {
 #pragma unroll
-    for (int kt = 0; kt < 2; ++kt)
+      for (int j = 0; j < 8; ++j) x[j] = st[j >> 2][j & 3] * scale_log2;
+    } else {
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int key = p * BS + 8 * g + 4 * kt + i;
-        const float v = key < tok1 ? st[kt][i] * scale_log2 : kNegInf;
-        x[kt * 4 + i] = v;
-        tmax = fmaxf(tmax, v);
-      }
-    tmax = fmaxf(tmax, __shfl_xor(tmax, 16, 64));
-    tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64));
-    const float mn = fmaxf(m, tmax);
-    const float mb = mn == kNegInf ? 0.f : mn;
-    const float alpha = exp2f(m - mb);
+      for (int j = 0; j < 8; ++j) x[j] = p * BS + 8 * g + j < tok1 ? st[j >> 2][j & 3] * scale_log2 : kNegInf;
+    }
+#pragma unroll
+    for (int j = 0; j < 8; ++j) tmax = fmaxf(tmax, x[j]);
+    tmax = row4_max(tmax);
+    if (__any(tmax > m)) {      // a larger maximum in some row: rescale (elsewhere the factor is 1)
+      const float mn = fmaxf(m, tmax);
+      const float alpha = __builtin_amdgcn_exp2f(m - (mn == kNegInf ? 0.f : mn));
+      m = mn;
+      l *= alpha;
+#pragma unroll
+      for (int dt = 0; dt < 8; ++dt) o[dt] *= alpha;
+    }
+    const float mb = m == kNegInf ? 0.f : m;
     bf16x8 pb;
-    float ps = 0.f;
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
-      const float pv = exp2f(x[j] - mb);
-      ps += pv;
+      const float pv = __builtin_amdgcn_exp2f(x[j] - mb);
+      l += pv;
       pb[j] = f2bf(pv);
     }
-    l = l * alpha + ps;
-    m = mn;
 #pragma unroll
-    for (int dt = 0; dt < 8; ++dt) {
-      o[dt] *= alpha;
-      o[dt] = mfma16(KV<CT>::widen(vf[dt]), pb, o[dt]);
-    }
+    for (int dt = 0; dt < 8; ++dt) o[dt] = mfma16(KV<CT>::widen(vf[dt]), pb, o[dt]);
   };
 
-  // software pipeline over this wave's pages (p0 + wid, +4, ...): the next page's K/V loads
+  // software pipeline over this wave's pages (p0 + wid, +NW, ...): the next page's K/V loads
   // are in flight while the current page is computed; two named register sets (rule 20).
   raw_t kA[2][4], vA[8], kB[2][4], vB[8];
   int p = p0 + wid;
   if (p < p1) load_page(p, kA, vA);
   if constexpr (sizeof(CT) == 2) {
     while (p < p1) {
-      if (p + 4 < p1) load_page(p + 4, kB, vB);
+      if (p + NW < p1) load_page(p + NW, kB, vB);
       compute_page(p, kA, vA);
-      p += 4;
+      p += NW;
       if (p >= p1) break;
-      if (p + 4 < p1) load_page(p + 4, kA, vA);
+      if (p + NW < p1) load_page(p + NW, kA, vA);
       compute_page(p, kB, vB);
-      p += 4;
+      p += NW;
     }
   } else {
     // FP8 pages are half the bytes: keep TWO pages in flight (three register sets in
     // rotation, the VGPRs of 1.5 bf16 sets) so the bytes in flight per wave, which bound a
     // latency-limited stream, match the bf16 kernel's
     raw_t kC[2][4], vC[8];
-    if (p + 4 < p1) load_page(p + 4, kB, vB);
+    if (p + NW < p1) load_page(p + NW, kB, vB);
     while (p < p1) {
-      if (p + 8 < p1) load_page(p + 8, kC, vC);
+      if (p + 2 * NW < p1) load_page(p + 2 * NW, kC, vC);
       compute_page(p, kA, vA);
-      p += 4;
+      p += NW;
       if (p >= p1) break;
-      if (p + 8 < p1) load_page(p + 8, kA, vA);
+      if (p + 2 * NW < p1) load_page(p + 2 * NW, kA, vA);
       compute_page(p, kB, vB);
-      p += 4;
+      p += NW;
       if (p >= p1) break;
-      if (p + 8 < p1) load_page(p + 8, kB, vB);
+      if (p + 2 * NW < p1) load_page(p + 2 * NW, kB, vB);
       compute_page(p, kC, vC);
-      p += 4;
+      p += NW;
     }
   }
-  l += __shfl_xor(l, 16, 64);
-  l += __shfl_xor(l, 32, 64);
+  l = row4_sum(l);
 
-  // Merge the 4 waves: o[dt][i] = O[query r][d = 16dt + 4g + i]
+  // Merge the waves: o[dt][i] = O[query r][d = 16dt + 4g + i]; only the G real rows go through LDS
+  if (r < G) {
 #pragma unroll
-  for (int dt = 0; dt < 8; ++dt)
+    for (int dt = 0; dt < 8; ++dt)
 #pragma unroll
-    for (int i = 0; i < 4; ++i) s_o[wid][dt][i][lane] = o[dt][i];
-  if (g == 0) {
-    s_m[wid][r] = m;
-    s_l[wid][r] = l;
+      for (int i = 0; i < 4; ++i) s_o[((wid * 32 + dt * 4 + i) * 4 + g) * G + r] = o[dt][i];
+    if (g == 0) {
+      s_m[wid][r] = m;
+      s_l[wid][r] = l;
+    }
   }
   __syncthreads();
-  for (int e = threadIdx.x; e < 16 * D; e += kAttnThreads) {
+  for (int e = threadIdx.x; e < G * D; e += 64 * NW) {
     const int qr = e / D, d = e % D;
-    if (qr >= G) continue;
     float M = kNegInf;
 #pragma unroll
-    for (int w = 0; w < 4; ++w) M = fmaxf(M, s_m[w][qr]);
+    for (int w = 0; w < NW; ++w) M = fmaxf(M, s_m[w][qr]);
     const float Mb = M == kNegInf ? 0.f : M;
     float L = 0.f, O = 0.f;
-    const int dt = d >> 4, i = d & 3, ln = qr + 16 * ((d & 15) >> 2);
+    const float* po = s_o + ((d >> 4) * 16 + (d & 3) * 4 + ((d & 15) >> 2)) * G + qr;
 #pragma unroll
-    for (int w = 0; w < 4; ++w) {
+    for (int w = 0; w < NW; ++w) {
       const float f = exp2f(s_m[w][qr] - Mb);
       L += f * s_l[w][qr];
-      O += f * s_o[w][dt][i][ln];
+      O += f * po[w * 128 * G];
     }
     if (nsplit == 1) {
       out[((long)b * Hq + h * G + qr) * D + d] = f2bf(L > 0.f ? O / L : 0.f);
@@ -713,13 +715,14 @@ int attn_decode_splits(int max_ctx, int part_tokens) {
 }
 
 // Context split size, from a split-size sweep on MI355X (tools/bench_attn.py --parts): aim at
-// ~256 (b, kv-head, split) workgroups (one per CU), splitting the context evenly and never
+// ~256 (b, kv-head, split) workgroups (one per CU, the nearest number: 192 pairs stay whole, 141 against 150 us at 24
+// sequences of up to 8k), splitting the context evenly and never
 // below 256 tokens per split; a single split skips the combine launch entirely.
 //   B=64 Hkv=8 ctx 1K: 1 split 46 us (2 splits 53);  B=8 ctx 4K: 4 splits 30 us (16: 38);
 //   B=64 Hkv=1: 4 splits 13.5 us (8: 15.4);        B=1 ctx 8K: 32 splits 27 us (64: 43).
 int attn_decode_part_tokens(int B, int Hkv, int max_ctx) {
   const int pairs = B * Hkv > 0 ? B * Hkv : 1;
-  const int splits = (256 + pairs - 1) / pairs;
+  const int splits = std::max(1, (256 + pairs / 2) / pairs);
   int part = (max_ctx + splits - 1) / splits;
   part = (part + 31) / 32 * 32;
   if (splits > 1 && part < 256) part = 256;
@@ -741,12 +744,33 @@ int launch_attn_decode(const bf16* q, long q_stride, const void* k_cache, const 
   if (nsplit > 1 && (part_o == nullptr || part_ml == nullptr)) return -3;
   const float scale_log2 = scale * 1.4426950408889634f;
   dim3 grid(nsplit, Hkv, B);
-#define DEC_LAUNCH(CT)                                                                                      \
-  attn_decode_kernel<128, 32, CT><<<grid, kAttnThreads, 0, stream>>>(                                        \
-      q, q_stride, static_cast<const CT*>(k_cache), static_cast<const CT*>(v_cache), block_tables, bt_stride, \
-      ctx_lens, Hq, Hkv, scale_log2, part_tokens, out, part_o, part_ml)
-  if (kv_fp8) DEC_LAUNCH(fp8_t);
-  else DEC_LAUNCH(bf16);
+  const int G = Hq / Hkv;
+  // Up to 320 workgroups (little more than one per compute unit): eight waves each, so that a compute unit keeps twice the
+  // pages in flight and a long context is walked by twice the waves. 32 heads on 8, contexts of 2.5k to 8k of 24 sequences:
+  // FP8 99 -> 61 us, bf16 135 -> 118; 37 sequences of 0.9k to 3k 69 -> 60 us; from 384 workgroups on four are level
+  // (64 sequences of 1040: 34 us against 36). Sixteen waves hold 128 registers each and spill.
+  const bool w8 = (long)nsplit * Hkv * B <= 320;
+#define DEC_LAUNCH1(CT, NW)                                                                                 \
+  {                                                                                                         \
+    const size_t lds = (size_t)NW * (128 * G + 32) * sizeof(float);                                         \
+    static bool once = false;                                                                               \
+    if (!once) {                                                                                            \
+      (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_decode_kernel<128, 32, CT, NW>),       \
+                                hipFuncAttributeMaxDynamicSharedMemorySize, NW * (128 * 16 + 32) * 4);      \
+      once = true;                                                                                          \
+    }                                                                                                       \
+    attn_decode_kernel<128, 32, CT, NW><<<grid, 64 * NW, lds, stream>>>(                                    \
+        q, q_stride, static_cast<const CT*>(k_cache), static_cast<const CT*>(v_cache), block_tables, bt_stride, \
+        ctx_lens, Hq, Hkv, scale_log2, part_tokens, out, part_o, part_ml);                                  \
+  }
+#define DEC_LAUNCH(CT)                        \
+  {                                           \
+    if (w8) DEC_LAUNCH1(CT, 8)                \
+    else DEC_LAUNCH1(CT, 4)                   \
+  }
+  if (kv_fp8) DEC_LAUNCH(fp8_t)
+  else DEC_LAUNCH(bf16)
+#undef DEC_LAUNCH1
 #undef DEC_LAUNCH
   if (nsplit > 1) {
     // Measured and dropped: merging the splits inside the decode kernel (last arriver, agent-

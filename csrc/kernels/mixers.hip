@@ -306,7 +306,7 @@ __global__ __launch_bounds__(256) void attn_window_f32_kernel(const float* __res
       sc[e] = ok ? x : -INFINITY;
       mx = fmaxf(mx, sc[e]);
     }
-    const float mn = fmaxf(m, quad_max(mx));
+    const float mn = fmaxf(m, row4_max(mx));
     const float corr = expf(m - mn);
     m = mn;
     l *= corr;
@@ -326,7 +326,7 @@ __global__ __launch_bounds__(256) void attn_window_f32_kernel(const float* __res
       }
     }
   }
-  l = quad_sum(l);
+  l = row4_sum(l);
   if (!rv) return;
   const float inv = (out_scale ? out_scale[row * H + h] : 1.f) / l;
 #pragma unroll

@@ -116,3 +116,33 @@ def test_chunks_over_a_cached_prefix(Hq, Hkv, seqs):
     err = (out[:, :Hq].cpu().to(F64) - torch.cat(want)).abs().max()
     assert err < 2.0 ** -8 * vc.float().abs().max() + 1e-3
     assert not out[:, Hq:].any()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("Hq,Hkv,ctx,max_ctx", [
+    (32, 8, [1, 31, 32, 33, 257, 700], 1024),      # split contexts, eight waves; most waves without a page
+    (8, 1, [40, 3000], 3008),                      # eight rows, split
+    (16, 8, list(range(5, 200, 8)), 256),          # 200 pairs: whole contexts, eight waves
+    (64, 8, [100 + i for i in range(48)], 160),    # 384 pairs: four waves
+    (16, 1, [65, 1], 96),                          # sixteen query heads on one
+])
+def test_decode_waves_and_splits(fp8, Hq, Hkv, ctx, max_ctx):
+    g = torch.Generator().manual_seed(Hq + len(ctx))
+    D, B, scale = 128, len(ctx), 1.5 / math.sqrt(128)
+    dt = torch.float8_e4m3fn if fp8 else torch.bfloat16
+    need = [(c + BS - 1) // BS for c in ctx]
+    kc, vc = torch.randn(sum(need), Hkv, BS, D, generator=g).to(dt), torch.randn(sum(need), Hkv, D, BS, generator=g).to(dt)
+    q = torch.randn(B, Hq, D, generator=g).bfloat16()
+    tables = torch.zeros(B, (max_ctx + BS - 1) // BS, dtype=torch.int32)
+    order, at, want = torch.randperm(sum(need), generator=g), 0, []
+    for b, c in enumerate(ctx):
+        pages = order[at:at + need[b]]
+        at += need[b]
+        tables[b, :need[b]] = pages.int()
+        k = kc.float()[pages].transpose(1, 2).reshape(-1, Hkv, D)[:c].to(F64)
+        v = vc.float()[pages].permute(0, 3, 1, 2).reshape(-1, Hkv, D)[:c].to(F64)
+        want.append(dense(q[b:b + 1].to(F64), k, v, torch.tensor([c - 1]), scale, 1 << 30, 0, None, None, 0, None))
+    got = ops.attn_decode(q.cuda(), kc.cuda(), vc.cuda(), tables.cuda(), torch.tensor(ctx, dtype=torch.int32).cuda(), scale, max_ctx)
+    err = (got.cpu().to(F64) - torch.cat(want)).abs().max()
+    assert err < 2.0 ** -8 * vc.float().abs().max() + 1e-3      # weights and output rounded to bf16
