@@ -8,12 +8,14 @@
 //                                    history pool, zeros before position 0
 //   short_conv_state_update_kernel   the pool takes the last taps - 1 rows of every sequence
 //   delta_scan_kernel                S <- g S; u = beta (v - S^T k); S <- S + k u^T; o = S^T q per
-//                                    (sequence, head), the state pooled per sequence
+//                                    (sequence, head), the state pooled per sequence; row by row
+//   delta_chunk_kernel               the same in chunks of 16 rows on the f32 matrix cores
 // Rows of a step are packed: sequence s owns rows row_cu[s] .. row_cu[s+1].
 #include <algorithm>
 
 #include "bfly_common.h"
 #include "bfly_delta.h"
+#include "bfly_recur_dev.h"
 
 namespace bfly {
 
@@ -475,6 +477,381 @@ __global__ __launch_bounds__(512) void delta_scan_kernel(const float* __restrict
   }
 }
 
+// orders one wave's LDS accesses: what its lanes wrote before is what they read after
+__device__ __forceinline__ void lds_wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+// Steps with more rows than sequences (prompts): chunks of 16 rows on the f32 matrix cores. Row by row every token is
+// two dot products and an update in one dependent chain (0.78 us a token at D = 128); a chunk needs one chain. With
+// k, q the unit rows, G_t = g_0 .. g_t and D_tj = g_(j+1) .. g_t (products of decays over the chunk's rows, never
+// quotients) and S the state before the chunk,
+//   U = (I + L)^-1 diag(beta) (V - diag(G) K S),   L_tj = beta_t D_tj k_t . k_j  (j < t)
+//   o_t = G_t q_t S + sum_(j <= t) D_tj (q_t . k_j) u_j,   S <- G_15 S + sum_j D_15,j k_j u_j^T
+// Workgroup = (sequence, head, 64 columns of Dv), eight waves in a pipeline of three chunks with one barrier per step:
+//   waves 4 .. 7 load chunk p (a quarter of the channels each, in the operand layout of the 16x16x4 tiles), put its raw
+//   rows into LDS and form their parts of K K^T, Q K^T and the squared norms; wave 6 also the products of its decays,
+//   which wave 7 has computed a step before;
+//   wave 4 turns those of chunk p - 1 into (I + L)^-1 diag(beta): forward substitution in the two 8 x 8 blocks on the
+//   diagonal (lane m: column m), the block below them as -T22 L21 T11; wave 5 the weights of the second sum;
+//   waves 0 .. 3 run chunk p - 2 with 16 columns of the state each. A state tile's accumulator layout (element e of lane
+//   group gg: row 16 i + 4 gg + e) is the B operand of K S and Q S, and the accumulators of V - ..., U are the B
+//   operands of the products that follow, so nothing of the chain goes through LDS.
+// The unit norms are factors of rows and columns. Rows past the sequence: k = q = 0, g = 1, beta = 0. D <= 16 NT. A
+// chunk is one matrix product: NaN or infinity in a row reaches all rows of its chunk.
+// Rounding: a chunk's scalars (decay products, norms, factors of L) are formed in 64 bits and rounded once, products over
+// channels are summed in pieces of 32 or 64, and the unit diagonal of (I + L)^-1 is applied without a product; with that
+// outputs and states are as far from a 64-bit recurrence as the row-by-row kernel's (rms 1.3e-7 and 1.0e-7 relative).
+// Eight sequences of 1024 rows, 16 heads, D = Dv = 128: 534 -> 222 us; bound by the two waves of a SIMD in turn, one
+// with products (2.2 us a chunk by itself), one with the scalars' chain (1.9 us).
+template <typename T, int NT>
+__global__ __launch_bounds__(512, NT <= 4 ? 4 : 2) void delta_chunk_kernel(
+    const float* __restrict__ q, long q_ld, const float* __restrict__ k, long k_ld, const float* __restrict__ v, long v_ld,
+    const T* __restrict__ bl, long b_ld, const T* __restrict__ al, long a_ld, const float* __restrict__ a_log,
+    const float* __restrict__ dt_bias, float* __restrict__ state, const int* __restrict__ state_slots,
+    const int* __restrict__ row_cu, const int* __restrict__ positions, float q_scale, float unit_eps, int vec,
+    float* __restrict__ o, int H, int G, int D, int Dv) {
+  constexpr int C = 16, NQ = NT / 4, NG = NT / 4, NS = NT <= 8 ? 2 : 4, KP = 16 * NT + 4, PP = C + 4;
+  extern __shared__ __attribute__((aligned(16))) float smem[];
+  float* sk = smem;                       // [3][C][KP] raw k
+  float* sq = sk + 3 * C * KP;            // [3][C][KP] raw q
+  float* skk = sq + 3 * C * KP;           // [2][4][64][4] the waves' parts of K K^T
+  float* sqk = skk + 2 * 4 * 256;         // [2][4][64][4] and of Q K^T
+  float* snk = sqk + 2 * 4 * 256;         // [2][4][C] of the squared norms
+  float* snq = snk + 2 * 4 * C;           // [2][4][C]
+  float* sd = snq + 2 * 4 * C;            // [2][64][4] D
+  float* sg = sd + 2 * 256;               // [2][4][C]: G, D_15, beta, G_15
+  float* sT = sg + 2 * 4 * C;             // [2][C][PP] (I + L)^-1 diag(beta)
+  float* sA = sT + 2 * C * PP;            // [2][C][PP] weights D_tj (q_t . k_j) / |k_j|
+  float* sc = sA + 2 * C * PP;            // [2][6][C]: G / |k|, D_15 / |k|, G, q_scale / |q|, G_15, beta
+  float* sl = sc + 2 * 6 * C;             // [2][2][C] decay and write strength of each row
+  const int s = blockIdx.x, h = blockIdx.y, c0 = blockIdx.z * 64;
+  const int hk = h / (H / G);
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, m = lane & 15, gg = lane >> 4;
+  const int r0 = __builtin_amdgcn_readfirstlane(row_cu[s]), r1 = __builtin_amdgcn_readfirstlane(row_cu[s + 1]);
+  const int slot = state_slots[s];
+  if (r1 <= r0) return;
+  if (slot < 0) {      // padding sequence of a fixed-shape step: defined output, no state
+    for (int i = tid; i < (r1 - r0) * 64; i += 512)
+      if (c0 + (i & 63) < Dv) o[((long)(r0 + (i >> 6)) * H + h) * Dv + c0 + (i & 63)] = 0.f;
+    return;
+  }
+  const int nch = (r1 - r0 + C - 1) / C;
+  if (wave < 4) {
+    const int col = c0 + 16 * wave + m;
+    const bool live = col < Dv;
+    float* S = state + (((long)slot * H + h) * Dv + min(col, Dv - 1)) * D;      // this lane's column
+    const bool fresh = positions[r0] == 0;
+    f32x4 st[NT];
+#pragma unroll
+    for (int i = 0; i < NT; ++i) {
+      const int d = 16 * i + 4 * gg;
+      st[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+      if (!fresh) {
+        if ((vec & 2) && d < D) st[i] = *reinterpret_cast<const f32x4*>(S + d);
+        else
+#pragma unroll
+          for (int e = 0; e < 4; ++e) st[i][e] = d + e < D ? S[d + e] : 0.f;
+      }
+    }
+    const float* vc = v + (long)h * Dv + min(col, Dv - 1);
+    float rv[4];
+    auto fetch = [&](int t0) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) rv[e] = vc[(long)min(t0 + 4 * gg + e, r1 - 1) * v_ld];
+    };
+    fetch(r0);
+    for (int i = 0; i < 3; ++i) __syncthreads();
+    for (int c = 0; c < nch; ++c) {
+      const int t0 = r0 + c * C;
+      const float* kb = sk + (c % 3) * C * KP;
+      const float* qb = sq + (c % 3) * C * KP;
+      const float* f = sc + (c & 1) * 6 * C;
+      // Operands come from LDS a group of four tiles ahead of their use. Partial sums by element and per NS tiles: short
+      // dependent chains, and no longer sums than a row's own dot product takes.
+      f32x4 ka[2][4], qa[2][4], pk = {0.f, 0.f, 0.f, 0.f}, pq = pk, u = pk, y = pk;
+      float ku[2][4][4];
+      auto rows = [&](int g) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          ka[g & 1][i] = *reinterpret_cast<const f32x4*>(kb + m * KP + 16 * (4 * g + i) + 4 * gg);
+          qa[g & 1][i] = *reinterpret_cast<const f32x4*>(qb + m * KP + 16 * (4 * g + i) + 4 * gg);
+        }
+      };
+      auto cols = [&](int g) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) ku[g & 1][i][e] = kb[(4 * gg + e) * KP + 16 * (4 * g + i) + m];
+      };
+      f32x4 ux[4], yx[4];
+      rows(0);
+      const f32x4 gk = *reinterpret_cast<const f32x4*>(f + 4 * gg), dk = *reinterpret_cast<const f32x4*>(f + C + 4 * gg);
+      const f32x4 gt = *reinterpret_cast<const f32x4*>(f + 2 * C + 4 * gg);
+      const f32x4 qn = *reinterpret_cast<const f32x4*>(f + 3 * C + 4 * gg);
+      const f32x4 ti = *reinterpret_cast<const f32x4*>(sT + ((c & 1) * C + m) * PP + 4 * gg);
+      const f32x4 wq = *reinterpret_cast<const f32x4*>(sA + ((c & 1) * C + m) * PP + 4 * gg);
+      const f32x4 bt = *reinterpret_cast<const f32x4*>(f + 5 * C + 4 * gg);
+      const float gn = f[4 * C];
+#pragma unroll
+      for (int g = 0; g < NG; ++g) {
+        if (g + 1 < NG) rows(g + 1);
+        else cols(0);
+#pragma unroll
+        for (int j = 0; j < 4; j += NS) {
+        f32x4 xk[4], xq[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) xk[e] = xq[e] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int i = j; i < j + NS; ++i)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            xk[e] = mfma_f32(ka[g & 1][i][e], st[4 * g + i][e], xk[e]);
+            xq[e] = mfma_f32(qa[g & 1][i][e], st[4 * g + i][e], xq[e]);
+          }
+        pk += (xk[0] + xk[1]) + (xk[2] + xk[3]);
+        pq += (xq[0] + xq[1]) + (xq[2] + xq[3]);
+}
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float vv = t0 + 4 * gg + e < r1 ? rv[e] : 0.f;
+        const float ve = fmaf(-gk[e], pk[e], vv);
+        ux[e] = mfma_f32(ti[e], ve, f32x4{0.f, 0.f, 0.f, 0.f});
+        u[e] = bt[e] * ve;
+      }
+      u += (ux[0] + ux[1]) + (ux[2] + ux[3]);
+      if (c + 1 < nch) fetch(t0 + C);      // in flight until the next chunk
+      const f32x4 ud = u * dk;
+#pragma unroll
+      for (int g = 0; g < NG; ++g) {
+        if (g + 1 < NG) cols(g + 1);
+        f32x4 x[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) x[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) x[i] = mfma_f32(ku[g & 1][i][e], ud[e], x[i]);
+          if (g == 0) yx[e] = mfma_f32(wq[e], u[e], f32x4{0.f, 0.f, 0.f, 0.f});
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) st[4 * g + i][e] = fmaf(st[4 * g + i][e], gn, x[i][e]);
+      }
+      y = (yx[0] + yx[1]) + (yx[2] + yx[3]);
+      if (live) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int t = t0 + 4 * gg + e;
+          if (t < r1) o[((long)t * H + h) * Dv + col] = fmaf(pq[e], gt[e], y[e]) * qn[e];
+        }
+      }
+      __syncthreads();
+    }
+    if (live) {
+#pragma unroll
+      for (int i = 0; i < NT; ++i) {
+        const int d = 16 * i + 4 * gg;
+        if ((vec & 2) && d < D) *reinterpret_cast<f32x4*>(S + d) = st[i];
+        else
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            if (d + e < D) S[d + e] = st[i][e];
+      }
+    }
+    return;
+  }
+  // ---- waves 4 .. 7: chunk p's rows and their products, then the 16 x 16 matrices of chunk p - 1 ----
+  __builtin_amdgcn_s_setprio(2);      // (a chunk's chain of scalars is as long as the products it waits for)
+  const int w = wave - 4;
+  const float rate = expf(a_log[h]), dtb = dt_bias[h];
+  f32x4 rk[NQ], rq[NQ];
+  T an = (T)0.f, bn = (T)0.f;      // wave 7: the logits of row m, as stored (a conversion here would wait for the loads)
+  auto gates = [&](int t0) {
+    const long t = min(t0 + m, r1 - 1);
+    an = al[t * a_ld + h];
+    bn = bl[t * b_ld + h];
+  };
+  // wave 7, chunk c: decay and write strength of row m
+  auto write_gates = [&](int c) {
+    const bool in = r0 + c * C + m < r1;
+    const float av = (float)an + dtb;
+    const float sp = av > 20.f ? av : log1pf(expf(av));            // softplus
+    sl[(c & 1) * 2 * C + m] = in ? expf(-rate * sp) : 1.f;
+    sl[((c & 1) * 2 + 1) * C + m] = in ? 1.f / (1.f + expf(-(float)bn)) : 0.f;
+  };
+  const float* k0 = k + (long)(r0 + m) * k_ld + (long)hk * D;
+  const float* q0 = q + (long)(r0 + m) * q_ld + (long)hk * D;
+  auto fetch = [&](int t0) {
+    long past = t0 - r0;
+    if (t0 + C > r1) past -= max(0, t0 + m - (r1 - 1));      // (rows past the sequence: its last row again)
+    const float* kr = k0 + past * k_ld;
+    const float* qr = q0 + past * q_ld;
+    if (vec & 1) {
+#pragma unroll
+      for (int i = 0; i < NQ; ++i) {
+        const int d = min(16 * (NQ * w + i) + 4 * gg, D - 4);
+        rk[i] = *reinterpret_cast<const f32x4*>(kr + d);
+        rq[i] = *reinterpret_cast<const f32x4*>(qr + d);
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < NQ; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int d = min(16 * (NQ * w + i) + 4 * gg + e, D - 1);
+          rk[i][e] = kr[d];
+          rq[i][e] = qr[d];
+        }
+    }
+  };
+  if (w == 3) {
+    gates(r0);
+    write_gates(0);
+    if (nch > 1) gates(r0 + C);
+  }
+  fetch(r0);
+  __syncthreads();
+  for (int p = 0; p < nch + 2; ++p) {
+    if (p < nch) {
+      const int t0 = r0 + p * C;
+      float* kb = sk + (p % 3) * C * KP + m * KP;
+      float* qb = sq + (p % 3) * C * KP + m * KP;
+      f32x4 nk = {0.f, 0.f, 0.f, 0.f}, nq = nk, kx[4], qx[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) kx[e] = qx[e] = nk;
+      const int in = t0 + m < r1, Dm = in ? D : 0;
+#pragma unroll
+      for (int i = 0; i < NQ; ++i) {
+        const int d = 16 * (NQ * w + i) + 4 * gg;
+        f32x4 a, b;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const bool ok = d + e < Dm;
+          a[e] = ok ? rk[i][e] : 0.f;
+          b[e] = ok ? rq[i][e] : 0.f;
+        }
+        *reinterpret_cast<f32x4*>(kb + d) = a;
+        *reinterpret_cast<f32x4*>(qb + d) = b;
+        nk += a * a;
+        nq += b * b;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          kx[e] = mfma_f32(a[e], a[e], kx[e]);
+          qx[e] = mfma_f32(b[e], a[e], qx[e]);
+        }
+      }
+      if (p + 1 < nch) fetch(t0 + C);
+      const float xk = row4_sum((nk[0] + nk[1]) + (nk[2] + nk[3])), xq = row4_sum((nq[0] + nq[1]) + (nq[2] + nq[3]));
+      const int at = (p & 1) * 4 + w;
+      const f32x4 kk = (kx[0] + kx[1]) + (kx[2] + kx[3]), qk = (qx[0] + qx[1]) + (qx[2] + qx[3]);
+      *reinterpret_cast<f32x4*>(skk + (at * 64 + lane) * 4) = kk;
+      *reinterpret_cast<f32x4*>(sqk + (at * 64 + lane) * 4) = qk;
+      snk[at * C + m] = xk;
+      snq[at * C + m] = xq;
+      if (w == 2) {
+        const float g = sl[(p & 1) * 2 * C + m];
+        // column m of D (rows 4 gg + e kept), G_m, D_15,m and G_15
+        int mm = m, gm = gg;
+        asm volatile("" : "+v"(mm), "+v"(gm));      // (compared anew per chunk: kept masks would fill the scalar registers)
+        double x = 1., y = 1.;
+        float Gm = 1.f;
+        f32x4 dm;
+#pragma unroll
+        for (int t = 0; t < C; ++t) {
+          const double gt = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, g), t));
+          y *= gt;
+          x = t > mm ? x * gt : 1.;
+          Gm = t == mm ? (float)y : Gm;
+          if (t < 4) dm[t] = (float)x;
+          else dm[t & 3] = gm == t >> 2 ? (float)x : dm[t & 3];
+        }
+        *reinterpret_cast<f32x4*>(sd + ((p & 1) * 64 + lane) * 4) = dm;
+        float* f = sg + (p & 1) * 4 * C + m;
+        f[0] = Gm;
+        f[C] = (float)x;
+        f[2 * C] = sl[((p & 1) * 2 + 1) * C + m];
+        f[3 * C] = (float)y;
+      } else if (w == 3 && p + 1 < nch) {
+        write_gates(p + 1);
+        if (p + 2 < nch) gates(t0 + 2 * C);
+      }
+    }
+    if (p > 0 && p <= nch && w < 2) {
+      const int b2 = (p - 1) & 1;
+      const f32x4 dm = *reinterpret_cast<const f32x4*>(sd + (b2 * 64 + lane) * 4);
+      const float* part = w ? sqk : skk;
+      float nk = 0.f, nq = 0.f;
+      f32x4 z = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        nk += snk[(b2 * 4 + i) * C + m];
+        nq += snq[(b2 * 4 + i) * C + m];
+        z += *reinterpret_cast<const f32x4*>(part + ((b2 * 4 + i) * 64 + lane) * 4);
+      }
+      const float* fg = sg + b2 * 4 * C + m;
+      const double kn = 1. / sqrt((double)nk + (double)unit_eps);
+      float* f = sc + b2 * 6 * C + m;
+      float* tb = sT + b2 * C * PP;
+      double zd[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) zd[e] = (double)z[e] * ((double)dm[e] * kn);
+      if (w) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) sA[(b2 * C + 4 * gg + e) * PP + m] = 4 * gg + e >= m ? (float)zd[e] : 0.f;
+        f[0] = (float)(fg[0] * kn);
+        f[C] = (float)(fg[C] * kn);
+        f[2 * C] = fg[0];
+        f[3 * C] = (float)((double)q_scale / sqrt((double)nq + (double)unit_eps));
+        f[4 * C] = fg[3 * C];
+        f[5 * C] = fg[2 * C];
+      } else {
+        const float beta = fg[2 * C];
+        const double rw = beta * kn;
+        const int b8 = m & 8, cc = m & 7;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) tb[(4 * gg + e) * PP + m] = (float)(zd[e] * __shfl(rw, 4 * gg + e, 64));
+        lds_wave_sync();
+        f32x4 l[8][2];      // rows of this lane's diagonal block
+#pragma unroll
+        for (int t = 1; t < 8; ++t) {
+          l[t][0] = *reinterpret_cast<const f32x4*>(tb + (b8 + t) * PP + b8);
+          if (t > 4) l[t][1] = *reinterpret_cast<const f32x4*>(tb + (b8 + t) * PP + b8 + 4);
+        }
+        f32x4 l21 = {0.f, 0.f, 0.f, 0.f};
+        if (m >= 8 && gg < 2) l21 = *reinterpret_cast<const f32x4*>(tb + m * PP + 4 * gg);
+        lds_wave_sync();
+        float x[8];
+#pragma unroll
+        for (int t = 0; t < 8; ++t) {
+          x[t] = t == cc ? 1.f : 0.f;
+#pragma unroll
+          for (int j = 0; j < t; ++j) x[t] = fmaf(-l[t][j >> 2][j & 3], x[j], x[t]);
+          tb[(b8 + t) * PP + m] = x[t];
+          tb[((b8 ^ 8) + t) * PP + m] = 0.f;
+        }
+        lds_wave_sync();
+        const f32x4 ta = *reinterpret_cast<const f32x4*>(tb + m * PP + 4 * gg);
+        float tc[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) tc[e] = tb[(4 * gg + e) * PP + m];
+        f32x4 y = {0.f, 0.f, 0.f, 0.f}, y2 = y;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) y = mfma_f32(l21[e], tc[e], y);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) y2 = mfma_f32(ta[e], y[e], y2);
+        lds_wave_sync();
+#pragma unroll
+        for (int e = 0; e < 4; ++e) tb[(4 * gg + e) * PP + m] = 4 * gg + e > m ? (tc[e] - y2[e]) * beta : 0.f;
+      }
+    }
+    __syncthreads();
+  }
+}
+
 // threads of a one-row workgroup: about four elements per thread, whole waves, at most 1024
 int row_threads(int W) { return std::min(1024, std::max(64, (W / 4 + 63) / 64 * 64)); }
 
@@ -559,11 +936,46 @@ void launch_short_conv_state_update(const void* z, long z_ld, float* state, cons
                                                               positions, C, n);
 }
 
+template <typename T, int NT>
+static void delta_chunk_launch(const float* q, long q_ld, const float* k, long k_ld, const float* v, long v_ld, const T* b,
+                               long b_ld, const T* a, long a_ld, const float* a_log, const float* dt_bias, float* state,
+                               const int* state_slots, const int* row_cu, int nseq, const int* positions, float q_scale,
+                               float unit_eps, float* o, int H, int G, int D, int Dv, hipStream_t s) {
+  constexpr int C = 16;
+  constexpr size_t lds = (size_t)(6 * C * (16 * NT + 4) + 18 * 256 + 24 * C + 4 * C * (C + 4) + 16 * C) * sizeof(float);
+  static bool once = false;
+  if (!once) {
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&delta_chunk_kernel<T, NT>),
+                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    once = true;
+  }
+  // 1: rows of q and k, 2: columns of the state in four-element accesses
+  int vec = 0;
+  if (D % 4 == 0 && rows_aligned(q, q_ld, 4) && rows_aligned(k, k_ld, 4)) vec |= 1;
+  if (D % 4 == 0) vec |= 2;
+  dim3 grid(nseq, H, (Dv + 63) / 64);
+  delta_chunk_kernel<T, NT><<<grid, 512, lds, s>>>(q, q_ld, k, k_ld, v, v_ld, b, b_ld, a, a_ld, a_log, dt_bias, state, state_slots,
+                                                   row_cu, positions, q_scale, unit_eps, vec, o, H, G, D, Dv);
+}
+
 template <typename T>
 static int delta_scan_t(const float* q, long q_ld, const float* k, long k_ld, const float* v, long v_ld, const T* b,
                         long b_ld, const T* a, long a_ld, const float* a_log, const float* dt_bias, float* state,
                         const int* state_slots, const int* row_cu, int nseq, const int* positions, float q_scale,
-                        float unit_eps, float* o, int H, int G, int D, int Dv, hipStream_t s) {
+                        float unit_eps, float* o, int T_, int H, int G, int D, int Dv, hipStream_t s) {
+  // Rows per sequence are not known here. Four rows for each of 16 sequences take 14 us row by row and 20 us in chunks (whose
+  // pipeline is three steps deep), 16 rows for each of eight 16 and 12; long prompts beside many single rows gain most.
+  if ((T_ >= 6 * nseq || T_ - nseq >= 256) && D <= 256) {
+#define BFLY_DCH(NT)                                                                                                    \
+  delta_chunk_launch<T, NT>(q, q_ld, k, k_ld, v, v_ld, b, b_ld, a, a_ld, a_log, dt_bias, state, state_slots, row_cu, nseq, \
+                            positions, q_scale, unit_eps, o, H, G, D, Dv, s)
+    if (D <= 64) BFLY_DCH(4);
+    else if (D <= 128) BFLY_DCH(8);
+    else if (D <= 192) BFLY_DCH(12);
+    else BFLY_DCH(16);
+#undef BFLY_DCH
+    return 0;
+  }
   dim3 grid(nseq, H, (Dv + 63) / 64);
 #define BFLY_DELTA(NR)                                                                                             \
   delta_scan_kernel<T, NR><<<grid, 512, 0, s>>>(q, q_ld, k, k_ld, v, v_ld, b, b_ld, a, a_ld, a_log, dt_bias, state, \
@@ -584,9 +996,9 @@ int launch_delta_scan(const float* q, long q_ld, const float* k, long k_ld, cons
   if (T <= 0 || nseq <= 0) return 0;
   if (f32)
     return delta_scan_t<float>(q, q_ld, k, k_ld, v, v_ld, (const float*)b, b_ld, (const float*)a, a_ld, a_log, dt_bias,
-                               state, state_slots, row_cu, nseq, positions, q_scale, unit_eps, o, H, G, D, Dv, s);
+                               state, state_slots, row_cu, nseq, positions, q_scale, unit_eps, o, T, H, G, D, Dv, s);
   return delta_scan_t<bf16>(q, q_ld, k, k_ld, v, v_ld, (const bf16*)b, b_ld, (const bf16*)a, a_ld, a_log, dt_bias, state,
-                            state_slots, row_cu, nseq, positions, q_scale, unit_eps, o, H, G, D, Dv, s);
+                            state_slots, row_cu, nseq, positions, q_scale, unit_eps, o, T, H, G, D, Dv, s);
 }
 
 }  // namespace bfly

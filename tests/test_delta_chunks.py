@@ -1,0 +1,51 @@
+"""The gated delta rule over prompt rows (chunks of 16 on the f32 matrix cores) against a float64 token loop."""
+import pytest
+import torch
+
+from butterfly_amd import ops
+
+F64 = torch.float64
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])      # (of the logits)
+@pytest.mark.parametrize("H,G,D,Dv,seqs", [
+    (4, 2, 128, 128, [(0, 17), (5, 16), (0, 1), (3, 2)]),       # chunk edges; fresh and continued sequences; one row beside prompts
+    (3, 1, 24, 40, [(0, 33)]), (2, 2, 64, 64, [(7, 15), (0, 48)]),
+    (2, 1, 70, 70, [(0, 31), (9, 32)]),                           # rows that are not a multiple of four elements
+    (1, 1, 150, 96, [(0, 40)]), (2, 1, 256, 128, [(1, 100)]), (1, 1, 96, 256, [(0, 300), (0, 3)]),
+])
+def test_prompt_chunks_match_the_token_loop(dt, H, G, D, Dv, seqs):
+    g = torch.Generator().manual_seed(D + Dv)
+    T, nslots = sum(n for _, n in seqs), len(seqs) + 1
+    rnd = lambda *s: torch.randn(*s, generator=g)            # noqa: E731
+    q, k, v = rnd(T, G, D), rnd(T, G, D), rnd(T, H, Dv)
+    k[1::5] = k[0::5][:len(k[1::5])]                        # the same key again at once: the strongest coupling inside a chunk
+    k[2::7] *= 1e-3
+    b, a = (1 + 3 * rnd(T, H)).to(dt), rnd(T, H).to(dt)
+    a[3::9] += 40.0                                         # rows that forget everything, and rows that forget nothing
+    a[4::3] -= 40.0
+    a_log, dt_bias = rnd(H) - 1, rnd(H)
+    st = rnd(nslots, H, Dv, D)
+    slots = torch.randperm(nslots, generator=g)[:len(seqs)].int()
+    cu = torch.tensor([sum(n for _, n in seqs[:i]) for i in range(len(seqs) + 1)], dtype=torch.int32)
+    pos = torch.cat([torch.arange(s, s + n) for s, n in seqs]).int()
+    unit = lambda x: (x / torch.sqrt((x * x).sum(-1, keepdim=True) + 1e-6)).repeat_interleave(H // G, 1)      # noqa: E731
+    qu, ku = unit(q.to(F64)) * D ** -0.5, unit(k.to(F64))
+    beta = torch.sigmoid(b.to(F64))
+    decay = torch.exp(-torch.exp(a_log.to(F64)) * torch.nn.functional.softplus(a.to(F64) + dt_bias.to(F64)))
+    want, state = torch.empty(T, H, Dv, dtype=F64), st.to(F64).clone()
+    for s, (start, n) in enumerate(seqs):
+        m = state[slots[s]] if start else torch.zeros(H, Dv, D, dtype=F64)
+        for t in range(int(cu[s]), int(cu[s]) + n):
+            m = decay[t][:, None, None] * m
+            u = beta[t][:, None] * (v[t].to(F64) - (m @ ku[t][:, :, None])[:, :, 0])
+            m = m + u[:, :, None] * ku[t][:, None]
+            want[t] = (m @ qu[t][:, :, None])[:, :, 0]
+        state[slots[s]] = m
+    d = lambda t: t.to("cuda")                             # noqa: E731
+    sd = d(st)
+    o = ops.delta_scan(d(q), d(k), d(v), d(b), d(a), d(a_log), d(dt_bias), sd, d(slots), d(cu), d(pos), D ** -0.5, 1e-6)
+    # f32 sums of up to 256 channels, a solve of up to 16 coupled rows, products of 16 decays (f32 eps 6e-8 each)
+    for got, ref in ((o, want), (sd, state)):
+        assert (got.cpu().to(F64) - ref).abs().max() < 5e-6 * ref.abs().max()
