@@ -407,14 +407,17 @@ void moe_glu_ffn(const Tensor& x, const Tensor& topk_ids, const Tensor& topk_w, 
   const bool big = bfly::moe_big_ok(x.data_ptr(), x.stride(0), gate_up_w.data_ptr(), down_w.data_ptr(), hmid.data_ptr(),
                                     y.data_ptr(), (int)T, (int)TK, (int)Hd, (int)F, plain_act != bfly::ACT_NONE, f32);
   const int tr = bfly::moe_tile_rows((int)TK, (int)E, f32, big, (int)Hd);
-  const int64_t gt = tr > 64 ? (TK + tr - 1) / tr + E : mt;      // tiles that this tile height can need
+  const bool stream = tr == 64 && bfly::moe_stream_ok(x.data_ptr(), x.stride(0), gate_up_w.data_ptr(), down_w.data_ptr(),
+                                                      hmid.data_ptr(), y.data_ptr(), (int)TK, (int)E, (int)Hd, (int)F, f32);
+  // tiles that this tile height can need (no more than rows)
+  const int64_t gt = std::min(TK, tr > 64 ? (TK + tr - 1) / tr + E : mt);
   bfly::launch_moe_sort(topk_ids.data_ptr<int>(), (int)TK, (int)E, perm, offsets, tiles, ntiles, tr, s);
   // scores on the expert's input (the row is scaled and the outputs are summed) or on its output
   bfly::launch_moe_glu_up(x.data_ptr(), x.stride(0), scale_input ? topk_w.data_ptr<float>() : nullptr, (int)K, perm,
                           offsets, tiles, ntiles, (int)gt, gate_up_w.data_ptr(), (float)limit, (float)alpha,
-                          (float)up_offset, hmid.data_ptr(), (int)Hd, (int)F, f32, tr, s, (int)plain_act);
+                          (float)up_offset, hmid.data_ptr(), (int)Hd, (int)F, f32, tr, s, (int)plain_act, stream);
   bfly::launch_moe_down(hmid.data_ptr(), perm, offsets, tiles, ntiles, (int)gt, down_w.data_ptr(), y.data_ptr<float>(),
-                        (int)Hd, (int)F, f32, tr, s);
+                        (int)Hd, (int)F, f32, tr, s, stream);
   bfly::launch_moe_sum(y.data_ptr<float>(), scale_input ? nullptr : topk_w.data_ptr<float>(), (int)K, out.data_ptr(),
                        (int)T, (int)Hd, f32, s, addp, (long)add_ld, identity ? topk_ids.data_ptr<int>() : nullptr, (int)E,
                        identity ? x.data_ptr() : nullptr, (long)x.stride(0));

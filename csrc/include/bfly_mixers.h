@@ -139,16 +139,21 @@ int moe_tile_rows(int TK, int E, bool f32, bool big, int Hd);
 // column tiles without a remainder. plain: experts without a gate
 bool moe_big_ok(const void* x, long ldx, const void* gate_up_w, const void* down_w, const void* hmid, const void* y, int T,
                 int TK, int Hd, int F, bool plain, bool f32);
+// whether few rows per expert go through the kernels that stream the weights past them (tiles of 64 rows): bf16, 16-byte
+// aligned rows, K steps and column tiles without a remainder
+bool moe_stream_ok(const void* x, long ldx, const void* gate_up_w, const void* down_w, const void* hmid, const void* y,
+                   int TK, int E, int Hd, int F, bool f32);
 // hmid[r, f] = g' sigmoid(alpha g') (u' + up_offset), (g', u') the clamped gate / up products of
 // expert e(r) on (w x) for grouped row r (topk_w == nullptr: on x itself). plain_act != ACT_NONE: experts
 // without a gate, gate_up_w [E, F, Hd] and hmid = act(up product) (ACT_RELU2)
 void launch_moe_glu_up(const void* x, long ldx, const float* topk_w, int K, const int* perm, const int* offsets,
                        const int* tiles, const int* ntiles, int max_tiles, const void* gate_up_w, float limit,
                        float alpha, float up_offset, void* hmid, int Hd, int F, bool f32, int tile_rows, hipStream_t s,
-                       int plain_act = ACT_NONE);
+                       int plain_act = ACT_NONE, bool stream = false);
 // y[perm[r], :] = down_e(r) hmid[r]     (y f32, pair order)
 void launch_moe_down(const void* hmid, const int* perm, const int* offsets, const int* tiles, const int* ntiles,
-                     int max_tiles, const void* down_w, float* y, int Hd, int F, bool f32, int tile_rows, hipStream_t s);
+                     int max_tiles, const void* down_w, float* y, int Hd, int F, bool f32, int tile_rows, hipStream_t s,
+                     bool stream = false);
 // out[t] = sum_j wts[t * K + j] y[t * K + j] (+ add[t], rows of stride add_ld)   (wts == nullptr: the plain sum).
 // ids (nullable, with wts): where ids[t * K + j] >= E, x[t] stands in for y[t * K + j]
 void launch_moe_sum(const float* y, const float* wts, int K, void* out, int T, int Hd, bool f32, hipStream_t s,

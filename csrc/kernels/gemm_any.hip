@@ -547,7 +547,7 @@ using BTile = bf16[2][(1 + PN) * 32 * WT][MLD];
 // rowX(r) / rowW(p, c) give the r-th X row / c-th row of panel p. VEC, SC and the two K steps in flight as in
 // tile_mac_f32 (a scaled row is rounded to bf16). Small groups are bound by the latency of their weight stream:
 // with branches around the loads and one step in flight, 16 tokens through 8 experts of 2048 (width 2048, 134 MB of gate
-// and up rows) took 63 us in the gate / up product and 33 in the down product, now 41 and 24.
+// and up rows) took 63 us in the gate / up product and 33 in the down product, then 41 and 24 (few rows: moe_stream_ok).
 template <int WT, int PN, bool VEC, bool SC, typename FX, typename FW>
 __device__ __forceinline__ void tile_mac_mfma(f32x4 (&acc)[PN][WT][WT], FX rowX, FW rowW, int K, BTile<WT, PN>& S) {
   constexpr int NS = WT / 2, BT = 32 * WT, PF = WT == 2 ? 2 : 1;      // staged rows per thread and operand; steps in flight
@@ -737,6 +737,140 @@ __global__ __launch_bounds__(256) void moe_down_mfma_kernel(const bf16* __restri
   });
 }
 
+// Experts over few rows: the weights of an expert stream past its rows once, straight into MFMA operands, nothing staged.
+// Workgroup = (16 columns of two weight panels, tile of up to 64 rows), four waves that take 64-element chunks of the K
+// dimension in turn (chunk c: wave c % 4) and keep U of them in flight, then sum their parts in LDS. The panels are gate and up
+// rows of the same columns, or (plain experts, down product) neighbouring columns. The order of a sum depends on K alone.
+// Such groups are bound by the latency of the weight stream: a 64 x 64 tile has a quarter as many workgroups, a barrier per
+// step and two steps in flight. One token through 2 of 8 experts (width 2048, GLU of 2048): 48 -> 22 us for the whole op.
+template <int RT, int U, bool SC>
+__device__ __forceinline__ void stream_chunks(f32x4 (&acc)[2][RT], const bf16* w0, const bf16* w1, const bf16* const (&xr)[RT],
+                                              const float (&sx)[RT], long k) {
+  bf16x8 a[U][2][2], b[U][RT][2];
+#pragma unroll
+  for (int u = 0; u < U; ++u)
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      a[u][0][h] = *reinterpret_cast<const bf16x8*>(w0 + k + 256 * u + 32 * h);
+      a[u][1][h] = *reinterpret_cast<const bf16x8*>(w1 + k + 256 * u + 32 * h);
+    }
+#pragma unroll
+  for (int u = 0; u < U; ++u)
+#pragma unroll
+    for (int t = 0; t < RT; ++t)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) b[u][t][h] = *reinterpret_cast<const bf16x8*>(xr[t] + k + 256 * u + 32 * h);
+#pragma unroll
+  for (int u = 0; u < U; ++u)
+#pragma unroll
+    for (int t = 0; t < RT; ++t)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        if (SC) {      // the expert's input row: the token row times its routing score, rounded to bf16
+#pragma unroll
+          for (int j = 0; j < 8; ++j) b[u][t][h][j] = (bf16)((float)b[u][t][h][j] * sx[t]);
+        }
+        acc[0][t] = mfma16(a[u][0][h], b[u][t][h], acc[0][t]);
+        acc[1][t] = mfma16(a[u][1][h], b[u][t][h], acc[1][t]);
+      }
+}
+
+// part[wave][panel][row tile][lane]: element i of a lane is (column 4 * (lane >> 4) + i, row 16 t + (lane & 15))
+template <int RT, bool SC, typename FX>
+__device__ __forceinline__ void stream_rows(f32x4* part, const bf16* w0, const bf16* w1, FX rowX, int K) {
+  constexpr int U = RT == 1 ? 4 : RT == 2 ? 2 : 1;
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, n = K / 64;
+  const bf16* xr[RT];
+  float sx[RT];
+#pragma unroll
+  for (int t = 0; t < RT; ++t) {
+    const RowRef r = rowX(16 * t + (lane & 15));
+    xr[t] = r.p + 8 * (lane >> 4);
+    sx[t] = r.s;
+  }
+  f32x4 acc[2][RT] = {};
+  int c = wave;
+  for (; c + 4 * (U - 1) < n; c += 4 * U) stream_chunks<RT, U, SC>(acc, w0, w1, xr, sx, 64L * c);
+  for (; c < n; c += 4) stream_chunks<RT, 1, SC>(acc, w0, w1, xr, sx, 64L * c);
+#pragma unroll
+  for (int p = 0; p < 2; ++p)
+#pragma unroll
+    for (int t = 0; t < RT; ++t) part[((wave * 2 + p) * 4 + t) * 64 + lane] = acc[p][t];
+}
+
+template <bool SC, typename FX>
+__device__ __forceinline__ void stream_tile(f32x4* part, const bf16* w0, const bf16* w1, FX rowX, int rows, int K) {
+  if (rows <= 16) stream_rows<1, SC>(part, w0, w1, rowX, K);
+  else if (rows <= 32) stream_rows<2, SC>(part, w0, w1, rowX, K);
+  else stream_rows<4, SC>(part, w0, w1, rowX, K);
+  __syncthreads();
+}
+// sums of the four waves' parts for row tile t
+__device__ __forceinline__ f32x4 stream_sum(const f32x4* part, int p, int t, int lane) {
+  const f32x4* q = part + (p * 4 + t) * 64 + lane;
+  return (q[0] + q[512]) + (q[1024] + q[1536]);
+}
+
+__global__ __launch_bounds__(256) void moe_up_stream_kernel(const bf16* __restrict__ x, long ldx,
+                                                            const float* __restrict__ topk_w, int Kc,
+                                                            const int* __restrict__ perm, const int* __restrict__ offsets_e,
+                                                            const int* __restrict__ tiles, const int* __restrict__ ntiles,
+                                                            const bf16* __restrict__ gu_w, float limit, float alpha,
+                                                            float up_offset, bf16* __restrict__ hmid, int Hd, int F,
+                                                            int plain) {
+  if ((int)blockIdx.y >= ntiles[0]) return;
+  __shared__ f32x4 part[4 * 2 * 4 * 64];
+  const int e = tiles[2 * blockIdx.y], r0 = tiles[2 * blockIdx.y + 1];
+  const int rows = min(64, offsets_e[e + 1] - r0);
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int col0 = blockIdx.x * (plain ? 32 : 16), dp = plain ? 16 : F;      // rows from the first panel to the second
+  const bf16* w0 = gu_w + ((long)e * (plain ? 1 : 2) * F + col0 + (lane & 15)) * Hd + 8 * (lane >> 4);
+  const bf16* w1 = w0 + (long)dp * Hd;
+  auto rowX = [&](int r) {      // (rows past the group: its last row again, never stored)
+    const int p = perm[r0 + min(r, rows - 1)];
+    return RowRef{x + (long)(p / Kc) * ldx, topk_w ? topk_w[p] : 1.f};
+  };
+  if (topk_w) stream_tile<true>(part, w0, w1, rowX, rows, Hd);
+  else stream_tile<false>(part, w0, w1, rowX, rows, Hd);
+  const int r = 16 * wave + (lane & 15);
+  if (r >= rows) return;
+  const f32x4 g = stream_sum(part, 0, wave, lane), u = stream_sum(part, 1, wave, lane);
+  bf16* out = hmid + (long)(r0 + r) * F + col0 + 4 * (lane >> 4);
+  bf16x4 o, o2;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    if (plain) {
+      o[i] = (bf16)apply_act(g[i], plain, 0.f, 0.f);
+      o2[i] = (bf16)apply_act(u[i], plain, 0.f, 0.f);
+    } else {
+      const float gg = fminf(g[i], limit), uu = fminf(fmaxf(u[i], -limit), limit);
+      o[i] = (bf16)(glu_gate(gg, alpha, expf(-alpha * gg)) * (uu + up_offset));
+    }
+  }
+  *reinterpret_cast<bf16x4*>(out) = o;
+  if (plain) *reinterpret_cast<bf16x4*>(out + 16) = o2;
+}
+
+__global__ __launch_bounds__(256) void moe_down_stream_kernel(const bf16* __restrict__ hmid, const int* __restrict__ perm,
+                                                              const int* __restrict__ offsets_e,
+                                                              const int* __restrict__ tiles, const int* __restrict__ ntiles,
+                                                              const bf16* __restrict__ down_w, float* __restrict__ y, int Hd,
+                                                              int F) {
+  if ((int)blockIdx.y >= ntiles[0]) return;
+  __shared__ f32x4 part[4 * 2 * 4 * 64];
+  const int e = tiles[2 * blockIdx.y], r0 = tiles[2 * blockIdx.y + 1];
+  const int rows = min(64, offsets_e[e + 1] - r0);
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, col0 = blockIdx.x * 32;
+  const bf16* w0 = down_w + ((long)e * Hd + col0 + (lane & 15)) * F + 8 * (lane >> 4);
+  auto rowX = [&](int r) { return RowRef{hmid + (long)(r0 + min(r, rows - 1)) * F, 1.f}; };
+  stream_tile<false>(part, w0, w0 + 16L * F, rowX, rows, F);
+  const int r = 16 * wave + (lane & 15);
+  if (r >= rows) return;
+  float* out = y + (long)perm[r0 + r] * Hd + col0 + 4 * (lane >> 4);
+  *reinterpret_cast<f32x4*>(out) = stream_sum(part, 0, wave, lane);
+  *reinterpret_cast<f32x4*>(out + 16) = stream_sum(part, 1, wave, lane);
+}
+
 // rows of `ld` elements of es bytes that allow 16-byte accesses everywhere
 inline bool rows16(const void* p, long ld, int es) { return ld * es % 16 == 0 && reinterpret_cast<uintptr_t>(p) % 16 == 0; }
 
@@ -828,6 +962,16 @@ int moe_tile_rows(int TKp, int E, bool f32, bool big, int Hd) {
   return (!f32 && TKp >= 512 * E) ? 128 : 64;
 }
 
+// Up to an average of 24 rows per expert (12 from width 4096 on) the weights stream past the rows. Whole op, 8 experts, two
+// choices, us of 64-row tiles -> streams: width 2048, GLU of 2048: 1 token 48 -> 22, 16 tokens 53 -> 49, 64 tokens (16 rows
+// per expert) 56 -> 53, but 128 tokens 57 -> 67; width 1024, 1024: 31 -> 15, 32 -> 20, 35 -> 24; width 4096, plain 6144: 16
+// tokens 202 -> 169, but 64 tokens 205 -> 216.
+bool moe_stream_ok(const void* x, long ldx, const void* gate_up_w, const void* down_w, const void* hmid, const void* y,
+                   int TKp, int E, int Hd, int F, bool f32) {
+  return !f32 && TKp <= (Hd >= 4096 ? 12 : 24) * E && Hd % 64 == 0 && F % 64 == 0 && rows16(x, ldx, 2) &&
+         rows16(gate_up_w, Hd, 2) && rows16(down_w, F, 2) && rows16(hmid, F, 2) && rows16(y, Hd, 4);
+}
+
 void launch_moe_sort(const int* ids, int TKp, int E, int* perm, int* offsets, int* tiles, int* ntiles, int tile_rows,
                      hipStream_t s) {
   moe_sort_kernel<<<1, 1024, 0, s>>>(ids, TKp, E, perm, offsets, tiles, ntiles, tile_rows);
@@ -836,7 +980,13 @@ void launch_moe_sort(const int* ids, int TKp, int E, int* perm, int* offsets, in
 void launch_moe_glu_up(const void* x, long ldx, const float* topk_w, int K, const int* perm, const int* offsets,
                        const int* tiles, const int* ntiles, int max_tiles, const void* gate_up_w, float limit,
                        float alpha, float up_offset, void* hmid, int Hd, int F, bool f32, int tile_rows, hipStream_t s,
-                       int plain_act) {
+                       int plain_act, bool stream) {
+  if (stream) {
+    moe_up_stream_kernel<<<dim3(F / (plain_act != ACT_NONE ? 32 : 16), max_tiles), 256, 0, s>>>(
+        (const bf16*)x, ldx, topk_w, K, perm, offsets, tiles, ntiles, (const bf16*)gate_up_w, limit, alpha, up_offset,
+        (bf16*)hmid, Hd, F, plain_act);
+    return;
+  }
   if (tile_rows == 256) {
     ExpertArgs ex;
     ex.perm = perm; ex.offsets = offsets; ex.tiles = tiles; ex.topk_w = topk_w; ex.choices = K;
@@ -861,7 +1011,13 @@ void launch_moe_glu_up(const void* x, long ldx, const float* topk_w, int K, cons
 }
 
 void launch_moe_down(const void* hmid, const int* perm, const int* offsets, const int* tiles, const int* ntiles,
-                     int max_tiles, const void* down_w, float* y, int Hd, int F, bool f32, int tile_rows, hipStream_t s) {
+                     int max_tiles, const void* down_w, float* y, int Hd, int F, bool f32, int tile_rows, hipStream_t s,
+                     bool stream) {
+  if (stream) {
+    moe_down_stream_kernel<<<dim3(Hd / 32, max_tiles), 256, 0, s>>>((const bf16*)hmid, perm, offsets, tiles, ntiles,
+                                                                    (const bf16*)down_w, y, Hd, F);
+    return;
+  }
   if (tile_rows == 256) {
     ExpertArgs ex;
     ex.perm = perm; ex.offsets = offsets; ex.tiles = tiles; ex.y = y;

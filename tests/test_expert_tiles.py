@@ -59,3 +59,30 @@ def test_experts_over_row_groups(counts, Hd, F, plain, scaled, limit, stride):
     # squared activation can double
     err = (got.cpu().to(F64) - want).norm() / want.norm()
     assert err < 2.0 ** -7
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("counts,Hd,F,plain,scaled", [
+    ([1, 0, 0, 0], 64, 64, False, True),                 # one row, one K step
+    ([16, 17, 1, 0], 320, 64, False, True),              # edges of the row tiles; fewer K steps than a wave keeps in flight
+    ([32, 33, 0, 3], 1088, 192, False, False),           # two and four row tiles; a remainder of the K steps
+    ([64, 5, 2, 1], 256, 320, True, False),              # a whole tile; plain experts
+    ([65, 4, 1, 1], 512, 64, True, True),                # one row in a second tile
+])
+def test_experts_over_few_rows(counts, Hd, F, plain, scaled):
+    """Weights streamed past the rows; rows of x with a stride, an addend, ids that name no expert here."""
+    g = torch.Generator().manual_seed(sum(counts) + F)
+    E, TK = len(counts), sum(counts)
+    flat = torch.cat([torch.full((c,), e) for e, c in enumerate(counts)])[torch.randperm(TK, generator=g)]
+    ids = flat.view(-1, 1)
+    bf = lambda *s, k=1.0: (k * torch.randn(*s, generator=g)).to(torch.bfloat16)            # noqa: E731
+    x, add, w = bf(TK, Hd + 8)[:, :Hd], bf(TK, Hd), torch.rand(TK, 1, generator=g) + 0.2
+    gu, dn = bf(E, F if plain else 2 * F, Hd, k=2 * Hd ** -0.5), bf(E, Hd, F, k=F ** -0.5)
+    d = lambda t: t.to("cuda")                                                           # noqa: E731
+    xd = torch.empty(TK, Hd + 8, dtype=torch.bfloat16, device="cuda")[:, :Hd].copy_(x)
+    got = ops.moe_glu_ffn(xd, d(ids.int()), d(w), d(gu), d(dn), 7.0, 1.702, 1.0, scaled, "relu2" if plain else None,
+                          addend=d(add))
+    want = reference(x.to(F64), ids, w.to(F64), gu.to(F64), dn.to(F64), 7.0, 1.702, 1.0, scaled, plain) + add.to(F64)
+    # bf16 input rows times their score, hidden rows and output (2^-9 each); the squared activation doubles the first
+    err = (got.cpu().to(F64) - want).norm() / want.norm()
+    assert err < 6e-3
