@@ -1758,15 +1758,24 @@ static GemmPlan plan_gemm_heuristic(int M, int N, int K) {
   if (M > 256 && (N % 256 == 0 || (N % 128 == 0 && N > 1024)) && K % 64 == 0) {
     // prefill / large batch: the 256x256 one-wave-per-SIMD tile (gemm_big4_kernel: 1.52-1.55
     // PF at M = 8192 on the 70B projections, 6-10 % over the 8-phase gemm_big8_kernel and ahead
-    // of it at M = 256-2048 too, profiles/r5_gemm_big4/); split K only when the tile grid cannot
-    // fill the 256 CUs
+    // of it at M = 256-2048 too, profiles/r5_gemm_big4/). Split K where that pays for the partial sums it writes and
+    // reads, in units of a K step of 64 (1.5 us): rounds of 256 workgroups times (steps + 8 for the pipeline's ends), plus
+    // 0.07 per tile and split for the sums. Splitting until the tiles outnumber the CUs instead: 6184 x 2048 x 2048 (two
+    // splits, now one) 100 -> 58 us, 3000 x 4096 x 14336 339 -> 268, 600 x 4096 x 4096 (8, now 4) 60 -> 42, 8192 x 1024 x 1024
+    // 46 -> 31; 700 x 2048 x 8192 keeps 8 (45)
     p.kind = 6;
     p.mt = 0;
     p.bm = p.bn = 256;
     const int tiles = ((M + 255) / 256) * ((N + 255) / 256);
-    int sk = 1;
-    while (tiles * sk < 256 && K / 64 >= sk * 2 * 8 && sk < 8) sk *= 2;
-    p.sk = sk;
+    p.sk = 1;
+    double best = 0;
+    for (int sk = 1; sk <= 8 && (sk == 1 || K / 64 >= sk * 8); sk *= 2) {
+      const double t = (double)((tiles * sk + 255) / 256) * ((double)K / 64 / sk + 8) + (sk > 1 ? 0.07 * tiles * sk : 0);
+      if (sk == 1 || t < best) {
+        best = t;
+        p.sk = sk;
+      }
+    }
     return p;
   }
   p.kind = 1;
