@@ -938,17 +938,22 @@ def moe_route_scores(x, wr, top_k: int, scoring: str = "softmax", renorm: bool =
     if not _gpu(x):
         return ref.moe_route_scores(x, wr, top_k, scoring, renorm, bias, select_bias, groups, renorm_eps, scale)
     T = x.shape[0]
+    ids = _empty(T, top_k, dtype=torch.int32, device=x.device)
+    w = _empty(T, top_k, dtype=torch.float32, device=x.device)
+    rest = (bias, top_k, {"softmax": 0, "sigmoid": 1}[scoring], bool(renorm), ids, w, select_bias, int(groups[0]),
+            int(groups[1]), float(renorm_eps), float(scale))
+    E = wr.shape[0]
+    if E <= 32 and T <= 256:      # a few rows: logits and choice in one launch
+        torch.ops.bfly.moe_route_rows(x, wr, *rest)
+        return ids, w
     # logits: up to 64 experts one wave per token (steps of a few rows: per token and expert), beyond that a
     # GEMM with f32 accumulation and f32 output; then one wave per token picks
-    if T * wr.shape[0] <= 4096 or wr.shape[0] <= 64:
-        logits = _empty(T, wr.shape[0], dtype=torch.float32, device=x.device)
+    if T * E <= 4096 or E <= 64:
+        logits = _empty(T, E, dtype=torch.float32, device=x.device)
         torch.ops.bfly.router_logits(x, wr, logits)
     else:
         logits = linear_act(x, wr, out_dtype=torch.float32)
-    ids = _empty(T, top_k, dtype=torch.int32, device=x.device)
-    w = _empty(T, top_k, dtype=torch.float32, device=x.device)
-    torch.ops.bfly.moe_topk_scores(logits, bias, top_k, {"softmax": 0, "sigmoid": 1}[scoring], bool(renorm), ids, w,
-                                   select_bias, int(groups[0]), int(groups[1]), float(renorm_eps), float(scale))
+    torch.ops.bfly.moe_topk_scores(logits, *rest)
     return ids, w
 
 

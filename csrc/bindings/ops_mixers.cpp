@@ -338,31 +338,53 @@ void router_logits(const Tensor& x, const Tensor& wr, Tensor& logits) {
                              is_f32(x), cur_stream());
 }
 
-void moe_topk_scores(const Tensor& logits, const optional<Tensor>& bias, int64_t top_k, int64_t scoring, bool renorm,
-                     Tensor& ids, Tensor& w, const optional<Tensor>& select_bias, int64_t ngroups, int64_t keep,
-                     double renorm_eps, double scale) {
-  CHK_GPU(logits); CHK_F32(logits); CHK_I32(ids); CHK_F32(w);
-  const float* bp = nullptr;
+struct Choice {
+  const float *bias = nullptr, *sel = nullptr;
+};
+static Choice choice_args(int64_t T, int64_t E, const optional<Tensor>& bias, int64_t top_k, const Tensor& ids, const Tensor& w,
+                          const optional<Tensor>& select_bias, int64_t ngroups, int64_t keep) {
+  CHK_I32(ids); CHK_F32(w);
+  Choice c;
   if (bias.has_value()) {
     CHK_F32(*bias);
-    TORCH_CHECK(bias->numel() == logits.size(1), "moe_topk_scores: bias [E]");
-    bp = bias->data_ptr<float>();
+    TORCH_CHECK(bias->numel() == E, "moe_topk_scores: bias [E]");
+    c.bias = bias->data_ptr<float>();
   }
-  const float* sbp = nullptr;
   if (select_bias.has_value()) {
     CHK_F32(*select_bias);
-    TORCH_CHECK(select_bias->is_cuda() && select_bias->numel() == logits.size(1), "moe_topk_scores: select_bias [E]");
-    sbp = select_bias->data_ptr<float>();
+    TORCH_CHECK(select_bias->is_cuda() && select_bias->numel() == E, "moe_topk_scores: select_bias [E]");
+    c.sel = select_bias->data_ptr<float>();
   }
-  TORCH_CHECK(logits.dim() == 2, "moe_topk_scores: logits [T, E]");
-  const int64_t T = logits.size(0), E = logits.size(1);
   TORCH_CHECK(E >= 1 && E <= 1024 && top_k >= 1 && top_k <= E, "moe_topk_scores: experts / top_k");
   TORCH_CHECK(ids.numel() == T * top_k && w.numel() == T * top_k, "moe_topk_scores: outputs");
   TORCH_CHECK(ngroups >= 1 && keep >= 1 && keep <= ngroups && E % ngroups == 0 && top_k <= E / ngroups * keep,
               "moe_topk_scores: groups");
-  bfly::launch_moe_topk_scores(logits.data_ptr<float>(), bp, (int)top_k, (int)scoring, renorm, ids.data_ptr<int>(),
-                               w.data_ptr<float>(), (int)T, (int)E, cur_stream(), sbp, (int)ngroups, (int)keep, (float)renorm_eps,
-                               (float)scale);
+  return c;
+}
+
+void moe_topk_scores(const Tensor& logits, const optional<Tensor>& bias, int64_t top_k, int64_t scoring, bool renorm,
+                     Tensor& ids, Tensor& w, const optional<Tensor>& select_bias, int64_t ngroups, int64_t keep,
+                     double renorm_eps, double scale) {
+  CHK_GPU(logits); CHK_F32(logits);
+  TORCH_CHECK(logits.dim() == 2, "moe_topk_scores: logits [T, E]");
+  const int64_t T = logits.size(0), E = logits.size(1);
+  const Choice c = choice_args(T, E, bias, top_k, ids, w, select_bias, ngroups, keep);
+  bfly::launch_moe_topk_scores(logits.data_ptr<float>(), c.bias, (int)top_k, (int)scoring, renorm, ids.data_ptr<int>(),
+                               w.data_ptr<float>(), (int)T, (int)E, cur_stream(), c.sel, (int)ngroups, (int)keep,
+                               (float)renorm_eps, (float)scale);
+}
+
+void moe_route_rows(const Tensor& x, const Tensor& wr, const optional<Tensor>& bias, int64_t top_k, int64_t scoring, bool renorm,
+                    Tensor& ids, Tensor& w, const optional<Tensor>& select_bias, int64_t ngroups, int64_t keep,
+                    double renorm_eps, double scale) {
+  CHK_GPU(x); CHK_SAME(x, wr);
+  TORCH_CHECK(x.dim() == 2 && x.stride(1) == 1 && wr.dim() == 2 && wr.is_contiguous(), "moe_route_rows: layouts");
+  const int64_t T = x.size(0), Hd = x.size(1), E = wr.size(0);
+  TORCH_CHECK(wr.size(1) == Hd && E <= 64, "moe_route_rows: router [E <= 64, H]");
+  const Choice c = choice_args(T, E, bias, top_k, ids, w, select_bias, ngroups, keep);
+  bfly::launch_route_rows(x.data_ptr(), x.stride(0), wr.data_ptr(), (int)Hd, c.bias, (int)top_k, (int)scoring, renorm,
+                          ids.data_ptr<int>(), w.data_ptr<float>(), (int)T, (int)E, is_f32(x), cur_stream(), c.sel,
+                          (int)ngroups, (int)keep, (float)renorm_eps, (float)scale);
 }
 
 int64_t moe_sort_max_tiles(int64_t TK, int64_t E) { return bfly::moe_sort_max_tiles((int)TK, (int)E); }
@@ -459,6 +481,8 @@ TORCH_LIBRARY_FRAGMENT(bfly, m) {
   m.def("router_logits(Tensor x, Tensor wr, Tensor(a!) logits) -> ()");
   m.def("moe_topk_scores(Tensor logits, Tensor? bias, int top_k, int scoring, bool renorm, Tensor(a!) ids, "
         "Tensor(b!) w, Tensor? select_bias=None, int ngroups=1, int keep=1, float renorm_eps=0.0, float scale=1.0) -> ()");
+  m.def("moe_route_rows(Tensor x, Tensor wr, Tensor? bias, int top_k, int scoring, bool renorm, Tensor(a!) ids, "
+        "Tensor(b!) w, Tensor? select_bias=None, int ngroups=1, int keep=1, float renorm_eps=0.0, float scale=1.0) -> ()");
   m.def("moe_sort_max_tiles(int tk, int experts) -> int", &moe_sort_max_tiles);
   m.def("moe_glu_ffn(Tensor x, Tensor topk_ids, Tensor topk_w, Tensor gate_up_w, Tensor down_w, float limit, "
         "float alpha, float up_offset, bool scale_input, Tensor(a!) work, Tensor(b!) hmid, Tensor(c!) y, "
@@ -482,5 +506,6 @@ TORCH_LIBRARY_IMPL(bfly, CUDA, m) {
   m.impl("gla_out", &gla_out);
   m.impl("router_logits", &router_logits);
   m.impl("moe_topk_scores", &moe_topk_scores);
+  m.impl("moe_route_rows", &moe_route_rows);
   m.impl("moe_glu_ffn", &moe_glu_ffn);
 }

@@ -127,6 +127,10 @@ void launch_router_logits(const void* x, long ldx, const void* wr, float* logits
 void launch_moe_topk_scores(const float* logits, const float* bias, int top_k, int scoring, bool renorm, int* ids,
                             float* w, int T, int E, hipStream_t s, const float* select_bias = nullptr, int ngroups = 1,
                             int keep = 1, float renorm_eps = 0.f, float scale = 1.f);
+// both in one launch, for steps of a few rows and E <= 64
+void launch_route_rows(const void* x, long ldx, const void* wr, int Hd, const float* bias, int top_k, int scoring, bool renorm,
+                       int* ids, float* w, int T, int E, bool f32, hipStream_t s, const float* select_bias = nullptr,
+                       int ngroups = 1, int keep = 1, float renorm_eps = 0.f, float scale = 1.f);
 // Group the T*K (token, choice) pairs by expert: perm [TK] pair indices grouped by expert,
 // offsets [E + 1], tiles [max_tiles][2] = (expert, first row) of every tile_rows-row tile, ntiles [1].
 void launch_moe_sort(const int* ids, int TK, int E, int* perm, int* offsets, int* tiles, int* ntiles, int tile_rows,

@@ -358,17 +358,10 @@ __global__ __launch_bounds__(256) void moe_sum4_kernel(const float* __restrict__
   }
 }
 
-// Router logits of a small step (a few rows): one wave per (token, expert), lanes split the
-// hidden dim, f32 accumulation. Large steps use the f32-output GEMM instead.
-// V = 8: eight elements per access (Hd and ldx multiples of 8, aligned rows).
+// <x row, router row> by one wave: lanes split the hidden dim, f32 accumulation. V = 8: eight elements per access (Hd and
+// the row strides multiples of 8, aligned rows).
 template <typename T, int V>
-__global__ __launch_bounds__(256) void router_logits_kernel(const T* __restrict__ x, long ldx,
-                                                            const T* __restrict__ wr, float* __restrict__ logits,
-                                                            int E, int Hd) {
-  const int t = blockIdx.x, e = blockIdx.y * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
-  if (e >= E) return;
-  const T* xr = x + (long)t * ldx;
-  const T* w = wr + (long)e * Hd;
+__device__ __forceinline__ float router_dot(const T* __restrict__ xr, const T* __restrict__ w, int Hd, int lane) {
   float a = 0.f;
   if (V > 1) {
     typedef T tv __attribute__((ext_vector_type(V)));
@@ -386,7 +379,17 @@ __global__ __launch_bounds__(256) void router_logits_kernel(const T* __restrict_
   } else {
     for (int k = lane; k < Hd; k += 64) a = fmaf(ldf(xr + k), ldf(w + k), a);
   }
-  a = wave_sum(a);
+  return wave_sum(a);
+}
+
+// Router logits of a small step (a few rows): one wave per (token, expert). Large steps use the f32-output GEMM instead.
+template <typename T, int V>
+__global__ __launch_bounds__(256) void router_logits_kernel(const T* __restrict__ x, long ldx,
+                                                            const T* __restrict__ wr, float* __restrict__ logits,
+                                                            int E, int Hd) {
+  const int t = blockIdx.x, e = blockIdx.y * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+  if (e >= E) return;
+  const float a = router_dot<T, V>(x + (long)t * ldx, wr + (long)e * Hd, Hd, lane);
   if (lane == 0) logits[(long)t * E + e] = a;
 }
 
@@ -420,18 +423,29 @@ __global__ __launch_bounds__(256) void router_rows_kernel(const T* __restrict__ 
   }
 }
 
-// Router choice of one token per wave from its f32 logits [E]: softmax or sigmoid scores, K rounds
-// of arg-max over the experts (ties to the lowest id). ngroups > keep: first the `keep` groups (of E / ngroups
+// orders one wave's LDS accesses: what its lanes wrote before is what they read after
+__device__ __forceinline__ void wave_order() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+// Router choice of token t by one wave from its f32 logits sc [E] (LDS, with their bias): softmax or sigmoid scores, K
+// rounds of arg-max over the experts (ties to the lowest id). ngroups > keep: first the `keep` groups (of E / ngroups
 // neighbours) with the largest choice score in them are found the same way, the others' members drop out.
-__global__ __launch_bounds__(64) void moe_topk_scores_kernel(const float* __restrict__ logits,
-                                                             const float* __restrict__ bias, int top_k, int scoring,
-                                                             int renorm, int* __restrict__ ids, float* __restrict__ w,
-                                                             int E, const float* __restrict__ sel, int ngroups, int keep,
-                                                             float renorm_eps, float scale) {
-  __shared__ float sc[1024], raw[1024], best[1024];
-  const int t = blockIdx.x, lane = threadIdx.x;
-  for (int e = lane; e < E; e += 64) sc[e] = logits[(long)t * E + e] + (bias ? bias[e] : 0.f);
-  __syncthreads();
+struct ChoiceArgs {
+  const float* bias;
+  const float* sel;
+  int* ids;
+  float* w;
+  int top_k, scoring, renorm, E, ngroups, keep;
+  float renorm_eps, scale;
+};
+__device__ __forceinline__ void choose_experts(const ChoiceArgs& c, int t, int lane, float* sc, float* raw, float* best) {
+  const int E = c.E, top_k = c.top_k, scoring = c.scoring, renorm = c.renorm, ngroups = c.ngroups, keep = c.keep;
+  const float renorm_eps = c.renorm_eps, scale = c.scale;
+  const float* sel = c.sel;
+  int* ids = c.ids;
+  float* w = c.w;
   if (scoring == 0) {
     float mx = -INFINITY;
     for (int e = lane; e < E; e += 64) mx = fmaxf(mx, sc[e]);
@@ -439,18 +453,18 @@ __global__ __launch_bounds__(64) void moe_topk_scores_kernel(const float* __rest
     float den = 0.f;
     for (int e = lane; e < E; e += 64) den += expf(sc[e] - mx);
     den = wave_sum(den);
-    __syncthreads();
+    wave_order();
     for (int e = lane; e < E; e += 64) sc[e] = expf(sc[e] - mx) / den;
   } else {
     for (int e = lane; e < E; e += 64) sc[e] = 1.f / (1.f + expf(-sc[e]));
   }
-  __syncthreads();
+  wave_order();
   if (sel) {      // the choice is made among score + sel; the weight is the plain score
     for (int e = lane; e < E; e += 64) {
       raw[e] = sc[e];
       sc[e] += sel[e];
     }
-    __syncthreads();
+    wave_order();
   }
   if (keep < ngroups) {
     const int gsz = E / ngroups;
@@ -459,7 +473,7 @@ __global__ __launch_bounds__(64) void moe_topk_scores_kernel(const float* __rest
       for (int e = 1; e < gsz; ++e) m = fmaxf(m, sc[g * gsz + e]);
       best[g] = m;
     }
-    __syncthreads();
+    wave_order();
     for (int k = 0; k < keep; ++k) {
       float bv = -INFINITY;
       int bi = 0x7fffffff;
@@ -471,13 +485,13 @@ __global__ __launch_bounds__(64) void moe_topk_scores_kernel(const float* __rest
         const int oi = __shfl_xor(bi, o, 64);
         if (ov > bv || (ov == bv && oi < bi)) { bv = ov; bi = oi; }
       }
-      __syncthreads();
+      wave_order();
       if (lane == 0 && bi < ngroups) best[bi] = -INFINITY;      // kept: it leaves the race
-      __syncthreads();
+      wave_order();
     }
     for (int e = lane; e < E; e += 64)
       if (best[e / gsz] != -INFINITY) sc[e] = -INFINITY;
-    __syncthreads();
+    wave_order();
   }
   float sum = 0.f;
   for (int k = 0; k < top_k; ++k) {
@@ -501,12 +515,36 @@ __global__ __launch_bounds__(64) void moe_topk_scores_kernel(const float* __rest
       w[(long)t * top_k + k] = ok ? bv : 0.f;
       if (ok) sc[bi] = -INFINITY;
     }
-    __syncthreads();
+    wave_order();
   }
   if (lane == 0 && (renorm || scale != 1.f)) {
     const float den = renorm ? sum + renorm_eps : 1.f;
     for (int k = 0; k < top_k; ++k) w[(long)t * top_k + k] = w[(long)t * top_k + k] / den * scale;
   }
+}
+
+__global__ __launch_bounds__(64) void moe_topk_scores_kernel(const float* __restrict__ logits, ChoiceArgs c) {
+  __shared__ float sc[1024], raw[1024], best[1024];
+  const int t = blockIdx.x, lane = threadIdx.x;
+  for (int e = lane; e < c.E; e += 64) sc[e] = logits[(long)t * c.E + e] + (c.bias ? c.bias[e] : 0.f);
+  wave_order();
+  choose_experts(c, t, lane, sc, raw, best);
+}
+
+// Logits and choice of a small step in one launch: workgroup = token, a wave per expert (in turn), then the first wave
+// chooses. Both parts are bound by latency (two
+// launches of 4.6 us for 16 tokens, 8 experts of width 2048): about 2 us less per layer of a decode step.
+template <typename T, int V>
+__global__ __launch_bounds__(1024) void route_rows_kernel(const T* __restrict__ x, long ldx, const T* __restrict__ wr, int Hd,
+                                                          ChoiceArgs c) {
+  __shared__ float sc[64], raw[64], best[64];
+  const int t = blockIdx.x, lane = threadIdx.x & 63, nw = blockDim.x >> 6;
+  for (int e = threadIdx.x >> 6; e < c.E; e += nw) {
+    const float a = router_dot<T, V>(x + (long)t * ldx, wr + (long)e * Hd, Hd, lane);
+    if (lane == 0) sc[e] = a + (c.bias ? c.bias[e] : 0.f);
+  }
+  __syncthreads();
+  if (threadIdx.x < 64) choose_experts(c, t, lane, sc, raw, best);
 }
 
 // ---------------------------------------------------------------------------------------
@@ -933,8 +971,23 @@ void launch_moe_topk_scores(const float* logits, const float* bias, int top_k, i
                             float* w, int T, int E, hipStream_t s, const float* select_bias, int ngroups, int keep,
                             float renorm_eps, float scale) {
   if (T <= 0) return;
-  moe_topk_scores_kernel<<<T, 64, 0, s>>>(logits, bias, top_k, scoring, renorm, ids, w, E, select_bias, ngroups, keep,
-                                          renorm_eps, scale);
+  const ChoiceArgs c{bias, select_bias, ids, w, top_k, scoring, renorm, E, ngroups, keep, renorm_eps, scale};
+  moe_topk_scores_kernel<<<T, 64, 0, s>>>(logits, c);
+}
+
+void launch_route_rows(const void* x, long ldx, const void* wr, int Hd, const float* bias, int top_k, int scoring, bool renorm,
+                       int* ids, float* w, int T, int E, bool f32, hipStream_t s, const float* select_bias, int ngroups,
+                       int keep, float renorm_eps, float scale) {
+  if (T <= 0) return;
+  const ChoiceArgs c{bias, select_bias, ids, w, top_k, scoring, renorm, E, ngroups, keep, renorm_eps, scale};
+  const size_t al = f32 ? 32 : 16;
+  const bool vec = Hd % 8 == 0 && ldx % 8 == 0 && reinterpret_cast<uintptr_t>(x) % al == 0 &&
+                   reinterpret_cast<uintptr_t>(wr) % al == 0;
+  const int nt = 64 * std::min(E, 16);
+#define BFLY_RR(TT, V) route_rows_kernel<TT, V><<<T, nt, 0, s>>>((const TT*)x, ldx, (const TT*)wr, Hd, c)
+  if (f32) { if (vec) BFLY_RR(float, 8); else BFLY_RR(float, 1); }
+  else { if (vec) BFLY_RR(bf16, 8); else BFLY_RR(bf16, 1); }
+#undef BFLY_RR
 }
 
 int moe_sort_max_tiles(int TKp, int E) { return (TKp + 63) / 64 + E; }
