@@ -1755,7 +1755,8 @@ static GemmPlan plan_gemm_heuristic(int M, int N, int K) {
   }
   // N % 256 == 128: a last column tile whose right half is wasted, 1 / 9 of the work at most; 8192 x 8320 x 2048 388 us on
   // 128 x 128 tiles -> 271 us, 6184 x 6272 x 2048 172 -> 159 us
-  if (M > 256 && (N % 256 == 0 || (N % 128 == 0 && N > 1024)) && K % 64 == 0) {
+  // (a single K step, K = 64, is left to the tiles below: this kernel's pipeline needs two)
+  if (M > 256 && (N % 256 == 0 || (N % 128 == 0 && N > 1024)) && K % 64 == 0 && K >= 128) {
     // prefill / large batch: the 256x256 one-wave-per-SIMD tile (gemm_big4_kernel: 1.52-1.55
     // PF at M = 8192 on the 70B projections, 6-10 % over the 8-phase gemm_big8_kernel and ahead
     // of it at M = 256-2048 too, profiles/r5_gemm_big4/). Split K where that pays for the partial sums it writes and
