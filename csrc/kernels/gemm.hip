@@ -31,6 +31,7 @@
 //    distinct bank slots; bijective XCD-aware tile remap (T1).
 #include "bfly_common.h"
 
+#include <algorithm>
 #include <cstdio>
 #include <string>
 #include <vector>
@@ -1734,6 +1735,25 @@ GemmPlan plan_gemm(int M, int N, int K) {
   return plan_gemm_heuristic(M, N, K);
 }
 
+// LDS-tiled kernel: 16 to 128 rows per tile, split K until the grid has `target` workgroups
+static GemmPlan plan_tile(int M, int N, int K) {
+  GemmPlan p{};
+  const int target = 448;
+  p.kind = 1;
+  p.mt = M >= 512 ? 2 : 3;   // tile plans: `mt` = pipeline depth (K-tiles in flight + 1)
+  if (M <= 16) { p.bm = 16; p.wk = 1; }
+  else if (M <= 32) { p.bm = 32; p.wk = 1; }
+  else if (M <= 64) { p.bm = 64; p.wk = 2; }
+  else { p.bm = 128; p.wk = 2; }
+  p.bn = 128;
+  const int tiles = ((M + p.bm - 1) / p.bm) * (N / p.bn);
+  int sk = 1;
+  const int ktiles = K / kBK;
+  while (tiles * sk < target && sk * 2 * 4 <= ktiles && sk < 16) sk *= 2;
+  p.sk = sk;
+  return p;
+}
+
 static GemmPlan plan_gemm_heuristic(int M, int N, int K) {
   GemmPlan p{};
   const int target = 448;
@@ -1779,30 +1799,21 @@ static GemmPlan plan_gemm_heuristic(int M, int N, int K) {
     }
     return p;
   }
-  p.kind = 1;
-  p.mt = M >= 512 ? 2 : 3;   // tile plans: `mt` = pipeline depth (K-tiles in flight + 1)
-  if (M <= 16) { p.bm = 16; p.wk = 1; }
-  else if (M <= 32) { p.bm = 32; p.wk = 1; }
-  else if (M <= 64) { p.bm = 64; p.wk = 2; }
-  else { p.bm = 128; p.wk = 2; }
-  p.bn = 128;
-  const int tiles = ((M + p.bm - 1) / p.bm) * (N / p.bn);
-  int sk = 1;
-  const int ktiles = K / kBK;
-  while (tiles * sk < target && sk * 2 * 4 <= ktiles && sk < 16) sk *= 2;
-  p.sk = sk;
-  return p;
+  return plan_tile(M, N, K);
 }
 
 static size_t plan_ws_bytes(const GemmPlan& p, int M, int N) {
   return p.sk > 1 ? kCounterBytes + (size_t)p.sk * M * N * sizeof(float) : 0;
 }
 
-// Enough for the tuned plan and for the heuristic plan it may fall back to (below).
+// A row scale with a half column tile: the 256 x 256 tile's epilogue has none, the 128-row tiles' has
+static bool rowscale_on_tile(const GemmPlan& p, int N) { return p.kind == 6 && N % 256 != 0; }
+
+// Enough for the tuned plan and for the plans it may fall back to (below).
 size_t gemm_workspace_bytes(int M, int N, int K) {
-  const size_t a = plan_ws_bytes(plan_gemm(M, N, K), M, N);
-  const size_t b = plan_ws_bytes(plan_gemm_heuristic(M, N, K), M, N);
-  return a > b ? a : b;
+  const GemmPlan h = plan_gemm_heuristic(M, N, K);
+  const size_t a = plan_ws_bytes(plan_gemm(M, N, K), M, N), b = plan_ws_bytes(h, M, N);
+  return std::max({a, b, rowscale_on_tile(h, N) ? plan_ws_bytes(plan_tile(M, N, K), M, N) : 0});
 }
 
 // `dry`: validate only (the plan is supported for this shape/epilogue) without launching.
@@ -1955,18 +1966,18 @@ int launch_gemm_plan(const GemmPlan& p, const bf16* X, long ldx, const bf16* W, 
 }
 
 // The plan for this call: the tuned/heuristic plan, or the heuristic one when a table entry
-// measured for another epilogue cannot run this one (e.g. odd skinny NT with SiLU).
-static GemmPlan select_plan(int M, int N, int K, int epi) {
+// measured for another epilogue cannot run this one (e.g. odd skinny NT with SiLU), or the tile plan for a row scale.
+static GemmPlan select_plan(int M, int N, int K, int epi, bool row_scale = false) {
   GemmPlan p = plan_gemm(M, N, K);
   if (run_plan(p, nullptr, 0, nullptr, 0, M, N, K, epi, nullptr, nullptr, 0, nullptr, nullptr, true) != 0)
     p = plan_gemm_heuristic(M, N, K);
-  return p;
+  return row_scale && rowscale_on_tile(p, N) ? plan_tile(M, N, K) : p;
 }
 
 int gemm_rowscale_check(int M, int N, int K, int epi) {
   if (M <= 0) return 0;
   const RowScale probe{nullptr, 0, 0.f, 0.f};
-  return run_plan(select_plan(M, N, K, epi), nullptr, 0, nullptr, 0, M, N, K, epi, nullptr, nullptr, 0,
+  return run_plan(select_plan(M, N, K, epi, true), nullptr, 0, nullptr, 0, M, N, K, epi, nullptr, nullptr, 0,
                   nullptr, nullptr, true, false, &probe);
 }
 
@@ -2065,7 +2076,7 @@ int launch_gemm_deferred(const bf16* X, long ldx, const bf16* W, long ldw, int M
                          bf16* out, long ldo, float* ws, size_t ws_bytes, hipStream_t stream,
                          const RowScale* rs) {
   if (M <= 0) return 1;
-  GemmPlan p = select_plan(M, N, K, EPI_NONE);
+  GemmPlan p = select_plan(M, N, K, EPI_NONE, rs != nullptr);
   if (p.sk > 1 && (ws == nullptr || ws_bytes < kCounterBytes + (size_t)p.sk * M * N * sizeof(float)))
     p.sk = 1;
   const bool defer = p.sk > 1;
@@ -2089,7 +2100,7 @@ int launch_gemm(const bf16* X, long ldx, const bf16* W, long ldw, int M, int N, 
                 const bf16* bias, bf16* out, long ldo, float* ws, size_t ws_bytes,
                 hipStream_t stream, const RowScale* rs) {
   if (M <= 0) return 0;
-  GemmPlan p = select_plan(M, N, K, epi);
+  GemmPlan p = select_plan(M, N, K, epi, rs != nullptr);
   if (p.sk > 1 && (ws == nullptr || ws_bytes < kCounterBytes + (size_t)p.sk * M * N * sizeof(float)))
     p.sk = 1;
   return run_plan(p, X, ldx, W, ldw, M, N, K, epi, bias, out, ldo, ws, stream, false, false, rs);

@@ -1,5 +1,6 @@
-"""Split-K choice of the 256 x 256 prefill tile."""
+"""Plans of the prefill GEMM: splits of the 256 x 256 tile, half column tiles, row scales."""
 import pytest
+import torch
 
 from butterfly_amd import ops
 
@@ -23,8 +24,36 @@ def test_splits_pay_for_their_sums(K, N):
 @pytest.mark.parametrize("N", [128, 256, 1024, 1152, 1408, 2048, 8320])
 def test_every_row_count_has_a_plan_that_runs(K, N):
     """One K step, whole and half column tiles: the plan chosen is one that its kernel takes."""
-    import torch
-
     for M in (1, 16, 64, 200, 256, 257, 300, 512, 1000, 5000):
         for epi in ("none", "bias", "silu", "relu2"):
             assert torch.ops.bfly.gemm_check(M, N, K, ops.EPILOGUES[epi]) == 0, (M, N, K, epi)
+
+
+HALF = [(300, 1152, 1024), (512, 1152, 1024), (1000, 1408, 4096), (5000, 8320, 256)]
+
+
+@pytest.mark.parametrize("M,N,K", HALF + [(257, 1152, 64)])
+def test_half_column_tiles_take_a_row_scale(M, N, K):
+    for epi in ("none", "bias", "silu"):
+        assert torch.ops.bfly.gemm_rowscale_check(M, N, K, ops.EPILOGUES[epi]) == 0, epi
+    assert torch.ops.bfly.gemm_rowscale_check(512, 2048, K, 0) != 0 or K == 64      # whole column tiles: as ever
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", HALF)
+@pytest.mark.parametrize("how", ["bias", "silu", "defer"])
+def test_row_scaled_product_with_a_half_column_tile(M, N, K, how):
+    g = torch.Generator().manual_seed(M + N)
+    x, w = torch.randn(M, K, generator=g).bfloat16().cuda(), (torch.randn(N, K, generator=g) * K ** -0.5).bfloat16().cuda()
+    b = torch.randn(N, generator=g).bfloat16().cuda() if how == "bias" else None
+    ssp = torch.rand(M, 3, generator=g).cuda() * K
+    y = ops.linear(ops.RowNormed(x, ssp, 1e-5), w, bias=b, epilogue="silu" if how == "silu" else "none", defer=how == "defer")
+    got = ops.materialize(y).cpu().double()
+    want = (x.double() @ w.double().T * torch.rsqrt(ssp.double().sum(1, keepdim=True) / K + 1e-5)).cpu()
+    if b is not None:
+        want += b.cpu().double()
+    if how == "silu":
+        u = want.view(M, N // 32, 2, 16)
+        want = (torch.nn.functional.silu(u[:, :, 0]) * u[:, :, 1]).reshape(M, N // 2)
+    # one rounding to bf16 (2^-9) of f32 sums of unit-sized products
+    assert ((got - want).abs() < 2.0 ** -8 * want.abs() + 1e-4).all()
