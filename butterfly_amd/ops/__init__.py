@@ -176,12 +176,12 @@ def reserve_workspace(device, max_tokens: int, max_n: int, max_k: int, max_batch
     """Pre-size every workspace for problems up to the given bounds (call before capture).
     `shapes`: the model's GEMM weight shapes (N, K); the split-K slab need is the max over them
     and every token-count bucket of the plan table (a tuned plan may split a small projection
-    more than the largest one is split)."""
+    more than the largest one is split) and every number of row tiles (a split's sums do not grow with the rows)."""
     if not load_library():
         return
     ws = 0
     nk = {(int(max_n), int(max_k))} | {(int(n), int(k)) for n, k in shapes}
-    for m in sorted({1, 16, 32, 48, 64, 128, 256, 512, max_tokens}):
+    for m in sorted({1, 16, 32, 48, 64, *range(128, max_tokens, 128), max_tokens}):
         if m > max_tokens:
             continue
         for n, k in nk:

@@ -1780,18 +1780,22 @@ static GemmPlan plan_gemm_heuristic(int M, int N, int K) {
     // prefill / large batch: the 256x256 one-wave-per-SIMD tile (gemm_big4_kernel: 1.52-1.55
     // PF at M = 8192 on the 70B projections, 6-10 % over the 8-phase gemm_big8_kernel and ahead
     // of it at M = 256-2048 too, profiles/r5_gemm_big4/). Split K where that pays for the partial sums it writes and
-    // reads, in units of a K step of 64 (1.5 us): rounds of 256 workgroups times (steps + 8 for the pipeline's ends), plus
-    // 0.07 per tile and split for the sums. Splitting until the tiles outnumber the CUs instead: 6184 x 2048 x 2048 (two
-    // splits, now one) 100 -> 58 us, 3000 x 4096 x 14336 339 -> 268, 600 x 4096 x 4096 (8, now 4) 60 -> 42, 8192 x 1024 x 1024
-    // 46 -> 31; 700 x 2048 x 8192 keeps 8 (45)
+    // reads, in units of a K step of 64 (1.15 us): rounds of 256 workgroups times (steps + 8 for the pipeline's ends), plus
+    // 0.07 per tile and split for the sums, twice that beyond 512 of them (128 MB no longer stay in the cache). Over
+    // 261 shapes of 10 to 3584 tiles the choice is never slower than splitting until the tiles outnumber the CUs. Unsplit, two
+    // and four splits, us: 2300 x 8192 x 8192 (288 tiles) 314, 340, 395; 2300 x 8192 x 28672 1096, 948, 913; 4337 x 8192 x 28672
+    // (544) 1754, 1672, 1685; 1800 x 4096 x 14336 (128) 246, 177, 209; 520 x 4096 x 4096 (48) 75, 53, 42; 6600 x 4096 x 14336
+    // (416) 589, 689, 730. At most 1024 tiles of partial sums: 256 MB of workspace, and a need that grows with whole
+    // tiles only (ops.reserve_workspace).
     p.kind = 6;
     p.mt = 0;
     p.bm = p.bn = 256;
-    const int tiles = ((M + 255) / 256) * ((N + 255) / 256);
+    const int tiles = ((M + 255) / 256) * ((N + 255) / 256), steps = K / 64;
     p.sk = 1;
     double best = 0;
-    for (int sk = 1; sk <= 8 && (sk == 1 || K / 64 >= sk * 8); sk *= 2) {
-      const double t = (double)((tiles * sk + 255) / 256) * ((double)K / 64 / sk + 8) + (sk > 1 ? 0.07 * tiles * sk : 0);
+    for (int sk = 1; sk <= 8 && (sk == 1 || (steps >= sk * 8 && tiles * sk <= 1024)); sk *= 2) {
+      const double sums = sk == 1 ? 0 : (tiles * sk <= 512 ? 0.07 : 0.14) * tiles * sk;
+      const double t = (double)((tiles * sk + 255) / 256) * ((double)steps / sk + 8) + sums;
       if (sk == 1 || t < best) {
         best = t;
         p.sk = sk;

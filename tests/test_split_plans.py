@@ -29,6 +29,37 @@ def test_every_row_count_has_a_plan_that_runs(K, N):
             assert torch.ops.bfly.gemm_check(M, N, K, ops.EPILOGUES[epi]) == 0, (M, N, K, epi)
 
 
+LLAMA = [(6144, 4096), (4096, 4096), (28672, 4096), (4096, 14336), (10240, 8192), (8192, 8192), (57344, 8192), (8192, 28672),
+         (2560, 28672), (1152, 4096), (8320, 2048)]
+
+
+def test_partial_sums_are_bounded_and_reserved(monkeypatch):
+    """No plan of a prefill step needs more than 256 MB of partial sums, and none more than what is reserved before serving
+    (an outgrown workspace is kept, a captured graph may still use it)."""
+    monkeypatch.setattr(ops, "_arena", ops._Arena())
+    ops.reserve_workspace(torch.device("cpu"), 8192, *LLAMA[0], shapes=LLAMA)
+    have = 4 * next(b for k, b in ops._arena.bufs.items() if k[1] == "gemm").numel()
+    rows = sorted({1, 7, 64, 200, 256, 512, 8192, *range(257, 8192, 61), *range(256, 8192, 256)})
+    for N, K in LLAMA:
+        for M in rows:
+            need = torch.ops.bfly.gemm_workspace_size(M, N, K)
+            assert need <= have, (M, N, K, need, have)
+            assert need <= (256 << 20) + 4 * torch.ops.bfly.gemm_slab_offset(), (M, N, K, need)
+
+
+# us of one step with 1, 2, 4 and 8 splits (measured once; whatever a plan's clock or unit, the order is what counts)
+TIMED = {(2300, 8192, 8192): (314, 340, 395, 551), (2300, 10240, 8192): (320, 372, 461), (2300, 8192, 28672): (1096, 948, 913, 1029),
+         (520, 4096, 4096): (75, 53, 42, 57), (1100, 4096, 14336): (235, 148, 168, 174), (2300, 4096, 14336): (256, 304, 298, 353),
+         (1800, 4096, 14336): (246, 177, 209, 272), (3300, 2560, 28672): (505, 587, 490, 502), (2300, 2560, 28672): (492, 319, 336, 329)}
+
+
+@pytest.mark.parametrize("shape", TIMED)
+def test_split_is_near_the_fastest(shape):
+    t = TIMED[shape]
+    sk = ops.gemm_plan(*shape)["splitk"]
+    assert t[(1, 2, 4, 8).index(sk)] < 1.08 * min(t), (shape, sk)
+
+
 HALF = [(300, 1152, 1024), (512, 1152, 1024), (1000, 1408, 4096), (5000, 8320, 256)]
 
 
