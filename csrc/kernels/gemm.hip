@@ -1773,10 +1773,8 @@ static GemmPlan plan_gemm_heuristic(int M, int N, int K) {
     p.sk = sk;
     return p;
   }
-  // N % 256 == 128: a last column tile whose right half is wasted, 1 / 9 of the work at most; 8192 x 8320 x 2048 388 us on
-  // 128 x 128 tiles -> 271 us, 6184 x 6272 x 2048 172 -> 159 us
-  // (a single K step, K = 64, is left to the tiles below: this kernel's pipeline needs two)
-  if (M > 256 && (N % 256 == 0 || (N % 128 == 0 && N > 1024)) && K % 64 == 0 && K >= 128) {
+  // 256 x 256 tile from two K steps on (its pipeline's least)
+  if (M > 256 && N % 128 == 0 && K % 64 == 0 && K >= 128 && (N % 256 == 0 || (N > 1024 && K >= 256))) {
     // prefill / large batch: the 256x256 one-wave-per-SIMD tile (gemm_big4_kernel: 1.52-1.55
     // PF at M = 8192 on the 70B projections, 6-10 % over the 8-phase gemm_big8_kernel and ahead
     // of it at M = 256-2048 too, profiles/r5_gemm_big4/). Split K where that pays for the partial sums it writes and
@@ -1801,7 +1799,17 @@ static GemmPlan plan_gemm_heuristic(int M, int N, int K) {
         p.sk = sk;
       }
     }
-    return p;
+    if (N % 256 == 0) return p;
+    // N % 256 == 128: half of the last column tile is wasted and 128 x 128 tiles have four times as many workgroups, two of
+    // them per compute unit. Their time in us, by rounds of 512 workgroups: (steps per split + 5) a round, and 6 + 0.02 per
+    // tile and split for the sums of a split K; the unit above is 1.22 us here. Over 324 shapes of 300 to 8192 rows the choice
+    // takes at most 9 % more than the 128 x 128 tiles. 128 x 128 and 256 x 256 tiles, us: 8192 x 8320 x 2048 348 and 253, 6200 x
+    // 6272 x 2048 200 and 153, 1000 x 4224 x 1024 37 and 30; 300 x 1408 x 1024 15 and 24, 1838 x 4224 x 1024 24 and 31, 1838 x 8320
+    // x 4096 139 and 164. Below 256 channels the small tiles are ahead nearly everywhere (4000 x 1152 x 128 10 and 15).
+    const GemmPlan q = plan_tile(M, N, K);
+    const long wgs = (long)((M + 127) / 128) * (N / 128) * q.sk;
+    const double tq = (double)((wgs + 511) / 512) * ((double)steps / q.sk + 5) + (q.sk > 1 ? 6 + 0.02 * wgs : 0);
+    return tq <= 1.22 * best ? q : p;
   }
   return plan_tile(M, N, K);
 }

@@ -60,6 +60,19 @@ def test_split_is_near_the_fastest(shape):
     assert t[(1, 2, 4, 8).index(sk)] < 1.08 * min(t), (shape, sk)
 
 
+# us of one step on 128 x 128 tiles and on 256 x 256 tiles
+TIMED_HALF = {(300, 1408, 1024): (15, 24), (520, 1152, 128): (7, 14), (4000, 1152, 128): (10, 15), (1838, 4224, 1024): (24, 31),
+              (1838, 8320, 4096): (139, 164), (520, 6272, 2048): (35, 46), (8192, 8320, 2048): (348, 253),
+              (6200, 6272, 2048): (200, 153), (1000, 4224, 1024): (37, 30), (4000, 1408, 1024): (43, 30), (6200, 1152, 4096): (98, 79)}
+
+
+@pytest.mark.parametrize("shape", TIMED_HALF)
+def test_half_column_tiles_go_to_the_faster_tile(shape):
+    t = TIMED_HALF[shape]
+    big = ops.gemm_plan(*shape)["kind"] == "big4"
+    assert t[big] < 1.1 * min(t), (shape, big)
+
+
 HALF = [(300, 1152, 1024), (512, 1152, 1024), (1000, 1408, 4096), (5000, 8320, 256)]
 
 
