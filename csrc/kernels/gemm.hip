@@ -960,7 +960,10 @@ __device__ __forceinline__ void b4_dma(__amdgpu_buffer_rsrc_t r, char* lds, int 
 // [gate | up]), so the clamped GLU runs on a lane's own accumulators; an expert that runs on (score x row) scales
 // the accumulators by the score instead of rounding scaled rows. The down projection leaves f32 rows at their
 // (token, choice) pair. Measured beside the smaller tiles: moe_tile_rows.
-template <int GROUPED = 0>
+// BIAS: the bias epilogue with the columns' values read once for all rows. Read row by row in tile_epilogue, each load waited
+// for by the only wave of its SIMD, they took 13 to 50 us of a product; in an instance of its own because
+// the branch alone costs the other epilogues 3 us.
+template <int GROUPED = 0, bool BIAS = false>
 __global__ void __launch_bounds__(kB4Threads) __attribute__((amdgpu_waves_per_eu(1, 1)))
 gemm_big4_kernel(const bf16* __restrict__ X, long ldx, const bf16* __restrict__ W, long ldw,
                  int M, int N, int K, int epi, const bf16* __restrict__ bias,
@@ -1160,6 +1163,17 @@ gemm_big4_kernel(const bf16* __restrict__ X, long ldx, const bf16* __restrict__ 
     return;
   }
   if (n0 + wc * 128 >= N) return;     // the columns past N of a half tile (their weight rows read zeros)
+  if constexpr (BIAS) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      f32x4 b;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) b[r] = bf2f(bias[n0 + wc * 128 + 16 * j + 4 * fq + r]);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) acc[i][j] += b;
+    }
+    epi = EPI_NONE;
+  }
   tile_epilogue<8, 8>(acc, m0 + wr * 128, n0 + wc * 128, lane, M, N, epi, bias, out, ldo,
                       part ? part + (long)blockIdx.y * M * N + (long)m0 * N : nullptr, m0,
                       RowScale{nullptr, 0, 0.f, 0.f});
@@ -1620,13 +1634,18 @@ static void run_big4(const bf16* X, long ldx, const bf16* W, long ldw, int M, in
                      int epi, const bf16* bias, bf16* out, long ldo, float* ws, int sk, hipStream_t stream) {
   static bool attr_set = false;
   if (!attr_set) {
-    hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_big4_kernel<false>),
+    hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_big4_kernel<0>),
+                        hipFuncAttributeMaxDynamicSharedMemorySize, kB4LdsBytes);
+    hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_big4_kernel<0, true>),
                         hipFuncAttributeMaxDynamicSharedMemorySize, kB4LdsBytes);
     attr_set = true;
   }
   dim3 grid(((M + 255) / 256) * ((N + 255) / 256), sk);
   float* part = sk > 1 ? splitk_part(ws) : nullptr;
-  gemm_big4_kernel<false><<<grid, kB4Threads, kB4LdsBytes, stream>>>(X, ldx, W, ldw, M, N, K, epi, bias, out, ldo, part);
+  if (epi == EPI_BIAS && sk == 1)      // (with a split K the reduce adds the bias)
+    gemm_big4_kernel<0, true><<<grid, kB4Threads, kB4LdsBytes, stream>>>(X, ldx, W, ldw, M, N, K, epi, bias, out, ldo, nullptr);
+  else
+    gemm_big4_kernel<0><<<grid, kB4Threads, kB4LdsBytes, stream>>>(X, ldx, W, ldw, M, N, K, epi, bias, out, ldo, part);
 }
 
 template <int BM, int BN, int SA, int SB, bool PK = false>

@@ -57,7 +57,7 @@ def test_experts(T, E, Hd, F, plain):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("M,N,K", [(257, 1152, 64 * 4), (300, 1408, 128), (1000, 1152, 1024), (512, 8320, 256), (513, 1024 + 128, 64 * 9),
-                                   (300, 1152, 64), (700, 2048, 64)])      # (one K step: the 128-row tiles)
+                                   (300, 1152, 64), (700, 2048, 64), (520, 1024, 256), (300, 1152, 1024)])      # (one K step: the 128-row tiles)
 @pytest.mark.parametrize("bias", [False, True])
 def test_prefill_tile_with_half_a_column_tile(M, N, K, bias):
     g = torch.Generator().manual_seed(M + N)
