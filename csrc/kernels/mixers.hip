@@ -199,7 +199,7 @@ __global__ __launch_bounds__(256) void attn_window_f32_kernel(const float* __res
   extern __shared__ __attribute__((aligned(16))) float f32_smem[];
   float* Ks = f32_smem;                  // [2][BS][KP]
   float* Vs = Ks + 2 * BS * KP;          // [2][Dv][VP]
-  __shared__ int s_range[4][2];
+  __shared__ int s_range[4][2], s_odd[2];      // s_odd[b]: 1 + the last page in buffer b with a value that is no number
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, qr = lane & 15, gg = lane >> 4;
   int tile = (int)(gridDim.x - 1 - blockIdx.x);
   const int g = blockIdx.y, R = H / G;
@@ -236,6 +236,7 @@ __global__ __launch_bounds__(256) void attn_window_f32_kernel(const float* __res
     pmax = max(pmax, __shfl_xor(pmax, x, 64));
   }
   if (lane == 0) { s_range[wave][0] = pmin; s_range[wave][1] = pmax; }
+  if (tid < 2) s_odd[tid] = 0;
   f32x4 qf[DT];
 #pragma unroll
   for (int c = 0; c < DT; ++c) {
@@ -280,7 +281,14 @@ __global__ __launch_bounds__(256) void attn_window_f32_kernel(const float* __res
       const int idx = tid + 256 * i;
       *reinterpret_cast<f32x4*>(Vb + idx / 8 * VP + 4 * (idx & 7)) = vreg[i];
     }
+    float zero = 0.f;      // (x * 0 of an infinity or NaN is NaN)
+#pragma unroll
+    for (int i = 0; i < NVS; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) zero = fmaf(vreg[i][e], 0.f, zero);
+    if (zero != 0.f) s_odd[pi & 1] = pi + 1;
     __syncthreads();      // the page is in LDS; every wave has left the buffer written next
+    const bool odd = s_odd[pi & 1] == pi + 1;
     if (pi + 1 < npages) gload(pi + 1);
     const int j0 = page_of(pi) * BS;
     if (j0 > pmax || (j0 + BS <= wlo && j0 >= keep_first)) continue;      // no row of this wave sees the page
@@ -314,6 +322,26 @@ __global__ __launch_bounds__(256) void attn_window_f32_kernel(const float* __res
     for (int e = 0; e < 8; ++e) {
       sc[e] = expf(sc[e] - mn);      // exp(-inf) = 0 for masked keys
       l += sc[e];
+    }
+    if (odd) {
+#pragma unroll
+      for (int t = 0; t < DVT; ++t) o[t] *= corr;
+#pragma unroll 1
+      for (int j = 0; j < BS; ++j) {
+        float pe = sc[0];      // the weight of key j: element 4 (j >> 4) + (j & 3) of lane group (j >> 2) & 3
+#pragma unroll
+        for (int e = 1; e < 8; ++e) pe = e == (j >> 4) * 4 + (j & 3) ? sc[e] : pe;
+        pe = __shfl(pe, qr + 16 * ((j >> 2) & 3), 64);
+        const int ok = (int)((unsigned)(p - j0 - j) < span) | (int)(j0 + j < kept);
+#pragma unroll
+        for (int t = 0; t < DVT; ++t)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const float x = fmaf(pe, Vb[(16 * t + 4 * gg + i) * VP + j], o[t][i]);
+            o[t][i] = ok ? x : o[t][i];
+          }
+      }
+      continue;
     }
 #pragma unroll
     for (int t = 0; t < DVT; ++t) {

@@ -146,3 +146,36 @@ def test_decode_waves_and_splits(fp8, Hq, Hkv, ctx, max_ctx):
     got = ops.attn_decode(q.cuda(), kc.cuda(), vc.cuda(), tables.cuda(), torch.tensor(ctx, dtype=torch.int32).cuda(), scale, max_ctx)
     err = (got.cpu().to(F64) - torch.cat(want)).abs().max()
     assert err < 2.0 ** -8 * vc.float().abs().max() + 1e-3      # weights and output rounded to bf16
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("bad", [float("nan"), float("inf")])
+@pytest.mark.parametrize("H,G,D,Dv,window,keep,start,n", [
+    (8, 2, 128, 128, 1 << 30, 0, 0, 40),      # one tile, the last page partly used
+    (4, 4, 64, 64, 40, 3, 50, 200),           # a kept prefix, several tiles
+    (6, 1, 256, 192, 64, 0, 7, 90),
+])
+def test_keys_that_no_row_sees_do_not_count_in_f32(H, G, D, Dv, window, keep, start, n, bad):
+    """f32 prompts: what an earlier owner left in the unused rows of a page, and a value outside a row's window or after it,
+    reach no output; the rows that see such a value are no numbers."""
+    g = torch.Generator().manual_seed(H * D)
+    r = lambda *s: torch.randn(*s, generator=g)                                     # noqa: E731
+    L, scale = start + n, 1.0 / math.sqrt(D)
+    need = (L + BS - 1) // BS
+    order = torch.randperm(need, generator=g)
+    q, k, v = r(n, H, D), r(need * BS, G, D), r(need * BS, G, Dv)
+    pos = torch.arange(start, L)
+    k[L:], v[L:] = bad, bad
+    odd = start + n // 2
+    for hit in (False, True):
+        if hit:
+            v[odd] = bad
+        kc, vc = torch.empty(need, G, BS, D), torch.empty(need, G, Dv, BS)
+        kc[order], vc[order] = k.view(-1, BS, G, D).transpose(1, 2), v.view(-1, BS, G, Dv).permute(0, 2, 3, 1)
+        cu = torch.tensor([0, n], dtype=torch.int32)
+        got = ops.attn_window_paged(q.cuda(), kc.cuda(), vc.cuda(), order.int()[None].cuda(), cu.cuda(), pos.int().cuda(), scale,
+                                    window, keep, None).cpu()
+        sees = (pos >= odd) & (pos - odd < window) if hit else torch.zeros(n, dtype=torch.bool)
+        want = dense(q.to(F64), k[:L].to(F64), v[:L].nan_to_num(0, 0, 0).to(F64), pos, scale, window, keep, None, None, 0, None)
+        assert (got[~sees].to(F64) - want[~sees]).abs().max() < 1e-5 * 5
+        assert not got[sees].isfinite().any()
