@@ -881,7 +881,8 @@ __global__ __launch_bounds__(512, NT <= 4 ? 4 : 2) void delta_chunk_kernel(
         z += *reinterpret_cast<const f32x4*>(part + ((b2 * 4 + i) * 64 + lane) * 4);
       }
       const float* fg = sg + b2 * 4 * C + m;
-      const double kn = 1. / sqrt((double)nk + (double)unit_eps);
+      // (rows past the sequence: no key, also where unit_eps is 0)
+      const double kn = r0 + (p - 1) * C + m < r1 ? 1. / sqrt((double)nk + (double)unit_eps) : 0.;
       float* f = sc + b2 * 6 * C + m;
       float* tb = sT + b2 * C * PP;
       double zd[4];

@@ -7,6 +7,33 @@ from butterfly_amd import ops
 F64 = torch.float64
 
 
+def step(seqs, H, G, D, Dv, seed, dt=torch.float32):
+    """Inputs of one step over sequences (first position, rows): delta_scan's arguments up to the positions, on the CPU."""
+    g = torch.Generator().manual_seed(seed)
+    T, n = sum(n for _, n in seqs), len(seqs)
+    rnd = lambda *s: torch.randn(*s, generator=g)            # noqa: E731
+    return dict(q=rnd(T, G, D), k=rnd(T, G, D), v=rnd(T, H, Dv), b=(1 + rnd(T, H)).to(dt), a=rnd(T, H).to(dt), a_log=rnd(H) - 1,
+                dt_bias=rnd(H), state=rnd(n, H, Dv, D), state_slots=torch.arange(n, dtype=torch.int32),
+                row_cu=torch.tensor([sum(m for _, m in seqs[:i]) for i in range(n + 1)], dtype=torch.int32),
+                positions=torch.cat([torch.arange(s, s + m) for s, m in seqs]).int())
+
+
+def both(x, D, eps):
+    """(outputs, state) of the kernel and of the f32 reference loop."""
+    got, ref = {k: t.cuda() for k, t in x.items()}, {k: t.clone() for k, t in x.items()}
+    o = ops.delta_scan(**got, q_scale=D ** -0.5, unit_eps=eps)
+    w = ops.delta_scan(**ref, q_scale=D ** -0.5, unit_eps=eps)
+    return (o.cpu(), got["state"].cpu()), (w, ref["state"])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("D,seqs", [(64, [(0, 17)]), (128, [(5, 20), (0, 39)]), (40, [(0, 30)])])
+def test_unit_vectors_without_an_epsilon(D, seqs):
+    """unit_eps 0: a last chunk that is partly empty has no vector of length zero."""
+    for got, want in zip(*both(step(seqs, 2, 1, D, 48, D), D, 0.0)):
+        assert (got - want).abs().max() < 1e-5 * want.abs().max()      # two f32 evaluations
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])      # (of the logits)
 @pytest.mark.parametrize("H,G,D,Dv,seqs", [
