@@ -586,8 +586,10 @@ __device__ __forceinline__ void lds_wave_sync() {
 //   waves 0 .. 3 run chunk p - 2 with 16 columns of the state each. A state tile's accumulator layout (element e of lane
 //   group gg: row 16 i + 4 gg + e) is the B operand of K S and Q S, and the accumulators of V - ..., U are the B
 //   operands of the products that follow, so nothing of the chain goes through LDS.
-// The unit norms are factors of rows and columns. Rows past the sequence: k = q = 0, g = 1, beta = 0. D <= 16 NT. A
-// chunk is one matrix product: NaN or infinity in a row reaches all rows of its chunk.
+// The unit norms are factors of rows and columns. Rows past the sequence: k = q = 0, g = 1, beta = 0. D <= 16 NT.
+// A chunk is one matrix product, in which a weight of zero does not hide a NaN: elements of k, v and the logits that are no
+// numbers go in as zeros (g = 1, beta = 0), and from the first row that had one on (k or logits: every column; v: its
+// column) outputs and the state are NaN, as a row-by-row scan leaves them; rows before it are untouched. (1 to 4 % of the time.)
 // Rounding: a chunk's scalars (decay products, norms, factors of L) are formed in 64 bits and rounded once, products over
 // channels are summed in pieces of 32 or 64, and the unit diagonal of (I + L)^-1 is applied without a product; with that
 // outputs and states are as far from a 64-bit recurrence as the row-by-row kernel's (rms 1.3e-7 and 1.0e-7 relative).
@@ -614,6 +616,7 @@ __global__ __launch_bounds__(512, NT <= 4 ? 4 : 2) void delta_chunk_kernel(
   float* sA = sT + 2 * C * PP;            // [2][C][PP] weights D_tj (q_t . k_j) / |k_j|
   float* sc = sA + 2 * C * PP;            // [2][6][C]: G / |k|, D_15 / |k|, G, q_scale / |q|, G_15, beta
   float* sl = sc + 2 * 6 * C;             // [2][2][C] decay and write strength of each row
+  int* sj = reinterpret_cast<int*>(sl + 2 * 2 * C);      // [4] first row of a chunk whose k or logits are no numbers, or C
   const int s = blockIdx.x, h = blockIdx.y, c0 = blockIdx.z * 64;
   const int hk = h / (H / G);
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, m = lane & 15, gg = lane >> 4;
@@ -676,42 +679,67 @@ __global__ __launch_bounds__(512, NT <= 4 ? 4 : 2) void delta_chunk_kernel(
       f32x4 ux[4], yx[4];
       rows(0);
       const f32x4 gk = *reinterpret_cast<const f32x4*>(f + 4 * gg), dk = *reinterpret_cast<const f32x4*>(f + C + 4 * gg);
-      const f32x4 gt = *reinterpret_cast<const f32x4*>(f + 2 * C + 4 * gg);
-      const f32x4 qn = *reinterpret_cast<const f32x4*>(f + 3 * C + 4 * gg);
       const f32x4 ti = *reinterpret_cast<const f32x4*>(sT + ((c & 1) * C + m) * PP + 4 * gg);
-      const f32x4 wq = *reinterpret_cast<const f32x4*>(sA + ((c & 1) * C + m) * PP + 4 * gg);
       const f32x4 bt = *reinterpret_cast<const f32x4*>(f + 5 * C + 4 * gg);
       const float gn = f[4 * C];
+      // what the chunk's end needs: early, or (NT <= 4, whose two workgroups per compute unit leave 128 registers) late
+      f32x4 gt, qn, wq;
+      auto weights = [&] { wq = *reinterpret_cast<const f32x4*>(sA + ((c & 1) * C + m) * PP + 4 * gg); };
+      auto last = [&] {
+        gt = *reinterpret_cast<const f32x4*>(f + 2 * C + 4 * gg);
+        qn = *reinterpret_cast<const f32x4*>(f + 3 * C + 4 * gg);
+      };
+      if (NT > 4) {
+        weights();
+        last();
+      }
 #pragma unroll
       for (int g = 0; g < NG; ++g) {
         if (g + 1 < NG) rows(g + 1);
         else cols(0);
 #pragma unroll
         for (int j = 0; j < 4; j += NS) {
-        f32x4 xk[4], xq[4];
+          f32x4 xk[4], xq[4];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) xk[e] = xq[e] = f32x4{0.f, 0.f, 0.f, 0.f};
+          for (int e = 0; e < 4; ++e) xk[e] = xq[e] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int i = j; i < j + NS; ++i)
+          for (int i = j; i < j + NS; ++i)
 #pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            xk[e] = mfma_f32(ka[g & 1][i][e], st[4 * g + i][e], xk[e]);
-            xq[e] = mfma_f32(qa[g & 1][i][e], st[4 * g + i][e], xq[e]);
-          }
-        pk += (xk[0] + xk[1]) + (xk[2] + xk[3]);
-        pq += (xq[0] + xq[1]) + (xq[2] + xq[3]);
-}
+            for (int e = 0; e < 4; ++e) {
+              xk[e] = mfma_f32(ka[g & 1][i][e], st[4 * g + i][e], xk[e]);
+              xq[e] = mfma_f32(qa[g & 1][i][e], st[4 * g + i][e], xq[e]);
+            }
+          pk += (xk[0] + xk[1]) + (xk[2] + xk[3]);
+          pq += (xq[0] + xq[1]) + (xq[2] + xq[3]);
+        }
       }
+      // no[e]: 0, or NaN from the first row of this lane's column on that is no number (x * 0 of such an x is NaN); the sums over
+      // rows by lane groups. Without a branch, which would split the chunk's one schedule.
+      f32x4 no;
+      float vv[4], sum = 0.f;
+      const int odd = sj[c & 3];
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const float vv = t0 + 4 * gg + e < r1 ? rv[e] : 0.f;
-        const float ve = fmaf(-gk[e], pk[e], vv);
+        const float x = t0 + 4 * gg + e < r1 ? rv[e] : 0.f, z = fmaf(x, 0.f, 0.f);
+        vv[e] = z == 0.f ? x : 0.f;
+        sum += z;
+        no[e] = sum + (4 * gg + e >= odd ? NAN : 0.f);
+      }
+      // lane groups 1 and 3 take the sum of 0 and 2, then 2 and 3 that of 0 and 1 (the swaps of row4_sum)
+      const auto up = __builtin_amdgcn_permlane16_swap(__float_as_uint(sum), __float_as_uint(sum), false, false);
+      const unsigned pair = __float_as_uint(__uint_as_float(up[0]) + __uint_as_float(up[1]));
+      const auto far = __builtin_amdgcn_permlane32_swap(pair, pair, false, false);
+      no += (gg & 1 ? __uint_as_float(up[0]) : 0.f) + (gg & 2 ? __uint_as_float(far[0]) : 0.f);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float ve = fmaf(-gk[e], pk[e], vv[e]);
         ux[e] = mfma_f32(ti[e], ve, f32x4{0.f, 0.f, 0.f, 0.f});
         u[e] = bt[e] * ve;
       }
       u += (ux[0] + ux[1]) + (ux[2] + ux[3]);
       if (c + 1 < nch) fetch(t0 + C);      // in flight until the next chunk
-      const f32x4 ud = u * dk;
+      if (NT <= 4) weights();
+      const f32x4 ud = (u + no) * dk;
 #pragma unroll
       for (int g = 0; g < NG; ++g) {
         if (g + 1 < NG) cols(g + 1);
@@ -722,13 +750,14 @@ __global__ __launch_bounds__(512, NT <= 4 ? 4 : 2) void delta_chunk_kernel(
         for (int e = 0; e < 4; ++e) {
 #pragma unroll
           for (int i = 0; i < 4; ++i) x[i] = mfma_f32(ku[g & 1][i][e], ud[e], x[i]);
-          if (g == 0) yx[e] = mfma_f32(wq[e], u[e], f32x4{0.f, 0.f, 0.f, 0.f});
+          if (g == 0) yx[e] = mfma_f32(wq[e], u[e], e == 0 ? no : f32x4{0.f, 0.f, 0.f, 0.f});
         }
 #pragma unroll
         for (int i = 0; i < 4; ++i)
 #pragma unroll
           for (int e = 0; e < 4; ++e) st[4 * g + i][e] = fmaf(st[4 * g + i][e], gn, x[i][e]);
       }
+      if (NT <= 4) last();
       y = (yx[0] + yx[1]) + (yx[2] + yx[3]);
       if (live) {
 #pragma unroll
@@ -763,13 +792,19 @@ __global__ __launch_bounds__(512, NT <= 4 ? 4 : 2) void delta_chunk_kernel(
     an = al[t * a_ld + h];
     bn = bl[t * b_ld + h];
   };
-  // wave 7, chunk c: decay and write strength of row m
+  // wave 7, chunk c: decay and write strength of row m (and a fresh mark of the chunk: its readers are two steps behind)
   auto write_gates = [&](int c) {
-    const bool in = r0 + c * C + m < r1;
     const float av = (float)an + dtb;
     const float sp = av > 20.f ? av : log1pf(expf(av));            // softplus
-    sl[(c & 1) * 2 * C + m] = in ? expf(-rate * sp) : 1.f;
-    sl[((c & 1) * 2 + 1) * C + m] = in ? 1.f / (1.f + expf(-(float)bn)) : 0.f;
+    const float g = expf(-rate * sp), b = 1.f / (1.f + expf(-(float)bn));
+    const bool nan = !(g == g && b == b), in = r0 + c * C + m < r1 && !nan;
+    sl[(c & 1) * 2 * C + m] = in ? g : 1.f;
+    sl[((c & 1) * 2 + 1) * C + m] = in ? b : 0.f;
+    if (lane == 0) sj[c & 3] = C;
+    if (__any(nan && r0 + c * C + m < r1)) {
+      lds_wave_sync();
+      if (nan && r0 + c * C + m < r1) atomicMin(&sj[c & 3], m);
+    }
   };
   const float* k0 = k + (long)(r0 + m) * k_ld + (long)hk * D;
   const float* q0 = q + (long)(r0 + m) * q_ld + (long)hk * D;
@@ -812,6 +847,18 @@ __global__ __launch_bounds__(512, NT <= 4 ? 4 : 2) void delta_chunk_kernel(
 #pragma unroll
       for (int e = 0; e < 4; ++e) kx[e] = qx[e] = nk;
       const int in = t0 + m < r1, Dm = in ? D : 0;
+      float zero = 0.f;
+#pragma unroll
+      for (int i = 0; i < NQ; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) zero = fmaf(rk[i][e], 0.f, zero);
+      if (__any(zero != 0.f)) {      // (channels past D are copies of the row's own)
+        if (zero != 0.f && in) atomicMin(&sj[p & 3], m);
+#pragma unroll
+        for (int i = 0; i < NQ; ++i)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) rk[i][e] = rk[i][e] * 0.f == 0.f ? rk[i][e] : 0.f;
+      }
 #pragma unroll
       for (int i = 0; i < NQ; ++i) {
         const int d = 16 * (NQ * w + i) + 4 * gg;
@@ -1044,7 +1091,7 @@ static void delta_chunk_launch(const float* q, long q_ld, const float* k, long k
                                const int* state_slots, const int* row_cu, int nseq, const int* positions, float q_scale,
                                float unit_eps, float* o, int H, int G, int D, int Dv, hipStream_t s) {
   constexpr int C = 16;
-  constexpr size_t lds = (size_t)(6 * C * (16 * NT + 4) + 18 * 256 + 24 * C + 4 * C * (C + 4) + 16 * C) * sizeof(float);
+  constexpr size_t lds = (size_t)(6 * C * (16 * NT + 4) + 18 * 256 + 24 * C + 4 * C * (C + 4) + 16 * C + 4) * sizeof(float);
   static bool once = false;
   if (!once) {
     (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&delta_chunk_kernel<T, NT>),

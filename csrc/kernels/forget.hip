@@ -65,6 +65,8 @@ __device__ __forceinline__ float half_sum(float v) {
 // lanes per row t share its channels, and q_t times the decays so far is carried down j. Rows past the sequence have f = 1,
 // k = q = 0. D <= 16 NT, NT even.
 // GLA: f = sigmoid(z)^(1 / tau) and k is an input, loaded by the lanes that hold k's channels.
+// In the second sum a weight of zero does not hide a NaN: values v that are no numbers go in as zeros, and the outputs of
+// their column are NaN from their row on, as a row-by-row scan leaves them. (All other factors meet rows after theirs only.)
 template <typename T, int NT, bool GLA>
 __global__ __launch_bounds__(512, NT <= 8 ? 4 : 2) void forget_chunk_kernel(const T* __restrict__ q, long q_ld,
                                                            const T* __restrict__ key, long k_ld, float inv_tau, float q_scale,
@@ -327,8 +329,26 @@ __global__ __launch_bounds__(512, NT <= 8 ? 4 : 2) void forget_chunk_kernel(cons
       }
 #pragma unroll
       for (int e = 0; e < 4; ++e) oc[e] += so[(4 * gg + e) * VP + cl];
+      float zero = 0.f;      // (x * 0 of an infinity or NaN is NaN)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) zero = fmaf(bv[e], 0.f, zero);
+      int odd = C;           // first row of this column that is no number
+      if (__any(zero != 0.f)) {
+#pragma unroll
+        for (int e = 3; e >= 0; --e) {
+          const bool bad = bv[e] * 0.f != 0.f;
+          odd = bad ? 4 * gg + e : odd;
+          bv[e] = bad ? 0.f : bv[e];
+        }
+        odd = min(odd, __shfl_xor(odd, 16, 64));
+        odd = min(odd, __shfl_xor(odd, 32, 64));
+      }
 #pragma unroll
       for (int e = 0; e < 4; ++e) oc = mfma_f32(a[e], bv[e], oc);
+      if (__any(odd < C)) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) oc[e] = 4 * gg + e >= odd ? NAN : oc[e];
+      }
       if (live) {
 #pragma unroll
         for (int e = 0; e < 4; ++e) {

@@ -76,3 +76,20 @@ def test_prompt_chunks_match_the_token_loop(dt, H, G, D, Dv, seqs):
     # f32 sums of up to 256 channels, a solve of up to 16 coupled rows, products of 16 decays (f32 eps 6e-8 each)
     for got, ref in ((o, want), (sd, state)):
         assert (got.cpu().to(F64) - ref).abs().max() < 5e-6 * ref.abs().max()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("bad", [float("nan"), float("inf")])
+@pytest.mark.parametrize("where", ["q", "k", "v", "a", "b"])
+@pytest.mark.parametrize("row", [0, 7, 11, 16, 18])      # of two chunks: first row, both blocks, the last rows
+def test_values_that_are_no_numbers_reach_later_rows_only(row, where, bad):
+    """As in a loop over the rows: from their row on (q: in it), in their column (v) or all of them, and not another sequence."""
+    D, Dv = 64, 80
+    x = step([(3, 19), (0, 20)], 2, 2, D, Dv, row)
+    x[where][row, 1, ...] = bad if where in "ab" else x[where][row, 1]
+    if where not in "ab":
+        x[where][row, 1, 5] = bad
+    for got, want in zip(*both(x, D, 1e-6)):
+        assert torch.equal(got.isfinite(), want.isfinite())
+        ok = want.isfinite()
+        assert (got - want)[ok].abs().max() < 1e-5 * want[ok].abs().max()

@@ -39,3 +39,25 @@ def test_prompt_chunks_match_the_token_loop(dt, tol, H, D, Dv, seqs):
     # f32 sums of up to 256 channels and products of 16 decays (f32 eps 6e-8 each); hardware exp / log for bf16 inputs
     for got, ref in ((o, want), (sd, state)):
         assert (got.cpu().to(F64) - ref).abs().max() < tol * ref.abs().max()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("bad", [float("nan"), float("inf")])
+@pytest.mark.parametrize("where", ["q", "k", "v", "z"])
+@pytest.mark.parametrize("row", [0, 7, 11, 16, 18])      # of two chunks: first row, both blocks, the last rows
+def test_values_that_are_no_numbers_reach_later_rows_only(row, where, bad):
+    """As in a loop over the rows: from their row on (q: in it), in their column (v) or state row (k, z), and not another
+    sequence."""
+    g = torch.Generator().manual_seed(row)
+    seqs, H, D, Dv = [(3, 19), (0, 20)], 2, 64, 80
+    T, rnd = 39, lambda *s: torch.randn(*s, generator=g)            # noqa: E731
+    x = dict(q=rnd(T, H, D), k=rnd(T, H, D), v=rnd(T, H, Dv), z=2 + rnd(T, H * D), state=rnd(2, H, D, Dv),
+             state_slots=torch.tensor([1, 0], dtype=torch.int32), row_cu=torch.tensor([0, 19, 39], dtype=torch.int32),
+             positions=torch.cat([torch.arange(s, s + n) for s, n in seqs]).int())
+    x[where].view(T, H, -1)[row, 1, 5] = bad
+    got, ref = {k: t.cuda() for k, t in x.items()}, {k: t.clone() for k, t in x.items()}
+    o, w = (ops.gla_scan(**a, tau=16.0, q_scale=D ** -0.5) for a in (got, ref))
+    for a, b in ((o.cpu(), w), (got["state"].cpu(), ref["state"])):
+        assert torch.equal(a.isfinite(), b.isfinite())
+        ok = b.isfinite()
+        assert (a - b)[ok].abs().max() < 1e-5 * b[ok].abs().max()
