@@ -85,7 +85,8 @@ __global__ __launch_bounds__(512) void gla_scan_kernel(const T* __restrict__ q, 
                                                        const int* __restrict__ state_slots,
                                                        const int* __restrict__ row_cu,
                                                        const int* __restrict__ positions, float inv_tau,
-                                                       float q_scale, float* __restrict__ o, int H, int D, int Dv) {
+                                                       float q_scale, float* __restrict__ o, int H, int D, int Dv,
+                                                       int below) {
   constexpr int TB = 16, DP = 8 * NR, NT = 512;
   __shared__ __attribute__((aligned(16))) float sa[TB * DP], sk[TB * DP], sq[TB * DP];
   __shared__ float sv[TB][64], so[TB][64];
@@ -96,7 +97,7 @@ __global__ __launch_bounds__(512) void gla_scan_kernel(const T* __restrict__ q, 
   const bool live = col < Dv;
   const int r0 = row_cu[s], r1 = row_cu[s + 1];
   const int slot = state_slots[s];
-  if (r1 <= r0) return;
+  if (r1 <= r0 || r1 - r0 >= below) return;      // (from `below` rows on: in chunks)
   if (slot < 0) {      // padding sequence of a fixed-shape step: defined output, no state
     for (int i = threadIdx.x; i < (r1 - r0) * 64; i += NT)
       if (c0 + (i & 63) < Dv) o[((long)(r0 + (i >> 6)) * H + h) * Dv + c0 + (i & 63)] = 0.f;
@@ -484,12 +485,12 @@ void launch_attn_window_paged(const void* q, long q_ld, const void* k_cache, con
 template <typename T>
 static int gla_scan_t(const T* q, long q_ld, const T* k, long k_ld, const T* v, long v_ld, const T* z, long z_ld,
                       float* state, const int* state_slots, const int* row_cu, int nseq, const int* positions,
-                      float tau, float q_scale, float* o, int H, int D, int Dv, hipStream_t s) {
+                      float tau, float q_scale, float* o, int H, int D, int Dv, hipStream_t s, int below) {
   dim3 grid(nseq, H, (Dv + 63) / 64);
   const float it = 1.f / tau;
 #define BFLY_GLA(NR)                                                                                              \
   gla_scan_kernel<T, NR><<<grid, 512, 0, s>>>(q, q_ld, k, k_ld, v, v_ld, z, z_ld, state, state_slots, row_cu, positions, \
-                                              it, q_scale, o, H, D, Dv)
+                                              it, q_scale, o, H, D, Dv, below)
   if (D <= 32) BFLY_GLA(4);
   else if (D <= 64) BFLY_GLA(8);
   else if (D <= 128) BFLY_GLA(16);
@@ -501,25 +502,30 @@ static int gla_scan_t(const T* q, long q_ld, const T* k, long k_ld, const T* v, 
 
 void launch_gla_chunks(const void* q, long q_ld, const void* k, long k_ld, const void* v, long v_ld, const void* z, long z_ld,
                        float* state, const int* state_slots, const int* row_cu, int nseq, const int* positions, float tau,
-                       float q_scale, float* o, int H, int D, int Dv, bool f32, hipStream_t s);      // forget.hip
+                       float q_scale, float* o, int H, int D, int Dv, bool f32, hipStream_t s, int from);      // forget.hip
 
 int launch_gla_scan(const void* q, long q_ld, const void* k, long k_ld, const void* v, long v_ld, const void* z,
                     long z_ld, float* state, const int* state_slots, const int* row_cu, int nseq,
                     const int* positions, float tau, float q_scale, float* o, int T, int H, int D, int Dv, bool f32,
                     hipStream_t s) {
   if (T <= 0 || nseq <= 0) return 0;
-  // any prompt rows (some sequence has more than one): chunks on the f32 matrix cores; the token loop keeps the steps of
-  // single rows, where a chunk would be 15 / 16 padding
-  if (T > nseq && D <= 256 && std::max({q_ld, k_ld, z_ld}) < (1L << 21)) {
+  // Chunks on the f32 matrix cores from 16 rows of a sequence on (true f32: 32), the token loop above where a chunk is mostly
+  // padding. 16 heads of 128, us of loop and chunks: one sequence of 8 rows 9.4 and 10.5, of 16 13.1 and 10.4 (f32 15.3 and
+  // 14.2, of 24 20.5 and 21.1); 16 of 4 11.6 and 18; 200 single rows beside 2 95 and 166. With each sequence in its own form:
+  // 32 single rows beside 128 87 and 66, now 67; 200 beside 256 218 and 224, now 176 (f32 249 and 352, now 198).
+  const int from = f32 ? 32 : 16;
+  ScanForms form = scan_forms(T, nseq, from, (long)H * ((Dv + 63) / 64));
+  if (D > 256 || std::max({q_ld, k_ld, z_ld}) >= (1L << 21)) form = {true, false};
+  if (form.chunks)
     launch_gla_chunks(q, q_ld, k, k_ld, v, v_ld, z, z_ld, state, state_slots, row_cu, nseq, positions, tau, q_scale, o, H, D,
-                      Dv, f32, s);
-    return 0;
-  }
+                      Dv, f32, s, form.rows ? from : 0);
+  if (!form.rows) return 0;
+  const int below = form.chunks ? from : kAllRows;
   if (f32)
     return gla_scan_t<float>((const float*)q, q_ld, (const float*)k, k_ld, (const float*)v, v_ld, (const float*)z, z_ld,
-                             state, state_slots, row_cu, nseq, positions, tau, q_scale, o, H, D, Dv, s);
+                             state, state_slots, row_cu, nseq, positions, tau, q_scale, o, H, D, Dv, s, below);
   return gla_scan_t<bf16>((const bf16*)q, q_ld, (const bf16*)k, k_ld, (const bf16*)v, v_ld, (const bf16*)z, z_ld, state,
-                          state_slots, row_cu, nseq, positions, tau, q_scale, o, H, D, Dv, s);
+                          state_slots, row_cu, nseq, positions, tau, q_scale, o, H, D, Dv, s, below);
 }
 
 void launch_head_norm_gate(const float* o, const float* w, float eps, const void* gate, long g_ld, int act, float mul,
