@@ -927,6 +927,24 @@ def gla_out(o, g, norm_w, eps: float, out_dtype):
     return out
 
 
+def route_form(T: int, E: int, H: int, f32: bool) -> str:
+    """How moe_route_scores computes its logits: "one launch" with the choice (a few rows), "waves" or "gemm", then a wave per
+    token that chooses. us per step, bf16:
+    one launch, a workgroup per token that reads the router's rows itself, up to 224 KB of them: 16 tokens, 8 experts of
+    width 2048 8.4 -> 6.4 beside two launches, 32 of 2048 12.5 -> 12.3, but 32 of 4096 13.0 -> 14.0 and of 7168 13.9 -> 16.7;
+    beyond 4096 logits the other forms take longer (256 tokens, 32 experts of 4096: 15 and 34).
+    waves (eight experts at a time, the router's rows from the caches) beside the GEMM, whose tile is mostly empty: 2048
+    tokens, 8 experts of 2048 12 and 33, 4096 tokens, 32 experts 44 and 48, but 8192 tokens 77 and 58; 48 experts of
+    1024, 512 tokens 26 and 23, of 4096 41 and 60. f32 has the slower GEMM: 8192 tokens, 32 experts of 2048 151 and 246,
+    16384 293 and 271."""
+    if E <= 32 and T <= 256 and (T * E > 4096 or E * H * (4 if f32 else 2) <= 224 << 10):
+        return "one launch"
+    E8 = -(-E // 8) * 8
+    if T * E <= 4096 or (E <= 64 and T * E8 <= (1 << (18 if f32 else 17)) and (f32 or E <= 32 or H >= 4096)):
+        return "waves"
+    return "gemm"
+
+
 def moe_route_scores(x, wr, top_k: int, scoring: str = "softmax", renorm: bool = True, bias=None, select_bias=None,
                      groups=(1, 1), renorm_eps: float = 0.0, scale: float = 1.0):
     """Router with f32 logits -> (topk_ids [T, k] int32, topk_w [T, k] f32); scoring "softmax" |
@@ -943,15 +961,14 @@ def moe_route_scores(x, wr, top_k: int, scoring: str = "softmax", renorm: bool =
     rest = (bias, top_k, {"softmax": 0, "sigmoid": 1}[scoring], bool(renorm), ids, w, select_bias, int(groups[0]),
             int(groups[1]), float(renorm_eps), float(scale))
     E = wr.shape[0]
-    if E <= 32 and T <= 256:      # a few rows: logits and choice in one launch
+    form = route_form(T, E, x.shape[1], x.dtype == torch.float32)
+    if form == "one launch":
         torch.ops.bfly.moe_route_rows(x, wr, *rest)
         return ids, w
-    # logits: up to 64 experts one wave per token (steps of a few rows: per token and expert), beyond that a
-    # GEMM with f32 accumulation and f32 output; then one wave per token picks
-    if T * E <= 4096 or E <= 64:
+    if form == "waves":      # one wave per token (steps of a few rows: per token and expert)
         logits = _empty(T, E, dtype=torch.float32, device=x.device)
         torch.ops.bfly.router_logits(x, wr, logits)
-    else:
+    else:                    # a GEMM with f32 accumulation and f32 output
         logits = linear_act(x, wr, out_dtype=torch.float32)
     torch.ops.bfly.moe_topk_scores(logits, *rest)
     return ids, w

@@ -382,7 +382,8 @@ __device__ __forceinline__ float router_dot(const T* __restrict__ xr, const T* _
   return wave_sum(a);
 }
 
-// Router logits of a small step (a few rows): one wave per (token, expert). Large steps use the f32-output GEMM instead.
+// Router logits of a small step (a few rows): one wave per (token, expert). Larger steps: router_rows_kernel or the f32-output
+// GEMM (ops.route_form).
 template <typename T, int V>
 __global__ __launch_bounds__(256) void router_logits_kernel(const T* __restrict__ x, long ldx,
                                                             const T* __restrict__ wr, float* __restrict__ logits,

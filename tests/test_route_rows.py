@@ -29,3 +29,17 @@ def test_one_launch_routes_like_two(dt, T, E, Hd, top, stride):
                 ids2, w2 = torch.empty_like(ids), torch.empty_like(w)
                 torch.ops.bfly.moe_topk_scores(logits, b, top, sc, renorm, ids2, w2, s, *groups, 1e-6, 1.5)
                 assert torch.equal(ids, ids2) and torch.equal(w, w2)
+
+
+# us with one launch, with waves, with the GEMM (both with a choice launch) for (tokens, experts, width, f32)
+TIMED = {(16, 8, 2048, False): (6.4, 8.4, None), (16, 32, 4096, False): (14.0, 13.0, None), (64, 16, 7168, True): (13.4, 10.8, None),
+         (16, 32, 7168, False): (16.7, 13.9, None), (256, 32, 4096, False): (15, 34, 62), (8192, 32, 2048, False): (None, 77, 58),
+         (4096, 32, 2048, False): (None, 44, 48), (512, 48, 1024, False): (None, 26, 23), (512, 48, 4096, False): (None, 41, 60),
+         (2048, 8, 2048, False): (None, 12, 33), (16384, 16, 2048, False): (None, 76, 62), (8192, 64, 1024, False): (None, 79, 42),
+         (8192, 32, 2048, True): (None, 151, 246), (16384, 32, 2048, True): (None, 293, 271), (8192, 64, 4096, True): (None, 531, 477)}
+
+
+@pytest.mark.parametrize("step", TIMED)
+def test_the_form_is_near_the_fastest(step):
+    t = TIMED[step][("one launch", "waves", "gemm").index(ops.route_form(*step))]
+    assert t < 1.05 * min(v for v in TIMED[step] if v), step
