@@ -927,7 +927,7 @@ def gla_out(o, g, norm_w, eps: float, out_dtype):
     return out
 
 
-def route_form(T: int, E: int, H: int, f32: bool) -> str:
+def route_form(T: int, E: int, H: int, f32: bool, contiguous: bool = True) -> str:
     """How moe_route_scores computes its logits: "one launch" with the choice (a few rows), "waves" or "gemm", then a wave per
     token that chooses. us per step, bf16:
     one launch, a workgroup per token that reads the router's rows itself, up to 224 KB of them: 16 tokens, 8 experts of
@@ -937,11 +937,12 @@ def route_form(T: int, E: int, H: int, f32: bool) -> str:
     tokens, 8 experts of 2048 12 and 33, 4096 tokens, 32 experts 44 and 48, but 8192 tokens 77 and 58; 48 experts of
     1024, 512 tokens 26 and 23, of 4096 41 and 60. f32 has the slower GEMM: 8192 tokens, 32 experts of 2048 151 and 246,
     16384 293 and 271."""
-    if E <= 32 and T <= 256 and (T * E > 4096 or E * H * (4 if f32 else 2) <= 224 << 10):
-        return "one launch"
-    E8 = -(-E // 8) * 8
-    if T * E <= 4096 or (E <= 64 and T * E8 <= (1 << (18 if f32 else 17)) and (f32 or E <= 32 or H >= 4096)):
-        return "waves"
+    if T * E <= 4096 or contiguous:
+        if E <= 32 and T <= 256 and (T * E > 4096 or E * H * (4 if f32 else 2) <= 224 << 10):
+            return "one launch"
+        E8 = -(-E // 8) * 8
+        if T * E <= 4096 or (E <= 64 and T * E8 <= (1 << (18 if f32 else 17)) and (f32 or E <= 32 or H >= 4096)):
+            return "waves"
     return "gemm"
 
 
@@ -961,7 +962,7 @@ def moe_route_scores(x, wr, top_k: int, scoring: str = "softmax", renorm: bool =
     rest = (bias, top_k, {"softmax": 0, "sigmoid": 1}[scoring], bool(renorm), ids, w, select_bias, int(groups[0]),
             int(groups[1]), float(renorm_eps), float(scale))
     E = wr.shape[0]
-    form = route_form(T, E, x.shape[1], x.dtype == torch.float32)
+    form = route_form(T, E, x.shape[1], x.dtype == torch.float32, wr.is_contiguous())
     if form == "one launch":
         torch.ops.bfly.moe_route_rows(x, wr, *rest)
         return ids, w

@@ -43,3 +43,14 @@ TIMED = {(16, 8, 2048, False): (6.4, 8.4, None), (16, 32, 4096, False): (14.0, 1
 def test_the_form_is_near_the_fastest(step):
     t = TIMED[step][("one launch", "waves", "gemm").index(ops.route_form(*step))]
     assert t < 1.05 * min(v for v in TIMED[step] if v), step
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T,E", [(300, 16), (200, 32), (300, 64), (70, 65)])
+def test_router_rows_with_a_stride(T, E):
+    """More than 4096 logits take a router whose rows are a view into wider ones."""
+    g = torch.Generator().manual_seed(E)
+    x, wide = torch.randn(T, 64, generator=g).cuda(), torch.randn(E, 80, generator=g).cuda()
+    ids, w = ops.moe_route_scores(x, wide[:, :64], 2)
+    ids2, w2 = ops.moe_route_scores(x, wide[:, :64].contiguous(), 2)
+    assert torch.equal(ids, ids2) and (w - w2).abs().max() < 1e-5      # (sums of 64 f32 products in another order)
