@@ -119,6 +119,26 @@ def test_chunks_over_a_cached_prefix(Hq, Hkv, seqs):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("start,n,rest", [(2000, 64, 5), (5000, 300, 40), (100, 40, 3)])      # pages split over workgroups, and not
+def test_rows_of_no_sequence_stay(start, n, rest):
+    """Rows before the first and after the last sequence keep what the output held, also where partial results are merged."""
+    g = torch.Generator().manual_seed(n)
+    H, G, D, dev = 32, 8, 128, "cuda"
+    need = (start + n + BS - 1) // BS
+    kc, vc = (torch.randn(need, G, *s, generator=g).bfloat16().to(dev) for s in ((BS, D), (D, BS)))
+    q = torch.randn(2 + n + rest, H, D, generator=g).bfloat16().to(dev)
+    tables = torch.arange(need, dtype=torch.int32, device=dev)[None]
+    pos = torch.cat([torch.zeros(2), torch.arange(start, start + n), torch.zeros(rest)]).int().to(dev)
+    cu = torch.tensor([2, 2 + n], dtype=torch.int32, device=dev)
+    out = torch.full_like(q, 3.0)
+    ops.attn_prefill_paged(q, kc, vc, tables, cu, pos, n, 0.1, out=out)
+    assert (out[:2] == 3).all() and (out[2 + n:] == 3).all()
+    alone = ops.attn_prefill_paged(q[2:2 + n], kc, vc, tables, cu - 2, pos[2:2 + n], n, 0.1)
+    # (weights and outputs rounded to bf16, the sums of another number of splits)
+    assert (out[2:2 + n].float() - alone.float()).abs().max() < 2.0 ** -7 * vc.float().abs().max()
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("fp8", [False, True])
 @pytest.mark.parametrize("Hq,Hkv,ctx,max_ctx", [
     (32, 8, [1, 31, 32, 33, 257, 700], 1024),      # split contexts, eight waves; most waves without a page
