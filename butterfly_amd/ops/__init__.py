@@ -580,12 +580,13 @@ def attn_prefill_paged(q, k_cache, v_cache, tables, cu_q, positions, max_q: int,
         return ref.attn_prefill_paged(q, k_cache, v_cache, tables, cu_q, positions, max_q, scale, out)
     if out is None:
         out = _empty(q.shape, dtype=q.dtype, device=q.device)
-    # few query rows over many cached pages: scratch so that workgroups can share a tile's pages (partial f32 rows of up
-    # to 8 splits, 64 MB at most; a step of more rows has tiles enough)
+    # few query rows over many cached pages: partial f32 rows of the workgroups that share a tile's pages
     part = None
-    row = q.shape[0] * q.shape[1] * (q.shape[2] + 2)
-    if row > 0 and k_cache.dtype == torch.bfloat16 and (n := min(8, (1 << 24) // row)) > 1:
-        part = torch.empty(n * row, dtype=torch.float32, device=q.device)
+    if k_cache.dtype == torch.bfloat16:
+        n = torch.ops.bfly.attn_prefill_paged_scratch(q.shape[0], cu_q.numel() - 1, q.shape[1], k_cache.shape[1], q.shape[2],
+                                                      tables.stride(0))
+        if n:
+            part = _empty(n, dtype=torch.float32, device=q.device)
     torch.ops.bfly.attn_prefill_paged(q, k_cache, v_cache, tables, cu_q, positions, int(max_q), float(scale), out, part)
     return out
 

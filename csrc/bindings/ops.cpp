@@ -1247,6 +1247,10 @@ TORCH_LIBRARY(bfly, m) {
   m.def("ep_ipc_combine(Tensor slot, int k, int capmax, int[] bases, int rank, Tensor(a!) out) -> ()");
   m.def("ep_ipc_stats(int ptr) -> int[]", &ep_ipc_stats);
   m.def("ep_ipc_error(int ptr) -> int", [](int64_t p) -> int64_t { return bfly::ep_ipc_error(reinterpret_cast<const void*>(p)); });
+  m.def("attn_prefill_paged_scratch(int rows, int nseq, int hq, int hkv, int d, int max_blocks) -> int",
+        [](int64_t rows, int64_t nseq, int64_t hq, int64_t hkv, int64_t d, int64_t max_blocks) -> int64_t {
+          return bfly::attn_prefill_paged_scratch((int)rows, (int)nseq, (int)hq, (int)hkv, (int)d, (int)max_blocks);
+        });
   m.def("attn_prefill_paged(Tensor q, Tensor k_cache, Tensor v_cache, Tensor tables, Tensor cu_q, "
         "Tensor positions, int max_q, float scale, Tensor(a!) out, Tensor(b!)? part=None) -> ()");
   m.def("attn_prefill(Tensor q, Tensor k, Tensor v, Tensor cu_seqlens, int max_seqlen, float scale, "

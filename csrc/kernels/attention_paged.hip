@@ -465,6 +465,18 @@ bool launch_attn_window_mfma_ext(const void* q, long q_ld, const void* k_cache, 
                                  int window, int keep_first, const float* sink, const float* out_scale, void* out, int T,
                                  int H, int G, int D, int Dv, int block_size, float* part, long part_floats,
                                  hipStream_t s, const AttnMod& md);
+// workgroups that share a tile's pages there, at most `fit`
+int attn_window_tile_splits(int T, int H, int G, int nseq, int D, int Dv, int max_blocks, long fit);
+
+// launch_attn_prefill_paged takes the tiled kernel
+static bool paged_tiles(int rows, int nseq, int Hq, int Hkv) { return (long)rows * (Hq / Hkv) >= 128L * nseq && (long)rows * Hq >= 512; }
+
+long attn_prefill_paged_scratch(int rows, int nseq, int Hq, int Hkv, int D, int max_blocks) {
+  if (rows <= 0 || Hkv <= 0 || Hq % Hkv != 0 || !paged_tiles(rows, nseq, Hq, Hkv)) return 0;
+  // (64 MB at most; a step of more rows has tiles enough)
+  const long split = (long)rows * Hq * (D + 2), n = attn_window_tile_splits(rows, Hq, Hkv, nseq, D, D, max_blocks, (1L << 24) / split);
+  return n > 1 ? n * split : 0;
+}
 
 int launch_attn_prefill_paged(const bf16* q, long q_stride, const void* k_cache, const void* v_cache,
                               const int* tables, int bt_stride, const int* cu_q, const int* positions,
@@ -481,7 +493,7 @@ int launch_attn_prefill_paged(const bf16* q, long q_stride, const void* k_cache,
   // 8, us of the kernels below -> tiled: 900 rows over 3000 keys 318 -> 138, 2000 over 6000 1290 -> 374, 64 over 8000
   // 331 -> 59, three chunks of 128 over 1000 56 -> 41, four of 1000 over 2000 404 -> 296 (0.55 PFLOP/s). Shorter chunks and
   // FP8 pages keep the kernels below.
-  if (!kv_fp8 && (long)rows * G >= 128L * nseq && (long)rows * Hq >= 512 && q_stride % 8 == 0 &&
+  if (!kv_fp8 && paged_tiles(rows, nseq, Hq, Hkv) && q_stride % 8 == 0 &&
       reinterpret_cast<uintptr_t>(q) % 16 == 0) {
     AttnMod md;
     md.dv_out = D;

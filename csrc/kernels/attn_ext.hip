@@ -10,6 +10,10 @@ namespace bfly {
 
 #include "attn_window.inc"
 
+int attn_window_tile_splits(int T, int H, int G, int nseq, int D, int Dv, int max_blocks, long fit) {
+  return attn_tile_plan(T, H, H / G, G, nseq, D / 32, Dv, 1 << 30, 0, 0, max_blocks, fit).splits;
+}
+
 bool launch_attn_window_mfma_ext(const void* q, long q_ld, const void* k_cache, const void* v_cache, const int* tables,
                                  int max_blocks, const int* row_cu, int nseq, const int* positions, float scale,
                                  int window, int keep_first, const float* sink, const float* out_scale, void* out, int T,

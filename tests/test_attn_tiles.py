@@ -138,6 +138,22 @@ def test_rows_of_no_sequence_stay(start, n, rest):
     assert (out[2:2 + n].float() - alone.float()).abs().max() < 2.0 ** -7 * vc.float().abs().max()
 
 
+@pytest.mark.skipif(not ops.load_library(), reason="kernel library not built")
+def test_scratch_of_split_pages():
+    """Scratch only where workgroups share a tile's pages: few tiles, enough pages; 64 MB at most."""
+    need = lambda *a: torch.ops.bfly.attn_prefill_paged_scratch(*a)                    # noqa: E731
+    row = 32 * 130
+    assert need(64, 1, 32, 8, 128, 250) == 8 * 64 * row          # a chunk over a long prefix
+    assert need(64, 1, 32, 8, 128, 20) == 0                      # too few pages to share
+    assert need(4000, 1, 32, 8, 128, 250) == 0                   # tiles enough
+    assert need(15, 1, 32, 4, 128, 250) == 0 and need(0, 1, 32, 8, 128, 250) == 0      # not on the tiled kernel
+    for rows in (16, 100, 500, 900, 2000, 8000):
+        for nseq in (1, 3, 16):
+            for Hq, Hkv in ((32, 8), (64, 8), (8, 8), (64, 64)):
+                n = need(rows, nseq, Hq, Hkv, 128, 4096)
+                assert n <= 1 << 24 and n % (rows * Hq * 130) == 0 and n // (rows * Hq * 130) in (0, *range(2, 9))
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("fp8", [False, True])
 @pytest.mark.parametrize("Hq,Hkv,ctx,max_ctx", [
