@@ -12,7 +12,7 @@ F64 = torch.float64
 BS = 32
 
 
-def dense(q, k, v, pos, scale, window, keep, sink, slopes, chunk, qt):
+def dense(q, k, v, pos, scale, window, keep, sink, slopes, chunk, qt, cap=0.0, logs=None):
     """q [n, H, D] at positions pos over k [L, G, D], v [L, G, Dv] of one sequence."""
     H, G = q.shape[1], k.shape[1]
     i, j = pos[:, None], torch.arange(k.shape[0])[None]
@@ -24,7 +24,11 @@ def dense(q, k, v, pos, scale, window, keep, sink, slopes, chunk, qt):
         s = q[:, h] @ k[:, g].T * scale
         if qt:
             s = s * (1 + qt[0] * torch.log(torch.floor((i + 1) / qt[1]) + 1))
-        if slopes is not None:
+        if cap:
+            s = cap * torch.tanh(s / cap)
+        if logs is not None:
+            s = s - slopes[h] * torch.log1p(logs[h] * (i - j).clamp(min=0))
+        elif slopes is not None:
             s = s - slopes[h] * (i - j)
         s = s.masked_fill(~see, -math.inf)
         if sink is not None:
@@ -43,6 +47,15 @@ def dense(q, k, v, pos, scale, window, keep, sink, slopes, chunk, qt):
     (16, 16, 64, 64, 100, 0, "chunk", [(0, 640)]),                    # no grouping, chunks instead of a window
     (32, 2, 128, 128, 512, 0, "slope", [(0, 1030), (5, 1000)]),       # sixteen query heads per key head, two tiles per wave
     (16, 4, 128, 128, 40, 3, "sink", [(700, 1), (31, 1), (32, 1), (0, 1)]),   # decoded rows: the 16-row form
+    (16, 4, 128, 128, 1 << 30, 0, "cap", [(0, 700), (0, 1501)]),      # capped scores, two row tiles per wave
+    (8, 2, 128, 128, 200, 3, "cap slope log sink", [(0, 300), (77, 411)]),    # a cap and the logarithmic distance bias, one row tile
+    (16, 16, 64, 64, 1 << 30, 0, "slope log temp", [(3, 640)]),
+    (8, 8, 32, 32, 100, 0, "", [(0, 333), (40, 200)]),                # the other head sizes
+    (8, 2, 96, 96, 1 << 30, 0, "sink", [(0, 333), (40, 200)]),
+    (8, 2, 128, 256, 64, 5, "", [(0, 333), (40, 200)]),
+    (4, 2, 192, 192, 1 << 30, 0, "cap", [(0, 333), (40, 200)]),
+    (6, 1, 256, 192, 90, 0, "", [(0, 333), (40, 200)]),
+    (4, 2, 256, 256, 1 << 30, 0, "slope log", [(0, 333), (40, 200)]),
 ])
 def test_paged_tiles_match_dense_attention(dt, H, G, D, Dv, window, keep, mods, seqs):
     g = torch.Generator().manual_seed(H + D + window % 1000)
@@ -52,6 +65,8 @@ def test_paged_tiles_match_dense_attention(dt, H, G, D, Dv, window, keep, mods, 
     slopes = 0.5 ** torch.linspace(2, 9, H) if "slope" in mods else None
     qt = (0.3, 50) if "temp" in mods else None
     chunk = 90 if "chunk" in mods else 0
+    cap = 3.0 if "cap" in mods else 0.0
+    logs = torch.linspace(0.1, 2, H) if "log" in mods else None
     need = [(s + n + BS - 1) // BS for s, n in seqs]
     order = torch.randperm(sum(need), generator=g)
     kc = torch.zeros(sum(need), G, BS, D, dtype=torch.bfloat16)
@@ -68,12 +83,12 @@ def test_paged_tiles_match_dense_attention(dt, H, G, D, Dv, window, keep, mods, 
         qs.append(q)
         L = start + n
         want.append(dense(q.to(F64), k[:L].to(F64), v[:L].to(F64), torch.arange(start, L), scale, window, keep, sink,
-                          slopes, chunk, qt))
+                          slopes, chunk, qt, cap, logs))
     cu = torch.tensor([sum(n for _, n in seqs[:i]) for i in range(len(seqs) + 1)], dtype=torch.int32, device=dev)
     pos = torch.cat([torch.arange(s, s + n) for s, n in seqs]).int().to(dev)
     got = ops.attn_window_paged(torch.cat(qs).to(dev, dt), kc.to(dev, dt), vc.to(dev, dt), tables.to(dev), cu, pos, scale, window, keep,
-                                None if sink is None else sink.to(dev), chunk=chunk, q_temp=qt,
-                                dist_bias=None if slopes is None else (slopes.to(dev), None))
+                                None if sink is None else sink.to(dev), chunk=chunk, q_temp=qt, softcap=cap,
+                                dist_bias=None if slopes is None else (slopes.to(dev), None if logs is None else logs.to(dev)))
     # bf16: weights rounded to bf16 (2^-9 each, together at most 2^-9 of the largest value), the output rounded once more;
     # f32: scores of up to 20 with a few eps (6e-8) of their size, which is the relative error of a weight
     err = (got.cpu().to(F64) - torch.cat(want)).abs().max()

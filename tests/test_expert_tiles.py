@@ -70,7 +70,7 @@ def test_experts_over_row_groups(counts, Hd, F, plain, scaled, limit, stride):
     ([65, 4, 1, 1], 512, 64, True, True),                # one row in a second tile
 ])
 def test_experts_over_few_rows(counts, Hd, F, plain, scaled):
-    """Weights streamed past the rows; rows of x with a stride, an addend, ids that name no expert here."""
+    """Weights streamed past the rows; rows of x with a stride, an addend."""
     g = torch.Generator().manual_seed(sum(counts) + F)
     E, TK = len(counts), sum(counts)
     flat = torch.cat([torch.full((c,), e) for e, c in enumerate(counts)])[torch.randperm(TK, generator=g)]
@@ -86,3 +86,34 @@ def test_experts_over_few_rows(counts, Hd, F, plain, scaled):
     # bf16 input rows times their score, hidden rows and output (2^-9 each); the squared activation doubles the first
     err = (got.cpu().to(F64) - want).norm() / want.norm()
     assert err < 6e-3
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("counts,rest,Hd,F,plain", [
+    ([5, 0, 16, 3], 20, 320, 128, False),        # weights streamed past the rows
+    ([40, 64, 1, 70], 40, 512, 128, False),      # the 64-row tiles
+    ([512, 769, 0, 500], 333, 256, 128, False),  # the 256-row tiles
+    ([500, 700], 111, 512, 256, True),
+    ([0, 0, 0], 9, 256, 256, False),             # no row for any expert
+])
+@pytest.mark.parametrize("beyond", [0, 3])
+def test_ids_that_name_no_expert(counts, rest, Hd, F, plain, beyond):
+    """ids from E on: they return the token's row itself (fewer grouped rows than pairs: the tail of the row groups and the pairs'
+    outputs stay unwritten and count nowhere)."""
+    g = torch.Generator().manual_seed(sum(counts) + F)
+    E = len(counts)
+    flat = torch.cat([torch.full((c,), e) for e, c in enumerate(counts)] + [torch.full((rest,), E + beyond)])
+    flat = flat[torch.randperm(len(flat), generator=g)]
+    ids = flat[:len(flat) // 2 * 2].view(-1, 2)
+    T = len(ids)
+    bf = lambda *s, k=1.0: (k * torch.randn(*s, generator=g)).to(torch.bfloat16)            # noqa: E731
+    x, w = bf(T, Hd), torch.rand(T, 2, generator=g) + 0.2
+    gu, dn = bf(E, F if plain else 2 * F, Hd, k=2 * Hd ** -0.5), bf(E, Hd, F, k=F ** -0.5)
+    ops.moe_glu_ffn(*(t.cuda() for t in (torch.full_like(x, 1e30), torch.zeros_like(ids).int(), w, gu, dn)), 7.0, 1.702, 1.0, False,
+                    "relu2" if plain else None)      # (leaves large values and infinities in the scratch)
+    got = ops.moe_glu_ffn(x.cuda(), ids.int().cuda(), w.cuda(), gu.cuda(), dn.cuda(), 7.0, 1.702, 1.0, False,
+                          "relu2" if plain else None, identity=True)
+    want = reference(x.to(F64), ids, w.to(F64), gu.to(F64), dn.to(F64), 7.0, 1.702, 1.0, False, plain)
+    want += (w.to(F64) * (ids >= E)).sum(1, keepdim=True) * x.to(F64)
+    # bf16 hidden rows and output, 2^-9 each
+    assert (got.cpu().to(F64) - want).norm() / want.norm() < 6e-3
