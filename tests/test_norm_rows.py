@@ -17,7 +17,7 @@ def norm(x, w, b, eps):
 @pytest.mark.gpu
 @pytest.mark.parametrize("dt,tol", [(torch.float32, 4e-6), (torch.bfloat16, 2.0 ** -8)])
 @pytest.mark.parametrize("rms", [False, True])
-@pytest.mark.parametrize("W", [4, 252, 1020, 1024, 1028, 2048, 2052, 4096, 4100])      # edges of a thread's share
+@pytest.mark.parametrize("W", [4, 252, 256, 260, 1020, 1024, 1028, 2048, 2052, 4096, 4100])      # edges of a thread's share
 def test_step_over_row_widths(dt, tol, rms, W):
     g = torch.Generator().manual_seed(W)
     T, eps, m = 3, 1e-5, 0.7
