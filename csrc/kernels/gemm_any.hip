@@ -178,12 +178,27 @@ __global__ __launch_bounds__(256) void gemm_any_kernel(const float* __restrict__
   tile_mac_f32<WT, 1, VEC, false>(
       acc, [&](int r) { return RowF{row0 + r < M ? x + (long)(row0 + r) * ldx : nullptr, 1.f}; },
       [&](int, int c) { return RowF{col0 + c < N ? w + (long)(col0 + c) * ldw : nullptr, 1.f}; }, K, S);
-  tile_each<WT>(acc[0], [&](int m, int n, float v) {
-    const int r = row0 + m, c = col0 + n;
-    if (r >= M || c >= N) return;
-    if (bias) v += bias[c];
-    out[(long)r * ldo + c] = apply_act(v, act, a0, a1);
-  });
+  // a lane's four columns in one access where the rows allow it: with few channels the stores are the time (4000 x 2048 x 16
+  // one value at a time 25 us)
+  const bool vec = (ldo & 3) == 0 && (reinterpret_cast<uintptr_t>(out) & 15) == 0;
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+#pragma unroll
+  for (int tn = 0; tn < WT; ++tn)
+#pragma unroll
+    for (int tm = 0; tm < WT; ++tm) {
+      const int r = row0 + (wave >> 1) * 16 * WT + 16 * tm + (lane & 15);
+      const int c = col0 + (wave & 1) * 16 * WT + 16 * tn + 4 * (lane >> 4);
+      if (r >= M || c >= N) continue;
+      f32x4 v = acc[0][tn][tm];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[i] = apply_act(bias ? v[i] + bias[min(c + i, N - 1)] : v[i], act, a0, a1);
+      float* o = out + (long)r * ldo + c;
+      if (vec && c + 4 <= N) *reinterpret_cast<f32x4*>(o) = v;
+      else
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          if (c + i < N) o[i] = v[i];
+    }
 }
 
 template <typename T>

@@ -24,6 +24,22 @@ def test_gemm_matches_float64(M, N, K, pad):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("T,H,N,K", [(70, 3, 64, 16), (130, 2, 66, 40), (5, 4, 7, 33)])
+@pytest.mark.parametrize("pad,shift", [(0, 0), (4, 0), (3, 0), (4, 1)])      # row strides and starts that allow 16-byte stores or not
+def test_outputs_in_views(T, H, N, K, pad, shift):
+    g = torch.Generator().manual_seed(T + N)
+    x, w = torch.randn(T, H, K, generator=g), torch.randn(H, N, K, generator=g)
+    wide = torch.full((T, H * N + pad + shift), 7.0, device="cuda")
+    out = wide.as_strided((T, H, N), (H * N + pad + shift, N, 1), shift)
+    ops.linear_heads(x.cuda(), w.cuda(), out)
+    want = torch.matmul(x.to(F64).transpose(0, 1), w.to(F64).transpose(1, 2)).transpose(0, 1)
+    assert (out.cpu().to(F64) - want).abs().max() < K * 6e-8 * K ** 0.5 * (want.abs().max() + 1)
+    keep = torch.ones(wide.shape[1], dtype=torch.bool)
+    keep[shift:shift + H * N] = False
+    assert (wide.cpu()[:, keep] == 7.0).all()
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("T,E,W", [(600, 8, 256), (1025, 5, 512), (700, 64, 264), (41, 100, 64), (515, 9, 130)])
 def test_router_choice(dt, T, E, W):
