@@ -748,8 +748,12 @@ int launch_attn_decode(const bf16* q, long q_stride, const void* k_cache, const 
   // Up to 320 workgroups (little more than one per compute unit): eight waves each, so that a compute unit keeps twice the
   // pages in flight and a long context is walked by twice the waves. 32 heads on 8, contexts of 2.5k to 8k of 24 sequences:
   // FP8 99 -> 61 us, bf16 135 -> 118; 37 sequences of 0.9k to 3k 69 -> 60 us; from 384 workgroups on four are level
-  // (64 sequences of 1040: 34 us against 36). Sixteen waves hold 128 registers each and spill.
-  const bool w8 = (long)nsplit * Hkv * B <= 320;
+  // (64 sequences of 1040: 34 us against 36). Sixteen waves hold 128 registers each and spill. Four where a split's pages are too
+  // few to repay the merge of eight waves: above one workgroup per compute unit (64 heads on 8, 37 sequences of 300 13 us
+  // with eight, 11 with four) and, as a merge of more rows takes longer, with more than eight query heads per key / value
+  // head (16 heads on one, 100 sequences of 1040 in three splits 23 and 19, 48 of up to 8k in five 42 and 54).
+  const long wgs = (long)nsplit * Hkv * B;
+  const bool w8 = wgs <= 256 ? G <= 8 || part_tokens >= 512 : wgs <= 320 && part_tokens >= (G <= 8 ? 1024 : 1536);
 #define DEC_LAUNCH1(CT, NW)                                                                                 \
   {                                                                                                         \
     const size_t lds = (size_t)NW * (128 * G + 32) * sizeof(float);                                         \
