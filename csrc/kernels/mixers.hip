@@ -393,9 +393,12 @@ bool launch_attn_window_f32(const float* q, long q_ld, const float* kc, const fl
                             const float* sink, const float* out_scale, float* out, int T, int H, int G, int D, int Dv,
                             int block_size, hipStream_t s, const AttnMod& md) {
   // prompts: from 32 (row, head) pairs per sequence and key / value head on, at head sizes of whole segments; decoded rows
-  // and other shapes keep the one-wave-per-row form
+  // and other shapes keep the one-wave-per-row form, and so do a few prompt rows, whose waves all run at once (one prompt of
+  // 16 rows: 8 heads on 2 of 128 12.2 and 10.1 us, 8 on 1 of 256 / 192 17 and 13; of 40 rows level with 16 heads)
   if ((reinterpret_cast<uintptr_t>(kc) | reinterpret_cast<uintptr_t>(vc)) & 15) return false;
-  if (block_size != 32 || md.maps != 1 || md.pool > 0 || md.sigmoid || T <= 0 || (long)T * (H / G) < 32L * nseq) return false;
+  if (block_size != 32 || md.maps != 1 || md.pool > 0 || md.sigmoid || T <= 0 || (long)T * (H / G) < 32L * nseq ||
+      (T != nseq && T < 64 && T * H < 1024))
+    return false;
 #define BFLY_AF(DT, DVT)                                                                                                \
   return attn_window_f32_launch<DT, DVT>(q, q_ld, kc, vc, tables, max_blocks, row_cu, nseq, positions, scale, window,   \
                                          keep_first, sink, out_scale, out, T, H, G, s, md)
