@@ -75,6 +75,8 @@ struct AttnMod {
   int dv_out = 0;                 // > 0: values written per head (the cached value rows may be padded)
   long out_ld = 0;                // row stride of out
   bool out_vec = false;           // bf16 out / gate rows allow 8-byte accesses at every head
+  bool heads = false;             // (launches) the alternative to the tiled form are tiles of one head
+  bool tiles = false;             // (launches) the tiled form wherever it can be taken
   __host__ __device__ bool ext() const { return dv_out > 0; }
   // no score modifiers
   bool plain() const { return chunk == 0 && softcap == 0.f && !dist_a && qt_coef == 0.f && maps == 1 && !out_f32; }

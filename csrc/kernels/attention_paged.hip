@@ -496,6 +496,7 @@ int launch_attn_prefill_paged(const bf16* q, long q_stride, const void* k_cache,
   if (!kv_fp8 && paged_tiles(rows, nseq, Hq, Hkv) && q_stride % 8 == 0 &&
       reinterpret_cast<uintptr_t>(q) % 16 == 0) {
     AttnMod md;
+    md.tiles = true;
     md.dv_out = D;
     md.out_ld = o_stride;
     md.out_vec = o_stride % 4 == 0 && reinterpret_cast<uintptr_t>(out) % 8 == 0;

@@ -11,7 +11,7 @@ namespace bfly {
 #include "attn_window.inc"
 
 int attn_window_tile_splits(int T, int H, int G, int nseq, int D, int Dv, int max_blocks, long fit) {
-  return attn_tile_plan(T, H, H / G, G, nseq, D / 32, Dv, 1 << 30, 0, 0, max_blocks, fit).splits;
+  return attn_tile_plan(T, H, G, nseq, D, Dv, max_blocks, fit, false, true).splits;
 }
 
 bool launch_attn_window_mfma_ext(const void* q, long q_ld, const void* k_cache, const void* v_cache, const int* tables,

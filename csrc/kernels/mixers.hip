@@ -449,17 +449,22 @@ bool launch_attn_window_mfma(const void* q, long q_ld, const void* k_cache, cons
     return launch_attn_window_mfma_ext(q, q_ld, k_cache, v_cache, tables, max_blocks, row_cu, nseq, positions, scale, window,
                                        keep_first, sink, out_scale, out, T, H, G, D, Dv, block_size, part, part_floats, s,
                                        md);
-  if (!fold && md.maps == 1) {
-    // any grouped attention: the query heads of a key / value head share its tiles, so a page is read once for all of
-    // them; the per-head tiles of MODE 0 read it once per query head and are left to several maps per value head. 16
-    // decoded rows of 16 heads on 4, 1040 keys: 53 -> 23 + 6 us; prompts: attn_fold_tile_kernel.
-    AttnMod mx = md;
-    mx.dv_out = Dv;
-    mx.out_ld = (long)H * Dv;
-    mx.out_vec = !md.out_f32 && (Dv & 3) == 0 && (reinterpret_cast<uintptr_t>(out) & 7) == 0;
-    return launch_attn_window_mfma_ext(q, q_ld, k_cache, v_cache, tables, max_blocks, row_cu, nseq, positions, scale, window,
-                                       keep_first, sink, out_scale, out, T, H, G, D, Dv, block_size, part, part_floats, s,
-                                       mx);
+  if (!fold && md.maps == 1 && G > 0 && H % G == 0) {
+    // any grouped attention: the query heads of a key / value head share its tiles where attn_grouped or attn_tile_plan say so; the
+    // per-head tiles of MODE 0 read a page once per query head, and are the ones for several maps per value head
+    const long pages = attn_pages(window, keep_first, md.chunk, max_blocks);
+    const long fit = part ? part_floats / ((long)T * H * (Dv + 2)) : 1;
+    if (T > 0 && (attn_grouped(T, H, G, nseq, D, pages) ||
+                  attn_tile_plan(T, H, G, nseq, D, Dv, pages, fit, true, false).tiled)) {
+      AttnMod mx = md;
+      mx.dv_out = Dv;
+      mx.out_ld = (long)H * Dv;
+      mx.out_vec = !md.out_f32 && (Dv & 3) == 0 && (reinterpret_cast<uintptr_t>(out) & 7) == 0;
+      mx.heads = true;
+      return launch_attn_window_mfma_ext(q, q_ld, k_cache, v_cache, tables, max_blocks, row_cu, nseq, positions, scale, window,
+                                         keep_first, sink, out_scale, out, T, H, G, D, Dv, block_size, part, part_floats, s,
+                                         mx);
+    }
   }
   return attn_mfma_launch<0>(q, q_ld, k_cache, v_cache, tables, max_blocks, row_cu, nseq, positions, scale, window,
                              keep_first, sink, out_scale, out, T, H, G, D, Dv, block_size, fold, part, part_floats, s, md);

@@ -56,6 +56,16 @@ def dense(q, k, v, pos, scale, window, keep, sink, slopes, chunk, qt, cap=0.0, l
     (4, 2, 192, 192, 1 << 30, 0, "cap", [(0, 333), (40, 200)]),
     (6, 1, 256, 192, 90, 0, "", [(0, 333), (40, 200)]),
     (4, 2, 256, 256, 1 << 30, 0, "slope log", [(0, 333), (40, 200)]),
+    (16, 4, 64, 64, 1 << 30, 0, "slope log", [(3, 1100), (0, 900)]),  # bf16: rows enough for the tiled form at these sizes
+    (16, 16, 64, 64, 100, 0, "chunk", [(0, 2600)]),
+    (16, 4, 32, 32, 500, 3, "", [(0, 4150)]),
+    (8, 2, 96, 96, 1 << 30, 0, "sink", [(0, 700), (40, 400)]),
+    (8, 2, 128, 256, 64, 5, "", [(0, 700), (40, 400)]),
+    (4, 2, 192, 192, 1 << 30, 0, "cap", [(0, 1100), (40, 400)]),
+    (6, 1, 256, 192, 90, 0, "", [(0, 700), (40, 300)]),
+    (4, 2, 256, 256, 1 << 30, 0, "slope log", [(0, 1100), (40, 400)]),
+    (16, 4, 128, 128, 1 << 30, 0, "sink", [(400 + 31 * i, 1) for i in range(17)]),      # decoded rows: grouped tiles, pages split
+    (16, 4, 128, 128, 1 << 30, 0, "", [(900, 9), (40, 60), (0, 3)]),                    # tiles of one head
 ])
 def test_paged_tiles_match_dense_attention(dt, H, G, D, Dv, window, keep, mods, seqs):
     g = torch.Generator().manual_seed(H + D + window % 1000)
