@@ -531,12 +531,13 @@ class TransformerLM:
                 # kernel's rate on fresh prompts, profiles/r5_prof/)
                 s1, r1 = fb.split_seqs, fb.split_rows
                 ops.attn_prefill_paged(qp[:r1], kc, vc, fb.prefix_tables[:s1], fb.cu_seqlens[:s1 + 1],
-                                       fb.positions[nd:nd + r1], fb.max_paged, self.scale, out=out[nd:nd + r1])
+                                       fb.positions[nd:nd + r1], fb.max_paged, self.scale, out=out[nd:nd + r1],
+                                       max_ctx=max(fb.prefix_lens) + fb.max_paged if fb.prefix_lens else 0)
                 ops.attn_prefill(qp[r1:], k[nd + r1:], v[nd + r1:], fb.cu_fresh, fb.max_fresh, self.scale, True,
                                  out=out[nd + r1:])
             elif fb.prefix_lens is not None and any(fb.prefix_lens):
                 ops.attn_prefill_paged(qp, kc, vc, fb.prefix_tables, fb.cu_seqlens, fb.positions[nd:], fb.max_seqlen,
-                                       self.scale, out=out[nd:])
+                                       self.scale, out=out[nd:], max_ctx=max(fb.prefix_lens) + fb.max_seqlen)
             else:
                 ops.attn_prefill(qp, k[nd:], v[nd:], fb.cu_seqlens, fb.max_seqlen, self.scale, True, out=out[nd:])
         return out

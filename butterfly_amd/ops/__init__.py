@@ -571,11 +571,12 @@ def attn_prefill(q, k, v, cu_seqlens, max_seqlen: int, scale: float, causal: boo
     return (out, lse) if return_lse else out
 
 
-def attn_prefill_paged(q, k_cache, v_cache, tables, cu_q, positions, max_q: int, scale: float, out=None):
+def attn_prefill_paged(q, k_cache, v_cache, tables, cu_q, positions, max_q: int, scale: float, out=None, max_ctx: int = 0):
     """Chunked prefill attention over the paged cache (attention_paged.hip): query rows
     [cu_q[s], cu_q[s+1]) of sequence s at `positions` attend causally to the sequence's cached
     keys through tables[s] — the cached prefix and the chunk itself (already appended by
-    rope_kv) in one pass, no gather, no log-sum-exp merge. Caches bf16 or FP8."""
+    rope_kv) in one pass, no gather, no log-sum-exp merge. Caches bf16 or FP8. `max_ctx`: a bound of the positions + 1 where
+    the caller knows one (short contexts have a kernel of their own; it changes no result)."""
     if not _gpu(q):
         return ref.attn_prefill_paged(q, k_cache, v_cache, tables, cu_q, positions, max_q, scale, out)
     if out is None:
@@ -584,10 +585,11 @@ def attn_prefill_paged(q, k_cache, v_cache, tables, cu_q, positions, max_q: int,
     part = None
     if k_cache.dtype == torch.bfloat16:
         n = torch.ops.bfly.attn_prefill_paged_scratch(q.shape[0], cu_q.numel() - 1, q.shape[1], k_cache.shape[1], q.shape[2],
-                                                      tables.stride(0))
+                                                      tables.stride(0), int(max_ctx))
         if n:
             part = _empty(n, dtype=torch.float32, device=q.device)
-    torch.ops.bfly.attn_prefill_paged(q, k_cache, v_cache, tables, cu_q, positions, int(max_q), float(scale), out, part)
+    torch.ops.bfly.attn_prefill_paged(q, k_cache, v_cache, tables, cu_q, positions, int(max_q), float(scale), out, part,
+                                     int(max_ctx))
     return out
 
 

@@ -704,7 +704,7 @@ void attn_decode(const Tensor& q, const Tensor& k_cache, const Tensor& v_cache,
 // sequence by cu_q, positions [T] their absolute positions, tables [nseq, max_blocks].
 void attn_prefill_paged(const Tensor& q, const Tensor& k_cache, const Tensor& v_cache, const Tensor& tables,
                         const Tensor& cu_q, const Tensor& positions, int64_t max_q, double scale, Tensor& out,
-                        const c10::optional<Tensor>& part) {
+                        const c10::optional<Tensor>& part, int64_t max_ctx) {
   CHECK_GPU(q); CHECK_BF16(q); CHECK_KV(k_cache, v_cache); CHECK_BF16(out);
   TORCH_CHECK(q.dim() == 3 && q.stride(2) == 1 && q.stride(1) == q.size(2), "attn_prefill_paged: q [T, Hq, D]");
   TORCH_CHECK(out.dim() == 3 && out.sizes() == q.sizes() && out.stride(2) == 1 && out.stride(1) == out.size(2),
@@ -730,7 +730,7 @@ void attn_prefill_paged(const Tensor& q, const Tensor& k_cache, const Tensor& v_
                                                  tables.data_ptr<int>(), tables.stride(0), cu_q.data_ptr<int>(),
                                                  positions.data_ptr<int>(), nseq, (int)max_q, Hq, Hkv, D, BS,
                                                  (float)scale, bf(out), out.stride(0), cur_stream(),
-                                                 k_cache.scalar_type() == at::kFloat8_e4m3fn, (int)q.size(0), partp, part_n);
+                                                 k_cache.scalar_type() == at::kFloat8_e4m3fn, (int)q.size(0), partp, part_n, (int)max_ctx);
   TORCH_CHECK(rc == 0, "attn_prefill_paged: unsupported configuration (rc=", rc, ")");
 }
 
@@ -1247,12 +1247,12 @@ TORCH_LIBRARY(bfly, m) {
   m.def("ep_ipc_combine(Tensor slot, int k, int capmax, int[] bases, int rank, Tensor(a!) out) -> ()");
   m.def("ep_ipc_stats(int ptr) -> int[]", &ep_ipc_stats);
   m.def("ep_ipc_error(int ptr) -> int", [](int64_t p) -> int64_t { return bfly::ep_ipc_error(reinterpret_cast<const void*>(p)); });
-  m.def("attn_prefill_paged_scratch(int rows, int nseq, int hq, int hkv, int d, int max_blocks) -> int",
-        [](int64_t rows, int64_t nseq, int64_t hq, int64_t hkv, int64_t d, int64_t max_blocks) -> int64_t {
-          return bfly::attn_prefill_paged_scratch((int)rows, (int)nseq, (int)hq, (int)hkv, (int)d, (int)max_blocks);
+  m.def("attn_prefill_paged_scratch(int rows, int nseq, int hq, int hkv, int d, int max_blocks, int max_ctx) -> int",
+        [](int64_t rows, int64_t nseq, int64_t hq, int64_t hkv, int64_t d, int64_t max_blocks, int64_t max_ctx) -> int64_t {
+          return bfly::attn_prefill_paged_scratch((int)rows, (int)nseq, (int)hq, (int)hkv, (int)d, (int)max_blocks, (int)max_ctx);
         });
   m.def("attn_prefill_paged(Tensor q, Tensor k_cache, Tensor v_cache, Tensor tables, Tensor cu_q, "
-        "Tensor positions, int max_q, float scale, Tensor(a!) out, Tensor(b!)? part=None) -> ()");
+        "Tensor positions, int max_q, float scale, Tensor(a!) out, Tensor(b!)? part=None, int max_ctx=0) -> ()");
   m.def("attn_prefill(Tensor q, Tensor k, Tensor v, Tensor cu_seqlens, int max_seqlen, float scale, "
         "bool causal, Tensor(a!) out, Tensor? cu_seqlens_k=None, Tensor(b!)? lse=None) -> ()");
   m.def("attn_lse_merge(Tensor(a!) acc_o, Tensor(b!) acc_lse, Tensor o, Tensor lse) -> ()");

@@ -170,9 +170,9 @@ int launch_attn_prefill_paged(const bf16* q, long q_stride, const void* k_cache,
                               const int* tables, int bt_stride, const int* cu_q, const int* positions,
                               int nseq, int max_q, int Hq, int Hkv, int D, int block_size, float scale,
                               bf16* out, long o_stride, hipStream_t stream, int kv_fp8 = 0, int rows = 0,
-                              float* part = nullptr, long part_floats = 0);
+                              float* part = nullptr, long part_floats = 0, int max_ctx = 0);
 // f32 values of `part` for a step over bf16 pages: 0, or the partial rows of the workgroups that share a tile's pages
-long attn_prefill_paged_scratch(int rows, int nseq, int Hq, int Hkv, int D, int max_blocks);
+long attn_prefill_paged_scratch(int rows, int nseq, int Hq, int Hkv, int D, int max_blocks, int max_ctx);
 // K16 (context parallel): acc_o [T, H, 128] f32 / acc_lse [T, H] f32 absorb (o, lse).
 int launch_attn_lse_merge(float* acc_o, float* acc_lse, const bf16* o, long o_stride,
                           const float* lse, int T, int H, int D, hipStream_t stream);

@@ -469,10 +469,12 @@ bool launch_attn_window_mfma_ext(const void* q, long q_ld, const void* k_cache, 
 int attn_window_tile_splits(int T, int H, int G, int nseq, int D, int Dv, int max_blocks, long fit);
 
 // launch_attn_prefill_paged takes the tiled kernel
-static bool paged_tiles(int rows, int nseq, int Hq, int Hkv) { return (long)rows * (Hq / Hkv) >= 128L * nseq && (long)rows * Hq >= 512; }
+static bool paged_tiles(int rows, int nseq, int Hq, int Hkv, int max_ctx) {
+  return (long)rows * (Hq / Hkv) >= 128L * nseq && (long)rows * Hq >= 512 && (max_ctx <= 0 || max_ctx > 256);
+}
 
-long attn_prefill_paged_scratch(int rows, int nseq, int Hq, int Hkv, int D, int max_blocks) {
-  if (rows <= 0 || Hkv <= 0 || Hq % Hkv != 0 || !paged_tiles(rows, nseq, Hq, Hkv)) return 0;
+long attn_prefill_paged_scratch(int rows, int nseq, int Hq, int Hkv, int D, int max_blocks, int max_ctx) {
+  if (rows <= 0 || Hkv <= 0 || Hq % Hkv != 0 || !paged_tiles(rows, nseq, Hq, Hkv, max_ctx)) return 0;
   // (64 MB at most; a step of more rows has tiles enough)
   const long split = (long)rows * Hq * (D + 2), n = attn_window_tile_splits(rows, Hq, Hkv, nseq, D, D, max_blocks, (1L << 24) / split);
   return n > 1 ? n * split : 0;
@@ -482,7 +484,7 @@ int launch_attn_prefill_paged(const bf16* q, long q_stride, const void* k_cache,
                               const int* tables, int bt_stride, const int* cu_q, const int* positions,
                               int nseq, int max_q, int Hq, int Hkv, int D, int block_size, float scale,
                               bf16* out, long o_stride, hipStream_t stream, int kv_fp8, int rows,
-                              float* part, long part_floats) {
+                              float* part, long part_floats, int max_ctx) {
   if (D != 128 || block_size != 32 || Hkv <= 0 || Hq % Hkv != 0) return -1;
   const int G = Hq / Hkv;
   if (G > 8) return -2;
@@ -491,9 +493,10 @@ int launch_attn_prefill_paged(const bf16* q, long q_stride, const void* k_cache,
   // bf16 pages, at least 128 (row, head) pairs of a key / value head per chunk: the tiled kernel of the windowed attention
   // (two row tiles per wave, pages staged once per 128 pairs and split over workgroups where chunks are few). 32 heads on
   // 8, us of the kernels below -> tiled: 900 rows over 3000 keys 318 -> 138, 2000 over 6000 1290 -> 374, 64 over 8000
-  // 331 -> 59, three chunks of 128 over 1000 56 -> 41, four of 1000 over 2000 404 -> 296 (0.55 PFLOP/s). Shorter chunks and
-  // FP8 pages keep the kernels below.
-  if (!kv_fp8 && paged_tiles(rows, nseq, Hq, Hkv) && q_stride % 8 == 0 &&
+  // 331 -> 59, three chunks of 128 over 1000 56 -> 41, four of 1000 over 2000 404 -> 296 (0.55 PFLOP/s). Shorter chunks,
+  // FP8 pages and contexts that are known to be short keep the kernels below (30 chunks of 60 rows over 32: 18 and 23 us, one of
+  // 100 rows over nothing 11 and 12; 16 of 200 over 200 72 and 59).
+  if (!kv_fp8 && paged_tiles(rows, nseq, Hq, Hkv, max_ctx) && q_stride % 8 == 0 &&
       reinterpret_cast<uintptr_t>(q) % 16 == 0) {
     AttnMod md;
     md.tiles = true;

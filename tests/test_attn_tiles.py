@@ -166,12 +166,13 @@ def test_rows_of_no_sequence_stay(start, n, rest):
 @pytest.mark.skipif(not ops.load_library(), reason="kernel library not built")
 def test_scratch_of_split_pages():
     """Scratch only where workgroups share a tile's pages: few tiles, enough pages; 64 MB at most."""
-    need = lambda *a: torch.ops.bfly.attn_prefill_paged_scratch(*a)                    # noqa: E731
+    need = lambda *a, ctx=0: torch.ops.bfly.attn_prefill_paged_scratch(*a, ctx)        # noqa: E731
     row = 32 * 130
     assert need(64, 1, 32, 8, 128, 250) == 8 * 64 * row          # a chunk over a long prefix
     assert need(64, 1, 32, 8, 128, 20) == 0                      # too few pages to share
     assert need(4000, 1, 32, 8, 128, 250) == 0                   # tiles enough
     assert need(15, 1, 32, 4, 128, 250) == 0 and need(0, 1, 32, 8, 128, 250) == 0      # not on the tiled kernel
+    assert need(64, 1, 32, 8, 128, 250, ctx=256) == 0 and need(64, 1, 32, 8, 128, 250, ctx=257) > 0      # nor short contexts
     for rows in (16, 100, 500, 900, 2000, 8000):
         for nseq in (1, 3, 16):
             for Hq, Hkv in ((32, 8), (64, 8), (8, 8), (64, 64)):
