@@ -391,7 +391,8 @@ class GevipelLM(PackedStack):
         q, k, v = y[:, :G * D].view(T, G, D), y[:, G * D:2 * G * D].view(T, G, D), y[:, 2 * G * D:].view(T, H, Dv)
         o1 = C + H * Dv
         o = ops.delta_scan(q, k, v, z[:, o1:o1 + H], z[:, o1 + H:o1 + 2 * H], p[pre + "A_log"], p[pre + "dt_bias"], S,
-                           meta["state_slots"], meta["row_cu"], fb.positions, D ** -0.5, UNIT_EPS)
+                           meta["state_slots"], meta["row_cu"], fb.positions, D ** -0.5, UNIT_EPS,
+                           max_rows=fb.max_seqlen if fb.is_prefill else 1)
         g = ops.gla_out(o, z[:, C:o1], p[pre + "gnorm"], self.cfg.norm_eps, self.dtype)
         return ops.linear_act(g, p[pre + "o"])
 

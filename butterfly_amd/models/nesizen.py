@@ -326,7 +326,7 @@ class NesizenLM(PackedStack):
         v, g = fz[:, o2:o3].view(T, H, Dv), fz[:, o3:o4]
         z = ops.linear_act(fz[:, o4:o4 + r], self.p[pre + "a2"], bias=self.p[pre + "a2b"])
         o = ops.gla_scan(q, k, v, z, self.state[self.state_index[sp["index"]]], meta["state_slots"], meta["row_cu"],
-                         fb.positions, sp["tau"], D ** -0.5)
+                         fb.positions, sp["tau"], D ** -0.5, max_rows=fb.max_seqlen if fb.is_prefill else 1)
         y = ops.gla_out(o, g, self.p[pre + "gnorm"], self.cfg.norm_eps, self.dtype)
         return ops.linear_act(y, self.p[pre + "o"])
 

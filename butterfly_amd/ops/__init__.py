@@ -912,13 +912,14 @@ def attn_window_paged(q, k_cache, v_cache, tables, row_cu, positions, scale: flo
     return out
 
 
-def gla_scan(q, k, v, z, state, state_slots, row_cu, positions, tau: float, q_scale: float):
+def gla_scan(q, k, v, z, state, state_slots, row_cu, positions, tau: float, q_scale: float, max_rows: int = 0):
     """Gated linear attention over packed rows with the state pooled in `state` [slots, H, D, Dv]
-    f32 (updated in place). Returns o [T, H, Dv] f32."""
+    f32 (updated in place). `max_rows`: the most rows of a sequence, where the caller knows it (it changes no result).
+    Returns o [T, H, Dv] f32."""
     if not _gpu(q):
         return ref.gla_scan(q, k, v, z, state, state_slots, row_cu, positions, tau, q_scale)
     o = _empty(q.shape[0], q.shape[1], v.shape[2], dtype=torch.float32, device=q.device)
-    torch.ops.bfly.gla_scan(q, k, v, z, state, state_slots, row_cu, positions, float(tau), float(q_scale), o)
+    torch.ops.bfly.gla_scan(q, k, v, z, state, state_slots, row_cu, positions, float(tau), float(q_scale), o, int(max_rows))
     return o
 
 
@@ -1317,16 +1318,16 @@ def short_conv_state_update_(z, state, state_slots, row_cu, positions):
 
 
 def delta_scan(q, k, v, b, a, a_log, dt_bias, state, state_slots, row_cu, positions, q_scale: float,
-               unit_eps: float = 1e-6):
+               unit_eps: float = 1e-6, max_rows: int = 0):
     """Gated delta rule over packed rows with the state pooled in `state` [slots, H, Dv, D] f32 (a
     head's D x Dv matrix stored column by column; updated in place; a sequence whose step starts at position 0 starts from zero). q, k [T, G, D],
     v [T, H, Dv] (views allowed); b, a [T, H] the logits of the write strength and the decay's step;
-    a_log, dt_bias [H] f32. See ops.reference.delta_scan. Returns o [T, H, Dv] f32."""
+    a_log, dt_bias [H] f32. `max_rows` as in gla_scan. See ops.reference.delta_scan. Returns o [T, H, Dv] f32."""
     if not _gpu(q):
         return ref.delta_scan(q, k, v, b, a, a_log, dt_bias, state, state_slots, row_cu, positions, q_scale, unit_eps)
     o = _empty(q.shape[0], v.shape[1], v.shape[2], dtype=torch.float32, device=q.device)
     torch.ops.bfly.delta_scan(q, k, v, b, a, a_log, dt_bias, state, state_slots, row_cu, positions, float(q_scale),
-                              float(unit_eps), o)
+                              float(unit_eps), o, int(max_rows))
     return o
 
 

@@ -135,7 +135,7 @@ void short_conv_state_update(const Tensor& z, Tensor& state, const Tensor& state
 
 void delta_scan(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& b, const Tensor& a, const Tensor& a_log,
                 const Tensor& dt_bias, Tensor& state, const Tensor& state_slots, const Tensor& row_cu,
-                const Tensor& positions, double q_scale, double unit_eps, Tensor& o) {
+                const Tensor& positions, double q_scale, double unit_eps, Tensor& o, int64_t max_rows) {
   CHK_HEADS_F32(q); CHK_HEADS_F32(k); CHK_HEADS_F32(v);
   CHK_GPU(b); CHK_GPU(a); CHK_SAME(a, b); CHK_GPU(a_log); CHK_GPU(dt_bias); CHK_GPU(state); CHK_GPU(o);
   CHK_F32(a_log); CHK_F32(dt_bias); CHK_F32(state); CHK_F32(o);
@@ -155,7 +155,7 @@ void delta_scan(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor&
                                          state.data_ptr<float>(), state_slots.data_ptr<int>(), row_cu.data_ptr<int>(),
                                          (int)state_slots.numel(), positions.data_ptr<int>(), (float)q_scale,
                                          (float)unit_eps, o.data_ptr<float>(), (int)T, (int)H, (int)G, (int)D, (int)Dv,
-                                         is_f32(b), cur_stream());
+                                         is_f32(b), cur_stream(), (int)max_rows);
   TORCH_CHECK(rc == 0, "delta_scan: key size ", D, " not supported (<= 256)");
 }
 
@@ -170,7 +170,7 @@ TORCH_LIBRARY_FRAGMENT(bfly, m) {
         "int act, Tensor(a!) out) -> ()");
   m.def("short_conv_state_update(Tensor z, Tensor(a!) state, Tensor state_slots, Tensor row_cu, Tensor positions) -> ()");
   m.def("delta_scan(Tensor q, Tensor k, Tensor v, Tensor b, Tensor a, Tensor a_log, Tensor dt_bias, Tensor(a!) state, "
-        "Tensor state_slots, Tensor row_cu, Tensor positions, float q_scale, float unit_eps, Tensor(b!) o) -> ()");
+        "Tensor state_slots, Tensor row_cu, Tensor positions, float q_scale, float unit_eps, Tensor(b!) o, int max_rows=0) -> ()");
 }
 
 TORCH_LIBRARY_IMPL(bfly, CUDA, m) {

@@ -301,7 +301,7 @@ void attn_window_paged(const Tensor& q, const Tensor& k_cache, const Tensor& v_c
 
 void gla_scan(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& z, Tensor& state,
               const Tensor& state_slots, const Tensor& row_cu, const Tensor& positions, double tau, double q_scale,
-              Tensor& o) {
+              Tensor& o, int64_t max_rows) {
   CHK_GPU(q); CHK_HEADS(q); CHK_HEADS(k); CHK_HEADS(v); CHK_SAME(k, q); CHK_SAME(v, q); CHK_SAME(z, q);
   CHK_F32(state); CHK_F32(o); CHK_I32(state_slots); CHK_I32(row_cu); CHK_I32(positions);
   const int64_t T = q.size(0), H = q.size(1), D = q.size(2), Dv = v.size(2);
@@ -316,7 +316,7 @@ void gla_scan(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& z
                                        z.data_ptr(), z.stride(0), state.data_ptr<float>(), state_slots.data_ptr<int>(),
                                        row_cu.data_ptr<int>(), (int)nseq, positions.data_ptr<int>(), (float)tau,
                                        (float)q_scale, o.data_ptr<float>(), (int)T, (int)H, (int)D, (int)Dv, is_f32(q),
-                                       cur_stream());
+                                       cur_stream(), (int)max_rows);
   TORCH_CHECK(rc == 0, "gla_scan: key size ", D, " not supported (<= 256)");
 }
 
@@ -476,7 +476,7 @@ TORCH_LIBRARY_FRAGMENT(bfly, m) {
         "float qt_coef=0., int qt_every=1, int maps=1, bool sigmoid=False, Tensor? key_bias=None, int pool=0, "
         "Tensor? k_pool=None, Tensor? v_pool=None, Tensor? gate=None, float out_mul=1., int dv_out=0) -> ()");
   m.def("gla_scan(Tensor q, Tensor k, Tensor v, Tensor z, Tensor(a!) state, Tensor state_slots, Tensor row_cu, "
-        "Tensor positions, float tau, float q_scale, Tensor(b!) o) -> ()");
+        "Tensor positions, float tau, float q_scale, Tensor(b!) o, int max_rows=0) -> ()");
   m.def("gla_out(Tensor o, Tensor g, Tensor norm_w, float eps, Tensor(a!) out) -> ()");
   m.def("router_logits(Tensor x, Tensor wr, Tensor(a!) logits) -> ()");
   m.def("moe_topk_scores(Tensor logits, Tensor? bias, int top_k, int scoring, bool renorm, Tensor(a!) ids, "

@@ -139,20 +139,23 @@ struct ExpertArgs {
   float* y = nullptr;               // down: f32 rows in pair order
 };
 
-// Scans over packed rows that come row by row and in chunks of 16 rows: which form takes which sequences of a step. A
-// sequence of `from` rows on is faster in chunks; the host knows only the sum, so a step that may hold both kinds launches both
-// forms, and every workgroup looks at its own sequence. The second launch (3 to 5 us) is saved where no sequence can
-// have rows enough to repay it (6 `from`, none of them empty), and for steps of prompts where the shorter sequences cost the
-// chunk form no more than that: `wgs` workgroups per sequence, at 11 to 25 ns for one with a single row.
+// Scans over packed rows that come row by row and in chunks of 16 rows: which form takes which sequences of a step. A chunk,
+// padded or not, takes the time of `cost` single rows: a sequence runs in chunks where that is no more than its rows. The host
+// knows only the sum of the rows, so a step that may hold both kinds launches both forms, and every workgroup looks at its own
+// sequence. The second launch (2 to 5 us) is saved where no sequence is long enough (max_rows, where the caller knows it) or
+// repays it (6 `cost` rows beyond one each, none of them empty), and for steps of prompts where the shorter sequences cost
+// the chunk form no more than that: `wgs` workgroups per sequence, at 11 to 25 ns for one with a single row.
 struct ScanForms {
   bool rows, chunks;
 };
-inline ScanForms scan_forms(long T, long nseq, int from, long wgs) {
-  if (nseq == 1) return {T < from, T >= from};
-  if (T - nseq < 6 * from) return {true, false};
-  return {!(T >= from * nseq && nseq * wgs <= 512), true};
+__host__ __device__ inline bool scan_in_chunks(long n, int cost) { return cost * ((n + 15) >> 4) <= n; }
+inline ScanForms scan_forms(long T, long nseq, int cost, long wgs, long max_rows) {
+  if (cost > 16) return {true, false};      // (a whole chunk takes longer than its rows)
+  if (nseq == 1) return {!scan_in_chunks(T, cost), scan_in_chunks(T, cost)};
+  if (T - nseq < 6 * cost || (max_rows > 0 && max_rows < cost)) return {true, false};
+  return {!(scan_in_chunks(T / nseq, cost) && nseq * wgs <= 512), true};
 }
-constexpr int kAllRows = 0x7fffffff;      // rows form: no sequence is left to the chunks
+// (`cost` 0 in a kernel: it takes every sequence)
 
 }  // namespace bfly
 

@@ -109,11 +109,12 @@ bool launch_attn_window_f32(const float* q, long q_ld, const float* k_cache, con
                             int keep_first, const float* sink, const float* out_scale, float* out, int T, int H, int G,
                             int D, int Dv, int block_size, hipStream_t s, const AttnMod& md);
 
-// Gated linear attention scan over packed rows (see ops.gla_scan). Returns < 0 if D > 256.
+// Gated linear attention scan over packed rows (see ops.gla_scan). Returns < 0 if D > 256. max_rows > 0: no sequence has
+// more rows
 int launch_gla_scan(const void* q, long q_ld, const void* k, long k_ld, const void* v, long v_ld, const void* z,
                     long z_ld, float* state, const int* state_slots, const int* row_cu, int nseq,
                     const int* positions, float tau, float q_scale, float* o, int T, int H, int D, int Dv, bool f32,
-                    hipStream_t s);
+                    hipStream_t s, int max_rows = 0);
 // out[t, h * Dv + j] = rms(o[t, h])[j] * w[j] * silu(g[t, h * Dv + j])
 void launch_gla_out(const float* o, const void* g, long g_ld, const float* norm_w, float eps, void* out, int T, int H,
                     int Dv, bool f32, hipStream_t s);

@@ -421,7 +421,7 @@ __global__ __launch_bounds__(512) void delta_scan_kernel(const float* __restrict
                                                          const int* __restrict__ row_cu,
                                                          const int* __restrict__ positions, float q_scale,
                                                          float unit_eps, float* __restrict__ o, int H, int G, int D,
-                                                         int Dv, int below) {
+                                                         int Dv, int cost) {
   constexpr int TB = 16, DP = 8 * NR, NT = 512, KQ = TB * DP / NT, VN = TB * 64 / NT;
   __shared__ __attribute__((aligned(16))) float sk[TB * DP], sq[TB * DP];
   __shared__ float sv[TB][64], so[TB][64];
@@ -434,7 +434,7 @@ __global__ __launch_bounds__(512) void delta_scan_kernel(const float* __restrict
   const bool live = col < Dv;
   const int r0 = row_cu[s], r1 = row_cu[s + 1];
   const int slot = state_slots[s];
-  if (r1 <= r0 || r1 - r0 >= below) return;      // (from `below` rows on: in chunks)
+  if (r1 <= r0 || (cost && scan_in_chunks(r1 - r0, cost))) return;      // (the chunk form's)
   if (slot < 0) {      // padding sequence of a fixed-shape step: defined output, no state
     for (int i = threadIdx.x; i < (r1 - r0) * 64; i += NT)
       if (c0 + (i & 63) < Dv) o[((long)(r0 + (i >> 6)) * H + h) * Dv + c0 + (i & 63)] = 0.f;
@@ -601,7 +601,7 @@ __global__ __launch_bounds__(512, NT <= 4 ? 4 : 2) void delta_chunk_kernel(
     const T* __restrict__ bl, long b_ld, const T* __restrict__ al, long a_ld, const float* __restrict__ a_log,
     const float* __restrict__ dt_bias, float* __restrict__ state, const int* __restrict__ state_slots,
     const int* __restrict__ row_cu, const int* __restrict__ positions, float q_scale, float unit_eps, int vec,
-    float* __restrict__ o, int H, int G, int D, int Dv, int from) {
+    float* __restrict__ o, int H, int G, int D, int Dv, int cost) {
   constexpr int C = 16, NQ = NT / 4, NG = NT / 4, NS = NT <= 8 ? 2 : 4, KP = 16 * NT + 4, PP = C + 4;
   extern __shared__ __attribute__((aligned(16))) float smem[];
   float* sk = smem;                       // [3][C][KP] raw k
@@ -622,7 +622,7 @@ __global__ __launch_bounds__(512, NT <= 4 ? 4 : 2) void delta_chunk_kernel(
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, m = lane & 15, gg = lane >> 4;
   const int r0 = __builtin_amdgcn_readfirstlane(row_cu[s]), r1 = __builtin_amdgcn_readfirstlane(row_cu[s + 1]);
   const int slot = state_slots[s];
-  if (r1 <= r0 || r1 - r0 < from) return;      // (below `from` rows: row by row)
+  if (r1 <= r0 || (cost && !scan_in_chunks(r1 - r0, cost))) return;      // (the row-by-row form's)
   if (slot < 0) {      // padding sequence of a fixed-shape step: defined output, no state
     for (int i = tid; i < (r1 - r0) * 64; i += 512)
       if (c0 + (i & 63) < Dv) o[((long)(r0 + (i >> 6)) * H + h) * Dv + c0 + (i & 63)] = 0.f;
@@ -1091,7 +1091,7 @@ template <typename T, int NT>
 static void delta_chunk_launch(const float* q, long q_ld, const float* k, long k_ld, const float* v, long v_ld, const T* b,
                                long b_ld, const T* a, long a_ld, const float* a_log, const float* dt_bias, float* state,
                                const int* state_slots, const int* row_cu, int nseq, const int* positions, float q_scale,
-                               float unit_eps, float* o, int H, int G, int D, int Dv, hipStream_t s, int from) {
+                               float unit_eps, float* o, int H, int G, int D, int Dv, hipStream_t s, int cost) {
   constexpr int C = 16;
   constexpr size_t lds = (size_t)(6 * C * (16 * NT + 4) + 18 * 256 + 24 * C + 4 * C * (C + 4) + 16 * C + 4) * sizeof(float);
   static bool once = false;
@@ -1106,24 +1106,28 @@ static void delta_chunk_launch(const float* q, long q_ld, const float* k, long k
   if (D % 4 == 0) vec |= 2;
   dim3 grid(nseq, H, (Dv + 63) / 64);
   delta_chunk_kernel<T, NT><<<grid, 512, lds, s>>>(q, q_ld, k, k_ld, v, v_ld, b, b_ld, a, a_ld, a_log, dt_bias, state, state_slots,
-                                                   row_cu, positions, q_scale, unit_eps, vec, o, H, G, D, Dv, from);
+                                                   row_cu, positions, q_scale, unit_eps, vec, o, H, G, D, Dv, cost);
 }
 
 template <typename T>
 static int delta_scan_t(const float* q, long q_ld, const float* k, long k_ld, const float* v, long v_ld, const T* b,
                         long b_ld, const T* a, long a_ld, const float* a_log, const float* dt_bias, float* state,
                         const int* state_slots, const int* row_cu, int nseq, const int* positions, float q_scale,
-                        float unit_eps, float* o, int T_, int H, int G, int D, int Dv, hipStream_t s) {
-  // Chunks from 12 rows of a sequence on: the loop below is faster where a chunk is mostly padding. 16 heads of 128, us of loop
-  // and chunks: one sequence of 6 rows 8.7 and 10.1; 16 of 6 16.5 and 20, of 16 26 and 20; 64 of 5 51 and 75. With each
-  // sequence in its own form: 32 single rows beside 128 114 and 63, now 58; 200 beside 300 249 and 291, now 173.
-  constexpr int from = 12;
-  ScanForms form = scan_forms(T_, nseq, from, (long)H * ((Dv + 63) / 64));
+                        float unit_eps, float* o, int T_, int H, int G, int D, int Dv, hipStream_t s, int max_rows) {
+  // A chunk takes the time of 10 rows of 128 channels while the workgroups all run at once, and of 14 where they queue (the
+  // loop's have half the LDS): 16 heads of 128, time of chunks over loop for one sequence of 8, 12, 16, 20, 32 rows 1.07, 0.88,
+  // 0.80, 0.85, 0.66, for 64 of them 1.24, 1.06, 1.05, 1.23, 0.91; channels of 64 0.82 and 0.94 at 16 rows, of 32 0.91 and 1.14,
+  // of 192 0.51 and 0.49. With each sequence in its own form: 32 single rows beside 128 114 and 63 us, now 58; 200 beside 300
+  // 249 and 291, now 173.
+  const long wgs = (long)H * ((Dv + 63) / 64);
+  const bool queue = nseq * wgs >= 1024;
+  const int cost = D > 128 ? 8 : D > 64 ? (queue ? 14 : 10) : D > 32 ? (queue ? 12 : 10) : queue ? 15 : 12;
+  ScanForms form = scan_forms(T_, nseq, cost, wgs, max_rows);
   if (D > 256) form = {true, false};
   if (form.chunks) {
 #define BFLY_DCH(NT)                                                                                                    \
   delta_chunk_launch<T, NT>(q, q_ld, k, k_ld, v, v_ld, b, b_ld, a, a_ld, a_log, dt_bias, state, state_slots, row_cu, nseq, \
-                            positions, q_scale, unit_eps, o, H, G, D, Dv, s, form.rows ? from : 0)
+                            positions, q_scale, unit_eps, o, H, G, D, Dv, s, form.rows ? cost : 0)
     if (D <= 64) BFLY_DCH(4);
     else if (D <= 128) BFLY_DCH(8);
     else if (D <= 192) BFLY_DCH(12);
@@ -1131,11 +1135,10 @@ static int delta_scan_t(const float* q, long q_ld, const float* k, long k_ld, co
 #undef BFLY_DCH
     if (!form.rows) return 0;
   }
-  const int below = form.chunks ? from : kAllRows;
   dim3 grid(nseq, H, (Dv + 63) / 64);
 #define BFLY_DELTA(NR)                                                                                             \
   delta_scan_kernel<T, NR><<<grid, 512, 0, s>>>(q, q_ld, k, k_ld, v, v_ld, b, b_ld, a, a_ld, a_log, dt_bias, state, \
-                                                state_slots, row_cu, positions, q_scale, unit_eps, o, H, G, D, Dv, below)
+                                                state_slots, row_cu, positions, q_scale, unit_eps, o, H, G, D, Dv, form.chunks ? cost : 0)
   if (D <= 32) BFLY_DELTA(4);
   else if (D <= 64) BFLY_DELTA(8);
   else if (D <= 128) BFLY_DELTA(16);
@@ -1148,13 +1151,14 @@ static int delta_scan_t(const float* q, long q_ld, const float* k, long k_ld, co
 int launch_delta_scan(const float* q, long q_ld, const float* k, long k_ld, const float* v, long v_ld, const void* b,
                       long b_ld, const void* a, long a_ld, const float* a_log, const float* dt_bias, float* state,
                       const int* state_slots, const int* row_cu, int nseq, const int* positions, float q_scale,
-                      float unit_eps, float* o, int T, int H, int G, int D, int Dv, bool f32, hipStream_t s) {
+                      float unit_eps, float* o, int T, int H, int G, int D, int Dv, bool f32, hipStream_t s, int max_rows) {
   if (T <= 0 || nseq <= 0) return 0;
   if (f32)
     return delta_scan_t<float>(q, q_ld, k, k_ld, v, v_ld, (const float*)b, b_ld, (const float*)a, a_ld, a_log, dt_bias,
-                               state, state_slots, row_cu, nseq, positions, q_scale, unit_eps, o, T, H, G, D, Dv, s);
+                               state, state_slots, row_cu, nseq, positions, q_scale, unit_eps, o, T, H, G, D, Dv, s,
+                               max_rows);
   return delta_scan_t<bf16>(q, q_ld, k, k_ld, v, v_ld, (const bf16*)b, b_ld, (const bf16*)a, a_ld, a_log, dt_bias, state,
-                            state_slots, row_cu, nseq, positions, q_scale, unit_eps, o, T, H, G, D, Dv, s);
+                            state_slots, row_cu, nseq, positions, q_scale, unit_eps, o, T, H, G, D, Dv, s, max_rows);
 }
 
 }  // namespace bfly

@@ -76,7 +76,7 @@ __global__ __launch_bounds__(512, NT <= 8 ? 4 : 2) void forget_chunk_kernel(cons
                                                            const int* __restrict__ state_slots,
                                                            const int* __restrict__ row_cu,
                                                            const int* __restrict__ positions, int act, int vec,
-                                                           float* __restrict__ o, int H, int D, int Dv, int from) {
+                                                           float* __restrict__ o, int H, int D, int Dv, int cost) {
   constexpr int C = 16, DP = 16 * NT, NH = NT / 2, NU = (DP + 127) / 128, KP = 128 * NU + 4, VP = 68, PP = C + 4;
   constexpr int NI = (2 * DP + 255) / 256, HC = C / 2, NP = NT < 8 ? NT : 8;
   constexpr bool FAST = sizeof(T) == 2, WHOLE = NI * 256 == 2 * DP;
@@ -95,7 +95,7 @@ __global__ __launch_bounds__(512, NT <= 8 ? 4 : 2) void forget_chunk_kernel(cons
   float* sl = sph + NP * HC * HC;       // [DP] F of the last row
   const int s = blockIdx.x, h = blockIdx.y, c0 = blockIdx.z * 64;
   const int r0 = __builtin_amdgcn_readfirstlane(row_cu[s]), r1 = __builtin_amdgcn_readfirstlane(row_cu[s + 1]);
-  if (r1 <= r0 || r1 - r0 < from) return;      // (below `from` rows: row by row)
+  if (r1 <= r0 || (cost && !scan_in_chunks(r1 - r0, cost))) return;      // (the row-by-row form's)
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, m = lane & 15, gg = lane >> 4;
   const int slot = state_slots[s];
   if (slot < 0) {      // padding sequence of a fixed-shape step: defined output, no state
@@ -499,7 +499,7 @@ __global__ __launch_bounds__(256) void head_norm_gate_kernel(const float* __rest
 template <typename T, int NT, bool GLA>
 void forget_chunk_launch(const T* q, long q_ld, const T* key, long k_ld, float inv_tau, float q_scale, const T* z, long z_ld, const T* v, long v_ld, const float* f_bias,
                          const float* lower, float* state, const int* state_slots, const int* row_cu, int nseq,
-                         const int* positions, int act, int vec, float* o, int H, int D, int Dv, hipStream_t s, int from) {
+                         const int* positions, int act, int vec, float* o, int H, int D, int Dv, hipStream_t s, int cost) {
   constexpr int DP = 16 * NT, KP = (DP + 127) / 128 * 128 + 4;
   constexpr size_t lds = (size_t)(97 * KP + 2 * 16 * 68 + 16 * 20 + 64 * (NT < 8 ? NT : 8) + DP) * sizeof(float);
   static bool once = false;
@@ -510,7 +510,7 @@ void forget_chunk_launch(const T* q, long q_ld, const T* key, long k_ld, float i
   }
   dim3 grid(nseq, H, (Dv + 63) / 64);
   forget_chunk_kernel<T, NT, GLA><<<grid, 512, lds, s>>>(q, q_ld, key, k_ld, inv_tau, q_scale, z, z_ld, v, v_ld, f_bias, lower,
-                                                         state, state_slots, row_cu, positions, act, vec, o, H, D, Dv, from);
+                                                         state, state_slots, row_cu, positions, act, vec, o, H, D, Dv, cost);
 }
 
 template <typename T>
@@ -542,11 +542,11 @@ void forget_scan_t(const T* q, long q_ld, const T* z, long z_ld, const T* v, lon
 template <typename T>
 void gla_chunks_t(const T* q, long q_ld, const T* k, long k_ld, const T* v, long v_ld, const T* z, long z_ld, float* state,
                   const int* state_slots, const int* row_cu, int nseq, const int* positions, float tau, float q_scale, float* o,
-                  int H, int D, int Dv, hipStream_t s, int from) {
+                  int H, int D, int Dv, hipStream_t s, int cost) {
   const int vec = (Dv % 4 == 0 && rows_aligned(v, v_ld, sizeof(T))) ? 2 : 0;
 #define BFLY_GCH(NT)                                                                                                   \
   forget_chunk_launch<T, NT, true>(q, q_ld, k, k_ld, 1.f / tau, q_scale, z, z_ld, v, v_ld, nullptr, nullptr, state,    \
-                                   state_slots, row_cu, nseq, positions, 0, vec, o, H, D, Dv, s, from)
+                                   state_slots, row_cu, nseq, positions, 0, vec, o, H, D, Dv, s, cost)
   if (D <= 32) BFLY_GCH(2);
   else if (D <= 64) BFLY_GCH(4);
   else if (D <= 96) BFLY_GCH(6);
@@ -587,13 +587,13 @@ void launch_forget_scan(const void* q, long q_ld, const void* z, long z_ld, cons
 
 void launch_gla_chunks(const void* q, long q_ld, const void* k, long k_ld, const void* v, long v_ld, const void* z, long z_ld,
                        float* state, const int* state_slots, const int* row_cu, int nseq, const int* positions, float tau,
-                       float q_scale, float* o, int H, int D, int Dv, bool f32, hipStream_t s, int from) {
+                       float q_scale, float* o, int H, int D, int Dv, bool f32, hipStream_t s, int cost) {
   if (f32)
     gla_chunks_t<float>((const float*)q, q_ld, (const float*)k, k_ld, (const float*)v, v_ld, (const float*)z, z_ld, state,
-                        state_slots, row_cu, nseq, positions, tau, q_scale, o, H, D, Dv, s, from);
+                        state_slots, row_cu, nseq, positions, tau, q_scale, o, H, D, Dv, s, cost);
   else
     gla_chunks_t<bf16>((const bf16*)q, q_ld, (const bf16*)k, k_ld, (const bf16*)v, v_ld, (const bf16*)z, z_ld, state,
-                       state_slots, row_cu, nseq, positions, tau, q_scale, o, H, D, Dv, s, from);
+                       state_slots, row_cu, nseq, positions, tau, q_scale, o, H, D, Dv, s, cost);
 }
 
 void launch_head_norm_gate(const float* o, const float* w, float eps, const void* gate, long g_ld, int act, float mul,

@@ -86,7 +86,7 @@ __global__ __launch_bounds__(512) void gla_scan_kernel(const T* __restrict__ q, 
                                                        const int* __restrict__ row_cu,
                                                        const int* __restrict__ positions, float inv_tau,
                                                        float q_scale, float* __restrict__ o, int H, int D, int Dv,
-                                                       int below) {
+                                                       int cost) {
   constexpr int TB = 16, DP = 8 * NR, NT = 512;
   __shared__ __attribute__((aligned(16))) float sa[TB * DP], sk[TB * DP], sq[TB * DP];
   __shared__ float sv[TB][64], so[TB][64];
@@ -97,7 +97,7 @@ __global__ __launch_bounds__(512) void gla_scan_kernel(const T* __restrict__ q, 
   const bool live = col < Dv;
   const int r0 = row_cu[s], r1 = row_cu[s + 1];
   const int slot = state_slots[s];
-  if (r1 <= r0 || r1 - r0 >= below) return;      // (from `below` rows on: in chunks)
+  if (r1 <= r0 || (cost && scan_in_chunks(r1 - r0, cost))) return;      // (the chunk form's)
   if (slot < 0) {      // padding sequence of a fixed-shape step: defined output, no state
     for (int i = threadIdx.x; i < (r1 - r0) * 64; i += NT)
       if (c0 + (i & 63) < Dv) o[((long)(r0 + (i >> 6)) * H + h) * Dv + c0 + (i & 63)] = 0.f;
@@ -493,12 +493,12 @@ void launch_attn_window_paged(const void* q, long q_ld, const void* k_cache, con
 template <typename T>
 static int gla_scan_t(const T* q, long q_ld, const T* k, long k_ld, const T* v, long v_ld, const T* z, long z_ld,
                       float* state, const int* state_slots, const int* row_cu, int nseq, const int* positions,
-                      float tau, float q_scale, float* o, int H, int D, int Dv, hipStream_t s, int below) {
+                      float tau, float q_scale, float* o, int H, int D, int Dv, hipStream_t s, int cost) {
   dim3 grid(nseq, H, (Dv + 63) / 64);
   const float it = 1.f / tau;
 #define BFLY_GLA(NR)                                                                                              \
   gla_scan_kernel<T, NR><<<grid, 512, 0, s>>>(q, q_ld, k, k_ld, v, v_ld, z, z_ld, state, state_slots, row_cu, positions, \
-                                              it, q_scale, o, H, D, Dv, below)
+                                              it, q_scale, o, H, D, Dv, cost)
   if (D <= 32) BFLY_GLA(4);
   else if (D <= 64) BFLY_GLA(8);
   else if (D <= 128) BFLY_GLA(16);
@@ -510,30 +510,36 @@ static int gla_scan_t(const T* q, long q_ld, const T* k, long k_ld, const T* v, 
 
 void launch_gla_chunks(const void* q, long q_ld, const void* k, long k_ld, const void* v, long v_ld, const void* z, long z_ld,
                        float* state, const int* state_slots, const int* row_cu, int nseq, const int* positions, float tau,
-                       float q_scale, float* o, int H, int D, int Dv, bool f32, hipStream_t s, int from);      // forget.hip
+                       float q_scale, float* o, int H, int D, int Dv, bool f32, hipStream_t s, int cost);      // forget.hip
 
 int launch_gla_scan(const void* q, long q_ld, const void* k, long k_ld, const void* v, long v_ld, const void* z,
                     long z_ld, float* state, const int* state_slots, const int* row_cu, int nseq,
                     const int* positions, float tau, float q_scale, float* o, int T, int H, int D, int Dv, bool f32,
-                    hipStream_t s) {
+                    hipStream_t s, int max_rows) {
   if (T <= 0 || nseq <= 0) return 0;
-  // Chunks on the f32 matrix cores from 16 rows of a sequence on (true f32: 32), the token loop above where a chunk is mostly
-  // padding. 16 heads of 128, us of loop and chunks: one sequence of 8 rows 9.4 and 10.5, of 16 13.1 and 10.4 (f32 15.3 and
-  // 14.2, of 24 20.5 and 21.1); 16 of 4 11.6 and 18; 200 single rows beside 2 95 and 166. With each sequence in its own form:
-  // 32 single rows beside 128 87 and 66, now 67; 200 beside 256 218 and 224, now 176 (f32 249 and 352, now 198).
-  const int from = f32 ? 32 : 16;
-  ScanForms form = scan_forms(T, nseq, from, (long)H * ((Dv + 63) / 64));
+  // A chunk on the f32 matrix cores takes the time of 12 rows of 128 channels, in true f32 (whose decays are precise
+  // functions) of 14, and somewhat more where the workgroups queue. 16 heads of 128, time of chunks over loop for one sequence of
+  // 8, 12, 16, 20, 32 rows: 1.09, 0.93, 0.79, 0.93, 0.69 (f32 1.43, 1.18, 0.93, 1.18, 0.83), for 200 of them 1.53, 1.26, 1.02,
+  // 1.04, 0.74 (1.87, 1.47, 1.07, 1.25, 0.76); channels of 64 0.88 and 0.99 (1.03 and 1.30) at 16 rows, of 32 0.97 and 1.24 (1.14
+  // and 1.58), of 192 0.53 and 0.52 (0.56 and 0.52). With each sequence in its own form: 32 single rows beside 128 87 and 66 us,
+  // now 67; 200 beside 256 218 and 224, now 176 (f32 249 and 352, now 198).
+  const long wgs = (long)H * ((Dv + 63) / 64);
+  const bool queue = nseq * wgs >= 1024;
+  int cost;
+  if (f32) cost = D > 128 ? 11 : D > 64 ? (queue ? 15 : 14) : D > 32 && !queue ? 15 : 18;
+  else cost = D > 128 ? 9 : D > 64 ? (queue ? 13 : 12) : D > 32 ? (queue ? 15 : 14) : queue ? 18 : 15;
+  ScanForms form = scan_forms(T, nseq, cost, wgs, max_rows);
   if (D > 256 || std::max({q_ld, k_ld, z_ld}) >= (1L << 21)) form = {true, false};
   if (form.chunks)
     launch_gla_chunks(q, q_ld, k, k_ld, v, v_ld, z, z_ld, state, state_slots, row_cu, nseq, positions, tau, q_scale, o, H, D,
-                      Dv, f32, s, form.rows ? from : 0);
+                      Dv, f32, s, form.rows ? cost : 0);
   if (!form.rows) return 0;
-  const int below = form.chunks ? from : kAllRows;
+  if (!form.chunks) cost = 0;
   if (f32)
     return gla_scan_t<float>((const float*)q, q_ld, (const float*)k, k_ld, (const float*)v, v_ld, (const float*)z, z_ld,
-                             state, state_slots, row_cu, nseq, positions, tau, q_scale, o, H, D, Dv, s, below);
+                             state, state_slots, row_cu, nseq, positions, tau, q_scale, o, H, D, Dv, s, cost);
   return gla_scan_t<bf16>((const bf16*)q, q_ld, (const bf16*)k, k_ld, (const bf16*)v, v_ld, (const bf16*)z, z_ld, state,
-                          state_slots, row_cu, nseq, positions, tau, q_scale, o, H, D, Dv, s, below);
+                          state_slots, row_cu, nseq, positions, tau, q_scale, o, H, D, Dv, s, cost);
 }
 
 void launch_head_norm_gate(const float* o, const float* w, float eps, const void* gate, long g_ld, int act, float mul,

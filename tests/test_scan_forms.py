@@ -11,6 +11,7 @@ STEPS = {
     "one prompt": [(3, 45)],
     "prompts alone": [(0, 70), (5, 33), (0, 40)],                                          # one launch of chunks
     "mixed": [(9, 1)] * 30 + [(0, 16), (4, 15), (0, 12), (8, 11), (20, 61), (0, 32), (3, 31)],
+    "a chunk and a little": [(9, 1)] * 20 + [(0, 17), (3, 20), (0, 24), (7, 28), (0, 33)],   # whether a padded chunk pays
     "empty and padded": [(9, 1)] * 9 + [(0, 0), (0, 50), (0, 0), (6, 14)] + [(1, 1)] * 3,      # (the last two: no slot)
 }
 
@@ -43,11 +44,12 @@ def test_every_sequence_of_a_mixed_step(which, name, H):
     T, n, D, Dv = len(pos), len(slots), 48, 96
     rows = torch.cat([torch.arange(int(a), int(b)) for a, b, s in zip(cu, cu[1:], slots) if s >= 0])
     idx = dict(state_slots=slots, row_cu=cu, positions=pos)
+    hint = {"max_rows": max(m for _, m in STEPS[name])} if H == 2 else {}
     if which == "delta":
         same(ops.delta_scan, dict(q=rnd(T, H // 2, D), k=rnd(T, H // 2, D), v=rnd(T, H, Dv), b=rnd(T, H), a=rnd(T, H), a_log=rnd(H) - 1,
-                                  dt_bias=rnd(H), state=rnd(n, H, Dv, D), **idx), rows, q_scale=D ** -0.5)
+                                  dt_bias=rnd(H), state=rnd(n, H, Dv, D), **idx), rows, q_scale=D ** -0.5, **hint)
         return
     dt = torch.bfloat16 if "bf16" in which else torch.float32
     x = dict(q=rnd(T, H, D).to(dt), k=rnd(T, H, D).to(dt), v=rnd(T, H, Dv).to(dt), z=(2 + rnd(T, H * D)).to(dt),
              state=rnd(n, H, D, Dv), **idx)
-    same(ops.gla_scan, x, rows, tau=16.0, q_scale=D ** -0.5)
+    same(ops.gla_scan, x, rows, tau=16.0, q_scale=D ** -0.5, **hint)
