@@ -179,13 +179,8 @@ def reserve_workspace(device, max_tokens: int, max_n: int, max_k: int, max_batch
     more than the largest one is split) and every number of row tiles (a split's sums do not grow with the rows)."""
     if not load_library():
         return
-    ws = 0
     nk = {(int(max_n), int(max_k))} | {(int(n), int(k)) for n, k in shapes}
-    for m in sorted({1, 16, 32, 48, 64, *range(128, max_tokens, 128), max_tokens}):
-        if m > max_tokens:
-            continue
-        for n, k in nk:
-            ws = max(ws, torch.ops.bfly.gemm_workspace_size(m, n, k))
+    ws = max(torch.ops.bfly.gemm_workspace_bound(int(max_tokens), n, k) for n, k in nk)
     _arena.get(device, "gemm", ws // 4 + 1, torch.float32, zero=True)
     if max_batch and max_ctx:
         ns = max(torch.ops.bfly.attn_decode_splits(max_ctx, torch.ops.bfly.attn_decode_part_tokens(b, num_kv_heads, max_ctx))

@@ -340,6 +340,16 @@ void tkp_final(Tensor& ws, int64_t rows, Tensor& thresh) {
   bfly::launch_tkp_final(v.state, rows, thresh.data_ptr<float>(), cur_stream());
 }
 
+// the most that any number of rows up to M asks for: the plan table's counts and every number of whole row tiles
+int64_t gemm_workspace_bound(int64_t M, int64_t N, int64_t K) {
+  if (M < 1) return 0;
+  size_t need = bfly::gemm_workspace_bytes((int)M, (int)N, (int)K);
+  for (int64_t m : {1, 16, 32, 48, 64})
+    if (m < M) need = std::max(need, bfly::gemm_workspace_bytes((int)m, (int)N, (int)K));
+  for (int64_t m = 128; m < M; m += 128) need = std::max(need, bfly::gemm_workspace_bytes((int)m, (int)N, (int)K));
+  return (int64_t)need;
+}
+
 int64_t gemm_workspace_size(int64_t M, int64_t N, int64_t K) {
   return (int64_t)bfly::gemm_workspace_bytes(M, N, K);
 }
@@ -1199,6 +1209,7 @@ TORCH_LIBRARY(bfly, m) {
   m.def("gemm_with_plan(Tensor x, Tensor w, Tensor(a!) out, int[] plan, int epilogue, Tensor(b!)? workspace, "
         "Tensor? bias=None) -> ()");
   m.def("gemm_workspace_size(int M, int N, int K) -> int", &gemm_workspace_size);
+  m.def("gemm_workspace_bound(int M, int N, int K) -> int", &gemm_workspace_bound);
   m.def("gemm_plan(int M, int N, int K) -> int[]", &gemm_plan);
   m.def("gemm_check(int M, int N, int K, int epilogue) -> int",
         [](int64_t M, int64_t N, int64_t K, int64_t e) -> int64_t { return bfly::gemm_check(M, N, K, e); });
