@@ -319,7 +319,8 @@ __device__ __forceinline__ bf16x8 lds_frag(const char* lds, int row, int chunk) 
 // `pslab`: this workgroup's split-K slab from row m0 on (nullptr: apply the epilogue).
 // `rsc`: RMSNorm row scale of a consumer GEMM (RowScale, ss == nullptr: none), applied to the
 // accumulators first, so split-K slabs, the bias and the SiLU all see the normalised rows.
-template <int TI, int TJ>
+// PLAIN: the caller has applied EPI_BIAS and EPI_RELU2 itself.
+template <int TI, int TJ, bool PLAIN = false>
 __device__ __forceinline__ void tile_epilogue(const f32x4 (&acc)[TI][TJ], int mw, int nw, int lane,
                                               int M, int N, int epi, const bf16* __restrict__ bias,
                                               bf16* __restrict__ out, long ldo, float* __restrict__ pslab,
@@ -387,11 +388,11 @@ __device__ __forceinline__ void tile_epilogue(const f32x4 (&acc)[TI][TJ], int mw
         }
       } else {
         f32x4 v = acc[i][j] * sc[i];
-        if (epi == EPI_BIAS) {
+        if (!PLAIN && epi == EPI_BIAS) {
 #pragma unroll
           for (int r = 0; r < 4; ++r) v[r] += bf2f(bias[n + r]);
         }
-        if (epi == EPI_RELU2) {
+        if (!PLAIN && epi == EPI_RELU2) {
 #pragma unroll
           for (int r = 0; r < 4; ++r) v[r] = fmaxf(v[r], 0.f) * fmaxf(v[r], 0.f);
         }
@@ -960,10 +961,11 @@ __device__ __forceinline__ void b4_dma(__amdgpu_buffer_rsrc_t r, char* lds, int 
 // [gate | up]), so the clamped GLU runs on a lane's own accumulators; an expert that runs on (score x row) scales
 // the accumulators by the score instead of rounding scaled rows. The down projection leaves f32 rows at their
 // (token, choice) pair. Measured beside the smaller tiles: moe_tile_rows.
-// BIAS: the bias epilogue with the columns' values read once for all rows. Read row by row in tile_epilogue, each load waited
-// for by the only wave of its SIMD, they took 13 to 50 us of a product; in an instance of its own because
-// the branch alone costs the other epilogues 3 us.
-template <int GROUPED = 0, bool BIAS = false>
+// E: the epilogue (-1: `epi`), in instances of their own because the branches of the others cost each of them up to 3 us, and
+// with every epilogue added more (8192 x 57344 x 8192 SwiGLU 5050 us with four of them, 5066 with five, 5028 alone).
+// EPI_BIAS reads the columns' values once for all rows (row by row in tile_epilogue, each load waited for by the only wave of its
+// SIMD, they took 13 to 50 us of a product).
+template <int GROUPED = 0, int E = -1>
 __global__ void __launch_bounds__(kB4Threads) __attribute__((amdgpu_waves_per_eu(1, 1)))
 gemm_big4_kernel(const bf16* __restrict__ X, long ldx, const bf16* __restrict__ W, long ldw,
                  int M, int N, int K, int epi, const bf16* __restrict__ bias,
@@ -1163,7 +1165,17 @@ gemm_big4_kernel(const bf16* __restrict__ X, long ldx, const bf16* __restrict__ 
     return;
   }
   if (n0 + wc * 128 >= N) return;     // the columns past N of a half tile (their weight rows read zeros)
-  if constexpr (BIAS) {
+  if constexpr (E >= 0) epi = E;
+  if constexpr (E == EPI_RELU2) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) acc[i][j][r] = fmaxf(acc[i][j][r], 0.f) * fmaxf(acc[i][j][r], 0.f);
+    epi = EPI_NONE;
+  }
+  if constexpr (E == EPI_BIAS) {
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
       f32x4 b;
@@ -1174,7 +1186,7 @@ gemm_big4_kernel(const bf16* __restrict__ X, long ldx, const bf16* __restrict__ 
     }
     epi = EPI_NONE;
   }
-  tile_epilogue<8, 8>(acc, m0 + wr * 128, n0 + wc * 128, lane, M, N, epi, bias, out, ldo,
+  tile_epilogue<8, 8, GROUPED == 0>(acc, m0 + wr * 128, n0 + wc * 128, lane, M, N, epi, bias, out, ldo,
                       part ? part + (long)blockIdx.y * M * N + (long)m0 * N : nullptr, m0,
                       RowScale{nullptr, 0, 0.f, 0.f});
 }
@@ -1632,20 +1644,24 @@ static void run_big8(const bf16* X, long ldx, const bf16* W, long ldw, int M, in
 
 static void run_big4(const bf16* X, long ldx, const bf16* W, long ldw, int M, int N, int K,
                      int epi, const bf16* bias, bf16* out, long ldo, float* ws, int sk, hipStream_t stream) {
-  static bool attr_set = false;
-  if (!attr_set) {
-    hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_big4_kernel<0>),
-                        hipFuncAttributeMaxDynamicSharedMemorySize, kB4LdsBytes);
-    hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_big4_kernel<0, true>),
-                        hipFuncAttributeMaxDynamicSharedMemorySize, kB4LdsBytes);
-    attr_set = true;
-  }
   dim3 grid(((M + 255) / 256) * ((N + 255) / 256), sk);
   float* part = sk > 1 ? splitk_part(ws) : nullptr;
-  if (epi == EPI_BIAS && sk == 1)      // (with a split K the reduce adds the bias)
-    gemm_big4_kernel<0, true><<<grid, kB4Threads, kB4LdsBytes, stream>>>(X, ldx, W, ldw, M, N, K, epi, bias, out, ldo, nullptr);
-  else
-    gemm_big4_kernel<0><<<grid, kB4Threads, kB4LdsBytes, stream>>>(X, ldx, W, ldw, M, N, K, epi, bias, out, ldo, part);
+#define BFLY_BIG4(E)                                                                                                     \
+  {                                                                                                                      \
+    static bool attr_set = false;                                                                                        \
+    if (!attr_set) {                                                                                                     \
+      hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_big4_kernel<0, E>),                                        \
+                          hipFuncAttributeMaxDynamicSharedMemorySize, kB4LdsBytes);                                      \
+      attr_set = true;                                                                                                   \
+    }                                                                                                                    \
+    gemm_big4_kernel<0, E><<<grid, kB4Threads, kB4LdsBytes, stream>>>(X, ldx, W, ldw, M, N, K, epi, bias, out, ldo, part); \
+  }
+  if (sk > 1 || epi == EPI_NONE) BFLY_BIG4(EPI_NONE)      // (with a split K the reduce applies the epilogue)
+  else if (epi == EPI_SILU) BFLY_BIG4(EPI_SILU)
+  else if (epi == EPI_BIAS) BFLY_BIG4(EPI_BIAS)
+  else if (epi == EPI_RELU2) BFLY_BIG4(EPI_RELU2)
+  else BFLY_BIG4(-1)
+#undef BFLY_BIG4
 }
 
 template <int BM, int BN, int SA, int SB, bool PK = false>
