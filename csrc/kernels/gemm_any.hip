@@ -1,5 +1,5 @@
 // Shape-generic GEMM family: any (M, N, K), bf16 or f32 operands, f32 accumulation in K order
-// (the sum of an output element never depends on M or on the other rows of the batch).
+// (in launch_gemm_any the sum of an output element never depends on M or on the other rows of the batch).
 // 64 x 64 or 128 x 128 output tile and 256 threads in both forms, operands staged through LDS with bounds
 // checks, so no shape or alignment restriction. f32 operands: 32-deep K step on the f32 matrix cores
 // (tile_mac_f32). bf16 operands: 64-deep K step staged as bf16, a quadrant per wave as MFMA 16x16x32
@@ -8,7 +8,10 @@
 // grouped expert GEMMs of a score-routed MoE with clamped GLU experts: rows are grouped by
 // expert (moe_sort_kernel), the up kernel gathers token rows scaled by their routing score and
 // applies the GLU to a (gate, up) accumulator pair, the down kernel scatters f32 rows back to
-// (token, choice) order for a fixed-order sum.
+// (token, choice) order for a fixed-order sum. The experts have two more forms in bf16, chosen by the step's (token, choice)
+// pairs per expert: weights streamed past few rows (moe_up / down_stream_kernel, four interleaved partial sums over K) and
+// 256-row tiles (gemm_big4_kernel, the score applied to the sums where the other forms round the scaled row to bf16). So an
+// expert row's rounding follows the size of the step, not the values of its other rows.
 #include <algorithm>
 
 #include "bfly_common.h"
@@ -1025,7 +1028,11 @@ bool moe_big_ok(const void* x, long ldx, const void* gate_up_w, const void* down
 // 256-row tiles: width 2048, GLU of 2048, 8192 tokens 1343 -> 458 (0.95 PFLOP/s in the two GEMMs), 1024 tokens 144 -> 112,
 // 768 tokens 117 -> 107, but 512 tokens 98 -> 102; width 4096, 4096: 8192 tokens 4774 -> 1397, 512 tokens 352 -> 295;
 // width 1024, plain 1536: 2048 tokens 103 -> 82, but 1024 tokens 66 -> 77. Shapes outside moe_big_ok: 128-row tiles
-// from 512 rows (bf16 only), else 64.
+// from 512 rows (bf16 only), else 64. Over 20 stacks of 2 to 256 experts (1 to 8 choices, widths 512 to 7168, 1 to 8192
+// tokens; 217 steps, all forms timed) the choice is never slower than the tiles before these forms; beside the best
+// form it is level but for the last doubling below a line where there are many experts or column tiles: 128 experts of 768, 8
+// choices, 2048 tokens 620 us and 492 on the 256-row tiles, 32 of 512 (width 1024), 4096 tokens 117 and 81; two experts of
+// 4096, 512 tokens 129 and 99 on the 64-row tiles.
 int moe_tile_rows(int TKp, int E, bool f32, bool big, int Hd) {
   if (big && TKp >= (Hd >= 4096 ? 128 : Hd >= 2048 ? 160 : 384) * E) return 256;
   return (!f32 && TKp >= 512 * E) ? 128 : 64;
@@ -1034,7 +1041,8 @@ int moe_tile_rows(int TKp, int E, bool f32, bool big, int Hd) {
 // Up to an average of 24 rows per expert (12 from width 4096 on) the weights stream past the rows. Whole op, 8 experts, two
 // choices, us of 64-row tiles -> streams: width 2048, GLU of 2048: 1 token 48 -> 22, 16 tokens 53 -> 49, 64 tokens (16 rows
 // per expert) 56 -> 53, but 128 tokens 57 -> 67; width 1024, 1024: 31 -> 15, 32 -> 20, 35 -> 24; width 4096, plain 6144: 16
-// tokens 202 -> 169, but 64 tokens 205 -> 216.
+// tokens 202 -> 169, but 64 tokens 205 -> 216. Many experts: 64 of 1408, 6 choices, 128 tokens (12 rows per expert) 251 -> 244,
+// 256 tokens 269 -> 292; 256 of 512, 8 choices, 512 tokens (16) 397 -> 384.
 bool moe_stream_ok(const void* x, long ldx, const void* gate_up_w, const void* down_w, const void* hmid, const void* y,
                    int TKp, int E, int Hd, int F, bool f32) {
   return !f32 && TKp <= (Hd >= 4096 ? 12 : 24) * E && Hd % 64 == 0 && F % 64 == 0 && rows16(x, ldx, 2) &&
