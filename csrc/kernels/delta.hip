@@ -571,7 +571,8 @@ __device__ __forceinline__ void lds_wave_sync() {
   __builtin_amdgcn_wave_barrier();
 }
 
-// Steps with more rows than sequences (prompts): chunks of 16 rows on the f32 matrix cores. Row by row every token is
+// Steps with more rows than sequences (prompts): chunks of 16 rows on the f32 matrix cores, in the published chunkwise form of the
+// delta rule (the inverse of a unit triangular matrix per chunk, the UT transform). Row by row every token is
 // two dot products and an update in one dependent chain (0.78 us a token at D = 128); a chunk needs one chain. With
 // k, q the unit rows, G_t = g_0 .. g_t and D_tj = g_(j+1) .. g_t (products of decays over the chunk's rows, never
 // quotients) and S the state before the chunk,
