@@ -163,6 +163,21 @@ def test_rows_of_no_sequence_stay(start, n, rest):
     assert (out[2:2 + n].float() - alone.float()).abs().max() < 2.0 ** -7 * vc.float().abs().max()
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("start,n,nseq", [(32, 60, 5), (0, 100, 1), (196, 60, 3), (197, 60, 3)])      # to 256 positions, and one more
+def test_a_known_context_changes_no_result(start, n, nseq):
+    g = torch.Generator().manual_seed(start + n)
+    H, G, D, dev = 32, 8, 128, "cuda"
+    per = (start + n + BS - 1) // BS
+    kc, vc = (torch.randn(nseq * per, G, *s, generator=g).bfloat16().to(dev) for s in ((BS, D), (D, BS)))
+    tables = torch.randperm(nseq * per, generator=g).int().view(nseq, per).to(dev)
+    q = torch.randn(nseq * n, H, D, generator=g).bfloat16().to(dev)
+    cu = torch.arange(0, nseq * n + 1, n, dtype=torch.int32, device=dev)
+    pos = torch.arange(start, start + n).int().repeat(nseq).to(dev)
+    plain, known = (ops.attn_prefill_paged(q, kc, vc, tables, cu, pos, n, 0.1, max_ctx=c).float() for c in (0, start + n))
+    assert (plain - known).abs().max() < 2.0 ** -7 * vc.float().abs().max()      # (weights and outputs rounded to bf16 in both)
+
+
 @pytest.mark.skipif(not ops.load_library(), reason="kernel library not built")
 def test_scratch_of_split_pages():
     """Scratch only where workgroups share a tile's pages: few tiles, enough pages; 64 MB at most."""
