@@ -812,6 +812,9 @@ void moe_route(const Tensor& x, const Tensor& wr, int64_t top_k, Tensor& gates, 
 }
 
 int64_t moe_max_tiles(int64_t TK, int64_t El, int64_t bm) { return bfly::moe_max_tiles(TK, El, (int)bm); }
+bool moe_grouped_on_big4(int64_t x_rows, int64_t ldx, int64_t ldw, bool silu, bool gathered) {
+  return bfly::grouped_on_big4(x_rows, ldx, ldw, silu, gathered);
+}
 
 // block counts (EP IPC receive buffer): rows form blocks of `bcap`; only the first bcnt[b] rows of
 // block b are valid (device-resident counts, so no host sync)
@@ -874,7 +877,7 @@ void moe_grouped_gemm(const Tensor& x, const Tensor& w, Tensor& out, const c10::
     pp = pt.data_ptr<float>();
   }
   c10::DeviceGuard g(x.device());
-  const int rc = bfly::launch_gemm_grouped(bf(x), x.stride(0), bf(w), ldw, w_estride, n, k, epilogue, rp,
+  const int rc = bfly::launch_gemm_grouped(bf(x), x.size(0), x.stride(0), bf(w), ldw, w_estride, n, k, epilogue, rp,
                                            reinterpret_cast<const int4*>(tiles.data_ptr<int>()), count.data_ptr<int>(),
                                            tiles.size(0), bf(out), out.stride(0), cur_stream(), (int)bm,
                                            (int)out.size(0), sk, pp);
@@ -1221,6 +1224,7 @@ TORCH_LIBRARY(bfly, m) {
   m.def("moe_route(Tensor x, Tensor wr, int top_k, Tensor(a!) gates, Tensor(b!) topk_ids, Tensor(c!) topk_w) -> ()");
   m.def("moe_gate_scale(Tensor(a!) h, Tensor gates, int e0, int num_local) -> ()");
   m.def("moe_max_tiles(int tk, int num_local, int bm=64) -> int", &moe_max_tiles);
+  m.def("moe_grouped_on_big4(int x_rows, int ldx, int ldw, bool silu, bool gathered) -> bool", &moe_grouped_on_big4);
   m.def("moe_align(Tensor topk_ids, int e0, int num_local, Tensor(a!) rows, Tensor(b!) slot_of, Tensor(c!) tiles, "
         "Tensor(d!) count, int bm=64, Tensor? bcnt=None, int bcap=0) -> ()");
   m.def("moe_grouped_gemm(Tensor x, Tensor w, Tensor(a!) out, Tensor? rows, Tensor tiles, Tensor count, int w_estride, "

@@ -248,7 +248,9 @@ int launch_moe_align(const int* topk_ids, int T, int K, int e0, int El, int BM, 
 int launch_moe_combine(const bf16* y, const int* slot_of, const float* w, int T, int K, int H,
                        bf16* out, hipStream_t stream, const int* bcnt = nullptr, int bcap = 0);
 constexpr int kMoeGroupBM = 64;
-int launch_gemm_grouped(const bf16* X, long ldx, const bf16* W, long ldw, long w_estride, int N,
+// whether its 256-row tiles run on gemm_big4_kernel (else gemm_big8_kernel)
+bool grouped_on_big4(long x_rows, long ldx, long ldw, bool silu, bool gathered);
+int launch_gemm_grouped(const bf16* X, long x_rows, long ldx, const bf16* W, long ldw, long w_estride, int N,
                         int K, int epi, const int* rows, const int4* tiles, const int* count,
                         int max_tiles, bf16* out, long ldo, hipStream_t stream, int bm = 64,
                         int slots = 0, int sk = 1, float* part = nullptr);

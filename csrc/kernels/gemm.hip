@@ -1001,13 +1001,16 @@ __device__ __forceinline__ void big4_tile(const bf16* __restrict__ X, long ldx, 
     va[e] = (int)((arow * ldx + ch * 8) * 2);
     vb[e] = (int)((brow * ldw + ch * 8) * 2);
   }
-  int ga[RI] = {};   // GROUPED: byte offsets from X of this lane's gathered rows (at its chunk)
-  const auto rsx = b8_rsrc(X, 1L << 30, 1);
+  // GROUPED: byte offsets of this lane's rows (at its chunk), from X where they are gathered (X has less than 2 GB:
+  // grouped_on_big4, moe_big_ok), from the tile's first row where they follow one another (slots know no such bound)
+  int ga[RI] = {};
+  const bool gather = GROUPED == 2 || grows != nullptr;
+  const auto rsx = b8_rsrc(gather ? X : X + (long)m0 * ldx, 1L << 30, 1);
   if constexpr (GROUPED == 1 || GROUPED == 2) {
 #pragma unroll
     for (int q = 0; q < RI; ++q) {
       const int slot = min(m0 + arow + 8 * q, M - 1);
-      const long src = GROUPED == 2 ? ex.perm[slot] / ex.choices : grows != nullptr ? grows[slot] : slot;
+      const long src = GROUPED == 2 ? ex.perm[slot] / ex.choices : gather ? grows[slot] : slot - m0;
       ga[q] = (int)((src * ldx + (((lane & 7) ^ (((lane >> 4) + 4 * (q & 1)) & 7)) * 8)) * 2);
     }
   }
@@ -2111,7 +2114,17 @@ static int launch_grouped_bm(const bf16* X, long ldx, const bf16* W, long ldw, l
   return 0;
 }
 
-int launch_gemm_grouped(const bf16* X, long ldx, const bf16* W, long ldw, long w_estride, int N,
+// 256-row expert tiles: the one-wave-per-SIMD tile, but for weights whose rows are a multiple of 32 KB apart: the 256 rows of a K
+// step then lie in one memory channel, and the tile, with less in flight, waits for it. 8 experts' down projection of 4096 x 14336,
+// rows 8 x 28 KB apart (7 x 32 KB) and 128 bytes more (4 KB: 235 at 300 tokens, 580 at 2870), us: big4 at 300, 976, 2870, 5000 tokens
+// 361, 433, 727, 1201 and 220, 315, 559, 956; big8 293, 347, 667, 1033 and 284, 327, 653, 1014. Its rows are offsets of 32 bits from
+// X (gathered) or from a tile's first row, those of the other one addresses.
+bool grouped_on_big4(long x_rows, long ldx, long ldw, bool silu, bool gathered) {
+  const long reach = (gathered ? x_rows : std::min(x_rows, 256L)) * ldx * 2;
+  return reach < 0x7fffffffL && (silu || ldw * 2 % 32768 != 0);
+}
+
+int launch_gemm_grouped(const bf16* X, long x_rows, long ldx, const bf16* W, long ldw, long w_estride, int N,
                         int K, int epi, const int* rows, const int4* tiles, const int* count,
                         int max_tiles, bf16* out, long ldo, hipStream_t stream, int bm, int slots,
                         int sk, float* part) {
@@ -2130,11 +2143,7 @@ int launch_gemm_grouped(const bf16* X, long ldx, const bf16* W, long ldw, long w
       attr = true;
     }
     dim3 grid(max_tiles * (N / 256), 1);
-    // The one-wave-per-SIMD tile, but for weights whose rows are a multiple of 32 KB apart: the 256 rows of a K step then lie
-    // in one memory channel, and the tile, with less in flight, waits for it. 8 experts' down projection of 4096 x 14336, rows
-    // 8 x 28 KB apart (7 x 32 KB) and 128 bytes more (4 KB: 235 at 300 tokens, 580 at 2870), us: big4 at 300, 976, 2870, 5000
-    // tokens 361, 433, 727, 1201 and 220, 315, 559, 956; big8 293, 347, 667, 1033 and 284, 327, 653, 1014.
-    if (epi == EPI_SILU || ldw * 2 % 32768 != 0)
+    if (grouped_on_big4(x_rows, ldx, ldw, epi == EPI_SILU, rows != nullptr))
       gemm_big4_kernel<1><<<dim3(max_tiles * (N / 256) + 128), kB4Threads, kB4LdsBytes, stream>>>(
           X, ldx, W, ldw, 0, N, K, epi, nullptr, out, ldo, nullptr, 0, rows, tiles, count, w_estride);
     else

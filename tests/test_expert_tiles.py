@@ -164,3 +164,39 @@ def test_sparse_experts_few_rows_per_big_tile(counts):
     want = ops.reference.moe_sparse_ffn(x.float(), ids, w, gu.float(), dn.float(), 0, E, F)
     # bf16 hidden rows, expert rows and output: 2^-9 each
     assert (got.cpu().float() - want).norm() < 2.0 ** -7 * want.norm()
+
+
+@pytest.mark.skipif(not ops.load_library(), reason="kernel library not built")
+def test_grouped_rows_beyond_32_bit_offsets():
+    """Gathered rows that 32-bit byte offsets do not reach go to the tile with 64-bit addresses, and so do slots whose single tile has
+    such rows; any number of slots stays, and so do down weights of rows 32 KB apart on the other tile."""
+    big4 = torch.ops.bfly.moe_grouped_on_big4                 # x rows, their stride, the weights', gate/up, gathered
+    wide, pad = 8 * 14336, 8 * 14336 + 2048
+    assert [big4(n, 4096, 4096, True, True) for n in (262143, 262144, 10 ** 6)] == [True, False, False]
+    assert [big4(n, 14336, pad, False, False) for n in (74897, 74899, 10 ** 6)] == [True] * 3
+    assert [big4(10 ** 6, ld, pad, False, False) for ld in (1 << 22, (1 << 22) - 8)] == [False, True]
+    assert not big4(300, 14336, wide, False, False)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("gathered", [False, True])
+def test_grouped_rows_of_far_strides(gathered):
+    """600 rows 4 MB apart: the last ones lie 2.5 GB behind the first, past 32-bit byte offsets."""
+    M, K, N, E, ld = 600, 256, 512, 2, 1 << 21
+    g = torch.Generator(device="cuda").manual_seed(M)
+    bf = lambda *s: torch.randn(*s, generator=g, device="cuda").to(torch.bfloat16)            # noqa: E731
+    x = torch.empty(M * ld, dtype=torch.bfloat16, device="cuda").view(M, ld)[:, :K].copy_(bf(M, K))
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device="cuda")                         # noqa: E731
+    tiles, rows = [(0, 0, 256, 0), (0, 256, 330, 0), (1, 330, 586, 0), (1, 586, 600, 0)], torch.randperm(M, generator=g, device="cuda")
+    if not gathered:
+        rows = torch.arange(M, device="cuda")
+    w = bf(E, N, K) * K ** -0.5
+    want = torch.cat([x[rows[:330]].float() @ w[0].float().T, x[rows[330:]].float() @ w[1].float().T])
+    if gathered:      # gate and up rows interleaved in groups of 16
+        v = want.view(M, N // 32, 2, 16)
+        want = (torch.nn.functional.silu(v[:, :, 0]) * v[:, :, 1]).reshape(M, N // 2)
+    out = torch.full_like(want, float("nan"), dtype=torch.bfloat16)
+    torch.ops.bfly.moe_grouped_gemm(x, w.view(E * N, K), out, rows.int() if gathered else None, i32(tiles), i32([4]), N * K, N, K, E,
+                                    ops.EPILOGUES["silu" if gathered else "none"], 256)
+    # one rounding to bf16 (2^-9), f32 sums of 256 products beside it
+    assert (out.float() - want).norm() < 2.0 ** -8 * want.norm()
