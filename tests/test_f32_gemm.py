@@ -1,4 +1,4 @@
-"""True-f32 products on the f32 matrix cores: plain GEMM, router logits and grouped experts against float64."""
+"""True-f32 products (three bf16 parts per value): plain GEMM, router logits and grouped experts against float64."""
 import pytest
 import torch
 
@@ -42,6 +42,26 @@ def test_sums_that_bf16_parts_cannot_hold(M, N, K):
     size = x[keep].to(F64).abs() @ w.to(F64).abs().T
     # K additions in f32, and 2^-25 of each product left out
     assert ((got - want)[keep].abs() <= (K + 2) * 6e-8 * size + 1e-43).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(65, 66, 20), (66, 64, 32), (70, 64, 96), (33, 130, 257), (2048, 1792, 64), (2048, 1792, 45)])
+@pytest.mark.parametrize("small,large", [(-126, 100), (-124, 60), (-115, 60), (-120, 20), (-140, 0), (-135, 100), (-75, -70), (-60, -45)])
+def test_small_operands_of_large_ones(M, N, K, small, large):
+    """Values whose last bits no bf16 part holds, denormal ones and products that underflow: as exact as sums in f32, alone, among
+    ordinary terms and on either side; the rows beside them keep their sums bit for bit."""
+    g = torch.Generator().manual_seed(M + K)
+    x, w = torch.randn(M, K, generator=g), torch.randn(N, K, generator=g)
+    plain = ops.linear_act(x.cuda(), w.cuda()).cpu()
+    x[1], x[2, ::3] = x[1] * 2.0 ** small, x[2, ::3] * 2.0 ** small      # a whole row, and some channels of one
+    w[5], w[6, ::3] = w[5] * 2.0 ** large, w[6, ::3] * 2.0 ** large
+    x[7], w[8] = x[7] * 2.0 ** min(large, 20), w[8] * 2.0 ** small
+    got, want = ops.linear_act(x.cuda(), w.cuda()).cpu(), x.to(F64) @ w.to(F64).T
+    size = x.to(F64).abs() @ w.to(F64).abs().T
+    # K additions in f32, 2^-25 of each product left out; below 2^-126 one denormal (2^-149) per addition
+    assert ((got.to(F64) - want).abs() <= (K + 2) * 6e-8 * size + K * 2.0 ** -149).all()
+    rows, cols = [r for r in range(M) if r not in (1, 2, 7)], [c for c in range(N) if c not in (5, 6, 8)]
+    assert torch.equal(got[rows][:, cols], plain[rows][:, cols])
 
 
 @pytest.mark.gpu
@@ -90,6 +110,28 @@ def test_experts(T, E, Hd, F, plain):
         a = torch.relu(h) ** 2 if plain else c * torch.sigmoid(1.702 * c) * (torch.clamp(h[:, F:], -7.0, 7.0) + 1)
         want.index_add_(0, t, a @ dn[e].to(F64).T)
     assert (got - want).abs().max() < 1e-5 * (1 + want.abs().max())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("H,F", [(64, 96), (100, 65)])
+def test_experts_of_small_operands(H, F):
+    """An expert's inputs of 2^-105 under weights of 2^105, and output columns of 2^-110: as exact as the others."""
+    g = torch.Generator().manual_seed(F)
+    T, E = 90, 3
+    x, ids, w = torch.randn(T, H, generator=g), (torch.arange(T) % E)[:, None], torch.rand(T, 1, generator=g) + 0.2
+    gu, dn = torch.randn(E, 2 * F, H, generator=g) * H ** -0.5, torch.randn(E, H, F, generator=g) * F ** -0.5
+    x[ids[:, 0] == 1] *= 2.0 ** -105
+    gu[1] *= 2.0 ** 105
+    dn[:, :8] *= 2.0 ** -110
+    got = ops.moe_glu_ffn(x.cuda(), ids.int().cuda(), w.cuda(), gu.cuda(), dn.cuda(), 7.0, 1.702).cpu().to(F64)
+    want = torch.zeros(T, H, dtype=F64)
+    for e in range(E):
+        t = (ids[:, 0] == e).nonzero()[:, 0]
+        h = (x[t].to(F64) * w[t].to(F64)) @ gu[e].to(F64).T
+        c = torch.clamp(h[:, :F], max=7.0)
+        want[t] = (c * torch.sigmoid(1.702 * c) * (torch.clamp(h[:, F:], -7.0, 7.0) + 1)) @ dn[e].to(F64).T
+    for part in (slice(0, 8), slice(8, H)):
+        assert (got - want)[:, part].abs().max() < 1e-5 * want[:, part].abs().max()
 
 
 @pytest.mark.gpu
