@@ -40,7 +40,7 @@ def test_sums_that_bf16_parts_cannot_hold(M, N, K):
     assert got[3, 1].isnan() and got[3, 2] == float("inf") and got[4].isnan().all() and (got[2] == 0).all()
     keep = torch.tensor([r for r in range(M) if r not in (3, 4)])
     size = x[keep].to(F64).abs() @ w.to(F64).abs().T
-    # K additions in f32, and 2^-25 of each product left out
+    # K additions in f32, and 2^-24 of each product left out
     assert ((got - want)[keep].abs() <= (K + 2) * 6e-8 * size + 1e-43).all()
 
 
@@ -58,10 +58,24 @@ def test_small_operands_of_large_ones(M, N, K, small, large):
     x[7], w[8] = x[7] * 2.0 ** min(large, 20), w[8] * 2.0 ** small
     got, want = ops.linear_act(x.cuda(), w.cuda()).cpu(), x.to(F64) @ w.to(F64).T
     size = x.to(F64).abs() @ w.to(F64).abs().T
-    # K additions in f32, 2^-25 of each product left out; below 2^-126 one denormal (2^-149) per addition
+    # K additions in f32, 2^-24 of each product left out; below 2^-126 one denormal (2^-149) per addition
     assert ((got.to(F64) - want).abs() <= (K + 2) * 6e-8 * size + K * 2.0 ** -149).all()
     rows, cols = [r for r in range(M) if r not in (1, 2, 7)], [c for c in range(N) if c not in (5, 6, 8)]
     assert torch.equal(got[rows][:, cols], plain[rows][:, cols])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("N", [64, 70])
+@pytest.mark.parametrize("K,units", [(1, 1), (4, 3), (32, 3), (40, 3)])
+def test_single_products(N, K, units):
+    """One channel that is not zero. Up to three channels: one rounding (2^-24). From four on, six products of parts leave out less
+    than 2^-24 of it, and the last addition cuts to 24 bits (2^-23)."""
+    g = torch.Generator().manual_seed(N)
+    x, w = torch.zeros(4096, K), torch.zeros(N, K)
+    x[:, K - 1], w[:, K - 1] = torch.randn(4096, generator=g), torch.randn(N, generator=g)
+    x[0, K - 1] = w[0, K - 1] = 1 + 2.0 ** -8 - 2.0 ** -17 - 2.0 ** -23
+    want = x.to(F64) @ w.to(F64).T
+    assert ((ops.linear_act(x.cuda(), w.cuda()).cpu().to(F64) - want).abs() <= units * 2.0 ** -24 * want.abs()).all()
 
 
 @pytest.mark.gpu
