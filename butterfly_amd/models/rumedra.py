@@ -313,7 +313,7 @@ class RumedraLM(PackedStack):
         part = lambda a, b: z[:, a:b].view(T, heads, -1)                                       # noqa: E731
         o = ops.forget_scan(part(0, n), part(n, 2 * n), part(2 * n, 2 * n + m), p[pre + "f.b"], p[pre + "lower"],
                             self.state[sp["index"]], meta["state_slots"], meta["row_cu"], fb.positions, "silu",
-                            meta["one_row"])
+                            meta["one_row"], fb.max_seqlen if fb.is_prefill else 1)
         y = ops.new_empty(T, m, dtype=self.dtype, device=self.device)
         ops.head_norm_gate(o, p[pre + "norm"], self.cfg.norm_eps, None, 1.0, y)
         return self._out(y, p[pre + "o"])

@@ -923,8 +923,8 @@ def attn_window_paged(q, k_cache, v_cache, tables, row_cu, positions, scale: flo
 
 def gla_scan(q, k, v, z, state, state_slots, row_cu, positions, tau: float, q_scale: float, max_rows: int = 0):
     """Gated linear attention over packed rows with the state pooled in `state` [slots, H, D, Dv]
-    f32 (updated in place). `max_rows`: the most rows of a sequence, where the caller knows it (it changes no result).
-    Returns o [T, H, Dv] f32."""
+    f32 (updated in place). `max_rows`: the most rows of a sequence, where the caller knows it (it picks the faster of forms
+    that differ in f32 rounding). Returns o [T, H, Dv] f32."""
     if not _gpu(q):
         return ref.gla_scan(q, k, v, z, state, state_slots, row_cu, positions, tau, q_scale)
     o = _empty(q.shape[0], q.shape[1], v.shape[2], dtype=torch.float32, device=q.device)
@@ -1462,16 +1462,18 @@ def decay_scan(q, k, v, dpow, state, state_slots, row_cu, positions, act: str = 
     return o
 
 
-def forget_scan(q, z, v, f_bias, lower, state, state_slots, row_cu, positions, act: str = "silu", one_row: bool = False):
+def forget_scan(q, z, v, f_bias, lower, state, state_slots, row_cu, positions, act: str = "silu", one_row: bool = False,
+                max_rows: int = 0):
     """Linear attention with a gate per head and channel as decay, its complement as key, over packed rows: f = lower +
     (1 - lower) sigmoid(z + f_bias), S <- diag(f) S + (1 - f) v^T, o = S^T act(q), the state pooled as in decay_scan. q, z
     [T, H, D], v [T, H, Dv] rows (views allowed); f_bias, lower [H * D] f32. Steps of several rows per sequence run
-    in chunks of 16 rows on the f32 matrix cores, steps of one row (`one_row`) in place. Returns o [T, H,
-    Dv] f32."""
+    in chunks of 16 rows on the f32 matrix cores, steps of one row (`one_row`) in place. `max_rows`: the most rows of a
+    sequence, where the caller knows it (it picks the faster of two forms; they differ in f32 rounding). Returns o [T, H, Dv] f32."""
     if not _gpu(q):
         return ref.forget_scan(q, z, v, f_bias, lower, state, state_slots, row_cu, positions, act)
     o = _empty(q.shape[0], q.shape[1], v.shape[2], dtype=torch.float32, device=q.device)
-    torch.ops.bfly.forget_scan(q, z, v, f_bias, lower, state, state_slots, row_cu, positions, CONV_ACTS[act], bool(one_row), o)
+    torch.ops.bfly.forget_scan(q, z, v, f_bias, lower, state, state_slots, row_cu, positions, CONV_ACTS[act], bool(one_row), o,
+                               int(max_rows))
     return o
 
 

@@ -320,7 +320,8 @@ void gla_scan(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& z
   TORCH_CHECK(row_cu.numel() == nseq + 1 && positions.numel() == T, "gla_scan: row_cu / positions");
   TORCH_CHECK(o.dim() == 3 && o.size(0) == T && o.size(1) == H && o.size(2) == Dv, "gla_scan: o");
   TORCH_CHECK(tau > 0, "gla_scan: tau");
-  const long n = bfly::gla_scan_scratch((int)T, (int)nseq, (int)H, (int)D, (int)Dv, is_f32(q), (int)max_rows);
+  const long n = bfly::gla_scan_scratch((int)T, (int)nseq, (int)H, (int)D, (int)Dv, is_f32(q), (int)max_rows,
+                                        std::max({q.stride(0), k.stride(0), z.stride(0)}));
   Tensor rec;
   if (n > 0) rec = at::empty({n}, o.options());
   const int rc = bfly::launch_gla_scan(q.data_ptr(), q.stride(0), k.data_ptr(), k.stride(0), v.data_ptr(), v.stride(0),
@@ -329,6 +330,11 @@ void gla_scan(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& z
                                        (float)q_scale, o.data_ptr<float>(), n > 0 ? rec.data_ptr<float>() : nullptr, (int)T,
                                        (int)H, (int)D, (int)Dv, is_f32(q), cur_stream(), (int)max_rows);
   TORCH_CHECK(rc == 0, "gla_scan: key size ", D, " not supported (<= 256)");
+}
+
+std::vector<int64_t> gla_scan_forms(int64_t T, int64_t nseq, int64_t H, int64_t D, int64_t Dv, bool f32, int64_t max_rows) {
+  const bfly::GlaSteps g = bfly::gla_scan_steps((int)T, (int)nseq, (int)H, (int)D, (int)Dv, f32, (int)max_rows);
+  return {g.rows, g.chunks, g.least};
 }
 
 void gla_out(const Tensor& o, const Tensor& g, const Tensor& norm_w, double eps, Tensor& out) {
@@ -497,6 +503,7 @@ TORCH_LIBRARY_FRAGMENT(bfly, m) {
         "Tensor? k_pool=None, Tensor? v_pool=None, Tensor? gate=None, float out_mul=1., int dv_out=0) -> ()");
   m.def("gla_scan(Tensor q, Tensor k, Tensor v, Tensor z, Tensor(a!) state, Tensor state_slots, Tensor row_cu, "
         "Tensor positions, float tau, float q_scale, Tensor(b!) o, int max_rows=0) -> ()");
+  m.def("gla_scan_forms(int T, int nseq, int H, int D, int Dv, bool f32, int max_rows) -> int[]", &gla_scan_forms);
   m.def("gla_out(Tensor o, Tensor g, Tensor norm_w, float eps, Tensor(a!) out) -> ()");
   m.def("router_logits(Tensor x, Tensor wr, Tensor(a!) logits) -> ()");
   m.def("moe_topk_scores(Tensor logits, Tensor? bias, int top_k, int scoring, bool renorm, Tensor(a!) ids, "

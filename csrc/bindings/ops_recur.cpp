@@ -73,7 +73,7 @@ void decay_scan(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor&
 
 void forget_scan(const Tensor& q, const Tensor& z, const Tensor& v, const Tensor& f_bias, const Tensor& lower, Tensor& state,
                  const Tensor& state_slots, const Tensor& row_cu, const Tensor& positions, int64_t act, bool one_row,
-                 Tensor& o) {
+                 Tensor& o, int64_t max_rows) {
   CHK_HEADS(q); CHK_HEADS(z); CHK_HEADS(v); CHK_SAME(z, q); CHK_SAME(v, q);
   CHK_F32(f_bias); CHK_F32(lower); CHK_F32(state); CHK_F32(o);
   const int64_t T = q.size(0), H = q.size(1), D = q.size(2), Dv = v.size(2);
@@ -86,14 +86,21 @@ void forget_scan(const Tensor& q, const Tensor& z, const Tensor& v, const Tensor
   TORCH_CHECK((act == 0 || act == 1) && D <= 4096, "forget_scan: act / key size");
   TORCH_CHECK(q.stride(0) < (1 << 21) && z.stride(0) < (1 << 21), "forget_scan: row strides");      // (24-bit byte offsets)
   TORCH_CHECK(o.dim() == 3 && o.size(0) == T && o.size(1) == H && o.size(2) == Dv, "forget_scan: o [T, H, Dv]");
+  const int64_t nseq = state_slots.numel();
   Tensor rec;
-  if (!one_row) rec = at::empty({bfly::chunk_record_floats(T, state_slots.numel(), H, D)}, state.options());
+  if (!one_row && !bfly::chunks_in_one_launch(T, nseq, H, D, Dv, is_f32(q), max_rows, std::max(q.stride(0), z.stride(0))))
+    rec = at::empty({bfly::chunk_record_floats(T, nseq, H, D)}, state.options());
   bfly::launch_forget_scan(q.data_ptr(), q.stride(0), z.data_ptr(), z.stride(0), v.data_ptr(), v.stride(0),
                            f_bias.data_ptr<float>(), lower.data_ptr<float>(), state.data_ptr<float>(),
                            state_slots.data_ptr<int>(), row_cu.data_ptr<int>(), (int)state_slots.numel(),
                            positions.data_ptr<int>(), (int)act, o.data_ptr<float>(),
-                           one_row ? nullptr : rec.data_ptr<float>(), (int)T, (int)H, (int)D, (int)Dv, one_row, is_f32(q),
+                           rec.defined() ? rec.data_ptr<float>() : nullptr, (int)T, (int)H, (int)D, (int)Dv, one_row, is_f32(q),
                            cur_stream());
+}
+
+// launches that a step of several rows takes
+int64_t forget_scan_launches(int64_t T, int64_t nseq, int64_t H, int64_t D, int64_t Dv, bool f32, int64_t max_rows) {
+  return D > 256 || bfly::chunks_in_one_launch(T, nseq, (int)H, (int)D, (int)Dv, f32, max_rows, H * D) ? 1 : 2;
 }
 
 void head_norm_gate(const Tensor& o, const optional<Tensor>& w, double eps, const optional<Tensor>& gate, int64_t act,
@@ -250,7 +257,8 @@ TORCH_LIBRARY_FRAGMENT(bfly, m) {
   m.def("decay_scan(Tensor q, Tensor k, Tensor v, Tensor dpow, Tensor(a!) state, Tensor state_slots, Tensor row_cu, "
         "Tensor positions, int act, bool one_row, Tensor(b!) o, Tensor? cs=None, float k_scale=1.0) -> ()");
   m.def("forget_scan(Tensor q, Tensor z, Tensor v, Tensor f_bias, Tensor lower, Tensor(a!) state, Tensor state_slots, "
-        "Tensor row_cu, Tensor positions, int act, bool one_row, Tensor(b!) o) -> ()");
+        "Tensor row_cu, Tensor positions, int act, bool one_row, Tensor(b!) o, int max_rows=0) -> ()");
+  m.def("forget_scan_launches(int T, int nseq, int H, int D, int Dv, bool f32, int max_rows) -> int", &forget_scan_launches);
   m.def("head_norm_gate(Tensor o, Tensor? w, float eps, Tensor? gate, int act, float mul, Tensor(a!) out) -> ()");
   m.def("row_norm_gate(Tensor o, Tensor w, float eps, Tensor? gate, float mul, Tensor(a!) out) -> ()");
   m.def("selective_scan(Tensor x, Tensor dtr, Tensor b, Tensor c, Tensor z, Tensor a_log, Tensor dt_bias, Tensor d, "

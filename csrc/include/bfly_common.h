@@ -143,9 +143,9 @@ struct ExpertArgs {
 // time of `first` single rows and of `each` more per chunk, padded or not (chunk_cost): a sequence runs in chunks where that is no
 // more than its rows. The host knows only the sum of the rows, so a step that may hold both kinds launches both forms, and every
 // workgroup looks at its own sequence. The second launch (2 to 5 us) is saved where no sequence is long enough (max_rows, where the
-// caller knows it) or repays it (six times the rows of the shortest sequence in chunks beyond one each, none of them empty), and
-// for steps of prompts where the shorter sequences cost the chunk form no more than that: `wgs` workgroups per sequence, at 11 to
-// 25 ns for one with a single row.
+// caller knows it) or repays it (six times the rows of the shortest sequence in chunks, or those of one chunk, beyond one each, none
+// of them empty), and for steps of prompts where the shorter sequences cost the chunk form no more than that: `wgs` workgroups per
+// sequence, at 11 to 25 ns for one with a single row.
 struct ScanForms {
   bool rows, chunks;
 };
@@ -155,7 +155,7 @@ inline ScanForms scan_forms(long T, long nseq, int cost, long wgs, long max_rows
   if (nseq == 1) return {!scan_in_chunks(T, cost), scan_in_chunks(T, cost)};
   long least = 1;
   while (least < 256 && !scan_in_chunks(least, cost)) ++least;
-  if (T - nseq < 6 * least || (max_rows > 0 && max_rows < least)) return {true, false};
+  if (T - nseq < 6 * (least < 16 ? least : 16) || (max_rows > 0 && max_rows < least)) return {true, false};
   return {!(scan_in_chunks(T / nseq, cost) && nseq * wgs <= 512), true};
 }
 // (`cost` 0 in a kernel: it takes every sequence)

@@ -114,8 +114,14 @@ bool launch_attn_window_f32(const float* q, long q_ld, const float* k_cache, con
                             int D, int Dv, int block_size, hipStream_t s, const AttnMod& md);
 
 // Gated linear attention scan over packed rows (see ops.gla_scan). Returns < 0 if D > 256. max_rows > 0: no sequence has
-// more rows. rec: scratch of gla_scan_scratch f32 elements
-long gla_scan_scratch(int T, int nseq, int H, int D, int Dv, bool f32, int max_rows);
+// more rows. rec: scratch of gla_scan_scratch f32 elements (0: null); max_ld: the largest row stride of q, k, z
+long gla_scan_scratch(int T, int nseq, int H, int D, int Dv, bool f32, int max_rows, long max_ld);
+// how it runs a step: row by row (0 or 1), chunks (0 none, 1 in one launch, 2 in two), the fewest rows of a sequence in chunks (0:
+// every one is, -1: none)
+struct GlaSteps {
+  int rows, chunks, least;
+};
+GlaSteps gla_scan_steps(int T, int nseq, int H, int D, int Dv, bool f32, int max_rows);
 int launch_gla_scan(const void* q, long q_ld, const void* k, long k_ld, const void* v, long v_ld, const void* z,
                     long z_ld, float* state, const int* state_slots, const int* row_cu, int nseq,
                     const int* positions, float tau, float q_scale, float* o, float* rec, int T, int H, int D, int Dv, bool f32,

@@ -21,11 +21,14 @@ void launch_decay_scan(const void* q, long q_ld, const void* k, long k_ld, const
                        int D, int Dv, bool one_row, bool f32, hipStream_t s);
 // Linear attention with a forget gate per head and channel over packed rows: f = lower + (1 - lower) sigmoid(z +
 // f_bias), S <- diag(f) S + (1 - f) v^T, o = S^T act(q). q, z [T, H, D], v [T, H, Dv] rows of the activation type with
-// row strides; f_bias, lower f32 [H * D]; state, o, one_row as above. rec: scratch of chunk_record_floats (unless one_row).
+// row strides; f_bias, lower f32 [H * D]; state, o, one_row as above. rec: scratch of chunk_record_floats (unless one_row; null
+// where chunks_in_one_launch).
 void launch_forget_scan(const void* q, long q_ld, const void* z, long z_ld, const void* v, long v_ld, const float* f_bias,
                         const float* lower, float* state, const int* state_slots, const int* row_cu, int nseq,
                         const int* positions, int act, float* o, float* rec, int T, int H, int D, int Dv, bool one_row,
                         bool f32, hipStream_t s);
+// Whether the chunks of a step go in one launch, without scratch (max_ld: the largest row stride)
+bool chunks_in_one_launch(long T, long nseq, int H, int D, int Dv, bool f32, long max_rows, long max_ld);
 // f32 elements of scratch for the chunks of a step of T rows and nseq sequences
 long chunk_record_floats(long T, long nseq, int H, int D);
 // out[t, h] = o[t, h] / sqrt(mean(o[t, h]^2) + eps) * w * act(gate[t, h]) * mul per head of Dv values; o f32 [T, H, Dv]

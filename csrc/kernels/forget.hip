@@ -4,6 +4,7 @@
 //   gate_chunk_kernel, gate_chain_kernel      f = l + (1 - l) sigmoid(z + b), S <- diag(f) S + (1 - f) v^T, o = S^T q,
 //                                             in chunks on the f32 matrix cores; also gated linear attention, whose key
 //                                             is an input (GLA)
+//   gate_scan_kernel                          the same in one launch, for short sequences
 //   forget_step_kernel                        the same row by row
 //   head_norm_gate_kernel                     RMS norm per head, times an optional weight, a gate and a factor
 // Rows of a step are packed: sequence s owns rows row_cu[s] .. row_cu[s+1]; a sequence whose first row is at
@@ -33,6 +34,17 @@ __device__ __forceinline__ float gla_decay(float z, float inv_tau) {
   const float e = FAST ? __expf(-fabsf(z)) : expf(-fabsf(z));
   const float ls = fminf(z, 0.f) - (FAST ? __logf(1.f + e) : log1pf(e));
   return FAST ? __expf(ls * inv_tau) : expf(ls * inv_tau);
+}
+
+// One element at a byte offset below 2^31 from a uniform base. (Rows of one chunk; callers clamp row and channel to the
+// tensor.)
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t rows_rsrc(const void* base) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0, 0x7fffffff, 0x00027000);
+}
+template <typename T>
+__device__ __forceinline__ T row_load(__amdgpu_buffer_rsrc_t r, int off) {
+  if constexpr (sizeof(T) == 2) return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b16(r, off, 0, 0));
+  else return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b32(r, off, 0, 0));
 }
 
 // sum over the 32 lanes of a half wave, in its upper sixteen lanes
@@ -399,6 +411,317 @@ __global__ __launch_bounds__(256, NT <= 8 ? 2 : 1) void gate_chain_kernel(
   }
 }
 
+// Both parts of a chunk in one launch, for steps whose longest sequence has one or a few chunks (one_launch_rows): the second
+// launch and the records' way through memory would be most of the time. Workgroup = (sequence, head, 64 value columns), eight
+// waves: wave & 3 names 16 columns, wave >> 2 a half of the state's rows. The first DP of 2 DP roles stage q, f and q F, the others
+// k and k B; the diagonal blocks of P are formed on the vector units while the matrix cores are busy. Row strides below 2^21
+// elements (24-bit byte offsets). Values that are no numbers as in gate_chain_kernel.
+template <typename T, int NT, bool GLA>
+__global__ __launch_bounds__(512, NT <= 8 ? 4 : 2) void gate_scan_kernel(const T* __restrict__ q, long q_ld,
+                                                           const T* __restrict__ key, long k_ld, float inv_tau, float q_scale,
+                                                           const T* __restrict__ z, long z_ld, const T* __restrict__ v, long v_ld,
+                                                           const float* __restrict__ f_bias,
+                                                           const float* __restrict__ lower, float* __restrict__ state,
+                                                           const int* __restrict__ state_slots,
+                                                           const int* __restrict__ row_cu,
+                                                           const int* __restrict__ positions, int act, int vec,
+                                                           float* __restrict__ o, int H, int D, int Dv, int cost) {
+  constexpr int C = 16, DP = 16 * NT, NH = NT / 2, NU = (DP + 127) / 128, KP = 128 * NU + 4, VP = 68, PP = C + 4;
+  constexpr int NI = (2 * DP + 255) / 256, HC = C / 2, NP = NT < 8 ? NT : 8;
+  constexpr bool FAST = sizeof(T) == 2, WHOLE = NI * 256 == 2 * DP;
+  extern __shared__ __attribute__((aligned(16))) float smem[];
+  float* sq = smem;                     // [C][KP] q
+  float* sk = sq + C * KP;              // [C][KP] k
+  float* sf = sk + C * KP;              // [C + 1][KP] f; row C holds ones
+  float* sqf = sf + (C + 1) * KP;       // [C][KP] q F
+  float* skb = sqf + C * KP;            // [C][KP] k B
+  float* sqh = skb + C * KP;            // [HC][KP] q times the decays from row 8 on, of rows 8 .. 15
+  float* skh = sqh + HC * KP;           // [HC][KP] k times the decays up to row 7, of rows 0 .. 7
+  float* sv = skh + HC * KP;            // [C][VP]
+  float* so = sv + C * VP;              // [C][VP] (q F) S over the second half of the state's rows
+  float* sp = so + C * VP;              // [C][PP] weights; those of rows 8 .. 15 on columns 0 .. 7 come as the sum of
+  float* sph = sp + C * PP;             // [NP][HC][HC] the waves' parts
+  float* sl = sph + NP * HC * HC;       // [DP] F of the last row
+  const int s = blockIdx.x, h = blockIdx.y, c0 = blockIdx.z * 64;
+  const int r0 = __builtin_amdgcn_readfirstlane(row_cu[s]), r1 = __builtin_amdgcn_readfirstlane(row_cu[s + 1]);
+  if (r1 <= r0 || (cost && !scan_in_chunks(r1 - r0, cost))) return;      // (the row-by-row form's)
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, m = lane & 15, gg = lane >> 4;
+  const int slot = state_slots[s];
+  if (slot < 0) {      // padding sequence of a fixed-shape step: defined output, no state
+    for (int i = tid; i < (r1 - r0) * 64; i += 512)
+      if (c0 + (i & 63) < Dv) o[((long)(r0 + (i >> 6)) * H + h) * Dv + c0 + (i & 63)] = 0.f;
+    return;
+  }
+  const int cl = 16 * (wave & 3) + m, col = c0 + cl, d0 = (wave >> 2) * 16 * NH;
+  const bool live = col < Dv;
+  float* S = state + ((long)slot * H + h) * D * Dv + col;
+  const bool fresh = positions[r0] == 0;
+  f32x4 st[NH];
+#pragma unroll
+  for (int i = 0; i < NH; ++i)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int d = d0 + 16 * i + 4 * gg + e;
+      st[i][e] = (!fresh && live && d < D) ? S[(long)d * Dv] : 0.f;
+    }
+  for (int i = tid; i < KP; i += 512) sf[C * KP + i] = 1.f;
+  if (tid < HC * HC) sp[(tid / HC) * PP + HC + tid % HC] = 0.f;      // (above the diagonal blocks, never written again)
+  if (DP < 128 * NU) {      // columns that no role stages
+    constexpr int R = 128 * NU - DP > 0 ? 128 * NU - DP : 1;
+    for (int i = tid; i < C * R; i += 512) {
+      const int at = (i / R) * KP + DP + i % R;
+      sq[at] = sk[at] = 0.f;
+      sf[at] = 1.f;
+    }
+  }
+  // this thread's roles: channel, rows ra .. ra + 7, bias and lower bound
+  const int role = 32 * wave + (lane & 31), hf = lane >> 5, ra = HC * hf;
+  float rb[NI], rl[NI];
+#pragma unroll
+  for (int u = 0; u < NI; ++u) {
+    const int idx = role + 256 * u, d = min(idx < DP ? idx : idx - DP, D - 1);
+    rb[u] = GLA ? 0.f : f_bias[(long)h * D + d];
+    rl[u] = GLA ? 0.f : lower[(long)h * D + d];
+  }
+  // the next chunk's inputs as they are stored (rows past the sequence: its last row again)
+  typedef T t4 __attribute__((ext_vector_type(4)));
+  T rq[NI][HC], rz[NI][HC];
+  t4 rv;
+  auto fetch = [&](int t0) {
+    const __amdgpu_buffer_rsrc_t qb = rows_rsrc(q + (long)t0 * q_ld + (long)h * D);
+    const __amdgpu_buffer_rsrc_t zb = rows_rsrc(z + (long)t0 * z_ld + (long)h * D);
+    const __amdgpu_buffer_rsrc_t kb = rows_rsrc(GLA ? key + (long)t0 * k_ld + (long)h * D : q);
+    const int qs = (int)q_ld * (int)sizeof(T), zs = (int)z_ld * (int)sizeof(T), ks = (int)k_ld * (int)sizeof(T);
+    const int last = r1 - 1 - t0;
+#pragma unroll
+    for (int u = 0; u < NI; ++u) {
+      const int idx = role + 256 * u;
+      const int d = min(idx < DP ? idx : idx - DP, D - 1) * (int)sizeof(T);
+      if (idx < DP) {
+#pragma unroll
+        for (int i = 0; i < HC; ++i) rq[u][i] = row_load<T>(qb, __umul24(min(ra + i, last), qs) + d);
+      } else if (GLA && (WHOLE || idx < 2 * DP)) {
+#pragma unroll
+        for (int i = 0; i < HC; ++i) rq[u][i] = row_load<T>(kb, __umul24(min(ra + i, last), ks) + d);
+      }
+      if (WHOLE || idx < 2 * DP) {
+#pragma unroll
+        for (int i = 0; i < HC; ++i) rz[u][i] = row_load<T>(zb, __umul24(min(ra + i, last), zs) + d);
+      }
+    }
+    if (tid >= 256) return;
+    const T* vr = v + (long)min(t0 + (tid >> 4), r1 - 1) * v_ld + (long)h * Dv;
+    const int c = c0 + 4 * (tid & 15);
+    if (vec & 2) {
+      rv = *reinterpret_cast<const t4*>(vr + min(c, Dv - 4));
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) rv[e] = vr[min(c + e, Dv - 1)];
+    }
+  };
+  // Gates of this thread's channels into LDS. No branch on rows or channels: a row past the sequence is set to f = 1, k =
+  // q = 0 by factors (`tail`: the last chunk has such rows), a channel past D has q = 0 (its state row is never read or
+  // stored). The running products cross from one half of the rows to the other between lanes l and l + 32.
+  auto stage = [&](int n, auto tail) {
+#pragma unroll
+    for (int u = 0; u < NI; ++u) {
+      const int idx = role + 256 * u;
+      const float one = 1.f - rl[u];
+      if (idx < DP) {
+        const float qm = idx < D ? 1.f : 0.f;
+        float F = 1.f, w[HC];
+#pragma unroll
+        for (int i = 0; i < HC; ++i) {
+          float f, qv;
+          if constexpr (GLA) {
+            f = gla_decay<FAST>((float)rz[u][i], inv_tau);
+            qv = (float)rq[u][i] * q_scale * qm;
+          } else {
+            float sg, cg;
+            sigmoid2<FAST>((float)rz[u][i] + rb[u], sg, cg);
+            f = fmaf(one, sg, rl[u]);
+            qv = act_in<FAST>((float)rq[u][i], act) * qm;
+          }
+          if (decltype(tail)::value) {
+            const float in = ra + i < n ? 1.f : 0.f;
+            f = fmaf(in, f, 1.f - in);
+            qv *= in;
+          }
+          F *= f;
+          sq[(ra + i) * KP + idx] = qv;
+          sf[(ra + i) * KP + idx] = f;
+          w[i] = qv * F;
+        }
+        const float Fo = __shfl_xor(F, 32, 64), by = hf ? Fo : 1.f;
+#pragma unroll
+        for (int i = 0; i < HC; ++i) {
+          sqf[(ra + i) * KP + idx] = w[i] * by;
+          if (hf) sqh[i * KP + idx] = w[i];
+        }
+        if (hf == 0) sl[idx] = F * Fo;
+      } else if (WHOLE || idx < 2 * DP) {
+        const int d = idx - DP;
+        float B = 1.f, w[HC];
+#pragma unroll
+        for (int i = HC - 1; i >= 0; --i) {
+          float f, k;
+          if constexpr (GLA) {
+            f = gla_decay<FAST>((float)rz[u][i], inv_tau);
+            k = (float)rq[u][i];
+          } else {
+            float sg, cg;
+            sigmoid2<FAST>((float)rz[u][i] + rb[u], sg, cg);
+            f = fmaf(one, sg, rl[u]);
+            k = one * cg;
+          }
+          if (decltype(tail)::value) {
+            const float in = ra + i < n ? 1.f : 0.f;
+            f = fmaf(in, f, 1.f - in);
+            k *= in;
+          }
+          sk[(ra + i) * KP + d] = k;
+          w[i] = k * B;
+          B *= f;
+        }
+        const float Bo = __shfl_xor(B, 32, 64), by = hf ? 1.f : Bo;
+#pragma unroll
+        for (int i = 0; i < HC; ++i) {
+          skb[(ra + i) * KP + d] = w[i] * by;
+          if (!hf) skh[i * KP + d] = w[i];
+        }
+      }
+    }
+    if (tid < 256) {
+      const int t = tid >> 4, c = 4 * (tid & 15);
+      f32x4 a;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) a[e] = (t < n && c0 + c + e < Dv) ? (float)rv[e] : 0.f;
+      *reinterpret_cast<f32x4*>(sv + t * VP + c) = a;
+    }
+  };
+  fetch(r0);
+  for (int t0 = r0; t0 < r1; t0 += C) {
+    const int n = min(C, r1 - t0);
+    if (n == C) stage(n, std::false_type{});
+    else stage(n, std::true_type{});
+    if (t0 + C < r1) fetch(t0 + C);      // in flight during the products below
+    __syncthreads();
+    // (q F) S, then the new state
+    f32x4 oc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < NH; ++i) {
+      const f32x4 a = *reinterpret_cast<const f32x4*>(sqf + m * KP + d0 + 16 * i + 4 * gg);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) oc = mfma_f32(a[e], st[i][e], oc);
+    }
+    float bv[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) bv[e] = sv[(4 * gg + e) * VP + cl];
+#pragma unroll
+    for (int i = 0; i < NH; ++i) {
+      st[i] *= *reinterpret_cast<const f32x4*>(sl + d0 + 16 * i + 4 * gg);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) st[i] = mfma_f32(skb[(4 * gg + e) * KP + d0 + 16 * i + m], bv[e], st[i]);
+    }
+    // weights of rows 8 .. 15 on columns 0 .. 7: this wave's channels
+    if (wave < NP) {
+      f32x4 w = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int i = 0; i < (NT + 7) / 8; ++i) {
+        const int at = (m & 7) * KP + 16 * (wave + 8 * i) + 4 * gg;
+        if (NT % 8 && wave + 8 * i >= NT) break;
+        const f32x4 a = *reinterpret_cast<const f32x4*>(sqh + at), b = *reinterpret_cast<const f32x4*>(skh + at);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) w = mfma_f32(a[e], b[e], w);
+      }
+      if (m < HC && gg < 2) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) sph[(wave * HC + 4 * gg + e) * HC + m] = w[e];
+      }
+    }
+    // the diagonal blocks: rows tb and 8 + tb, 32 lanes each share the row's channels, lane 16 + j keeps column j
+    {
+      const int tb = wave < 4 ? wave : 11 - wave, l4 = 4 * (lane & 31);      // (SIMDs get rows of equal work)
+      f32x4 qd[NU];
+#pragma unroll
+      for (int u = 0; u < NU; ++u) qd[u] = *reinterpret_cast<const f32x4*>(sq + (ra + tb) * KP + 128 * u + l4);
+      float keep = 0.f;
+#pragma unroll
+      for (int j = HC - 1; j >= 0; --j) {
+        if (j > tb) continue;
+        const float* fr = sf + (j < tb ? ra + j + 1 : C) * KP + l4;      // (its own column: not decayed yet)
+        const float* kr = sk + (ra + j) * KP + l4;
+        float w = 0.f;
+#pragma unroll
+        for (int u = 0; u < NU; ++u) {
+          qd[u] *= *reinterpret_cast<const f32x4*>(fr + 128 * u);
+          const f32x4 kk = *reinterpret_cast<const f32x4*>(kr + 128 * u);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) w = fmaf(qd[u][e], kk[e], w);
+        }
+        w = half_sum(w);
+        keep = m == j ? w : keep;
+      }
+      if ((lane & 16) && m < HC) sp[(ra + tb) * PP + ra + m] = keep;
+    }
+    if (wave >= 4) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) so[(4 * gg + e) * VP + cl] = oc[e];
+    }
+    __syncthreads();
+    if (wave < 4) {
+      f32x4 a = *reinterpret_cast<const f32x4*>(sp + m * PP + 4 * gg);
+      if (m >= HC && gg < 2) {
+        a = *reinterpret_cast<const f32x4*>(sph + (m - HC) * HC + 4 * gg);
+#pragma unroll
+        for (int i = 1; i < NP; ++i) a += *reinterpret_cast<const f32x4*>(sph + (i * HC + m - HC) * HC + 4 * gg);
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e) oc[e] += so[(4 * gg + e) * VP + cl];
+      float zero = 0.f;      // (x * 0 of an infinity or NaN is NaN)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) zero = fmaf(bv[e], 0.f, zero);
+      int odd = C;           // first row of this column that is no number
+      if (__any(zero != 0.f)) {
+#pragma unroll
+        for (int e = 3; e >= 0; --e) {
+          const bool bad = bv[e] * 0.f != 0.f;
+          odd = bad ? 4 * gg + e : odd;
+          bv[e] = bad ? 0.f : bv[e];
+        }
+        odd = min(odd, __shfl_xor(odd, 16, 64));
+        odd = min(odd, __shfl_xor(odd, 32, 64));
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e) oc = mfma_f32(a[e], bv[e], oc);
+      if (__any(odd < C)) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) oc[e] = 4 * gg + e >= odd ? NAN : oc[e];
+      }
+      if (live) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int t = 4 * gg + e;
+          if (t < n) o[((long)(t0 + t) * H + h) * Dv + col] = oc[e];
+        }
+      }
+    }
+    // (the next chunk's staging writes nothing that is read after the barrier above; sp, sph and so are rewritten only
+    // after its own first barrier)
+  }
+  int De = D;
+  asm volatile("" : "+s"(De));      // (the bounds are compared anew: kept masks would fill the scalar registers)
+  if (live) {
+#pragma unroll
+    for (int i = 0; i < NH; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int d = d0 + 16 * i + 4 * gg + e;
+        if (d < De) S[(long)d * Dv] = st[i][e];
+      }
+  }
+}
+
 // The same recurrence row by row, for steps of one row per sequence (decoding) and for any D. Workgroup =
 // (sequence, head, 64 value columns): 16 lanes of four columns by 16 groups of state rows; the state is read and
 // written in place, the row groups' partial read-outs are summed in LDS.
@@ -530,10 +853,32 @@ long records_at_once(long T, long nseq, int H, int D) {
 }
 
 template <typename T, int NT, bool GLA>
+void one_launch(const T* q, long q_ld, const T* key, long k_ld, float inv_tau, float q_scale, const T* z, long z_ld, const T* v,
+                long v_ld, const float* f_bias, const float* lower, float* state, const int* state_slots, const int* row_cu,
+                int nseq, const int* positions, int act, float* o, int H, int D, int Dv, hipStream_t s, int cost) {
+  constexpr int DP = 16 * NT, KP = (DP + 127) / 128 * 128 + 4;
+  constexpr size_t lds = (size_t)(97 * KP + 2 * 16 * 68 + 16 * 20 + 64 * (NT < 8 ? NT : 8) + DP) * sizeof(float);
+  static bool once = false;
+  if (!once) {
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&gate_scan_kernel<T, NT, GLA>),
+                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    once = true;
+  }
+  const int vec = (Dv % 4 == 0 && rows_aligned(v, v_ld, sizeof(T))) ? 2 : 0;
+  gate_scan_kernel<T, NT, GLA><<<dim3(nseq, H, (Dv + 63) / 64), 512, lds, s>>>(
+      q, q_ld, key, k_ld, inv_tau, q_scale, z, z_ld, v, v_ld, f_bias, lower, state, state_slots, row_cu, positions, act, vec, o, H,
+      D, Dv, cost);
+}
+
+// (rec null: in one launch)
+template <typename T, int NT, bool GLA>
 void chunk_launch(const T* q, long q_ld, const T* key, long k_ld, float inv_tau, float q_scale, const T* z, long z_ld, const T* v,
                   long v_ld, const float* f_bias, const float* lower, float* state, const int* state_slots, const int* row_cu,
                   int nseq, const int* positions, int act, float* o, float* rec, int T_, int H, int D, int Dv, hipStream_t s,
                   int cost) {
+  if (!rec)
+    return one_launch<T, NT, GLA>(q, q_ld, key, k_ld, inv_tau, q_scale, z, z_ld, v, v_ld, f_bias, lower, state, state_slots,
+                                  row_cu, nseq, positions, act, o, H, D, Dv, s, cost);
   constexpr int KP = 16 * NT + 4;
   constexpr size_t lds = (size_t)(81 * KP + 16 * 20 + 32 * NT) * sizeof(float);
   constexpr size_t chain_lds = (size_t)kChainSlots * (chunk_record(NT) + 1024) * sizeof(float);
@@ -614,6 +959,28 @@ void head_norm_gate_t(const float* o, const float* w, float eps, const T* gate, 
 }
 
 }  // namespace
+
+// Rows of a step's longest sequence up to which one launch takes its chunks: beyond, a chunk's 3 to 6 us there outweigh the second
+// launch, the records that go through memory, and 1.1 to 3 us a chunk. `wgs` workgroups of one launch; where they queue, it is their
+// work that counts. One launch and two, us, sequences of 16, 32, 64 rows (forget gates, bf16): one of 16 heads of 128 9.4 11.5, 13.0
+// 12.8, 20.7 15.6, eight 11.3 13.7, 15.2 16.7, 22.5 22.7, 64 57 55, 79 67, 119 99; one of 8 heads of 64 6.6 10.2, 9.7 11.0, 15.8 12.7, 64
+// 9.9 15.3, 14.5 20.4, 24 32, 200 28 39, 43 46, 72 68; 8 of 32 heads of 32 6.3 12.2, 9.2 13.4, 15 16.5, 64 24 25, 40 35, 72 53; one of 8
+// heads of 256 11.8 16.8, 17.6 19.3, 29 25, 64 102 115, 150 148, 244 214; in f32 one of 16 heads of 128 10.0 12.2, 14.4 13.6, 23 16.
+static int one_launch_rows(long wgs, int D, bool f32) {
+  if (f32) return wgs < 256 ? 16 : wgs < 512 ? (D > 64 ? 32 : 16) : 0;
+  if (D <= 32) return wgs < 64 ? 32 : wgs < 256 ? 48 : wgs < 512 ? 64 : wgs <= 768 ? 96 : wgs <= 1024 ? 48 : wgs <= 2048 ? 16 : 0;
+  if (D <= 64) return wgs < 128 ? 32 : wgs < 256 ? 48 : wgs <= 512 ? 96 : 64;
+  if (D <= 128) return wgs < 256 ? 16 : wgs <= (D <= 96 ? 512 : 256) ? 32 : wgs <= 1024 ? 16 : 0;
+  if (D <= 192) return wgs <= 1024 ? 16 : 0;
+  return wgs < 256 ? 32 : wgs < 512 ? 64 : wgs <= 1024 ? 32 : 16;
+}
+
+// The workgroups that count are those of sequences as long as the longest (max_rows 0: it may have every row but one of each other);
+// in f32 all of them (16 single rows beside 4 times 8, 16 heads of 128: 26.5 and 23.8 us, in bf16 23.0 and 22.9).
+bool chunks_in_one_launch(long T, long nseq, int H, int D, int Dv, bool f32, long max_rows, long max_ld) {
+  const long longest = std::max(1L, max_rows > 0 ? max_rows : T - nseq + 1), like = f32 ? nseq : std::min(nseq, (T + longest - 1) / longest);
+  return D <= 256 && max_ld < (1L << 21) && longest <= one_launch_rows(like * H * ((Dv + 63) / 64), D, f32);
+}
 
 long chunk_record_floats(long T, long nseq, int H, int D) {
   return D > 256 ? 0 : records_at_once(T, nseq, H, D) * H * chunk_record(record_tiles(D));

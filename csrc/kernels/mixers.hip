@@ -514,34 +514,71 @@ void launch_gla_chunks(const void* q, long q_ld, const void* k, long k_ld, const
                        int cost);      // forget.hip
 long chunk_record_floats(long T, long nseq, int H, int D);
 
-static ScanForms gla_forms(long T, long nseq, int H, int D, int Dv, bool f32, int max_rows, int& cost) {
-  // The chunks' two launches take some 11 us and 1.3 us a chunk of 128 channels, the loop 2.5 us and 0.6 us a row (f32 0.75), until
-  // the workgroups queue: then it is their work that counts. Chunks and loop in us, 16 heads of 128, one sequence of 16, 20, 32, 64
-  // rows: 12.3 11.7, 13.5 14.8, 13.0 20, 15.9 37; eight of them 13.9 13.9, 16.1 16.5, 16.9 21.6, 22.6 36.9; 200 149 185, 193 222, 200
-  // 347, 333 700; 200 of 12 rows 129 and 149; heads of 64, eight and 200 sequences of 32 rows 14.0 14.8, 72 91, of 32 channels 64
-  // rows 15.2 20.3, 77 119, of 192 12 rows 25 38, 355 747. (One launch per form that did both parts of a chunk, 1.5 to 6 us each,
-  // took 10.1 us for the one sequence of 16 rows, 2 us less than now; 22.5 for that of 64.)
+bool chunks_in_one_launch(long T, long nseq, int H, int D, int Dv, bool f32, long max_rows, long max_ld);
+
+struct GlaForms {
+  ScanForms form;
+  int cost;      // the chunks' (scan_in_chunks)
+  bool one;      // in one launch
+};
+static GlaForms gla_forms(long T, long nseq, int H, int D, int Dv, bool f32, int max_rows, long max_ld) {
   const long wgs = (long)H * ((Dv + 63) / 64);
   const bool queue = nseq * wgs >= 1024;
-  if (D > 128) cost = queue ? chunk_cost(4, 3) : chunk_cost(8, 2);
-  else if (D > 64) cost = queue ? chunk_cost(6, 6) : f32 ? chunk_cost(14, 3) : chunk_cost(14, 2);
-  else if (D > 32) cost = queue ? chunk_cost(14, 8) : chunk_cost(24, 3);
-  else cost = queue ? chunk_cost(36, 5) : chunk_cost(38, 2);
-  if (D > 256) return {true, false};
-  return scan_forms(T, nseq, cost, wgs, max_rows);
+  GlaForms f{{true, false}, 0, T > 0 && nseq > 0 && chunks_in_one_launch(T, nseq, H, D, Dv, f32, max_rows, max_ld)};
+  if (f.one) {
+    // One launch takes the time of 12 rows of 128 channels a chunk, in true f32 (whose decays are precise functions) of 14, and
+    // somewhat more where the workgroups queue. 16 heads of 128, time of chunks over loop for one sequence of 8, 12, 16, 20, 32
+    // rows: 1.09, 0.93, 0.79, 0.93, 0.69 (f32 1.43, 1.18, 0.93, 1.18, 0.83), for 200 of them 1.53, 1.26, 1.02, 1.04, 0.74;
+    // channels of 64 0.88 and 0.99 (1.03 and 1.30; queueing 1.06) at 16 rows, of 32 0.97 and 1.24 (1.14 and 1.58), of 192 0.53
+    // (0.56), of 256 0.87 at 8.
+    if (f32) f.cost = chunk_cost(0, D > 128 ? 11 : D > 64 ? (queue ? 15 : 14) : D > 32 && !queue ? 15 : 18);
+    else f.cost = chunk_cost(0, D > 128 ? 7 : D > 64 ? (queue ? 13 : 12) : D > 32 && !queue ? 14 : queue ? 18 : 15);
+    // More than a chunk only for a longest sequence that is worth it, and (wide channels) with many workgroups. One and two
+    // launches, us: 16 heads of 128, one sequence of 32 rows 13.9 12.9, eight 15.8 17.1 (f32 24.7 19.5); 8 heads of 256, one 20.7
+    // 19.6, eight 23.2 24.1, of 64 rows 37 32
+    const long longest = max_rows > 0 ? max_rows : T - nseq + 1;
+    f.one = longest <= 16 || (!f32 && scan_in_chunks(longest, f.cost) && (D <= 32 || (nseq * wgs >= 256 && (D <= 64 || longest <= 32))));
+    f.form = scan_forms(T, nseq, f.cost, wgs, max_rows);
+    // (beside a launch of the loop two launches are as good, and their line lies later: 16 single rows and four of 32 in 32 heads of
+    // 32 14.9 and 12.5 us, in 16 of 128 31.2 and 27.6)
+    if ((f32 && nseq * wgs >= 256) || (f.form.rows && f.form.chunks)) f.one = false;
+  }
+  if (!f.one) {
+    // The chunks' two launches take some 11 us and 1.3 us a chunk of 128 channels, the loop 2.5 us and 0.6 us a row (f32 0.75),
+    // until the workgroups queue: then it is their work that counts. Chunks and loop in us, 16 heads of 128, one sequence of 20,
+    // 32, 64 rows: 13.5 14.8, 13.0 20, 15.9 37; eight of them 16.1 16.5, 16.9 21.6, 22.6 36.9; 200 of 16, 20, 32, 64 149 185, 193
+    // 222, 200 347, 333 700; 200 of 12 rows 129 and 149; heads of 64, 200 sequences of 32 rows 72 91, of 32 channels 64 rows 77
+    // 119, of 192 12 rows 355 747.
+    if (D > 128) f.cost = queue ? chunk_cost(4, 3) : chunk_cost(8, 2);
+    else if (D > 64) f.cost = queue ? chunk_cost(6, 6) : f32 ? chunk_cost(14, 3) : chunk_cost(14, 2);
+    else if (D > 32) f.cost = queue ? chunk_cost(14, 8) : chunk_cost(24, 3);
+    else f.cost = queue ? chunk_cost(36, 5) : chunk_cost(38, 2);
+  }
+  if (D <= 256 && !f.one) f.form = scan_forms(T, nseq, f.cost, wgs, max_rows);
+  return f;
 }
 
-long gla_scan_scratch(int T, int nseq, int H, int D, int Dv, bool f32, int max_rows) {
-  int cost;
-  return T > 0 && nseq > 0 && gla_forms(T, nseq, H, D, Dv, f32, max_rows, cost).chunks ? chunk_record_floats(T, nseq, H, D) : 0;
+GlaSteps gla_scan_steps(int T, int nseq, int H, int D, int Dv, bool f32, int max_rows) {
+  const GlaForms f = gla_forms(T, nseq, H, D, Dv, f32, max_rows, (long)H * D);
+  if (!f.form.chunks) return {1, 0, -1};
+  int least = f.form.rows;
+  while (f.form.rows && !scan_in_chunks(least, f.cost)) ++least;
+  return {f.form.rows, f.one ? 1 : 2, least};
+}
+
+long gla_scan_scratch(int T, int nseq, int H, int D, int Dv, bool f32, int max_rows, long max_ld) {
+  if (T <= 0 || nseq <= 0) return 0;
+  const GlaForms f = gla_forms(T, nseq, H, D, Dv, f32, max_rows, max_ld);
+  return f.form.chunks && !f.one ? chunk_record_floats(T, nseq, H, D) : 0;
 }
 int launch_gla_scan(const void* q, long q_ld, const void* k, long k_ld, const void* v, long v_ld, const void* z,
                     long z_ld, float* state, const int* state_slots, const int* row_cu, int nseq,
                     const int* positions, float tau, float q_scale, float* o, float* rec, int T, int H, int D, int Dv, bool f32,
                     hipStream_t s, int max_rows) {
   if (T <= 0 || nseq <= 0) return 0;
-  int cost;
-  const ScanForms form = gla_forms(T, nseq, H, D, Dv, f32, max_rows, cost);
+  const GlaForms f = gla_forms(T, nseq, H, D, Dv, f32, max_rows, std::max({q_ld, k_ld, z_ld}));
+  const ScanForms form = f.form;
+  int cost = f.cost;
   if (form.chunks)
     launch_gla_chunks(q, q_ld, k, k_ld, v, v_ld, z, z_ld, state, state_slots, row_cu, nseq, positions, tau, q_scale, o, rec, T, H,
                       D, Dv, f32, s, form.rows ? cost : 0);

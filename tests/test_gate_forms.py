@@ -1,0 +1,63 @@
+"""Chunks of gated linear attention and of the forget gate in one launch (short sequences) and in two (records, then a chain): the
+line between them, and that both give what a loop over the rows gives."""
+import pytest
+import torch
+
+from butterfly_amd import ops
+
+built = pytest.mark.skipif(not ops.load_library(), reason="kernel library not built")
+
+
+@built
+def test_which_steps_take_one_launch():
+    forget, gla = torch.ops.bfly.forget_scan_launches, torch.ops.bfly.gla_scan_forms      # T, sequences, H, D, Dv, f32, max_rows
+    assert [forget(n, 1, 16, 128, 128, False, 0) for n in (1, 16, 17, 1000)] == [1, 1, 2, 2]
+    assert [forget(8 * n, 8, 16, 128, 128, False, n) for n in (32, 33)] == [1, 2]
+    assert [forget(n, 1, 16, 128, 128, True, 0) for n in (16, 17)] == [1, 2]
+    assert [forget(n, 1, 8, 64, 64, False, 0) for n in (32, 33)] == [1, 2]
+    assert [forget(8 * 16, 8, 16, 128, 128, False, m) for m in (16, 0, 100)] == [1, 2, 2]      # (0: one might have them all)
+    assert [forget(64 * 16, 64, 16, 128, 128, False, 16), forget(64 * 64, 64, 8, 64, 64, False, 64)] == [2, 1]
+    assert forget(300, 1, 4, 512, 64, False, 0) == 1                                          # row by row
+    # rows?, chunks (0 none, 1 in one launch, 2 in two), the fewest rows of a sequence in chunks
+    assert [gla(n, 1, 16, 128, 128, False, 0) for n in (8, 16, 64)] == [[1, 0, -1], [0, 1, 0], [0, 2, 0]]
+    assert [gla(8 * n, 8, 16, 128, 128, False, n)[1] for n in (16, 20, 32, 33)] == [1, 2, 1, 2]
+    assert gla(16 + 256, 17, 32, 32, 32, False, 256) == [1, 2, 44]
+    assert gla(16 + 64, 17, 16, 128, 128, False, 64) == [1, 0, -1]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["gla", "forget"])
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("D,Dv", [(24, 40), (64, 64), (96, 130), (128, 64), (192, 60), (256, 128)])
+@pytest.mark.parametrize("bad", [0.0, float("inf")])
+def test_one_launch_and_two(kind, dt, D, Dv, bad):
+    """Whole and padded chunks, an empty sequence and one without a slot; a value that is no number in a chunk's middle."""
+    seqs = [(0, 16), (5, 17), (0, 32), (9, 15), (3, 0), (0, 31), (4, 9), (2, 12)]
+    g = torch.Generator().manual_seed(D)
+    n, H, T = len(seqs), 2, sum(m for _, m in seqs)
+    rnd = lambda *s: torch.randn(*s, generator=g).to(torch.bfloat16).to(dt)            # noqa: E731
+    x = dict(q=rnd(T, H, D), v=rnd(T, H, Dv), state=torch.randn(n, H, D, Dv, generator=g))
+    x["v"][20, 1, 3] += bad                                   # row 4 of the second sequence
+    x["state_slots"] = torch.tensor([7, 6, 5, 4, 3, 2, -1, 0], dtype=torch.int32)
+    x["row_cu"] = torch.tensor([sum(m for _, m in seqs[:i]) for i in range(n + 1)], dtype=torch.int32)
+    x["positions"] = torch.cat([torch.arange(s, s + m) for s, m in seqs]).int()
+    z = 2 + 2 * rnd(T, H * D)
+    if kind == "gla":
+        op, kw = ops.gla_scan, dict(tau=16.0, q_scale=D ** -0.5)
+        x.update(k=rnd(T, H, D), z=z)
+    else:
+        op, kw = ops.forget_scan, dict(act="silu")
+        x.update(z=z.view(T, H, D), f_bias=torch.randn(H * D, generator=g), lower=0.9 * torch.rand(H * D, generator=g))
+    ref = {k: t.clone() for k, t in x.items()}
+    want = op(**ref, **kw)
+    rows = torch.ones(T, dtype=torch.bool)
+    rows[16 + 17 + 32 + 15 + 31:][:9] = False                 # (no slot)
+    for m in (32, 1000):                                      # as many rows are said to be the most: one launch, and two
+        got = {k: t.clone().cuda() for k, t in x.items()}
+        o = op(**got, **kw, max_rows=m).cpu()
+        assert (o[~rows] == 0).all()
+        for a, b in ((o[rows], want[rows]), (got["state"].cpu(), ref["state"])):
+            ok = b.isfinite()
+            assert torch.equal(a.isfinite(), ok)
+            # f32 sums over up to 256 channels in another order, products of up to 16 decays; hardware exp / log for bf16 inputs
+            assert (a - b)[ok].abs().max() < (3e-5 if dt == torch.bfloat16 else 1e-5) * b[ok].abs().max()
