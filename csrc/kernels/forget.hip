@@ -234,21 +234,24 @@ __global__ __launch_bounds__(32 * NT) void gate_chunk_kernel(const T* __restrict
   *reinterpret_cast<f32x4*>(rec + 33 * DP + (lane << 2)) = p;
 }
 
-// Workgroup = (sequence, head, 64 value columns), four waves of 16 columns with the whole height of the state each. The state
-// stays in the accumulator layout (tile i, element e: row d = 16 i + 4 gg + e of lane group gg), which is also the B operand
-// of (q F) S. Records arrive by LDS-DMA, SL chunks ahead (a chunk's products take 0.9 us, a record from memory two). The
-// records [first, first + count) of the step; a sequence that
-// goes on in the next ones leaves its state in its slot.
+// Workgroup = (sequence, head, 64 value columns), four waves of 16 columns with the whole height of the state each. The columns of a
+// head read the same records: they follow eight workgroups apart, in one XCD, and heads and sequences over all of them, also the few
+// whose records a launch of a long step holds (64 heads of 128, 32 sequences of 512 rows in five launches: 590 us each with the
+// sequences first, now 141). The state stays in the accumulator layout (tile i, element e: row d = 16 i + 4 gg + e of lane group gg),
+// which is also the B operand of (q F) S. Records arrive by LDS-DMA, SL chunks ahead (a chunk's products take 0.9 us, a record from
+// memory two). The records [first, first + count) of the step; a sequence that goes on in the next ones leaves its state in its slot.
 // A weight of zero does not hide a NaN: values v that are no numbers go in as zeros, and the outputs of their column are NaN
 // from their row on, as a row-by-row scan leaves them. (All other factors meet rows after theirs only.)
 template <typename T, int NT>
 __global__ __launch_bounds__(256, NT <= 8 ? 2 : 1) void gate_chain_kernel(
     const float* __restrict__ rec, const T* __restrict__ v, long v_ld, float* __restrict__ state,
     const int* __restrict__ state_slots, const int* __restrict__ row_cu, const int* __restrict__ positions,
-    float* __restrict__ o, int H, int D, int Dv, int cost, int first, int count) {
+    float* __restrict__ o, int nseq, int H, int D, int Dv, int cost, int first, int count) {
   constexpr int C = 16, DP = 16 * NT, SL = kChainSlots, REC = chunk_record(NT), U = REC / 256, PER = (U + 3) / 4;
   extern __shared__ __attribute__((aligned(16))) float smem[];      // [SL][REC], then values: [SL][4 waves][4][64]
-  const int s = blockIdx.x, h = blockIdx.y, c0 = blockIdx.z * 64;
+  const int nz = (Dv + 63) / 64, u = blockIdx.x >> 3, pair = u / nz * 8 + (blockIdx.x & 7), s = pair / H, h = pair - s * H;
+  const int c0 = u % nz * 64;
+  if (s >= nseq) return;
   const int r0 = __builtin_amdgcn_readfirstlane(row_cu[s]), r1 = __builtin_amdgcn_readfirstlane(row_cu[s + 1]);
   if (r1 <= r0 || (cost && !scan_in_chunks(r1 - r0, cost))) return;      // (the row-by-row form's)
   const int at = (r0 >> 4) + s, cb = max(0, first - at), ce = min((r1 - r0 + C - 1) / C, first + count - at);
@@ -896,8 +899,8 @@ void chunk_launch(const T* q, long q_ld, const T* key, long k_ld, float inv_tau,
     gate_chunk_kernel<T, NT, GLA><<<dim3(H, count), 32 * NT, lds, s>>>(q, q_ld, key, k_ld, inv_tau, q_scale, z, z_ld, f_bias, lower,
                                                                       state_slots, row_cu, nseq, act, rec, H, D, cost,
                                                                       (int)first);
-    gate_chain_kernel<T, NT><<<dim3(nseq, H, (Dv + 63) / 64), 256, chain_lds, s>>>(rec, v, v_ld, state, state_slots, row_cu, positions, o,
-                                                                           H, D, Dv, cost, (int)first, count);
+    gate_chain_kernel<T, NT><<<(nseq * H + 7) / 8 * 8 * ((Dv + 63) / 64), 256, chain_lds, s>>>(
+        rec, v, v_ld, state, state_slots, row_cu, positions, o, nseq, H, D, Dv, cost, (int)first, count);
   }
 }
 
