@@ -84,11 +84,13 @@ void forget_scan(const Tensor& q, const Tensor& z, const Tensor& v, const Tensor
   check_step(state_slots, row_cu, positions, T, "forget_scan");
   TORCH_CHECK(!one_row || state_slots.numel() == T, "forget_scan: one_row needs one row per sequence");
   TORCH_CHECK((act == 0 || act == 1) && D <= 4096, "forget_scan: act / key size");
-  TORCH_CHECK(q.stride(0) < (1 << 21) && z.stride(0) < (1 << 21), "forget_scan: row strides");      // (24-bit byte offsets)
   TORCH_CHECK(o.dim() == 3 && o.size(0) == T && o.size(1) == H && o.size(2) == Dv, "forget_scan: o [T, H, Dv]");
   const int64_t nseq = state_slots.numel();
+  const bool one = !one_row && bfly::chunks_in_one_launch(T, nseq, H, D, Dv, is_f32(q), max_rows, std::max(q.stride(0), z.stride(0)),
+                                                          v.stride(0));
+  TORCH_CHECK(one_row || one || D > 256 || bfly::gate_rows_near(H, Dv, v.stride(0)), "forget_scan: row strides");
   Tensor rec;
-  if (!one_row && !bfly::chunks_in_one_launch(T, nseq, H, D, Dv, is_f32(q), max_rows, std::max(q.stride(0), z.stride(0))))
+  if (!one_row && !one)
     rec = at::empty({bfly::chunk_record_floats(T, nseq, H, D)}, state.options());
   bfly::launch_forget_scan(q.data_ptr(), q.stride(0), z.data_ptr(), z.stride(0), v.data_ptr(), v.stride(0),
                            f_bias.data_ptr<float>(), lower.data_ptr<float>(), state.data_ptr<float>(),
@@ -100,7 +102,7 @@ void forget_scan(const Tensor& q, const Tensor& z, const Tensor& v, const Tensor
 
 // launches that a step of several rows takes
 int64_t forget_scan_launches(int64_t T, int64_t nseq, int64_t H, int64_t D, int64_t Dv, bool f32, int64_t max_rows) {
-  return D > 256 || bfly::chunks_in_one_launch(T, nseq, (int)H, (int)D, (int)Dv, f32, max_rows, H * D) ? 1 : 2;
+  return D > 256 || bfly::chunks_in_one_launch(T, nseq, (int)H, (int)D, (int)Dv, f32, max_rows, H * D, H * Dv) ? 1 : 2;
 }
 
 void head_norm_gate(const Tensor& o, const optional<Tensor>& w, double eps, const optional<Tensor>& gate, int64_t act,

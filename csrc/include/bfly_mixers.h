@@ -115,7 +115,7 @@ bool launch_attn_window_f32(const float* q, long q_ld, const float* k_cache, con
 
 // Gated linear attention scan over packed rows (see ops.gla_scan). Returns < 0 if D > 256. max_rows > 0: no sequence has
 // more rows. rec: scratch of gla_scan_scratch f32 elements (0: null); max_ld: the largest row stride of q, k, z
-long gla_scan_scratch(int T, int nseq, int H, int D, int Dv, bool f32, int max_rows, long max_ld);
+long gla_scan_scratch(int T, int nseq, int H, int D, int Dv, bool f32, int max_rows, long max_ld, long v_ld);
 // how it runs a step: row by row (0 or 1), chunks (0 none, 1 in one launch, 2 in two), the fewest rows of a sequence in chunks (0:
 // every one is, -1: none)
 struct GlaSteps {

@@ -27,8 +27,10 @@ void launch_forget_scan(const void* q, long q_ld, const void* z, long z_ld, cons
                         const float* lower, float* state, const int* state_slots, const int* row_cu, int nseq,
                         const int* positions, int act, float* o, float* rec, int T, int H, int D, int Dv, bool one_row,
                         bool f32, hipStream_t s);
-// Whether the chunks of a step go in one launch, without scratch (max_ld: the largest row stride)
-bool chunks_in_one_launch(long T, long nseq, int H, int D, int Dv, bool f32, long max_rows, long max_ld);
+// Whether the chunks of a step go in one launch, without scratch (max_ld: the largest row stride but v's). Two launches reach v and o
+// where gate_rows_near (16 rows within 2 GB).
+bool chunks_in_one_launch(long T, long nseq, int H, int D, int Dv, bool f32, long max_rows, long max_ld, long v_ld);
+bool gate_rows_near(int H, int Dv, long v_ld);
 // f32 elements of scratch for the chunks of a step of T rows and nseq sequences
 long chunk_record_floats(long T, long nseq, int H, int D);
 // out[t, h] = o[t, h] / sqrt(mean(o[t, h]^2) + eps) * w * act(gate[t, h]) * mul per head of Dv values; o f32 [T, H, Dv]

@@ -980,7 +980,10 @@ static int one_launch_rows(long wgs, int D, bool f32) {
 
 // The workgroups that count are those of sequences as long as the longest (max_rows 0: it may have every row but one of each other);
 // in f32 all of them (16 single rows beside 4 times 8, 16 heads of 128: 26.5 and 23.8 us, in bf16 23.0 and 22.9).
-bool chunks_in_one_launch(long T, long nseq, int H, int D, int Dv, bool f32, long max_rows, long max_ld) {
+// Its row strides of q, k, z are of 24 bits (max_ld), those of v of any size; two launches have it the other way round (gate_rows_near).
+bool gate_rows_near(int H, int Dv, long v_ld) { return std::max(v_ld, (long)H * Dv) * 64 < (1L << 31); }
+bool chunks_in_one_launch(long T, long nseq, int H, int D, int Dv, bool f32, long max_rows, long max_ld, long v_ld) {
+  if (!gate_rows_near(H, Dv, v_ld)) return D <= 256 && max_ld < (1L << 21);
   const long longest = std::max(1L, max_rows > 0 ? max_rows : T - nseq + 1), like = f32 ? nseq : std::min(nseq, (T + longest - 1) / longest);
   return D <= 256 && max_ld < (1L << 21) && longest <= one_launch_rows(like * H * ((Dv + 63) / 64), D, f32);
 }

@@ -514,17 +514,18 @@ void launch_gla_chunks(const void* q, long q_ld, const void* k, long k_ld, const
                        int cost);      // forget.hip
 long chunk_record_floats(long T, long nseq, int H, int D);
 
-bool chunks_in_one_launch(long T, long nseq, int H, int D, int Dv, bool f32, long max_rows, long max_ld);
+bool chunks_in_one_launch(long T, long nseq, int H, int D, int Dv, bool f32, long max_rows, long max_ld, long v_ld);
+bool gate_rows_near(int H, int Dv, long v_ld);
 
 struct GlaForms {
   ScanForms form;
   int cost;      // the chunks' (scan_in_chunks)
   bool one;      // in one launch
 };
-static GlaForms gla_forms(long T, long nseq, int H, int D, int Dv, bool f32, int max_rows, long max_ld) {
+static GlaForms gla_forms(long T, long nseq, int H, int D, int Dv, bool f32, int max_rows, long max_ld, long v_ld) {
   const long wgs = (long)H * ((Dv + 63) / 64);
   const bool queue = nseq * wgs >= 1024;
-  GlaForms f{{true, false}, 0, T > 0 && nseq > 0 && chunks_in_one_launch(T, nseq, H, D, Dv, f32, max_rows, max_ld)};
+  GlaForms f{{true, false}, 0, T > 0 && nseq > 0 && chunks_in_one_launch(T, nseq, H, D, Dv, f32, max_rows, max_ld, v_ld)};
   if (f.one) {
     // One launch takes the time of 12 rows of 128 channels a chunk, in true f32 (whose decays are precise functions) of 14, and
     // somewhat more where the workgroups queue. 16 heads of 128, time of chunks over loop for one sequence of 8, 12, 16, 20, 32
@@ -554,21 +555,22 @@ static GlaForms gla_forms(long T, long nseq, int H, int D, int Dv, bool f32, int
     else if (D > 32) f.cost = queue ? chunk_cost(14, 8) : chunk_cost(24, 3);
     else f.cost = queue ? chunk_cost(36, 5) : chunk_cost(38, 2);
   }
-  if (D <= 256 && !f.one) f.form = scan_forms(T, nseq, f.cost, wgs, max_rows);
+  if (!f.one) f.form = {true, false};
+  if (D <= 256 && !f.one && gate_rows_near(H, Dv, v_ld)) f.form = scan_forms(T, nseq, f.cost, wgs, max_rows);
   return f;
 }
 
 GlaSteps gla_scan_steps(int T, int nseq, int H, int D, int Dv, bool f32, int max_rows) {
-  const GlaForms f = gla_forms(T, nseq, H, D, Dv, f32, max_rows, (long)H * D);
+  const GlaForms f = gla_forms(T, nseq, H, D, Dv, f32, max_rows, (long)H * D, (long)H * Dv);
   if (!f.form.chunks) return {1, 0, -1};
   int least = f.form.rows;
   while (f.form.rows && !scan_in_chunks(least, f.cost)) ++least;
   return {f.form.rows, f.one ? 1 : 2, least};
 }
 
-long gla_scan_scratch(int T, int nseq, int H, int D, int Dv, bool f32, int max_rows, long max_ld) {
+long gla_scan_scratch(int T, int nseq, int H, int D, int Dv, bool f32, int max_rows, long max_ld, long v_ld) {
   if (T <= 0 || nseq <= 0) return 0;
-  const GlaForms f = gla_forms(T, nseq, H, D, Dv, f32, max_rows, max_ld);
+  const GlaForms f = gla_forms(T, nseq, H, D, Dv, f32, max_rows, max_ld, v_ld);
   return f.form.chunks && !f.one ? chunk_record_floats(T, nseq, H, D) : 0;
 }
 int launch_gla_scan(const void* q, long q_ld, const void* k, long k_ld, const void* v, long v_ld, const void* z,
@@ -576,7 +578,7 @@ int launch_gla_scan(const void* q, long q_ld, const void* k, long k_ld, const vo
                     const int* positions, float tau, float q_scale, float* o, float* rec, int T, int H, int D, int Dv, bool f32,
                     hipStream_t s, int max_rows) {
   if (T <= 0 || nseq <= 0) return 0;
-  const GlaForms f = gla_forms(T, nseq, H, D, Dv, f32, max_rows, std::max({q_ld, k_ld, z_ld}));
+  const GlaForms f = gla_forms(T, nseq, H, D, Dv, f32, max_rows, std::max({q_ld, k_ld, z_ld}), v_ld);
   const ScanForms form = f.form;
   int cost = f.cost;
   if (form.chunks)

@@ -61,3 +61,29 @@ def test_one_launch_and_two(kind, dt, D, Dv, bad):
             assert torch.equal(a.isfinite(), ok)
             # f32 sums over up to 256 channels in another order, products of up to 16 decays; hardware exp / log for bf16 inputs
             assert (a - b)[ok].abs().max() < (3e-5 if dt == torch.bfloat16 else 1e-5) * b[ok].abs().max()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["gla", "forget"])
+@pytest.mark.parametrize("far,ld", [("qkz", (1 << 21) + 8), ("v", 1 << 26)])
+def test_rows_far_apart(kind, far, ld):
+    """Row strides that the 24-bit offsets of one launch and the 32-bit ones of two do not hold give what dense rows give."""
+    n, H, D, Dv = 40, 2, 64, 64
+    g = torch.Generator().manual_seed(1)
+    rnd = lambda *s: torch.randn(*s, generator=g).to(torch.bfloat16).cuda()            # noqa: E731
+    q, k, v, z = rnd(n, H, D), rnd(n, H, D), rnd(n, H, Dv), rnd(n, H, D) + 2
+    idx = [torch.tensor(t, dtype=torch.int32, device="cuda") for t in ([0], [0, n], list(range(n)))]
+    apart = lambda t: torch.empty(n, ld, dtype=t.dtype, device="cuda")[:, :t[0].numel()].view(t.shape).copy_(t)      # noqa: E731
+    fb, lo = torch.randn(H * D, generator=g).cuda(), (0.9 * torch.rand(H * D, generator=g)).cuda()
+
+    def run(q, k, v, z):
+        state = torch.zeros(1, H, D, Dv, device="cuda")
+        if kind == "gla":
+            return ops.gla_scan(q, k, v, z.view(n, H * D), state, *idx, 16.0, D ** -0.5), state
+        return ops.forget_scan(q, z, v, fb, lo, state, *idx, "silu"), state
+
+    want = run(q, k, v, z)
+    got = run(apart(q), apart(k), v, apart(z)) if far == "qkz" else run(q, k, apart(v), z)
+    # the same sums in f32, in another order
+    for a, b in zip(got, want):
+        assert (a - b).abs().max() < 3e-5 * b.abs().max()
