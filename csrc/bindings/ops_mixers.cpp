@@ -320,6 +320,7 @@ void gla_scan(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& z
   TORCH_CHECK(row_cu.numel() == nseq + 1 && positions.numel() == T, "gla_scan: row_cu / positions");
   TORCH_CHECK(o.dim() == 3 && o.size(0) == T && o.size(1) == H && o.size(2) == Dv, "gla_scan: o");
   TORCH_CHECK(tau > 0, "gla_scan: tau");
+  if (!o.numel()) return;
   const long n = bfly::gla_scan_scratch((int)T, (int)nseq, (int)H, (int)D, (int)Dv, is_f32(q), (int)max_rows,
                                         std::max({q.stride(0), k.stride(0), z.stride(0)}), v.stride(0));
   Tensor rec;

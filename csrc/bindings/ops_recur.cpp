@@ -85,6 +85,7 @@ void forget_scan(const Tensor& q, const Tensor& z, const Tensor& v, const Tensor
   TORCH_CHECK(!one_row || state_slots.numel() == T, "forget_scan: one_row needs one row per sequence");
   TORCH_CHECK((act == 0 || act == 1) && D <= 4096, "forget_scan: act / key size");
   TORCH_CHECK(o.dim() == 3 && o.size(0) == T && o.size(1) == H && o.size(2) == Dv, "forget_scan: o [T, H, Dv]");
+  if (!o.numel()) return;
   const int64_t nseq = state_slots.numel();
   const bool one = !one_row && bfly::chunks_in_one_launch(T, nseq, H, D, Dv, is_f32(q), max_rows, std::max(q.stride(0), z.stride(0)),
                                                           v.stride(0));

@@ -87,3 +87,12 @@ def test_rows_far_apart(kind, far, ld):
     # the same sums in f32, in another order
     for a, b in zip(got, want):
         assert (a - b).abs().max() < 3e-5 * b.abs().max()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T,H", [(40, 0), (0, 2)])
+def test_nothing_to_scan(T, H):
+    D, Dv, z = 32, 64, lambda *s: torch.zeros(*s, device="cuda")            # noqa: E731
+    idx = [torch.tensor(t, dtype=torch.int32, device="cuda") for t in ([0], [0, T], list(range(T)))]
+    assert ops.gla_scan(z(T, H, D), z(T, H, D), z(T, H, Dv), z(T, H * D), z(1, H, D, Dv), *idx, 16.0, 1.0).shape == (T, H, Dv)
+    assert ops.forget_scan(z(T, H, D), z(T, H, D), z(T, H, Dv), z(H * D), z(H * D), z(1, H, D, Dv), *idx).shape == (T, H, Dv)
