@@ -281,7 +281,7 @@ class NesizenLM(PackedStack):
         for n, (sp, q) in enumerate(subs):
             pre = f"l{sp['index']}."
             if q == 2:
-                y = self._ffn(sp["ffn"], pre, h, n + 1 < len(subs) and self.streams <= 4)
+                y = self._ffn(sp["ffn"], pre, h)
             elif sp["type"] == "attention":
                 y = self._attention(sp, pre, h, fb, meta, kv_caches)
             else:
@@ -330,11 +330,10 @@ class NesizenLM(PackedStack):
         y = ops.gla_out(o, g, self.p[pre + "gnorm"], self.cfg.norm_eps, self.dtype)
         return ops.linear_rows(y, self.p[pre + "o"])
 
-    def _ffn(self, fs, pre, h, fused):
+    def _ffn(self, fs, pre, h):
         if fs["kind"] == "dense":
             return ops.linear_rows(ops.linear_act(h, self.p[pre + "up"], act="relu2"), self.p[pre + "down"])
         ids, w = ops.moe_route_scores(h, self.p[pre + "router"], fs["top"], scoring="sigmoid", renorm=False)
-        # fused: hc_post_pre_ is next and sums the choices
-        experts = ops.moe_glu_rows if fused else ops.moe_glu_ffn
-        return experts(h, ids, w, self.p[pre + "gate_up"], self.p[pre + "edown"],
-                       float("inf") if fs["limit"] is None else fs["limit"], GLU_ALPHA)
+        # (hc_post_pre_ sums the choices)
+        return ops.moe_glu_rows(h, ids, w, self.p[pre + "gate_up"], self.p[pre + "edown"],
+                                float("inf") if fs["limit"] is None else fs["limit"], GLU_ALPHA)

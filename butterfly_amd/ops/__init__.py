@@ -215,7 +215,7 @@ class Partial:
 
 
 def materialize(x):
-    return x.materialize() if isinstance(x, Partial) else x
+    return x.materialize() if isinstance(x, (Partial, ExpertRows)) else x
 
 
 class RowNormed:
@@ -835,7 +835,8 @@ def hc_post_pre_(xs, y, mix, w_out, w_in2, norm_w2, eps: float, offset: float, o
         ref.hc_post_(xs, y, mix, w_out)
         return ref.hc_pre(xs, w_in2, norm_w2, eps, offset, out_dtype)
     out = _empty(xs.shape[0], xs.shape[2], dtype=out_dtype, device=xs.device)
-    y, parts = _row_parts(y, xs.shape[2], xs.shape[1] <= 4)
+    ok = xs.shape[1] <= 4 and all(t.data_ptr() % 16 == 0 for t in (xs, norm_w2, out))
+    y, parts = _row_parts(y, xs.shape[2], ok, out_dtype)
     torch.ops.bfly.hc_post_pre(xs, y, mix, w_out, w_in2, norm_w2, eps, offset, out, *parts[:2], *parts[3:])
     return out
 
@@ -1021,27 +1022,33 @@ def _moe_glu(x, topk_ids, topk_w, gate_up_w, down_w, limit, alpha, up_offset, sc
 
 class ExpertRows:
     """Outputs of a token's experts whose sum is left to the row kernel that reads it (moe_glu_rows): `y` [T * choices, W]
-    f32 in the shared workspace, to be consumed (post_norm_add_norm, hc_post_pre_) before the next experts run; `w` their
-    weights (None: the plain sum), `dtype` that of the row."""
+    f32 in the shared workspace, to be consumed (post_norm_add_norm, hc_post_pre_) or `materialize()`d before the next experts
+    run; `w` their weights (None: the plain sum), `dtype` that of the row."""
 
     __slots__ = ("y", "w", "choices", "dtype")
 
     def __init__(self, y, w, choices, dtype):
         self.y, self.w, self.choices, self.dtype = y, w, choices, dtype
 
+    def materialize(self) -> torch.Tensor:
+        out = _empty(self.y.shape[0] // self.choices, self.y.shape[1], dtype=self.dtype, device=self.y.device)
+        torch.ops.bfly.moe_sum(self.y, self.w, self.choices, out)
+        return out
+
 
 def _rows_take_parts(W: int) -> bool:
     return W % 4 == 0 and 256 < W <= 4096
 
 
-def _row_parts(y, W: int, ok: bool):
-    """A row kernel's input as (tensor, (parts, weights, f32, slabs))."""
-    if isinstance(y, ExpertRows):
-        return y.y, (y.choices, y.w, y.dtype == torch.float32, False)
-    if isinstance(y, Partial):
-        if ok and _rows_take_parts(W):
-            return y.slabs.view(-1, W), (y.slabs.shape[0], None, False, True)
-        y = y.materialize()
+def _row_parts(y, W: int, ok: bool, dtype):
+    """A row kernel's input as (tensor, (parts, weights, f32, slabs)). ok: the kernel sums parts of its rows itself, of the type
+    `dtype`."""
+    if isinstance(y, (ExpertRows, Partial)):
+        if not (ok and _rows_take_parts(W) and dtype == (y.dtype if isinstance(y, ExpertRows) else y.out.dtype)):
+            return y.materialize(), (0, None, False, False)
+        if isinstance(y, ExpertRows):
+            return y.y, (y.choices, y.w, y.dtype == torch.float32, False)
+        return y.slabs.view(-1, W), (y.slabs.shape[0], None, False, True)
     return y, (0, None, False, False)
 
 
@@ -1056,8 +1063,8 @@ def linear_rows(x, w):
 
 def moe_glu_rows(x, topk_ids, topk_w, gate_up_w, down_w, limit: float, alpha: float, up_offset: float = 1.0,
                  scale_input: bool = True, plain_act=None):
-    """moe_glu_ffn for post_norm_add_norm (with a norm) or hc_post_pre_ (up to four streams) right behind it, which form the
-    sum over the choices themselves where their rows stay in registers: ExpertRows then, else the sum."""
+    """moe_glu_ffn for post_norm_add_norm or hc_post_pre_ right behind it, which form the sum over the choices themselves where
+    their rows stay in registers: ExpertRows then, else the sum."""
     if not (_gpu(x) and _rows_take_parts(x.shape[1]) and topk_ids.numel() > 0):
         return moe_glu_ffn(x, topk_ids, topk_w, gate_up_w, down_w, limit, alpha, up_offset, scale_input, plain_act)
     return _moe_glu(x, topk_ids, topk_w, gate_up_w, down_w, limit, alpha, up_offset, scale_input, plain_act, None, False, True)
@@ -1324,7 +1331,7 @@ def post_norm_add_norm(x, y, norm_w, norm_b, eps: float, mult: float, extra, nor
         return ref.post_norm_add_norm(x, y, norm_w, norm_b, eps, mult, extra, norm2_w, norm2_b, out_dtype, rms)
     h = None if norm2_w is None else _empty(x.shape[0], x.shape[1], dtype=out_dtype, device=x.device)
     rest = (norm_w, norm_b, float(eps), float(mult), extra, norm2_w, norm2_b, h, bool(rms))
-    y, parts = _row_parts(y, x.shape[1], norm_w is not None)
+    y, parts = _row_parts(y, x.shape[1], norm_w is not None, out_dtype)
     torch.ops.bfly.post_norm_add_norm(x, y, *rest, *parts)
     return h
 

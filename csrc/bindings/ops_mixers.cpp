@@ -480,6 +480,20 @@ void sample_greedy_f32(const Tensor& logits, int64_t vstart, Tensor& out_ids, Te
                                  out_ids.data_ptr<int>(), out_scores.data_ptr<float>(), cur_stream(), check_finite ? 1 : 0);
 }
 
+// out[t] = sum_j w[t, j] y[t * choices + j] (w null: the plain sum)
+void moe_sum(const Tensor& y, const optional<Tensor>& w, int64_t choices, Tensor& out) {
+  CHK_GPU(y); CHK_F32(y);
+  TORCH_CHECK(y.dim() == 2 && out.is_cuda() && out.dim() == 2 && out.is_contiguous() && choices > 0 &&
+                  y.size(0) == out.size(0) * choices && y.size(1) == out.size(1), "moe_sum: y [T * choices, W], out [T, W]");
+  TORCH_CHECK(is_f32(out) || out.scalar_type() == at::kBFloat16, "moe_sum: out");
+  if (w.has_value()) {
+    CHK_F32(*w);
+    TORCH_CHECK(w->numel() == y.size(0), "moe_sum: weights [T, choices]");
+  }
+  bfly::launch_moe_sum(y.data_ptr<float>(), w.has_value() ? w->data_ptr<float>() : nullptr, (int)choices, out.data_ptr(),
+                       (int)out.size(0), (int)out.size(1), is_f32(out), cur_stream(), nullptr, 0, nullptr, 0, nullptr, 0);
+}
+
 }  // namespace
 
 TORCH_LIBRARY_FRAGMENT(bfly, m) {
@@ -512,6 +526,7 @@ TORCH_LIBRARY_FRAGMENT(bfly, m) {
   m.def("moe_route_rows(Tensor x, Tensor wr, Tensor? bias, int top_k, int scoring, bool renorm, Tensor(a!) ids, "
         "Tensor(b!) w, Tensor? select_bias=None, int ngroups=1, int keep=1, float renorm_eps=0.0, float scale=1.0) -> ()");
   m.def("moe_sort_max_tiles(int tk, int experts) -> int", &moe_sort_max_tiles);
+  m.def("moe_sum(Tensor y, Tensor? w, int choices, Tensor(a!) out) -> ()");
   m.def("moe_glu_ffn(Tensor x, Tensor topk_ids, Tensor topk_w, Tensor gate_up_w, Tensor down_w, float limit, "
         "float alpha, float up_offset, bool scale_input, Tensor(a!) work, Tensor(b!) hmid, Tensor(c!) y, "
         "Tensor(d!)? out, int plain_act=0, Tensor? addend=None, bool identity=False) -> ()");
@@ -535,5 +550,6 @@ TORCH_LIBRARY_IMPL(bfly, CUDA, m) {
   m.impl("router_logits", &router_logits);
   m.impl("moe_topk_scores", &moe_topk_scores);
   m.impl("moe_route_rows", &moe_route_rows);
+  m.impl("moe_sum", &moe_sum);
   m.impl("moe_glu_ffn", &moe_glu_ffn);
 }

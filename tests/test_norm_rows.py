@@ -93,3 +93,37 @@ def test_slabs_summed_by_the_row_kernels(M, N, K):
         ops.hc_post_(got, ops.linear_rows(x, w), mix, wo)
         ops.hc_post_(want, ops.linear_act(x, w), mix, wo)
         assert torch.equal(got, want)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("W,scaled", [(512, True), (1028, False), (4096, False)])
+def test_experts_summed_where_the_row_kernel_cannot(dt, W, scaled):
+    """Outputs of experts in front of kernels that take whole rows only (no norm on them, five streams, the last update, streams off
+    a 16-byte line) are summed first, bit for bit as by moe_glu_ffn; rows of another type stay refused."""
+    g = torch.Generator().manual_seed(W)
+    d = lambda *s, k=1.0: (k * torch.randn(*s, generator=g)).cuda()            # noqa: E731
+    T, E, F = 6, 5, 64
+    x, gu, dn = d(T, W).to(dt), d(E, 2 * F, W, k=W ** -0.5).to(dt), d(E, W, F, k=F ** -0.5).to(dt)
+    ids, w = torch.rand(T, E, generator=g).topk(2, -1).indices.int().cuda(), torch.rand(T, 2, generator=g).cuda()
+    args = (x, ids, w, gu, dn, 7.0, 1.702, 1.0, scaled)
+    want_y = ops.moe_glu_ffn(*args)
+    rows = ops.moe_glu_rows(*args)
+    assert isinstance(rows, ops.ExpertRows) and torch.equal(ops.materialize(rows), want_y)
+    r, w1 = d(T, W), d(W)
+    got, want = r.clone(), r.clone()
+    h = ops.post_norm_add_norm(got, ops.moe_glu_rows(*args), None, None, 1e-5, 0.7, None, w1, None, dt, rms=True)
+    h2 = ops.post_norm_add_norm(want, want_y, None, None, 1e-5, 0.7, None, w1, None, dt, rms=True)
+    assert torch.equal(got, want) and torch.equal(h, h2)
+    for S, off in ((5, 0), (2, 1)):
+        xs, mix, wo, wi = d(T * S * W + 1)[off:][:T * S * W].view(T, S, W), d(S, S), d(S), d(S)
+        got, want = torch.empty(T * S * W + 1, device="cuda")[off:][:T * S * W].view(T, S, W).copy_(xs), xs.clone()
+        h = ops.hc_post_pre_(got, ops.moe_glu_rows(*args), mix, wo, wi, w1, 1e-5, 1.0, dt)
+        h2 = ops.hc_post_pre_(want if off == 0 else xs, want_y, mix, wo, wi, w1, 1e-5, 1.0, dt)
+        assert torch.equal(got, want if off == 0 else xs) and torch.equal(h, h2)
+        ops.hc_post_(got, ops.moe_glu_rows(*args), mix, wo)
+        ops.hc_post_(want if off == 0 else xs, want_y, mix, wo)
+        assert torch.equal(got, want if off == 0 else xs)
+        with pytest.raises(RuntimeError):
+            ops.hc_post_pre_(got, ops.moe_glu_rows(*args), mix, wo, wi, w1, 1e-5, 1.0,
+                             torch.float32 if dt == torch.bfloat16 else torch.bfloat16)
