@@ -15,6 +15,23 @@ F64 = torch.float64
     (1, 200, 70, [(0, 31)]), (2, 256, 128, [(1, 100)]), (2, 64, 256, [(0, 300), (0, 3)]),
 ])
 def test_prompt_chunks_match_the_token_loop(dt, tol, H, D, Dv, seqs):
+    token_loop(dt, tol, H, D, Dv, seqs)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dt,tol", [(torch.float32, 3e-6), (torch.bfloat16, 3e-5)])
+@pytest.mark.parametrize("H,D,Dv,seqs", [      # whole chunks, one row over, one short; all channel tiles
+    (2, 128, 128, [(0, 64)]), (2, 128, 128, [(5, 65), (0, 111), (0, 1), (3, 2)]), (3, 128, 72, [(0, 79), (7, 33)]),
+    (3, 24, 40, [(0, 127)]), (2, 32, 64, [(4, 97), (0, 160)]), (1, 96, 64, [(7, 81), (0, 48)]), (2, 80, 100, [(0, 144)]),
+    (1, 192, 128, [(0, 49), (2, 64)]), (2, 64, 64, [(0, 113), (6, 64)]), (1, 250, 30, [(0, 35)]),
+])
+def test_long_prompts_match_the_token_loop(dt, tol, H, D, Dv, seqs):
+    """Steps whose every sequence runs in chunks, in two launches."""
+    assert torch.ops.bfly.gla_scan_forms(sum(n for _, n in seqs), len(seqs), H, D, Dv, dt == torch.float32, 0) == [0, 2, 0]
+    token_loop(dt, tol, H, D, Dv, seqs)
+
+
+def token_loop(dt, tol, H, D, Dv, seqs):
     g = torch.Generator().manual_seed(D + Dv)
     T, nslots, tau = sum(n for _, n in seqs), len(seqs) + 1, 16.0
     rnd = lambda *s: torch.randn(*s, generator=g).to(torch.bfloat16).to(dt)            # noqa: E731
@@ -53,6 +70,29 @@ def test_values_that_are_no_numbers_reach_later_rows_only(row, where, bad):
     T, rnd = 75, lambda *s: torch.randn(*s, generator=g)            # noqa: E731
     x = dict(q=rnd(T, H, D), k=rnd(T, H, D), v=rnd(T, H, Dv), z=2 + rnd(T, H * D), state=rnd(2, H, D, Dv),
              state_slots=torch.tensor([1, 0], dtype=torch.int32), row_cu=torch.tensor([0, 35, 75], dtype=torch.int32),
+             positions=torch.cat([torch.arange(s, s + n) for s, n in seqs]).int())
+    x[where].view(T, H, -1)[row, 1, 5] = bad
+    got, ref = {k: t.cuda() for k, t in x.items()}, {k: t.clone() for k, t in x.items()}
+    o, w = (ops.gla_scan(**a, tau=16.0, q_scale=D ** -0.5) for a in (got, ref))
+    for a, b in ((o.cpu(), w), (got["state"].cpu(), ref["state"])):
+        assert torch.equal(a.isfinite(), b.isfinite())
+        ok = b.isfinite()
+        assert (a - b)[ok].abs().max() < 1e-5 * b[ok].abs().max()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("bad", [float("nan"), float("inf")])
+@pytest.mark.parametrize("where", ["q", "k", "v", "z"])
+@pytest.mark.parametrize("row", [0, 7, 11, 16, 47, 69])
+@pytest.mark.parametrize("D", [64, 128])
+def test_values_that_are_no_numbers_in_long_prompts(D, row, where, bad):
+    """The same where both sequences are long enough for chunks in two launches; the first ends in a chunk of six rows."""
+    g = torch.Generator().manual_seed(row)
+    seqs, H, Dv = [(3, 70), (0, 100)], 2, 80
+    T, rnd = 170, lambda *s: torch.randn(*s, generator=g)            # noqa: E731
+    assert torch.ops.bfly.gla_scan_forms(T, 2, H, D, Dv, True, 0) == [0, 2, 0]
+    x = dict(q=rnd(T, H, D), k=rnd(T, H, D), v=rnd(T, H, Dv), z=2 + rnd(T, H * D), state=rnd(2, H, D, Dv),
+             state_slots=torch.tensor([1, 0], dtype=torch.int32), row_cu=torch.tensor([0, 70, T], dtype=torch.int32),
              positions=torch.cat([torch.arange(s, s + n) for s, n in seqs]).int())
     x[where].view(T, H, -1)[row, 1, 5] = bad
     got, ref = {k: t.cuda() for k, t in x.items()}, {k: t.clone() for k, t in x.items()}
