@@ -75,6 +75,22 @@ def test_experts_summed_by_the_row_kernels(dt, T, W, K, scaled):
 @pytest.mark.parametrize("N,K", [(256, 2048), (384, 4096), (1024, 2048), (2048, 1024), (4096, 6144), (4224, 4096)])
 def test_slabs_summed_by_the_row_kernels(M, N, K):
     """The slabs of a product with K split are summed inside the row kernels as by the reduce launch, bit for bit."""
+    slabs(M, N, K)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K,kind,splits", [
+    (257, 2048, 2048, "big4", 4), (300, 1024, 2048, "big4", 4), (513, 4096, 4096, "big4", 4),      # a row past a tile, short last tiles
+    (300, 4096, 6144, "big4", 8), (777, 4096, 6144, "big4", 4), (257, 4096, 4096, "mid8", 4), (300, 1152, 4096, "tile", 16),
+])
+def test_slabs_of_prompts(M, N, K, kind, splits):
+    """The same behind the tiles that prompts run on."""
+    plan = ops.gemm_plan(M, N, K)
+    assert (plan["kind"], plan["splitk"]) == (kind, splits)
+    slabs(M, N, K)
+
+
+def slabs(M, N, K):
     g = torch.Generator().manual_seed(M + N)
     d = lambda *s, k=1.0: (k * torch.randn(*s, generator=g)).cuda()            # noqa: E731
     dt = torch.bfloat16
