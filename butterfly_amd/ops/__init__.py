@@ -671,7 +671,7 @@ def moe_sparse_ffn(x, topk_ids, topk_w, gu_w, down_w, e0: int, num_local: int, f
     # `expected_slots`: (token, k) pairs expected to be local (the EP dispatch pads with
     # non-local / empty slots; they cost nothing but must not size the launch)
     exp = TK if expected_slots is None else max(1, min(TK, expected_slots))
-    bm = moe_sparse_tile_rows(exp, num_local, H, ffn)
+    bm = moe_sparse_tile_rows(exp, num_local, H, ffn, down_w.stride(0) * down_w.element_size() % 32768 == 0)
     rows = _arena.get(dev, "moe_rows", TK, torch.int32)[:TK]
     slot_of = _arena.get(dev, "moe_slot", TK, torch.int32)[:TK]
     nt = L.moe_max_tiles(TK, num_local, bm)
@@ -719,18 +719,27 @@ def ep_combine(back, slot):
     return out
 
 
-def moe_sparse_tile_rows(exp: int, num_local: int, H: int, ffn: int) -> int:
+def moe_sparse_tile_rows(exp: int, num_local: int, H: int, ffn: int, aliased: bool = False) -> int:
     """Rows of a grouped expert tile for `exp` expected (token, expert) pairs. The 256-row tile (128 rows of it where an expert
-    has no more) reads an expert's weights once and gathers rows without a load in its K loop, so it is ahead from few rows on
-    where its workgroups, one per expert and 256 columns, occupy the compute units. Gate/up + down + combine in us on 64- and
-    256-row tiles: 8 experts of 4096 x 14336, 8, 16, 25, 75, 250 rows per expert 526 531, 539 538, 585 546, 981 586, 2190 880; 64
-    experts of 2048 x 1408, 19, 28, 47, 75 rows 224 235, 237 240, 254 247, 394 256; 16 of 2048 x 2048, 12, 100 rows 121 106, 156
-    115. With fewer column tiles of the down projection the line lies later: four experts of 4096 x 14336 (64), 32, 50 rows 290
-    358, 451 374; two (32), 64, 100, 150 rows 240 282, 277 293, 358 281; eight of 1024 x 2048 (32), 50, 75, 200 rows 42 49, 58 50,
-    82 54."""
+    has no more) reads an expert's weights once, which counts from where many experts have more than 64 rows, if its workgroups, one
+    per expert and 256 columns, occupy the compute units; for up to 16 experts it is as good or better from 24 rows on, as it gathers
+    rows without a load in its K loop. `aliased`: rows of the down projection a multiple of 32 KB apart, which it waits for.
+    Gate/up + down + combine on it over 64-row tiles, at 24, 40, 50, 64, 80, 100, 150 rows per expert: 8 experts of 4096 x 14336 1.02
+    0.96 0.95 0.72 0.61 0.59 0.49 (aliased 1.15 1.11 1.10 0.81 0.68 0.66 0.52), of 4096 x 4096 0.91 0.88 0.87 0.86 0.64 (0.96 0.94 0.93
+    0.89), 16 of 2048 x 1408 0.83 0.86 0.86 0.61, of 4096 x 3072 0.96 0.98 0.96 0.73 (1.22 1.19 1.19 0.88), 32 of 2048 x 1024 1.22 1.20
+    1.16 0.88 0.71 (1.41 1.40 1.37 1.01 0.84), 64 of 2048 x 1408 1.08 1.05 1.03 0.81; with 64 column tiles of all experts, four of 4096
+    x 14336 1.29 1.21 0.84 0.82, of 4096 x 4096 1.07 1.06 1.02 1.08 0.70 (1.23 1.18 1.16 1.16 0.80), 8 of 2048 x 5632 1.18 1.16 1.16
+    0.97; with 32, two of 4096 x 14336 1.61 1.19 1.23 1.19 1.10 1.09 0.83, eight of 1024 x 4096 1.16 1.09 1.07 1.04 0.86 0.82 (1.61 1.54
+    1.53 1.44 1.21 1.18 1.00)."""
     if H % 256 == 0 and (2 * ffn) % 256 == 0 and _BIG_MOE:
         down = num_local * (H // 256)     # column tiles of all experts
-        if exp >= (24 if down >= 96 else 40 if down >= 64 else 96) * num_local:
+        if down >= 96:
+            line = 24 if num_local <= 16 and not aliased else 56
+        elif down >= 64:
+            line = 72 if aliased else 56
+        else:
+            line = 150 if aliased else 96
+        if exp >= line * num_local:
             return 256
     return 128 if exp >= 96 * num_local else 64
 

@@ -140,7 +140,10 @@ def test_sparse_tile_rows():
     """64-row tiles for a few rows per expert, 256-row tiles as soon as their workgroups pay; 128-row tiles for other sizes."""
     rows = lambda n, E, H, F: ops.moe_sparse_tile_rows(n, E, H, F)                       # noqa: E731
     assert [rows(n, 8, 4096, 14336) for n in (191, 192, 4096)] == [64, 256, 256]
-    assert [rows(n, 4, 4096, 14336) for n in (159, 160)] == [64, 256]
+    assert [rows(n, 4, 4096, 14336) for n in (223, 224)] == [64, 256]      # (40 rows each: 302 us and 365, 50: 444 and 373)
+    assert [rows(n, 32, 2048, 1024) for n in (1791, 1792)] == [64, 256]
+    lines = lambda E, H, F: next(n for n in range(1, 200) if ops.moe_sparse_tile_rows(n * E, E, H, F, True) == 256)      # noqa: E731
+    assert [lines(8, 4096, 14336), lines(4, 4096, 4096), lines(8, 1024, 4096)] == [56, 72, 150]      # rows 32 KB apart
     assert [rows(n, 2, 4096, 14336) for n in (191, 192)] == [64, 256]
     assert rows(10 ** 6, 8, 4096 + 128, 14336) == 128 and rows(10 ** 6, 8, 4096, 64) == 128
 
