@@ -1,4 +1,4 @@
-"""True-f32 products (three bf16 parts per value): plain GEMM, router logits and grouped experts against float64."""
+"""True-f32 products (f32 tiles, and three bf16 parts per value): plain GEMM, router logits and grouped experts against float64."""
 import pytest
 import torch
 
@@ -25,7 +25,7 @@ def test_gemm_matches_float64(M, N, K, pad):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("M,N,K", [(65, 66, 16), (65, 66, 32), (64, 64, 64), (70, 64, 96), (70, 64, 160), (2048, 1792, 64), (2048, 1792, 96),
-                                   (2048, 1792, 45)])      # one K step, few, and the 128 x 128 tile
+                                   (2048, 1792, 45), (70, 64, 192), (65, 130, 320), (2048, 1792, 192)])      # one K step, few, and the 128 x 128 tile
 def test_sums_that_bf16_parts_cannot_hold(M, N, K):
     g = torch.Generator().manual_seed(M + K)
     x, w = torch.randn(M, K, generator=g), torch.randn(N, K, generator=g)
@@ -45,7 +45,8 @@ def test_sums_that_bf16_parts_cannot_hold(M, N, K):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("M,N,K", [(65, 66, 20), (66, 64, 32), (70, 64, 96), (33, 130, 257), (2048, 1792, 64), (2048, 1792, 45)])
+@pytest.mark.parametrize("M,N,K", [(65, 66, 20), (66, 64, 32), (70, 64, 192), (33, 130, 257), (130, 70, 160), (2048, 1792, 160),
+                                   (2048, 1792, 45)])
 @pytest.mark.parametrize("small,large", [(-126, 100), (-124, 60), (-115, 60), (-120, 20), (-140, 0), (-135, 100), (-75, -70), (-60, -45)])
 def test_small_operands_of_large_ones(M, N, K, small, large):
     """Values whose last bits no bf16 part holds, denormal ones and products that underflow: as exact as sums in f32, alone, among
@@ -66,10 +67,10 @@ def test_small_operands_of_large_ones(M, N, K, small, large):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("N", [64, 70])
-@pytest.mark.parametrize("K,units", [(1, 1), (4, 3), (32, 3), (40, 3)])
+@pytest.mark.parametrize("K,units", [(1, 1), (4, 1), (32, 1), (128, 1), (200, 1), (160, 3), (256, 3)])
 def test_single_products(N, K, units):
-    """One channel that is not zero. Up to three channels: one rounding (2^-24). From four on, six products of parts leave out less
-    than 2^-24 of it, and the last addition cuts to 24 bits (2^-23)."""
+    """One channel that is not zero. On f32 tiles (up to four steps of 32 channels, or rows without whole steps): one rounding (2^-24). As
+    products of parts: less than 2^-24 of it is left out, and the last addition cuts to 24 bits (2^-23)."""
     g = torch.Generator().manual_seed(N)
     x, w = torch.zeros(4096, K), torch.zeros(N, K)
     x[:, K - 1], w[:, K - 1] = torch.randn(4096, generator=g), torch.randn(N, generator=g)
