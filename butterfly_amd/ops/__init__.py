@@ -679,7 +679,7 @@ def moe_sparse_ffn(x, topk_ids, topk_w, gu_w, down_w, e0: int, num_local: int, f
     count = _arena.get(dev, "moe_count", 1, torch.int32)[:1]
     L.moe_align(topk_ids, e0, num_local, rows, slot_of, tiles, count, bm, bcnt, bcap)
     hmid = _empty(TK, ffn, dtype=x.dtype, device=dev)
-    L.moe_grouped_gemm(x, gu_w, hmid, rows, tiles, count, 2 * ffn * H, 2 * ffn, H, num_local, EPILOGUES["silu"], bm)
+    L.moe_grouped_gemm(x, gu_w, hmid, rows, tiles, count, 2 * ffn * gu_w.stride(0), 2 * ffn, H, num_local, EPILOGUES["silu"], bm)
     out = _empty(T, H, dtype=x.dtype, device=dev)
     sk = moe_down_splits(exp, num_local, H, ffn, bm)
     if sk > 1:

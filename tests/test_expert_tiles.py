@@ -203,3 +203,23 @@ def test_grouped_rows_of_far_strides(gathered):
                                     ops.EPILOGUES["silu" if gathered else "none"], 256)
     # one rounding to bf16 (2^-9), f32 sums of 256 products beside it
     assert (out.float() - want).norm() < 2.0 ** -8 * want.norm()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T", [40, 1000])
+def test_sparse_experts_of_padded_rows(T):
+    """Gate/up and down rows further apart than they are wide, as models lay out rows of a multiple of 32 KB, on both tiles."""
+    E, K, H, F = 4, 2, 512, 256
+    g = torch.Generator().manual_seed(T)
+    bf = lambda *s, k=1.0: (k * torch.randn(*s, generator=g)).to(torch.bfloat16)            # noqa: E731
+    x, ids, w = bf(T, H), torch.rand(T, E, generator=g).topk(K, -1).indices, torch.rand(T, K, generator=g)
+    gu, dn = bf(E * 2 * F, H, k=H ** -0.5), bf(H, E * F, k=F ** -0.5)
+    d = [t.cuda() for t in (x, ids.int(), w)]
+    apart = lambda t: torch.zeros(t.shape[0], t.shape[1] + 64, dtype=t.dtype, device="cuda")[:, :t.shape[1]].copy_(t)      # noqa: E731
+    want = ops.moe_sparse_ffn(*d, gu.cuda(), dn.cuda(), 0, E, F)
+    ref = ops.reference.moe_sparse_ffn(x.float(), ids, w, gu.float(), dn.float(), 0, E, F)
+    # bf16 hidden rows, expert rows and output: 2^-9 each
+    assert (want.cpu().float() - ref).norm() < 2.0 ** -7 * ref.norm()
+    for a, b in ((apart(gu), dn.cuda()), (gu.cuda(), apart(dn)), (apart(gu), apart(dn))):
+        got = ops.moe_sparse_ffn(*d, a, b, 0, E, F)
+        assert (got.float() - want.float()).norm() < 2.0 ** -8 * want.float().norm()
