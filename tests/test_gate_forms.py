@@ -64,6 +64,28 @@ def test_one_launch_and_two(kind, dt, D, Dv, bad):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("bad", [float("nan"), float("inf")])
+@pytest.mark.parametrize("where", ["q", "k", "v", "z"])
+@pytest.mark.parametrize("row", [0, 7, 11, 16, 30])      # of a whole chunk and one of 15 rows: both blocks, the last row
+def test_values_that_are_no_numbers_in_one_launch(row, where, bad):
+    g = torch.Generator().manual_seed(row)
+    n, H, D, Dv = 31, 2, 32, 80
+    assert torch.ops.bfly.gla_scan_forms(n, 1, H, D, Dv, False, 0) == [0, 1, 0]
+    rnd = lambda *s: torch.randn(*s, generator=g).to(torch.bfloat16)            # noqa: E731
+    x = dict(q=rnd(n, H, D), k=rnd(n, H, D), v=rnd(n, H, Dv), z=2 + rnd(n, H * D), state=torch.randn(1, H, D, Dv, generator=g),
+             state_slots=torch.tensor([0], dtype=torch.int32), row_cu=torch.tensor([0, n], dtype=torch.int32),
+             positions=torch.arange(3, 3 + n).int())
+    x[where].view(n, H, -1)[row, 1, 5] = bad
+    got, ref = {k: t.cuda() for k, t in x.items()}, {k: t.clone() for k, t in x.items()}
+    o, w = (ops.gla_scan(**a, tau=16.0, q_scale=D ** -0.5) for a in (got, ref))
+    for a, b in ((o.cpu(), w), (got["state"].cpu(), ref["state"])):
+        ok = b.isfinite()
+        assert torch.equal(a.isfinite(), ok)
+        # f32 sums in another order, products of up to 16 decays; hardware exp / log
+        assert (a - b)[ok].abs().max() < 3e-5 * b[ok].abs().max()
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("kind", ["gla", "forget"])
 @pytest.mark.parametrize("far,ld", [("qkz", (1 << 21) + 8), ("v", 1 << 26)])
 def test_rows_far_apart(kind, far, ld):
