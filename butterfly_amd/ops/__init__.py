@@ -183,10 +183,11 @@ def reserve_workspace(device, max_tokens: int, max_n: int, max_k: int, max_batch
     ws = max(torch.ops.bfly.gemm_workspace_bound(int(max_tokens), n, k) for n, k in nk)
     _arena.get(device, "gemm", ws // 4 + 1, torch.float32, zero=True)
     if max_batch and max_ctx:
-        ns = max(torch.ops.bfly.attn_decode_splits(max_ctx, torch.ops.bfly.attn_decode_part_tokens(b, num_kv_heads, max_ctx))
-                 for b in range(1, max_batch + 1))
-        _arena.get(device, "attn_o", max_batch * num_kv_heads * ns * 16 * head_dim, torch.float32)
-        _arena.get(device, "attn_ml", max_batch * num_kv_heads * ns * 16 * 2, torch.float32)
+        # (a key / value head's query group has at most 16 rows)
+        rows = max(torch.ops.bfly.attn_decode_part_rows(b, 16 * num_kv_heads, num_kv_heads, max_ctx, 0)
+                   for b in range(1, max_batch + 1))
+        _arena.get(device, "attn_o", rows * head_dim, torch.float32)
+        _arena.get(device, "attn_ml", rows * 2, torch.float32)
     _arena.get(device, "sample", max(max_batch, max_tokens, 1) * 64, torch.int64)
     _arena.get(device, "tkp", max(max_batch, max_tokens, 1) * 521, torch.float32)
 
@@ -608,13 +609,11 @@ def attn_decode(q, k_cache, v_cache, block_tables, ctx_lens, scale: float, max_c
     Hkv = k_cache.shape[1]
     if out is None:
         out = _empty(B, Hq, D, dtype=q.dtype, device=q.device)
-    if part_tokens <= 0:
-        part_tokens = torch.ops.bfly.attn_decode_part_tokens(B, Hkv, max_ctx)
-    ns = torch.ops.bfly.attn_decode_splits(max_ctx, part_tokens)
+    rows = torch.ops.bfly.attn_decode_part_rows(B, Hq, Hkv, max_ctx, part_tokens)
     po = pml = None
-    if ns > 1:
-        po = _arena.get(q.device, "attn_o", B * Hkv * ns * 16 * D, torch.float32)
-        pml = _arena.get(q.device, "attn_ml", B * Hkv * ns * 16 * 2, torch.float32)
+    if rows > 0:
+        po = _arena.get(q.device, "attn_o", rows * D, torch.float32)
+        pml = _arena.get(q.device, "attn_ml", rows * 2, torch.float32)
     torch.ops.bfly.attn_decode(q, k_cache, v_cache, block_tables, ctx_lens, scale, max_ctx,
                                part_tokens, out, po, pml)
     return out

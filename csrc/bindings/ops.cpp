@@ -675,6 +675,10 @@ int64_t attn_decode_part_tokens(int64_t B, int64_t Hkv, int64_t max_ctx) {
   return bfly::attn_decode_part_tokens(B, Hkv, max_ctx);
 }
 
+int64_t attn_decode_part_rows(int64_t B, int64_t Hq, int64_t Hkv, int64_t max_ctx, int64_t part_tokens) {
+  return bfly::attn_decode_part_rows(B, Hq, Hkv, max_ctx, part_tokens);
+}
+
 void attn_decode(const Tensor& q, const Tensor& k_cache, const Tensor& v_cache,
                  const Tensor& block_tables, const Tensor& ctx_lens, double scale,
                  int64_t max_ctx, int64_t part_tokens, Tensor& out,
@@ -691,13 +695,12 @@ void attn_decode(const Tensor& q, const Tensor& k_cache, const Tensor& v_cache,
               "attn_decode: block_tables");
   TORCH_CHECK(ctx_lens.numel() >= B, "attn_decode: ctx_lens");
   TORCH_CHECK((long)block_tables.size(1) * BS >= max_ctx, "attn_decode: block table too narrow for max_ctx");
-  if (part_tokens <= 0) part_tokens = bfly::attn_decode_part_tokens(B, Hkv, max_ctx);
-  const int nsplit = bfly::attn_decode_splits(max_ctx, part_tokens);
+  const long rows = bfly::attn_decode_part_rows(B, Hq, Hkv, max_ctx, part_tokens);
   float *po = nullptr, *pml = nullptr;
-  if (nsplit > 1) {
+  if (rows > 0) {
     TORCH_CHECK(part_o.has_value() && part_ml.has_value(), "attn_decode: partial buffers required");
-    TORCH_CHECK(part_o->numel() >= (long)B * Hkv * nsplit * 16 * D, "attn_decode: part_o too small");
-    TORCH_CHECK(part_ml->numel() >= (long)B * Hkv * nsplit * 16 * 2, "attn_decode: part_ml too small");
+    TORCH_CHECK(part_o->numel() >= rows * D, "attn_decode: part_o too small");
+    TORCH_CHECK(part_ml->numel() >= rows * 2, "attn_decode: part_ml too small");
     po = part_o->data_ptr<float>();
     pml = part_ml->data_ptr<float>();
   }
@@ -1218,6 +1221,7 @@ TORCH_LIBRARY(bfly, m) {
         [](int64_t M, int64_t N, int64_t K, int64_t e) -> int64_t { return bfly::gemm_check(M, N, K, e); });
   m.def("attn_decode_splits(int max_ctx, int part_tokens) -> int", &attn_decode_splits);
   m.def("attn_decode_part_tokens(int B, int Hkv, int max_ctx) -> int", &attn_decode_part_tokens);
+  m.def("attn_decode_part_rows(int B, int Hq, int Hkv, int max_ctx, int part_tokens) -> int", &attn_decode_part_rows);
   m.def("attn_decode(Tensor q, Tensor k_cache, Tensor v_cache, Tensor block_tables, Tensor ctx_lens, "
         "float scale, int max_ctx, int part_tokens, Tensor(a!) out, Tensor(b!)? part_o, "
         "Tensor(c!)? part_ml) -> ()");

@@ -21,6 +21,8 @@
 // read by ds_read_b128 as the 32x32x16 A operand of S^T = K . Q^T, V by ds_read_b64_tr_b16 as
 // the A operand of O^T = V^T . P^T; the S^T accumulator is converted in registers into the
 // P^T B operand (§3 "An accumulator tile as the next MFMA's operand").
+#include <limits.h>
+
 #include <algorithm>
 #include <type_traits>
 
@@ -36,10 +38,59 @@ typedef __attribute__((address_space(3))) s16x4* lds_s4_ptr;
 
 constexpr int kAttnThreads = 256;
 constexpr float kNegInf = -INFINITY;
+constexpr int kFlatMaxBatch = 256;        // sequences whose places fit in four registers a lane
 
 // ---------------------------------------------------------------------------------------
 // Decode
 // ---------------------------------------------------------------------------------------
+// One page of one wave: its scores against the query group, the running softmax and the products with its values. `end`: keys
+// of the context (or of the split).
+// CLEAR: with a first maximum o starts from zero, whatever it holds.
+template <int BS, typename CT, bool CLEAR = false>
+__device__ __forceinline__ void decode_page(int p, int end, int g, float scale_log2, const bf16x8 (&qf)[4],
+                                            const typename KV<CT>::raw_t (&kf)[2][4], const typename KV<CT>::raw_t (&vf)[8],
+                                            f32x4 (&o)[8], float& m, float& l) {
+  f32x4 st[2];
+#pragma unroll
+  for (int kt = 0; kt < 2; ++kt) {
+    st[kt] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int ds = 0; ds < 4; ++ds) st[kt] = mfma16(KV<CT>::widen(kf[kt][ds]), qf[ds], st[kt]);
+  }
+  // st[kt][i] = S[key = p*BS + 8g + 4kt + i][query r]; only the context's last page has keys past its end
+  float x[8];
+  float tmax = kNegInf;
+  if ((p + 1) * BS <= end) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) x[j] = st[j >> 2][j & 3] * scale_log2;
+  } else {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) x[j] = p * BS + 8 * g + j < end ? st[j >> 2][j & 3] * scale_log2 : kNegInf;
+  }
+#pragma unroll
+  for (int j = 0; j < 8; ++j) tmax = fmaxf(tmax, x[j]);
+  tmax = row4_max(tmax);
+  if (__any(tmax > m)) {      // a larger maximum in some row: rescale (elsewhere the factor is 1)
+    const float mn = fmaxf(m, tmax);
+    const float alpha = __builtin_amdgcn_exp2f(m - (mn == kNegInf ? 0.f : mn));
+    const bool first = CLEAR && m == kNegInf;
+    m = mn;
+    l *= alpha;
+#pragma unroll
+    for (int dt = 0; dt < 8; ++dt) o[dt] = first ? f32x4{0.f, 0.f, 0.f, 0.f} : o[dt] * alpha;
+  }
+  const float mb = m == kNegInf ? 0.f : m;
+  bf16x8 pb;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    const float pv = __builtin_amdgcn_exp2f(x[j] - mb);
+    l += pv;
+    pb[j] = f2bf(pv);
+  }
+#pragma unroll
+  for (int dt = 0; dt < 8; ++dt) o[dt] = mfma16(KV<CT>::widen(vf[dt]), pb, o[dt]);
+}
+
 template <int D, int BS, typename CT, int NW>
 __global__ void __launch_bounds__(64 * NW)
 attn_decode_kernel(const bf16* __restrict__ q, long q_stride, const CT* __restrict__ k_cache,
@@ -124,44 +175,7 @@ attn_decode_kernel(const bf16* __restrict__ q, long q_stride, const CT* __restri
       vf[dt] = KV<CT>::ld(vb + (16 * dt + r) * BS + 8 * g);
   };
   auto compute_page = [&](int p, const raw_t (&kf)[2][4], const raw_t (&vf)[8]) {
-    f32x4 st[2];
-#pragma unroll
-    for (int kt = 0; kt < 2; ++kt) {
-      st[kt] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int ds = 0; ds < 4; ++ds) st[kt] = mfma16(KV<CT>::widen(kf[kt][ds]), qf[ds], st[kt]);
-    }
-    // st[kt][i] = S[key = p*BS + 8g + 4kt + i][query r]; only the context's last page has keys past its end
-    float x[8];
-    float tmax = kNegInf;
-    if ((p + 1) * BS <= tok1) {
-#pragma unroll
-      for (int j = 0; j < 8; ++j) x[j] = st[j >> 2][j & 3] * scale_log2;
-    } else {
-#pragma unroll
-      for (int j = 0; j < 8; ++j) x[j] = p * BS + 8 * g + j < tok1 ? st[j >> 2][j & 3] * scale_log2 : kNegInf;
-    }
-#pragma unroll
-    for (int j = 0; j < 8; ++j) tmax = fmaxf(tmax, x[j]);
-    tmax = row4_max(tmax);
-    if (__any(tmax > m)) {      // a larger maximum in some row: rescale (elsewhere the factor is 1)
-      const float mn = fmaxf(m, tmax);
-      const float alpha = __builtin_amdgcn_exp2f(m - (mn == kNegInf ? 0.f : mn));
-      m = mn;
-      l *= alpha;
-#pragma unroll
-      for (int dt = 0; dt < 8; ++dt) o[dt] *= alpha;
-    }
-    const float mb = m == kNegInf ? 0.f : m;
-    bf16x8 pb;
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const float pv = __builtin_amdgcn_exp2f(x[j] - mb);
-      l += pv;
-      pb[j] = f2bf(pv);
-    }
-#pragma unroll
-    for (int dt = 0; dt < 8; ++dt) o[dt] = mfma16(KV<CT>::widen(vf[dt]), pb, o[dt]);
+    decode_page<BS, CT>(p, tok1, g, scale_log2, qf, kf, vf, o, m, l);
   };
 
   // software pipeline over this wave's pages (p0 + wid, +NW, ...): the next page's K/V loads
@@ -237,6 +251,347 @@ attn_decode_kernel(const bf16* __restrict__ q, long q_stride, const CT* __restri
       }
     }
   }
+}
+
+// pages of a context (a length outside of [0, max_ctx] counts as the nearer end)
+template <int BS>
+__device__ __forceinline__ int ctx_pages(int ctx, int max_ctx) {
+  return (min(max(ctx, 0), max_ctx) + BS - 1) / BS;
+}
+// pages that the time of a segment's end is worth (elements of `es` bytes)
+__host__ __device__ constexpr int flat_extra(int es) { return 8 / es; }
+// inclusive sum over the lanes up to this one
+__device__ __forceinline__ int wave_scan(int x) {
+  x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xF, 0xF, false);     // row_shr 1, 2, 4, 8
+  x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xF, 0xF, false);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xF, 0xF, false);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xF, 0xF, false);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xA, 0xF, false);     // row_bcast 15, 31
+  return x + __builtin_amdgcn_update_dpp(0, x, 0x143, 0xC, 0xF, false);
+}
+// pages per workgroup when the P pages of a step are cut into (at most) N equal pieces; one page per wave at least
+__device__ __forceinline__ int flat_chunk(int P, int N, int NW) { return max((P + N - 1) / N, NW); }
+
+// Decode over the step's pages laid end to end: per kv head the pages of all sequences form one list, workgroup i of N takes
+// the i-th of N equal pieces, whatever sequences it covers. With one split per sequence (above) the longest context sets the time,
+// rows that only pad the batch hold workgroups of their own, and the bound `max_ctx` rather than the contexts sets the splits.
+// A piece's parts of sequences ("segments") follow each other in one software pipeline: a wave asks for the first pages of the
+// next segment before the last ones of this one are computed, page ids one page ahead of that, and the queries of the next QS
+// segments wait in LDS. A segment costs a barrier and a sum over the waves, so each sequence counts as flat_extra pages more than
+// it has. A segment that holds its whole sequence is written out, the others leave (sum, maximum, weights) at slot i + b of the
+// head, which attn_decode_flat_combine_kernel adds up. The sequences' places in the list are in lanes (R registers, B <= 64 R).
+template <int D, int BS, typename CT, int NW, int R, int QS>
+__global__ void __launch_bounds__(64 * NW)
+attn_decode_flat_kernel(const bf16* __restrict__ q, long q_stride, const CT* __restrict__ k_cache,
+                        const CT* __restrict__ v_cache, const int* __restrict__ block_tables, int bt_stride,
+                        const int* __restrict__ ctx_lens, int B, int max_ctx, int Hq, int Hkv, float scale_log2,
+                        bf16* __restrict__ out, float* __restrict__ part_o, float* __restrict__ part_ml) {
+  static_assert(D == 128 && BS == 32, "decode kernel is specialised for D=128, BS=32");
+  const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int ci = blockIdx.x, N = gridDim.x, h = blockIdx.y;
+  const int G = Hq / Hkv;
+  extern __shared__ __attribute__((aligned(16))) float dec_smem[];
+  constexpr int LD = D + 4;                    // (four floats more: rows start in different banks)
+  const int stage = NW * (LD * G + 32);        // [NW][G][LD], [NW][16] maxima, [NW][16] sums; two of them
+  bf16* s_q = reinterpret_cast<bf16*>(dec_smem + 2 * stage);      // [QS][G][D]
+
+  // lane j of set i: keys, first position and the position behind the last page of sequence 64 i + j
+  // (R > 1: then in LDS, where every wave writes the same)
+  int vctx[R], vbeg[R], vend[R], P = 0;
+  int* s_tab = reinterpret_cast<int*>(s_q + QS * G * D);          // [3][64 R]
+  unsigned long long some[R];                  // sequences that are not empty
+#pragma unroll
+  for (int i = 0; i < R; ++i) vctx[i] = 64 * i + lane < B ? min(ctx_lens[64 * i + lane], max_ctx) : 0;
+#pragma unroll
+  for (int i = 0; i < R; ++i) {
+    const int n = ctx_pages<BS>(vctx[i], max_ctx), w = n > 0 ? n + flat_extra(sizeof(CT)) : 0, x = wave_scan(w);
+    vbeg[i] = P + x - w;
+    vend[i] = vbeg[i] + n;
+    some[i] = __ballot(n > 0);
+    P += __builtin_amdgcn_readlane(x, 63);
+    if constexpr (R > 1) {
+      s_tab[64 * i + lane] = vctx[i];
+      s_tab[64 * (R + i) + lane] = vbeg[i];
+      s_tab[64 * (2 * R + i) + lane] = vend[i];
+    }
+  }
+  const int c = flat_chunk(P, N, NW), a = ci * c, e = min(P, a + c);
+  if (a >= e) return;
+  auto get = [&](int which, const int (&v)[R], int i) {
+    if constexpr (R > 1) return __builtin_amdgcn_readfirstlane(s_tab[64 * R * which + i]);
+    else return __builtin_amdgcn_readlane(v[0], i);
+  };
+  // the first sequence behind number i that is not empty; B or more: none
+  auto after = [&](int i) {
+    int k = 64 * R;
+#pragma unroll
+    for (int j = R - 1; j >= 0; --j) {
+      const unsigned long long rest = i < 64 * j ? some[j] : i < 64 * j + 63 ? some[j] >> (i - 64 * j + 1) << (i - 64 * j + 1) : 0;
+      if (rest) k = 64 * j + __builtin_ctzll(rest);
+    }
+    return k;
+  };
+  // bounds of sequence i in the list (end = INT_MAX: not of this piece)
+  auto bounds = [&](int i, int& beg, int& end) {
+    beg = i < B ? get(1, vbeg, i) : INT_MAX;
+    end = beg < e ? get(2, vend, i) : INT_MAX;
+  };
+  int k = 64 * R, sbeg, send;                  // the segment being computed: the first one that ends behind a
+#pragma unroll
+  for (int i = R - 1; i >= 0; --i) {
+    const unsigned long long in = __ballot(vend[i] > a) & some[i];
+    if (in) k = 64 * i + __builtin_ctzll(in);
+  }
+  bounds(k, sbeg, send);
+  if (send == INT_MAX) return;
+
+  const int g = lane >> 4, r = lane & 15;
+  constexpr bool kF8 = sizeof(CT) == 1;
+  auto d_off = [&](int ds) { return kF8 ? 64 * (ds >> 1) + 16 * g + 8 * (ds & 1) : 32 * ds + 8 * g; };
+  // segment j's queries are in LDS slot j % QS (a sequence's rows of this head are contiguous)
+  int kq = k, nq = 0, js = 0;                   // the next sequence whose queries go there, and its number; number of segment k
+  auto q_ok = [&] { return kq < B && get(1, vbeg, kq) < e; };
+  {
+    bf16x8 t[QS];
+    int n = 0;
+#pragma unroll
+    for (int j = 0; j < QS; ++j)
+      if (q_ok()) {
+        if ((int)threadIdx.x < G * D / 8) t[j] = *reinterpret_cast<const bf16x8*>(q + (long)kq * q_stride + (long)h * G * D + 8 * threadIdx.x);
+        kq = after(kq);
+        ++n;
+      }
+#pragma unroll
+    for (int j = 0; j < QS; ++j)
+      if (j < n && (int)threadIdx.x < G * D / 8) *reinterpret_cast<bf16x8*>(s_q + (j * G * D + 8 * threadIdx.x)) = t[j];
+    nq = n;
+  }
+  bf16x8 qf[4];
+  auto load_q = [&](int j) {
+    const bf16* p = s_q + ((j & (QS - 1)) * G + (r < G ? r : 0)) * D;
+#pragma unroll
+    for (int ds = 0; ds < 4; ++ds) {
+      qf[ds] = *reinterpret_cast<const bf16x8*>(p + d_off(ds));
+      if (r >= G) qf[ds] = bf16x8{};
+    }
+  };
+
+  // this wave's pages: positions a + wid, + NW, ... without the ones that only stand for a sequence's cost. lf: the next one to be
+  // asked for, lblk its page id (itself asked for a page ahead)
+  typedef typename KV<CT>::raw_t raw_t;
+  int lk = k, lbeg = sbeg, lend = send, lf = a + wid, lblk = 0;
+  auto seek = [&] {                            // the first such position at or behind lf
+    if (lf < lbeg) lf += (lbeg - lf + NW - 1) / NW * NW;
+    while (lf >= lend) {                       // (INT_MAX: no more)
+      lk = after(lk);
+      bounds(lk, lbeg, lend);
+      if (lend == INT_MAX) {
+        lf = INT_MAX;
+        return;
+      }
+      if (lf < lbeg) lf += (lbeg - lf + NW - 1) / NW * NW;
+    }
+    if (lf < e) lblk = block_tables[(long)lk * bt_stride + (lf - lbeg)];
+  };
+  seek();
+  auto take = [&](int& f, raw_t (&kf)[2][4], raw_t (&vf)[8]) {
+    f = lf;
+    if (lf >= e) return;
+    const CT* kb = k_cache + (((long)lblk * Hkv + h) * BS) * D;
+    const CT* vb = v_cache + ((long)lblk * Hkv + h) * (long)D * BS;
+#pragma unroll
+    for (int kt = 0; kt < 2; ++kt) {
+      const int key = 8 * (r >> 2) + 4 * kt + (r & 3);
+#pragma unroll
+      for (int ds = 0; ds < 4; ++ds)
+        if constexpr (kF8) {
+          if (ds & 1) continue;
+          const u32x4 w = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(kb + key * D + d_off(ds)));
+          kf[kt][ds] = raw_t{w[0], w[1]};
+          kf[kt][ds + 1] = raw_t{w[2], w[3]};
+        } else {
+          kf[kt][ds] = KV<CT>::ld(kb + key * D + d_off(ds));
+        }
+    }
+#pragma unroll
+    for (int dt = 0; dt < 8; ++dt) vf[dt] = KV<CT>::ld(vb + (16 * dt + r) * BS + 8 * g);
+    lf += NW;
+    seek();
+  };
+  // (the sums of a segment are not cleared for the next one: its first maximum above -inf replaces them)
+  f32x4 o[8];
+#pragma unroll
+  for (int dt = 0; dt < 8; ++dt) o[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float m = kNegInf, l = 0.f;
+  int ctx = get(0, vctx, k), buf = 0;
+  // the segment's sums over the waves: its part, or its rows of `out`
+  auto flush = [&] {
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));               // (addresses formed here, not held through the loop over the pages)
+    const int g = (tid & 63) >> 4, r = tid & 15;
+    const float ls = row4_sum(l);
+    float* s_o = dec_smem + buf * stage;
+    float(*s_m)[16] = reinterpret_cast<float(*)[16]>(s_o + NW * LD * G);
+    float(*s_l)[16] = s_m + NW;
+    if (r < G) {
+#pragma unroll
+      for (int dt = 0; dt < 8; ++dt) *reinterpret_cast<f32x4*>(s_o + (wid * G + r) * LD + 16 * dt + 4 * g) = o[dt];
+      if (g == 0) {
+        s_m[wid][r] = m;
+        s_l[wid][r] = ls;
+      }
+    }
+    const int b = k;
+    const bool whole = sbeg >= a && send <= e;
+    m = kNegInf;
+    l = 0.f;
+    k = after(k);
+    bounds(k, sbeg, send);
+    ++js;
+    __syncthreads();
+    if (send != INT_MAX) {
+      load_q(js);
+      ctx = get(0, vctx, k);
+      if (q_ok()) {                             // into the slot of the queries just done with
+        if (tid < G * D / 8)
+          *reinterpret_cast<bf16x8*>(s_q + ((nq & (QS - 1)) * G * D + 8 * tid)) =
+              *reinterpret_cast<const bf16x8*>(q + (long)kq * q_stride + (long)h * G * D + 8 * tid);
+        kq = after(kq);
+        ++nq;
+      }
+    }
+    const long slot = (long)h * (N + B) + ci + b;
+    for (int t = tid; t < G * D; t += 64 * NW) {
+      const int qr = t / D, d = t % D;
+      float M = kNegInf;
+#pragma unroll
+      for (int w = 0; w < NW; ++w) M = fmaxf(M, s_m[w][qr]);
+      const float Mb = M == kNegInf ? 0.f : M;
+      float L = 0.f, O = 0.f;
+      const float* po = s_o + qr * LD + d;
+#pragma unroll
+      for (int w = 0; w < NW; ++w) {
+        const float x = exp2f(s_m[w][qr] - Mb), y = po[w * G * LD];
+        L += x != 0.f ? x * s_l[w][qr] : 0.f;   // (0: no page, what it holds is an older segment's)
+        O += x != 0.f ? x * y : 0.f;
+      }
+      if (whole) {
+        out[((long)b * Hq + h * G + qr) * D + d] = f2bf(L > 0.f ? O / L : 0.f);
+      } else {
+        part_o[(slot * G + qr) * D + d] = O;
+        if (d == 0) {
+          part_ml[(slot * G + qr) * 2 + 0] = M;
+          part_ml[(slot * G + qr) * 2 + 1] = L;
+        }
+      }
+    }
+    buf ^= 1;                                   // (the buffer after next is written behind the next barrier)
+  };
+  // every wave flushes every segment, in order, also those in which it has no page
+  auto compute = [&](int f, const raw_t (&kf)[2][4], const raw_t (&vf)[8]) {
+    while (f >= send) flush();
+    decode_page<BS, CT, true>(f - sbeg, ctx, g, scale_log2, qf, kf, vf, o, m, l);
+  };
+
+  raw_t kA[2][4], vA[8], kB[2][4], vB[8];
+  int fA, fB;
+  take(fA, kA, vA);
+  __syncthreads();                              // queries
+  load_q(0);
+  if constexpr (!kF8) {
+    while (fA < e) {
+      take(fB, kB, vB);
+      compute(fA, kA, vA);
+      if (fB >= e) break;
+      take(fA, kA, vA);
+      compute(fB, kB, vB);
+    }
+  } else {
+    // FP8 pages are half the bytes: two of them in flight
+    raw_t kC[2][4], vC[8];
+    int fC;
+    take(fB, kB, vB);
+    while (fA < e) {
+      take(fC, kC, vC);
+      compute(fA, kA, vA);
+      if (fB >= e) break;
+      take(fA, kA, vA);
+      compute(fB, kB, vB);
+      if (fC >= e) break;
+      take(fB, kB, vB);
+      compute(fC, kC, vC);
+    }
+  }
+  while (send != INT_MAX) flush();
+}
+
+// The segments of the sequences that attn_decode_flat_kernel cut, added up: workgroup = (kv head, sequence), 32 threads per query
+// row with four columns each
+template <int D, int BS>
+__global__ void __launch_bounds__(512)
+attn_decode_flat_combine_kernel(const float* __restrict__ part_o, const float* __restrict__ part_ml,
+                                const int* __restrict__ ctx_lens, int B, int max_ctx, int extra, int N, int NW, int Hq,
+                                int Hkv, bf16* __restrict__ out) {
+  static_assert(D == 128, "32 threads per row");
+  const int h = blockIdx.x, b = blockIdx.y, G = Hq / Hkv;
+  const int qr = threadIdx.x >> 5, lane = threadIdx.x & 31;
+  int P = 0, beg = 0;
+  for (int b0 = lane; b0 < B; b0 += 32) {
+    const int n = ctx_pages<BS>(ctx_lens[b0], max_ctx), w = n > 0 ? n + extra : 0;
+    P += w;
+    beg += b0 < b ? w : 0;
+  }
+  auto all = [&](auto x, auto f) {
+#pragma unroll
+    for (int o = 16; o > 0; o >>= 1) x = f(x, __shfl_xor(x, o, 32));
+    return x;
+  };
+  auto add = [](auto x, auto y) { return x + y; };
+  P = all(P, add);
+  beg = all(beg, add);
+  const int n = ctx_pages<BS>(ctx_lens[b], max_ctx), c = flat_chunk(P, N, NW);
+  bf16* to = out + ((long)b * Hq + h * G + qr) * D + 4 * lane;
+  auto store = [&](bf16x4 y) {
+    if (reinterpret_cast<uintptr_t>(out) % 8 == 0) *reinterpret_cast<bf16x4*>(to) = y;
+    else
+      for (int i = 0; i < 4; ++i) to[i] = y[i];
+  };
+  if (n == 0) {
+    store(bf16x4{});
+    return;
+  }
+  const int i0 = beg / c, ns = (beg + n - 1) / c - i0 + 1;
+  if (ns == 1) return;                          // written by its workgroup
+  const long base = (long)h * (N + B) + i0 + b;
+  auto ml = [&](int s) { return *reinterpret_cast<const float2*>(part_ml + ((base + s) * G + qr) * 2); };
+  float M = kNegInf, L = 0.f;
+  for (int s = lane; s < ns; s += 32) M = fmaxf(M, ml(s).x);
+  M = all(M, [](float x, float y) { return fmaxf(x, y); });
+  const float Mb = M == kNegInf ? 0.f : M;
+  f32x4 O = {0.f, 0.f, 0.f, 0.f};
+  const float* po = part_o + (base * G + qr) * D + 4 * lane;
+  for (int s0 = 0; s0 < ns; s0 += 32) {
+    float w = 0.f;
+    if (s0 + lane < ns) {
+      const float2 x = ml(s0 + lane);
+      w = exp2f(x.x - Mb);
+      L += w * x.y;
+    }
+    const int cnt = min(32, ns - s0);
+#pragma unroll 4
+    for (int s = 0; s < cnt; ++s) {
+      const float ws = __shfl(w, s, 32);
+      const f32x4 x = *reinterpret_cast<const f32x4*>(po + (long)(s0 + s) * G * D);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) O[i] += ws != 0.f ? ws * x[i] : 0.f;
+    }
+  }
+  L = all(L, add);
+  const float inv = L > 0.f ? 1.f / L : 0.f;
+  bf16x4 y;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) y[i] = f2bf(O[i] * inv);
+  store(y);
 }
 
 // One workgroup per (query row, kv head, sequence); thread = head dim element. The split
@@ -731,12 +1086,63 @@ int attn_decode_part_tokens(int B, int Hkv, int max_ctx) {
   return part;
 }
 
+// Workgroups per kv head of the form over all pages end to end (attn_decode_flat_kernel; 0: a workgroup per sequence and split), one
+// per compute unit in all. 32 heads on 8, us of a workgroup per split -> end to end, contexts of 0.3 to 1 of the bound / all at the
+// bound: bf16, 32 sequences of up to 8192 147 -> 114 / 174 -> 169, 48 of 4096 115 -> 87 / 153 -> 132, 16 of 2048 25 -> 23 / 28 -> 30,
+// 128 of 2048 136 -> 124 / 169 -> 173; FP8, 24 of 8192 in a batch of 32 73 -> 52, 96 of 4096 132 -> 95; one head of 8, 96 of 8192
+// 66 -> 54. Its start (lengths, their sum, then pages) and its second launch take 3 us more, so small steps keep the other form:
+// 32 of up to 1024 22 and 25, 8 of 4096 27 and 29, 64 of 1024 39 and 39. Under a far bound, many sequences of 60 tokens take longer
+// too, as several share a workgroup (48 under 4096 6 -> 11).
+static int attn_decode_flat_pieces(int B, int Hkv, int max_ctx) {
+  if (B > kFlatMaxBatch || max_ctx < 1536 || (long)B * Hkv * max_ctx < 1L << 18) return 0;
+  return std::max(1, 256 / Hkv);
+}
+
+long attn_decode_part_rows(int B, int Hq, int Hkv, int max_ctx, int part_tokens) {
+  if (B <= 0 || Hkv <= 0) return 0;
+  const int n = part_tokens > 0 ? 0 : attn_decode_flat_pieces(B, Hkv, max_ctx);
+  if (n > 0) return (long)(n + B) * Hq;
+  const int ns = attn_decode_splits(max_ctx, part_tokens > 0 ? part_tokens : attn_decode_part_tokens(B, Hkv, max_ctx));
+  return ns > 1 ? (long)B * Hkv * ns * 16 : 0;
+}
+
 int launch_attn_decode(const bf16* q, long q_stride, const void* k_cache, const void* v_cache,
                        const int* block_tables, int bt_stride, const int* ctx_lens, int B, int Hq,
                        int Hkv, int D, int block_size, float scale, int max_ctx, int part_tokens,
                        bf16* out, float* part_o, float* part_ml, hipStream_t stream, int kv_fp8) {
   if (B <= 0) return 0;
   if (D != 128 || block_size != 32 || Hq % Hkv != 0 || Hq / Hkv > 16) return -1;
+  const int pieces = part_tokens > 0 ? 0 : attn_decode_flat_pieces(B, Hkv, max_ctx);
+  if (pieces > 0) {
+    if (part_o == nullptr || part_ml == nullptr) return -3;
+    const float sl2 = scale * 1.4426950408889634f;
+    const int G = Hq / Hkv;
+    constexpr int NW = 8, QS = 4;
+    const size_t lds = (size_t)2 * NW * (132 * G + 32) * sizeof(float) + QS * G * 256 + (B <= 64 ? 0 : 3 * 256 * sizeof(int));
+#define FLAT_LAUNCH(CT, R)                                                                                               \
+  {                                                                                                                      \
+    static bool once = false;                                                                                            \
+    if (!once) {                                                                                                         \
+      (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_decode_flat_kernel<128, 32, CT, NW, R, QS>),         \
+                                hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);                                 \
+      once = true;                                                                                                       \
+    }                                                                                                                    \
+    attn_decode_flat_kernel<128, 32, CT, NW, R, QS><<<dim3(pieces, Hkv), 64 * NW, lds, stream>>>(                        \
+        q, q_stride, static_cast<const CT*>(k_cache), static_cast<const CT*>(v_cache), block_tables, bt_stride, ctx_lens, \
+        B, max_ctx, Hq, Hkv, sl2, out, part_o, part_ml);                                                                 \
+  }
+    if (kv_fp8) {
+      if (B <= 64) FLAT_LAUNCH(fp8_t, 1)
+      else FLAT_LAUNCH(fp8_t, 4)
+    } else {
+      if (B <= 64) FLAT_LAUNCH(bf16, 1)
+      else FLAT_LAUNCH(bf16, 4)
+    }
+    attn_decode_flat_combine_kernel<128, 32><<<dim3(Hkv, B), 32 * G, 0, stream>>>(part_o, part_ml, ctx_lens, B, max_ctx,
+                                                                                 flat_extra(kv_fp8 ? 1 : 2), pieces, NW, Hq, Hkv, out);
+#undef FLAT_LAUNCH
+    return 0;
+  }
   if (part_tokens <= 0) part_tokens = attn_decode_part_tokens(B, Hkv, max_ctx);
   if (part_tokens % block_size != 0) return -2;
   if (attn_decode_splits(max_ctx, part_tokens) > 256) return -4;

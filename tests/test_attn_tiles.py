@@ -226,6 +226,53 @@ def test_decode_waves_and_splits(fp8, Hq, Hkv, ctx, max_ctx):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("Hq,Hkv,ctx,max_ctx", [
+    (8, 8, [0, 1, 0, 31, 32, 33, 4096, 0], 4096),              # empty sequences, one of many pieces
+    (32, 8, [2047, 5, 5, 5, 5, 5, 5, 5, 5, 5, 5, 2048, 700, 1, 256, 257], 2048),     # more segments in a piece than wait in LDS
+    (16, 1, [3000], 1 << 18),                                   # sixteen query heads on one, a single sequence far below its bound
+    (16, 8, [30 + 11 * i for i in range(64)], 1536),            # the most sequences of one register
+    (4, 4, [1 + 23 * i % 1500 for i in range(65)], 1536),       # one more than that
+    (4, 4, [0] * 200 + [1600] + [0] * 54 + [9], 2048),          # the most there are
+    (24, 3, [0] * 90, 1536),                                    # nothing at all
+])
+def test_decode_pages_end_to_end(fp8, Hq, Hkv, ctx, max_ctx):
+    g = torch.Generator().manual_seed(Hq + len(ctx))
+    D, B, scale = 128, len(ctx), 1.5 / math.sqrt(128)
+    assert torch.ops.bfly.attn_decode_part_rows(B, Hq, Hkv, max_ctx, 0) == (256 // Hkv + B) * Hq
+    dt = torch.float8_e4m3fn if fp8 else torch.bfloat16
+    need = [(c + BS - 1) // BS for c in ctx]
+    n = sum(need)
+    kc, vc = torch.randn(n + 1, Hkv, BS, D, generator=g).to(dt), torch.randn(n + 1, Hkv, D, BS, generator=g).to(dt)
+    q = torch.randn(B, Hq, D, generator=g).bfloat16()
+    tables = torch.full((B, (max_ctx + BS - 1) // BS), n, dtype=torch.int32)
+    order, at, want = torch.randperm(n, generator=g), 0, []
+    for b, c in enumerate(ctx):
+        pages = order[at:at + need[b]]
+        at += need[b]
+        tables[b, :need[b]] = pages.int()
+        if not c:
+            want.append(torch.zeros(1, Hq, D, dtype=F64))
+            continue
+        k = kc.float()[pages].transpose(1, 2).reshape(-1, Hkv, D)[:c].to(F64)
+        v = vc.float()[pages].permute(0, 3, 1, 2).reshape(-1, Hkv, D)[:c].to(F64)
+        want.append(dense(q[b:b + 1].to(F64), k, v, torch.tensor([c - 1]), scale, 1 << 30, 0, None, None, 0, None))
+    run = lambda vv: ops.attn_decode(q.cuda(), kc.cuda(), vv.cuda(), tables.cuda(), torch.tensor(ctx, dtype=torch.int32).cuda(),  # noqa: E731
+                                     scale, max_ctx)
+    got = run(vc)
+    err = (got.cpu().to(F64) - torch.cat(want)).abs().max()
+    assert err < 2.0 ** -8 * vc.float().abs().max() + 1e-3      # weights and output rounded to bf16
+    if n > 1 and not fp8:                                       # values that are no numbers stay in their sequence
+        longest = max(range(B), key=lambda b: ctx[b])
+        bad = vc.clone()
+        bad[tables[longest, 0].item()] = float("nan")
+        poisoned = run(bad)
+        assert poisoned[longest].isnan().all()
+        rest = [b for b in range(B) if b != longest]
+        assert torch.equal(poisoned[rest], got[rest])
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("bad", [float("nan"), float("inf")])
 @pytest.mark.parametrize("H,G,D,Dv,window,keep,start,n", [
     (8, 2, 128, 128, 1 << 30, 0, 0, 40),      # one tile, the last page partly used
