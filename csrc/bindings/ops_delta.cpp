@@ -156,19 +156,27 @@ void delta_scan(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor&
               "delta_scan: state [slots, H, Dv, D]");
   check_step(state_slots, row_cu, positions, T, state.size(0), "delta_scan");
   TORCH_CHECK(o.dim() == 3 && o.size(0) == T && o.size(1) == H && o.size(2) == Dv, "delta_scan: o");
+  const long n = bfly::delta_record_floats(T, state_slots.numel(), (int)H, (int)G, (int)D, (int)Dv, v.stride(0), (int)max_rows);
+  Tensor rec;
+  if (n > 0) rec = at::empty({n}, state.options());
   const int rc = bfly::launch_delta_scan(q.data_ptr<float>(), q.stride(0), k.data_ptr<float>(), k.stride(0),
                                          v.data_ptr<float>(), v.stride(0), b.data_ptr(), b.stride(0), a.data_ptr(),
                                          a.stride(0), a_log.data_ptr<float>(), dt_bias.data_ptr<float>(),
                                          state.data_ptr<float>(), state_slots.data_ptr<int>(), row_cu.data_ptr<int>(),
                                          (int)state_slots.numel(), positions.data_ptr<int>(), (float)q_scale,
-                                         (float)unit_eps, o.data_ptr<float>(), (int)T, (int)H, (int)G, (int)D, (int)Dv,
-                                         is_f32(b), cur_stream(), (int)max_rows);
+                                         (float)unit_eps, o.data_ptr<float>(), n > 0 ? rec.data_ptr<float>() : nullptr, (int)T,
+                                         (int)H, (int)G, (int)D, (int)Dv, is_f32(b), cur_stream(), (int)max_rows);
   TORCH_CHECK(rc == 0, "delta_scan: key size ", D, " not supported (<= 256)");
+}
+
+int64_t delta_record_floats(int64_t T, int64_t nseq, int64_t H, int64_t G, int64_t D, int64_t Dv, int64_t v_ld, int64_t max_rows) {
+  return bfly::delta_record_floats(T, nseq, (int)H, (int)G, (int)D, (int)Dv, v_ld, (int)max_rows);
 }
 
 }  // namespace
 
 TORCH_LIBRARY_FRAGMENT(bfly, m) {
+  m.def("delta_record_floats(int T, int nseq, int H, int G, int D, int Dv, int v_ld, int max_rows) -> int", &delta_record_floats);
   m.def("post_norm_add_norm(Tensor(a!) x, Tensor y, Tensor? nw, Tensor? nb, float eps, float mult, Tensor? extra, "
         "Tensor? nw2, Tensor? nb2, Tensor(b!)? h, bool rms=False, int choices=0, Tensor? yw=None, bool f32=False, "
         "bool slabs=False) -> ()");

@@ -35,10 +35,12 @@ void launch_short_conv_state_update(const void* z, long z_ld, float* state, cons
 // Gated delta rule over packed rows (see ops.delta_scan): q, k f32 [T, G, D], v f32 [T, H, Dv] with row
 // strides, b / a [T, H] logits of the activation type, state f32 [slots, H, Dv, D] (a head's state
 // column by column), o f32 [T, H, Dv].
-// Returns < 0 if D > 256. max_rows > 0: no sequence has more rows
+// Returns < 0 if D > 256. max_rows > 0: no sequence has more rows. rec: scratch of delta_record_floats (0: none).
 int launch_delta_scan(const float* q, long q_ld, const float* k, long k_ld, const float* v, long v_ld, const void* b,
                       long b_ld, const void* a, long a_ld, const float* a_log, const float* dt_bias, float* state,
                       const int* state_slots, const int* row_cu, int nseq, const int* positions, float q_scale,
-                      float unit_eps, float* o, int T, int H, int G, int D, int Dv, bool f32, hipStream_t s, int max_rows = 0);
+                      float unit_eps, float* o, float* rec, int T, int H, int G, int D, int Dv, bool f32, hipStream_t s,
+                      int max_rows = 0);
+long delta_record_floats(long T, long nseq, int H, int G, int D, int Dv, long v_ld, int max_rows);
 
 }  // namespace bfly

@@ -11,8 +11,11 @@
 //   delta_scan_kernel                S <- g S; u = beta (v - S^T k); S <- S + k u^T; o = S^T q per
 //                                    (sequence, head), the state pooled per sequence; row by row
 //   delta_chunk_kernel               the same in chunks of 16 rows on the f32 matrix cores
+//   delta_record_kernel,
+//   delta_chain_kernel               the chunks in two launches, for longer sequences
 // Rows of a step are packed: sequence s owns rows row_cu[s] .. row_cu[s+1].
 #include <algorithm>
+#include <cmath>
 
 #include "bfly_common.h"
 #include "bfly_delta.h"
@@ -997,6 +1000,432 @@ __global__ __launch_bounds__(512, NT <= 4 ? 4 : 2) void delta_chunk_kernel(
   }
 }
 
+// The same chunks in two launches, for longer sequences: all of a chunk but its products with the state is independent of the
+// chunks before it. delta_record_kernel leaves k and q ([16][KP] rows each, what is no number as zero) of every chunk and key head
+// and (I + L)^-1 diag(beta), the weights (both in the operand layout of the 16x16x4 tiles) and the factors of every chunk and head
+// in records; delta_chain_kernel runs down a sequence's records with nothing but matrix products and the copies of the next ones.
+// A chunk's records are at its sequence's first row / 16 + the sequence's number + its own number there: no two chunks of a step
+// share one, and (rows / 16 + sequences) are enough. Sums and their order are those of delta_chunk_kernel.
+constexpr int kDeltaSlots = 3, kDeltaHead = 768;      // (floats of a head's record: [64][4], [64][4], six factors of 16 rows, the mark)
+constexpr int delta_rows(int NT) { return (32 * (16 * NT + 4) + 255) / 256 * 256; }
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t delta_buffer(const void* base, long bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0, (int)min(bytes, 0x7fffffffL), 0x00020000);
+}
+template <int N>
+__device__ __forceinline__ void delta_vm_wait() {
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+
+// Workgroup = (key head, chunk): four waves share the channels of the chunk's products, then take the key head's heads in turn.
+template <typename T, int NT>
+__global__ __launch_bounds__(256) void delta_record_kernel(
+    const float* __restrict__ q, long q_ld, const float* __restrict__ k, long k_ld, const T* __restrict__ bl, long b_ld,
+    const T* __restrict__ al, long a_ld, const float* __restrict__ a_log, const float* __restrict__ dt_bias,
+    const int* __restrict__ state_slots, const int* __restrict__ row_cu, int nseq, float q_scale, float unit_eps, int vec,
+    float* __restrict__ rec, int H, int G, int D, int cost, int first) {
+  constexpr int C = 16, NQ = NT / 4, KP = 16 * NT + 4, PP = C + 4;
+  __shared__ __attribute__((aligned(16))) float skk[4][64][4], sqk[4][64][4], snk[4][C], snq[4][C], stb[4][C * PP];
+  __shared__ int s_mark;
+  const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, m = lane & 15, gg = lane >> 4;
+  const int hk = blockIdx.x, b = first + blockIdx.y;
+  int s = -1;      // the last sequence whose records begin at or before b
+  for (int i0 = 0; i0 < nseq; i0 += 64) {
+    const int i = i0 + lane;
+    const unsigned long long le = __ballot(i < nseq && (row_cu[min(i, nseq)] >> 4) + i <= b);
+    s += __popcll(le);
+    if (~le) break;
+  }
+  if (s < 0) return;
+  const int r0 = __builtin_amdgcn_readfirstlane(row_cu[s]), r1 = __builtin_amdgcn_readfirstlane(row_cu[s + 1]);
+  const int t0 = r0 + C * (b - (r0 >> 4) - s);
+  if (t0 >= r1 || (cost && !scan_in_chunks(r1 - r0, cost)) || state_slots[s] < 0) return;
+  const int t = min(t0 + m, r1 - 1);            // (rows past the sequence: its last row again)
+  const bool in = t0 + m < r1;
+  if (tid == 0) s_mark = C;
+  __syncthreads();
+  {
+    const float* kr = k + (long)t * k_ld + (long)hk * D;
+    const float* qr = q + (long)t * q_ld + (long)hk * D;
+    f32x4 rk[NQ], rq[NQ];
+    if (vec & 1) {
+#pragma unroll
+      for (int i = 0; i < NQ; ++i) {
+        const int d = min(16 * (NQ * w + i) + 4 * gg, D - 4);
+        rk[i] = *reinterpret_cast<const f32x4*>(kr + d);
+        rq[i] = *reinterpret_cast<const f32x4*>(qr + d);
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < NQ; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int d = min(16 * (NQ * w + i) + 4 * gg + e, D - 1);
+          rk[i][e] = kr[d];
+          rq[i][e] = qr[d];
+        }
+    }
+    float* kb = rec + ((long)blockIdx.y * G + hk) * delta_rows(NT) + m * KP;
+    f32x4 nk = {0.f, 0.f, 0.f, 0.f}, nq = nk, kx[4], qx[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) kx[e] = qx[e] = nk;
+    const int Dm = in ? D : 0;
+    float zero = 0.f;
+#pragma unroll
+    for (int i = 0; i < NQ; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) zero = fmaf(rk[i][e], 0.f, zero);
+    if (__any(zero != 0.f)) {      // (channels past D are copies of the row's own)
+      if (zero != 0.f && in) atomicMin(&s_mark, m);
+#pragma unroll
+      for (int i = 0; i < NQ; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) rk[i][e] = rk[i][e] * 0.f == 0.f ? rk[i][e] : 0.f;
+    }
+#pragma unroll
+    for (int i = 0; i < NQ; ++i) {
+      const int d = 16 * (NQ * w + i) + 4 * gg;
+      f32x4 x, y;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const bool ok = d + e < Dm;
+        x[e] = ok ? rk[i][e] : 0.f;
+        y[e] = ok ? rq[i][e] : 0.f;
+      }
+      *reinterpret_cast<f32x4*>(kb + d) = x;
+      *reinterpret_cast<f32x4*>(kb + C * KP + d) = y;
+      nk += x * x;
+      nq += y * y;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        kx[e] = mfma_f32(x[e], x[e], kx[e]);
+        qx[e] = mfma_f32(y[e], x[e], qx[e]);
+      }
+    }
+    const float xk = row4_sum((nk[0] + nk[1]) + (nk[2] + nk[3])), xq = row4_sum((nq[0] + nq[1]) + (nq[2] + nq[3]));
+    *reinterpret_cast<f32x4*>(skk[w][lane]) = (kx[0] + kx[1]) + (kx[2] + kx[3]);
+    *reinterpret_cast<f32x4*>(sqk[w][lane]) = (qx[0] + qx[1]) + (qx[2] + qx[3]);
+    snk[w][m] = xk;
+    snq[w][m] = xq;
+  }
+  __syncthreads();
+  rec += (long)gridDim.y * G * delta_rows(NT);
+  const int HH = H / G, km = s_mark;
+  float nk = 0.f, nq = 0.f;
+  f32x4 zk = {0.f, 0.f, 0.f, 0.f}, zq = zk;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    nk += snk[i][m];
+    nq += snq[i][m];
+    zk += *reinterpret_cast<const f32x4*>(skk[i][lane]);
+    zq += *reinterpret_cast<const f32x4*>(sqk[i][lane]);
+  }
+  // (rows past the sequence: no key, also where unit_eps is 0)
+  const double kn = in ? 1. / sqrt((double)nk + (double)unit_eps) : 0.;
+  const float qn = (float)((double)q_scale / sqrt((double)nq + (double)unit_eps));
+  float* tb = stb[w];
+  for (int h = hk * HH + w; h < (hk + 1) * HH; h += 4) {
+    float* to = rec + ((long)blockIdx.y * H + h) * kDeltaHead;
+    const float av = (float)al[(long)t * a_ld + h] + dt_bias[h], bv = (float)bl[(long)t * b_ld + h];
+    const float sp = av > 20.f ? av : log1pf(expf(av));            // softplus
+    float g = expf(-expf(a_log[h]) * sp), beta = 1.f / (1.f + expf(-bv));
+    const bool nan = !(g == g && beta == beta);
+    const unsigned odd = (unsigned)__ballot(nan && in) & 0xffffu;
+    g = in && !nan ? g : 1.f;
+    beta = in && !nan ? beta : 0.f;
+    // column m of D (rows 4 gg + e kept), G_m, D_15,m and G_15
+    double x = 1., y = 1.;
+    float Gm = 1.f;
+    f32x4 dm = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < C; ++i) {
+      const double gi = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, g), i));
+      y *= gi;
+      x = i > m ? x * gi : 1.;
+      Gm = i == m ? (float)y : Gm;
+      dm[i & 3] = gg == i >> 2 ? (float)x : dm[i & 3];
+    }
+    double zd[4];
+    // the second sum's weights D_tj (q_t . k_j) / |k_j|
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      zd[e] = (double)zq[e] * ((double)dm[e] * kn);
+      tb[(4 * gg + e) * PP + m] = 4 * gg + e >= m ? (float)zd[e] : 0.f;
+    }
+    lds_wave_sync();
+    *reinterpret_cast<f32x4*>(to + 256 + 4 * lane) = *reinterpret_cast<const f32x4*>(tb + m * PP + 4 * gg);
+    if (gg == 0) {
+      float* f = to + 512 + m;
+      f[0] = (float)(Gm * kn);
+      f[C] = (float)((float)x * kn);
+      f[2 * C] = Gm;
+      f[3 * C] = qn;
+      f[4 * C] = (float)y;
+      f[5 * C] = beta;
+      if (m == 0) *reinterpret_cast<int*>(to + 512 + 6 * C) = min(km, odd ? __builtin_ctz(odd) : C);
+    }
+    lds_wave_sync();
+    // (I + L)^-1 diag(beta) as in delta_chunk_kernel
+#pragma unroll
+    for (int e = 0; e < 4; ++e) zd[e] = (double)zk[e] * ((double)dm[e] * kn);
+    const double rw = beta * kn;
+    const int b8 = m & 8, cc = m & 7;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) tb[(4 * gg + e) * PP + m] = (float)(zd[e] * __shfl(rw, 4 * gg + e, 64));
+    lds_wave_sync();
+    f32x4 l[8][2];      // rows of this lane's diagonal block
+#pragma unroll
+    for (int i = 1; i < 8; ++i) {
+      l[i][0] = *reinterpret_cast<const f32x4*>(tb + (b8 + i) * PP + b8);
+      if (i > 4) l[i][1] = *reinterpret_cast<const f32x4*>(tb + (b8 + i) * PP + b8 + 4);
+    }
+    f32x4 l21 = {0.f, 0.f, 0.f, 0.f};
+    if (m >= 8 && gg < 2) l21 = *reinterpret_cast<const f32x4*>(tb + m * PP + 4 * gg);
+    lds_wave_sync();
+    float xs[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      xs[i] = i == cc ? 1.f : 0.f;
+#pragma unroll
+      for (int j = 0; j < i; ++j) xs[i] = fmaf(-l[i][j >> 2][j & 3], xs[j], xs[i]);
+      tb[(b8 + i) * PP + m] = xs[i];
+      tb[((b8 ^ 8) + i) * PP + m] = 0.f;
+    }
+    lds_wave_sync();
+    const f32x4 ta = *reinterpret_cast<const f32x4*>(tb + m * PP + 4 * gg);
+    float tc[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) tc[e] = tb[(4 * gg + e) * PP + m];
+    f32x4 y1 = {0.f, 0.f, 0.f, 0.f}, y2 = y1;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) y1 = mfma_f32(l21[e], tc[e], y1);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) y2 = mfma_f32(ta[e], y1[e], y2);
+    lds_wave_sync();
+#pragma unroll
+    for (int e = 0; e < 4; ++e) tb[(4 * gg + e) * PP + m] = 4 * gg + e > m ? (tc[e] - y2[e]) * beta : 0.f;
+    lds_wave_sync();
+    *reinterpret_cast<f32x4*>(to + 4 * lane) = *reinterpret_cast<const f32x4*>(tb + m * PP + 4 * gg);
+    lds_wave_sync();
+  }
+}
+
+// Workgroup = (sequence, head, 64 columns of Dv), four waves of 16 columns with the whole height of the state each, in the accumulator
+// layout (see delta_chunk_kernel). Bound by the vector units, which f32 products occupy for 32 clocks each and share with everything
+// else: 104 products and 250 vector instructions, 2.3 us a chunk at 128 x 128. (As products of three-part bf16 operands, which run
+// beside vector instructions, 2.0: splitting the state takes as long as the products did.) All workgroups of a sequence's key head read the same rows: they follow eight apart, in one XCD.
+// Records arrive by LDS-DMA, kDeltaSlots chunks ahead. The records [first, first + count) of the step; a sequence that goes on in the
+// next ones leaves its state in its slot.
+template <int NT>
+__global__ __launch_bounds__(256, NT <= 8 ? 2 : 1) void delta_chain_kernel(
+    const float* __restrict__ rec, const float* __restrict__ v, long v_ld, float* __restrict__ state,
+    const int* __restrict__ state_slots, const int* __restrict__ row_cu, const int* __restrict__ positions, int vec,
+    float* __restrict__ o, int nseq, int H, int G, int D, int Dv, int cost, int first, int count) {
+  constexpr int C = 16, SL = kDeltaSlots, KP = 16 * NT + 4, RR = delta_rows(NT), U1 = RR / 256, U = U1 + kDeltaHead / 256,
+                PER = (U + 3) / 4, REC = U * 256, NS = NT <= 8 ? 2 : 4;
+  extern __shared__ __attribute__((aligned(16))) float smem[];      // [SL][REC], then values: [SL][4 waves][4][64]
+  const int nz = (Dv + 63) / 64, HH = H / G, per = HH * nz, u = blockIdx.x >> 3, grp = u / per * 8 + (blockIdx.x & 7);
+  const int s = grp / G, hk = grp - s * G, h = hk * HH + u % per / nz, c0 = u % nz * 64;
+  if (s >= nseq) return;
+  const int r0 = __builtin_amdgcn_readfirstlane(row_cu[s]), r1 = __builtin_amdgcn_readfirstlane(row_cu[s + 1]);
+  if (r1 <= r0 || (cost && !scan_in_chunks(r1 - r0, cost))) return;      // (the row-by-row form's)
+  const int at = (r0 >> 4) + s, cb = max(0, first - at), ce = min((r1 - r0 + C - 1) / C, first + count - at);
+  if (cb >= ce) return;
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, m = lane & 15, gg = lane >> 4;
+  const int slot = state_slots[s];
+  if (slot < 0) {      // padding sequence of a fixed-shape step: defined output, no state
+    const int ta = r0 + cb * C, n = min(r1, r0 + ce * C) - ta;
+    for (int i = tid; i < n * 64; i += 256)
+      if (c0 + (i & 63) < Dv) o[((long)(ta + (i >> 6)) * H + h) * Dv + c0 + (i & 63)] = 0.f;
+    return;
+  }
+  const int col = c0 + 16 * wave + m;
+  const bool live = col < Dv;
+  // Addresses are a scalar base and offset per chunk and a constant per lane. Rows past the sequence, rows of the state past D and
+  // columns past the head lie past the buffer's end: they read zeros and are not stored, and no lane takes a branch of its own.
+  const int dead = live ? 0 : -1;
+  float* S = state + ((long)slot * H + h) * Dv * D;
+  auto place = [&](int d) { return (col * D + d) * 4 | dead | (d < D ? 0 : -1); };
+  f32x4 st[NT];
+  {
+    const bool fresh = cb == 0 && positions[r0] == 0;
+    const auto ss = __builtin_amdgcn_make_buffer_rsrc(S, (short)0, fresh ? 0 : Dv * D * 4, 0x00020000);
+#pragma unroll
+    for (int i = 0; i < NT; ++i) {
+      const int d = 16 * i + 4 * gg;
+      if (vec & 2) st[i] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(ss, place(d), 0, 0));
+      else
+#pragma unroll
+        for (int e = 0; e < 4; ++e) st[i][e] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(ss, place(d + e), 0, 0));
+    }
+  }
+  const auto rs = delta_buffer(rec, 0x7fffffff);
+  const int lastn = min(C, r1 - r0 - (ce - 1) * C);      // rows of the last chunk here
+  const long vl = (long)(lastn - 1) * v_ld + Dv, ve1 = (long)(C - 1) * v_ld + Dv, ol = ((long)(lastn - 1) * H + 1) * Dv;
+  const int vbytes = (int)min(ve1 * 4, 0x7fffffffL), vlast = (int)min(vl * 4, 0x7fffffffL), olast = (int)min(ol * 4, 0x7fffffffL);
+  int va[4], oo[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    va[e] = (int)((4 * gg + e) * v_ld + col) * 4 | dead;
+    oo[e] = ((4 * gg + e) * H * Dv + col) * 4 | dead;
+  }
+  const float* vp = v + (long)(r0 + cb * C) * v_ld + (long)h * Dv;
+  float* op = o + ((long)(r0 + cb * C) * H + h) * Dv;
+  const int rel = at + cb - first, rbase = (rel * G + hk) * RR * 4, hbase = (count * G * RR + (rel * H + h) * kDeltaHead) * 4;
+  // operation j of PER + 4 of chunk c's copy: a part of its records, then the lanes' own four values. Past the last chunk: that one
+  // again, into a slot nobody reads.
+  typedef __attribute__((address_space(3))) void* lds_ptr_t;
+  auto dma = [&](int c, int sl, int j) {
+    c = min(c, ce - 1) - cb;
+    if (j < PER) {
+      const int x = min(wave + 4 * j, U - 1);
+      const int off = x < U1 ? rbase + c * G * RR * 4 + 1024 * x : hbase + c * H * kDeltaHead * 4 + 1024 * (x - U1);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_ptr_t)(smem + sl * REC + 256 * x), 16, 16 * lane, off, 0, 0);
+    } else {
+      const auto vs = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(vp + (long)(c * C) * v_ld), (short)0,
+                                                        c == ce - 1 - cb ? vlast : vbytes, 0x00020000);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(vs, (lds_ptr_t)(smem + SL * REC + ((sl * 4 + wave) * 4 + j - PER) * 64), 4,
+                                               va[j - PER], 0, 0, 0);
+    }
+  };
+#pragma unroll
+  for (int i = 0; i < SL; ++i)
+#pragma unroll
+    for (int j = 0; j < PER + 4; ++j) dma(cb + i, i, j);
+  f32x4 ka[NT], qa[NT];
+  float ku[NT][4], raw[4];
+  auto krow = [&](int sl, int i) { ka[i] = *reinterpret_cast<const f32x4*>(smem + sl * REC + m * KP + 16 * i + 4 * gg); };
+  auto values = [&](int sl) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) raw[e] = smem[SL * REC + ((sl * 4 + wave) * 4 + e) * 64 + lane];
+  };
+  delta_vm_wait<(SL - 1) * (PER + 4)>();
+  __builtin_amdgcn_s_barrier();
+#pragma unroll
+  for (int i = 0; i < NT; ++i) krow(0, i);
+  values(0);
+  int sl = 0;
+  const f32x4 z4 = {0.f, 0.f, 0.f, 0.f};
+  // K S first; Q S runs while its sums, (I + L)^-1 and the factors turn them into U, so the matrix cores do not wait. Fragments are
+  // read a product ahead: q during K S, the columns of k during Q S, the next chunk's k during the state's update. The one barrier
+  // of a chunk lies before the update: behind it the chunk's slot is free.
+  for (int c = cb; c < ce; ++c) {
+    const float* x0 = smem + sl * REC;
+    const float* f = x0 + RR + 512;
+    const f32x4 ti = *reinterpret_cast<const f32x4*>(x0 + RR + 4 * lane), wq = *reinterpret_cast<const f32x4*>(x0 + RR + 256 + 4 * lane);
+    const f32x4 gk = *reinterpret_cast<const f32x4*>(f + 4 * gg), dk = *reinterpret_cast<const f32x4*>(f + C + 4 * gg);
+    const f32x4 gt = *reinterpret_cast<const f32x4*>(f + 2 * C + 4 * gg), qn = *reinterpret_cast<const f32x4*>(f + 3 * C + 4 * gg);
+    const f32x4 bt = *reinterpret_cast<const f32x4*>(f + 5 * C + 4 * gg);
+    const float gn = f[4 * C];
+    const int odd = __builtin_amdgcn_readfirstlane(reinterpret_cast<const int*>(f)[6 * C]);
+    f32x4 pk = z4, pq = z4;
+#pragma unroll
+    for (int i = 0; i < NT; i += NS) {
+      f32x4 xk[4] = {z4, z4, z4, z4};
+#pragma unroll
+      for (int j = i; j < i + NS; ++j) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          xk[e] = mfma_f32(ka[j][e], st[j][e], xk[e]);
+          if (e == 1) qa[j] = *reinterpret_cast<const f32x4*>(x0 + C * KP + m * KP + 16 * j + 4 * gg);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+      pk += (xk[0] + xk[1]) + (xk[2] + xk[3]);
+    }
+    // no[e]: 0, or NaN from the first row of this lane's column on that is no number (as in delta_chunk_kernel)
+    f32x4 no, ux[4], u = z4;
+    float ve[4];
+#pragma unroll
+    for (int i = 0; i < NT; i += NS) {
+      f32x4 xq[4] = {z4, z4, z4, z4};
+#pragma unroll
+      for (int j = i; j < i + NS; ++j) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          xq[e] = mfma_f32(qa[j][e], st[j][e], xq[e]);
+          ku[j][e] = x0[(4 * gg + e) * KP + 16 * j + m];
+        }
+        if (j == 0) {
+          float vv[4], sum = 0.f;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const float z = fmaf(raw[e], 0.f, 0.f);
+            vv[e] = z == 0.f ? raw[e] : 0.f;
+            sum += z;
+            no[e] = sum + (4 * gg + e >= odd ? NAN : 0.f);
+          }
+          // lane groups 1 and 3 take the sum of 0 and 2, then 2 and 3 that of 0 and 1 (the swaps of row4_sum)
+          const auto up = __builtin_amdgcn_permlane16_swap(__float_as_uint(sum), __float_as_uint(sum), false, false);
+          const unsigned pair = __float_as_uint(__uint_as_float(up[0]) + __uint_as_float(up[1]));
+          const auto far = __builtin_amdgcn_permlane32_swap(pair, pair, false, false);
+          no += (gg & 1 ? __uint_as_float(up[0]) : 0.f) + (gg & 2 ? __uint_as_float(far[0]) : 0.f);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) ve[e] = fmaf(-gk[e], pk[e], vv[e]);
+        }
+        if (j == NT / 2 - 1) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            ux[e] = mfma_f32(ti[e], ve[e], z4);
+            u[e] = bt[e] * ve[e];
+          }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      pq += (xq[0] + xq[1]) + (xq[2] + xq[3]);
+    }
+    u += (ux[0] + ux[1]) + (ux[2] + ux[3]);
+    const f32x4 ud = (u + no) * dk;
+    // A turn of the loop issues PER + 8 memory operations (records, values, outputs), the start has no outputs: with as many of the
+    // newest in flight, the next chunk's records have landed (own part).
+    if (c - cb < SL - 1) delta_vm_wait<(SL - 2) * (PER + 4)>();
+    else delta_vm_wait<(SL - 2) * (PER + 8)>();
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    const int nx = sl + 1 == SL ? 0 : sl + 1;
+    constexpr int OPS = PER + 4, QS = NT / 2;
+    f32x4 yx[4];
+#pragma unroll
+    for (int i = 0; i < NT; i += 4) {
+      f32x4 x[4] = {z4, z4, z4, z4};
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) x[j] = mfma_f32(ku[i + j][e], ud[e], x[j]);
+        if (i == 0) yx[e] = mfma_f32(wq[e], u[e], e == 0 ? no : z4);
+        krow(nx, i + e);
+        const int n = i + e - QS;      // the copies, spread over the second half
+        if (n >= 0) {
+#pragma unroll
+          for (int j = n * OPS / QS; j < (n + 1) * OPS / QS; ++j) dma(c + SL, sl, j);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      if (i == 0) values(nx);
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) st[i + j][e] = fmaf(st[i + j][e], gn, x[j][e]);
+    }
+    sl = nx;
+    const f32x4 y = (yx[0] + yx[1]) + (yx[2] + yx[3]);
+    const auto out = __builtin_amdgcn_make_buffer_rsrc(op, (short)0, c == ce - 1 ? olast : 0x7fffffff, 0x00020000);
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(fmaf(pq[e], gt[e], y[e]) * qn[e]), out, oo[e], 0, 0);
+    op += (long)C * H * Dv;
+  }
+  delta_vm_wait<0>();      // no LDS-DMA may outlive the workgroup
+  const auto ss = __builtin_amdgcn_make_buffer_rsrc(S, (short)0, Dv * D * 4, 0x00020000);
+#pragma unroll
+  for (int i = 0; i < NT; ++i) {
+    const int d = 16 * i + 4 * gg;
+    if (vec & 2) __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, st[i]), ss, place(d), 0, 0);
+    else
+#pragma unroll
+      for (int e = 0; e < 4; ++e) __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(st[i][e]), ss, place(d + e), 0, 0);
+  }
+}
+
 // threads of a one-row workgroup: about four elements per thread, whole waves, at most 1024
 int row_threads(int W) { return std::min(1024, std::max(64, (W / 4 + 63) / 64 * 64)); }
 
@@ -1127,11 +1556,34 @@ static void delta_chunk_launch(const float* q, long q_ld, const float* k, long k
                                                    row_cu, positions, q_scale, unit_eps, vec, o, H, G, D, Dv, cost);
 }
 
-template <typename T>
-static int delta_scan_t(const float* q, long q_ld, const float* k, long k_ld, const float* v, long v_ld, const T* b,
-                        long b_ld, const T* a, long a_ld, const float* a_log, const float* dt_bias, float* state,
-                        const int* state_slots, const int* row_cu, int nseq, const int* positions, float q_scale,
-                        float unit_eps, float* o, int T_, int H, int G, int D, int Dv, hipStream_t s, int max_rows) {
+// 16-channel tiles of the chunk kernels
+static int delta_tiles(int D) { return D <= 64 ? 4 : D <= 128 ? 8 : D <= 192 ? 12 : 16; }
+// floats of the records of one chunk, and the chunks of a launch: those of the step, at most 256 MB of records
+static long delta_chunk_floats(int H, int G, int D) { return (long)G * delta_rows(delta_tiles(D)) + (long)H * kDeltaHead; }
+static long delta_chunks_at_once(long T, long nseq, int H, int G, int D) {
+  return std::min((T >> 4) + nseq, std::max(1L, (64L << 20) / delta_chunk_floats(H, G, D)));
+}
+
+// Two launches where the times of both forms say so (us, measured): a chunk of one workgroup after the other takes `one` in one launch
+// and `two` in the chains, times the rounds of workgroups or, where two share a compute unit, the share; the records come on top.
+// 16 heads of 128 on 4, us of one launch -> two: one sequence of 64 rows 20.1 and 20.3, of 128 32.5 -> 29.6, of 2000 397 -> 292,
+// 11 of 200 to 800 245 -> 179, 32 of 32 52 -> 40, 64 of 320 560 -> 389; 32 heads of 64 on 8, 64 of 320 312 -> 291; heads of 256, 32 of
+// 320 872 -> 781. Of 824 steps that were timed none is slower than in one launch by more than 4 %.
+static bool delta_two_launches(long T, long nseq, int H, int G, int D, int Dv, long wgs, int max_rows) {
+  const long longest = std::max(1L, max_rows > 0 ? max_rows : T - nseq + 1), like = std::min(nseq, (T + longest - 1) / longest);
+  const float one[] = {2.15f, 3.2f, 4.2f, 5.3f}, two[] = {1.4f, 2.35f, 3.8f, 5.1f};
+  const float n = (float)((longest + 15) >> 4), w = (float)(like * wgs), share = std::max(1.f, w / 280), rounds = std::ceil(w / 256);
+  const int d = (D - 1) / 64;
+  const float records = 3.5f + (float)((T >> 4) + nseq) * G * (3 + 2 * (H / G)) * 1e-3f;
+  return records + two[d] * n * (D <= 128 ? share : rounds) < one[d] * n * (D <= 64 ? share : rounds);
+}
+
+struct DeltaPlan {
+  ScanForms form;
+  int cost;
+  bool records;      // chunks in two launches
+};
+static DeltaPlan delta_plan(long T, long nseq, int H, int G, int D, int Dv, long v_ld, int max_rows) {
   // A chunk takes the time of 10 rows of 128 channels while the workgroups all run at once, and of 14 where they queue (the
   // loop's have half the LDS): 16 heads of 128, time of chunks over loop for one sequence of 8, 12, 16, 20, 32 rows 1.07, 0.88,
   // 0.80, 0.85, 0.66, for 64 of them 1.24, 1.06, 1.05, 1.23, 0.91; channels of 64 0.82 and 0.94 at 16 rows, of 32 0.91 and 1.14,
@@ -1139,24 +1591,74 @@ static int delta_scan_t(const float* q, long q_ld, const float* k, long k_ld, co
   // 249 and 291, now 173.
   const long wgs = (long)H * ((Dv + 63) / 64);
   const bool queue = nseq * wgs >= 1024;
-  const int cost = D > 128 ? 8 : D > 64 ? (queue ? 14 : 10) : D > 32 ? (queue ? 12 : 10) : queue ? 15 : 12;
-  ScanForms form = scan_forms(T_, nseq, cost, wgs, max_rows);
-  if (D > 256) form = {true, false};
-  if (form.chunks) {
-#define BFLY_DCH(NT)                                                                                                    \
-  delta_chunk_launch<T, NT>(q, q_ld, k, k_ld, v, v_ld, b, b_ld, a, a_ld, a_log, dt_bias, state, state_slots, row_cu, nseq, \
-                            positions, q_scale, unit_eps, o, H, G, D, Dv, s, form.rows ? cost : 0)
-    if (D <= 64) BFLY_DCH(4);
-    else if (D <= 128) BFLY_DCH(8);
-    else if (D <= 192) BFLY_DCH(12);
-    else BFLY_DCH(16);
+  DeltaPlan p;
+  p.cost = D > 128 ? 8 : D > 64 ? (queue ? 14 : 10) : D > 32 ? (queue ? 12 : 10) : queue ? 15 : 12;
+  p.form = D > 256 ? ScanForms{true, false} : scan_forms(T, nseq, p.cost, wgs, max_rows);
+  p.records = p.form.chunks && std::max({v_ld, (long)H * Dv, (long)D * Dv}) * 64 < (1L << 31) &&      // (32-bit byte offsets)
+              delta_two_launches(T, nseq, H, G, D, Dv, wgs, max_rows);
+  return p;
+}
+
+long delta_record_floats(long T, long nseq, int H, int G, int D, int Dv, long v_ld, int max_rows) {
+  if (T <= 0 || nseq <= 0 || !delta_plan(T, nseq, H, G, D, Dv, v_ld, max_rows).records) return 0;
+  return delta_chunks_at_once(T, nseq, H, G, D) * delta_chunk_floats(H, G, D);
+}
+
+template <typename T, int NT>
+static void delta_records_launch(const float* q, long q_ld, const float* k, long k_ld, const float* v, long v_ld, const T* b,
+                                 long b_ld, const T* a, long a_ld, const float* a_log, const float* dt_bias, float* state,
+                                 const int* state_slots, const int* row_cu, int nseq, const int* positions, float q_scale,
+                                 float unit_eps, float* o, float* rec, int T_, int H, int G, int D, int Dv, hipStream_t s, int cost) {
+  constexpr size_t lds = (size_t)kDeltaSlots * (delta_rows(NT) + kDeltaHead + 1024) * sizeof(float);
+  static bool once = false;
+  if (!once) {
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&delta_chain_kernel<NT>), hipFuncAttributeMaxDynamicSharedMemorySize,
+                              (int)lds);
+    once = true;
+  }
+  // 1: rows of q and k, 2: columns of the state in four-element accesses
+  int vec = 0;
+  if (D % 4 == 0 && rows_aligned(q, q_ld, 4) && rows_aligned(k, k_ld, 4)) vec |= 1;
+  if (D % 4 == 0) vec |= 2;
+  const long all = (T_ >> 4) + nseq, most = delta_chunks_at_once(T_, nseq, H, G, D);
+  for (long first = 0; first < all; first += most) {
+    const int count = (int)std::min(most, all - first);
+    delta_record_kernel<T, NT><<<dim3(G, count), 256, 0, s>>>(q, q_ld, k, k_ld, b, b_ld, a, a_ld, a_log, dt_bias, state_slots, row_cu,
+                                                             nseq, q_scale, unit_eps, vec, rec, H, G, D, cost, (int)first);
+    delta_chain_kernel<NT><<<(nseq * G + 7) / 8 * 8 * (H / G) * ((Dv + 63) / 64), 256, lds, s>>>(
+        rec, v, v_ld, state, state_slots, row_cu, positions, vec, o, nseq, H, G, D, Dv, cost, (int)first, count);
+  }
+}
+
+template <typename T>
+static int delta_scan_t(const float* q, long q_ld, const float* k, long k_ld, const float* v, long v_ld, const T* b,
+                        long b_ld, const T* a, long a_ld, const float* a_log, const float* dt_bias, float* state,
+                        const int* state_slots, const int* row_cu, int nseq, const int* positions, float q_scale,
+                        float unit_eps, float* o, float* rec, int T_, int H, int G, int D, int Dv, hipStream_t s, int max_rows) {
+  const DeltaPlan plan = delta_plan(T_, nseq, H, G, D, Dv, v_ld, max_rows);
+  const int cost = plan.form.rows ? plan.cost : 0;
+  if (plan.form.chunks) {
+    if (plan.records && !rec) return -2;
+#define BFLY_DCH(NT)                                                                                                      \
+  (plan.records ? delta_records_launch<T, NT>(q, q_ld, k, k_ld, v, v_ld, b, b_ld, a, a_ld, a_log, dt_bias, state,         \
+                                              state_slots, row_cu, nseq, positions, q_scale, unit_eps, o, rec, T_, H, G, D, \
+                                              Dv, s, cost)                                                                \
+                : delta_chunk_launch<T, NT>(q, q_ld, k, k_ld, v, v_ld, b, b_ld, a, a_ld, a_log, dt_bias, state,           \
+                                            state_slots, row_cu, nseq, positions, q_scale, unit_eps, o, H, G, D, Dv, s, cost))
+    switch (delta_tiles(D)) {
+      case 4: BFLY_DCH(4); break;
+      case 8: BFLY_DCH(8); break;
+      case 12: BFLY_DCH(12); break;
+      default: BFLY_DCH(16);
+    }
 #undef BFLY_DCH
-    if (!form.rows) return 0;
+    if (!plan.form.rows) return 0;
   }
   dim3 grid(nseq, H, (Dv + 63) / 64);
 #define BFLY_DELTA(NR)                                                                                             \
   delta_scan_kernel<T, NR><<<grid, 512, 0, s>>>(q, q_ld, k, k_ld, v, v_ld, b, b_ld, a, a_ld, a_log, dt_bias, state, \
-                                                state_slots, row_cu, positions, q_scale, unit_eps, o, H, G, D, Dv, form.chunks ? cost : 0)
+                                                state_slots, row_cu, positions, q_scale, unit_eps, o, H, G, D, Dv, \
+                                                plan.form.chunks ? plan.cost : 0)
   if (D <= 32) BFLY_DELTA(4);
   else if (D <= 64) BFLY_DELTA(8);
   else if (D <= 128) BFLY_DELTA(16);
@@ -1169,14 +1671,15 @@ static int delta_scan_t(const float* q, long q_ld, const float* k, long k_ld, co
 int launch_delta_scan(const float* q, long q_ld, const float* k, long k_ld, const float* v, long v_ld, const void* b,
                       long b_ld, const void* a, long a_ld, const float* a_log, const float* dt_bias, float* state,
                       const int* state_slots, const int* row_cu, int nseq, const int* positions, float q_scale,
-                      float unit_eps, float* o, int T, int H, int G, int D, int Dv, bool f32, hipStream_t s, int max_rows) {
+                      float unit_eps, float* o, float* rec, int T, int H, int G, int D, int Dv, bool f32, hipStream_t s,
+                      int max_rows) {
   if (T <= 0 || nseq <= 0) return 0;
   if (f32)
     return delta_scan_t<float>(q, q_ld, k, k_ld, v, v_ld, (const float*)b, b_ld, (const float*)a, a_ld, a_log, dt_bias,
-                               state, state_slots, row_cu, nseq, positions, q_scale, unit_eps, o, T, H, G, D, Dv, s,
-                               max_rows);
+                               state, state_slots, row_cu, nseq, positions, q_scale, unit_eps, o, rec, T, H, G, D, Dv,
+                               s, max_rows);
   return delta_scan_t<bf16>(q, q_ld, k, k_ld, v, v_ld, (const bf16*)b, b_ld, (const bf16*)a, a_ld, a_log, dt_bias, state,
-                            state_slots, row_cu, nseq, positions, q_scale, unit_eps, o, T, H, G, D, Dv, s, max_rows);
+                            state_slots, row_cu, nseq, positions, q_scale, unit_eps, o, rec, T, H, G, D, Dv, s, max_rows);
 }
 
 }  // namespace bfly

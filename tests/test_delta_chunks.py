@@ -93,3 +93,66 @@ def test_values_that_are_no_numbers_reach_later_rows_only(row, where, bad):
         assert torch.equal(got.isfinite(), want.isfinite())
         ok = want.isfinite()
         assert (got - want)[ok].abs().max() < 1e-5 * want[ok].abs().max()
+
+
+def loop64(x, D, eps):
+    """The token loop in float64 on the GPU: outputs [T, H, Dv] and the state pool."""
+    x = {k: t.cuda() for k, t in x.items()}
+    H, G, cu = x["v"].shape[1], x["q"].shape[1], x["row_cu"].tolist()
+    unit = lambda t: (t.to(F64) / torch.sqrt((t.to(F64) ** 2).sum(-1, keepdim=True) + eps)).repeat_interleave(H // G, 1)      # noqa: E731
+    q, k, v, beta = unit(x["q"]) * D ** -0.5, unit(x["k"]), x["v"].to(F64), torch.sigmoid(x["b"].to(F64))
+    decay = torch.exp(-torch.exp(x["a_log"].to(F64)) * torch.nn.functional.softplus(x["a"].to(F64) + x["dt_bias"].to(F64)))
+    o, state = torch.zeros(v.shape, dtype=F64, device="cuda"), x["state"].to(F64).clone()
+    for s, slot in enumerate(x["state_slots"].tolist()):
+        if slot < 0 or cu[s] == cu[s + 1]:
+            continue
+        m = state[slot] if int(x["positions"][cu[s]]) else torch.zeros_like(state[slot])
+        for t in range(cu[s], cu[s + 1]):
+            m = decay[t][:, None, None] * m
+            u = beta[t][:, None] * (v[t] - (m @ k[t][:, :, None])[:, :, 0])
+            m = m + u[:, :, None] * k[t][:, None]
+            o[t] = (m @ q[t][:, :, None])[:, :, 0]
+        state[slot] = m
+    return o.cpu(), state.cpu()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("H,G,D,Dv,seqs,no_slot", [
+    (8, 2, 128, 128, [(0, 300), (5, 161), (0, 2), (9, 0), (0, 17)], 3),       # an empty sequence; one without a slot
+    (3, 3, 40, 33, [(7, 200), (0, 176)], None),                                 # one head to a key head, rows not a multiple of four
+    (6, 1, 64, 80, [(0, 143), (3, 144), (0, 145)], 1),                          # last chunks of 15, 16 and 1 rows
+    (10, 2, 96, 64, [(1, 257)], None), (4, 2, 150, 64, [(0, 250)], None), (8, 1, 256, 48, [(2, 400)], None),
+    (64, 32, 128, 16, [(0, 6000)], None),                                       # more records than a launch holds
+])
+def test_chunks_in_two_launches_match_the_token_loop(H, G, D, Dv, seqs, no_slot):
+    x = step(seqs, H, G, D, Dv, D + H, torch.bfloat16)
+    if no_slot is not None:
+        x["state_slots"][no_slot] = -1
+    T, most = len(x["q"]), max(n for _, n in seqs)
+    assert torch.ops.bfly.delta_record_floats(T, len(seqs), H, G, D, Dv, H * Dv, most) > 0
+    got = {k: t.cuda() for k, t in x.items()}
+    o = ops.delta_scan(**got, q_scale=D ** -0.5, unit_eps=1e-6, max_rows=most)
+    want, state = loop64(x, D, 1e-6)
+    # f32 sums of up to 256 channels, a solve of up to 16 coupled rows, products of 16 decays (f32 eps 6e-8 each)
+    for a, b in ((o, want), (got["state"], state)):
+        assert (a.cpu().to(F64) - b).abs().max() < 5e-6 * b.abs().max()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("bad", [float("nan"), float("inf")])
+@pytest.mark.parametrize("where", ["q", "k", "v", "a", "b"])
+@pytest.mark.parametrize("row", [0, 23, 31, 149])      # of ten chunks: first row, both blocks, the last row
+def test_two_launches_values_that_are_no_numbers_reach_later_rows_only(row, where, bad):
+    D, Dv = 64, 80
+    x = step([(3, 150), (0, 160)], 4, 2, D, Dv, row)
+    assert torch.ops.bfly.delta_record_floats(310, 2, 4, 2, D, Dv, 4 * Dv, 160) > 0
+    x[where][row, 1, ...] = bad if where in "ab" else x[where][row, 1]
+    if where not in "ab":
+        x[where][row, 1, 5] = bad
+    got, ref = {k: t.cuda() for k, t in x.items()}, {k: t.clone() for k, t in x.items()}
+    o = ops.delta_scan(**got, q_scale=D ** -0.5, unit_eps=1e-6, max_rows=160)
+    w = ops.delta_scan(**ref, q_scale=D ** -0.5, unit_eps=1e-6)
+    for a, b in ((o.cpu(), w), (got["state"].cpu(), ref["state"])):
+        assert torch.equal(a.isfinite(), b.isfinite())
+        ok = b.isfinite()
+        assert (a - b)[ok].abs().max() < 1e-5 * b[ok].abs().max()      # two f32 evaluations
