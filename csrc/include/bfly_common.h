@@ -35,6 +35,16 @@ __device__ __forceinline__ float wave_max(float v) {
   return v;
 }
 
+// Inclusive sum over the lanes up to this one
+__device__ __forceinline__ int lane_scan(int x) {
+  x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xF, 0xF, false);     // row_shr 1, 2, 4, 8
+  x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xF, 0xF, false);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xF, 0xF, false);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xF, 0xF, false);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xA, 0xF, false);     // row_bcast 15, 31
+  return x + __builtin_amdgcn_update_dpp(0, x, 0x143, 0xC, 0xF, false);
+}
+
 // Maximum / sum over the four lanes l, l ^ 16, l ^ 32, l ^ 48 (one column of a 16x16 MFMA result) without LDS traffic
 __device__ __forceinline__ float row4_max(float x) {
   const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);

@@ -260,15 +260,6 @@ __device__ __forceinline__ int ctx_pages(int ctx, int max_ctx) {
 }
 // pages that the time of a segment's end is worth (elements of `es` bytes)
 __host__ __device__ constexpr int flat_extra(int es) { return 8 / es; }
-// inclusive sum over the lanes up to this one
-__device__ __forceinline__ int wave_scan(int x) {
-  x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xF, 0xF, false);     // row_shr 1, 2, 4, 8
-  x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xF, 0xF, false);
-  x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xF, 0xF, false);
-  x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xF, 0xF, false);
-  x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xA, 0xF, false);     // row_bcast 15, 31
-  return x + __builtin_amdgcn_update_dpp(0, x, 0x143, 0xC, 0xF, false);
-}
 // pages per workgroup when the P pages of a step are cut into (at most) N equal pieces; one page per wave at least
 __device__ __forceinline__ int flat_chunk(int P, int N, int NW) { return max((P + N - 1) / N, NW); }
 
@@ -304,7 +295,7 @@ attn_decode_flat_kernel(const bf16* __restrict__ q, long q_stride, const CT* __r
   for (int i = 0; i < R; ++i) vctx[i] = 64 * i + lane < B ? min(ctx_lens[64 * i + lane], max_ctx) : 0;
 #pragma unroll
   for (int i = 0; i < R; ++i) {
-    const int n = ctx_pages<BS>(vctx[i], max_ctx), w = n > 0 ? n + flat_extra(sizeof(CT)) : 0, x = wave_scan(w);
+    const int n = ctx_pages<BS>(vctx[i], max_ctx), w = n > 0 ? n + flat_extra(sizeof(CT)) : 0, x = lane_scan(w);
     vbeg[i] = P + x - w;
     vend[i] = vbeg[i] + n;
     some[i] = __ballot(n > 0);

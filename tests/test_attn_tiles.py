@@ -144,6 +144,59 @@ def test_chunks_over_a_cached_prefix(Hq, Hkv, seqs):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("H,G,D,Dv,window,keep,seqs", [
+    (16, 4, 128, 128, 512, 4, [(0, 31), (0, 32), (0, 33), (20, 1100), (600, 65)]),      # two pages a step, an odd number of them last
+    (16, 4, 128, 128, 1 << 30, 0, [(1000 + i, 8) for i in range(65)]),      # more sequences than lanes, 31 to 33 pages in splits
+    (32, 8, 128, 128, 511, 70, [(0, 300), (1000, 200), (3, 40)]),             # one page a step
+    (6, 1, 256, 192, 1 << 30, 0, [(0, 140)] * 3 + [(33, 200)]),               # pages of uneven segments
+    (16, 4, 128, 128, 700, 4, [(1 + 13 * i, 1) for i in range(130)]),        # decoded rows of 130 sequences
+    (8, 2, 128, 128, 512, 40, [(2000, 1)]), (16, 1, 256, 192, 1 << 30, 0, [(300, 1), (5, 1), (0, 1)]),      # most splits without a page
+])
+def test_extended_tiles_match_dense_attention(H, G, D, Dv, window, keep, seqs):
+    g = torch.Generator().manual_seed(H + D + len(seqs))
+    bf = lambda *s: torch.randn(*s, generator=g).to(torch.bfloat16)                  # noqa: E731
+    dev, scale = "cuda", 2.0 / math.sqrt(D)
+    need = [(s + n + BS - 1) // BS for s, n in seqs]
+    order = torch.randperm(sum(need), generator=g)
+    kc, vc = bf(sum(need), G, BS, D), bf(sum(need), G, Dv, BS)
+    tables = torch.zeros(len(seqs), max(need) + 2, dtype=torch.int32)
+    qs, want, at = [], [], 0
+    for s, (start, n) in enumerate(seqs):
+        pages = order[at:at + need[s]]
+        at += need[s]
+        tables[s, :need[s]] = pages.int()
+        k = kc[pages].transpose(1, 2).reshape(-1, G, D)[:start + n]
+        v = vc[pages].permute(0, 3, 1, 2).reshape(-1, G, Dv)[:start + n]
+        qs.append(bf(n, H, D))
+        want.append(dense(qs[-1].to(F64), k.to(F64), v.to(F64), torch.arange(start, start + n), scale, window, keep, None, None, 0,
+                          None))
+    cu = torch.tensor([sum(n for _, n in seqs[:i]) for i in range(len(seqs) + 1)], dtype=torch.int32, device=dev)
+    pos = torch.cat([torch.arange(s, s + n) for s, n in seqs]).int().to(dev)
+    got = ops.attn_window_paged(torch.cat(qs).to(dev), kc.to(dev), vc.to(dev), tables.to(dev), cu, pos, scale, window, keep, None,
+                                dv_out=Dv)
+    err = (got.cpu().to(F64).view(-1, H, Dv) - torch.cat(want)).abs().max()
+    assert err < 2.0 ** -8 * vc.float().abs().max() + 1e-3      # weights and output rounded to bf16
+
+
+@pytest.mark.gpu
+def test_pages_that_no_row_of_a_wave_sees_do_not_count():
+    """Rows up to a page's end beside rows behind it in one workgroup, the next page's values no numbers."""
+    g = torch.Generator().manual_seed(1)
+    H, G, D, start, n, dev = 16, 4, 128, 20, 600, "cuda"
+    need = (start + n + BS - 1) // BS
+    kc, vc = (torch.randn(need, G, *s, generator=g).bfloat16() for s in ((BS, D), (D, BS)))
+    q, cu = torch.randn(n, H, D, generator=g).bfloat16().to(dev), torch.tensor([0, n], dtype=torch.int32, device=dev)
+    tables, pos = torch.arange(need, dtype=torch.int32, device=dev)[None], torch.arange(start, start + n).int().to(dev)
+    run = lambda v: ops.attn_window_paged(q, kc.to(dev), v.to(dev), tables, cu, pos, 0.1, 1 << 30, 0, None, dv_out=D)      # noqa: E731
+    clean = run(vc)
+    bad = vc.clone()
+    bad[1] = float("nan")
+    got = run(bad)
+    first = 8 * ((BS - start) // 8)      # (a wave has 32 rows: 8 tokens of 4 heads)
+    assert first and torch.equal(got[:first], clean[:first]) and got[BS - start:].isnan().all()
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("start,n,rest", [(2000, 64, 5), (5000, 300, 40), (100, 40, 3)])      # pages split over workgroups, and not
 def test_rows_of_no_sequence_stay(start, n, rest):
     """Rows before the first and after the last sequence keep what the output held, also where partial results are merged."""
