@@ -319,8 +319,7 @@ __device__ __forceinline__ bf16x8 lds_frag(const char* lds, int row, int chunk) 
 // `pslab`: this workgroup's split-K slab from row m0 on (nullptr: apply the epilogue).
 // `rsc`: RMSNorm row scale of a consumer GEMM (RowScale, ss == nullptr: none), applied to the
 // accumulators first, so split-K slabs, the bias and the SiLU all see the normalised rows.
-// PLAIN: the caller has applied EPI_BIAS and EPI_RELU2 itself.
-template <int TI, int TJ, bool PLAIN = false>
+template <int TI, int TJ>
 __device__ __forceinline__ void tile_epilogue(const f32x4 (&acc)[TI][TJ], int mw, int nw, int lane,
                                               int M, int N, int epi, const bf16* __restrict__ bias,
                                               bf16* __restrict__ out, long ldo, float* __restrict__ pslab,
@@ -388,11 +387,11 @@ __device__ __forceinline__ void tile_epilogue(const f32x4 (&acc)[TI][TJ], int mw
         }
       } else {
         f32x4 v = acc[i][j] * sc[i];
-        if (!PLAIN && epi == EPI_BIAS) {
+        if (epi == EPI_BIAS) {
 #pragma unroll
           for (int r = 0; r < 4; ++r) v[r] += bf2f(bias[n + r]);
         }
-        if (!PLAIN && epi == EPI_RELU2) {
+        if (epi == EPI_RELU2) {
 #pragma unroll
           for (int r = 0; r < 4; ++r) v[r] = fmaxf(v[r], 0.f) * fmaxf(v[r], 0.f);
         }
@@ -944,6 +943,7 @@ gemm_big8_kernel(const bf16* __restrict__ X, long ldx, const bf16* __restrict__ 
 // end on the barrier, A's DMA moved into ks 0, immediate-offset fragment addresses.
 // ---------------------------------------------------------------------------------------
 constexpr int kB4Threads = 256;
+constexpr int kB4Parts = -2;                       // in place of an epilogue: the sums of a part of K, in f32
 constexpr int kB4Slot = 256 * 128;                 // one operand half of a K-tile: 32 KiB
 constexpr int kB4LdsBytes = 5 * kB4Slot;           // A slots 0-2, B slots 3-4: 160 KiB
 
@@ -961,14 +961,82 @@ __device__ __forceinline__ void b4_dma(__amdgpu_buffer_rsrc_t r, char* lds, int 
 // [gate | up]), so the clamped GLU runs on a lane's own accumulators; an expert that runs on (score x row) scales
 // the accumulators by the score instead of rounding scaled rows. The down projection leaves f32 rows at their
 // (token, choice) pair. Measured beside the smaller tiles: moe_tile_rows.
-// E: the epilogue (-1: `epi`), in instances of their own because the branches of the others cost each of them up to 3 us, and
-// with every epilogue added more (8192 x 57344 x 8192 SwiGLU 5050 us with four of them, 5066 with five, 5028 alone).
-// EPI_BIAS reads the columns' values once for all rows (row by row in tile_epilogue, each load waited for by the only wave of its
+// E: the epilogue, or kB4Parts, in instances of their own because the branches of the others cost each of them up to 3 us, and
+// with every epilogue added more (8192 x 57344 x 8192 SwiGLU 5050 us with four of them, 5066 with five, 5028 alone); two that share
+// one also spill. EPI_BIAS reads the columns' values once for all rows (row by row, each load waited for by the only wave of its
 // SIMD, they took 13 to 50 us of a product).
+// The results leave through LDS: an MFMA leaves a lane 4 columns of a row, so that a store straight from the accumulators writes 16 rows
+// of 32 bytes (64 in f32), and the last level's cache reads a line it does not hold before it takes a part of it. A wave puts its
+// rows into its own piece of the rings (free behind the last K-tile) and stores them as whole lines, 16 bytes a lane. Before and
+// after, us: 8192 x 8192 x 512 88 and 76, x 2048 214 and 204, 8192 x 16384 x 2048 (268 MB of results) 580 and 410, with SwiGLU 407
+// and 390, 6184 x 8448 x 2048 184 and 170, 937 x 6144 x 4096 53 and 50. Non-temporal stores from there: 8192 x 8192 x 512 75 -> 86,
+// the others level.
+// ROWS rows of RB bytes, one every RB + 16: at row(r) each, while r < left. `whole`: rows that are aligned to 16 bytes.
+template <int RB, int ROWS, class Row>
+__device__ __forceinline__ void b4_rows_out(const char* piece, int lane, int left, bool whole, Row&& row) {
+  constexpr int LPR = RB / 16, RPI = 64 / LPR;      // lanes of a row, rows of an instruction
+  const int r0 = lane / LPR, c = (lane % LPR) * 16;
+  static_assert(ROWS % (8 * RPI) == 0, "");
+#pragma unroll
+  for (int r = 0; r < ROWS; r += 8 * RPI) {
+    f32x4 v[8];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) v[q] = *reinterpret_cast<const f32x4*>(piece + (r + r0 + q * RPI) * (RB + 16) + c);
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      const int rq = r + r0 + q * RPI;
+      char* to = row(rq) + c;      // (by all lanes: they may hold it for each other)
+      if (rq >= left) continue;
+      if (whole) {
+        *reinterpret_cast<f32x4*>(to) = v[q];
+      } else {
+        const bf16x8 e = __builtin_bit_cast(bf16x8, v[q]);
+#pragma unroll
+        for (int x = 0; x < 8; ++x) reinterpret_cast<bf16*>(to)[x] = e[x];
+      }
+    }
+  }
+}
+
+// RI x NJ blocks of 16 x 16 results, value(i, j) a lane's four of one, as bf16 rows from dst on
+template <int RI, int NJ, class Value>
+__device__ __forceinline__ void b4_out(char* smem, int wid, int lane, int left, bf16* dst, long ldo, Value&& value) {
+  constexpr int RB = 32 * NJ;
+  char* piece = smem + wid * 16 * RI * (RB + 16);
+  char* at = piece + (lane & 15) * (RB + 16) + 8 * (lane >> 4);
+#pragma unroll
+  for (int i = 0; i < RI; ++i)
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+      const f32x4 v = value(i, j);
+      bf16x4 w;
+#pragma unroll
+      for (int x = 0; x < 4; ++x) w[x] = f2bf(v[x]);
+      *reinterpret_cast<bf16x4*>(at + 16 * i * (RB + 16) + 32 * j) = w;
+    }
+  const bool whole = (ldo & 7) == 0 && (reinterpret_cast<uintptr_t>(dst) & 15) == 0;
+  b4_rows_out<RB, 16 * RI>(piece, lane, left, whole, [&](int r) { return reinterpret_cast<char*>(dst + r * ldo); });
+}
+
+// The same in f32, 64 rows at a time: row r of the q-th 64 at row(q, r)
+template <int RI, class Row>
+__device__ __forceinline__ void b4_out_f32(char* smem, int wid, int lane, int left, const f32x4 (&acc)[RI][8], Row&& row) {
+  char* piece = smem + wid * 64 * 528;
+  char* at = piece + (lane & 15) * 528 + 16 * (lane >> 4);
+#pragma unroll
+  for (int h = 0; h < RI; h += 4) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int j = 0; j < 8; ++j) *reinterpret_cast<f32x4*>(at + 16 * i * 528 + 64 * j) = acc[h + i][j];
+    b4_rows_out<512, 64>(piece, lane, left - 16 * h, true, [&](int r) { return reinterpret_cast<char*>(row(h / 4, r)); });
+  }
+}
+
 // One tile of BM rows (256, or 128: half of one) and 256 columns from row m0 of rows below M and column n0 on.
 template <int GROUPED, int E, int BM>
 __device__ __forceinline__ void big4_tile(const bf16* __restrict__ X, long ldx, const bf16* __restrict__ W, long ldw, int m0,
-                                          int M, int n0, int N, int K, int epi, const bf16* __restrict__ bias,
+                                          int M, int n0, int N, int K, const bf16* __restrict__ bias,
                                           bf16* __restrict__ out, long ldo, float* __restrict__ part,
                                           const int* __restrict__ grows, const ExpertArgs& ex) {
   constexpr int RI = BM / 32;      // a wave's row blocks of 16, and its DMA instructions for a slot of A
@@ -1115,73 +1183,81 @@ __device__ __forceinline__ void big4_tile(const bf16* __restrict__ X, long ldx, 
   }
   ks1(nk - 1, sa, SB == 2 ? (nk - 1) & 1 : sbk, sa == SA - 1 ? 0 : sa + 1);
   vm_wait<0>();                       // no LDS-DMA may outlive the workgroup
-  if constexpr (GROUPED >= 2) {
+  __builtin_amdgcn_s_barrier();       // every wave has read the last K-tile: the rings are free
+  int el = lane;
+  asm volatile("" : "+v"(el));        // (nothing of what follows is computed ahead of the K loop)
+  const int mw = m0 + wr * (BM / 2), nw = n0 + wc * 128, left = M - mw;      // the wave's block and its rows
+  if constexpr (GROUPED == 3) {
+    int pairs[RI / 4];      // the (token, choice) pairs of a lane's rows
+#pragma unroll
+    for (int q = 0; q < RI / 4; ++q) pairs[q] = ex.perm[min(mw + 64 * q + el, M - 1)];
+    b4_out_f32<RI>(smem, wid, el, left, acc, [&](int q, int r) { return ex.y + (long)__shfl(pairs[q], r, 64) * ldo + nw; });
+    return;
+  } else if constexpr (GROUPED == 2) {
+    float sc[RI];
 #pragma unroll
     for (int i = 0; i < RI; ++i) {
-      const int r = m0 + wr * (BM / 2) + 16 * i + fr;
-      if (r >= M) continue;
-      const int p = ex.perm[r];
-      if constexpr (GROUPED == 3) {
-        float* yr = ex.y + (long)p * ldo + n0 + wc * 128 + 4 * fq;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) *reinterpret_cast<f32x4*>(yr + 16 * j) = acc[i][j];
-      } else {
-        const float sc = ex.topk_w ? ex.topk_w[p] : 1.f;
-        if (ex.plain) {      // squared ReLU
-          bf16* hr = out + (long)r * ldo + n0 + wc * 128 + 4 * fq;
-#pragma unroll
-          for (int j = 0; j < 8; ++j) {
-            bf16x4 w;
-#pragma unroll
-            for (int x = 0; x < 4; ++x) {
-              const float v = fmaxf(acc[i][j][x] * sc, 0.f);
-              w[x] = (bf16)(v * v);
-            }
-            *reinterpret_cast<bf16x4*>(hr + 16 * j) = w;
-          }
-        } else {
-          bf16* hr = out + (long)r * ldo + (n0 >> 1) + wc * 64 + 4 * fq;
-#pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            bf16x4 w;
-#pragma unroll
-            for (int x = 0; x < 4; ++x) {
-              const float g = fminf(acc[i][j][x] * sc, ex.limit);
-              const float u = fminf(fmaxf(acc[i][j + 4][x] * sc, -ex.limit), ex.limit);
-              w[x] = (bf16)(glu_gate(g, ex.alpha, __expf(-ex.alpha * g)) * (u + ex.up_offset));
-            }
-            *reinterpret_cast<bf16x4*>(hr + 16 * j) = w;
-          }
-        }
-      }
+      const int r = 16 * i + (el & 15);
+      sc[i] = ex.topk_w && r < left ? ex.topk_w[ex.perm[mw + r]] : 1.f;
     }
+    if (ex.plain)      // squared ReLU
+      b4_out<RI, 8>(smem, wid, el, left, out + (long)mw * ldo + nw, ldo, [&](int i, int j) {
+        f32x4 v;
+#pragma unroll
+        for (int x = 0; x < 4; ++x) v[x] = fmaxf(acc[i][j][x] * sc[i], 0.f);
+        return v * v;
+      });
+    else
+      b4_out<RI, 4>(smem, wid, el, left, out + (long)mw * ldo + (nw >> 1), ldo, [&](int i, int j) {
+        f32x4 v;
+#pragma unroll
+        for (int x = 0; x < 4; ++x) {
+          const float g = fminf(acc[i][j][x] * sc[i], ex.limit);
+          const float u = fminf(fmaxf(acc[i][j + 4][x] * sc[i], -ex.limit), ex.limit);
+          v[x] = glu_gate(g, ex.alpha, __expf(-ex.alpha * g)) * (u + ex.up_offset);
+        }
+        return v;
+      });
     return;
   }
   if (n0 + wc * 128 >= N) return;     // the columns past N of a half tile (their weight rows read zeros)
-  if constexpr (E >= 0) epi = E;
-  if constexpr (E == EPI_RELU2) {
+  if constexpr (E == kB4Parts) {
+    float* slab = part + (long)blockIdx.y * M * N;
+    b4_out_f32<RI>(smem, wid, el, left, acc, [&](int q, int r) { return slab + (long)(mw + 64 * q + r) * N + nw; });
+  } else if constexpr (E == EPI_SILU || E == EPI_GLU) {      // the wave's column blocks are gate and up in turn
+    const GluPar gp = E == EPI_GLU ? glu_par(bias, N) : GluPar{};
+    b4_out<RI, 4>(smem, wid, el, left, out + (long)mw * ldo + (nw >> 1), ldo, [&](int i, int j) {
+      f32x4 v;
 #pragma unroll
-    for (int i = 0; i < RI; ++i)
+      for (int x = 0; x < 4; ++x) {
+        const float g = acc[i][2 * j][x], u = acc[i][2 * j + 1][x];
+        if constexpr (E == EPI_GLU) {
+          const bf16* b = bias + nw + 32 * j + 4 * (el >> 4) + x;
+          v[x] = glu_clamped(g + bf2f(b[0]), u + bf2f(b[16]), gp);
+        } else {
+          v[x] = silu(g) * u;
+        }
+      }
+      return v;
+    });
+  } else {
+    f32x4 b[8] = {};
+    if constexpr (E == EPI_BIAS) {
 #pragma unroll
       for (int j = 0; j < 8; ++j)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) acc[i][j][r] = fmaxf(acc[i][j][r], 0.f) * fmaxf(acc[i][j][r], 0.f);
-    epi = EPI_NONE;
-  }
-  if constexpr (E == EPI_BIAS) {
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      f32x4 b;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) b[r] = bf2f(bias[n0 + wc * 128 + 16 * j + 4 * fq + r]);
-#pragma unroll
-      for (int i = 0; i < RI; ++i) acc[i][j] += b;
+        for (int x = 0; x < 4; ++x) b[j][x] = bf2f(bias[nw + 16 * j + 4 * (el >> 4) + x]);
     }
-    epi = EPI_NONE;
+    b4_out<RI, 8>(smem, wid, el, left, out + (long)mw * ldo + nw, ldo, [&](int i, int j) {
+      f32x4 v = acc[i][j];
+      if constexpr (E == EPI_BIAS) v += b[j];
+      if constexpr (E == EPI_RELU2) {
+#pragma unroll
+        for (int x = 0; x < 4; ++x) v[x] = fmaxf(v[x], 0.f) * fmaxf(v[x], 0.f);
+      }
+      return v;
+    });
   }
-  tile_epilogue<RI, 8, GROUPED == 0>(acc, m0 + wr * (BM / 2), n0 + wc * 128, lane, M, N, epi, bias, out, ldo,
-                      part ? part + (long)blockIdx.y * M * N + (long)m0 * N : nullptr, m0,
-                      RowScale{nullptr, 0, 0.f, 0.f});
 }
 
 // Tiles at the end of the walk that run as two halves of 128 rows each: those of a last round of 256 workgroups that would leave
@@ -1192,10 +1268,10 @@ __device__ __forceinline__ void big4_tile(const bf16* __restrict__ X, long ldx, 
 // tiles everywhere.
 __host__ __device__ __forceinline__ int big4_halved(int tiles) { return tiles % 256 <= 128 ? tiles % 256 : 0; }
 
-template <int GROUPED = 0, int E = -1>
+template <int GROUPED, int E>
 __global__ void __launch_bounds__(kB4Threads) __attribute__((amdgpu_waves_per_eu(1, 1)))
 gemm_big4_kernel(const bf16* __restrict__ X, long ldx, const bf16* __restrict__ W, long ldw,
-                 int M, int N, int K, int epi, const bf16* __restrict__ bias,
+                 int M, int N, int K, const bf16* __restrict__ bias,
                  bf16* __restrict__ out, long ldo, float* __restrict__ part, int halved = 0,
                  const int* __restrict__ grows = nullptr, const int4* __restrict__ gtiles = nullptr,
                  const int* __restrict__ gcount = nullptr, long w_estride = 0, ExpertArgs ex = ExpertArgs()) {
@@ -1239,9 +1315,9 @@ gemm_big4_kernel(const bf16* __restrict__ X, long ldx, const bf16* __restrict__ 
     if (m0 >= M) return;
   }
   if (M - m0 <= BM / 2)
-    big4_tile<GROUPED, E, BM / 2>(X, ldx, W, ldw, m0, M, n0, N, K, epi, bias, out, ldo, part, grows, ex);
+    big4_tile<GROUPED, E, BM / 2>(X, ldx, W, ldw, m0, M, n0, N, K, bias, out, ldo, part, grows, ex);
   else
-    big4_tile<GROUPED, E, BM>(X, ldx, W, ldw, m0, M, n0, N, K, epi, bias, out, ldo, part, grows, ex);
+    big4_tile<GROUPED, E, BM>(X, ldx, W, ldw, m0, M, n0, N, K, bias, out, ldo, part, grows, ex);
 }
 
 // ---------------------------------------------------------------------------------------
@@ -1708,14 +1784,15 @@ static void run_big4(const bf16* X, long ldx, const bf16* W, long ldw, int M, in
                           hipFuncAttributeMaxDynamicSharedMemorySize, kB4LdsBytes);                                      \
       attr_set = true;                                                                                                   \
     }                                                                                                                    \
-    gemm_big4_kernel<0, E><<<grid, kB4Threads, kB4LdsBytes, stream>>>(X, ldx, W, ldw, M, N, K, epi, bias, out, ldo, part, \
+    gemm_big4_kernel<0, E><<<grid, kB4Threads, kB4LdsBytes, stream>>>(X, ldx, W, ldw, M, N, K, bias, out, ldo, part, \
                                                                       halved);                                           \
   }
-  if (sk > 1 || epi == EPI_NONE) BFLY_BIG4(EPI_NONE)      // (with a split K the reduce applies the epilogue)
+  if (sk > 1) BFLY_BIG4(kB4Parts)      // (the reduce applies the epilogue)
+  else if (epi == EPI_NONE) BFLY_BIG4(EPI_NONE)
   else if (epi == EPI_SILU) BFLY_BIG4(EPI_SILU)
   else if (epi == EPI_BIAS) BFLY_BIG4(EPI_BIAS)
   else if (epi == EPI_RELU2) BFLY_BIG4(EPI_RELU2)
-  else BFLY_BIG4(-1)
+  else BFLY_BIG4(EPI_GLU)
 #undef BFLY_BIG4
 }
 
@@ -2138,14 +2215,16 @@ int launch_gemm_grouped(const bf16* X, long x_rows, long ldx, const bf16* W, lon
     if (!attr) {
       hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_big8_kernel<true>),
                           hipFuncAttributeMaxDynamicSharedMemorySize, kB8LdsBytes);
-      hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_big4_kernel<1>),
-                          hipFuncAttributeMaxDynamicSharedMemorySize, kB4LdsBytes);
+      for (const void* k : {reinterpret_cast<const void*>(&gemm_big4_kernel<1, EPI_NONE>),
+                            reinterpret_cast<const void*>(&gemm_big4_kernel<1, EPI_SILU>)})
+        hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, kB4LdsBytes);
       attr = true;
     }
     dim3 grid(max_tiles * (N / 256), 1);
     if (grouped_on_big4(x_rows, ldx, ldw, epi == EPI_SILU, rows != nullptr))
-      gemm_big4_kernel<1><<<dim3(max_tiles * (N / 256) + 128), kB4Threads, kB4LdsBytes, stream>>>(
-          X, ldx, W, ldw, 0, N, K, epi, nullptr, out, ldo, nullptr, 0, rows, tiles, count, w_estride);
+      (epi == EPI_SILU ? &gemm_big4_kernel<1, EPI_SILU> : &gemm_big4_kernel<1, EPI_NONE>)
+          <<<dim3(max_tiles * (N / 256) + 128), kB4Threads, kB4LdsBytes, stream>>>(
+              X, ldx, W, ldw, 0, N, K, nullptr, out, ldo, nullptr, 0, rows, tiles, count, w_estride, ExpertArgs());
     else
       gemm_big8_kernel<true><<<grid, kB8Threads, kB8LdsBytes, stream>>>(
           X, ldx, W, ldw, max_tiles * 256, N, K, epi, nullptr, out, ldo, nullptr, rows, tiles, count, w_estride);
@@ -2165,18 +2244,18 @@ void launch_moe_big(bool down, const bf16* X, long ldx, const bf16* W, int N, in
                     bf16* out, long ldo, const ExpertArgs& ex, hipStream_t stream) {
   static bool attr = false;
   if (!attr) {
-    hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_big4_kernel<2>), hipFuncAttributeMaxDynamicSharedMemorySize,
+    hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_big4_kernel<2, EPI_NONE>), hipFuncAttributeMaxDynamicSharedMemorySize,
                         kB4LdsBytes);
-    hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_big4_kernel<3>), hipFuncAttributeMaxDynamicSharedMemorySize,
+    hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_big4_kernel<3, EPI_NONE>), hipFuncAttributeMaxDynamicSharedMemorySize,
                         kB4LdsBytes);
     attr = true;
   }
   const dim3 grid(max_tiles * (N / 256) + 128, 1);      // (the kernel counts the tiles and halves up to 128 of them)
   if (down)
-    gemm_big4_kernel<3><<<grid, kB4Threads, kB4LdsBytes, stream>>>(X, ldx, W, K, 0, N, K, EPI_NONE, nullptr, out, ldo, nullptr, 0,
+    gemm_big4_kernel<3, EPI_NONE><<<grid, kB4Threads, kB4LdsBytes, stream>>>(X, ldx, W, K, 0, N, K, nullptr, out, ldo, nullptr, 0,
                                                                    nullptr, nullptr, ntiles, (long)N * K, ex);
   else
-    gemm_big4_kernel<2><<<grid, kB4Threads, kB4LdsBytes, stream>>>(X, ldx, W, K, 0, N, K, EPI_NONE, nullptr, out, ldo, nullptr, 0,
+    gemm_big4_kernel<2, EPI_NONE><<<grid, kB4Threads, kB4LdsBytes, stream>>>(X, ldx, W, K, 0, N, K, nullptr, out, ldo, nullptr, 0,
                                                                    nullptr, nullptr, ntiles, (long)N * K, ex);
 }
 

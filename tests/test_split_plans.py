@@ -101,3 +101,32 @@ def test_row_scaled_product_with_a_half_column_tile(M, N, K, how):
         want = (torch.nn.functional.silu(u[:, :, 0]) * u[:, :, 1]).reshape(M, N // 2)
     # one rounding to bf16 (2^-9) of f32 sums of unit-sized products
     assert ((got - want).abs() < 2.0 ** -8 * want.abs() + 1e-4).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(4100, 1024, 512), (4225, 4224, 1024), (2300, 2560, 192), (1100, 4096, 14336)])
+@pytest.mark.parametrize("epi", ["none", "bias", "silu", "relu2", "glu"])
+def test_results_of_the_large_tile_into_any_rows(M, N, K, epi):
+    """A short last row tile, a half column tile, half tiles, split K: rows of any stride and alignment take the same values and
+    nothing beside them is written."""
+    assert ops.gemm_plan(M, N, K)["kind"] == "big4"
+    g = torch.Generator(device="cuda").manual_seed(M + N)
+    x, w, b = (torch.randn(*s, device="cuda", generator=g).to(torch.bfloat16) for s in ((M, K), (N, K), (N,)))
+    w = w * K ** -0.5
+    bias = {"bias": b, "glu": ops.glu_bias_block(b, 7.0, 1.702, 1.0)}.get(epi)
+    name = "none" if epi == "bias" else epi
+    n = N // 2 if epi in ("silu", "glu") else N
+    want = ops.linear(x, w, bias=bias, epilogue=name)
+    for first, ld in ((0, n + 8), (8, n + 24), (4, n + 4), (1, n + 1), (3, n + 16)):
+        buf = torch.full((M, ld), 77.0, device="cuda", dtype=torch.bfloat16)
+        ops.linear(x, w, bias=bias, epilogue=name, out=buf[:, first:first + n])
+        assert torch.equal(buf[:, first:first + n], want), (first, ld)
+        assert (buf[:, :first] == 77).all() and (buf[:, first + n:] == 77).all(), (first, ld)
+    s = x.float() @ w.float().t()
+    size = x.float().abs() @ w.float().abs().t()          # sums of K products: 2^-24 of it a step, at most, in any order
+    if epi in ("none", "bias"):
+        s = s + (b.float() if epi == "bias" else 0)
+        assert ((want.float() - s).abs() <= 2.0 ** -8 * s.abs() + K * 2.0 ** -24 * size).all()
+    elif epi == "relu2":
+        r, d = s.clamp_min(0), K * 2.0 ** -24 * size
+        assert ((want.float() - r * r).abs() <= 2.0 ** -8 * (r + d) ** 2 + 2 * r * d + d * d).all()
