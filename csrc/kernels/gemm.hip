@@ -934,8 +934,8 @@ gemm_big8_kernel(const bf16* __restrict__ X, long ldx, const bf16* __restrict__ 
 // every other slot} fenced by sched_barrier(0) (cdna_hip_programming.md T19: left alone, the
 // scheduler clusters the memory operations, and a lone wave has nothing to hide the stall
 // behind). A lane's fragments of one (slot, ks) share one address VGPR (immediate offsets: 4
-// VALU per K-tile). Branch-free: past the last K-tile the DMA re-reads it into a slot nobody
-// reads any more (a guard made hipcc wait vmcnt(0) per slot: 3.5x slower).
+// VALU per K-tile). No guards: past the last K-tile the DMA takes the next tile's first ones, or
+// this tile's once more for nobody (a guard made hipcc wait vmcnt(0) per slot: 3.5x slower).
 // Measured (profiles/r5_gemm_big4/): 1.52-1.55 PF at M = 8192 on the Llama-3-70B projections
 // against 1.39-1.47 for gemm_big8_kernel and 1.53-1.64 for hipBLASLt on the same box. Steps that
 // got it there from 1.0 PF: LDS-DMA rings instead of register staging (no accumulator moves),
@@ -971,244 +971,119 @@ __device__ __forceinline__ void b4_dma(__amdgpu_buffer_rsrc_t r, char* lds, int 
 // after, us: 8192 x 8192 x 512 88 and 76, x 2048 214 and 204, 8192 x 16384 x 2048 (268 MB of results) 580 and 410, with SwiGLU 407
 // and 390, 6184 x 8448 x 2048 184 and 170, 937 x 6144 x 4096 53 and 50. Non-temporal stores from there: 8192 x 8192 x 512 75 -> 86,
 // the others level.
-// ROWS rows of RB bytes, one every RB + 16: at row(r) each, while r < left. `whole`: rows that are aligned to 16 bytes.
-template <int RB, int ROWS, class Row>
-__device__ __forceinline__ void b4_rows_out(const char* piece, int lane, int left, bool whole, Row&& row) {
-  constexpr int LPR = RB / 16, RPI = 64 / LPR;      // lanes of a row, rows of an instruction
-  const int r0 = lane / LPR, c = (lane % LPR) * 16;
-  static_assert(ROWS % (8 * RPI) == 0, "");
+typedef unsigned u32x4_b4 __attribute__((ext_vector_type(4)));
+typedef unsigned short u16x8_b4 __attribute__((ext_vector_type(8)));
+
+// A wave's piece is 8 KB. Rows of RB bytes, their 16-byte chunks turned by the row so that both ways meet every bank alike.
+template <int RB>
+__device__ __forceinline__ int b4_place(int row, int chunk) {
+  return row * RB + 16 * (chunk ^ (RB == 128 ? (row >> 1) & 7 : row & 15));
+}
+
+// What a lane holds of the piece's rows: 16 bytes at chunk lane % LPR of row lane / LPR + q RPI
+template <int RB>
+struct B4Rows {
+  static constexpr int LPR = RB / 16, RPI = 64 / LPR;      // lanes of a row, rows of an instruction
+  f32x4 v[8];
+  __device__ __forceinline__ B4Rows(const char* piece, int lane) {
 #pragma unroll
-  for (int r = 0; r < ROWS; r += 8 * RPI) {
-    f32x4 v[8];
-#pragma unroll
-    for (int q = 0; q < 8; ++q) v[q] = *reinterpret_cast<const f32x4*>(piece + (r + r0 + q * RPI) * (RB + 16) + c);
+    for (int q = 0; q < 8; ++q) v[q] = *reinterpret_cast<const f32x4*>(piece + b4_place<RB>(lane / LPR + q * RPI, lane % LPR));
+  }
+  // at base + row * stride bytes, rows below left: branches over the last ones would be taken 32 times. `whole`: rows that are
+  // aligned to 16 bytes.
+  __device__ __forceinline__ void out(__amdgpu_buffer_rsrc_t to, int lane, int row0, int left, int stride, bool whole) const {
+    int off[8];
 #pragma unroll
     for (int q = 0; q < 8; ++q) {
-      const int rq = r + r0 + q * RPI;
-      char* to = row(rq) + c;      // (by all lanes: they may hold it for each other)
-      if (rq >= left) continue;
-      if (whole) {
-        *reinterpret_cast<f32x4*>(to) = v[q];
-      } else {
-        const bf16x8 e = __builtin_bit_cast(bf16x8, v[q]);
+      const int r = row0 + lane / LPR + q * RPI;
+      off[q] = r < left ? r * stride + 16 * (lane % LPR) : -1;      // (past every bound)
+    }
+    if (whole) {
 #pragma unroll
-        for (int x = 0; x < 8; ++x) reinterpret_cast<bf16*>(to)[x] = e[x];
-      }
+      for (int q = 0; q < 8; ++q) __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_b4, v[q]), to, off[q], 0, 0);
+    } else {
+#pragma unroll
+      for (int q = 0; q < 8; ++q)
+#pragma unroll
+        for (int x = 0; x < 8; ++x)
+          __builtin_amdgcn_raw_buffer_store_b16(__builtin_bit_cast(u16x8_b4, v[q])[x], to, off[q] < 0 ? -1 : off[q] + 2 * x, 0, 0);
     }
   }
-}
+};
 
 // RI x NJ blocks of 16 x 16 results, value(i, j) a lane's four of one, as bf16 rows from dst on
 template <int RI, int NJ, class Value>
-__device__ __forceinline__ void b4_out(char* smem, int wid, int lane, int left, bf16* dst, long ldo, Value&& value) {
-  constexpr int RB = 32 * NJ;
-  char* piece = smem + wid * 16 * RI * (RB + 16);
-  char* at = piece + (lane & 15) * (RB + 16) + 8 * (lane >> 4);
-#pragma unroll
-  for (int i = 0; i < RI; ++i)
-#pragma unroll
-    for (int j = 0; j < NJ; ++j) {
-      const f32x4 v = value(i, j);
-      bf16x4 w;
-#pragma unroll
-      for (int x = 0; x < 4; ++x) w[x] = f2bf(v[x]);
-      *reinterpret_cast<bf16x4*>(at + 16 * i * (RB + 16) + 32 * j) = w;
-    }
+__device__ __forceinline__ void b4_out(char* piece, int lane, int left, bf16* dst, long ldo, Value&& value) {
+  constexpr int RB = 32 * NJ, RP = 8192 / RB / 16;      // row blocks of a piece
   const bool whole = (ldo & 7) == 0 && (reinterpret_cast<uintptr_t>(dst) & 15) == 0;
-  b4_rows_out<RB, 16 * RI>(piece, lane, left, whole, [&](int r) { return reinterpret_cast<char*>(dst + r * ldo); });
+  const auto to = __builtin_amdgcn_make_buffer_rsrc((void*)dst, (short)0, 0x7fffffff, 0x00020000);
+#pragma unroll
+  for (int h = 0; h < RI; h += RP) {
+#pragma unroll
+    for (int i = 0; i < RP; ++i) {
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) {
+        const f32x4 v = value(h + i, j);
+        bf16x4 w;
+#pragma unroll
+        for (int x = 0; x < 4; ++x) w[x] = f2bf(v[x]);
+        *reinterpret_cast<bf16x4*>(piece + b4_place<RB>(16 * i + (lane & 15), 2 * j + (lane >> 5)) + 8 * (lane >> 4 & 1)) = w;
+        if (j & 1) __builtin_amdgcn_sched_barrier(0);      // (a few values at a time: together they do not fit)
+      }
+    }
+    B4Rows<RB>(piece, lane).out(to, lane, 16 * h, left, (int)(ldo * 2), whole);
+    __builtin_amdgcn_sched_barrier(0);
+  }
 }
 
-// The same in f32, 64 rows at a time: row r of the q-th 64 at row(q, r)
-template <int RI, class Row>
-__device__ __forceinline__ void b4_out_f32(char* smem, int wid, int lane, int left, const f32x4 (&acc)[RI][8], Row&& row) {
-  char* piece = smem + wid * 64 * 528;
-  char* at = piece + (lane & 15) * 528 + 16 * (lane >> 4);
+// Row block i of f32 results into the piece
+template <int RI>
+__device__ __forceinline__ B4Rows<512> b4_rows_f32(char* piece, int lane, const f32x4 (&acc)[RI][8], int i) {
 #pragma unroll
-  for (int h = 0; h < RI; h += 4) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-      for (int j = 0; j < 8; ++j) *reinterpret_cast<f32x4*>(at + 16 * i * 528 + 64 * j) = acc[h + i][j];
-    b4_rows_out<512, 64>(piece, lane, left - 16 * h, true, [&](int r) { return reinterpret_cast<char*>(row(h / 4, r)); });
-  }
+  for (int j = 0; j < 8; ++j) *reinterpret_cast<f32x4*>(piece + b4_place<512>(lane & 15, 4 * j + (lane >> 4))) = acc[i][j];
+  return B4Rows<512>(piece, lane);
 }
 
-// One tile of BM rows (256, or 128: half of one) and 256 columns from row m0 of rows below M and column n0 on.
-template <int GROUPED, int E, int BM>
-__device__ __forceinline__ void big4_tile(const bf16* __restrict__ X, long ldx, const bf16* __restrict__ W, long ldw, int m0,
-                                          int M, int n0, int N, int K, const bf16* __restrict__ bias,
-                                          bf16* __restrict__ out, long ldo, float* __restrict__ part,
-                                          const int* __restrict__ grows, const ExpertArgs& ex) {
-  constexpr int RI = BM / 32;      // a wave's row blocks of 16, and its DMA instructions for a slot of A
-  // Slots of the rings and their places: a half tile's products cover half of the latency only, and its smaller slots leave room
-  // for one more of each.
-  constexpr int SA = BM == 256 ? 3 : 4, SB = BM == 256 ? 2 : 3, kSlotA = BM * 128, kRingB = SA * kSlotA;
-  extern __shared__ __attribute__((aligned(16))) char smem[];
-  // wave index in an SGPR: the DMA's LDS destinations (M0) and the fragment row bases are then
-  // scalar (a VGPR wave index cost a readfirstlane + s_nop per DMA instruction)
-  const int tid = threadIdx.x, lane = tid & 63, wid = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wr = wid >> 1, wc = wid & 1;
-  const int ktiles = K / 64;
-  const int kt0 = (int)(((long)ktiles * blockIdx.y) / gridDim.y);
-  const int kt1 = (int)(((long)ktiles * (blockIdx.y + 1)) / gridDim.y);
-  const int nk = kt1 - kt0;   // >= 2 (host check)
+// What a workgroup runs: lane i holds its i-th tile, rows [m0, end) and columns from n0 on, of expert e (GROUPED)
+struct B4Items {
+  int m0, end, n0, e;
+};
 
-  // DMA: instruction s (0..7) of wave w fills LDS row block 8 w + s (8 rows x 128 B, lane-
-  // linear); lane L supplies row 8 (8 w + s) + (L >> 3) at the chunk lds_frag expects in
-  // position L & 7: chunk = (L & 7) ^ ((row >> 1) & 7) = (L & 7) ^ ((L >> 4) + 4 (s & 1)) & 7
-  const auto rsa = b8_rsrc(X + (long)m0 * ldx, M - m0, ldx);   // A rows past M read zeros
-  const bool glu = GROUPED == 2 && !ex.plain;
-  const auto rsb = glu ? b8_rsrc(W, N, ldw) : b8_rsrc(W + (long)n0 * ldw, N - n0, ldw);
-  const int drow = 64 * wid + (lane >> 3), arow = 8 * RI * wid + (lane >> 3);
-  // weight row of LDS row drow: with a gate, waves 0 / 2 stage gate rows and 1 / 3 the up rows of the same columns
-  const int brow = glu ? (wid & 1) * (N >> 1) + (n0 >> 1) + (wid >> 1) * 64 + (lane >> 3) : drow;
-  int va[2], vb[2];
-#pragma unroll
-  for (int e = 0; e < 2; ++e) {
-    const int ch = (lane & 7) ^ (((lane >> 4) + 4 * e) & 7);
-    va[e] = (int)((arow * ldx + ch * 8) * 2);
-    vb[e] = (int)((brow * ldw + ch * 8) * 2);
-  }
-  // GROUPED: byte offsets of this lane's rows (at its chunk), from X where they are gathered (X has less than 2 GB:
-  // grouped_on_big4, moe_big_ok), from the tile's first row where they follow one another (slots know no such bound)
-  int ga[RI] = {};
-  const bool gather = GROUPED == 2 || grows != nullptr;
-  const auto rsx = b8_rsrc(gather ? X : X + (long)m0 * ldx, 1L << 30, 1);
-  if constexpr (GROUPED == 1 || GROUPED == 2) {
-#pragma unroll
-    for (int q = 0; q < RI; ++q) {
-      const int slot = min(m0 + arow + 8 * q, M - 1);
-      const long src = GROUPED == 2 ? ex.perm[slot] / ex.choices : gather ? grows[slot] : slot - m0;
-      ga[q] = (int)((src * ldx + (((lane & 7) ^ (((lane >> 4) + 4 * (q & 1)) & 7)) * 8)) * 2);
-    }
-  }
-  auto dma_a = [&](int k, int slot, int s) {
-    if constexpr (GROUPED == 1 || GROUPED == 2)
-      b4_dma(rsx, smem + slot * kSlotA + (RI * wid + s) * 1024, ga[s], (kt0 + k) * 128);
-    else
-      b4_dma(rsa, smem + slot * kSlotA + (RI * wid + s) * 1024, va[s & 1], (kt0 + k) * 128 + (int)(8 * s * ldx * 2));
-  };
-  auto dma_b = [&](int k, int slot, int s) {
-    b4_dma(rsb, smem + kRingB + slot * kB4Slot + (8 * wid + s) * 1024, vb[s & 1], (kt0 + k) * 128 + (int)(8 * s * ldw * 2));
-  };
-  const int fr = lane & 15, fq = lane >> 4;
-  // fragment idx 0-7: B rows (output columns) 16 idx, 8-15: A rows 16 (idx - 8), of k-step ks.
-  // lds_frag's swizzle depends on row bits 1-3 = fr bits 1-3 only, so a lane's fragments of one
-  // (slot, ks) share one VGPR address and differ by immediates of 2048 B (16 rows)
-  int lo[2][2];   // [operand A / B][ks] lane byte offset inside a slot
-#pragma unroll
-  for (int ks = 0; ks < 2; ++ks) {
-    const int ch = ((ks * 4 + fq) ^ ((fr >> 1) & 7)) * 16;
-    lo[0][ks] = (wr * (BM / 2) + fr) * 128 + ch;
-    lo[1][ks] = (wc * 128 + fr) * 128 + ch;
-  }
-  auto rd1 = [&](int sa_, int sb_, int ks, int idx, bf16x8 (&f)[8 + RI]) {
-    const char* p = idx < 8 ? smem + kRingB + sb_ * kB4Slot + lo[1][ks] + 2048 * idx
-                            : smem + sa_ * kSlotA + lo[0][ks] + 2048 * (idx - 8);
-    f[idx] = *reinterpret_cast<const bf16x8*>(p);
-  };
-  f32x4 acc[RI][8];
-#pragma unroll
-  for (int i = 0; i < RI; ++i)
-#pragma unroll
-    for (int j = 0; j < 8; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  // MFMA group n (0 .. 2 RI - 1): output row block i = n / 2, column blocks 4 (n & 1) .. + 3
-  auto mf4 = [&](int n, const bf16x8 (&f)[8 + RI]) {
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int i = n >> 1, j = 4 * (n & 1) + q;
-      acc[i][j] = mfma16(f[j], f[8 + i], acc[i][j]);
-    }
-  };
-  bf16x8 f0[8 + RI], f1[8 + RI];   // all fragments of k-step 0 / k-step 1
-
-  // prologue: A(0), B(0), A(1), B(1), A(2) (the ring's load order: B(t+2) then A(t+3))
-#pragma unroll
-  for (int s = 0; s < RI; ++s) dma_a(0, 0, s);
-#pragma unroll
-  for (int s = 0; s < 8; ++s) dma_b(0, 0, s);
-#pragma unroll
-  for (int s = 0; s < RI; ++s) dma_a(1, 1, s);
-#pragma unroll
-  for (int s = 0; s < 8; ++s) dma_b(1, 1, s);
-  if constexpr (SB == 3) {
-#pragma unroll
-    for (int s = 0; s < RI; ++s) dma_a(min(2, nk - 1), 2, s);
-#pragma unroll
-    for (int s = 0; s < 8; ++s) dma_b(min(2, nk - 1), 2, s);
-  }
-  vm_wait<(SB - 1) * (8 + RI)>();     // K-tile 0 landed (own part); A(1), B(1) (and A(2), B(2)) fly
-  __builtin_amdgcn_s_barrier();
-#pragma unroll
-  for (int idx = 0; idx < 8 + RI; ++idx) rd1(0, 0, 0, idx, f0);
-
-  // The loop is rotated so its back edge sits right after the barrier (the compiler puts a
-  // conservative lgkmcnt(0) at a loop header: there it finds nothing outstanding): iteration k =
-  // ks 1 of K-tile k, then ks 0 of K-tile k + 1, then the barrier; the last ks 1 is peeled.
-  auto next_b = [](int sb_) { return SB == 2 ? sb_ ^ 1 : sb_ == SB - 1 ? 0 : sb_ + 1; };
-  auto ks0 = [&](int k, int sa_, int sb_) {   // ks 0 of K-tile k: its ks-1 fragments read
-#pragma unroll
-    for (int n = 0; n < 2 * RI; ++n) {
-      mf4(n, f0);
-      // A(k + SA - 1) into the slot K-tile k-1 left (its last reads precede the previous barrier)
-      if (n & 1) dma_a(min(k + SA - 1, nk - 1), sa_ == 0 ? SA - 1 : sa_ - 1, n >> 1);
-      rd1(sa_, sb_, 1, n, f1);
-      if (RI == 4 && n < 4) rd1(sa_, sb_, 1, 8 + n, f1);      // (twelve fragments in eight slots)
-      __builtin_amdgcn_sched_barrier(0);
-    }
-    vm_wait<RI + (SB - 2) * (8 + RI)>();      // A(k+1), B(k+1) landed; A(k+2) (B(k+2), A(k+3)) may fly
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    __builtin_amdgcn_s_barrier();
-  };
-  auto ks1 = [&](int k, int sa_, int sb_, int sa1_) {   // ks 1 of K-tile k: next ks-0 read, DMA
-    const int kb = min(k + SB, nk - 1);
-#pragma unroll
-    for (int n = 0; n < 2 * RI; ++n) {
-      mf4(n, f1);
-      rd1(sa1_, next_b(sb_), 0, n, f0);
-      if (RI == 4 && n < 4) rd1(sa1_, next_b(sb_), 0, 8 + n, f0);
-      if (RI == 4) dma_b(kb, sb_, n);      // B(k + SB) into the slot K-tile k just left
-      else if (n & 1) dma_b(kb, sb_, n >> 1);
-      __builtin_amdgcn_sched_barrier(0);
-    }
-  };
-  int sa = 0, sbk = 0;   // slots of K-tile k (k % SA, k % SB)
-  ks0(0, 0, 0);
-  for (int k = 0; k + 1 < nk; ++k) {
-    const int sb = SB == 2 ? k & 1 : sbk, sa1 = sa == SA - 1 ? 0 : sa + 1;
-    ks1(k, sa, sb, sa1);
-    ks0(k + 1, sa1, next_b(sb));
-    sa = sa1;
-    sbk = next_b(sb);
-  }
-  ks1(nk - 1, sa, SB == 2 ? (nk - 1) & 1 : sbk, sa == SA - 1 ? 0 : sa + 1);
-  vm_wait<0>();                       // no LDS-DMA may outlive the workgroup
-  __builtin_amdgcn_s_barrier();       // every wave has read the last K-tile: the rings are free
+// The results of a wave's block, rows [mw, end) and 128 columns from nw on, through its piece of LDS. GROUPED 2 / 3: of row
+// mw + 64 q + lane the score, the pair.
+template <int GROUPED, int E, int RI>
+__device__ __forceinline__ void big4_results(const f32x4 (&acc)[RI][8], char* piece, int lane, int mw, int end, int nw, int M, int N,
+                                             const bf16* __restrict__ bias, bf16* __restrict__ out, long ldo,
+                                             float* __restrict__ part, const ExpertArgs& ex, const int (&pairs)[RI / 4],
+                                             const float (&scores)[RI / 4]) {
   int el = lane;
   asm volatile("" : "+v"(el));        // (nothing of what follows is computed ahead of the K loop)
-  const int mw = m0 + wr * (BM / 2), nw = n0 + wc * 128, left = M - mw;      // the wave's block and its rows
+  const int left = end - mw;
   if constexpr (GROUPED == 3) {
-    int pairs[RI / 4];      // the (token, choice) pairs of a lane's rows
 #pragma unroll
-    for (int q = 0; q < RI / 4; ++q) pairs[q] = ex.perm[min(mw + 64 * q + el, M - 1)];
-    b4_out_f32<RI>(smem, wid, el, left, acc, [&](int q, int r) { return ex.y + (long)__shfl(pairs[q], r, 64) * ldo + nw; });
+    for (int i = 0; i < RI; ++i) {
+      const auto rows = b4_rows_f32<RI>(piece, el, acc, i);
+#pragma unroll
+      for (int q = 0; q < 8; ++q) {
+        const int r = 16 * (i & 3) + (el >> 5) + 2 * q;
+        float* yr = ex.y + (long)__shfl(pairs[i / 4], r, 64) * ldo + nw + 4 * (el & 31);      // (by all lanes)
+        if (64 * (i / 4) + r < left) *reinterpret_cast<f32x4*>(yr) = rows.v[q];
+      }
+    }
     return;
   } else if constexpr (GROUPED == 2) {
     float sc[RI];
 #pragma unroll
-    for (int i = 0; i < RI; ++i) {
-      const int r = 16 * i + (el & 15);
-      sc[i] = ex.topk_w && r < left ? ex.topk_w[ex.perm[mw + r]] : 1.f;
-    }
-    if (ex.plain)      // squared ReLU
-      b4_out<RI, 8>(smem, wid, el, left, out + (long)mw * ldo + nw, ldo, [&](int i, int j) {
+    for (int i = 0; i < RI; ++i) sc[i] = __shfl(scores[i / 4], 16 * (i & 3) + (el & 15), 64);
+    if constexpr (E == EPI_RELU2)
+      b4_out<RI, 8>(piece, el, left, out + (long)mw * ldo + nw, ldo, [&](int i, int j) {
         f32x4 v;
 #pragma unroll
         for (int x = 0; x < 4; ++x) v[x] = fmaxf(acc[i][j][x] * sc[i], 0.f);
         return v * v;
       });
     else
-      b4_out<RI, 4>(smem, wid, el, left, out + (long)mw * ldo + (nw >> 1), ldo, [&](int i, int j) {
+      b4_out<RI, 4>(piece, el, left, out + (long)mw * ldo + (nw >> 1), ldo, [&](int i, int j) {
         f32x4 v;
 #pragma unroll
         for (int x = 0; x < 4; ++x) {
@@ -1220,13 +1095,15 @@ __device__ __forceinline__ void big4_tile(const bf16* __restrict__ X, long ldx, 
       });
     return;
   }
-  if (n0 + wc * 128 >= N) return;     // the columns past N of a half tile (their weight rows read zeros)
+  if (nw >= N) return;     // the columns past N of a half tile (their weight rows read zeros)
   if constexpr (E == kB4Parts) {
-    float* slab = part + (long)blockIdx.y * M * N;
-    b4_out_f32<RI>(smem, wid, el, left, acc, [&](int q, int r) { return slab + (long)(mw + 64 * q + r) * N + nw; });
+    float* slab = part + ((long)blockIdx.y * M + mw) * N + nw;
+    const auto to = __builtin_amdgcn_make_buffer_rsrc((void*)slab, (short)0, 0x7fffffff, 0x00020000);
+#pragma unroll
+    for (int i = 0; i < RI; ++i) b4_rows_f32<RI>(piece, el, acc, i).out(to, el, 16 * i, left, N * 4, true);
   } else if constexpr (E == EPI_SILU || E == EPI_GLU) {      // the wave's column blocks are gate and up in turn
     const GluPar gp = E == EPI_GLU ? glu_par(bias, N) : GluPar{};
-    b4_out<RI, 4>(smem, wid, el, left, out + (long)mw * ldo + (nw >> 1), ldo, [&](int i, int j) {
+    b4_out<RI, 4>(piece, el, left, out + (long)mw * ldo + (nw >> 1), ldo, [&](int i, int j) {
       f32x4 v;
 #pragma unroll
       for (int x = 0; x < 4; ++x) {
@@ -1248,7 +1125,7 @@ __device__ __forceinline__ void big4_tile(const bf16* __restrict__ X, long ldx, 
 #pragma unroll
         for (int x = 0; x < 4; ++x) b[j][x] = bf2f(bias[nw + 16 * j + 4 * (el >> 4) + x]);
     }
-    b4_out<RI, 8>(smem, wid, el, left, out + (long)mw * ldo + nw, ldo, [&](int i, int j) {
+    b4_out<RI, 8>(piece, el, left, out + (long)mw * ldo + nw, ldo, [&](int i, int j) {
       f32x4 v = acc[i][j];
       if constexpr (E == EPI_BIAS) v += b[j];
       if constexpr (E == EPI_RELU2) {
@@ -1257,6 +1134,257 @@ __device__ __forceinline__ void big4_tile(const bf16* __restrict__ X, long ldx, 
       }
       return v;
     });
+  }
+}
+
+// A run of tiles from the at-th item on: of 256 rows (BM 256) while each has more than 128, one of 128 or less. Returns the item behind it.
+// The rings run on from a tile to the next: its first K-tiles are on their way through the last two of the one before, the slot
+// that the last K-tile's A leaves holds the results on their way out (a wave's quarter of it is the part that its own next DMA
+// fills, so nobody waits for anybody), and the stores go on under the next products. With a workgroup per tile and walked, us:
+// 5000 x 5120 x 1024 54 and 51, 8192 x 8192 x 512 76 and 70, x 1024 117 and 111, x 2560 250 and 244, x 4096 374 and 374, 6184 x 8448
+// x 1024 102 and 95, x 2048 175 and 169, 4000 x 28672 x 2048 (SwiGLU) 350 and 340; longer K, where power bounds the step, level
+// (8192 x 10240 x 8192 928 and 927, 8192 x 57344 x 8192 SwiGLU 5143 and 5178).
+template <int GROUPED, int BM, int E>
+__device__ __forceinline__ int big4_run(const bf16* __restrict__ X, long ldx, const bf16* __restrict__ W, long ldw, long w_estride,
+                                        const B4Items& items, int at, int count, int M, int N, int K,
+                                        const bf16* __restrict__ bias, bf16* __restrict__ out, long ldo,
+                                        float* __restrict__ part, const int* __restrict__ grows, const ExpertArgs& ex) {
+  constexpr int RI = BM / 32;      // a wave's row blocks of 16, and its DMA instructions for a slot of A
+  // Slots of the rings and their places: a half tile's products cover half of the latency only, and its smaller slots leave room
+  // for one more of each.
+  constexpr int SA = BM == 256 ? 3 : 4, SB = BM == 256 ? 2 : 3, kSlotA = BM * 128, kRingB = SA * kSlotA;
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  // wave index in an SGPR: the DMA's LDS destinations (M0) and the fragment row bases are then
+  // scalar (a VGPR wave index cost a readfirstlane + s_nop per DMA instruction)
+  const int tid = threadIdx.x, lane = tid & 63, wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wr = wid >> 1, wc = wid & 1;
+  const int ktiles = K / 64;
+  const int kt0 = (int)(((long)ktiles * blockIdx.y) / gridDim.y);
+  const int kt1 = (int)(((long)ktiles * (blockIdx.y + 1)) / gridDim.y);
+  const int nk = kt1 - kt0;   // >= 2 (host check)
+
+  // DMA: instruction s (0..7) of wave w fills LDS row block 8 w + s (8 rows x 128 B, lane-
+  // linear); lane L supplies row 8 (8 w + s) + (L >> 3) at the chunk lds_frag expects in
+  // position L & 7: chunk = (L & 7) ^ ((row >> 1) & 7) = (L & 7) ^ ((L >> 4) + 4 (s & 1)) & 7
+  constexpr bool glu = GROUPED == 2 && E == EPI_GLU;
+  const int drow = 64 * wid + (lane >> 3), arow = 8 * RI * wid + (lane >> 3);
+  // weight row of LDS row drow: with a gate, waves 0 / 2 stage gate rows and 1 / 3 the up rows of the same columns
+  const int brow = glu ? (wid & 1) * (N >> 1) + (wid >> 1) * 64 + (lane >> 3) : drow;
+  int va[2], vb[2];
+#pragma unroll
+  for (int e = 0; e < 2; ++e) {
+    const int ch = (lane & 7) ^ (((lane >> 4) + 4 * e) & 7);
+    va[e] = (int)((arow * ldx + ch * 8) * 2);
+    vb[e] = (int)((brow * ldw + ch * 8) * 2);
+  }
+  // Where an item's rows come from: the base and the bytes behind it (A rows past the tile's end and weight rows past N read
+  // zeros). GROUPED 1 / 2: byte offsets of this lane's rows (at its chunk), from X where they are gathered (X has less than 2 GB:
+  // grouped_on_big4, moe_big_ok), from the tile's first row where they follow one another (slots know no such bound)
+  constexpr bool kRows = GROUPED == 1 || GROUPED == 2;
+  const bool gather = GROUPED == 2 || grows != nullptr;
+  struct Side {
+    const char* base;
+    int bytes;
+  };
+  auto item = [&](int v, int i) { return __builtin_amdgcn_readlane(v, i); };
+  auto side = [](const bf16* base, long rows, long ld) {
+    const long bytes = rows * ld * 2;
+    return Side{reinterpret_cast<const char*>(base), (int)(bytes < 0x7fffffffL ? bytes : 0x7fffffffL)};
+  };
+  auto side_a = [&](int i) {
+    const int m0 = item(items.m0, i);
+    if (kRows) return side(gather ? X : X + (long)m0 * ldx, 1L << 30, 1);
+    return side(X + (long)m0 * ldx, item(items.end, i) - m0, ldx);
+  };
+  auto side_b = [&](int i) {
+    const int n = glu ? item(items.n0, i) >> 1 : item(items.n0, i);
+    return side(W + (GROUPED ? (long)item(items.e, i) * w_estride : 0) + (long)n * ldw, N - n, ldw);
+  };
+  auto rows_of = [&](int i, int (&g)[RI]) {      // an item's rows (grows) or pairs (perm) ...
+    if constexpr (kRows) {
+      const int m0 = item(items.m0, i), end = item(items.end, i);
+#pragma unroll
+      for (int q = 0; q < RI; ++q) g[q] = min(m0 + arow + 8 * q, end - 1) - (gather ? 0 : m0);
+      if (gather) {
+        const int* from = GROUPED == 2 ? ex.perm : grows;
+#pragma unroll
+        for (int q = 0; q < RI; ++q) g[q] = from[g[q]];
+      }
+    }
+  };
+  auto offsets_of = [&](int (&g)[RI]) {      // ... and where they lie
+    if constexpr (kRows) {
+#pragma unroll
+      for (int q = 0; q < RI; ++q) {
+        const long src = GROUPED == 2 ? g[q] / ex.choices : g[q];
+        g[q] = (int)((src * ldx + (((lane & 7) ^ (((lane >> 4) + 4 * (q & 1)) & 7)) * 8)) * 2);
+        asm volatile("" : "+v"(g[q]));      // (here: behind the stores the wait for them would be one for those too)
+      }
+    }
+  };
+  auto rsrc = [](const Side& f) { return __builtin_amdgcn_make_buffer_rsrc((void*)f.base, (short)0, f.bytes, 0x00020000); };
+  Side fa = side_a(at), fb = side_b(at);      // what the rings take next: tile and K-tile (bytes into a row)
+  int ga[RI] = {}, oa = kt0 * 128, ob = kt0 * 128;
+  auto dma_a = [&](int slot, int s) {
+    if constexpr (kRows)
+      b4_dma(rsrc(fa), smem + slot * kSlotA + (RI * wid + s) * 1024, ga[s], oa);
+    else
+      b4_dma(rsrc(fa), smem + slot * kSlotA + (RI * wid + s) * 1024, va[s & 1], oa + (int)(8 * s * ldx * 2));
+  };
+  auto dma_b = [&](int slot, int s) {
+    b4_dma(rsrc(fb), smem + kRingB + slot * kB4Slot + (8 * wid + s) * 1024, vb[s & 1], ob + (int)(8 * s * ldw * 2));
+  };
+  const int fr = lane & 15, fq = lane >> 4;
+  // fragment idx 0-7: B rows (output columns) 16 idx, 8-15: A rows 16 (idx - 8), of k-step ks.
+  // lds_frag's swizzle depends on row bits 1-3 = fr bits 1-3 only, so a lane's fragments of one
+  // (slot, ks) share one VGPR address and differ by immediates of 2048 B (16 rows)
+  int lo[2][2];   // [operand A / B][ks] lane byte offset inside a slot
+#pragma unroll
+  for (int ks = 0; ks < 2; ++ks) {
+    const int ch = ((ks * 4 + fq) ^ ((fr >> 1) & 7)) * 16;
+    lo[0][ks] = (wr * (BM / 2) + fr) * 128 + ch;
+    lo[1][ks] = (wc * 128 + fr) * 128 + ch;
+  }
+  auto rd1 = [&](int sa_, int sb_, int ks, int idx, bf16x8 (&f)[8 + RI]) {
+    const char* p = idx < 8 ? smem + kRingB + sb_ * kB4Slot + lo[1][ks] + 2048 * idx
+                            : smem + sa_ * kSlotA + lo[0][ks] + 2048 * (idx - 8);
+    f[idx] = *reinterpret_cast<const bf16x8*>(p);
+  };
+  // store instructions of a full tile's results, at least
+  constexpr int kStores = GROUPED == 3 || E == kB4Parts ? 8 * RI : E == EPI_SILU || E == EPI_GLU ? 2 * RI : 4 * RI;
+  f32x4 acc[RI][8];
+  // MFMA group n (0 .. 2 RI - 1): output row block i = n / 2, column blocks 4 (n & 1) .. + 3
+  auto mf4 = [&](int n, const bf16x8 (&f)[8 + RI], bool first) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int i = n >> 1, j = 4 * (n & 1) + q;
+      acc[i][j] = mfma16(f[j], f[8 + i], first ? f32x4{0.f, 0.f, 0.f, 0.f} : acc[i][j]);
+    }
+  };
+  bf16x8 f0[8 + RI], f1[8 + RI];   // all fragments of k-step 0 / k-step 1
+
+  rows_of(at, ga);
+  offsets_of(ga);
+  // the next item goes on in the rings (BM 256): a whole tile whose rows are known before its first K-tile is due
+  auto follows = [&](int i) { return BM == 256 && i < count && nk >= 4 && item(items.end, i) - item(items.m0, i) > 128; };
+  bool more = follows(at + 1);
+  int gn[RI] = {};      // the rows of the next item, or of this one where none follows: its first K-tiles once more, for nobody
+  Side na = side_a(more ? at + 1 : at), nb = side_b(more ? at + 1 : at);
+  // Ahead of the barrier in K-tile k: to the next item behind the last K-tile. One branch that the others fall through: a lone wave
+  // waits for every jump (three of them took 2 % of a long K), and selects at the DMA would stand before the next products.
+  auto turn = [&](int k) {
+    oa += 128;
+    if (__builtin_expect(k + SA >= nk, 0)) {
+      asm volatile("");
+      if (k + SA == nk) {
+        fa = na;
+        oa -= nk * 128;
+#pragma unroll
+        for (int q = 0; q < RI; ++q) ga[q] = gn[q];
+      }
+      if (k + SB == nk) {
+        fb = nb;
+        ob -= nk * 128;
+      }
+    }
+  };
+
+  // prologue: A(0), B(0), A(1), B(1), A(2) (the ring's load order: B(t+2) then A(t+3))
+#pragma unroll
+  for (int t = 0; t < SB; ++t) {
+#pragma unroll
+    for (int s = 0; s < RI; ++s) dma_a(t, s);
+#pragma unroll
+    for (int s = 0; s < 8; ++s) dma_b(t, s);
+    oa = t + 1 < nk || nk >= SA ? oa + 128 : kt0 * 128;      // (fewer K-tiles than slots: nobody turns)
+    ob = t + 1 < nk || nk >= SB ? ob + 128 : kt0 * 128;
+  }
+  rows_of(more ? at + 1 : at, gn);
+  offsets_of(gn);
+  vm_wait<(SB - 1) * (8 + RI)>();     // K-tile 0 landed (own part); A(1), B(1) (and A(2), B(2)) fly
+  __builtin_amdgcn_s_barrier();
+#pragma unroll
+  for (int idx = 0; idx < 8 + RI; ++idx) rd1(0, 0, 0, idx, f0);
+
+  // The loop is rotated so its back edge sits right after the barrier (the compiler puts a
+  // conservative lgkmcnt(0) at a loop header: there it finds nothing outstanding): iteration k =
+  // ks 1 of K-tile k, then ks 0 of K-tile k + 1, then the barrier; the last ks 1 is peeled.
+  auto next_b = [](int sb_) { return SB == 2 ? sb_ ^ 1 : sb_ == SB - 1 ? 0 : sb_ + 1; };
+  auto ks0 = [&](int k, int sa_, int sb_, bool first, bool stores) {   // ks 0 of K-tile k: its ks-1 fragments read
+#pragma unroll
+    for (int n = 0; n < 2 * RI; ++n) {
+      mf4(n, f0, first);
+      // into the slot K-tile k-1 left (its last reads precede the previous barrier)
+      if (n & 1) dma_a(sa_ == 0 ? SA - 1 : sa_ - 1, n >> 1);
+      rd1(sa_, sb_, 1, n, f1);
+      if (RI == 4 && n < 4) rd1(sa_, sb_, 1, 8 + n, f1);      // (twelve fragments in eight slots)
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    turn(k);
+    // A(k+1), B(k+1) landed; A(k+2) (B(k+2), A(k+3)) may fly, and behind a tile the stores of its results (kStores or more)
+    if (stores) vm_wait<RI + kStores < 63 ? RI + kStores : 63>();
+    else vm_wait<RI + (SB - 2) * (8 + RI)>();
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+  };
+  auto ks1 = [&](int k, int sa_, int sb_, int sa1_) {   // ks 1 of K-tile k: next ks-0 read, DMA
+#pragma unroll
+    for (int n = 0; n < 2 * RI; ++n) {
+      mf4(n, f1, false);
+      rd1(sa1_, next_b(sb_), 0, n, f0);
+      if (RI == 4 && n < 4) rd1(sa1_, next_b(sb_), 0, 8 + n, f0);
+      if (RI == 4) dma_b(sb_, n);      // B(k + SB) into the slot K-tile k just left
+      else if (n & 1) dma_b(sb_, n >> 1);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    ob += 128;
+  };
+  int sa = 0, sb = 0;   // slots of K-tile k: those of a stream's K-tiles in turn
+  bool stores = false;
+  for (;;) {
+    int pairs[RI / 4] = {};
+    float scores[RI / 4];
+    if constexpr (GROUPED >= 2) {
+#pragma unroll
+      for (int q = 0; q < RI / 4; ++q)
+        pairs[q] = ex.perm[min(item(items.m0, at) + wr * (BM / 2) + 64 * q + lane, item(items.end, at) - 1)];
+    }
+    ks0(0, sa, sb, true, stores);
+    for (int k = 0; k + 1 < nk; ++k) {
+      const int sa1 = sa == SA - 1 ? 0 : sa + 1;
+      ks1(k, sa, sb, sa1);
+      sb = next_b(sb);
+      ks0(k + 1, sa1, sb, false, false);
+      sa = sa1;
+    }
+    const int last = sa;
+    sa = sa == SA - 1 ? 0 : sa + 1;
+    const bool again = more && follows(at + 2);
+    rows_of(again ? at + 2 : more ? at + 1 : at, gn);       // (the next tile's own have become ga)
+#pragma unroll
+    for (int q = 0; q < RI / 4; ++q) scores[q] = 1.f;
+    if (GROUPED == 2 && ex.topk_w) {
+#pragma unroll
+      for (int q = 0; q < RI / 4; ++q) scores[q] = ex.topk_w[pairs[q]];
+    }
+    ks1(nk - 1, last, sb, sa);
+    offsets_of(gn);
+    sb = next_b(sb);
+    if (!more) {
+      vm_wait<0>();                       // no LDS-DMA may outlive the workgroup, none lands where results wait
+      if (BM == 128) __builtin_amdgcn_s_barrier();       // (its smaller slots: pieces over several of them)
+    }
+    big4_results<GROUPED, E, RI>(acc, smem + (BM == 256 ? last * kSlotA : 0) + 8192 * wid, lane, item(items.m0, at) + wr * (BM / 2),
+                                 item(items.end, at), item(items.n0, at) + wc * 128, M, N, bias, out, ldo, part, ex, pairs, scores);
+    stores = item(items.end, at) - item(items.m0, at) >= BM && item(items.n0, at) + 256 <= N;
+    ++at;
+    if (!more) return at;
+    more = again;
+    if (more) {
+      na = side_a(at + 1);
+      nb = side_b(at + 1);
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");      // the piece is read: the next A may land in it
   }
 }
 
@@ -1280,45 +1408,59 @@ gemm_big4_kernel(const bf16* __restrict__ X, long ldx, const bf16* __restrict__ 
   const int ntiles = (N + BN - 1) / BN;      // (N % 256 == 128: half a last column tile)
   const int tiles = mtiles * ntiles;
   if constexpr (GROUPED != 0) halved = big4_halved(tiles);
-  const int whole = tiles - halved;
-  int t = blockIdx.x, half = -1;
-  if (t < whole) {
-    t = xcd_remap(t, whole);
-  } else {
-    t -= whole;
-    if (t >= 2 * halved) return;
-    t = xcd_remap(t, 2 * halved);
-    half = t & 1;
-    t = whole + (t >> 1);
+  const int whole = tiles - halved, all = whole + 2 * halved;
+  const int count = (int)blockIdx.x < all ? (all - 1 - (int)blockIdx.x) / (int)gridDim.x + 1 : 0;
+  B4Items items{0, 0, 0, 0};      // lane i: tile blockIdx.x + i gridDim.x of the walk
+  {
+    int t = (int)blockIdx.x + (int)(threadIdx.x & 63) * (int)gridDim.x, half = -1;
+    if (t < all) {
+      if (t < whole) {
+        t = xcd_remap(t, whole);
+      } else {
+        t = xcd_remap(t - whole, 2 * halved);
+        half = t & 1;
+        t = whole + (t >> 1);
+      }
+      const int per_group = kBigGroupM * ntiles;
+      const int grp = t / per_group, first_m = grp * kBigGroupM;
+      const int gsize = min(mtiles - first_m, kBigGroupM);
+      const int ti = first_m + (t % per_group) % gsize;
+      items.n0 = ((t % per_group) / gsize) * BN;
+      if constexpr (GROUPED == 0) {
+        items.m0 = ti * BM;
+        items.end = min(M, items.m0 + BM);
+      } else if constexpr (GROUPED == 1) {
+        const int4 info = gtiles[ti];      // rows [y, z) of the slot space
+        items.e = info.x;
+        items.m0 = info.y;
+        items.end = min(info.z, info.y + BM);
+      } else {
+        items.e = ex.tiles[2 * ti];
+        items.m0 = ex.tiles[2 * ti + 1];
+        items.end = min(ex.offsets[items.e + 1], items.m0 + BM);      // rows of the expert's group
+      }
+      if (half >= 0) {      // rows [m0, m0 + 128) or the 128 behind them
+        items.m0 += half * (BM / 2);
+        items.end = min(items.end, items.m0 + BM / 2);
+      }
+    }
   }
-  const int per_group = kBigGroupM * ntiles;
-  const int grp = t / per_group, first_m = grp * kBigGroupM;
-  const int gsize = min(mtiles - first_m, kBigGroupM);
-  int m0 = (first_m + (t % per_group) % gsize) * BM;
-  const int n0 = ((t % per_group) / gsize) * BN;
-  if constexpr (GROUPED >= 2) {
-    const int ti = m0 / BM;
-    const int e = ex.tiles[2 * ti];
-    W += (long)e * w_estride;
-    m0 = ex.tiles[2 * ti + 1];
-    M = ex.offsets[e + 1];         // rows [m0, M) of the expert's group
+  for (int i = 0; i < count;) {
+    const int rows = __builtin_amdgcn_readlane(items.end, i) - __builtin_amdgcn_readlane(items.m0, i);
+    if (rows <= 0) {
+      ++i;
+      continue;
+    }
+    if (rows <= BM / 2)
+      i = big4_run<GROUPED, BM / 2, E>(X, ldx, W, ldw, w_estride, items, i, count, M, N, K, bias, out, ldo, part, grows, ex);
+    else
+      i = big4_run<GROUPED, BM, E>(X, ldx, W, ldw, w_estride, items, i, count, M, N, K, bias, out, ldo, part, grows, ex);
+    __builtin_amdgcn_s_barrier();      // (the rings are everybody's again)
   }
-  if constexpr (GROUPED == 1) {
-    const int4 info = gtiles[m0 / BM];
-    W += (long)info.x * w_estride;
-    m0 = info.y;
-    M = info.z;                    // rows [m0, M) of the slot space
-  }
-  if (half >= 0) {      // rows [m0, m0 + 128) or the 128 behind them
-    m0 += half * (BM / 2);
-    M = min(M, m0 + BM / 2);
-    if (m0 >= M) return;
-  }
-  if (M - m0 <= BM / 2)
-    big4_tile<GROUPED, E, BM / 2>(X, ldx, W, ldw, m0, M, n0, N, K, bias, out, ldo, part, grows, ex);
-  else
-    big4_tile<GROUPED, E, BM>(X, ldx, W, ldw, m0, M, n0, N, K, bias, out, ldo, part, grows, ex);
 }
+
+// Workgroups for `tiles` tiles: one per compute unit, which walks them; more where a wave's lanes could not hold its list
+static int big4_grid(long tiles) { return (int)std::min(tiles, 256 * ((tiles + 256 * 64 - 1) / (256 * 64))); }
 
 // ---------------------------------------------------------------------------------------
 // Mid-M GEMM (plan kind 5): the tensor-parallel shard projections at M = 128-512 rows (tp2-tp8
@@ -1774,7 +1916,7 @@ static void run_big8(const bf16* X, long ldx, const bf16* W, long ldw, int M, in
 static void run_big4(const bf16* X, long ldx, const bf16* W, long ldw, int M, int N, int K,
                      int epi, const bf16* bias, bf16* out, long ldo, float* ws, int sk, hipStream_t stream) {
   const int tiles = ((M + 255) / 256) * ((N + 255) / 256), halved = sk > 1 ? 0 : big4_halved(tiles);
-  dim3 grid(tiles + halved, sk);
+  dim3 grid(sk > 1 ? tiles : big4_grid(tiles + halved), sk);
   float* part = sk > 1 ? splitk_part(ws) : nullptr;
 #define BFLY_BIG4(E)                                                                                                     \
   {                                                                                                                      \
@@ -2223,7 +2365,7 @@ int launch_gemm_grouped(const bf16* X, long x_rows, long ldx, const bf16* W, lon
     dim3 grid(max_tiles * (N / 256), 1);
     if (grouped_on_big4(x_rows, ldx, ldw, epi == EPI_SILU, rows != nullptr))
       (epi == EPI_SILU ? &gemm_big4_kernel<1, EPI_SILU> : &gemm_big4_kernel<1, EPI_NONE>)
-          <<<dim3(max_tiles * (N / 256) + 128), kB4Threads, kB4LdsBytes, stream>>>(
+          <<<dim3(big4_grid((long)max_tiles * (N / 256) + 128)), kB4Threads, kB4LdsBytes, stream>>>(
               X, ldx, W, ldw, 0, N, K, nullptr, out, ldo, nullptr, 0, rows, tiles, count, w_estride, ExpertArgs());
     else
       gemm_big8_kernel<true><<<grid, kB8Threads, kB8LdsBytes, stream>>>(
@@ -2244,19 +2386,19 @@ void launch_moe_big(bool down, const bf16* X, long ldx, const bf16* W, int N, in
                     bf16* out, long ldo, const ExpertArgs& ex, hipStream_t stream) {
   static bool attr = false;
   if (!attr) {
-    hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_big4_kernel<2, EPI_NONE>), hipFuncAttributeMaxDynamicSharedMemorySize,
-                        kB4LdsBytes);
-    hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_big4_kernel<3, EPI_NONE>), hipFuncAttributeMaxDynamicSharedMemorySize,
-                        kB4LdsBytes);
+    for (const void* k : {reinterpret_cast<const void*>(&gemm_big4_kernel<2, EPI_GLU>),
+                          reinterpret_cast<const void*>(&gemm_big4_kernel<2, EPI_RELU2>),
+                          reinterpret_cast<const void*>(&gemm_big4_kernel<3, EPI_NONE>)})
+      hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, kB4LdsBytes);
     attr = true;
   }
-  const dim3 grid(max_tiles * (N / 256) + 128, 1);      // (the kernel counts the tiles and halves up to 128 of them)
+  const dim3 grid(big4_grid((long)max_tiles * (N / 256) + 128), 1);      // (the kernel counts the tiles and halves up to 128 of them)
   if (down)
     gemm_big4_kernel<3, EPI_NONE><<<grid, kB4Threads, kB4LdsBytes, stream>>>(X, ldx, W, K, 0, N, K, nullptr, out, ldo, nullptr, 0,
                                                                    nullptr, nullptr, ntiles, (long)N * K, ex);
   else
-    gemm_big4_kernel<2, EPI_NONE><<<grid, kB4Threads, kB4LdsBytes, stream>>>(X, ldx, W, K, 0, N, K, nullptr, out, ldo, nullptr, 0,
-                                                                   nullptr, nullptr, ntiles, (long)N * K, ex);
+    (ex.plain ? &gemm_big4_kernel<2, EPI_RELU2> : &gemm_big4_kernel<2, EPI_GLU>)<<<grid, kB4Threads, kB4LdsBytes, stream>>>(
+        X, ldx, W, K, 0, N, K, nullptr, out, ldo, nullptr, 0, nullptr, nullptr, ntiles, (long)N * K, ex);
 }
 
 int gemm_check(int M, int N, int K, int epi) {

@@ -206,6 +206,54 @@ def test_grouped_rows_of_far_strides(gathered):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("counts", [[2100, 3000, 129, 0, 2500, 391], [256] * 34, [128, 8400, 1]])
+@pytest.mark.parametrize("Hd,F,plain,scaled", [(256, 2048, False, True), (512, 4096, True, False), (4096, 256, False, False)])
+def test_workgroups_that_walk_expert_tiles(counts, Hd, F, plain, scaled):
+    """More tiles than compute units: whole, short and half ones in turn, four and more steps of K."""
+    g = torch.Generator(device="cuda").manual_seed(sum(counts) + F)
+    E, TK = len(counts), sum(counts) // 2 * 2
+    flat = torch.cat([torch.full((c,), e, device="cuda") for e, c in enumerate(counts)])
+    ids = flat[torch.randperm(len(flat), generator=g, device="cuda")][:TK].view(-1, 2)
+    bf = lambda *s, k=1.0: (k * torch.randn(*s, generator=g, device="cuda")).to(torch.bfloat16)            # noqa: E731
+    x, w = bf(TK // 2, Hd), torch.rand(TK // 2, 2, generator=g, device="cuda") + 0.2
+    gu, dn = bf(E, F if plain else 2 * F, Hd, k=2 * Hd ** -0.5), bf(E, Hd, F, k=F ** -0.5)
+    got = ops.moe_glu_ffn(x, ids.int(), w, gu, dn, 7.0, 1.702, 1.0, scaled, "relu2" if plain else None).double()
+    with torch.device("cuda"):
+        want = reference(x.double(), ids, w.double(), gu.double(), dn.double(), 7.0, 1.702, 1.0, scaled, plain)
+    # bf16 hidden rows and output (2^-9 each), in every row
+    assert ((got - want).norm(dim=1) < 2.0 ** -7 * want.norm(dim=1)).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("epi", ["none", "silu"])
+@pytest.mark.parametrize("gathered", [False, True])
+@pytest.mark.parametrize("K", [128, 256, 1024])
+def test_workgroups_that_walk_grouped_tiles(epi, gathered, K):
+    """Groups of 2600, 70, 1800 and 4000 rows over 20 column tiles."""
+    counts, N = [2600, 70, 1800, 4000], 5120
+    M, E = sum(counts), len(counts)
+    g = torch.Generator(device="cuda").manual_seed(K)
+    x, w = (torch.randn(*s, generator=g, device="cuda").to(torch.bfloat16) for s in ((M, K), (E, N, K)))
+    w = w * K ** -0.5
+    rows = torch.randperm(M, generator=g, device="cuda") if gathered else torch.arange(M, device="cuda")
+    tiles, start, want = [], 0, []
+    for e, c in enumerate(counts):
+        tiles += [(e, r, start + c, 0) for r in range(start, start + c, 256)]
+        want.append(x[rows[start:start + c]].float() @ w[e].float().T)
+        start += c
+    want = torch.cat(want)
+    if epi == "silu":
+        v = want.view(M, N // 32, 2, 16)
+        want = (torch.nn.functional.silu(v[:, :, 0]) * v[:, :, 1]).reshape(M, N // 2)
+    out = torch.full_like(want, float("nan"), dtype=torch.bfloat16)
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device="cuda")                         # noqa: E731
+    torch.ops.bfly.moe_grouped_gemm(x, w.view(E * N, K), out, rows.int() if gathered else None, i32(tiles), i32([len(tiles)]), N * K,
+                                    N, K, E, ops.EPILOGUES[epi], 256)
+    # one rounding to bf16 (2^-9), f32 sums of K products beside it, in every row
+    assert ((out.float() - want).norm(dim=1) < 2.0 ** -8 * want.norm(dim=1)).all()
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("T", [40, 1000])
 def test_sparse_experts_of_padded_rows(T):
     """Gate/up and down rows further apart than they are wide, as models lay out rows of a multiple of 32 KB, on both tiles."""

@@ -104,11 +104,12 @@ def test_row_scaled_product_with_a_half_column_tile(M, N, K, how):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("M,N,K", [(4100, 1024, 512), (4225, 4224, 1024), (2300, 2560, 192), (1100, 4096, 14336)])
+@pytest.mark.parametrize("M,N,K", [(4100, 1024, 512), (4225, 4224, 1024), (2300, 2560, 192), (1100, 4096, 14336),
+                                   (8200, 5120, 128), (8200, 5120, 256), (8192, 8320, 2048)])
 @pytest.mark.parametrize("epi", ["none", "bias", "silu", "relu2", "glu"])
 def test_results_of_the_large_tile_into_any_rows(M, N, K, epi):
-    """A short last row tile, a half column tile, half tiles, split K: rows of any stride and alignment take the same values and
-    nothing beside them is written."""
+    """A short last row tile, a half column tile, half tiles, split K, workgroups that walk several tiles: rows of any stride and
+    alignment take the same values and nothing beside them is written."""
     assert ops.gemm_plan(M, N, K)["kind"] == "big4"
     g = torch.Generator(device="cuda").manual_seed(M + N)
     x, w, b = (torch.randn(*s, device="cuda", generator=g).to(torch.bfloat16) for s in ((M, K), (N, K), (N,)))
