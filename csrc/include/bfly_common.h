@@ -45,6 +45,24 @@ __device__ __forceinline__ int lane_scan(int x) {
   return x + __builtin_amdgcn_update_dpp(0, x, 0x143, 0xC, 0xF, false);
 }
 
+// Which sequence takes the pos-th place of a launch whose workgroups run down a sequence each, two of them on a compute unit: the
+// longer first where `round` sequences fill the units once. Where the others are second workgroups there, those of the first `round`
+// come from the shortest up, so that the longest run alone and the shortest beside the others. 16 heads of 128 x 128, in the order given
+// and so, us: 11 sequences of 200 to 700 rows 195 and 136 (delta rule), 142 and 108 (gated), 14 to 500 140 and 97, 105 and 81, 20 to
+// 400 157 and 131, 144 and 138, of one length level. With more sequences the places even out and the ranks cost more than they give:
+// 40 to 200 178 and 170, 123 and 120, 60 to 130 194 and 195, 113 and 121.
+__device__ __forceinline__ int by_length(const int* __restrict__ row_cu, int nseq, int pos, int round) {
+  if (nseq <= round || nseq > min(64, 5 * round)) return pos;
+  const int lane = threadIdx.x & 63, n = lane < nseq ? row_cu[lane + 1] - row_cu[lane] : -1;
+  int before = 0;
+  for (int j = 0; j < nseq; ++j) {
+    const int l = __builtin_amdgcn_readlane(n, j);
+    before += l > n || (l == n && j < lane);
+  }
+  const int want = nseq <= 2 * round && pos < round ? round - 1 - pos : pos;
+  return __builtin_ctzll(__ballot(lane < nseq && before == want));
+}
+
 // Maximum / sum over the four lanes l, l ^ 16, l ^ 32, l ^ 48 (one column of a 16x16 MFMA result) without LDS traffic
 __device__ __forceinline__ float row4_max(float x) {
   const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);

@@ -1224,8 +1224,9 @@ __global__ __launch_bounds__(256, NT <= 8 ? 2 : 1) void delta_chain_kernel(
                 PER = (U + 3) / 4, REC = U * 256, NS = NT <= 8 ? 2 : 4;
   extern __shared__ __attribute__((aligned(16))) float smem[];      // [SL][REC], then values: [SL][4 waves][4][64]
   const int nz = (Dv + 63) / 64, HH = H / G, per = HH * nz, u = blockIdx.x >> 3, grp = u / per * 8 + (blockIdx.x & 7);
-  const int s = grp / G, hk = grp - s * G, h = hk * HH + u % per / nz, c0 = u % nz * 64;
-  if (s >= nseq) return;
+  if (grp / G >= nseq) return;
+  const int s = NT <= 8 ? by_length(row_cu, nseq, grp / G, 256 / (H * nz)) : grp / G;
+  const int hk = grp % G, h = hk * HH + u % per / nz, c0 = u % nz * 64;
   const int r0 = __builtin_amdgcn_readfirstlane(row_cu[s]), r1 = __builtin_amdgcn_readfirstlane(row_cu[s + 1]);
   if (r1 <= r0 || (cost && !scan_in_chunks(r1 - r0, cost))) return;      // (the row-by-row form's)
   const int at = (r0 >> 4) + s, cb = max(0, first - at), ce = min((r1 - r0 + C - 1) / C, first + count - at);

@@ -249,9 +249,9 @@ __global__ __launch_bounds__(256, NT <= 8 ? 2 : 1) void gate_chain_kernel(
     float* __restrict__ o, int nseq, int H, int D, int Dv, int cost, int first, int count) {
   constexpr int C = 16, DP = 16 * NT, SL = kChainSlots, REC = chunk_record(NT), U = REC / 256, PER = (U + 3) / 4;
   extern __shared__ __attribute__((aligned(16))) float smem[];      // [SL][REC], then values: [SL][4 waves][4][64]
-  const int nz = (Dv + 63) / 64, u = blockIdx.x >> 3, pair = u / nz * 8 + (blockIdx.x & 7), s = pair / H, h = pair - s * H;
-  const int c0 = u % nz * 64;
-  if (s >= nseq) return;
+  const int nz = (Dv + 63) / 64, u = blockIdx.x >> 3, pair = u / nz * 8 + (blockIdx.x & 7);
+  if (pair / H >= nseq) return;
+  const int s = NT <= 8 ? by_length(row_cu, nseq, pair / H, 256 / (H * nz)) : pair / H, h = pair % H, c0 = u % nz * 64;
   const int r0 = __builtin_amdgcn_readfirstlane(row_cu[s]), r1 = __builtin_amdgcn_readfirstlane(row_cu[s + 1]);
   if (r1 <= r0 || (cost && !scan_in_chunks(r1 - r0, cost))) return;      // (the row-by-row form's)
   const int at = (r0 >> 4) + s, cb = max(0, first - at), ce = min((r1 - r0 + C - 1) / C, first + count - at);

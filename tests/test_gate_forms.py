@@ -118,3 +118,40 @@ def test_nothing_to_scan(T, H):
     idx = [torch.tensor(t, dtype=torch.int32, device="cuda") for t in ([0], [0, T], list(range(T)))]
     assert ops.gla_scan(z(T, H, D), z(T, H, D), z(T, H, Dv), z(T, H * D), z(1, H, D, Dv), *idx, 16.0, 1.0).shape == (T, H, Dv)
     assert ops.forget_scan(z(T, H, D), z(T, H, D), z(T, H, Dv), z(H * D), z(H * D), z(1, H, D, Dv), *idx).shape == (T, H, Dv)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["gla", "forget", "delta"])
+@pytest.mark.parametrize("n", [8, 9, 16, 17, 40, 41])
+def test_ragged_sequences_in_any_order(kind, n):
+    """Sequences of the same, of no and of very different lengths (up to five rounds of 256 workgroups take their places by length):
+    each has the same result wherever it stands in the step."""
+    g = torch.Generator(device="cuda").manual_seed(n)
+    H, D = 16, 128
+    lens = [(0, 300, 300, 1, 17, 190, 64, 33)[i % 8] + 5 * (i // 8) * (i % 3) for i in range(n)]
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda")            # noqa: E731
+    heads = {k: [rnd(m, h, D) for m in lens] for k, h in (("q", H), ("k", H), ("v", H), ("z", H))}
+    logits = {k: [rnd(m, H).to(torch.bfloat16) for m in lens] for k in "ab"}
+    states = [rnd(H, D, D) for _ in lens]
+    const = dict(a_log=0.5 * rnd(H) - 1, dt_bias=rnd(H), f_bias=rnd(H * D), lower=0.9 * torch.rand(H * D, generator=g, device="cuda"))
+
+    def run(order):
+        pick = lambda v: torch.cat([v[i] for i in order])                   # noqa: E731
+        q, k, v, z = (pick(heads[x]) for x in "qkvz")
+        cu = torch.tensor([sum(lens[i] for i in order[:j]) for j in range(n + 1)], dtype=torch.int32, device="cuda")
+        pos = torch.cat([torch.arange(lens[i]) + 7 * (i % 2) for i in order]).int().cuda()
+        st, slots = torch.stack([states[i] for i in order]), torch.arange(n, dtype=torch.int32, device="cuda")
+        if kind == "delta":
+            o = ops.delta_scan(q, k, v, pick(logits["b"]), pick(logits["a"]), const["a_log"], const["dt_bias"], st, slots, cu, pos,
+                               D ** -0.5, 1e-6, max_rows=max(lens))
+        elif kind == "gla":
+            b = lambda t: t.to(torch.bfloat16)                              # noqa: E731
+            o = ops.gla_scan(b(q), b(k), b(v), b(2 + z).view(-1, H * D), st, slots, cu, pos, 16.0, D ** -0.5, max_rows=max(lens))
+        else:
+            o = ops.forget_scan(q, z, v, const["f_bias"], const["lower"], st, slots, cu, pos, max_rows=max(lens))
+        at = cu.tolist()
+        return {i: (o[at[j]:at[j + 1]], st[j]) for j, i in enumerate(order)}
+
+    a, b = run(list(range(n))), run([(5 * i + 3) % n if n % 5 else n - 1 - i for i in range(n)])
+    for i in range(n):
+        assert torch.equal(a[i][0], b[i][0]) and torch.equal(a[i][1], b[i][1]), (i, lens[i])
