@@ -22,42 +22,110 @@ namespace bfly {
 
 namespace {
 
-template <typename T>
+// RB rows per workgroup. A row's sines and cosines (of the f32 angle, in f64) are found once for all its heads; the values of a page
+// lie beside those of the rows before and after them, so that rows which follow one another leave as one store, or at least meet in
+// the same L2. 8192 rows of 16 + 4 heads of 128, half of each rotated, in bf16: with a row a workgroup, an angle per pair and accesses of two
+// bytes 40 us, with this 22.
+template <typename T, int RB>
 __global__ __launch_bounds__(256) void rope_partial_kv_kernel(T* __restrict__ q, long q_ld, T* __restrict__ k, long k_ld,
                                                               const T* __restrict__ v, long v_ld,
                                                               const int* __restrict__ positions,
                                                               const float* __restrict__ inv_freq, int nrot,
                                                               const int* __restrict__ slots, T* __restrict__ k_cache,
                                                               T* __restrict__ v_cache, int H, int G, int D, int Dv,
-                                                              int bs) {
-  const long t = blockIdx.x;
-  const float p = (float)positions[t];
-  const int slot = (slots && k) ? slots[t] : -1;
-  // rotated pairs of the q heads, then of the k heads
-  const int nq = H * nrot, nk = k ? G * nrot : 0;
-  for (int i = threadIdx.x; i < nq + nk; i += blockDim.x) {
-    const bool isq = i < nq;
-    const int j = isq ? i : i - nq;
-    const int h = j / nrot, r = j % nrot;
-    T* ptr = (isq ? q + t * q_ld : k + t * k_ld) + (long)h * D + 2 * r;
-    const float a = p * inv_freq[r];
+                                                              int bs, int T_) {
+  constexpr int kTab = RB == 1 ? 512 : 128, E = 16 / sizeof(T);
+  typedef T unit __attribute__((ext_vector_type(E)));
+  typedef T run __attribute__((ext_vector_type(RB)));
+  __shared__ float2 cs[RB][kTab];
+  const long t0 = (long)blockIdx.x * RB;
+  const int rows = (int)min((long)RB, T_ - t0), tab = min(nrot, kTab);
+  auto turn = [&](int j, int r) {
+    const float a = (float)positions[t0 + j] * inv_freq[r];
     double sd, cd;
     sincos((double)a, &sd, &cd);
-    const float c = (float)cd, s = (float)sd;
-    const float u = (float)ptr[0], w = (float)ptr[1];
-    ptr[0] = (T)(u * c - w * s);
-    ptr[1] = (T)(w * c + u * s);
+    return make_float2((float)cd, (float)sd);
+  };
+  for (int i = threadIdx.x; i < rows * tab; i += 256) cs[i / tab][i % tab] = turn(i / tab, i % tab);
+  __syncthreads();
+  // rotated pairs of the q heads, then of the k heads: in units of 16 bytes, several of them asked for together, where rows allow it
+  if (2 * nrot % E == 0 && nrot <= kTab && D % E == 0 && q_ld % E == 0 && (!k || k_ld % E == 0) &&
+      (reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(k)) % 16 == 0) {
+    constexpr int U = RB == 1 ? 1 : 5;
+    const int un = 2 * nrot / E, per = (H + (k ? G : 0)) * un, total = rows * per;
+    for (int i0 = threadIdx.x; i0 < total; i0 += 256 * U) {
+      unit x[U];
+      T* p[U];
+      const float2* a[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int i = min(i0 + 256 * u, total - 1), j = i / per, jj = i - j * per, h = jj / un, r = jj - h * un;
+        p[u] = (h < H ? q + (t0 + j) * q_ld + (long)h * D : k + (t0 + j) * k_ld + (long)(h - H) * D) + r * E;
+        a[u] = &cs[j][r * (E / 2)];
+        x[u] = *reinterpret_cast<const unit*>(p[u]);
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        if (i0 + 256 * u >= total) break;
+#pragma unroll
+        for (int e = 0; e < E; e += 2) {
+          const float2 c = a[u][e / 2];
+          const float f = (float)x[u][e], w = (float)x[u][e + 1];
+          x[u][e] = (T)(f * c.x - w * c.y);
+          x[u][e + 1] = (T)(w * c.x + f * c.y);
+        }
+        *reinterpret_cast<unit*>(p[u]) = x[u];
+      }
+    }
+  } else {
+    const int nq = H * nrot, nk = k ? G * nrot : 0;
+    for (int j = 0; j < rows; ++j) {
+      const long t = t0 + j;
+      for (int i = threadIdx.x; i < nq + nk; i += 256) {
+        const bool isq = i < nq;
+        const int jj = isq ? i : i - nq, h = jj / nrot, r = jj % nrot;
+        T* ptr = (isq ? q + t * q_ld : k + t * k_ld) + (long)h * D + 2 * r;
+        const float2 a = r < kTab ? cs[j][r] : turn(j, r);
+        const float u = (float)ptr[0], w = (float)ptr[1];
+        ptr[0] = (T)(u * a.x - w * a.y);
+        ptr[1] = (T)(w * a.x + u * a.y);
+      }
+    }
   }
-  if (slot < 0) return;
+  if (!slots || !k) return;
   __syncthreads();      // the rotated k is read back below
-  const long blk = slot / bs, off = slot % bs;
-  for (int i = threadIdx.x; i < G * D; i += blockDim.x) {
-    const int g = i / D, d = i % D;
-    k_cache[((blk * G + g) * bs + off) * D + d] = k[t * k_ld + i];
+  const bool wide = D % E == 0 && k_ld % E == 0 && (reinterpret_cast<uintptr_t>(k) | reinterpret_cast<uintptr_t>(k_cache)) % 16 == 0;
+  int slot[RB];
+  bool follow = rows == RB && bs % RB == 0 && reinterpret_cast<uintptr_t>(v_cache) % 16 == 0;
+#pragma unroll
+  for (int j = 0; j < RB; ++j) {
+    slot[j] = j < rows ? slots[t0 + j] : -1;
+    follow = follow && slot[j] == slot[0] + j;
   }
-  for (int i = threadIdx.x; i < G * Dv; i += blockDim.x) {
-    const int g = i / Dv, d = i % Dv;
-    v_cache[((blk * G + g) * Dv + d) * bs + off] = v[t * v_ld + i];
+  follow = follow && slot[0] >= 0 && slot[0] % RB == 0;
+  for (int j = 0; j < rows; ++j) {
+    const int sl = slots[t0 + j];
+    if (sl < 0) continue;
+    const long blk = sl / bs, off = sl % bs;
+    T* to = k_cache + (blk * G * bs + off) * D;
+    const T* from = k + (t0 + j) * k_ld;
+    if (wide)
+      for (int i = threadIdx.x * E; i < G * D; i += 256 * E)
+        *reinterpret_cast<unit*>(to + (long)(i / D) * bs * D + i % D) = *reinterpret_cast<const unit*>(from + i);
+    else
+      for (int i = threadIdx.x; i < G * D; i += 256) to[(long)(i / D) * bs * D + i % D] = from[i];
+  }
+  for (int i = threadIdx.x; i < G * Dv; i += 256) {
+    run x;
+#pragma unroll
+    for (int j = 0; j < RB; ++j) x[j] = v[(t0 + min(j, rows - 1)) * v_ld + i];
+    if (follow) {
+      *reinterpret_cast<run*>(v_cache + ((long)(slot[0] / bs) * G * Dv + i) * bs + slot[0] % bs) = x;
+    } else {
+#pragma unroll
+      for (int j = 0; j < RB; ++j)
+        if (slot[j] >= 0) v_cache[((long)(slot[j] / bs) * G * Dv + i) * bs + slot[j] % bs] = x[j];
+    }
   }
 }
 
@@ -418,14 +486,20 @@ void launch_rope_partial_kv(void* q, long q_ld, void* k, long k_ld, const void* 
                             const float* inv_freq, int nrot, const int* slots, void* k_cache, void* v_cache,
                             int T, int H, int G, int D, int Dv, int block_size, bool f32, hipStream_t s) {
   if (T <= 0) return;
-  if (f32)
-    rope_partial_kv_kernel<float><<<T, 256, 0, s>>>((float*)q, q_ld, (float*)k, k_ld, (const float*)v, v_ld, positions,
-                                                    inv_freq, nrot, slots, (float*)k_cache, (float*)v_cache, H, G, D,
-                                                    Dv, block_size);
-  else
-    rope_partial_kv_kernel<bf16><<<T, 256, 0, s>>>((bf16*)q, q_ld, (bf16*)k, k_ld, (const bf16*)v, v_ld, positions,
-                                                   inv_freq, nrot, slots, (bf16*)k_cache, (bf16*)v_cache, H, G, D, Dv,
-                                                   block_size);
+  const int rb = nrot > 128 || T < 1024 ? 1 : T < 4096 ? 4 : 8;      // (workgroups enough for the chip first)
+#define BFLY_RP(TT, RB)                                                                                                       \
+  rope_partial_kv_kernel<TT, RB><<<(T + RB - 1) / RB, 256, 0, s>>>((TT*)q, q_ld, (TT*)k, k_ld, (const TT*)v, v_ld, positions, \
+                                                                   inv_freq, nrot, slots, (TT*)k_cache, (TT*)v_cache, H, G,   \
+                                                                   D, Dv, block_size, T)
+#define BFLY_RPN(TT)                   \
+  {                                    \
+    if (rb == 1) BFLY_RP(TT, 1);       \
+    else if (rb == 4) BFLY_RP(TT, 4);  \
+    else BFLY_RP(TT, 8);               \
+  }
+  if (f32) BFLY_RPN(float) else BFLY_RPN(bf16)
+#undef BFLY_RPN
+#undef BFLY_RP
 }
 
 void launch_row_seq(const int* row_cu, int nseq, int* row_seq, int T, hipStream_t s) {

@@ -293,9 +293,17 @@ __global__ __launch_bounds__(256) void rope_heads_copy_kernel(const T* __restric
                                                               const int* __restrict__ positions,
                                                               const float* __restrict__ inv_freq, int nrot, int H,
                                                               int n, int nd) {
+  constexpr int kTab = 512;
+  __shared__ float2 cs[kTab];      // the row's sines and cosines, once for all its heads
   const long t = blockIdx.x;
-  const float p = (float)positions[t];
   const int half = (nd + 1) / 2;
+  auto turn = [&](int r) {
+    double sd, cd;
+    sincos((double)((float)positions[t] * inv_freq[r]), &sd, &cd);
+    return make_float2((float)cd, (float)sd);
+  };
+  for (int r = threadIdx.x; r < min(nrot, kTab); r += blockDim.x) cs[r] = turn(r);
+  __syncthreads();
   for (int i = threadIdx.x; i < H * half; i += blockDim.x) {
     const int h = i / half, r = i % half;
     const T* sp = src + t * s_ld + h * s_hd + 2 * r;
@@ -303,10 +311,8 @@ __global__ __launch_bounds__(256) void rope_heads_copy_kernel(const T* __restric
     const bool two = 2 * r + 1 < nd;
     float u = 2 * r < n ? (float)sp[0] : 0.f, w = 2 * r + 1 < n ? (float)sp[1] : 0.f;
     if (r < nrot) {                                  // (2 nrot <= n: both elements exist)
-      double sd, cd;
-      sincos((double)(p * inv_freq[r]), &sd, &cd);
-      const float c = (float)cd, s = (float)sd;
-      const float u2 = u * c - w * s, w2 = w * c + u * s;
+      const float2 a = r < kTab ? cs[r] : turn(r);
+      const float u2 = u * a.x - w * a.y, w2 = w * a.x + u * a.y;
       u = u2;
       w = w2;
     }
