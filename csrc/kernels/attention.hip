@@ -12,6 +12,7 @@
 //   CONSECUTIVE keys: with V^T pages ([D][BS], written transposed by rope_kv) the PV A
 //   operand is then one 16-B load.
 //   Split-K over the context (flash-decoding) with an f32 partial combine kernel.
+// Long contexts of many sequences (attn_decode_flat_kernel): the step's pages end to end, cut into equal pieces.
 //   The cache may hold FP8 e4m3 instead of bf16 (bfly_kv.h): half the bytes per page, widened
 //   to bf16 in registers before the same MFMAs.
 //
