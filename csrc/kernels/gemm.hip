@@ -1009,6 +1009,18 @@ struct B4Rows {
           __builtin_amdgcn_raw_buffer_store_b16(__builtin_bit_cast(u16x8_b4, v[q])[x], to, off[q] < 0 ? -1 : off[q] + 2 * x, 0, 0);
     }
   }
+  // the same of bf16 rows too far apart for 32-bit offsets
+  __device__ __forceinline__ void out_far(bf16* dst, long ldo, int lane, int row0, int left) const {
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      const int r = row0 + lane / LPR + q * RPI;
+      bf16* o = dst + r * ldo + 8 * (lane % LPR);
+      const bf16x8 e = __builtin_bit_cast(bf16x8, v[q]);
+      if (r < left)
+#pragma unroll
+        for (int x = 0; x < 8; ++x) o[x] = e[x];
+    }
+  }
 };
 
 // RI x NJ blocks of 16 x 16 results, value(i, j) a lane's four of one, as bf16 rows from dst on
@@ -1031,7 +1043,9 @@ __device__ __forceinline__ void b4_out(char* piece, int lane, int left, bf16* ds
         if (j & 1) __builtin_amdgcn_sched_barrier(0);      // (a few values at a time: together they do not fit)
       }
     }
-    B4Rows<RB>(piece, lane).out(to, lane, 16 * h, left, (int)(ldo * 2), whole);
+    const B4Rows<RB> rows(piece, lane);
+    if (__builtin_expect(ldo < 1 << 20, 1)) rows.out(to, lane, 16 * h, left, (int)(ldo * 2), whole);
+    else rows.out_far(dst, ldo, lane, 16 * h, left);
     __builtin_amdgcn_sched_barrier(0);
   }
 }

@@ -131,3 +131,16 @@ def test_results_of_the_large_tile_into_any_rows(M, N, K, epi):
     elif epi == "relu2":
         r, d = s.clamp_min(0), K * 2.0 ** -24 * size
         assert ((want.float() - r * r).abs() <= 2.0 ** -8 * (r + d) ** 2 + 2 * r * d + d * d).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("epi", ["none", "silu"])
+def test_results_of_the_large_tile_into_far_rows(epi):
+    """Rows 2 MB apart and more leave by 64-bit addresses."""
+    M, N, K = 2300, 2560, 192
+    g = torch.Generator(device="cuda").manual_seed(N)
+    x, w = (torch.randn(*s, device="cuda", generator=g).to(torch.bfloat16) for s in ((M, K), (N, K)))
+    want = ops.linear(x, w, epilogue=epi)
+    far = torch.empty(M * (1 << 20), device="cuda", dtype=torch.bfloat16).view(M, 1 << 20)[:, 3:3 + want.shape[1]]
+    ops.linear(x, w, epilogue=epi, out=far)
+    assert torch.equal(far, want)
