@@ -71,8 +71,8 @@ __global__ __launch_bounds__(256) void rope_partial_kv_kernel(T* __restrict__ q,
         for (int e = 0; e < E; e += 2) {
           const float2 c = a[u][e / 2];
           const float f = (float)x[u][e], w = (float)x[u][e + 1];
-          x[u][e] = (T)(f * c.x - w * c.y);
-          x[u][e + 1] = (T)(w * c.x + f * c.y);
+          x[u][e] = (T)fmaf(f, c.x, -(w * c.y));      // (as everywhere else: left to the compiler, the forms round differently)
+          x[u][e + 1] = (T)fmaf(w, c.x, f * c.y);
         }
         *reinterpret_cast<unit*>(p[u]) = x[u];
       }
@@ -87,8 +87,8 @@ __global__ __launch_bounds__(256) void rope_partial_kv_kernel(T* __restrict__ q,
         T* ptr = (isq ? q + t * q_ld : k + t * k_ld) + (long)h * D + 2 * r;
         const float2 a = r < kTab ? cs[j][r] : turn(j, r);
         const float u = (float)ptr[0], w = (float)ptr[1];
-        ptr[0] = (T)(u * a.x - w * a.y);
-        ptr[1] = (T)(w * a.x + u * a.y);
+        ptr[0] = (T)fmaf(u, a.x, -(w * a.y));
+        ptr[1] = (T)fmaf(w, a.x, u * a.y);
       }
     }
   }

@@ -312,7 +312,7 @@ __global__ __launch_bounds__(256) void rope_heads_copy_kernel(const T* __restric
     float u = 2 * r < n ? (float)sp[0] : 0.f, w = 2 * r + 1 < n ? (float)sp[1] : 0.f;
     if (r < nrot) {                                  // (2 nrot <= n: both elements exist)
       const float2 a = r < kTab ? cs[r] : turn(r);
-      const float u2 = u * a.x - w * a.y, w2 = w * a.x + u * a.y;
+      const float u2 = fmaf(u, a.x, -(w * a.y)), w2 = fmaf(w, a.x, u * a.y);      // (written out: one rounding in every form)
       u = u2;
       w = w2;
     }

@@ -34,3 +34,31 @@ def test_rows_together_and_alone(dt, T, H, G, D, Dv, nrot, bs):
 
     for a, b in zip(run(T), run(512)):
         assert torch.equal(a, b)
+
+
+def _turned(x, pos, inv):
+    """Pairs (2 i, 2 i + 1) of the last dimension: u c - (w s), w c + (u s), the products in brackets rounded to f32, then the sums."""
+    a = (pos.float()[:, None] * inv).double()[:, None]
+    c, s = a.cos().float(), a.sin().float()
+    u, w = x[..., 0::2].float(), x[..., 1::2].float()
+    y = torch.stack([u.double() * c.double() - (w * s).double(), w.double() * c.double() + (u * s).double()], -1)
+    return y.float().flatten(-2)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("T", [5, 1024, 4096])
+@pytest.mark.parametrize("D", [64, 66])               # accesses of 16 bytes and single pairs
+def test_every_form_rounds_alike(dt, T, D):
+    """The rotation's two products are rounded in one order everywhere, so that a row's values depend neither on the rows beside it
+    nor on which kernel turned it (a float64 sum is off by a second rounding in fewer than one of 2^28 values)."""
+    g = torch.Generator(device="cuda").manual_seed(T + D)
+    x = torch.randn(T, 4, D, generator=g, device="cuda").to(dt)
+    pos = torch.randint(0, 5000, (T,), generator=g, device="cuda").int()
+    inv = 10000.0 ** (-torch.arange(D // 2, device="cuda") / (D // 2))
+    want = _turned(x, pos, inv).to(dt)
+    out = torch.empty_like(x)
+    ops.rope_heads_copy(x, out, pos, inv)
+    assert torch.equal(out, want)
+    ops.rope_partial_kv(x, None, None, pos, inv)
+    assert torch.equal(x, want)
