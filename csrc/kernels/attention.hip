@@ -243,7 +243,7 @@ attn_decode_kernel(const bf16* __restrict__ q, long q_stride, const CT* __restri
       O += f * po[w * 128 * G];
     }
     if (nsplit == 1) {
-      out[((long)b * Hq + h * G + qr) * D + d] = f2bf(L > 0.f ? O / L : 0.f);
+      out[((long)b * Hq + h * G + qr) * D + d] = f2bf(L == 0.f ? 0.f : O / L);
     } else {
       part_o[(part_base * 16 + qr) * D + d] = O;
       if (d == 0) {
@@ -464,11 +464,11 @@ attn_decode_flat_kernel(const bf16* __restrict__ q, long q_stride, const CT* __r
 #pragma unroll
       for (int w = 0; w < NW; ++w) {
         const float x = exp2f(s_m[w][qr] - Mb), y = po[w * G * LD];
-        L += x != 0.f ? x * s_l[w][qr] : 0.f;   // (0: no page, what it holds is an older segment's)
-        O += x != 0.f ? x * y : 0.f;
+        L += x * s_l[w][qr];                    // (no page: 0; keys that are no numbers: NaN)
+        O += x != 0.f ? x * y : 0.f;            // (0: no page, what it holds is an older segment's)
       }
       if (whole) {
-        out[((long)b * Hq + h * G + qr) * D + d] = f2bf(L > 0.f ? O / L : 0.f);
+        out[((long)b * Hq + h * G + qr) * D + d] = f2bf(L == 0.f ? 0.f : O / L);
       } else {
         part_o[(slot * G + qr) * D + d] = O;
         if (d == 0) {
@@ -579,7 +579,7 @@ attn_decode_flat_combine_kernel(const float* __restrict__ part_o, const float* _
     }
   }
   L = all(L, add);
-  const float inv = L > 0.f ? 1.f / L : 0.f;
+  const float inv = L == 0.f ? 0.f : 1.f / L;
   bf16x4 y;
 #pragma unroll
   for (int i = 0; i < 4; ++i) y[i] = f2bf(O[i] * inv);
@@ -624,7 +624,7 @@ attn_decode_combine_kernel(const float* __restrict__ part_o, const float* __rest
     }
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) L += __shfl_xor(L, o, 64);
-    if (d == 0) s_inv = L > 0.f ? 1.f / L : 0.f;
+    if (d == 0) s_inv = L == 0.f ? 0.f : 1.f / L;      // (keys that are no numbers: NaN)
   }
   __syncthreads();
   const float* po = part_o + (base * 16 + qr) * D + d;

@@ -310,19 +310,27 @@ def test_decode_pages_end_to_end(fp8, Hq, Hkv, ctx, max_ctx):
         k = kc.float()[pages].transpose(1, 2).reshape(-1, Hkv, D)[:c].to(F64)
         v = vc.float()[pages].permute(0, 3, 1, 2).reshape(-1, Hkv, D)[:c].to(F64)
         want.append(dense(q[b:b + 1].to(F64), k, v, torch.tensor([c - 1]), scale, 1 << 30, 0, None, None, 0, None))
-    run = lambda vv: ops.attn_decode(q.cuda(), kc.cuda(), vv.cuda(), tables.cuda(), torch.tensor(ctx, dtype=torch.int32).cuda(),  # noqa: E731
-                                     scale, max_ctx)
-    got = run(vc)
+    run = lambda kk, vv, part=0: ops.attn_decode(q.cuda(), kk.cuda(), vv.cuda(), tables.cuda(),  # noqa: E731
+                                                 torch.tensor(ctx, dtype=torch.int32).cuda(), scale, max_ctx, part)
+    got = run(kc, vc)
     err = (got.cpu().to(F64) - torch.cat(want)).abs().max()
     assert err < 2.0 ** -8 * vc.float().abs().max() + 1e-3      # weights and output rounded to bf16
     if n > 1 and not fp8:                                       # values that are no numbers stay in their sequence
         longest = max(range(B), key=lambda b: ctx[b])
-        bad = vc.clone()
-        bad[tables[longest, 0].item()] = float("nan")
-        poisoned = run(bad)
-        assert poisoned[longest].isnan().all()
         rest = [b for b in range(B) if b != longest]
+        page = tables[longest, 0].item()
+        bad = vc.clone()
+        bad[page] = float("nan")
+        poisoned = run(kc, bad)
+        assert poisoned[longest].isnan().all()
         assert torch.equal(poisoned[rest], got[rest])
+        bad = kc.clone()                                        # and keys: a page that is all of a wave's share has no maximum
+        bad[page] = float("nan")
+        for part in (0, max_ctx // 8, max_ctx):                 # (and with a workgroup per split, eight and one)
+            poisoned, clean = run(bad, vc, part), run(kc, vc, part)
+            assert poisoned[longest].isnan().all(), part
+            some = [b for b in rest if ctx[b] or not part]      # (a workgroup per split leaves the rows of empty sequences)
+            assert torch.equal(poisoned[some], clean[some])
 
 
 @pytest.mark.gpu
