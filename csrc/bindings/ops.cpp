@@ -695,7 +695,13 @@ void attn_decode(const Tensor& q, const Tensor& k_cache, const Tensor& v_cache,
               "attn_decode: block_tables");
   TORCH_CHECK(ctx_lens.numel() >= B, "attn_decode: ctx_lens");
   TORCH_CHECK((long)block_tables.size(1) * BS >= max_ctx, "attn_decode: block table too narrow for max_ctx");
-  const long rows = bfly::attn_decode_part_rows(B, Hq, Hkv, max_ctx, part_tokens);
+  long rows = bfly::attn_decode_part_rows(B, Hq, Hkv, max_ctx, part_tokens);
+  const auto held = [&](const c10::optional<Tensor>& t, long n) { return t.has_value() && t->numel() >= n; };
+  if (part_tokens <= 0 && rows > 0 && !(held(part_o, rows * D) && held(part_ml, rows * 2))) {
+    // buffers that a workgroup per split would do with (none, for one split): that form
+    part_tokens = bfly::attn_decode_part_tokens(B, Hkv, max_ctx);
+    rows = bfly::attn_decode_part_rows(B, Hq, Hkv, max_ctx, part_tokens);
+  }
   float *po = nullptr, *pml = nullptr;
   if (rows > 0) {
     TORCH_CHECK(part_o.has_value() && part_ml.has_value(), "attn_decode: partial buffers required");

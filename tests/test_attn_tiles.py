@@ -334,6 +334,27 @@ def test_decode_pages_end_to_end(fp8, Hq, Hkv, ctx, max_ctx):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("B,Hkv", [(128, 8), (16, 8), (1, 8), (3, 128)])
+def test_decode_with_buffers_of_a_workgroup_per_split(B, Hkv):
+    """The operator takes the buffers that its split sizes ask for, none at all for one split, also where pages would run end to end."""
+    max_ctx, D, G = 2048 if B > 1 else 1 << 18, 128, 4
+    g = torch.Generator(device="cuda").manual_seed(B)
+    ctx = torch.randint(1, 300, (B,), generator=g, device="cuda").int()
+    kc, vc = (torch.randn(40, Hkv, *s, generator=g, device="cuda").bfloat16() for s in ((BS, D), (D, BS)))
+    q = torch.randn(B, Hkv * G, D, generator=g, device="cuda").bfloat16()
+    tables = torch.randint(0, 40, (B, max_ctx // BS), generator=g, device="cuda").int()
+    op = torch.ops.bfly
+    assert op.attn_decode_part_rows(B, Hkv * G, Hkv, max_ctx, 0) == (max(1, 256 // Hkv) + B) * Hkv * G
+    part = op.attn_decode_part_tokens(B, Hkv, max_ctx)
+    ns = op.attn_decode_splits(max_ctx, part)
+    bufs = [torch.empty(B * Hkv * ns * 16 * n, device="cuda") for n in (D, 2)] if ns > 1 else [None, None]
+    out = torch.empty_like(q)
+    op.attn_decode(q, kc, vc, tables, ctx, 0.1, max_ctx, 0, out, *bufs)
+    want = ops.attn_decode(q, kc, vc, tables, ctx, 0.1, max_ctx, part)
+    assert torch.equal(out, want) if ns == 1 else torch.allclose(out.float(), want.float(), atol=2e-2)      # (larger ones may do for both)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("bad", [float("nan"), float("inf")])
 @pytest.mark.parametrize("H,G,D,Dv,window,keep,start,n", [
     (8, 2, 128, 128, 1 << 30, 0, 0, 40),      # one tile, the last page partly used
