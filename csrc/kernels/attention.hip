@@ -464,7 +464,8 @@ attn_decode_flat_kernel(const bf16* __restrict__ q, long q_stride, const CT* __r
 #pragma unroll
       for (int w = 0; w < NW; ++w) {
         const float x = exp2f(s_m[w][qr] - Mb), y = po[w * G * LD];
-        L += x * s_l[w][qr];                    // (no page: 0; keys that are no numbers: NaN)
+        const float z = s_l[w][qr];
+        L += x != 0.f || z != z ? x * z : 0.f;  // (no page: 0; keys that are no numbers: NaN)
         O += x != 0.f ? x * y : 0.f;            // (0: no page, what it holds is an older segment's)
       }
       if (whole) {
