@@ -54,7 +54,10 @@ class _DecodeGraph:
     | seeds (int64)], so a step stages them with a single host-to-device copy from a pinned
     buffer (two, alternating, each reused only after the event of its previous copy). A last
     stage's graph ends with the sampling kernel (and the TP merge) on those per-request
-    temperatures / seeds: `ids` are the step's tokens, one replay per step."""
+    temperatures / seeds: `ids` are the step's tokens, one replay per step.
+
+    `near` > 0: the step is captured a second time under this bound of its contexts, for steps
+    that lie within it (ModelRunner._near_ctx); `output` / `ids` are those of the latest replay."""
 
     def __init__(self, bucket: int, max_blocks: int, device, hidden: int, first: bool):
         b = bucket
@@ -87,6 +90,8 @@ class _DecodeGraph:
         self.hidden_in = None if first else torch.zeros(bucket, hidden, dtype=torch.bfloat16).to(device)
         self.graph: Optional[torch.cuda.CUDAGraph] = None
         self.output: Optional[torch.Tensor] = None
+        self.near = 0
+        self.forms: list = []        # (graph, output, ids) under max_seq_len and under `near`
         self.send_done = None        # event: the send of `output` has completed (pipeline stages)
 
 
@@ -138,6 +143,20 @@ class ModelRunner:
 
     def bucket_of(self, n: int) -> int:
         return self.buckets[bisect.bisect_left(self.buckets, n)]
+
+    def _near_ctx(self, rows: int) -> int:
+        """A nearer bound under which decode attention of `rows` rows is faster while no context
+        exceeds it (0: max_seq_len serves them all)."""
+        near = getattr(self.model, "near_ctx", None)
+        return near(rows, self.max_seq_len) if near is not None else 0
+
+    def _longest(self, ctx) -> int:
+        """The longest context of a step, where the host has them."""
+        if isinstance(ctx, torch.Tensor):
+            if ctx.device.type != "cpu":
+                return self.max_seq_len
+            ctx = ctx.numpy()
+        return min(max(int(np.max(ctx, initial=1)), 1), self.max_seq_len)
 
     # ------------------------------------------------------------------------------------
     def prefill_batch(self, plan, tokens_of) -> ForwardBatch:
@@ -205,7 +224,7 @@ class ModelRunner:
         lens = [cu[i + 1] - cu[i] for i in range(len(cu) - 1)]
         fb = ForwardBatch(input_ids=t32(ids), positions=t32(pos), slots=t32(slots), is_prefill=True,
                           cu_seqlens=t32(cu), max_seqlen=max(lens, default=0),
-                          block_tables=bt, ctx_lens=ctx, max_ctx=self.max_seq_len,
+                          block_tables=bt, ctx_lens=ctx, max_ctx=self._longest(self._ctx_host[:nd]),
                           logits_idx=torch.tensor(rows, dtype=torch.int64).to(dev, non_blocking=True),
                           num_decode=nd, prefix_lens=prefix if any(prefix) else None, prefix_cu=pre_cu,
                           prefix_tables=pre_tab,
@@ -236,7 +255,7 @@ class ModelRunner:
         t = lambda a: _to_dev(a, dev)  # noqa: E731
         return ForwardBatch(input_ids=t(inp["ids"]), positions=t(inp["pos"]), slots=t(inp["slots"]),
                             is_prefill=False, block_tables=t(inp["tables"]), ctx_lens=t(inp["ctx"]),
-                            max_ctx=self.max_seq_len, logits_idx=None, ep_tokens=ep_tokens,
+                            max_ctx=self._longest(inp["ctx"]), logits_idx=None, ep_tokens=ep_tokens,
                             state_slots=t(inp["state"]) if inp.get("state") is not None else None)
 
     # ------------------------------------------------------------------------------------
@@ -282,9 +301,7 @@ class ModelRunner:
                 _recover_from_capture(self.device)
                 return self.run(self.decode_batch(inp, ep_tokens), hidden_in)
         self._stage(g, inp, hidden_in)
-        g.graph.replay()
-        if g.ids is not None:
-            self.last_ids = g.ids[:B]
+        self._replay(g, inp)
         return g.output[:B]
 
     def precapture(self, rows: int) -> bool:
@@ -342,9 +359,7 @@ class ModelRunner:
             g.send_done = None
         self._stage(g, inp, None if self.recv_fn is not None else hidden_in)
         if g.graph is not None:
-            g.graph.replay()
-            if g.ids is not None:
-                self.last_ids = g.ids[:B]
+            self._replay(g, inp)
         else:
             if self.recv_fn is not None:
                 self.recv_fn(g.hidden_in)
@@ -400,36 +415,48 @@ class ModelRunner:
         if g.hidden_in is not None and hidden_in is not None:
             g.hidden_in[:B].copy_(hidden_in)
 
-    def _graph_batch(self, g: _DecodeGraph) -> ForwardBatch:
+    def _replay(self, g: _DecodeGraph, inp: dict) -> None:
+        graph, g.output, g.ids = g.forms[g.near > 0 and self._longest(inp["ctx"]) <= g.near]
+        graph.replay()
+        if g.ids is not None:
+            self.last_ids = g.ids[:len(inp["ids"])]
+
+    def _graph_batch(self, g: _DecodeGraph, max_ctx: int = 0) -> ForwardBatch:
         return ForwardBatch(input_ids=g.input_ids, positions=g.positions, slots=g.slots,
                             is_prefill=False, block_tables=g.block_tables, ctx_lens=g.ctx_lens,
-                            max_ctx=self.max_seq_len, logits_idx=None, ep_tokens=g.bucket,
+                            max_ctx=max_ctx or self.max_seq_len, logits_idx=None, ep_tokens=g.bucket,
                             state_slots=g.state_slots if self.stateful else None)
 
     def _capture(self, bucket: int, register: bool = True) -> _DecodeGraph:
         m = self.model
         g = _DecodeGraph(bucket, self.max_blocks, self.device, m.cfg.hidden_size, m.first)
-        fb = self._graph_batch(g)
+        # Both forms at once: the ranks of a group capture a bucket together, and which form a rank
+        # replays follows its own contexts (the collectives are the same in both).
+        near = self._near_ctx(bucket)
+        fbs = [self._graph_batch(g), self._graph_batch(g, near)][:2 if near else 1]
         s = torch.cuda.Stream(self.device)
         s.wait_stream(torch.cuda.current_stream(self.device))
         sample = self.sample_fn if (self.sample_fn is not None and self.model.last) else None
         with torch.cuda.stream(s):
-            for _ in range(2):   # warm up allocator / workspaces outside capture (no receive:
-                out = self.run(fb, g.hidden_in)   # a transfer would consume a real message)
+            for fb in fbs * 2 if len(fbs) == 1 else fbs:   # warm up allocator / workspaces outside capture (no
+                out = self.run(fb, g.hidden_in)            # receive: a transfer would consume a real message)
                 if sample is not None:
                     sample(out, g.temps, g.seeds)
         torch.cuda.current_stream(self.device).wait_stream(s)
         torch.cuda.synchronize(self.device)
         if self.pool is None:
             self.pool = torch.cuda.graph_pool_handle()
-        graph = torch.cuda.CUDAGraph()
-        with torch.cuda.graph(graph, pool=self.pool):
-            if self.recv_fn is not None and g.hidden_in is not None:
-                self.recv_fn(g.hidden_in)       # the boundary receive is the graph's first node
-            g.output = self.run(fb, g.hidden_in)
-            if sample is not None:
-                g.ids = sample(g.output, g.temps, g.seeds)
-        g.graph = graph
+        for fb in fbs:
+            graph, ids = torch.cuda.CUDAGraph(), None
+            with torch.cuda.graph(graph, pool=self.pool):
+                if self.recv_fn is not None and g.hidden_in is not None:
+                    self.recv_fn(g.hidden_in)       # the boundary receive is the graph's first node
+                out = self.run(fb, g.hidden_in)
+                if sample is not None:
+                    ids = sample(out, g.temps, g.seeds)
+            g.forms.append((graph, out, ids))
+        g.graph, g.output, g.ids = g.forms[0]
+        g.near = near
         if register:
             self.graphs[bucket] = g
         return g
@@ -440,6 +467,7 @@ class ModelRunner:
         for v in self.graphs.values():
             for g in (v if isinstance(v, list) else [v]):
                 g.graph = None
+                g.forms.clear()
                 g.send_done = None
         self.graphs.clear()
         self.last_instance = None

@@ -458,6 +458,9 @@ class TransformerLM:
             attn = ops.attn_decode(q, kc, vc, fb.block_tables, fb.ctx_lens, self.scale, fb.max_ctx)
         return self._o_proj(pre, attn, T)
 
+    def near_ctx(self, rows: int, max_ctx: int) -> int:
+        return ops.attn_decode_near(rows, self.dims.hkv, max_ctx)
+
     def _o_proj(self, pre: str, attn: torch.Tensor, T: int):
         d, D = self.dims, self.cfg.head_dim
         o_b = self.p.get(pre + "o_b") if self.shard.tp_rank == 0 else None

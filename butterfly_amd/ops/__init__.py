@@ -184,7 +184,7 @@ def reserve_workspace(device, max_tokens: int, max_n: int, max_k: int, max_batch
     _arena.get(device, "gemm", ws // 4 + 1, torch.float32, zero=True)
     if max_batch and max_ctx:
         # (a key / value head's query group has at most 16 rows)
-        rows = max(torch.ops.bfly.attn_decode_part_rows(b, 16 * num_kv_heads, num_kv_heads, max_ctx, 0)
+        rows = max(torch.ops.bfly.attn_decode_part_rows_up_to(b, 16 * num_kv_heads, num_kv_heads, max_ctx)
                    for b in range(1, max_batch + 1))
         _arena.get(device, "attn_o", rows * head_dim, torch.float32)
         _arena.get(device, "attn_ml", rows * 2, torch.float32)
@@ -617,6 +617,12 @@ def attn_decode(q, k_cache, v_cache, block_tables, ctx_lens, scale: float, max_c
     torch.ops.bfly.attn_decode(q, k_cache, v_cache, block_tables, ctx_lens, scale, max_ctx,
                                part_tokens, out, po, pml)
     return out
+
+
+def attn_decode_near(rows: int, num_kv_heads: int, max_ctx: int) -> int:
+    """The bound that decode attention of `rows` sequences should be told instead of `max_ctx` while no context
+    exceeds it, because a workgroup per sequence is then faster than pages end to end; 0 where `max_ctx` serves."""
+    return torch.ops.bfly.attn_decode_near(rows, num_kv_heads, max_ctx) if load_library() and not _FORCE_REF else 0
 
 
 def init_hash_(out, grow0: int, gcol0: int, gcols: int, seed: int, amp: float):

@@ -679,6 +679,12 @@ int64_t attn_decode_part_rows(int64_t B, int64_t Hq, int64_t Hkv, int64_t max_ct
   return bfly::attn_decode_part_rows(B, Hq, Hkv, max_ctx, part_tokens);
 }
 
+int64_t attn_decode_part_rows_up_to(int64_t B, int64_t Hq, int64_t Hkv, int64_t max_ctx) {
+  return bfly::attn_decode_part_rows_up_to(B, Hq, Hkv, max_ctx);
+}
+
+int64_t attn_decode_near(int64_t B, int64_t Hkv, int64_t max_ctx) { return bfly::attn_decode_near(B, Hkv, max_ctx); }
+
 void attn_decode(const Tensor& q, const Tensor& k_cache, const Tensor& v_cache,
                  const Tensor& block_tables, const Tensor& ctx_lens, double scale,
                  int64_t max_ctx, int64_t part_tokens, Tensor& out,
@@ -1228,6 +1234,8 @@ TORCH_LIBRARY(bfly, m) {
   m.def("attn_decode_splits(int max_ctx, int part_tokens) -> int", &attn_decode_splits);
   m.def("attn_decode_part_tokens(int B, int Hkv, int max_ctx) -> int", &attn_decode_part_tokens);
   m.def("attn_decode_part_rows(int B, int Hq, int Hkv, int max_ctx, int part_tokens) -> int", &attn_decode_part_rows);
+  m.def("attn_decode_part_rows_up_to(int B, int Hq, int Hkv, int max_ctx) -> int", &attn_decode_part_rows_up_to);
+  m.def("attn_decode_near(int B, int Hkv, int max_ctx) -> int", &attn_decode_near);
   m.def("attn_decode(Tensor q, Tensor k_cache, Tensor v_cache, Tensor block_tables, Tensor ctx_lens, "
         "float scale, int max_ctx, int part_tokens, Tensor(a!) out, Tensor(b!)? part_o, "
         "Tensor(c!)? part_ml) -> ()");

@@ -155,6 +155,10 @@ int attn_decode_splits(int max_ctx, int part_tokens);
 int attn_decode_part_tokens(int B, int Hkv, int max_ctx);
 // rows of D (part_o) and of 2 (part_ml) floats that launch_attn_decode needs
 long attn_decode_part_rows(int B, int Hq, int Hkv, int max_ctx, int part_tokens);
+// the most of them under any bound up to max_ctx (part_tokens chosen here)
+long attn_decode_part_rows_up_to(int B, int Hq, int Hkv, int max_ctx);
+// the bound to launch with instead of max_ctx while no context exceeds it (0: max_ctx serves)
+int attn_decode_near(int B, int Hkv, int max_ctx);
 int launch_attn_decode(const bf16* q, long q_stride, const void* k_cache, const void* v_cache,
                        const int* block_tables, int bt_stride, const int* ctx_lens, int B, int Hq,
                        int Hkv, int D, int block_size, float scale, int max_ctx, int part_tokens,

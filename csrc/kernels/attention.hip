@@ -1084,11 +1084,24 @@ int attn_decode_part_tokens(int B, int Hkv, int max_ctx) {
 // bound: bf16, 32 sequences of up to 8192 147 -> 114 / 174 -> 169, 48 of 4096 115 -> 87 / 153 -> 132, 16 of 2048 25 -> 23 / 28 -> 30,
 // 128 of 2048 136 -> 124 / 169 -> 173; FP8, 24 of 8192 in a batch of 32 73 -> 52, 96 of 4096 132 -> 95; one head of 8, 96 of 8192
 // 66 -> 54. Its start (lengths, their sum, then pages) and its second launch take 3 us more, so small steps keep the other form:
-// 32 of up to 1024 22 and 25, 8 of 4096 27 and 29, 64 of 1024 39 and 39. Under a far bound, many sequences of 60 tokens take longer
-// too, as several share a workgroup (48 under 4096 6 -> 11).
+// 32 of up to 1024 22 and 25, 8 of 4096 27 and 29, 64 of 1024 39 and 39. Contexts all at the bound lose up to 4 % with eight key / value
+// heads (64 of 8192 323 -> 334, 96 of 2048 129 -> 136) and up to 11 % with one (200 of 2048 42 -> 47). Contexts far below the bound, which
+// share workgroups, lose most (attn_decode_near).
 static int attn_decode_flat_pieces(int B, int Hkv, int max_ctx) {
   if (B > kFlatMaxBatch || max_ctx < 1536 || (long)B * Hkv * max_ctx < 1L << 18) return 0;
   return std::max(1, 256 / Hkv);
+}
+
+// While no context exceeds 768 tokens (1504 for many pairs), a workgroup per sequence and split of that bound. 32 heads on 8 under 4096, us of a workgroup per
+// split of 4096, end to end, and per split of the longest context, contexts of 0.3 to 1 of 64, 256, 768, 1024 tokens: 16 sequences 7.7 8.9 4.7,
+// 10.6 11.6 7.5, 18.1 14.0 12.9, 22.7 15.9 15.6; 32 5.0 11.1 5.0, 8.2 13.6 8.1, 17.0 20.7 17.1, 21.3 22.5 21.2; 48 6.3 11.7 6.3, 11.8 15.9
+// 11.9, 27.1 26.4 27.1, 36.2 30.5 36.3; 64 6.5 13.6 6.5, 13.0 18.0 12.9, 29.1 31.3 29.2, 38.0 37.8 38.0; 128 11.4 21.2 11.5, 22.6 30.6 22.6,
+// 50.8 53.0 51.1, 69.0 67.2 66.2. Past 768, one long context beside short ones turns it (32 of which one has 1024 and the others 170 on
+// average 19.2 14.2 19.2); not where a compute unit has four workgroups and more, whose shares even out by themselves (128 25.2 30.7 25.0,
+// at 1504 36.0 37.5 36.0, with 0.3 to 1 of 1504 100.8 94.8 97.4, all of them 125.5 130.8 120.3; 200 48.5 54.5 46.9, 151.5 143.5 150.7,
+// 204.6 203.1 204.7).
+int attn_decode_near(int B, int Hkv, int max_ctx) {
+  return attn_decode_flat_pieces(B, Hkv, max_ctx) == 0 ? 0 : (long)B * Hkv < 1024 ? 768 : 1504;
 }
 
 long attn_decode_part_rows(int B, int Hq, int Hkv, int max_ctx, int part_tokens) {
@@ -1097,6 +1110,12 @@ long attn_decode_part_rows(int B, int Hq, int Hkv, int max_ctx, int part_tokens)
   if (n > 0) return (long)(n + B) * Hq;
   const int ns = attn_decode_splits(max_ctx, part_tokens > 0 ? part_tokens : attn_decode_part_tokens(B, Hkv, max_ctx));
   return ns > 1 ? (long)B * Hkv * ns * 16 : 0;
+}
+
+long attn_decode_part_rows_up_to(int B, int Hq, int Hkv, int max_ctx) {
+  if (B <= 0 || Hkv <= 0) return 0;
+  const long pairs = (long)B * Hkv, splits = std::min(std::max(1L, (256 + pairs / 2) / pairs), (max_ctx + 255L) / 256);
+  return std::max(splits > 1 ? pairs * splits * 16 : 0, attn_decode_part_rows(B, Hq, Hkv, max_ctx, 0));
 }
 
 int launch_attn_decode(const bf16* q, long q_stride, const void* k_cache, const void* v_cache,
