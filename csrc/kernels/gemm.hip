@@ -1073,6 +1073,12 @@ __device__ __forceinline__ void big4_results(const f32x4 (&acc)[RI][8], char* pi
   int el = lane;
   asm volatile("" : "+v"(el));        // (nothing of what follows is computed ahead of the K loop)
   const int left = end - mw;
+  // (read where it is used: copies of many sums ahead of their use are registers that the next tile's fragments need)
+  auto sum = [&](int i, int j) {
+    f32x4 v = acc[i][j];
+    asm volatile("" : "+a"(v));
+    return v;
+  };
   if constexpr (GROUPED == 3) {
 #pragma unroll
     for (int i = 0; i < RI; ++i) {
@@ -1118,15 +1124,15 @@ __device__ __forceinline__ void big4_results(const f32x4 (&acc)[RI][8], char* pi
   } else if constexpr (E == EPI_SILU || E == EPI_GLU) {      // the wave's column blocks are gate and up in turn
     const GluPar gp = E == EPI_GLU ? glu_par(bias, N) : GluPar{};
     b4_out<RI, 4>(piece, el, left, out + (long)mw * ldo + (nw >> 1), ldo, [&](int i, int j) {
+      const f32x4 g = sum(i, 2 * j), u = sum(i, 2 * j + 1);
       f32x4 v;
 #pragma unroll
       for (int x = 0; x < 4; ++x) {
-        const float g = acc[i][2 * j][x], u = acc[i][2 * j + 1][x];
         if constexpr (E == EPI_GLU) {
           const bf16* b = bias + nw + 32 * j + 4 * (el >> 4) + x;
-          v[x] = glu_clamped(g + bf2f(b[0]), u + bf2f(b[16]), gp);
+          v[x] = glu_clamped(g[x] + bf2f(b[0]), u[x] + bf2f(b[16]), gp);
         } else {
-          v[x] = silu(g) * u;
+          v[x] = silu(g[x]) * u[x];
         }
       }
       return v;

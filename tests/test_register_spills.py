@@ -44,7 +44,7 @@ def _spilled():
     return out
 
 
-@pytest.mark.parametrize("kernel", ["attn_window_mfma_kernelILi2ELi16E", "attn_window_mfma_kernelILi4ELi8E", "attn_decode_flat_kernel"])
+@pytest.mark.parametrize("kernel", ["attn_window_mfma_kernelILi2ELi16E", "attn_window_mfma_kernelILi4ELi8E", "attn_decode_flat_kernel", "gemm_big4_kernel"])
 def test_kernels_without_spills(kernel):
     if not ops.load_library():
         pytest.skip("kernel library not built")
