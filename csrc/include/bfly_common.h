@@ -49,16 +49,18 @@ __device__ __forceinline__ int lane_scan(int x) {
 // longer first where `round` sequences fill the units once. Where the others are second workgroups there, those of the first `round`
 // come from the shortest up, so that the longest run alone and the shortest beside the others. 16 heads of 128 x 128, in the order given
 // and so, us: 11 sequences of 200 to 700 rows 195 and 136 (delta rule), 142 and 108 (gated), 14 to 500 140 and 97, 105 and 81, 20 to
-// 400 157 and 131, 144 and 138, of one length level. With more sequences the places even out and the ranks cost more than they give:
-// 40 to 200 178 and 170, 123 and 120, 60 to 130 194 and 195, 113 and 121.
+// 400 157 and 131, 144 and 138. Steps of one length keep their order, and a rank is three instructions per sequence, of which the compiler
+// sees sixteen at a time: short sequences notice either (gated, 8 heads, 64 of 32 rows 39 us, 45 with ranks in a loop; 40 of 5 to 95 with
+// 16 heads 76 and 80). With more sequences the places even out: 40 to 200 178 and 170, 123 and 120, 60 to 130 194 and 195, 113 and 121.
 __device__ __forceinline__ int by_length(const int* __restrict__ row_cu, int nseq, int pos, int round) {
   if (nseq <= round || nseq > min(64, 5 * round)) return pos;
   const int lane = threadIdx.x & 63, n = lane < nseq ? row_cu[lane + 1] - row_cu[lane] : -1;
+  if (!__any(lane < nseq && n != __builtin_amdgcn_readfirstlane(n))) return pos;
+  const int key = 64 * n + 63 - lane;      // (all different: of one length the first comes first)
   int before = 0;
-  for (int j = 0; j < nseq; ++j) {
-    const int l = __builtin_amdgcn_readlane(n, j);
-    before += l > n || (l == n && j < lane);
-  }
+  for (int j = 0; j < nseq; j += 16)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) before += __builtin_amdgcn_readlane(key, j + i) > key;
   const int want = nseq <= 2 * round && pos < round ? round - 1 - pos : pos;
   return __builtin_ctzll(__ballot(lane < nseq && before == want));
 }
