@@ -486,7 +486,12 @@ void launch_rope_partial_kv(void* q, long q_ld, void* k, long k_ld, const void* 
                             const float* inv_freq, int nrot, const int* slots, void* k_cache, void* v_cache,
                             int T, int H, int G, int D, int Dv, int block_size, bool f32, hipStream_t s) {
   if (T <= 0) return;
-  const int rb = nrot > 128 || T < 1024 ? 1 : T < 4096 ? 4 : 8;      // (workgroups enough for the chip first)
+  // Workgroups enough for the chip first; rows of few elements make up for the start of theirs later. bf16, us with a workgroup per row, four
+  // rows, eight rows: 16 + 4 heads of 128 / 128, half rotated, 600 rows 7.0 7.4 8.5, 1024 8.7 8.2 9.0, 2000 12.6 10.7 9.9, 4000 19.6 16.2
+  // 13.5, 8192 31.5 25.9 19.8; 8 + 2 of 64 1024 5.6 6.5 7.8, 1500 7.0 7.8 7.9, 2000 8.4 8.1 8.1, 4000 13.1 11.0 10.9; 16 + 1 of 256 / 192
+  // 1500 7.9 8.4 8.5, 2000 9.6 8.9 8.8; f32, 16 + 1 4000 17.6 12.5 13.9, 8192 29.1 22.2 20.5.
+  const int row = 2 * (H + G) * nrot + G * (D + Dv);
+  const int rb = nrot > 128 || T < (row < 2048 ? 1792 : 1024) ? 1 : T < 4096 ? 4 : 8;
 #define BFLY_RP(TT, RB)                                                                                                       \
   rope_partial_kv_kernel<TT, RB><<<(T + RB - 1) / RB, 256, 0, s>>>((TT*)q, q_ld, (TT*)k, k_ld, (const TT*)v, v_ld, positions, \
                                                                    inv_freq, nrot, slots, (TT*)k_cache, (TT*)v_cache, H, G,   \

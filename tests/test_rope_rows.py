@@ -7,7 +7,7 @@ from butterfly_amd import ops
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
-@pytest.mark.parametrize("T", [1024, 1027, 4096, 4099])
+@pytest.mark.parametrize("T", [1024, 1027, 1792, 1795, 4096, 4099])
 @pytest.mark.parametrize("H,G,D,Dv,nrot,bs", [(4, 2, 128, 64, 32, 32), (3, 1, 36, 40, 5, 12), (2, 2, 20, 17, 10, 16), (1, 1, 300, 8, 140, 8)])
 def test_rows_together_and_alone(dt, T, H, G, D, Dv, nrot, bs):
     g = torch.Generator(device="cuda").manual_seed(T + D)
@@ -47,7 +47,7 @@ def _turned(x, pos, inv):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
-@pytest.mark.parametrize("T", [5, 1024, 4096])
+@pytest.mark.parametrize("T", [5, 1792, 4096])
 @pytest.mark.parametrize("D", [64, 66])               # accesses of 16 bytes and single pairs
 def test_every_form_rounds_alike(dt, T, D):
     """The rotation's two products are rounded in one order everywhere, so that a row's values depend neither on the rows beside it
