@@ -14,7 +14,7 @@ def draw(seed):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("M,N,K", [(512, 128, 16), (513, 129, 72), (700, 200, 128), (600, 331, 40), (2000, 1000, 192), (511, 127, 24)])
+@pytest.mark.parametrize("M,N,K", [(512, 128, 16), (513, 129, 72), (700, 200, 128), (600, 331, 40), (2000, 1000, 192), (511, 127, 24), (4200, 1001, 16)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("first,pad", [(0, 0), (8, 16), (3, 5), (1, 8)])
 def test_products_into_any_rows(M, N, K, dtype, first, pad):
