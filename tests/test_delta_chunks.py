@@ -156,3 +156,21 @@ def test_two_launches_values_that_are_no_numbers_reach_later_rows_only(row, wher
         assert torch.equal(a.isfinite(), b.isfinite())
         ok = b.isfinite()
         assert (a - b)[ok].abs().max() < 1e-5 * b[ok].abs().max()      # two f32 evaluations
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("H,G,D,Dv,rows,one,two", [
+    (16, 4, 128, 128, [64], 64, 128), (16, 4, 192, 192, [150] * 4, 150, 300), (8, 2, 256, 256, [100], 100, 500),
+    (32, 8, 64, 64, [100] * 20, 100, 500), (6, 3, 200, 70, [90, 46, 33], 90, 450), (16, 4, 128, 100, [61], 61, 128),
+])
+def test_one_and_two_launches_agree_to_the_bit(H, G, D, Dv, rows, one, two):
+    """Which form runs follows the bound that the caller gives; the values do not."""
+    x = {k: t.cuda() for k, t in step([(3 * (i % 2), n) for i, n in enumerate(rows)], H, G, D, Dv, D + len(rows)).items()}
+    floats = lambda m: torch.ops.bfly.delta_record_floats(sum(rows), len(rows), H, G, D, Dv, H * Dv, m)      # noqa: E731
+    assert floats(one) == 0 < floats(two)
+    outs = []
+    for m in (one, two):
+        state = x["state"].clone()
+        outs.append((ops.delta_scan(**dict(x, state=state), q_scale=D ** -0.5, max_rows=m), state))
+    for a, b in zip(*outs):
+        assert torch.equal(a, b)

@@ -131,12 +131,20 @@ def test_results_of_the_large_tile_into_any_rows(M, N, K, epi):
     elif epi == "relu2":
         r, d = s.clamp_min(0), K * 2.0 ** -24 * size
         assert ((want.float() - r * r).abs() <= 2.0 ** -8 * (r + d) ** 2 + 2 * r * d + d * d).all()
+    else:                                                 # blocks of 16 gate and 16 up columns in turn
+        part = lambda t: t.view(-1, N // 32, 2, 16).unbind(2)                                             # noqa: E731
+        (gate, up), (dg, du), (bg, bu) = part(s), part(K * 2.0 ** -24 * size), part(b.float())
+        if epi == "glu":
+            gate, up = (gate + bg).clamp_max(7.0), (up + bu).clamp(-7.0, 7.0) + 1.0
+        act = gate * torch.sigmoid((1.702 if epi == "glu" else 1.0) * gate)      # (its slope is below 1.1 in either form)
+        bound = 2.0 ** -8 * (act * up).abs() + 1.1 * dg * (up.abs() + du) + act.abs() * du + 1e-6
+        assert ((want.float().view_as(act) - act * up).abs() <= bound).all()
 
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("epi", ["none", "silu"])
 def test_results_of_the_large_tile_into_far_rows(epi):
-    """Rows 2 MB apart and more leave by 64-bit addresses."""
+    """Rows 2 MB apart and more leave by 64-bit addresses (the values of rows side by side, which the test above has)."""
     M, N, K = 2300, 2560, 192
     g = torch.Generator(device="cuda").manual_seed(N)
     x, w = (torch.randn(*s, device="cuda", generator=g).to(torch.bfloat16) for s in ((M, K), (N, K)))
