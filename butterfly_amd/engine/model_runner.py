@@ -5,7 +5,9 @@ Decode graphs are captured per batch-size bucket on static input buffers; a step
 inputs into the bucket's buffers (padding rows: slot -1 = no cache write, ctx_len 1) and
 replays. Everything inside — GEMMs, RoPE/KV append, paged attention, norms, TP all-reduces
 (RCCL or the one-shot P2P kernel), the LM head and the TP sampling all-gather — is captured,
-so the host cost per token is one replay.
+so the host cost per token is one replay. Decode attention is told a bound of the contexts: eager
+steps tell it their longest one, a captured bucket max_seq_len, and where that means a form for long
+contexts, a second graph of the bucket tells it a nearer bound for the steps that lie within it.
 
 Pipeline stages on native RCCL (`set_pipeline_io`): a non-first stage's decode graph starts
 with the receive of the previous stage's boundary rows (Communicator.recv_native, captured in
@@ -363,7 +365,7 @@ class ModelRunner:
         else:
             if self.recv_fn is not None:
                 self.recv_fn(g.hidden_in)
-            g.output = self.run(self._graph_batch(g), g.hidden_in)
+            g.output = self.run(self._graph_batch(g, self._longest(inp["ctx"])), g.hidden_in)
         self.last_instance = g
         return g.output[:B]
 
