@@ -601,7 +601,9 @@ def attn_lse_merge_(acc_o, acc_lse, o, lse):
 def attn_decode(q, k_cache, v_cache, block_tables, ctx_lens, scale: float, max_ctx: int,
                 part_tokens: int = DECODE_PART_TOKENS, out=None):
     """One query token per sequence against the paged cache. `max_ctx` bounds ctx_lens (it
-    fixes the split-KV grid, so it is a static parameter under graph capture)."""
+    fixes the split-KV grid and the form, so it is a static parameter under graph capture). A bound near the
+    longest context is faster than a far one (attn_decode_near). In one form pages of all sequences are cut into
+    equal pieces: there the order of a sequence's sums, and with it its last bits, follows the others' lengths."""
     if not _gpu(q):
         return ref.attn_decode(q, k_cache, v_cache, block_tables, ctx_lens, scale, max_ctx,
                                part_tokens, out)

@@ -151,6 +151,7 @@ int launch_gemm_silu_gate(const bf16* X, long ldx, const bf16* W, long ldw, int 
                           hipStream_t stream);
 
 // attention.hip
+// of a workgroup per split: splits of part_tokens, and the part_tokens that launch_attn_decode chooses for it
 int attn_decode_splits(int max_ctx, int part_tokens);
 int attn_decode_part_tokens(int B, int Hkv, int max_ctx);
 // rows of D (part_o) and of 2 (part_ml) floats that launch_attn_decode needs

@@ -1063,8 +1063,8 @@ int attn_decode_splits(int max_ctx, int part_tokens) {
 }
 
 // Context split size, from a split-size sweep on MI355X (tools/bench_attn.py --parts): aim at
-// ~256 (b, kv-head, split) workgroups (one per CU, the nearest number: 192 pairs stay whole, 141 against 150 us at 24
-// sequences of up to 8k), splitting the context evenly and never
+// ~256 (b, kv-head, split) workgroups (one per CU, the nearest number: 192 pairs stay whole, 24 sequences of 1400 tokens 30.4 us
+// against 34.9 in two, of 700 17.6 and 21.3), splitting the context evenly and never
 // below 256 tokens per split; a single split skips the combine launch entirely.
 //   B=64 Hkv=8 ctx 1K: 1 split 46 us (2 splits 53);  B=8 ctx 4K: 4 splits 30 us (16: 38);
 //   B=64 Hkv=1: 4 splits 13.5 us (8: 15.4);        B=1 ctx 8K: 32 splits 27 us (64: 43).

@@ -82,9 +82,11 @@ def main():
                 ops.attn_decode(q, kcs[i], vcs[i], bt, cl, 0.088, ctx, part_tokens=pt, out=out)
             us = timed(f)
             byts = 2 * B * ctx * Hkv * D * kc.element_size()
-            used = pt if pt > 0 else torch.ops.bfly.attn_decode_part_tokens(B, Hkv, ctx)
+            flat = pt <= 0 and ops.attn_decode_near(B, Hkv, ctx) > 0      # pages end to end: no split size
+            used = pt if pt > 0 else 0 if flat else torch.ops.bfly.attn_decode_part_tokens(B, Hkv, ctx)
             print(json.dumps({"B": B, "ctx": ctx, "Hq": Hq, "Hkv": Hkv, "kv": kvd, "us": round(us, 2),
-                              "TBps": round(byts / us / 1e6, 3), "part_tokens": used, "rotate": a.rotate}), flush=True)
+                              "TBps": round(byts / us / 1e6, 3), "form": "end to end" if flat else "splits",
+                              "part_tokens": used, "rotate": a.rotate}), flush=True)
 
 if __name__ == "__main__":
     main()
