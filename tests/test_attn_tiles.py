@@ -151,6 +151,9 @@ def test_chunks_over_a_cached_prefix(Hq, Hkv, seqs):
     (6, 1, 256, 192, 1 << 30, 0, [(0, 140)] * 3 + [(33, 200)]),               # pages of uneven segments
     (16, 4, 128, 128, 700, 4, [(1 + 13 * i, 1) for i in range(130)]),        # decoded rows of 130 sequences
     (8, 2, 128, 128, 512, 40, [(2000, 1)]), (16, 1, 256, 192, 1 << 30, 0, [(300, 1), (5, 1), (0, 1)]),      # most splits without a page
+    (16, 4, 128, 128, 1 << 30, 0, [(900, 2), (32, 0), (40, 1), (500, 1)]),    # as many rows as sequences, but not one each
+    (48, 2, 128, 128, 1 << 30, 0, [(900, 3), (32, 0), (32, 0), (7, 1)]),      # tiles of 24 rows a token, one of them short
+    (16, 4, 64, 256, 1024, 0, [(1000 + 37 * i, 1) for i in range(20)]), (16, 4, 128, 128, 224, 0, [(900, 1), (100, 1)]),
 ])
 def test_extended_tiles_match_dense_attention(H, G, D, Dv, window, keep, seqs):
     g = torch.Generator().manual_seed(H + D + len(seqs))
