@@ -359,6 +359,11 @@ std::vector<int64_t> gemm_plan(int64_t M, int64_t N, int64_t K) {
   return {p.kind, p.mt, p.nt, p.bm, p.bn, p.sk, p.wk};
 }
 
+// whether gemm() of few rows streams its weights (without a row scale)
+bool gemm_streams(int64_t M, int64_t N, int64_t K, int64_t epilogue) {
+  return bfly::gemm_streams((int)M, (int)N, (int)K, (int)epilogue);
+}
+
 void gemm(const Tensor& x, const Tensor& w, Tensor& out, const c10::optional<Tensor>& bias,
           int64_t epilogue, const c10::optional<Tensor>& workspace) {
   CHECK_GPU(x); CHECK_BF16(x); CHECK_BF16(w); CHECK_BF16(out);
@@ -1229,6 +1234,7 @@ TORCH_LIBRARY(bfly, m) {
   m.def("gemm_workspace_size(int M, int N, int K) -> int", &gemm_workspace_size);
   m.def("gemm_workspace_bound(int M, int N, int K) -> int", &gemm_workspace_bound);
   m.def("gemm_plan(int M, int N, int K) -> int[]", &gemm_plan);
+  m.def("gemm_streams(int M, int N, int K, int epilogue) -> bool", &gemm_streams);
   m.def("gemm_check(int M, int N, int K, int epilogue) -> int",
         [](int64_t M, int64_t N, int64_t K, int64_t e) -> int64_t { return bfly::gemm_check(M, N, K, e); });
   m.def("attn_decode_splits(int max_ctx, int part_tokens) -> int", &attn_decode_splits);

@@ -38,7 +38,8 @@ struct RowScale {
 
 struct GemmPlan {
   int kind;  // 0 = skinny (decode), 1 = LDS-tiled, 3 = decode ring, 5 = mid-M 8-wave,
-             // 4 = 256x256 8-phase big tile (BK 64, prefill; kind 2 was the removed ring kernel)
+             // 4 = 256x256 8-phase big tile (BK 64, prefill; kind 2 was the removed ring kernel),
+             // 6 = 256x256 one wave per SIMD, 7 = mid-M one wave per SIMD, 8 = streamed (few rows)
   int mt, nt;
   int wk;    // skinny: waves splitting K inside a workgroup (1, 2, 4)
   int bm, bn;
@@ -121,6 +122,7 @@ int launch_gemm_plan(const GemmPlan& p, const bf16* X, long ldx, const bf16* W, 
                      int N, int K, int epi, const bf16* bias, bf16* out, long ldo, float* ws,
                      size_t ws_bytes, hipStream_t stream);
 int gemm_check(int M, int N, int K, int epi);
+bool gemm_streams(int M, int N, int K, int epi);      // the plan is the streamed product of few rows
 // 0 if the auto plan for this shape takes a RowScale (tile and decode-ring kernels)
 int gemm_rowscale_check(int M, int N, int K, int epi);
 // Y = X W^T without epilogue; when the plan splits K, the f32 slabs are left in the workspace

@@ -12,7 +12,7 @@
 //               + bias, limit), u = clamp(up + bias, +-limit); bias and the three constants come
 //               in one block (bfly_kernels.h)
 //
-// Two kernels, picked by M on the host:
+// Kernels, picked by M on the host (gemm_stream_kernel, gemm_dec_kernel, gemm_mid*_kernel and gemm_big4_kernel have their own notes):
 //  * gemm_skinny (M <= 64, decode): weight-streaming. Each wave streams 16*NT rows of W
 //    straight into VGPRs with non-temporal 16-B loads (no LDS round trip for an operand that is
 //    read exactly once: cdna_hip_programming.md §5 table, "GEMV / M <= 16" row), X fragments
@@ -254,6 +254,131 @@ gemm_skinny_kernel(const bf16* __restrict__ X, long ldx, const bf16* __restrict_
     } else {
       store_out(out, ldo, m, n, epi == EPI_BIAS ? v + bf2f(bias[n]) : epi == EPI_RELU2 ? fmaxf(v, 0.f) * fmaxf(v, 0.f) : v);
     }
+  }
+}
+
+// ---------------------------------------------------------------------------------------
+// Streamed product of few rows (kind 8)
+// ---------------------------------------------------------------------------------------
+// Workgroup = RB NT columns and all of K: NW waves take chunks of K in turn (chunk c: wave c % NW), straight into MFMA operands with
+// U chunks in flight, and sum their parts in LDS: nothing staged, no partial sums in memory, no launch behind it.
+// FOLD > 1 (up to RB = 16 / FOLD rows of X): the operands' 16 rows hold RB rows of FOLD neighbouring pieces of K, and the sum of the
+// FOLD diagonal blocks is the product. A compute unit takes in 26 KB of weights a microsecond wherever they come from, which is what
+// memory gives 256 of them together, so time goes by the unit with the most rows: folded tiles deal them out in fours and
+// eights. 16-row tiles (gemm_skinny_kernel: 32 of them a workgroup) leave most units idle on narrow results and a last round nearly
+// empty on others, and split products pay for their sums. One row, us, weights from memory: 1024 x 1024 5.0 -> 2.8, 2048 x 2048 7.9 ->
+// 4.3, 4096 x 4096 9.3 -> 7.8, 6144 x 4096 14.5 -> 10.3, 8320 x 2048 13.4 -> 8.1, 28672 x 4096 41.5 -> 35.7 (6.6 TB/s), 128256 x
+// 4096 172 -> 143; eight rows: 2048 x 2048 7.3 -> 4.6, 3072 x 2048 9.3 -> 6.0.
+template <int MT, int NT, int U, int FOLD, bool LAST>
+__device__ __forceinline__ void stream_step(f32x4 (&acc)[NT][MT], const bf16* const (&w)[NT], const bf16* const (&x)[MT], int c, int nw,
+                                            long ktile, int left) {
+  bf16x8 a[U][NT][2], b[U][MT][2];
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    if (LAST && u >= left) break;
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+        a[u][t][h] = ld_nt(reinterpret_cast<const bf16x8*>(w[t] + (FOLD * (c + u * nw) + FOLD / 2 * h) * ktile + (FOLD == 1 ? 32 * h : 0)));
+  }
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    if (LAST && u >= left) break;
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int t = 0; t < MT; ++t)
+        b[u][t][h] = *reinterpret_cast<const bf16x8*>(x[t] + 64L * FOLD * (c + u * nw) + 32 * FOLD * h);
+  }
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    if (LAST && u >= left) break;
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int m = 0; m < MT; ++m) acc[t][m] = mfma16(a[u][t][h], b[u][m][h], acc[t][m]);
+  }
+}
+
+// Element k of a weight row: k / 64 * ktile + k % 64, with ktile = 64 in rows of ldw, or (packed: [N / 256][K / 64][256][64]) ldw = 64 and
+// ktile = 256 * 64.
+template <int MT, int NT, int NW, int U, int FOLD>
+__global__ void __launch_bounds__(64 * NW)
+gemm_stream_kernel(const bf16* __restrict__ X, long ldx, const bf16* __restrict__ W, long ldw, long ktile, int M, int N, int K, int epi,
+                   const bf16* __restrict__ bias, bf16* __restrict__ out, long ldo) {
+  static_assert(MT == 1 || FOLD == 1, "folded tiles hold one row tile");
+  constexpr int RB = 16 / FOLD, KC = 64 * FOLD;
+  __shared__ f32x4 parts[NW * NT * MT * 64];
+  // (the wave as a scalar: matrix products run whatever lanes are masked off, so the last step has to branch around them)
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int chunks = K / KC, r = lane & 15, ko = 8 * (lane >> 4) + 32 * (r / RB), tile0 = (int)blockIdx.x * NT;
+  const bool halves = epi == EPI_SILU || epi == EPI_GLU;
+  // weight row of a tile's row i; with gate and up halves the tile's first half are gate rows, the other their up rows
+  const auto wrow = [&](int t, int i) {
+    if (!halves) return (tile0 + t) * RB + i;
+    const int f = (tile0 + t) * (RB / 2) + i % (RB / 2);
+    return f + (f & ~15) + (i >= RB / 2 ? 16 : 0);
+  };
+  const bf16 *w[NT], *x[MT];
+#pragma unroll
+  for (int t = 0; t < NT; ++t) {
+    const int n = wrow(t, r % RB);
+    w[t] = W + (ktile == 64 ? n * ldw : (long)(n >> 8) * 256 * K + (n & 255) * ldw) + ko / 64 * ktile + ko % 64;
+  }
+#pragma unroll
+  for (int t = 0; t < MT; ++t) x[t] = X + (long)min(16 * t + r % RB, M - 1) * ldx + ko;
+  f32x4 acc[NT][MT] = {};
+  int c = wave;
+  for (; c + (U - 1) * NW < chunks; c += U * NW) stream_step<MT, NT, U, FOLD, false>(acc, w, x, c, NW, ktile, U);
+  if (c < chunks) stream_step<MT, NT, U, FOLD, true>(acc, w, x, c, NW, ktile, (chunks - c + NW - 1) / NW);
+#pragma unroll
+  for (int t = 0; t < NT; ++t)
+#pragma unroll
+    for (int m = 0; m < MT; ++m) parts[((wave * NT + t) * MT + m) * 64 + lane] = acc[t][m];
+  __syncthreads();
+  const bool vec = (ldo & 3) == 0 && (reinterpret_cast<uintptr_t>(out) & 7) == 0;
+  constexpr int Q = RB / 4;      // groups of four rows of a tile
+  for (int i = threadIdx.x; i < NT * MT * Q * RB; i += 64 * NW) {
+    const int row = i % RB + RB * (i / (RB * Q) % MT), q = i / RB % Q, t = i / (RB * Q * MT);
+    if (row >= M) continue;
+    const auto sum = [&](int q) {      // over waves and pieces of K
+      f32x4 v{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int k = 0; k < NW; ++k)
+#pragma unroll
+        for (int f = 0; f < FOLD; ++f) v += parts[((k * NT + t) * MT + row / 16) * 64 + 16 * (Q * f + q) + RB * f + row % RB];
+      return v;
+    };
+    const int n = wrow(t, 4 * q);
+    f32x4 v = sum(q);
+    if (halves) {
+      // four gates here and their ups Q / 2 groups on, or (tiles of four rows) two of each
+      constexpr int C = RB == 4 ? 2 : 4;
+      if (q >= (Q + 1) / 2) continue;
+      const f32x4 up = RB == 4 ? f32x4{v[2], v[3], 0.f, 0.f} : sum(q + Q / 2);
+      bf16* o = out + (long)row * ldo + (tile0 + t) * (RB / 2) + 4 * q;
+#pragma unroll
+      for (int e = 0; e < C; ++e) {
+        if (epi == EPI_GLU) v[e] = glu_clamped(v[e] + bf2f(bias[n + e]), up[e] + bf2f(bias[n + 16 + e]), glu_par(bias, N));
+        else v[e] = silu(v[e]) * up[e];
+      }
+      if constexpr (RB == 4) {
+        o[0] = f2bf(v[0]);
+        o[1] = f2bf(v[1]);
+      } else {
+        store_out4(o, 0, 0, 0, v, vec);
+      }
+      continue;
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      if (epi == EPI_BIAS) v[e] += bf2f(bias[n + e]);
+      if (epi == EPI_RELU2) v[e] = fmaxf(v[e], 0.f) * fmaxf(v[e], 0.f);
+    }
+    store_out4(out, ldo, row, n, v, vec);
   }
 }
 
@@ -1872,6 +1997,13 @@ static void run_skinny(const bf16* X, long ldx, const bf16* W, long ldw, int M, 
       X, ldx, W, ldw, M, N, K, epi, bias, out, ldo, sk > 1 ? splitk_part(ws) : nullptr);
 }
 
+template <int MT, int NT, int NW, int U, int FOLD>
+static void run_stream(const bf16* X, long ldx, const bf16* W, long ldw, int M, int N, int K, int epi, const bf16* bias,
+                       bf16* out, long ldo, hipStream_t stream, bool packed) {
+  gemm_stream_kernel<MT, NT, NW, U, FOLD><<<N / (16 / FOLD * NT), 64 * NW, 0, stream>>>(
+      X, ldx, W, packed ? 64 : ldw, packed ? 256 * 64 : 64, M, N, K, epi, bias, out, ldo);
+}
+
 static void init_nt_policy() {
   static bool done = false;
   if (done) return;
@@ -2170,8 +2302,8 @@ static int run_plan(const GemmPlan& p, const bf16* X, long ldx, const bf16* W, l
   const RowScale rsc = rs ? *rs : RowScale{nullptr, 0, 0.f, 0.f};
   if (rs != nullptr && p.kind != 1 && p.kind != 3 && p.kind != 5 && p.kind != 7) return -4;   // row scale: tile / ring / mid epilogues
   if (epi == EPI_SILU_GATE && (p.kind != 1 || p.sk != 1)) return -4;   // gate: tile epilogue, no slabs
-  // packed (pack_w256) weights: the tile plans mark it with nt = 1, the mid-M kernels take it here
-  if (packed && p.kind != 5 && p.kind != 7) return -5;
+  // packed (pack_w256) weights: the tile plans mark it with nt = 1, the others take it here
+  if (packed && p.kind != 5 && p.kind != 7 && p.kind != 8) return -5;
   if (p.kind == 4) {
     // 8-phase big tile: every split needs >= 2 K-tiles of 64
     if (N % 256 != 0 || K % 64 != 0 || K / 64 < 2 * p.sk) return -1;
@@ -2231,6 +2363,22 @@ static int run_plan(const GemmPlan& p, const bf16* X, long ldx, const bf16* W, l
     DEC_CASE(128, 64, 4, 2, 8) DEC_CASE(64, 128, 4, 2, 6) DEC_CASE(64, 256, 4, 2, 4)
     DEC_CASE(64, 224, 4, 1, 4) DEC_CASE(64, 160, 4, 2, 5) DEC_CASE(64, 64, 4, 2, 8)
 #undef DEC_CASE
+    if (!done) return -2;
+  } else if (p.kind == 8) {
+    // streamed product of few rows: plan {8, row tiles, column tiles, waves, chunks in flight, fold, 1}
+    const int fold = p.bn;
+    if ((fold != 1 && fold != 2 && fold != 4) || p.sk != 1) return -2;
+    if (K % (64 * fold) != 0 || N % (16 / fold * p.nt) != 0 || M > 16 / fold * p.mt) return -1;
+    if (epi == EPI_SILU_GATE || (epi_halves(epi) && N % 32 != 0)) return -1;
+    bool done = false;
+#define ST_CASE(MT_, NT_, NW_, U_, F_)                                                                         \
+  if (!done && p.mt == MT_ && p.nt == NT_ && p.wk == NW_ && p.bm == U_ && fold == F_) {                        \
+    if (!dry) run_stream<MT_, NT_, NW_, U_, F_>(X, ldx, W, ldw, M, N, K, epi, bias, out, ldo, stream, packed); \
+    done = true;                                                                                               \
+  }
+    ST_CASE(1, 1, 4, 4, 4) ST_CASE(1, 1, 4, 4, 2) ST_CASE(1, 1, 8, 4, 2) ST_CASE(1, 2, 8, 4, 2)
+    ST_CASE(1, 1, 4, 4, 1) ST_CASE(1, 1, 8, 4, 1) ST_CASE(1, 2, 8, 4, 1) ST_CASE(2, 1, 8, 4, 1)
+#undef ST_CASE
     if (!done) return -2;
   } else if (p.kind == 0) {
     if (K % 128 != 0 || M > 16 * p.mt) return -1;
@@ -2311,18 +2459,65 @@ int launch_gemm_plan(const GemmPlan& p, const bf16* X, long ldx, const bf16* W, 
   return run_plan(p, X, ldx, W, ldw, M, N, K, epi, bias, out, ldo, ws, stream);
 }
 
+// Whether a product of few rows streams (gemm_stream_kernel) in place of plan `base`, and how: of the tiles that take M rows the one
+// whose busiest compute unit has the least to take in, its weight rows and, at 0.6 of their cost (from the L2), the rows of X past the first
+// once per workgroup (1 to 3 % off the best tile on average over 135 N x K by six row counts).
+// Up to four rows always, but where a split tile's sums cost nothing extra because their reader takes them as they are: it reads as
+// fast then (4096 x 14336 20.0 and 21.2 us, 6144 x 4096 by four rows 10.7 and 12.2) except for one row up to 8192 channels (10240 x
+// 8192 28.5 and 26.9). Up to eight rows where X does not weigh in: 4096 channels and 10240 columns (5120 x 2048 11.4 -> 8.3 us, 4096 x
+// 4096 9.9 -> 9.0; 14336 x 4096 23.6 and 25.2), in place of split sums 4096 x 4096 or 2048 channels (2048 x 2048 7.3 -> 4.6, read as
+// they are 5.1). Up to 16 rows to 1024 channels (1024 x 1024 5.9 -> 4.3), and to 2048 in place of split sums of a product that widens
+// its rows (3072 x 2048 9.6 -> 6.8; those of one that does not are read as they are: 2048 x 2048 5.4 and 6.6). Up to 32 rows to 1024 channels
+// and 4096 columns (2688 x 1024 7.4 -> 5.4).
+static bool stream_plan(int M, int N, int K, int epi, const GemmPlan& base, GemmPlan& p) {
+  if (M > 32 || K % 128 != 0 || epi == EPI_SILU_GATE || !plan_overrides().empty()) return false;
+  const bool split = base.sk > 1;
+  if (M <= 4) {
+    if (split && base.kind == 1 && (M > 1 || K > 8192)) return false;
+  } else if (M <= 8) {
+    if (K > 4096 || N > 10240 || (split && K > 2048 && N > 4096)) return false;
+  } else if (M <= 16) {
+    if (!(!split && K <= 1024 && N <= 8192) && !(split && K <= 2048 && N > K && N <= 10240)) return false;
+  } else if (split || K > 1024 || N > 4096) {
+    return false;
+  }
+  double best = 0;
+  const auto tile = [&](int rows, GemmPlan q) {
+    const double cost = (N / rows + 255) / 256 * (rows + 0.6 * (M - 1));
+    if (best != 0 && cost >= best) return;
+    best = cost;
+    p = q;
+  };
+  if (M > 16) {
+    p = GemmPlan{8, 2, 1, 8, 4, 1, 1};
+  } else if (M > 8) {
+    tile(16, GemmPlan{8, 1, 1, K <= 1024 ? 4 : 8, 4, 1, 1});
+    tile(32, GemmPlan{8, 1, 2, 8, 4, 1, 1});
+  } else {
+    if (M <= 4 && K % 256 == 0) tile(4, GemmPlan{8, 1, 1, 4, 4, 4, 1});
+    tile(8, GemmPlan{8, 1, 1, K < 2048 ? 4 : 8, 4, 2, 1});
+    if (K >= 2048) tile(16, GemmPlan{8, 1, 2, 8, 4, 2, 1});
+  }
+  return true;
+}
+
 // The plan for this call: the tuned/heuristic plan, or the heuristic one when a table entry
-// measured for another epilogue cannot run this one (e.g. odd skinny NT with SiLU), or the tile plan for a row scale.
+// measured for another epilogue cannot run this one (e.g. odd skinny NT with SiLU), or the tile plan for a row scale;
+// for few rows the streamed product.
 static GemmPlan select_plan(int M, int N, int K, int epi, bool row_scale = false) {
-  GemmPlan p = plan_gemm(M, N, K);
+  GemmPlan p = plan_gemm(M, N, K), q;
   if (run_plan(p, nullptr, 0, nullptr, 0, M, N, K, epi, nullptr, nullptr, 0, nullptr, nullptr, true) != 0)
     p = plan_gemm_heuristic(M, N, K);
-  return row_scale && rowscale_on_tile(p, N) ? plan_tile(M, N, K) : p;
+  if (row_scale) return rowscale_on_tile(p, N) ? plan_tile(M, N, K) : p;
+  return stream_plan(M, N, K, epi, p, q) ? q : p;
 }
+
+bool gemm_streams(int M, int N, int K, int epi) { return M > 0 && select_plan(M, N, K, epi).kind == 8; }
 
 int gemm_rowscale_check(int M, int N, int K, int epi) {
   if (M <= 0) return 0;
   const RowScale probe{nullptr, 0, 0.f, 0.f};
+  if (gemm_streams(M, N, K, epi)) return -4;      // streamed without one
   return run_plan(select_plan(M, N, K, epi, true), nullptr, 0, nullptr, 0, M, N, K, epi, nullptr, nullptr, 0,
                   nullptr, nullptr, true, false, &probe);
 }
@@ -2463,7 +2658,7 @@ int launch_gemm(const bf16* X, long ldx, const bf16* W, long ldw, int M, int N, 
 
 // Decode GEMM over a K-tile-blocked copy of the weight (layout [N/256][K/64][256][64], made
 // once by the engine when HBM allows, models/transformer.pack_decode_weights): the plan the
-// row-major weight would run (16 / 32 / 64-row tiles and the mid-M kernels of kinds 5 / 7, with
+// row-major weight would run (streams of few rows, 16 / 32 / 64-row tiles and the mid-M kernels of kinds 5 / 7, with
 // their split-K; EPI_SILU_GATE: the gate plan) on the packed copy. Each 128-row weight stage is then one 16 KiB run of memory instead of 128
 // runs of 128 B a row pitch apart: the Llama-3-70B gate/up GEMM at M = 64 in 145 against
 // 158 us, bitwise the same result (tools/packed_probe.py). Returns < 0 (nothing launched)
@@ -2486,6 +2681,13 @@ int launch_gemm_packed(const bf16* X, long ldx, const bf16* Wp, int M, int N, in
                        bool defer) {
   if (M <= 0) return dry ? 0 : 1;
   if (N % 256 != 0 || K % 64 != 0) return -1;
+  if (rs == nullptr) {
+    const GemmPlan q = select_plan(M, N, K, epi);
+    if (q.kind == 8) {
+      const int rc = run_plan(q, X, ldx, Wp, K, M, N, K, epi, nullptr, out, ldo, ws, stream, dry, false, nullptr, true);
+      return rc != 0 || dry ? rc : 1;
+    }
+  }
   GemmPlan p = plan_gemm(M, N, K);
   if (tuned_enabled() && plan_overrides().empty() && epi != EPI_SILU_GATE) {
     static const int kB[] = {1, 16, 32, 64, 128, 256, 512};
