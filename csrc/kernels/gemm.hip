@@ -2221,6 +2221,14 @@ static GemmPlan plan_gemm_heuristic(int M, int N, int K) {
   const bool skinny_ok = K % 128 == 0 && N % 128 == 0;
   // register-streaming kernel: GEMV-like M, and short-K shapes (row-parallel projections
   // after TP splits K) where the LDS pipeline cannot fill before the K loop ends
+  // (not where the results are wide: there the tiles fill the chip without splitting K, and a row of X is read once per 128 columns
+  // where it was once per 32. us, skinny -> tile: 24576 x 1024 by 16 rows 14.3 -> 11.2, by 64 30 -> 13.4, 10240 x 1024 by 32 12.4 -> 10.5, 32000 x
+  // 1024 by 64 40 -> 14.5, 50304 x 768 by 16 23 -> 16; 16384 x 1024 by 16 rows 10.3 and 10.5, 8192 x 1024 by 32 8.0 and 10.4)
+  if (skinny_ok && M > 4 && M <= 64 && K <= 1024 && N > (M <= 16 ? 16384 : 8192)) {
+    p = plan_tile(M, N, K);
+    p.sk = 1;
+    return p;
+  }
   if (skinny_ok && (M <= 4 || (M <= 64 && K <= 1024))) {
     p.kind = 0;
     p.mt = (M + 15) / 16;
@@ -2710,6 +2718,13 @@ int launch_gemm_packed(const bf16* X, long ldx, const bf16* Wp, int M, int N, in
     const int bm = M <= 16 ? 16 : M <= 32 ? 32 : M <= 64 ? 64 : 128;
     p = GemmPlan{1, 3, 0, bm <= 32 ? 1 : 2, bm, 128, 1};
   }
+  // 160 to 256 tiles of 128 columns: one a compute unit, K unsplit, four stages in flight. Split by what row-major weights need (neighbouring
+  // tiles' rows then meet in few memory channels, packed ones do not) they pay for sums. us, before -> here: 20480 x 4096 by 16 rows 37.8 ->
+  // 30.0, by 32 39.9 -> 33.0, 24576 x 4096 by 6, 32 and 64 38.9 -> 33.1, 46.7 -> 34.6, 50.9 -> 39.0, 28672 x 4096 by 32 40.3 -> 39.3 and 43.8 -> 35.8 on another
+  // card, 28672 x 8192 by 16 88 -> 76; outside: 16384 x 4096 by 16 and 32 26.7 and 27.6, 30.0 and 35.0, 36864 x 4096 by 32 62.6 and 64.8.
+  const int ctiles = N / 128;
+  if (p.kind == 1 && M <= 64 && ctiles >= 160 && ctiles <= 256 && K >= 256 && epi != EPI_SILU_GATE && plan_overrides().empty())
+    p = GemmPlan{1, 4, 1, M <= 32 ? 1 : 2, M <= 16 ? 16 : M <= 32 ? 32 : 64, 128, 1};
   // mid-M kernels (kinds 5 / 7): their weight DMA takes the packed layout as a template flag
   const bool mid = (p.kind == 5 || p.kind == 7) && (p.bn == 128 || p.bn == 256);
   if (!mid && (p.kind != 1 || (p.bm != 16 && p.bm != 32 && p.bm != 64) || (p.bn != 128 && p.bn != 256))) return -2;

@@ -1,0 +1,44 @@
+"""Tiles of few rows that do not split K: packed weights with a column tile for each compute unit, short K under wide results."""
+import pytest
+import torch
+
+from butterfly_amd import ops
+
+pytestmark = pytest.mark.skipif(not ops.load_library(), reason="kernel library not built")
+
+
+@pytest.mark.parametrize("M,N,kind", [(16, 16384, "skinny"), (16, 16512, "tile"), (17, 8192, "skinny"), (17, 8320, "tile"), (64, 32000, "tile"), (4, 32000, "skinny")])
+def test_short_products_under_wide_results(M, N, kind):
+    p = ops.gemm_plan(M, N, 1024)
+    assert (p["kind"], p["splitk"]) == (kind, 1)
+
+
+def _check(M, N, K, packed):
+    g = torch.Generator(device="cuda").manual_seed(M + N)
+    x = torch.randn(M, K, generator=g, device="cuda").to(torch.bfloat16)
+    w = (torch.randn(N, K, generator=g, device="cuda") * K ** -0.5).to(torch.bfloat16)
+    wp = ops.pack_w256(w) if packed else None
+    want = x.double() @ w.double().T
+    # one rounding to bf16 (at most 2^-9 of an element) beside f32 sums
+    assert (ops.linear(x, w, packed=wp).double() - want).norm() < 2.0 ** -8 * want.norm()
+    if packed:
+        d = ops.linear(x, w, packed=wp, defer=True)
+        assert (ops.materialize(d).double() - want).norm() < 2.0 ** -8 * want.norm()
+        v = want.view(M, N // 32, 2, 16)
+        want = (torch.nn.functional.silu(v[:, :, 0]) * v[:, :, 1]).reshape(M, N // 2)
+        assert (ops.linear(x, w, packed=wp, epilogue="silu").double() - want).norm() < 2.0 ** -8 * want.norm()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M", [5, 16, 17, 32, 33, 64, 65])
+@pytest.mark.parametrize("N,K", [(20224, 256), (20480, 192), (20480, 1088), (32768, 256), (33024, 512)])
+def test_packed(M, N, K):
+    """Both sides of the rule's lines: 158, 160, 256 and 258 column tiles, three and four K steps."""
+    _check(M, N, K, True)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M", [5, 16, 17, 33, 64])
+@pytest.mark.parametrize("N,K", [(8320, 1024), (16512, 64), (16512, 960), (32000, 1024)])
+def test_short(M, N, K):
+    _check(M, N, K, False)
