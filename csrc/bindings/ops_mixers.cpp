@@ -451,7 +451,9 @@ void moe_glu_ffn(const Tensor& x, const Tensor& topk_ids, const Tensor& topk_w, 
   const bool f32 = is_f32(x);
   const bool big = bfly::moe_big_ok(x.data_ptr(), x.stride(0), gate_up_w.data_ptr(), down_w.data_ptr(), hmid.data_ptr(),
                                     y.data_ptr(), (int)T, (int)TK, (int)Hd, (int)F, plain_act != bfly::ACT_NONE, f32);
-  const int tr = bfly::moe_tile_rows((int)TK, (int)E, f32, big, (int)Hd);
+  const bool parts = bfly::moe_parts_ok(x.data_ptr(), x.stride(0), gate_up_w.data_ptr(), down_w.data_ptr(), hmid.data_ptr(), (int)Hd,
+                                        (int)F, f32);
+  const int tr = bfly::moe_tile_rows((int)TK, (int)E, f32, big, parts, (int)Hd, (int)F, plain_act != bfly::ACT_NONE);
   const bool stream = tr == 64 && bfly::moe_stream_ok(x.data_ptr(), x.stride(0), gate_up_w.data_ptr(), down_w.data_ptr(),
                                                       hmid.data_ptr(), y.data_ptr(), (int)TK, (int)E, (int)Hd, (int)F, f32);
   // tiles that this tile height can need (no more than rows)

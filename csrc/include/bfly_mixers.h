@@ -150,9 +150,11 @@ void launch_route_rows(const void* x, long ldx, const void* wr, int Hd, const fl
 void launch_moe_sort(const int* ids, int TK, int E, int* perm, int* offsets, int* tiles, int* ntiles, int tile_rows,
                      hipStream_t s);
 int moe_sort_max_tiles(int TK, int E);
-// rows per tile of the grouped expert GEMMs for this problem (64, 128 for large bf16 groups, 256 where `big` allows the
-// LDS-DMA tile: moe_big_ok)
-int moe_tile_rows(int TK, int E, bool f32, bool big, int Hd);
+// rows per tile of the grouped expert GEMMs for this problem (64, 128 for large bf16 groups and, where `parts` allows, f32 ones,
+// 256 where `big` allows the LDS-DMA tile: moe_parts_ok, moe_big_ok)
+int moe_tile_rows(int TK, int E, bool f32, bool big, bool parts, int Hd, int F, bool plain);
+// whether f32 operands are 16-byte aligned rows of whole K steps
+bool moe_parts_ok(const void* x, long ldx, const void* gate_up_w, const void* down_w, const void* hmid, int Hd, int F, bool f32);
 // whether the operands fit the 256 x 256 LDS-DMA tile: bf16, 16-byte aligned rows, byte offsets below 2^31, K steps and
 // column tiles without a remainder. plain: experts without a gate
 bool moe_big_ok(const void* x, long ldx, const void* gate_up_w, const void* down_w, const void* hmid, const void* y, int T,
