@@ -2172,6 +2172,22 @@ static const std::vector<PlanOverride>& plan_overrides() {
   return v;
 }
 
+// token-count buckets of the sweep: M uses the entry of its bucket, or the heuristic plan when the sweep found nothing better there
+static bool tuned_plan(int M, int N, int K, GemmPlan& p) {
+  if (!tuned_enabled()) return false;
+  static const int kBuckets[] = {1, 16, 32, 64, 128, 256, 512};
+  int bucket = 0;
+  for (int b : kBuckets)
+    if (b >= M) { bucket = b; break; }
+  if (bucket == 0) return false;
+  for (const TunedPlan& t : kTuned)
+    if (t.N == N && t.K == K && t.M == bucket) {   // 256x256 entries (swept on big8) run big4: >= big8 at every swept M / sk
+      p = t.kind == 4 ? GemmPlan{6, 0, 0, 0, 256, 256, t.sk} : GemmPlan{t.kind, t.mt, t.nt, t.wk, t.bm, t.bn, t.sk};
+      return true;
+    }
+  return false;
+}
+
 GemmPlan plan_gemm(int M, int N, int K) {
   if (!plan_overrides().empty()) {
     static const int kB[] = {1, 16, 32, 64, 128, 256, 512};
@@ -2181,19 +2197,8 @@ GemmPlan plan_gemm(int M, int N, int K) {
     for (const PlanOverride& o : plan_overrides())
       if (o.N == N && o.K == K && o.M == bucket) return o.p;
   }
-  if (!tuned_enabled()) return plan_gemm_heuristic(M, N, K);
-  // token-count buckets of the sweep: M uses the entry of its bucket, or the heuristic plan
-  // when the sweep found nothing better there
-  static const int kBuckets[] = {1, 16, 32, 64, 128, 256, 512};
-  int bucket = 0;
-  for (int b : kBuckets)
-    if (b >= M) { bucket = b; break; }
-  if (bucket == 0) return plan_gemm_heuristic(M, N, K);
-  for (const TunedPlan& t : kTuned)
-    if (t.N == N && t.K == K && t.M == bucket)   // 256x256 entries (swept on big8) run big4:
-      return t.kind == 4 ? GemmPlan{6, 0, 0, 0, 256, 256, t.sk}   // >= big8 at every swept M / sk
-                         : GemmPlan{t.kind, t.mt, t.nt, t.wk, t.bm, t.bn, t.sk};
-  return plan_gemm_heuristic(M, N, K);
+  GemmPlan p;
+  return tuned_plan(M, N, K, p) ? p : plan_gemm_heuristic(M, N, K);
 }
 
 // LDS-tiled kernel: 16 to 128 rows per tile, split K until the grid has `target` workgroups
@@ -2212,6 +2217,27 @@ static GemmPlan plan_tile(int M, int N, int K) {
   const int ktiles = K / kBK;
   while (tiles * sk < target && sk * 2 * 4 <= ktiles && sk < 16) sk *= 2;
   p.sk = sk;
+  return p;
+}
+
+// The mid-M tile (gemm_mid4_kernel) that takes least, in us: rounds of 256 workgroups of 128 x 128, 128 x 256 or (half column tiles) 256 x
+// 128 at 0.5, 0.7 and 0.75 a K step and 4 for the pipeline's ends, and 2 + 0.5 per MB for the sums of a split K (within 12 % over 180
+// M x N x K of 65 to 2000 rows).
+static GemmPlan plan_mid(int M, int N, int K, double& least) {
+  static const struct { int bm, bn, sa, sb; double step; } kTiles[] = {{128, 128, 3, 7, 0.5}, {128, 256, 4, 3, 0.7}, {256, 128, 3, 4, 0.75}};
+  GemmPlan p{};
+  const int steps = K / 64;
+  least = 0;
+  for (const auto& t : kTiles) {
+    if (N % t.bn != 0 || (t.bm == 256 && N % 256 == 0)) continue;
+    const long tiles = (long)((M + t.bm - 1) / t.bm) * (N / t.bn);
+    for (int sk = 1; sk <= 8 && (sk == 1 || (steps >= 4 * sk && tiles * sk <= 256)); sk *= 2) {
+      const double us = (double)((tiles * sk + 255) / 256) * (t.step * steps / sk + 4) + (sk > 1 ? 2 + 2e-6 * sk * M * N : 0);
+      if (least != 0 && us >= least) continue;
+      least = us;
+      p = GemmPlan{7, t.sa, t.sb, 0, t.bm, t.bn, sk};
+    }
+  }
   return p;
 }
 
@@ -2242,6 +2268,14 @@ static GemmPlan plan_gemm_heuristic(int M, int N, int K) {
     p.sk = sk;
     return p;
   }
+  // 65 to 256 rows: mid-M tiles, whose rings keep K steps in flight that the 128-row tiles of plan_tile wait for, split or not.
+  // us, before -> here: 100 x 2048 x 2048 12.4 -> 11.9, 256 x 2688 x 1024 17.9 -> 12.8, 65 x 6272 x 2048 22.7 -> 14.4, 256 rows 42.6 ->
+  // 20.8, 128 x 8320 x 2048 35.5 -> 20.0, 180 x 12416 x 4096 71.7 -> 35.3; not where few rows split a long K in 16 (65 x 2048 x 8192 15.1, here
+  // 16.6).
+  double mid = 0;
+  const bool mid_ok = M > 64 && N % 128 == 0 && K % 64 == 0 && K >= 256;
+  const GemmPlan pm = mid_ok ? plan_mid(M, N, K, mid) : GemmPlan{};
+  if (mid_ok && M <= 256 && !(M <= 128 && K >= 8192 && plan_tile(M, N, K).sk == 16)) return pm;
   // 256 x 256 tile from two K steps on (its pipeline's least)
   if (M > 256 && N % 128 == 0 && K % 64 == 0 && K >= 128 && (N % 256 == 0 || (N > 1024 && K >= 256))) {
     // prefill / large batch: the 256x256 one-wave-per-SIMD tile (gemm_big4_kernel: 1.52-1.55 PF at M = 8192 on the 70B
@@ -2272,6 +2306,16 @@ static GemmPlan plan_gemm_heuristic(int M, int N, int K) {
         best = t;
         p.sk = sk;
       }
+    }
+    // The mid-M tiles where they take 15 % less (what the estimates are off by), this tile's time in us: 1.13 a K step (half tiles
+    // 0.72 or, behind other rounds, 0.85) and 5 a round, sums as theirs. Few rows or columns leave it most compute units idle or many sums. us, before -> here: 937 x 4096 x 4096 49.5
+    // -> 37.7, 1000 x 2048 x 2048 25.5 -> 20.3, 500 rows 23.9 -> 17.4, 700 x 3072 x 2048 25.7 -> 20.4, 1400 x 2048 x 4096 42 -> 36, 700 x 1024 x 4096
+    // 27.2 -> 20.9, 400 x 2688 x 1024 25.4 -> 12.9, 1000 x 8192 x 8192 stays (102 and 105).
+    if (mid_ok) {
+      const int halved = p.sk == 1 ? big4_halved(tiles) : 0;
+      const double big = (double)(((long)(tiles - halved) * p.sk + 255) / 256) * (1.13 * steps / p.sk + 5) +
+                         (halved ? (tiles > 256 ? 0.85 : 0.72) * steps + 5 : 0) + (p.sk > 1 ? 2 + 2e-6 * p.sk * M * N : 0);
+      if (mid < 0.85 * big) return pm;
     }
     if (N % 256 == 0) return p;
     // N % 256 == 128: half of the last column tile is wasted and 128 x 128 tiles have four times as many workgroups, two of
@@ -2526,6 +2570,9 @@ int gemm_rowscale_check(int M, int N, int K, int epi) {
   if (M <= 0) return 0;
   const RowScale probe{nullptr, 0, 0.f, 0.f};
   if (gemm_streams(M, N, K, epi)) return -4;      // streamed without one
+  // (whole column tiles of many rows: behind a norm in one launch, whichever tile runs)
+  GemmPlan t;
+  if (M > 256 && N % 256 == 0 && !tuned_plan(M, N, K, t)) return -4;
   return run_plan(select_plan(M, N, K, epi, true), nullptr, 0, nullptr, 0, M, N, K, epi, nullptr, nullptr, 0,
                   nullptr, nullptr, true, false, &probe);
 }
