@@ -248,7 +248,8 @@ __global__ void rope_table_kernel(const int* __restrict__ positions, const float
 // (lane l owns dims l, l + 64, ...: NL per lane), staged in LDS so that a rotated dimension finds its
 // partner, and leaves rotated. A wave's HPW heads go through each phase together (all loads, all
 // reductions, all hand-overs, all stores), so their latencies overlap: large steps take HPW = 4,
-// steps of few rows HPW = 1 (more workgroups).
+// steps of few rows HPW = 1 (more workgroups). Neighbouring tokens of a large step run on one die, whose L2
+// then gathers whole lines of the transposed values: 6184 tokens of 16 + 4 heads of 128 48.6 -> 46 us.
 template <typename T, int HPW, int NL>
 __global__ __launch_bounds__(256) void qk_norm_rope_kv_kernel(const T* __restrict__ q, long q_ld, const T* __restrict__ k,
                                                               long k_ld, const T* __restrict__ v, long v_ld,
@@ -259,7 +260,7 @@ __global__ __launch_bounds__(256) void qk_norm_rope_kv_kernel(const T* __restric
                                                               T* __restrict__ k_cache, T* __restrict__ v_cache, int Hq,
                                                               int Gk, int Gv, int D, int Dp, int Dv, int Dvp, int bs) {
   extern __shared__ float smem[];        // head staging [4][HPW][D]
-  const long t = blockIdx.x;
+  const long t = HPW > 1 ? xcd_remap(blockIdx.x, gridDim.x) : blockIdx.x;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const float* scos = cs + t * 2 * nrot;       // the token's row of the step's rotation table
   const float* ssin = scos + nrot;

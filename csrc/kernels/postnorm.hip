@@ -32,6 +32,23 @@ __global__ __launch_bounds__(256) void embed_scaled_kernel(const int* __restrict
   for (int c = threadIdx.x; c < W; c += blockDim.x) out[t * W + c] = (float)row[c] * scale;
 }
 
+// The same four columns at a time, a few per thread (W % 4 == 0): 6184 rows of 2048 27.1 -> 17.9 us (4.2 TB/s)
+template <typename T>
+__global__ __launch_bounds__(256) void embed_scaled4_kernel(const int* __restrict__ ids, const T* __restrict__ table, float scale,
+                                                            float* __restrict__ out, int T_, int W, int vocab) {
+  typedef T tv __attribute__((ext_vector_type(4)));
+  const int per = W / 4;
+  for (long i = blockIdx.x * 256L + threadIdx.x; i < (long)T_ * per; i += gridDim.x * 256L) {
+    const long t = i / per;
+    const int c = 4 * (int)(i - t * per), id = min(max(ids[t], 0), vocab - 1);
+    const tv v = *reinterpret_cast<const tv*>(table + (long)id * W + c);
+    f32x4 o;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) o[e] = (float)v[e] * scale;
+    *reinterpret_cast<f32x4*>(out + t * W + c) = o;
+  }
+}
+
 // the sequence whose row range holds row t (row_cu is non-decreasing; -1: none)
 __device__ __forceinline__ int seq_of_row(const int* __restrict__ row_cu, int nseq, int t) {
   int lo = 0, hi = nseq;            // the last s with row_cu[s] <= t
@@ -336,6 +353,56 @@ __global__ __launch_bounds__(1024) void layer_norm_rows_kernel(const float* __re
   for (int c = threadIdx.x; c < W; c += blockDim.x) out[i * W + c] = (TO)((sy[c] - mean) * rstd * nw[c] + nb[c]);
 }
 
+// The same with the row in registers (W % 4 == 0, W <= 1024 NV): all of it is asked for at once and two sums go through LDS.
+// 6184 rows of 2048 to bf16 37.2 -> 13.9 us (5.5 TB/s), one row of 1024 6.3 -> 3.6.
+template <typename TO, int NV>
+__global__ __launch_bounds__(256) void layer_norm_regs_kernel(const float* __restrict__ x, const float* __restrict__ nw,
+                                                              const float* __restrict__ nb, float eps,
+                                                              const long* __restrict__ idx, TO* __restrict__ out, int W) {
+  typedef TO tv __attribute__((ext_vector_type(4)));
+  __shared__ float red[2][4];
+  const long i = blockIdx.x, t = idx ? idx[i] : i;
+  const int tid = threadIdx.x;
+  f32x4 v[NV], wv[NV], bv[NV];
+#pragma unroll
+  for (int j = 0; j < NV; ++j) {
+    const int c = 4 * tid + 1024 * j;
+    v[j] = wv[j] = bv[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    if (c >= W) continue;
+    v[j] = *reinterpret_cast<const f32x4*>(x + t * W + c);
+    wv[j] = *reinterpret_cast<const f32x4*>(nw + c);
+    bv[j] = *reinterpret_cast<const f32x4*>(nb + c);
+  }
+  const auto all = [&](float a, int slot) {
+    a = wave_sum(a);
+    if ((tid & 63) == 0) red[slot][tid >> 6] = a;
+    __syncthreads();
+    return (red[slot][0] + red[slot][1]) + (red[slot][2] + red[slot][3]);
+  };
+  float a = 0.f, q = 0.f;
+#pragma unroll
+  for (int j = 0; j < NV; ++j) a += (v[j][0] + v[j][1]) + (v[j][2] + v[j][3]);
+  const float mean = all(a, 0) / (float)W;
+#pragma unroll
+  for (int j = 0; j < NV; ++j)
+    if (4 * tid + 1024 * j < W)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float d = v[j][e] - mean;
+        q = fmaf(d, d, q);
+      }
+  const float rstd = 1.f / sqrtf(all(q, 1) / (float)W + eps);
+#pragma unroll
+  for (int j = 0; j < NV; ++j) {
+    const int c = 4 * tid + 1024 * j;
+    if (c >= W) continue;
+    tv o;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) o[e] = (TO)((v[j][e] - mean) * rstd * wv[j][e] + bv[j][e]);
+    *reinterpret_cast<tv*>(out + i * W + c) = o;
+  }
+}
+
 }  // namespace
 
 // threads of a one-row workgroup: about four elements per thread, whole waves, at most 1024
@@ -344,6 +411,12 @@ static int row_threads(int W) { return std::min(1024, std::max(64, (W / 4 + 63) 
 void launch_embed_scaled(const int* ids, const void* table, float scale, float* out, int T, int W, int vocab, bool f32,
                          hipStream_t s) {
   if (T <= 0) return;
+  if (W % 4 == 0 && reinterpret_cast<uintptr_t>(table) % (f32 ? 16 : 8) == 0 && reinterpret_cast<uintptr_t>(out) % 16 == 0) {
+    const int blocks = (int)std::min<long>(((long)T * (W / 4) + 255) / 256, 4096);
+    if (f32) embed_scaled4_kernel<float><<<blocks, 256, 0, s>>>(ids, (const float*)table, scale, out, T, W, vocab);
+    else embed_scaled4_kernel<bf16><<<blocks, 256, 0, s>>>(ids, (const bf16*)table, scale, out, T, W, vocab);
+    return;
+  }
   if (f32) embed_scaled_kernel<float><<<T, 256, 0, s>>>(ids, (const float*)table, scale, out, W, vocab);
   else embed_scaled_kernel<bf16><<<T, 256, 0, s>>>(ids, (const bf16*)table, scale, out, W, vocab);
 }
@@ -427,6 +500,17 @@ void launch_rope_heads_copy(const void* src, long s_ld, long s_hd, void* dst, lo
 void launch_layer_norm_rows(const float* x, const float* nw, const float* nb, float eps, const long* idx, void* out,
                             int R, int W, bool f32, hipStream_t s) {
   if (R <= 0) return;
+  const auto al = [](const void* p, int n) { return reinterpret_cast<uintptr_t>(p) % n == 0; };
+  if (W % 4 == 0 && W <= 8192 && al(x, 16) && al(nw, 16) && al(nb, 16) && al(out, f32 ? 16 : 8)) {
+#define BFLY_LN(NV)                                                                                              \
+  {                                                                                                              \
+    if (f32) layer_norm_regs_kernel<float, NV><<<R, 256, 0, s>>>(x, nw, nb, eps, idx, (float*)out, W);           \
+    else layer_norm_regs_kernel<bf16, NV><<<R, 256, 0, s>>>(x, nw, nb, eps, idx, (bf16*)out, W);                 \
+  }
+    if (W <= 1024) BFLY_LN(1) else if (W <= 2048) BFLY_LN(2) else if (W <= 4096) BFLY_LN(4) else BFLY_LN(8)
+#undef BFLY_LN
+    return;
+  }
   const size_t sm = (size_t)W * sizeof(float);
   if (f32) layer_norm_rows_kernel<float><<<R, row_threads(W), sm, s>>>(x, nw, nb, eps, idx, (float*)out, W);
   else layer_norm_rows_kernel<bf16><<<R, row_threads(W), sm, s>>>(x, nw, nb, eps, idx, (bf16*)out, W);
