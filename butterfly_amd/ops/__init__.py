@@ -996,7 +996,7 @@ def moe_route_scores(x, wr, top_k: int, scoring: str = "softmax", renorm: bool =
             int(groups[1]), float(renorm_eps), float(scale))
     E = wr.shape[0]
     form = route_form(T, E, x.shape[1], x.dtype == torch.float32, wr.is_contiguous())
-    if form == "one launch":
+    if form == "one launch" or torch.ops.bfly.moe_route_tiles(x, wr, top_k, int(groups[0]), int(groups[1])):
         torch.ops.bfly.moe_route_rows(x, wr, *rest)
         return ids, w
     if form == "waves":      # one wave per token (steps of a few rows: per token and expert)
@@ -1030,7 +1030,7 @@ def _moe_glu(x, topk_ids, topk_w, gate_up_w, down_w, limit, alpha, up_offset, sc
     TK = T * topk_ids.shape[1]
     mt = torch.ops.bfly.moe_sort_max_tiles(TK, E)
     dev = x.device
-    work = _arena.get(dev, "moe_glu_work", TK + E + 1 + 2 * mt + 1, torch.int32)
+    work = _arena.get(dev, "moe_glu_work", TK + E + 1 + 2 * mt + 1 + torch.ops.bfly.moe_sort_counts(TK, E), torch.int32)
     hmid = _arena.get(dev, "moe_glu_mid", TK * F, x.dtype)
     y = _arena.get(dev, "moe_glu_y", TK * H, torch.float32)
     out = None if rows else _empty(T, H, dtype=x.dtype, device=dev)

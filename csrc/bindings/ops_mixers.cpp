@@ -405,9 +405,17 @@ void moe_route_rows(const Tensor& x, const Tensor& wr, const optional<Tensor>& b
                           (int)ngroups, (int)keep, (float)renorm_eps, (float)scale);
 }
 
+// whether moe_route_rows takes a large step on the matrix cores
+bool moe_route_tiles(const Tensor& x, const Tensor& wr, int64_t top_k, int64_t ngroups, int64_t keep) {
+  return wr.is_contiguous() && x.dim() == 2 && x.stride(1) == 1 && bfly::route_tiles_ok(x.data_ptr(), x.stride(0), wr.data_ptr(), (int)x.size(1), (int)top_k, (int)x.size(0),
+                                                    (int)wr.size(0), is_f32(x), (int)ngroups, (int)keep);
+}
+
 int64_t moe_sort_max_tiles(int64_t TK, int64_t E) { return bfly::moe_sort_max_tiles((int)TK, (int)E); }
 
-// work: int32 [TK + (E + 1) + 2 * max_tiles + 1] = perm | offsets | tiles | ntiles
+int64_t moe_sort_counts(int64_t TK, int64_t E) { return bfly::moe_sort_counts((int)TK, (int)E); }
+
+// work: int32 [TK + (E + 1) + 2 * max_tiles + 1] = perm | offsets | tiles | ntiles, and moe_sort_counts more if there are any
 void moe_glu_ffn(const Tensor& x, const Tensor& topk_ids, const Tensor& topk_w, const Tensor& gate_up_w,
                  const Tensor& down_w, double limit, double alpha, double up_offset, bool scale_input, Tensor& work,
                  Tensor& hmid, Tensor& y, const optional<Tensor>& out, int64_t plain_act, const optional<Tensor>& addend,
@@ -447,6 +455,8 @@ void moe_glu_ffn(const Tensor& x, const Tensor& topk_ids, const Tensor& topk_w, 
   int* offsets = perm + TK;
   int* tiles = offsets + E + 1;
   int* ntiles = tiles + 2 * mt;
+  const int64_t nc = bfly::moe_sort_counts((int)TK, (int)E);
+  int* counts = nc > 0 && work.numel() >= TK + E + 1 + 2 * mt + 1 + nc ? ntiles + 1 : nullptr;
   hipStream_t s = cur_stream();
   const bool f32 = is_f32(x);
   const bool big = bfly::moe_big_ok(x.data_ptr(), x.stride(0), gate_up_w.data_ptr(), down_w.data_ptr(), hmid.data_ptr(),
@@ -459,7 +469,7 @@ void moe_glu_ffn(const Tensor& x, const Tensor& topk_ids, const Tensor& topk_w, 
   // tiles that this tile height can need (no more than rows)
   const int64_t gt = std::min(TK, tr > 64 ? (TK + tr - 1) / tr + E : mt);
   const int* ids = stream && bfly::moe_stream_unsorted((int)TK) ? topk_ids.data_ptr<int>() : nullptr;
-  if (!ids) bfly::launch_moe_sort(topk_ids.data_ptr<int>(), (int)TK, (int)E, perm, offsets, tiles, ntiles, tr, s);
+  if (!ids) bfly::launch_moe_sort(topk_ids.data_ptr<int>(), (int)TK, (int)E, perm, offsets, tiles, ntiles, tr, s, counts);
   // scores on the expert's input (the row is scaled and the outputs are summed) or on its output
   bfly::launch_moe_glu_up(x.data_ptr(), x.stride(0), scale_input ? topk_w.data_ptr<float>() : nullptr, (int)K, perm,
                           offsets, tiles, ntiles, (int)gt, gate_up_w.data_ptr(), (float)limit, (float)alpha,
@@ -527,7 +537,9 @@ TORCH_LIBRARY_FRAGMENT(bfly, m) {
         "Tensor(b!) w, Tensor? select_bias=None, int ngroups=1, int keep=1, float renorm_eps=0.0, float scale=1.0) -> ()");
   m.def("moe_route_rows(Tensor x, Tensor wr, Tensor? bias, int top_k, int scoring, bool renorm, Tensor(a!) ids, "
         "Tensor(b!) w, Tensor? select_bias=None, int ngroups=1, int keep=1, float renorm_eps=0.0, float scale=1.0) -> ()");
+  m.def("moe_route_tiles(Tensor x, Tensor wr, int top_k, int ngroups, int keep) -> bool");
   m.def("moe_sort_max_tiles(int tk, int experts) -> int", &moe_sort_max_tiles);
+  m.def("moe_sort_counts(int tk, int experts) -> int", &moe_sort_counts);
   m.def("moe_sum(Tensor y, Tensor? w, int choices, Tensor(a!) out) -> ()");
   m.def("moe_glu_ffn(Tensor x, Tensor topk_ids, Tensor topk_w, Tensor gate_up_w, Tensor down_w, float limit, "
         "float alpha, float up_offset, bool scale_input, Tensor(a!) work, Tensor(b!) hmid, Tensor(c!) y, "
@@ -536,6 +548,7 @@ TORCH_LIBRARY_FRAGMENT(bfly, m) {
 
 TORCH_LIBRARY_IMPL(bfly, CUDA, m) {
   m.impl("sample_greedy_f32", &sample_greedy_f32);
+  m.impl("moe_route_tiles", &moe_route_tiles);
   m.impl("gemm_any", &gemm_any);
   m.impl("linear_heads", &linear_heads);
   m.impl("act_", &act_);

@@ -141,14 +141,17 @@ void launch_router_logits(const void* x, long ldx, const void* wr, float* logits
 void launch_moe_topk_scores(const float* logits, const float* bias, int top_k, int scoring, bool renorm, int* ids,
                             float* w, int T, int E, hipStream_t s, const float* select_bias = nullptr, int ngroups = 1,
                             int keep = 1, float renorm_eps = 0.f, float scale = 1.f);
-// both in one launch, for steps of a few rows and E <= 64
+// both in one launch, for steps of a few rows and E <= 64, and for large ones where route_tiles_ok
+bool route_tiles_ok(const void* x, long ldx, const void* wr, int Hd, int top_k, int T, int E, bool f32, int ngroups, int keep);
 void launch_route_rows(const void* x, long ldx, const void* wr, int Hd, const float* bias, int top_k, int scoring, bool renorm,
                        int* ids, float* w, int T, int E, bool f32, hipStream_t s, const float* select_bias = nullptr,
                        int ngroups = 1, int keep = 1, float renorm_eps = 0.f, float scale = 1.f);
 // Group the T*K (token, choice) pairs by expert: perm [TK] pair indices grouped by expert,
 // offsets [E + 1], tiles [max_tiles][2] = (expert, first row) of every tile_rows-row tile, ntiles [1].
+// counts (nullable): moe_sort_counts words of scratch, with which many pairs are dealt out to workgroups.
 void launch_moe_sort(const int* ids, int TK, int E, int* perm, int* offsets, int* tiles, int* ntiles, int tile_rows,
-                     hipStream_t s);
+                     hipStream_t s, int* counts = nullptr);
+int moe_sort_counts(int TK, int E);      // 0: one workgroup is as fast
 int moe_sort_max_tiles(int TK, int E);
 // rows per tile of the grouped expert GEMMs for this problem (64, 128 for large bf16 groups and, where `parts` allows, f32 ones,
 // 256 where `big` allows the LDS-DMA tile: moe_parts_ok, moe_big_ok)
