@@ -2201,21 +2201,34 @@ GemmPlan plan_gemm(int M, int N, int K) {
   return tuned_plan(M, N, K, p) ? p : plan_gemm_heuristic(M, N, K);
 }
 
-// LDS-tiled kernel: 16 to 128 rows per tile, split K until the grid has `target` workgroups
+// LDS-tiled kernel: 16 to 128 rows per tile, K split in two until there are 448 workgroups. Where that fills the chip with
+// more than 16 column tiles, up to 64 rows (a weight stream) take the split with the least of the stream (all of it at 6.3 TB/s, the busiest compute unit's at 40 KB a microsecond, rows of
+// X at 0.6 of the weights' cost) and the sums (1 us, 0.2 a split, 0.65 per MB): 2 % off the best of 16 splits on average over 26 N x K by
+// 6, 16, 32, 64 rows with weights from memory, where 448 workgroups were 19 % off (a few past a round of 256, or sums for nothing). us, before -> here: 8320 x 2048 by
+// 32 rows 19.0 -> 13.3, by 48 21.9 -> 15.3, 16384 x 2048 by 16 18.2 -> 15.9, 12416 x 4096 by 32 31.1 -> 26, 5120 x 6144 by 6 21.7 -> 17.4.
 static GemmPlan plan_tile(int M, int N, int K) {
   GemmPlan p{};
   const int target = 448;
   p.kind = 1;
-  p.mt = M >= 512 ? 2 : 3;   // tile plans: `mt` = pipeline depth (K-tiles in flight + 1)
+  p.mt = M >= 512 ? 2 : M > 64 ? 3 : 4;   // tile plans: `mt` = pipeline depth (K-tiles in flight + 1)
   if (M <= 16) { p.bm = 16; p.wk = 1; }
   else if (M <= 32) { p.bm = 32; p.wk = 1; }
   else if (M <= 64) { p.bm = 64; p.wk = 2; }
   else { p.bm = 128; p.wk = 2; }
   p.bn = 128;
   const int tiles = ((M + p.bm - 1) / p.bm) * (N / p.bn);
+  if (M > 32 && M <= 64 && tiles > 256) p.mt = 3;      // (two workgroups a compute unit: 128256 x 4096 by 40 rows 182 and 190)
   int sk = 1;
   const int ktiles = K / kBK;
   while (tiles * sk < target && sk * 2 * 4 <= ktiles && sk < 16) sk *= 2;
+  if (M <= 64 && tiles * sk >= 256 && tiles > 16) {
+    double least = 0;
+    for (int n = 1; n <= 16 && (n == 1 || ktiles >= 4 * n); ++n) {
+      const double unit = ((long)tiles * n + 255) / 256 * (K / (double)n) * (256 + 1.2 * M);      // bytes
+      const double us = std::max(2. * N * K / 6.3e6, unit / 40e3) + (n > 1 ? 1 + 0.2 * n + 2.6e-6 * n * M * N : 0);
+      if (n == 1 || us < least) least = us, sk = n;
+    }
+  }
   p.sk = sk;
   return p;
 }
@@ -2519,7 +2532,8 @@ int launch_gemm_plan(const GemmPlan& p, const bf16* X, long ldx, const bf16* W, 
 // 8192 28.5 and 26.9). Up to eight rows where X does not weigh in: 4096 channels and 10240 columns (5120 x 2048 11.4 -> 8.3 us, 4096 x
 // 4096 9.9 -> 9.0; 14336 x 4096 23.6 and 25.2), in place of split sums 4096 x 4096 or 2048 channels (2048 x 2048 7.3 -> 4.6, read as
 // they are 5.1). Up to 16 rows to 1024 channels (1024 x 1024 5.9 -> 4.3), and to 2048 in place of split sums of a product that widens
-// its rows (3072 x 2048 9.6 -> 6.8; those of one that does not are read as they are: 2048 x 2048 5.4 and 6.6). Up to 32 rows to 1024 channels
+// its rows, to two rounds of its tiles (3072 x 2048 9.6 -> 7.0, 8320 x 2048 15.8 and 11.7; those of one that does not are read as they are:
+// 2048 x 2048 5.4 and 6.6). Up to 32 rows to 1024 channels
 // and 4096 columns (2688 x 1024 7.4 -> 5.4).
 static bool stream_plan(int M, int N, int K, int epi, const GemmPlan& base, GemmPlan& p) {
   if (M > 32 || K % 128 != 0 || epi == EPI_SILU_GATE || !plan_overrides().empty()) return false;
@@ -2529,7 +2543,7 @@ static bool stream_plan(int M, int N, int K, int epi, const GemmPlan& base, Gemm
   } else if (M <= 8) {
     if (K > 4096 || N > 10240 || (split && K > 2048 && N > 4096)) return false;
   } else if (M <= 16) {
-    if (!(!split && K <= 1024 && N <= 8192) && !(split && K <= 2048 && N > K && N <= 10240)) return false;
+    if (!(!split && K <= 1024 && N <= 8192) && !(split && K <= 2048 && N > K && N <= 8192)) return false;
   } else if (split || K > 1024 || N > 4096) {
     return false;
   }

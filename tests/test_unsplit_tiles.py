@@ -42,3 +42,15 @@ def test_packed(M, N, K):
 @pytest.mark.parametrize("N,K", [(8320, 1024), (16512, 64), (16512, 960), (32000, 1024)])
 def test_short(M, N, K):
     _check(M, N, K, False)
+
+
+@pytest.mark.parametrize("M,N,K,sk", [(16, 8320, 2048, 3), (64, 8320, 2048, 3), (32, 16384, 2048, 2), (32, 2048, 2048, 8), (16, 1024, 1536, 4)])
+def test_splits_of_streams(M, N, K, sk):
+    p = ops.gemm_plan(M, N, K)
+    assert (p["kind"], p["splitk"]) == ("tile", sk)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(16, 8320, 2048), (17, 12416, 1280), (33, 8448, 1088), (64, 16640, 320), (48, 12416, 4096)])
+def test_splits_that_divide_nothing(M, N, K):
+    _check(M, N, K, N % 256 == 0)
