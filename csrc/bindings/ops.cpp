@@ -359,9 +359,9 @@ std::vector<int64_t> gemm_plan(int64_t M, int64_t N, int64_t K) {
   return {p.kind, p.mt, p.nt, p.bm, p.bn, p.sk, p.wk};
 }
 
-// whether gemm() of few rows streams its weights (without a row scale)
+// whether gemm() of few rows streams its weights (without a row scale) faster than gemm_packed() takes a packed copy
 bool gemm_streams(int64_t M, int64_t N, int64_t K, int64_t epilogue) {
-  return bfly::gemm_streams((int)M, (int)N, (int)K, (int)epilogue);
+  return bfly::gemm_streams((int)M, (int)N, (int)K, (int)epilogue) && !bfly::gemm_packed_first((int)M, (int)N, (int)K);
 }
 
 void gemm(const Tensor& x, const Tensor& w, Tensor& out, const c10::optional<Tensor>& bias,

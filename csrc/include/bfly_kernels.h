@@ -122,6 +122,7 @@ int launch_gemm_plan(const GemmPlan& p, const bf16* X, long ldx, const bf16* W, 
                      int N, int K, int epi, const bf16* bias, bf16* out, long ldo, float* ws,
                      size_t ws_bytes, hipStream_t stream);
 int gemm_check(int M, int N, int K, int epi);
+bool gemm_packed_first(int M, int N, int K);           // ... but not where a packed copy of the weights is there
 bool gemm_streams(int M, int N, int K, int epi);      // the plan is the streamed product of few rows
 // 0 if the auto plan for this shape takes a RowScale (tile and decode-ring kernels)
 int gemm_rowscale_check(int M, int N, int K, int epi);

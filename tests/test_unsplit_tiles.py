@@ -54,3 +54,11 @@ def test_splits_of_streams(M, N, K, sk):
 @pytest.mark.parametrize("M,N,K", [(16, 8320, 2048), (17, 12416, 1280), (33, 8448, 1088), (64, 16640, 320), (48, 12416, 4096)])
 def test_splits_that_divide_nothing(M, N, K):
     _check(M, N, K, N % 256 == 0)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M", [1, 2, 3, 4, 5])
+@pytest.mark.parametrize("N,K", [(7936, 4096), (8192, 4096), (8448, 8192), (28672, 4096), (8192, 4032)])
+def test_packed_weights_of_many_columns(M, N, K):
+    """Two to four rows run the tiles of five; both sides of the rule's lines."""
+    _check(M, N, K, True)
