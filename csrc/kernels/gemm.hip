@@ -2323,12 +2323,13 @@ static GemmPlan plan_gemm_heuristic(int M, int N, int K) {
     // The mid-M tiles where they take 15 % less (what the estimates are off by), this tile's time in us: 1.13 a K step (half tiles
     // 0.72 or, behind other rounds, 0.85) and 5 a round, sums as theirs. Few rows or columns leave it most compute units idle or many sums. us, before -> here: 937 x 4096 x 4096 49.5
     // -> 37.7, 1000 x 2048 x 2048 25.5 -> 20.3, 500 rows 23.9 -> 17.4, 700 x 3072 x 2048 25.7 -> 20.4, 1400 x 2048 x 4096 42 -> 36, 700 x 1024 x 4096
-    // 27.2 -> 20.9, 400 x 2688 x 1024 25.4 -> 12.9, 1000 x 8192 x 8192 stays (102 and 105).
+    // 27.2 -> 20.9, 400 x 2688 x 1024 25.4 -> 12.9, 1000 x 8192 x 8192 stays (102 and 105). Up to 320 rows plans keep their splits, whose sums'
+    // order row kernels are compared in (300 x 2048 x 2048 20.6 where a mid-M tile takes 13.2).
     if (mid_ok) {
       const int halved = p.sk == 1 ? big4_halved(tiles) : 0;
       const double big = (double)(((long)(tiles - halved) * p.sk + 255) / 256) * (1.13 * steps / p.sk + 5) +
                          (halved ? (tiles > 256 ? 0.85 : 0.72) * steps + 5 : 0) + (p.sk > 1 ? 2 + 2e-6 * p.sk * M * N : 0);
-      if (mid < 0.85 * big) return pm;
+      if (M > 320 && mid < 0.85 * big) return pm;
     }
     if (N % 256 == 0) return p;
     // N % 256 == 128: half of the last column tile is wasted and 128 x 128 tiles have four times as many workgroups, two of
