@@ -2210,18 +2210,19 @@ static GemmPlan plan_tile(int M, int N, int K) {
   GemmPlan p{};
   const int target = 448;
   p.kind = 1;
-  p.mt = M >= 512 ? 2 : M > 64 ? 3 : 4;   // tile plans: `mt` = pipeline depth (K-tiles in flight + 1)
+  const bool stream = M <= 64 && 2. * N * K <= 300e6;      // (what the estimate was fitted to; 8192 x 28672 stays at eight splits)
+  p.mt = M >= 512 ? 2 : stream ? 4 : 3;   // tile plans: `mt` = pipeline depth (K-tiles in flight + 1)
   if (M <= 16) { p.bm = 16; p.wk = 1; }
   else if (M <= 32) { p.bm = 32; p.wk = 1; }
   else if (M <= 64) { p.bm = 64; p.wk = 2; }
   else { p.bm = 128; p.wk = 2; }
   p.bn = 128;
   const int tiles = ((M + p.bm - 1) / p.bm) * (N / p.bn);
-  if (M > 32 && M <= 64 && tiles > 256) p.mt = 3;      // (two workgroups a compute unit: 128256 x 4096 by 40 rows 182 and 190)
+  if (M > 32 && stream && tiles > 256) p.mt = 3;      // (two workgroups a compute unit)
   int sk = 1;
   const int ktiles = K / kBK;
   while (tiles * sk < target && sk * 2 * 4 <= ktiles && sk < 16) sk *= 2;
-  if (M <= 64 && tiles * sk >= 256 && tiles > 16) {
+  if (stream && tiles * sk >= 256 && tiles > 16) {
     double least = 0;
     for (int n = 1; n <= 16 && (n == 1 || ktiles >= 4 * n); ++n) {
       const double unit = ((long)tiles * n + 255) / 256 * (K / (double)n) * (256 + 1.2 * M);      // bytes
