@@ -548,11 +548,17 @@ def linear_silu_gate(x, w, gates, e0: int, num_local: int, packed=None):
     return out
 
 
-def gemm_plan(M: int, N: int, K: int) -> dict:
+def gemm_plan(M: int, N: int, K: int, epilogue=None, ldx=None, ldw=None) -> dict:
+    """The planner's choice for a product of M rows; with an `epilogue`, what `linear` runs for it on rows ldx and ldw apart (K where
+    not given): few rows stream their weights instead (kind "stream"), rows that a tile cannot reach go to one that does."""
     load_library()
-    k, mt, nt, bm, bn, sk, wk = torch.ops.bfly.gemm_plan(M, N, K)
-    return {"kind": ("skinny", "tile", "big", "dec", "big8", "mid8", "big4", "mid4")[k], "mt": mt, "nt": nt, "wk": wk, "bm": bm, "bn": bn,
-            "splitk": sk}
+    if epilogue is None:
+        p = torch.ops.bfly.gemm_plan(M, N, K)
+    else:
+        p = torch.ops.bfly.gemm_call_plan(M, N, K, EPILOGUES[epilogue], K if ldx is None else ldx, K if ldw is None else ldw)
+    k, mt, nt, bm, bn, sk, wk = p
+    return {"kind": ("skinny", "tile", "big", "dec", "big8", "mid8", "big4", "mid4", "stream")[k], "mt": mt, "nt": nt, "wk": wk, "bm": bm,
+            "bn": bn, "splitk": sk}
 
 
 def attn_prefill(q, k, v, cu_seqlens, max_seqlen: int, scale: float, causal: bool = True,

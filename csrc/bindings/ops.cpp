@@ -354,9 +354,13 @@ int64_t gemm_workspace_size(int64_t M, int64_t N, int64_t K) {
   return (int64_t)bfly::gemm_workspace_bytes(M, N, K);
 }
 
-std::vector<int64_t> gemm_plan(int64_t M, int64_t N, int64_t K) {
-  const bfly::GemmPlan p = bfly::plan_gemm(M, N, K);
-  return {p.kind, p.mt, p.nt, p.bm, p.bn, p.sk, p.wk};
+static std::vector<int64_t> plan_list(const bfly::GemmPlan& p) { return {p.kind, p.mt, p.nt, p.bm, p.bn, p.sk, p.wk}; }
+
+std::vector<int64_t> gemm_plan(int64_t M, int64_t N, int64_t K) { return plan_list(bfly::plan_gemm(M, N, K)); }
+
+// what gemm() runs on rows ldx and ldw apart
+std::vector<int64_t> gemm_call_plan(int64_t M, int64_t N, int64_t K, int64_t epilogue, int64_t ldx, int64_t ldw) {
+  return plan_list(bfly::gemm_call_plan((int)M, (int)N, (int)K, (int)epilogue, ldx, ldw));
 }
 
 // whether gemm() of few rows streams its weights (without a row scale) faster than gemm_packed() takes a packed copy
@@ -1234,6 +1238,7 @@ TORCH_LIBRARY(bfly, m) {
   m.def("gemm_workspace_size(int M, int N, int K) -> int", &gemm_workspace_size);
   m.def("gemm_workspace_bound(int M, int N, int K) -> int", &gemm_workspace_bound);
   m.def("gemm_plan(int M, int N, int K) -> int[]", &gemm_plan);
+  m.def("gemm_call_plan(int M, int N, int K, int epilogue, int ldx, int ldw) -> int[]", &gemm_call_plan);
   m.def("gemm_streams(int M, int N, int K, int epilogue) -> bool", &gemm_streams);
   m.def("gemm_check(int M, int N, int K, int epilogue) -> int",
         [](int64_t M, int64_t N, int64_t K, int64_t e) -> int64_t { return bfly::gemm_check(M, N, K, e); });

@@ -121,6 +121,8 @@ size_t gemm_workspace_bytes(int M, int N, int K);
 int launch_gemm_plan(const GemmPlan& p, const bf16* X, long ldx, const bf16* W, long ldw, int M,
                      int N, int K, int epi, const bf16* bias, bf16* out, long ldo, float* ws,
                      size_t ws_bytes, hipStream_t stream);
+// The plan that launch_gemm runs (without a row scale) on rows ldx and ldw apart; plan_gemm's is where it starts from
+GemmPlan gemm_call_plan(int M, int N, int K, int epi, long ldx, long ldw);
 int gemm_check(int M, int N, int K, int epi);
 bool gemm_packed_first(int M, int N, int K);           // ... but not where a packed copy of the weights is there
 bool gemm_streams(int M, int N, int K, int epi);      // the plan is the streamed product of few rows

@@ -2518,12 +2518,23 @@ static int run_plan(const GemmPlan& p, const bf16* X, long ldx, const bf16* W, l
   return 0;
 }
 
+// Whether a plan's kernel finds rows ldx and ldw apart. Those that load through buffer descriptors (kinds 4 to 7) have a row's place in a
+// tile as 32-bit byte offset below 2^31, and what lies behind rows * ld bytes reads as zeros: rows that overlap, or are one and the same
+// (an expanded vector), as much as rows far apart. The others address each row in 64 bits.
+static bool plan_reaches(const GemmPlan& p, int K, long ldx, long ldw) {
+  if (p.kind < 4 || p.kind > 7) return true;
+  const bool mid = p.kind == 5 || p.kind == 7;
+  const long reach = 0x7fffffffL / 2, bm = mid ? p.bm : 256, bn = mid ? p.bn : 256;
+  return ldx >= K && ldw >= K && ldx <= reach / bm && ldw <= reach / bn;
+}
+
 int launch_gemm_plan(const GemmPlan& p, const bf16* X, long ldx, const bf16* W, long ldw, int M,
                      int N, int K, int epi, const bf16* bias, bf16* out, long ldo, float* ws,
                      size_t ws_bytes, hipStream_t stream) {
   if (M <= 0) return 0;
   if (p.sk > 1 && (ws == nullptr || ws_bytes < kCounterBytes + (size_t)p.sk * M * N * sizeof(float)))
     return -3;
+  if (!plan_reaches(p, K, ldx, ldw)) return -6;
   return run_plan(p, X, ldx, W, ldw, M, N, K, epi, bias, out, ldo, ws, stream);
 }
 
@@ -2579,6 +2590,22 @@ static GemmPlan select_plan(int M, int N, int K, int epi, bool row_scale = false
     p = plan_gemm_heuristic(M, N, K);
   if (row_scale) return rowscale_on_tile(p, N) ? plan_tile(M, N, K) : p;
   return stream_plan(M, N, K, epi, p, q) ? q : p;
+}
+
+// The plan for operands with these row pitches: where its kernel does not reach the rows, 128-row tiles, K split as far as the workspace holds
+static GemmPlan call_plan(int M, int N, int K, int epi, bool row_scale, long ldx, long ldw, size_t ws_bytes) {
+  const auto parts = [&](int sk) { return kCounterBytes + (size_t)sk * M * N * sizeof(float); };
+  GemmPlan p = select_plan(M, N, K, epi, row_scale);
+  if (!plan_reaches(p, K, ldx, ldw)) {
+    p = plan_tile(M, N, K);
+    while (p.sk > 1 && ws_bytes < parts(p.sk)) --p.sk;
+  }
+  if (p.sk > 1 && ws_bytes < parts(p.sk)) p.sk = 1;
+  return p;
+}
+
+GemmPlan gemm_call_plan(int M, int N, int K, int epi, long ldx, long ldw) {
+  return call_plan(M, N, K, epi, false, ldx, ldw, ~(size_t)0);
 }
 
 bool gemm_streams(int M, int N, int K, int epi) { return M > 0 && select_plan(M, N, K, epi).kind == 8; }
@@ -2703,9 +2730,7 @@ int launch_gemm_deferred(const bf16* X, long ldx, const bf16* W, long ldw, int M
                          bf16* out, long ldo, float* ws, size_t ws_bytes, hipStream_t stream,
                          const RowScale* rs) {
   if (M <= 0) return 1;
-  GemmPlan p = select_plan(M, N, K, EPI_NONE, rs != nullptr);
-  if (p.sk > 1 && (ws == nullptr || ws_bytes < kCounterBytes + (size_t)p.sk * M * N * sizeof(float)))
-    p.sk = 1;
+  const GemmPlan p = call_plan(M, N, K, EPI_NONE, rs != nullptr, ldx, ldw, ws ? ws_bytes : 0);
   const bool defer = p.sk > 1;
   const int rc = run_plan(p, X, ldx, W, ldw, M, N, K, EPI_NONE, nullptr, out, ldo, ws, stream,
                           false, defer, rs);
@@ -2727,9 +2752,7 @@ int launch_gemm(const bf16* X, long ldx, const bf16* W, long ldw, int M, int N, 
                 const bf16* bias, bf16* out, long ldo, float* ws, size_t ws_bytes,
                 hipStream_t stream, const RowScale* rs) {
   if (M <= 0) return 0;
-  GemmPlan p = select_plan(M, N, K, epi, rs != nullptr);
-  if (p.sk > 1 && (ws == nullptr || ws_bytes < kCounterBytes + (size_t)p.sk * M * N * sizeof(float)))
-    p.sk = 1;
+  const GemmPlan p = call_plan(M, N, K, epi, rs != nullptr, ldx, ldw, ws ? ws_bytes : 0);
   return run_plan(p, X, ldx, W, ldw, M, N, K, epi, bias, out, ldo, ws, stream, false, false, rs);
 }
 
@@ -2797,6 +2820,7 @@ int launch_gemm_packed(const bf16* X, long ldx, const bf16* Wp, int M, int N, in
     p = GemmPlan{1, 4, 1, M <= 32 ? 1 : 2, M <= 16 ? 16 : M <= 32 ? 32 : 64, 128, 1};
   // mid-M kernels (kinds 5 / 7): their weight DMA takes the packed layout as a template flag
   const bool mid = (p.kind == 5 || p.kind == 7) && (p.bn == 128 || p.bn == 256);
+  if (mid && !dry && !plan_reaches(p, K, ldx, K)) return -2;
   if (!mid && (p.kind != 1 || (p.bm != 16 && p.bm != 32 && p.bm != 64) || (p.bn != 128 && p.bn != 256))) return -2;
   if (!dry && p.sk > 1 && (ws == nullptr || ws_bytes < kCounterBytes + (size_t)p.sk * M * N * sizeof(float)))
     return -3;
