@@ -175,8 +175,7 @@ def reserve_workspace(device, max_tokens: int, max_n: int, max_k: int, max_batch
                       max_ctx: int = 0, num_kv_heads: int = 0, head_dim: int = 128, shapes=()) -> None:
     """Pre-size every workspace for problems up to the given bounds (call before capture).
     `shapes`: the model's GEMM weight shapes (N, K); the split-K slab need is the max over them
-    and every token-count bucket of the plan table (a tuned plan may split a small projection
-    more than the largest one is split) and every number of row tiles (a split's sums do not grow with the rows)."""
+    and every number of rows up to max_tokens (neither more rows nor a larger weight asks for more sums)."""
     if not load_library():
         return
     nk = {(int(max_n), int(max_k))} | {(int(n), int(k)) for n, k in shapes}

@@ -340,15 +340,7 @@ void tkp_final(Tensor& ws, int64_t rows, Tensor& thresh) {
   bfly::launch_tkp_final(v.state, rows, thresh.data_ptr<float>(), cur_stream());
 }
 
-// the most that any number of rows up to M asks for: the plan table's counts and every number of whole row tiles
-int64_t gemm_workspace_bound(int64_t M, int64_t N, int64_t K) {
-  if (M < 1) return 0;
-  size_t need = bfly::gemm_workspace_bytes((int)M, (int)N, (int)K);
-  for (int64_t m = 1; m <= 64; ++m)      // (fewer rows may split K more)
-    if (m < M) need = std::max(need, bfly::gemm_workspace_bytes((int)m, (int)N, (int)K));
-  for (int64_t m = 128; m < M; m += 128) need = std::max(need, bfly::gemm_workspace_bytes((int)m, (int)N, (int)K));
-  return (int64_t)need;
-}
+int64_t gemm_workspace_bound(int64_t M, int64_t N, int64_t K) { return (int64_t)bfly::gemm_workspace_bound((int)M, (int)N, (int)K); }
 
 int64_t gemm_workspace_size(int64_t M, int64_t N, int64_t K) {
   return (int64_t)bfly::gemm_workspace_bytes(M, N, K);

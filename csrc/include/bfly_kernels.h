@@ -118,6 +118,7 @@ void launch_tkp_final(const float* state, int rows, float* thresh, hipStream_t s
 // gemm.hip
 GemmPlan plan_gemm(int M, int N, int K);
 size_t gemm_workspace_bytes(int M, int N, int K);
+size_t gemm_workspace_bound(int M, int N, int K);      // for any number of rows up to M
 int launch_gemm_plan(const GemmPlan& p, const bf16* X, long ldx, const bf16* W, long ldw, int M,
                      int N, int K, int epi, const bf16* bias, bf16* out, long ldo, float* ws,
                      size_t ws_bytes, hipStream_t stream);

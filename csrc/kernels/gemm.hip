@@ -2354,12 +2354,21 @@ static size_t plan_ws_bytes(const GemmPlan& p, int M, int N) {
 // A row scale with a half column tile: the 256 x 256 tile's epilogue has none, the 128-row tiles' has
 static bool rowscale_on_tile(const GemmPlan& p, int N) { return p.kind == 6 && N % 256 != 0; }
 
-// Enough for the tuned plan and for the plans it may fall back to (below).
+// Enough for the tuned plan, for the plans it may fall back to (below) and for the one of five rows where packed weights take that.
 size_t gemm_workspace_bytes(int M, int N, int K) {
-  if (gemm_packed_first(M, N, K)) return gemm_workspace_bytes(5, N, K);
   const GemmPlan h = plan_gemm_heuristic(M, N, K);
   const size_t a = plan_ws_bytes(plan_gemm(M, N, K), M, N), b = plan_ws_bytes(h, M, N);
-  return std::max({a, b, rowscale_on_tile(h, N) ? plan_ws_bytes(plan_tile(M, N, K), M, N) : 0});
+  return std::max({a, b, rowscale_on_tile(h, N) ? plan_ws_bytes(plan_tile(M, N, K), M, N) : 0,
+                   gemm_packed_first(M, N, K) ? gemm_workspace_bytes(5, N, K) : 0});
+}
+
+// The most that any number of rows up to M asks for. Each is asked: fewer rows may split K more inside a row tile (2048 x 1024 4 MB at 256
+// rows, 8 at 244), and tiles change between any two (1 ms for 8192 rows). Beyond 512 tiles of 256 x 256 nothing is split.
+size_t gemm_workspace_bound(int M, int N, int K) {
+  const long split = 256L * std::max(2, 512 / ((N + 255) / 256));
+  size_t need = 0;
+  for (int m = 1; m <= (int)std::min<long>(M, split); ++m) need = std::max(need, gemm_workspace_bytes(m, N, K));
+  return need;
 }
 
 // `dry`: validate only (the plan is supported for this shape/epilogue) without launching.

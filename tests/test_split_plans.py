@@ -152,3 +152,34 @@ def test_results_of_the_large_tile_into_far_rows(epi):
     far = torch.empty(M * (1 << 20), device="cuda", dtype=torch.bfloat16).view(M, 1 << 20)[:, 3:3 + want.shape[1]]
     ops.linear(x, w, epilogue=epi, out=far)
     assert torch.equal(far, want)
+
+
+BOUNDED = [(2048, 1024), (2048, 8192), (1024, 1024), (28672, 4096), (8192, 4160), (3584, 4096), (4096, 7168), (4096, 4096), (6144, 4096),
+           (10240, 8192), (8192, 28672), (128, 512), (1152, 4096), (8320, 2048), (4224, 1024), (128256, 4096)]
+
+
+@pytest.mark.parametrize("shape", BOUNDED, ids=str)
+@pytest.mark.parametrize("most", [1, 64, 128, 200, 512, 1000, 8192])
+def test_no_number_of_rows_asks_for_more_than_the_bound(shape, most):
+    """Each shape by itself, every number of rows: fewer may split K more, so none stands for the others."""
+    have = torch.ops.bfly.gemm_workspace_bound(most, *shape)
+    need = [torch.ops.bfly.gemm_workspace_size(m, *shape) for m in range(1, most + 1)]
+    assert max(need) == have
+
+
+@pytest.mark.parametrize("N", [128, 384, 2048, 10240])
+def test_nothing_is_split_behind_the_rows_that_the_bound_looks_at(N):
+    for K in (1024, 8192, 28672):
+        last = 256 * (512 // -(-N // 256))
+        for M in (*range(last + 1, last + 600, 7), 2 * last, 3 * last + 5):
+            assert torch.ops.bfly.gemm_workspace_size(M, N, K) == 0, (M, K)
+
+
+@pytest.mark.parametrize("M", [2, 3, 4, 5])
+@pytest.mark.parametrize("N,K", [(8192, 4160), (8192, 4096), (16384, 4160), (10240, 8192)])
+def test_few_rows_have_room_for_every_plan(M, N, K):
+    """Row-major weights run the plan of their own rows, packed ones of many columns that of five."""
+    room = torch.ops.bfly.gemm_workspace_size(M, N, K)
+    for rows in (M, 5 if N % 256 == 0 else M):
+        sk = ops.gemm_plan(rows, N, K)["splitk"]
+        assert sk == 1 or room >= 4 * (torch.ops.bfly.gemm_slab_offset() + sk * M * N)
