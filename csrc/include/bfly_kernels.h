@@ -125,8 +125,8 @@ int launch_gemm_plan(const GemmPlan& p, const bf16* X, long ldx, const bf16* W, 
 // The plan that launch_gemm runs (without a row scale) on rows ldx and ldw apart; plan_gemm's is where it starts from
 GemmPlan gemm_call_plan(int M, int N, int K, int epi, long ldx, long ldw);
 int gemm_check(int M, int N, int K, int epi);
-bool gemm_packed_first(int M, int N, int K);           // ... but not where a packed copy of the weights is there
-bool gemm_streams(int M, int N, int K, int epi);      // the plan is the streamed product of few rows
+bool gemm_streams(int M, int N, int K, int epi);      // the plan is the streamed product of few rows ...
+bool gemm_packed_first(int M, int N, int K);           // ... which a packed copy of the weights, where there is one, goes ahead of
 // 0 if the auto plan for this shape takes a RowScale (tile and decode-ring kernels)
 int gemm_rowscale_check(int M, int N, int K, int epi);
 // Y = X W^T without epilogue; when the plan splits K, the f32 slabs are left in the workspace

@@ -56,3 +56,19 @@ def test_rules(M, N, K):
     _near(ops.linear(x, w, bias=glu, epilogue="glu"), ref.linear(x.double(), w.double(), glu, "glu").double())
     # a reader that takes the sums gets the same rows
     assert torch.equal(ops.materialize(ops.linear(x, w, defer=True)), ops.linear(x, w))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K,epi", [(1, 10240, 8192, "none"), (1, 28672, 4096, "silu"), (1, 57344, 8192, "silu"), (3, 28672, 4096, "none"), (4, 24576, 4096, "silu")])
+def test_packed_copies_of_few_rows(M, N, K, epi):
+    """What reads a packed copy where rows stream from the weight itself: its tiles, asked for past `linear`, which would not take them."""
+    assert ops.load_library() and torch.ops.bfly.gemm_packed_check(M, N, K, ops.EPILOGUES[epi]) == 0
+    x, w = _operands(M, N, K)
+    out = torch.full((M, N // 2 if epi == "silu" else N), float("nan"), device=DEV, dtype=torch.bfloat16)
+    ws = torch.zeros(torch.ops.bfly.gemm_workspace_size(M, N, K) // 4 + 1, dtype=torch.float32, device=DEV)
+    assert torch.ops.bfly.gemm_packed(x, ops.pack_w256(w), out, ops.EPILOGUES[epi], None, 0.0, None, 0, 1, ws) == 1
+    want = (x.double() @ w.double().T)
+    if epi == "silu":
+        v = want.view(M, N // 32, 2, 16)
+        want = (torch.nn.functional.silu(v[:, :, 0]) * v[:, :, 1]).reshape(M, N // 2)
+    _near(out, want)
