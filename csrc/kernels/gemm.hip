@@ -2229,8 +2229,8 @@ static GemmPlan plan_tile(int M, int N, int K) {
 }
 
 // The mid-M tile (gemm_mid4_kernel) that takes least, in us: rounds of 256 workgroups of 128 x 128, 128 x 256 or (half column tiles) 256 x
-// 128 at 0.5, 0.7 and 0.75 a K step and 4 for the pipeline's ends, and 2 + 0.5 per MB for the sums of a split K (within 12 % over 180
-// M x N x K of 65 to 2000 rows).
+// 128 at 0.5, 0.7 and 0.75 a K step and 4 for the pipeline's ends, and 2 + 0.5 per MB for the sums of a split K. Over 224 M x N x K of 65 to
+// 2000 rows what the planner takes is within 4 % of the best tile on average (28 % at most: 1400 x 4096 x 4096 on the 256 x 256 tile).
 static GemmPlan plan_mid(int M, int N, int K, double& least) {
   static const struct { int bm, bn, sa, sb; double step; } kTiles[] = {{128, 128, 3, 7, 0.5}, {128, 256, 4, 3, 0.7}, {256, 128, 3, 4, 0.75}};
   GemmPlan p{};
@@ -2318,13 +2318,14 @@ static GemmPlan plan_gemm_heuristic(int M, int N, int K) {
     // The mid-M tiles where they take 15 % less (what the estimates are off by), this tile's time in us: 1.13 a K step (half tiles
     // 0.72 or, behind other rounds, 0.85) and 5 a round, sums as theirs. Few rows or columns leave it most compute units idle or many sums. us, before -> here: 937 x 4096 x 4096 49.5
     // -> 37.7, 1000 x 2048 x 2048 25.5 -> 20.3, 500 rows 23.9 -> 17.4, 700 x 3072 x 2048 25.7 -> 20.4, 1400 x 2048 x 4096 42 -> 36, 700 x 1024 x 4096
-    // 27.2 -> 20.9, 400 x 2688 x 1024 25.4 -> 12.9, 1000 x 8192 x 8192 stays (102 and 105). Up to 320 rows plans keep their splits, whose sums'
-    // order row kernels are compared in (300 x 2048 x 2048 20.6 where a mid-M tile takes 13.2).
+    // 27.2 -> 20.9, 400 x 2688 x 1024 25.4 -> 12.9, 257 x 2688 x 1024 17.8 -> 12.6, 300 x 1152 x 4096 24.7 -> 16.4, 320 x 8320 x 2048 41.6 -> 28.3, 1000 x 8192 x
+    // 8192 stays (102 and 105). With a row kernel behind that sums the splits: 300 rows of 1024 x 1024 19.5 -> 13.9, 2048 x 2048 24.7 -> 18.9, 4096 x 2048
+    // 45.6 -> 25.3, 2048 x 4096 26.7 -> 24.0, 4096 x 6144 40.9 -> 39.2.
     if (mid_ok) {
       const int halved = p.sk == 1 ? big4_halved(tiles) : 0;
       const double big = (double)(((long)(tiles - halved) * p.sk + 255) / 256) * (1.13 * steps / p.sk + 5) +
                          (halved ? (tiles > 256 ? 0.85 : 0.72) * steps + 5 : 0) + (p.sk > 1 ? 2 + 2e-6 * p.sk * M * N : 0);
-      if (M > 320 && mid < 0.85 * big) return pm;
+      if (mid < 0.85 * big) return pm;
     }
     if (N % 256 == 0) return p;
     // N % 256 == 128: half of the last column tile is wasted and 128 x 128 tiles have four times as many workgroups, two of

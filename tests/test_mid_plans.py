@@ -9,7 +9,9 @@ pytestmark = pytest.mark.skipif(not ops.load_library(), reason="kernel library n
 
 
 @pytest.mark.parametrize("M,N,K,kind", [(64, 2048, 2048, "tile"), (65, 2048, 2048, "mid4"), (256, 6272, 2048, "mid4"), (100, 2048, 192, "tile"),
-                                        (100, 2048, 8192, "tile"), (200, 2048, 8192, "mid4"), (937, 4096, 4096, "mid4"), (1000, 2048, 2048, "mid4"),
+                                        (100, 2048, 8192, "tile"), (200, 2048, 8192, "mid4"), (257, 2048, 2048, "mid4"), (300, 1024, 1024, "mid4"),
+                                        (320, 2688, 1024, "mid4"), (320, 4096, 2048, "mid4"), (300, 4096, 8192, "big4"),
+                                        (937, 4096, 4096, "mid4"), (1000, 2048, 2048, "mid4"),
                                         (2100, 2048, 2048, "big4"), (1000, 8192, 8192, "big4"), (1000, 4224, 1024, "big4"), (8192, 8192, 8192, "big4")])
 def test_where_they_run(M, N, K, kind):
     assert ops.gemm_plan(M, N, K)["kind"] == kind
