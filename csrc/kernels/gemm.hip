@@ -2195,12 +2195,17 @@ GemmPlan plan_gemm(int M, int N, int K) {
   return tuned_plan(M, N, K, p) ? p : plan_gemm_heuristic(M, N, K);
 }
 
-// LDS-tiled kernel: 16 to 128 rows per tile, K split in two until there are 448 workgroups. Where that fills the chip with
-// more than 16 column tiles, up to 64 rows (a weight stream) take the split with the least of the stream (all of it at 6.3 TB/s, the busiest compute unit's at 40 KB a microsecond, rows of
-// X at 0.6 of the weights' cost) and the sums (1 us, 0.2 a split, 0.65 per MB): 2 % off the best of 16 splits on average over 26 N x K by
-// 6, 16, 32, 64 rows with weights from memory, where 448 workgroups were 19 % off (a few past a round of 256, or sums for nothing). us, before -> here: 8320 x 2048 by
-// 32 rows 19.0 -> 13.3, by 48 21.9 -> 15.3, 16384 x 2048 by 16 18.2 -> 15.9, 12416 x 4096 by 32 31.1 -> 26, 5120 x 6144 by 6 21.7 -> 17.4.
-static GemmPlan plan_tile(int M, int N, int K) {
+// LDS-tiled kernel: 16 to 128 rows per tile, K split in two until there are 448 workgroups. Where that fills the chip with more than 16 column
+// tiles, up to 64 rows (a weight stream) take the split with the least of the stream (all of it at 6.3 TB/s or the busiest compute unit's
+// at 40 KB a microsecond, rows of X at 0.6 of the weights' cost, and half of the latter again; 1.2 of it with one workgroup a unit whose splits
+// begin whole 4 KB apart, since their reads then meet in the same memory channels) and the sums (2 us, 0.2 a split, 0.65 per MB). Over 476 M x N x K of 6
+// to 64 rows with weights from memory that is 1.3 % off the best of 16 splits on average, where 448 workgroups were 20 % off (a few past a round
+// of 256, or sums for nothing). us, 448 workgroups -> here: 8320 x 2048 by 32 rows 19.0 -> 13.3, by 48 21.9 -> 15.3, 16384 x 2048 by 16 18.2 -> 15.9,
+// 12416 x 4096 by 32 31.1 -> 26, 5120 x 6144 by 6 21.7 -> 17.4; 15360 x 4096 by 6 and 32 stay at 24.7 and 29.5 (two splits 30.9 and 33.5).
+// More than 32 rows: four stages where a compute unit has one workgroup, three where it has two (32768 x 4096 by 64 in four up to 1.24 of that).
+// Packed weights have no such channels and cheaper ends: the stream alone, the sums at 1 us less (14336 x 4096 by 8 and 32 rows in two splits 22.7 and
+// 24.9, in the four of row-major weights 24.7 and 28.2).
+static GemmPlan plan_tile(int M, int N, int K, bool packed = false) {
   GemmPlan p{};
   const int target = 448;
   p.kind = 1;
@@ -2212,18 +2217,21 @@ static GemmPlan plan_tile(int M, int N, int K) {
   else { p.bm = 128; p.wk = 2; }
   p.bn = 128;
   const int tiles = ((M + p.bm - 1) / p.bm) * (N / p.bn);
-  if (M > 32 && stream && tiles > 256) p.mt = 3;      // (two workgroups a compute unit)
   int sk = 1;
   const int ktiles = K / kBK;
   while (tiles * sk < target && sk * 2 * 4 <= ktiles && sk < 16) sk *= 2;
   if (stream && tiles * sk >= 256 && tiles > 16) {
     double least = 0;
     for (int n = 1; n <= 16 && (n == 1 || ktiles >= 4 * n); ++n) {
-      const double unit = ((long)tiles * n + 255) / 256 * (K / (double)n) * (256 + 1.2 * M);      // bytes
-      const double us = std::max(2. * N * K / 6.3e6, unit / 40e3) + (n > 1 ? 1 + 0.2 * n + 2.6e-6 * n * M * N : 0);
+      const int rounds = (tiles * n + 255) / 256;
+      const double unit = rounds * (K / (double)n) * (256 + 1.2 * M) / 40e3;
+      const double most = std::max(2. * N * K / 6.3e6, unit), sums = n > 1 ? 1 + 0.2 * n + 2.6e-6 * n * M * N : 0;
+      const double us = packed ? most + sums
+                               : (most + 0.5 * unit) * (rounds == 1 && 2 * K % (4096 * n) == 0 ? 1.2 : 1) + (n > 1 ? 1 + sums : 0);
       if (n == 1 || us < least) least = us, sk = n;
     }
   }
+  if (M > 32 && stream && (packed ? tiles : tiles * sk) > 256) p.mt = 3;
   p.sk = sk;
   return p;
 }
@@ -2349,11 +2357,18 @@ static size_t plan_ws_bytes(const GemmPlan& p, int M, int N) {
 // A row scale with a half column tile: the 256 x 256 tile's epilogue has none, the 128-row tiles' has
 static bool rowscale_on_tile(const GemmPlan& p, int N) { return p.kind == 6 && N % 256 != 0; }
 
-// Enough for the tuned plan, for the plans it may fall back to (below) and for the one of five rows where packed weights take that.
+// Packed weights of up to 64 rows take the split of their own estimate where no entry of the table has the shape
+static bool packed_tile(const GemmPlan& p, int M, int N, int K) {
+  GemmPlan t;
+  return p.kind == 1 && p.sk > 1 && M <= 64 && N % 256 == 0 && plan_overrides().empty() && !tuned_plan(M, N, K, t);
+}
+
+// Enough for the tuned plan, for the plans it may fall back to (below), for packed weights' splits and for the plan of five rows where those take it.
 size_t gemm_workspace_bytes(int M, int N, int K) {
   const GemmPlan h = plan_gemm_heuristic(M, N, K);
   const size_t a = plan_ws_bytes(plan_gemm(M, N, K), M, N), b = plan_ws_bytes(h, M, N);
   return std::max({a, b, rowscale_on_tile(h, N) ? plan_ws_bytes(plan_tile(M, N, K), M, N) : 0,
+                   packed_tile(h, M, N, K) ? plan_ws_bytes(plan_tile(M, N, K, true), M, N) : 0,
                    gemm_packed_first(M, N, K) ? gemm_workspace_bytes(5, N, K) : 0});
 }
 
@@ -2787,6 +2802,7 @@ int launch_gemm_packed(const bf16* X, long ldx, const bf16* Wp, int M, int N, in
   if (N % 256 != 0 || K % 64 != 0) return -1;
   const int rows = gemm_packed_first(M, N, K) ? 5 : M;      // the plan's
   GemmPlan p = plan_gemm(rows, N, K);
+  if (packed_tile(p, rows, N, K)) p = plan_tile(rows, N, K, true);
   if (tuned_enabled() && plan_overrides().empty() && epi != EPI_SILU_GATE) {
     static const int kB[] = {1, 16, 32, 64, 128, 256, 512};
     int bucket = 0;

@@ -7,9 +7,9 @@ from butterfly_amd import ops
 pytestmark = pytest.mark.skipif(not ops.load_library(), reason="kernel library not built")
 
 
-@pytest.mark.parametrize("M,N,kind", [(16, 16384, "skinny"), (16, 16512, "tile"), (17, 8192, "skinny"), (17, 8320, "tile"), (64, 32000, "tile"), (4, 32000, "skinny")])
+@pytest.mark.parametrize("M,N,kind", [(16, 16384, "skinny"), (16, 16512, "tile"), (17, 8192, "skinny"), (17, 8320, "tile"), (64, 32000, "tile"), (4, 32000, "stream")])
 def test_short_products_under_wide_results(M, N, kind):
-    p = ops.gemm_plan(M, N, 1024)
+    p = ops.gemm_plan(M, N, 1024, "none")
     assert (p["kind"], p["splitk"]) == (kind, 1)
 
 
@@ -44,7 +44,8 @@ def test_short(M, N, K):
     _check(M, N, K, False)
 
 
-@pytest.mark.parametrize("M,N,K,sk", [(16, 8320, 2048, 3), (64, 8320, 2048, 3), (32, 16384, 2048, 2), (32, 2048, 2048, 8), (16, 1024, 1536, 4)])
+@pytest.mark.parametrize("M,N,K,sk", [(16, 8320, 2048, 3), (64, 8320, 2048, 3), (32, 16384, 2048, 2), (32, 2048, 2048, 8), (16, 1024, 1536, 4),
+                                       (6, 15360, 4096, 4), (32, 16384, 4096, 4), (12, 65536, 2048, 1)])
 def test_splits_of_streams(M, N, K, sk):
     p = ops.gemm_plan(M, N, K)
     assert (p["kind"], p["splitk"]) == ("tile", sk)
@@ -54,6 +55,14 @@ def test_splits_of_streams(M, N, K, sk):
 @pytest.mark.parametrize("M,N,K", [(16, 8320, 2048), (17, 12416, 1280), (33, 8448, 1088), (64, 16640, 320), (48, 12416, 4096)])
 def test_splits_that_divide_nothing(M, N, K):
     _check(M, N, K, N % 256 == 0)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M", [5, 16, 32, 33, 64])
+@pytest.mark.parametrize("N,K", [(14336, 4096), (16384, 2048), (9216, 4096)])
+def test_packed_weights_split_by_their_own_estimate(M, N, K):
+    """Fewer splits than of the row-major weight, or more; the sums have room in either."""
+    _check(M, N, K, True)
 
 
 @pytest.mark.gpu
