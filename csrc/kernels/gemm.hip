@@ -2237,10 +2237,11 @@ static GemmPlan plan_tile(int M, int N, int K, bool packed = false) {
 }
 
 // The mid-M tile (gemm_mid4_kernel) that takes least, in us: rounds of 256 workgroups of 128 x 128, 128 x 256 or (half column tiles) 256 x
-// 128 at 0.5, 0.7 and 0.75 a K step and 4 for the pipeline's ends, and 2 + 0.5 per MB for the sums of a split K. Over 224 M x N x K of 65 to
-// 2000 rows what the planner takes is within 4 % of the best tile on average (28 % at most: 1400 x 4096 x 4096 on the 256 x 256 tile).
+// 128 at 0.5, 0.7 and 0.75 a K step (0.58, 0.88 and 0.75 from 2048 channels on, where more of a step's rows meet in a memory channel) and 4 for
+// the pipeline's ends, and 2 + 0.5 per MB for the sums of a split K. Over 325 M x N x K of 65 to 2000 rows what the planner takes is within 2.3 % of the
+// best tile on average (33 % at most: 1500 x 4096 x 4096 on the 256 x 256 tile).
 static GemmPlan plan_mid(int M, int N, int K, double& least) {
-  static const struct { int bm, bn, sa, sb; double step; } kTiles[] = {{128, 128, 3, 7, 0.5}, {128, 256, 4, 3, 0.7}, {256, 128, 3, 4, 0.75}};
+  static const struct { int bm, bn, sa, sb; double step, long_k; } kTiles[] = {{128, 128, 3, 7, 0.5, 0.58}, {128, 256, 4, 3, 0.7, 0.88}, {256, 128, 3, 4, 0.75, 0.75}};
   GemmPlan p{};
   const int steps = K / 64;
   least = 0;
@@ -2248,7 +2249,7 @@ static GemmPlan plan_mid(int M, int N, int K, double& least) {
     if (N % t.bn != 0 || (t.bm == 256 && N % 256 == 0)) continue;
     const long tiles = (long)((M + t.bm - 1) / t.bm) * (N / t.bn);
     for (int sk = 1; sk <= 8 && (sk == 1 || (steps >= 4 * sk && tiles * sk <= 256)); sk *= 2) {
-      const double us = (double)((tiles * sk + 255) / 256) * (t.step * steps / sk + 4) + (sk > 1 ? 2 + 2e-6 * sk * M * N : 0);
+      const double us = (double)((tiles * sk + 255) / 256) * ((K >= 2048 ? t.long_k : t.step) * steps / sk + 4) + (sk > 1 ? 2 + 2e-6 * sk * M * N : 0);
       if (least != 0 && us >= least) continue;
       least = us;
       p = GemmPlan{7, t.sa, t.sb, 0, t.bm, t.bn, sk};
@@ -2286,12 +2287,13 @@ static GemmPlan plan_gemm_heuristic(int M, int N, int K) {
   }
   // 65 to 256 rows: mid-M tiles, whose rings keep K steps in flight that the 128-row tiles of plan_tile wait for, split or not.
   // us, before -> here: 100 x 2048 x 2048 12.4 -> 11.9, 256 x 2688 x 1024 17.9 -> 12.8, 65 x 6272 x 2048 22.7 -> 14.4, 256 rows 42.6 ->
-  // 20.8, 128 x 8320 x 2048 35.5 -> 20.0, 180 x 12416 x 4096 71.7 -> 35.3; not where few rows split a long K in 16 (65 x 2048 x 8192 15.1, here
-  // 16.6).
+  // 20.8, 128 x 8320 x 2048 35.5 -> 20.0, 180 x 12416 x 4096 71.7 -> 35.3; not where few rows split a long K in 16 and fit one round of workgroups (65 and
+  // 128 x 2048 x 6144 13.6 and 16.9, on mid-M tiles 17.1 and 19.8, 65 x 1024 x 8192 18.0 and 21.1, 65 x 2048 x 4096 12.6 and 14.6; 65 x 1408 x 4096 16.1 and 15.3, two rounds
+  // 65 x 4096 x 6144 28.6 and 21.1, 128 x 3072 x 8192 32.5 and 24.7).
   double mid = 0;
   const bool mid_ok = M > 64 && N % 128 == 0 && K % 64 == 0 && K >= 256;
   const GemmPlan pm = mid_ok ? plan_mid(M, N, K, mid) : GemmPlan{};
-  if (mid_ok && M <= 256 && !(M <= 128 && K >= 8192 && plan_tile(M, N, K).sk == 16)) return pm;
+  if (mid_ok && M <= 256 && !(M <= 128 && N <= 2048 && (long)N * K >= 8 << 20 && plan_tile(M, N, K).sk == 16)) return pm;
   // 256 x 256 tile from two K steps on (its pipeline's least)
   if (M > 256 && N % 128 == 0 && K % 64 == 0 && K >= 128 && (N % 256 == 0 || (N > 1024 && K >= 256))) {
     // prefill / large batch: the 256x256 one-wave-per-SIMD tile (gemm_big4_kernel: 1.52-1.55 PF at M = 8192 on the 70B

@@ -82,7 +82,7 @@ def test_slabs_summed_by_the_row_kernels(M, N, K):
 @pytest.mark.parametrize("M,N,K,kind,splits", [
     (257, 4096, 8192, "big4", 8), (1025, 2048, 4096, "big4", 4), (513, 4096, 4096, "big4", 4),      # a row past a tile, short last tiles
     (555, 2048, 8192, "big4", 8), (777, 4096, 6144, "big4", 4), (257, 4096, 4096, "mid8", 4), (100, 1152, 8192, "tile", 16),
-    (257, 2048, 2048, "mid4", 4), (300, 1024, 2048, "mid4", 4), (300, 4096, 6144, "mid4", 4), (300, 1152, 4096, "mid4", 8),
+    (257, 2048, 2048, "mid4", 4), (300, 1024, 2048, "mid4", 4), (300, 4096, 6144, "big4", 8), (300, 1152, 4096, "mid4", 8),
 ])
 def test_slabs_of_prompts(M, N, K, kind, splits):
     """The same behind the tiles that prompts run on."""
