@@ -271,7 +271,7 @@ gemm_skinny_kernel(const bf16* __restrict__ X, long ldx, const bf16* __restrict_
 // 4096 172 -> 143; eight rows: 2048 x 2048 7.3 -> 4.6, 3072 x 2048 9.3 -> 6.0.
 template <int MT, int NT, int U, int FOLD, bool LAST>
 __device__ __forceinline__ void stream_step(f32x4 (&acc)[NT][MT], const bf16* const (&w)[NT], const bf16* const (&x)[MT], int c, int nw,
-                                            int left) {
+                                            long ktile, int left) {
   bf16x8 a[U][NT][2], b[U][MT][2];
 #pragma unroll
   for (int u = 0; u < U; ++u) {
@@ -280,7 +280,7 @@ __device__ __forceinline__ void stream_step(f32x4 (&acc)[NT][MT], const bf16* co
     for (int h = 0; h < 2; ++h)
 #pragma unroll
       for (int t = 0; t < NT; ++t)
-        a[u][t][h] = ld_nt(reinterpret_cast<const bf16x8*>(w[t] + 64L * FOLD * (c + u * nw) + 32 * FOLD * h));
+        a[u][t][h] = ld_nt(reinterpret_cast<const bf16x8*>(w[t] + (FOLD * (c + u * nw) + FOLD / 2 * h) * ktile + (FOLD == 1 ? 32 * h : 0)));
   }
 #pragma unroll
   for (int u = 0; u < U; ++u) {
@@ -303,9 +303,11 @@ __device__ __forceinline__ void stream_step(f32x4 (&acc)[NT][MT], const bf16* co
   }
 }
 
+// Element k of a weight row: k / 64 * ktile + k % 64, with ktile = 64 in rows of ldw, or (packed: [N / 256][K / 64][256][64]) ldw = 64 and
+// ktile = 256 * 64. (For rows alone, with constants in its place, the loads are issued closer together: one sequence of 8B 909 -> 916 us a step.)
 template <int MT, int NT, int NW, int U, int FOLD>
 __global__ void __launch_bounds__(64 * NW)
-gemm_stream_kernel(const bf16* __restrict__ X, long ldx, const bf16* __restrict__ W, long ldw, int M, int N, int K, int epi,
+gemm_stream_kernel(const bf16* __restrict__ X, long ldx, const bf16* __restrict__ W, long ldw, long ktile, int M, int N, int K, int epi,
                    const bf16* __restrict__ bias, bf16* __restrict__ out, long ldo) {
   static_assert(MT == 1 || FOLD == 1, "folded tiles hold one row tile");
   constexpr int RB = 16 / FOLD, KC = 64 * FOLD;
@@ -322,13 +324,16 @@ gemm_stream_kernel(const bf16* __restrict__ X, long ldx, const bf16* __restrict_
   };
   const bf16 *w[NT], *x[MT];
 #pragma unroll
-  for (int t = 0; t < NT; ++t) w[t] = W + wrow(t, r % RB) * ldw + ko;
+  for (int t = 0; t < NT; ++t) {
+    const int n = wrow(t, r % RB);
+    w[t] = W + (ktile == 64 ? n * ldw : (long)(n >> 8) * 256 * K + (n & 255) * ldw) + ko / 64 * ktile + ko % 64;
+  }
 #pragma unroll
   for (int t = 0; t < MT; ++t) x[t] = X + (long)min(16 * t + r % RB, M - 1) * ldx + ko;
   f32x4 acc[NT][MT] = {};
   int c = wave;
-  for (; c + (U - 1) * NW < chunks; c += U * NW) stream_step<MT, NT, U, FOLD, false>(acc, w, x, c, NW, U);
-  if (c < chunks) stream_step<MT, NT, U, FOLD, true>(acc, w, x, c, NW, (chunks - c + NW - 1) / NW);
+  for (; c + (U - 1) * NW < chunks; c += U * NW) stream_step<MT, NT, U, FOLD, false>(acc, w, x, c, NW, ktile, U);
+  if (c < chunks) stream_step<MT, NT, U, FOLD, true>(acc, w, x, c, NW, ktile, (chunks - c + NW - 1) / NW);
 #pragma unroll
   for (int t = 0; t < NT; ++t)
 #pragma unroll
@@ -1994,8 +1999,9 @@ static void run_skinny(const bf16* X, long ldx, const bf16* W, long ldw, int M, 
 
 template <int MT, int NT, int NW, int U, int FOLD>
 static void run_stream(const bf16* X, long ldx, const bf16* W, long ldw, int M, int N, int K, int epi, const bf16* bias,
-                       bf16* out, long ldo, hipStream_t stream) {
-  gemm_stream_kernel<MT, NT, NW, U, FOLD><<<N / (16 / FOLD * NT), 64 * NW, 0, stream>>>(X, ldx, W, ldw, M, N, K, epi, bias, out, ldo);
+                       bf16* out, long ldo, hipStream_t stream, bool packed) {
+  gemm_stream_kernel<MT, NT, NW, U, FOLD><<<N / (16 / FOLD * NT), 64 * NW, 0, stream>>>(
+      X, ldx, W, packed ? 64 : ldw, packed ? 256 * 64 : 64, M, N, K, epi, bias, out, ldo);
 }
 
 static void init_nt_policy() {
@@ -2391,8 +2397,8 @@ static int run_plan(const GemmPlan& p, const bf16* X, long ldx, const bf16* W, l
   const RowScale rsc = rs ? *rs : RowScale{nullptr, 0, 0.f, 0.f};
   if (rs != nullptr && p.kind != 1 && p.kind != 3 && p.kind != 5 && p.kind != 7) return -4;   // row scale: tile / ring / mid epilogues
   if (epi == EPI_SILU_GATE && (p.kind != 1 || p.sk != 1)) return -4;   // gate: tile epilogue, no slabs
-  // packed (pack_w256) weights: the tile plans mark it with nt = 1, the mid-M kernels take it here
-  if (packed && p.kind != 5 && p.kind != 7) return -5;
+  // packed (pack_w256) weights: the tile plans mark it with nt = 1, the others take it here
+  if (packed && p.kind != 5 && p.kind != 7 && p.kind != 8) return -5;
   if (p.kind == 4) {
     // 8-phase big tile: every split needs >= 2 K-tiles of 64
     if (N % 256 != 0 || K % 64 != 0 || K / 64 < 2 * p.sk) return -1;
@@ -2460,10 +2466,10 @@ static int run_plan(const GemmPlan& p, const bf16* X, long ldx, const bf16* W, l
     if (K % (64 * fold) != 0 || N % (16 / fold * p.nt) != 0 || M > 16 / fold * p.mt) return -1;
     if (epi == EPI_SILU_GATE || (epi_halves(epi) && N % 32 != 0)) return -1;
     bool done = false;
-#define ST_CASE(MT_, NT_, NW_, U_, F_)                                                                 \
-  if (!done && p.mt == MT_ && p.nt == NT_ && p.wk == NW_ && p.bm == U_ && fold == F_) {                \
-    if (!dry) run_stream<MT_, NT_, NW_, U_, F_>(X, ldx, W, ldw, M, N, K, epi, bias, out, ldo, stream); \
-    done = true;                                                                                       \
+#define ST_CASE(MT_, NT_, NW_, U_, F_)                                                                         \
+  if (!done && p.mt == MT_ && p.nt == NT_ && p.wk == NW_ && p.bm == U_ && fold == F_) {                        \
+    if (!dry) run_stream<MT_, NT_, NW_, U_, F_>(X, ldx, W, ldw, M, N, K, epi, bias, out, ldo, stream, packed); \
+    done = true;                                                                                               \
   }
     ST_CASE(1, 1, 4, 4, 4) ST_CASE(1, 1, 4, 4, 2) ST_CASE(1, 1, 8, 4, 2) ST_CASE(1, 2, 8, 4, 2)
     ST_CASE(1, 1, 4, 4, 1) ST_CASE(1, 1, 8, 4, 1) ST_CASE(1, 2, 8, 4, 1) ST_CASE(2, 1, 8, 4, 1)
@@ -2779,7 +2785,7 @@ int launch_gemm(const bf16* X, long ldx, const bf16* W, long ldw, int M, int N, 
 
 // Decode GEMM over a K-tile-blocked copy of the weight (layout [N/256][K/64][256][64], made
 // once by the engine when HBM allows, models/transformer.pack_decode_weights): the plan the
-// row-major weight would run if it did not stream (16 / 32 / 64-row tiles and the mid-M kernels of kinds 5 / 7, with
+// row-major weight would run (streams of few rows, 16 / 32 / 64-row tiles and the mid-M kernels of kinds 5 / 7, with
 // their split-K; EPI_SILU_GATE: the gate plan) on the packed copy. Each 128-row weight stage is then one 16 KiB run of memory instead of 128
 // runs of 128 B a row pitch apart: the Llama-3-70B gate/up GEMM at M = 64 in 145 against
 // 158 us, bitwise the same result (tools/packed_probe.py). Returns < 0 (nothing launched)
@@ -2803,6 +2809,13 @@ int launch_gemm_packed(const bf16* X, long ldx, const bf16* Wp, int M, int N, in
   if (M <= 0) return dry ? 0 : 1;
   if (N % 256 != 0 || K % 64 != 0) return -1;
   const int rows = gemm_packed_first(M, N, K) ? 5 : M;      // the plan's
+  if (rs == nullptr && rows == M) {
+    const GemmPlan q = select_plan(M, N, K, epi);
+    if (q.kind == 8) {
+      const int rc = run_plan(q, X, ldx, Wp, K, M, N, K, epi, nullptr, out, ldo, ws, stream, dry, false, nullptr, true);
+      return rc != 0 || dry ? rc : 1;
+    }
+  }
   GemmPlan p = plan_gemm(rows, N, K);
   if (packed_tile(p, rows, N, K)) p = plan_tile(rows, N, K, true);
   if (tuned_enabled() && plan_overrides().empty() && epi != EPI_SILU_GATE) {

@@ -5,6 +5,8 @@ import torch
 from butterfly_amd import ops
 from butterfly_amd.ops import reference as ref
 
+pytestmark = pytest.mark.skipif(not ops.load_library(), reason="kernel library not built")
+
 DEV = "cuda"
 # [kind, row tiles, column tiles, waves, chunks in flight, fold, 1] and the rows it takes
 PLANS = [([8, 1, 1, 4, 4, 4, 1], 4), ([8, 1, 1, 4, 4, 2, 1], 8), ([8, 1, 1, 8, 4, 2, 1], 8), ([8, 1, 2, 8, 4, 2, 1], 8),
@@ -59,16 +61,21 @@ def test_rules(M, N, K):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("M,N,K,epi", [(1, 10240, 8192, "none"), (1, 28672, 4096, "silu"), (1, 57344, 8192, "silu"), (3, 28672, 4096, "none"), (4, 24576, 4096, "silu")])
+@pytest.mark.parametrize("M,N,K,epi", [(1, 10240, 8192, "none"), (1, 1024, 1024, "none"), (1, 57344, 8192, "silu"), (4, 2048, 2048, "silu"), (8, 4096, 4096, "none"),
+                                       (16, 3072, 2048, "none"), (30, 2560, 1024, "none"), (3, 28672, 4096, "none"), (4, 24576, 4096, "silu")])
 def test_packed_copies_of_few_rows(M, N, K, epi):
-    """What reads a packed copy where rows stream from the weight itself: its tiles, asked for past `linear`, which would not take them."""
-    assert ops.load_library() and torch.ops.bfly.gemm_packed_check(M, N, K, ops.EPILOGUES[epi]) == 0
+    """The operator over a packed copy, which `linear` leaves for the weight where rows stream: the same streams, bit for bit, or (two to four rows
+    of many columns) the tiles of five."""
     x, w = _operands(M, N, K)
-    out = torch.full((M, N // 2 if epi == "silu" else N), float("nan"), device=DEV, dtype=torch.bfloat16)
+    want = ops.linear(x, w, epilogue=epi)
+    assert ops.gemm_plan(M, N, K, epi)["kind"] == "stream" and torch.ops.bfly.gemm_packed_check(M, N, K, ops.EPILOGUES[epi]) == 0
+    out = torch.full_like(want, float("nan"))
     ws = torch.zeros(torch.ops.bfly.gemm_workspace_size(M, N, K) // 4 + 1, dtype=torch.float32, device=DEV)
     assert torch.ops.bfly.gemm_packed(x, ops.pack_w256(w), out, ops.EPILOGUES[epi], None, 0.0, None, 0, 1, ws) == 1
-    want = (x.double() @ w.double().T)
+    if torch.ops.bfly.gemm_streams(M, N, K, ops.EPILOGUES[epi]):
+        assert torch.equal(out, want)
+    exact = x.double() @ w.double().T
     if epi == "silu":
-        v = want.view(M, N // 32, 2, 16)
-        want = (torch.nn.functional.silu(v[:, :, 0]) * v[:, :, 1]).reshape(M, N // 2)
-    _near(out, want)
+        v = exact.view(M, N // 32, 2, 16)
+        exact = (torch.nn.functional.silu(v[:, :, 0]) * v[:, :, 1]).reshape(M, N // 2)
+    _near(out, exact)
