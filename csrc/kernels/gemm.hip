@@ -2243,11 +2243,11 @@ static GemmPlan plan_tile(int M, int N, int K, bool packed = false) {
 }
 
 // The mid-M tile (gemm_mid4_kernel) that takes least, in us: rounds of 256 workgroups of 128 x 128, 128 x 256 or (half column tiles) 256 x
-// 128 at 0.5, 0.7 and 0.75 a K step (0.58, 0.88 and 0.75 from 2048 channels on, where more of a step's rows meet in a memory channel) and 4 for
+// 128 at 0.5, 0.7 and 0.75 a K step (0.56, 0.88 and 0.75 from 2048 channels on, where more of a step's rows meet in a memory channel) and 4 for
 // the pipeline's ends, and 2 + 0.5 per MB for the sums of a split K. Over 325 M x N x K of 65 to 2000 rows what the planner takes is within 2.3 % of the
 // best tile on average (33 % at most: 1500 x 4096 x 4096 on the 256 x 256 tile).
 static GemmPlan plan_mid(int M, int N, int K, double& least) {
-  static const struct { int bm, bn, sa, sb; double step, long_k; } kTiles[] = {{128, 128, 3, 7, 0.5, 0.58}, {128, 256, 4, 3, 0.7, 0.88}, {256, 128, 3, 4, 0.75, 0.75}};
+  static const struct { int bm, bn, sa, sb; double step, long_k; } kTiles[] = {{128, 128, 3, 7, 0.5, 0.56}, {128, 256, 4, 3, 0.7, 0.88}, {256, 128, 3, 4, 0.75, 0.75}};
   GemmPlan p{};
   const int steps = K / 64;
   least = 0;
