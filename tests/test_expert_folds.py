@@ -16,6 +16,10 @@ from tests.test_expert_tiles import reference
     ([60, 2, 3, 1] + [1] * 60, 2048, 128, False, False),         # rows found through the sorted list
     ([3, 0, 1, 7, 9, 2, 1, 17], 2048, 1024, False, True),         # loaded past the caches
     ([3, 0, 1, 7, 9, 2, 1, 17, 10], 2048, 1024, True, False),
+    # sixteen pairs, of which no group can be crowded, and one more
+    ([16, 0, 0, 0, 0, 0, 0, 0], 2048, 640, False, True),
+    ([9, 0, 7, 0, 0, 0, 0, 0], 2304, 384, True, False),
+    ([16, 0, 0, 1, 0, 0, 0, 0], 2048, 2048, False, False),
     # crowded groups: 17 to 64 rows at once, pieces that do not fill their eights, groups whose pieces alternate, both products
     ([17, 31, 0, 0, 0, 0, 0, 0], 2048, 128, False, True),
     ([32, 16, 0, 0, 0, 0, 0, 0], 2176, 640, True, False),
