@@ -2244,7 +2244,7 @@ static GemmPlan plan_tile(int M, int N, int K, bool packed = false) {
 
 // The mid-M tile (gemm_mid4_kernel) that takes least, in us: rounds of 256 workgroups of 128 x 128, 128 x 256 or (half column tiles) 256 x
 // 128 at 0.5, 0.7 and 0.75 a K step (0.56, 0.88 and 0.75 from 2048 channels on, where more of a step's rows meet in a memory channel) and 4 for
-// the pipeline's ends, and 2 + 0.5 per MB for the sums of a split K. Over 325 M x N x K of 65 to 2000 rows what the planner takes is within 2.3 % of the
+// the pipeline's ends, and 2 + 0.5 per MB for the sums of a split K. Over 325 M x N x K of 65 to 2000 rows what the planner takes is within 2.2 % of the
 // best tile on average (33 % at most: 1500 x 4096 x 4096 on the 256 x 256 tile).
 static GemmPlan plan_mid(int M, int N, int K, double& least) {
   static const struct { int bm, bn, sa, sb; double step, long_k; } kTiles[] = {{128, 128, 3, 7, 0.5, 0.56}, {128, 256, 4, 3, 0.7, 0.88}, {256, 128, 3, 4, 0.75, 0.75}};
@@ -2268,6 +2268,7 @@ static GemmPlan plan_gemm_heuristic(int M, int N, int K) {
   GemmPlan p{};
   const int target = 448;
   const bool skinny_ok = K % 128 == 0 && N % 128 == 0;
+  // (one to four rows: for the gate epilogue, and what stream_plan compares with; the products themselves stream)
   // register-streaming kernel: GEMV-like M, and short-K shapes (row-parallel projections
   // after TP splits K) where the LDS pipeline cannot fill before the K loop ends
   // (not where the results are wide: there the tiles fill the chip without splitting K, and a row of X is read once per 128 columns
@@ -2335,7 +2336,8 @@ static GemmPlan plan_gemm_heuristic(int M, int N, int K) {
     // 0.72 or, behind other rounds, 0.85) and 5 a round, sums as theirs. Few rows or columns leave it most compute units idle or many sums. us, before -> here: 937 x 4096 x 4096 49.5
     // -> 37.7, 1000 x 2048 x 2048 25.5 -> 20.3, 500 rows 23.9 -> 17.4, 700 x 3072 x 2048 25.7 -> 20.4, 1400 x 2048 x 4096 42 -> 36, 700 x 1024 x 4096
     // 27.2 -> 20.9, 400 x 2688 x 1024 25.4 -> 12.9, 257 x 2688 x 1024 17.8 -> 12.6, 300 x 1152 x 4096 24.7 -> 16.4, 320 x 8320 x 2048 41.6 -> 28.3, 1000 x 8192 x
-    // 8192 stays (102 and 105). With a row kernel behind that sums the splits: 300 rows of 1024 x 1024 19.5 -> 13.9, 2048 x 2048 24.7 -> 18.9, 4096 x 2048
+    // 8192 stays (102 and 105). Where a reader took a split's sums as they are a step saves less: with the norm behind 850 and 1000 x 4096 x 4096 49.1 -> 46.6
+    // and 52.8 -> 48.9. With a row kernel behind that sums the splits: 300 rows of 1024 x 1024 19.5 -> 13.9, 2048 x 2048 24.7 -> 18.9, 4096 x 2048
     // 45.6 -> 25.3, 2048 x 4096 26.7 -> 24.0, 4096 x 6144 40.9 -> 39.2.
     if (mid_ok) {
       const int halved = p.sk == 1 ? big4_halved(tiles) : 0;
@@ -2571,7 +2573,8 @@ int launch_gemm_plan(const GemmPlan& p, const bf16* X, long ldx, const bf16* W, 
 // Up to four rows always, but where a split tile's sums cost nothing extra because their reader takes them as they are: it reads as
 // fast then (4096 x 14336 20.0 and 21.2 us, 6144 x 4096 by four rows 10.7 and 12.2) except for one row up to 8192 channels (10240 x
 // 8192 28.5 and 26.9). Up to eight rows where X does not weigh in: 4096 channels and 10240 columns (5120 x 2048 11.4 -> 8.3 us, 4096 x
-// 4096 9.9 -> 9.0; 14336 x 4096 23.6 and 25.2), in place of split sums 4096 x 4096 or 2048 channels (2048 x 2048 7.3 -> 4.6, read as
+// 4096 9.9 -> 9.0; 14336 x 4096 31.7 and 30.7, but 22.7 on tiles over
+// packed weights, which streams would go ahead of), in place of split sums 4096 x 4096 or 2048 channels (2048 x 2048 7.3 -> 4.6, read as
 // they are 5.1). Up to 16 rows to 1024 channels (1024 x 1024 5.9 -> 4.3), and to 2048 in place of split sums of a product that widens
 // its rows, to two rounds of its tiles (3072 x 2048 9.6 -> 7.0, 8320 x 2048 15.8 and 11.7; those of one that does not are read as they are:
 // 2048 x 2048 5.4 and 6.6). Up to 32 rows to 1024 channels
@@ -2841,8 +2844,8 @@ int launch_gemm_packed(const bf16* X, long ldx, const bf16* Wp, int M, int N, in
   }
   // 160 to 256 tiles of 128 columns: one a compute unit, K unsplit, four stages in flight. Split by what row-major weights need (neighbouring
   // tiles' rows then meet in few memory channels, packed ones do not) they pay for sums. us, before -> here: 20480 x 4096 by 16 rows 37.8 ->
-  // 30.0, by 32 39.9 -> 33.0, 24576 x 4096 by 6, 32 and 64 38.9 -> 33.1, 46.7 -> 34.6, 50.9 -> 39.0, 28672 x 4096 by 32 40.3 -> 39.3 and 43.8 -> 35.8 on another
-  // card, 28672 x 8192 by 16 88 -> 76; outside: 16384 x 4096 by 16 and 32 26.7 and 27.6, 30.0 and 35.0, 36864 x 4096 by 32 62.6 and 64.8.
+  // 30.0, by 32 39.9 -> 33.0, 24576 x 4096 by 6, 32 and 64 38.9 -> 33.1, 46.7 -> 34.6, 50.9 -> 39.0, 28672 x 4096 by 32 (64-row tiles unsplit before) 40.3 -> 39.3, 43.8
+  // -> 35.8 and 39.4 -> 36.4 on three cards, 28672 x 8192 by 16 88 -> 76; outside: 16384 x 4096 by 16 and 32 26.7 and 27.6, 30.0 and 35.0, 36864 x 4096 by 32 62.6 and 64.8.
   const int ctiles = N / 128;
   if (p.kind == 1 && M <= 64 && ctiles >= 160 && ctiles <= 256 && K >= 256 && epi != EPI_SILU_GATE && plan_overrides().empty())
     p = GemmPlan{1, 4, 1, M <= 32 ? 1 : 2, M <= 16 ? 16 : M <= 32 ? 32 : 64, 128, 1};
