@@ -100,8 +100,8 @@ def main():
                 x = torch.randn(M, K, device="cuda", dtype=torch.bfloat16)
                 nout = N // 2 if epi == "silu" else N
                 out = torch.empty(M, nout, device="cuda", dtype=torch.bfloat16)
-                plan = ops.gemm_plan(M, N, K)
-                auto = [("skinny", "tile", "big", "dec", "big8", "mid8", "big4", "mid4").index(plan["kind"]), plan["mt"], plan["nt"], plan["wk"], plan["bm"],
+                plan = ops.gemm_plan(M, N, K, epi)
+                auto = [("skinny", "tile", "big", "dec", "big8", "mid8", "big4", "mid4", "stream").index(plan["kind"]), plan["mt"], plan["nt"], plan["wk"], plan["bm"],
                         plan["bn"], plan["splitk"]]
                 t = timeit(lambda i: torch.ops.bfly.gemm_with_plan(x, Ws[i % copies], out, auto, ops.EPILOGUES[epi], ws),
                            tag={"shape": f"{group}.{name}", "M": M, "N": N, "K": K, "plan": auto, "auto": True})

@@ -43,7 +43,7 @@ def main():
     x = torch.randn(M, K, device="cuda", dtype=torch.bfloat16)
     out = torch.empty(M, N // 2 if a.epi == "silu" else N, device="cuda", dtype=torch.bfloat16)
     ws = torch.zeros(64 << 20, dtype=torch.float32, device="cuda")
-    auto = ops.gemm_plan(M, N, K)
+    auto = ops.gemm_plan(M, N, K, a.epi)
     print(f"shape N={N} K={K} M={M} auto plan {auto}", flush=True)
     for spec in a.plans.split(";"):
         pl = [int(v) for v in spec.split(",")]

@@ -134,7 +134,7 @@ if rank == 0:
               "down": (cfg.hidden_size, cfg.intermediate_size // world)}
     plans = []
     for name, (n, k) in shapes.items():
-        pl = ops.gemm_plan(B, n, k)
+        pl = ops.gemm_plan(B, n, k, "none")
         plans.append(f"{name} {pl['kind']} {pl['bm']}x{pl['bn']} sk{pl['splitk']}")
     print(f"tp{world} {preset} (2 layers) rows {B}: prefill rel {rel_p:.2e} decode rel {rel_d:.2e} "
           f"all-reduces/step {ar_calls} plans: " + ", ".join(plans), flush=True)

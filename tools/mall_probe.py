@@ -36,7 +36,7 @@ def main():
     for name, N, K in SHAPES:
         x = (torch.rand(M, K, device="cuda") * 2 - 1).to(torch.bfloat16)
         w = ((torch.rand(N, K, device="cuda") * 2 - 1) * 0.02).to(torch.bfloat16)
-        sk = ops.gemm_plan(M, N, K)["splitk"]
+        sk = ops.gemm_plan(M, N, K, "none")["splitk"]
         wv = w.view(N, sk, K // sk)
 
         def gemm():

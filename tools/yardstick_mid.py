@@ -52,7 +52,7 @@ def main():
                 ours = timed(lambda i: ops.linear(x, Ws[i % copies], epilogue=epi), a.iters)
                 lib = timed(lambda i: torch.matmul(x, Ws[i % copies].t()), a.iters)
                 fl = 2.0 * M * N * K
-                print(json.dumps({"shape": f"{group}.{name}", "M": M, "N": N, "K": K, "plan": ops.gemm_plan(M, N, K),
+                print(json.dumps({"shape": f"{group}.{name}", "M": M, "N": N, "K": K, "plan": ops.gemm_plan(M, N, K, "none"),
                                   "ours_us": round(ours, 2), "hipblaslt_us": round(lib, 2),
                                   "ours_TF": round(fl / ours / 1e6, 1), "hipblaslt_TF": round(fl / lib / 1e6, 1)}),
                       flush=True)
